@@ -110,6 +110,25 @@ int mist_inter_stage_search_bounded(int n_families, const MistDpShape *shapes,
                                     int64_t *out_stats, void *stream, const double *host_estimate,
                                     double limit_factor, int32_t *out_unresolved);
 
+/* Search of the uniform granularities (inter_stage_tune_with_fixed_inter_partition,
+ * mist/analyzer/inter_tuning_uniform.py:261-397) for every table row and every stage count of a
+ * call in one launch: layers and devices split evenly, so a (row, stage count) pair is a sum over
+ * given stages of the cheapest ckpt count of a cell.  A stage costs float32(stable) +
+ * float32(delta) / G in float64; total = sum + (G - 1) * largest, stages in order.
+ *   tables, index : the intra-stage tables (variants as in MistOutTables; sample position `slot`)
+ *   d_grad_accum[n_rows]: G of every table row;  d_problems[n_problems][2]: (stage count S, mesh
+ *                   index q); stage i of S takes L / S layers, the last L % S stages one more
+ *                   (:95-102), at p = S - 1 - i pre-saved micro-batches
+ *   ckpt_mode     : 0 = every ckpt count 0..l of a stage, 1 = l only, 2 = one count for all stages,
+ *                   0..smallest layer count (uniform-pp-simple-heuristic-mem-opt, :335-343)
+ * d_total[n_rows][n_problems] (+inf: infeasible), d_ckpt and d_row [n_rows][n_problems][max_stages]:
+ * ckpt count and strategy row index of every stage (first minimum, as the reference's strict "<"). */
+int mist_uniform_search(const MistOutTables *tables, int num_layers, int p_dim, int sample_size,
+                        int slot, int num_mesh, const int32_t *d_grad_accum, int n_rows,
+                        const int32_t *problems, const int32_t *d_problems, int n_problems,
+                        int max_stages, int ckpt_mode, double *d_total, int32_t *d_ckpt,
+                        int32_t *d_row, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

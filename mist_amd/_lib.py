@@ -345,6 +345,10 @@ _INTER_SIGNATURES = {
         [ctypes.c_int, _VP, _VP, ctypes.POINTER(DpCosts), ctypes.POINTER(StrategyIndex),
          ctypes.c_int, ctypes.c_int, _VP, _VP, ctypes.c_int,
          _VP, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _VP, ctypes.c_double, _VP]),
+    "mist_uniform_search": (
+        ctypes.c_int,
+        [ctypes.POINTER(OutTables), ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
+         _VP, ctypes.c_int, _VP, _VP, ctypes.c_int, ctypes.c_int, ctypes.c_int, _VP, _VP, _VP, _VP]),
 }
 
 PLAN_MAX_LIST = 32

@@ -215,6 +215,91 @@ __global__ void strategy_rows_kernel(const MistStrategyIndex tabs, const int32_t
   out[e] = row;
 }
 
+// Evenly split pipelines: one wavefront per (table row, stage count).  Reads a few hundred cells
+// in all, so what it costs is the launch and one chain of loads per stage; on the host the same
+// look-ups needed every table copied over (two thirds of a second for a 32-layer plan).
+__global__ __launch_bounds__(64) void uniform_search_kernel(
+    const MistOutTables tabs, int L, int P1, int S_samples, int slot, int Q,
+    const int32_t *__restrict__ grad_accum, const int32_t *__restrict__ problems, int max_stages,
+    int ckpt_mode, double *__restrict__ out_total, int32_t *__restrict__ out_ckpt,
+    int32_t *__restrict__ out_row) {
+  const int64_t g = blockIdx.y;
+  const int k = blockIdx.x, n_problems = gridDim.x, lane = threadIdx.x;
+  const int S = problems[2 * k], q = problems[2 * k + 1];
+  const double G = (double)grad_accum[g];
+  const int64_t gq = g * Q + q;
+  const int per_stage = L / S, longer = S - L % S;  // stages from `longer` on take one more layer
+  auto layers_of = [&](int s) { return per_stage + (s >= longer ? 1 : 0); };
+  // cell of stage s with c ckpt layers: variant and element (inter_tuning_uniform.py:290-330)
+  auto cell_of = [&](int s, int c, int *variant) {
+    const int64_t l = layers_of(s), p = S - 1 - s, C = L + 1;
+    int64_t at;
+    if (S == 1) { *variant = 3; at = gq * C + c; }
+    else if (s == 0) { *variant = 1; at = ((gq * P1 + p) * L + l - 1) * C + c; }
+    else if (s == S - 1) { *variant = 2; at = (gq * L + l - 1) * C + c; }
+    else { *variant = 0; at = ((gq * P1 + p) * L + l - 1) * C + c; }
+    return at * S_samples + slot;
+  };
+  auto cost_of = [&](int s, int c) {
+    int v;
+    const int64_t at = cell_of(s, c, &v);
+    return (double)(float)tabs.stable[v][at] + (double)(float)tabs.delta[v][at] / G;
+  };
+  // first smallest (cost, ckpt count) over the lanes
+  auto first_min = [&](double &t, int &c) {
+    for (int step = 32; step > 0; step >>= 1) {
+      const double ot = __shfl_xor(t, step);
+      const int oc = __shfl_xor(c, step);
+      if (ot < t || (ot == t && oc < c)) { t = ot; c = oc; }
+    }
+  };
+  int32_t *ckpt = out_ckpt + (g * n_problems + k) * max_stages;
+  int32_t *row = out_row + (g * n_problems + k) * max_stages;
+  double total = INFINITY;
+  if (ckpt_mode == 2) {
+    int best_c = 0x7fffffff;
+    for (int c = lane; c <= per_stage; c += 64) {
+      double sum = 0.0, largest = 0.0;
+      for (int s = 0; s < S; ++s) {
+        const double t = cost_of(s, c);
+        sum += t;
+        largest = s == 0 ? t : fmax(largest, t);
+      }
+      const double candidate = sum < INFINITY ? largest * (G - 1.0) + sum : (double)INFINITY;
+      if (candidate < total) { total = candidate; best_c = c; }
+    }
+    first_min(total, best_c);
+    for (int s = lane; s < S; s += 64) {
+      int v;
+      const int64_t at = total < INFINITY ? cell_of(s, best_c, &v) : -1;
+      ckpt[s] = at < 0 ? -1 : best_c;
+      row[s] = at < 0 ? -1 : tabs.index[v][at];
+    }
+  } else {
+    double sum = 0.0, largest = 0.0;
+    for (int s = 0; s < S; ++s) {
+      const int l = layers_of(s);
+      double t = INFINITY;
+      int c_best = 0x7fffffff;
+      for (int c = ckpt_mode == 1 ? l + lane : lane; c <= l; c += 64) {
+        const double tc = cost_of(s, c);
+        if (tc < t) { t = tc; c_best = c; }
+      }
+      first_min(t, c_best);
+      sum += t;
+      largest = s == 0 ? t : fmax(largest, t);
+      if (lane == 0) {
+        int v;
+        const int64_t at = t < INFINITY ? cell_of(s, c_best, &v) : -1;
+        ckpt[s] = at < 0 ? -1 : c_best;
+        row[s] = at < 0 ? -1 : tabs.index[v][at];
+      }
+    }
+    if (sum < INFINITY) total = largest * (G - 1.0) + sum;
+  }
+  if (lane == 0) out_total[g * n_problems + k] = total;
+}
+
 struct Search {
   int n_families;
   const MistDpShape *shapes;  // [n_families]
@@ -1131,6 +1216,32 @@ static int search_families(int n_families, const MistDpShape *shapes,
     out_stats[4] = S.round_trips;
     out_stats[5] = S.left_to_host;
   }
+  return 0;
+}
+
+int mist_uniform_search(const MistOutTables *tables, int num_layers, int p_dim, int sample_size,
+                        int slot, int num_mesh, const int32_t *d_grad_accum, int n_rows,
+                        const int32_t *problems, const int32_t *d_problems, int n_problems,
+                        int max_stages, int ckpt_mode, double *d_total, int32_t *d_ckpt,
+                        int32_t *d_row, void *stream) {
+  if (!tables || !d_grad_accum || !problems || !d_problems || !d_total || !d_ckpt || !d_row)
+    return fail(MIST_E_INVALID, "null pointer argument");
+  if (num_layers < 1 || p_dim < 1 || sample_size < 1 || num_mesh < 1 || slot < 0 || slot >= sample_size)
+    return fail(MIST_E_INVALID, "table extents must be positive and slot %d below %d", slot, sample_size);
+  if (n_rows < 1 || n_rows > 65535 || n_problems < 1 || ckpt_mode < 0 || ckpt_mode > 2)
+    return fail(MIST_E_INVALID, "%d table rows, %d problems, ckpt mode %d", n_rows, n_problems, ckpt_mode);
+  for (int v = 0; v < 4; ++v)
+    if (!tables->stable[v] || !tables->delta[v] || !tables->index[v])
+      return fail(MIST_E_INVALID, "null table of variant %d", v);
+  for (int k = 0; k < n_problems; ++k) {
+    const int S = problems[2 * k], q = problems[2 * k + 1];
+    if (S < 1 || S > num_layers || S > max_stages || S > p_dim || q < 0 || q >= num_mesh)
+      return fail(MIST_E_INVALID, "problem %d: %d stages on mesh %d", k, S, q);
+  }
+  hipLaunchKernelGGL(uniform_search_kernel, dim3(n_problems, n_rows), dim3(64), 0, (hipStream_t)stream,
+                     *tables, num_layers, p_dim, sample_size, slot, num_mesh, d_grad_accum, d_problems,
+                     max_stages, ckpt_mode, d_total, d_ckpt, d_row);
+  MIST_HIP_CHECK(hipGetLastError());
   return 0;
 }
 

@@ -307,6 +307,9 @@ class IntraStageTuner:
         # reads nothing else (the stage assignment; with 30 samples the fill of the whole tables
         # is a tenth of its search)
         self.prefill_wanted_cells_only = False
+        # True: the tables hold the evaluated ``sample_slots`` only (slot i of the tables is
+        # ``sample_slots[i]``), for a caller that knows which it asked for
+        self.compact_samples = False
         self.results: Optional[IntraStageTunerOutput] = None
         self.stats: Dict[str, float] = {}
 
@@ -549,7 +552,7 @@ class IntraStageTuner:
         cfg, L = self.config, self.num_layers
         Gs, Q = self.gradient_accumulation_steps_candidates, self.device_mesh_candidates
         P = self.max_possible_pre_saved_micro_batches
-        problem = make_problem(cfg, L, P + 1, self.sample_size, len(self.tp_sizes) * len(Gs), len(Q))
+        problem = make_problem(cfg, L, P + 1, self.table_samples, len(self.tp_sizes) * len(Gs), len(Q))
         if len(groups):
             problem["max_scout_rows"] = max_scout_rows
             problem["max_group_keys"] = max_group_keys
@@ -594,11 +597,16 @@ class IntraStageTuner:
             first = last
         return bounds
 
+    @property
+    def table_samples(self) -> int:
+        """Extent of the tables' sample axis."""
+        return len(self.sample_slots) if self.compact_samples else self.sample_size
+
     def _table_layout(self):
         """Shapes of the four variants' tables and where each starts in the flat allocations."""
         Gn = len(self.tp_sizes) * len(self.gradient_accumulation_steps_candidates)
         Qn = len(self.device_mesh_candidates)
-        P1, L, S = self.max_possible_pre_saved_micro_batches + 1, self.num_layers, self.sample_size
+        P1, L, S = self.max_possible_pre_saved_micro_batches + 1, self.num_layers, self.table_samples
         shapes = [(Gn, Qn, P1, L, L + 1, S), (Gn, Qn, P1, L, L + 1, S), (Gn, Qn, L, L + 1, S), (Gn, Qn, L + 1, S)]
         starts = [0]
         for shape in shapes:
@@ -776,6 +784,8 @@ class IntraStageTuner:
             if events is None and not self.exhaustive and len(self.sample_slots) > 1:
                 slots = np.array(self.sample_slots, dtype=np.int32)
                 all_ratios = np.ascontiguousarray(ratios[slots], dtype=np.float64)
+                if self.compact_samples:
+                    slots = np.arange(len(slots), dtype=np.int32)
                 rc = lib.mist_intra_stage_eval_samples(
                     prob_ptr, _ptr(d["groups"]), d["n_groups"], _ptr(d["terms_prefix"]),
                     d["n_terms_blocks"], _ptr(d["reduce_prefix"]), d["n_reduce_blocks"],
@@ -787,6 +797,7 @@ class IntraStageTuner:
                 _lib.check(rc, "mist_intra_stage_eval_samples")
                 continue
             for i, slot in enumerate(self.sample_slots):
+                at = i if self.compact_samples else slot
                 if events is None and not self.exhaustive:
                     rc = lib.mist_intra_stage_eval(
                         prob_ptr, _ptr(d["groups"]), d["n_groups"],
@@ -794,7 +805,7 @@ class IntraStageTuner:
                         _ptr(d["reduce_prefix"]), d["n_reduce_blocks"],
                         _ptr(d["scout_prefix"]), d["n_scout_blocks"],
                         _ptr(w["row_terms"]), _ptr(w["stage_floor"]), _ptr(w["key_terms"]),
-                        _ptr(w["partial_cost"]), _ptr(w["partial_index"]), float(ratios[slot]), int(slot),
+                        _ptr(w["partial_cost"]), _ptr(w["partial_index"]), float(ratios[slot]), int(at),
                         1 if i == 0 else 0, ctypes.byref(out), stream,
                     )
                     _lib.check(rc, "mist_intra_stage_eval")
@@ -807,7 +818,7 @@ class IntraStageTuner:
                 timed("eval_reduce", lambda: reduce_call(slot))
                 timed("finalize", lambda: lib.mist_finalize(
                     prob_ptr, _ptr(d["groups"]), d["n_groups"], _ptr(d["reduce_prefix"]),
-                    _ptr(w["row_terms"]), _ptr(w["partial_cost"]), _ptr(w["partial_index"]), int(slot),
+                    _ptr(w["row_terms"]), _ptr(w["partial_cost"]), _ptr(w["partial_index"]), int(at),
                     ctypes.byref(out), stream))
         if len(streams) > 1:
             current.wait_stream(streams[1])
@@ -824,7 +835,8 @@ class IntraStageTuner:
             spaces = _SpacesOfEntry(plan["spaces"], t)
             outs.append(IntraStageTunerOutput(
                 self.gradient_accumulation_steps_candidates, self.device_mesh_candidates, view,
-                spaces, self.sample_slots, batch=tables, batch_index=t,
+                spaces, range(self.table_samples) if self.compact_samples else self.sample_slots,
+                batch=tables, batch_index=t,
             ))
         return outs
 

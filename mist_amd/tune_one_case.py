@@ -35,7 +35,8 @@ from . import _lib
 from . import inter_tuning as _inter_tuning
 from .config import OFFLOADING_RATIO_CANDIDATES, MistConfig, tp_candidates
 from .inter_tuning import inter_stage_tune, inter_stage_tune_batch
-from .inter_tuning_uniform import inter_stage_tune as inter_stage_tune_uniform
+from .inter_tuning_uniform import cells_wanted as uniform_cells_wanted
+from .inter_tuning_uniform import inter_stage_tune_batch_uniform
 from .inter_tuning_uniform_device import inter_stage_tune_batch_uniform_device
 from .inter_tuning_mip import cells_wanted as mip_cells_wanted
 from .inter_tuning_mip import inter_stage_tune_batch as inter_stage_tune_batch_mip
@@ -174,6 +175,11 @@ class PreparedSearch:
                                      tp_candidates(mist_config), mist_config,
                                      sample_size=sample_size, sample_slots=[0], device=device,
                                      exhaustive=exhaustive)
+        if self.granularity.startswith("uniform-pp"):
+            # the search reads sample 0 of a few layer counts per (G, mesh): nothing else is
+            # evaluated, filled or kept (tables of all 30 samples of the 7B plan are 9.7 GB)
+            self.tuner.cells_wanted = uniform_cells_wanted(self.L, hw.num_nodes, hw.num_gpus_per_node)
+            self.tuner.prefill_wanted_cells_only = self.tuner.compact_samples = True
         self.plan = self.tuner.prepare()
         with torch.cuda.device(self.tuner.device):
             self.dev_plan = self.tuner.upload(self.plan)
@@ -200,10 +206,11 @@ class PreparedSearch:
         = rows * sum_l (l + 1) * (#pre-saved micro-batch values), groups."""
         L = self.L
         pairs = L * (L + 1) // 2 + L
-        g = self.plan["groups"]
-        rows = int(g["n_rows"].sum())
-        cells = int((g["n_rows"] * g["num_p"]).sum()) * pairs
-        groups = len(g)
+        P1 = self.tuner.max_possible_pre_saved_micro_batches + 1
+        n_rows = {key: space.n_rows for key, space in self.plan["spaces"].items()}
+        rows = sum(n_rows.values())
+        cells = sum(n * min(self.Gs[g], L, P1) for (_, g, _), n in n_rows.items()) * pairs
+        groups = sum(n > 0 for n in n_rows.values())
         return dict(rows=rows, candidates=rows * (L + 1), cells=cells, groups=groups)
 
     def run(self, stats: Optional[dict] = None, split_timing: bool = False):
@@ -245,10 +252,8 @@ class PreparedSearch:
                 self.config, slot=0, stats=stats, only_best_solution=True, table_limit=table_limit,
             )
         else:
-            outcomes = [
-                inter_stage_tune_uniform(self.L, hw.num_nodes, hw.num_gpus_per_node, self.Gs, r, self.config)
-                for r in results
-            ]
+            outcomes = inter_stage_tune_batch_uniform(
+                self.L, hw.num_nodes, hw.num_gpus_per_node, self.Gs, results, self.config)
         stats["intra_launch_s"] = stats.get("intra_launch_s", 0.0) + (t1 - t0)
         stats["inter_s"] = stats.get("inter_s", 0.0) + (time.perf_counter() - t1)
         best_cost, best_solution = float("inf"), None
