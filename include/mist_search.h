@@ -34,7 +34,7 @@ extern "C" {
 #endif
 #define MIST_MAX_MESH 16    /* device-mesh candidates of the inter-stage DP */
 #define MIST_MAX_SCOUT_PAIRS 8 /* offload pairs whose rows the scout pass of a group gathers */
-#define MIST_MAX_SAMPLE_BATCH 16 /* alpha samples per mist_eval_reduce_samples call */
+#define MIST_MAX_SAMPLE_BATCH 32 /* alpha samples per mist_eval_reduce_samples call */
 
 #define MIST_E_INVALID (-1) /* argument / shape check failed, nothing was launched */
 #define MIST_E_HIP (-2)     /* a HIP runtime call failed */
@@ -122,7 +122,11 @@ typedef struct MistProblem {
                                   * bound(G) of the estimate it finds in place.  For the first call
                                   * after the incumbent was set to +inf; later calls of the same
                                   * search (further groups) read what the earlier ones left. */
-  int32_t reserved0;
+  int32_t reduce_max_p;          /* largest num_p of the call's groups */
+  /* Sizes of the reduce workspace (mist_reduce_workspace_doubles), at least what the call's groups
+   * need: sum over groups of n_lc_tiles * MIST_LC_TILE * (2 num_p + 2); rows / 512 + 2 groups + 1;
+   * sum over groups of n_lc_tiles * ceil(n_rows / mist_reduce_stage_rows()). */
+  int64_t reduce_cells, reduce_supers, reduce_items;
 } MistProblem;
 
 /* One (gradient-accumulation steps, device mesh) group = one call of the reference's
@@ -139,14 +143,14 @@ typedef struct MistGroupDesc {
   int32_t num_p;                /* pre-saved micro-batch candidates 0..num_p-1 */
   int32_t n_par, n_pair, n_oo, n_ao, n_off;
   int32_t pp_wre, pp_gre;       /* ZeRO flags of the pre/post layer strategy */
-  int32_t rows_per_chunk, n_chunks, n_lc_tiles, n_p_tiles; /* decomposition of the reduce kernel */
+  int32_t rows_per_chunk, n_chunks, n_lc_tiles, n_p_tiles; /* decomposition of the filter launch */
   int32_t lc_tile_begin;        /* the group's n_lc_tiles tiles of 64 (layers, ckpt) pairs start at
                                  * this tile of the pair list: 0 with all tiles for the whole
                                  * tables; a caller that reads a range of layer counts only (the
                                  * stage assignment of inter_tuning_mip.py:282-290) evaluates the
                                  * tiles that hold it, the cells of the other tiles keep their
                                  * pre-filled +inf / -1 */
-  int32_t scout_stride;         /* reduce kernel: 0 = no scout pass for this group; m >= 1 = the
+  int32_t scout_stride;         /* 0 = no scout pass (seeds) for this group; m >= 1 = the
                                  * scout pass reduces the rows of the m (weight, gradient) offload
                                  * pairs scout_pair[0 .. m-1] (n_par * n_oo * n_ao rows each) */
   int16_t scout_pair[MIST_MAX_SCOUT_PAIRS]; /* indices into the pair list, distinct */
@@ -154,6 +158,8 @@ typedef struct MistGroupDesc {
   int64_t row_offset;           /* first row of this group in the row-term workspace */
   int64_t key_offset;           /* first key of this group in the key-term workspace: keys are
                                  * (par * n_ao + ao) * n_pair + pair, n_par * n_ao * n_pair per group */
+  int64_t cell_offset;          /* first entry of this group in the minima of the reduce workspace:
+                                 * n_lc_tiles * MIST_LC_TILE * (2 num_p + 2) entries per group */
   double par[MIST_MAX_PAR][MIST_PAR_FIELDS];
   double wo[MIST_MAX_RATIOS], go[MIST_MAX_RATIOS], oo[MIST_MAX_RATIOS], ao[MIST_MAX_RATIOS];
   uint8_t pair_wo[MIST_MAX_PAIRS], pair_go[MIST_MAX_PAIRS];
@@ -196,6 +202,10 @@ int mist_max_scout_pairs(void);  /* MIST_MAX_SCOUT_PAIRS the library was built w
 int64_t mist_stage_floor_doubles(int64_t total_rows, int n_groups);
 /* doubles of the key-term workspace for `total_keys` keys (sum of n_par * n_ao * n_pair) */
 int64_t mist_key_terms_doubles(int64_t total_keys);
+/* doubles of the reduce workspace `d_partial_cost` of the entry points below for the sizes in
+ * MistProblem.reduce_cells / _supers / _items and n_samples samples per call; `d_partial_index` is
+ * reduce_cells * n_samples int32 */
+int64_t mist_reduce_workspace_doubles(int64_t cells, int64_t supers, int64_t items, int n_samples);
 
 /* Row-invariant terms of every candidate row: decodes the row index, evaluates the alpha-beta
  * communication terms, the 36 interference evaluations and the memory pieces that do not
@@ -226,24 +236,21 @@ int mist_row_terms(const MistProblem *problem, const MistGroupDesc *d_groups, in
                    const int32_t *d_block_prefix, int n_blocks, double *d_row_terms,
                    double *d_stage_floor, double *d_key_terms, void *stream);
 
-/* Per (group, row chunk, (l, c) tile, p tile): evaluates latency and memory per cell, applies
- * the memory mask and keeps the running lexicographic (cost, row) minimum per bucket.
- * Replaces the two hot loops of batched_stage_analyze (batched_module_analyzer.py:2218-3106)
- * and compute_indices (mist/utils/pareto.py:124-144) for one ratio r = alpha/(1-alpha).
- * d_block_prefix[n_groups+1]: first workgroup of each group; a group owns
+/* Evaluates latency and memory of the rows, applies the memory mask and keeps the lexicographic
+ * (cost, row) minimum of every cell.  Replaces the two hot loops of batched_stage_analyze
+ * (batched_module_analyzer.py:2218-3106) and compute_indices (mist/utils/pareto.py:124-144) for
+ * one ratio r = alpha/(1-alpha).
+ * The minima lie in one table in device memory, which five launches lower: *seed* reduces the
+ * rows of the group's scout pairs (MistGroupDesc.scout_stride; the search's winners sit almost
+ * exclusively on rows without weight / gradient offloading; n_scout_blocks 0 = empty minima),
+ * *filter* and *open* rule out 64-row stages by their summaries, *reduce* evaluates the rows of
+ * what is left, *resolve* finds the rows of the minima that were lowered meanwhile.
+ * d_block_prefix[n_groups+1]: first workgroup of each group in the filter launch; a group owns
  * n_lc_tiles*n_p_tiles*n_chunks workgroups ordered (chunk, lc_tile, p_tile), p_tile fastest.
- * Optional scout pass (n_scout_blocks > 0): d_scout_prefix[n_groups+1] gives each group
- * n_lc_tiles*n_p_tiles*mist_reduce_scout_split() workgroups that first reduce the rows of the
- * group's scout pairs (MistGroupDesc.scout_stride; the search's winners sit almost exclusively
- * on rows without weight / gradient offloading; a small kernel then combines the slabs of a
- * tile's scout workgroups into the first of them); every chunk then starts from those minima (they
- * belong to real rows of the group, so the result is unchanged) and lets far fewer rows through
- * to the memory model.
- * d_partial_cost / d_partial_index: [n_blocks + n_scout_blocks][2*MIST_P_TILE+2][MIST_LC_TILE];
- * the first n_blocks slabs are the per-chunk results mist_finalize reads.  A chunk other than
- * the first of its tile whose minima are still its seeds does not write its slab: it stores -2
- * as the slab's first row index (rows are >= -1) and mist_finalize skips the slab; the first
- * chunk always writes and carries the seeds. */
+ * d_scout_prefix[n_groups+1]: n_lc_tiles*n_p_tiles*mist_reduce_scout_split() per group.
+ * d_partial_cost: mist_reduce_workspace_doubles(reduce_cells, .., 1) doubles (any contents on
+ * entry), d_partial_index: reduce_cells int32.  At most 65535 groups, 65535 tiles of the (l, c)
+ * list and 9000 values of p. */
 int mist_eval_reduce(const MistProblem *problem, const MistGroupDesc *d_groups, int n_groups,
                      const int32_t *d_block_prefix, int n_blocks,
                      const int32_t *d_scout_prefix, int n_scout_blocks,
@@ -258,22 +265,21 @@ int mist_eval_reduce(const MistProblem *problem, const MistGroupDesc *d_groups, 
  * (same cells, latencies and memory tests as the tables: batched_module_analyzer.py:2165-2216,
  * 2755-2834, 2866-2923, 2946-3106), the cheapest feasible cost of each stage is kept, and
  * sum + (G - 1) * largest (inter_tuning.py:342) lowers *stage_cost_incumbent.  Needs the row terms
- * of the scout rows (mist_row_terms).  Scratch: the first 4096 doubles of each such group's scout
- * slabs, d_partial_cost + (n_blocks + d_scout_prefix[group]) slabs, which a later scout pass
- * overwrites. */
+ * of the scout rows (mist_row_terms).  Scratch: the group's minima in d_partial_cost, which a
+ * later scout pass overwrites. */
 int mist_stage_cost_first_estimate(const MistProblem *problem, const MistGroupDesc *d_groups,
                                    int n_groups, const int32_t *d_scout_prefix, int n_blocks,
                                    const double *d_row_terms, double ratio, double *d_partial_cost,
                                    void *stream);
 
 /* mist_eval_reduce + mist_finalize for n_samples <= MIST_MAX_SAMPLE_BATCH ratios of the same
- * row terms (reference: the S samples of one compute_indices call, mist/utils/pareto.py:124-144):
- * the scout passes of all samples run as ONE launch (a single one fills a tenth of the GPU), then
- * the main launches, each seeded from its sample's scout slabs, and the finalize launches into
- * sample position sample_index[i], `main_batch` samples per launch (1 <= main_batch <= n_samples;
- * the wavefronts of one sample's tail then run beside the next sample's).  `ratios` and
- * `sample_index` are HOST arrays.
- * d_partial_cost / d_partial_index: [main_batch * n_blocks + n_samples * n_scout_blocks] slabs. */
+ * row terms (reference: the S samples of one compute_indices call, mist/utils/pareto.py:124-144),
+ * into sample positions sample_index[i]: one set of launches, which reads a row and prices its
+ * latency, memory and feasibility once for all of them (`main_batch`, 1 .. n_samples, is the
+ * number of samples a caller of the launches one by one would take together; it is checked and
+ * does not change anything here).  `ratios` and `sample_index` are HOST arrays.
+ * d_partial_cost: mist_reduce_workspace_doubles(reduce_cells, .., n_samples) doubles,
+ * d_partial_index: reduce_cells * n_samples int32. */
 int mist_eval_reduce_samples(const MistProblem *problem, const MistGroupDesc *d_groups,
                              int n_groups, const int32_t *d_block_prefix, int n_blocks,
                              const int32_t *d_scout_prefix, int n_scout_blocks,
@@ -283,16 +289,13 @@ int mist_eval_reduce_samples(const MistProblem *problem, const MistGroupDesc *d_
                              const MistOutTables *tables, void *stream);
 
 /* mist_row_terms + mist_eval_reduce_samples for ALL n_samples ratios of a tuner call (any
- * number; batches of `sample_batch` <= MIST_MAX_SAMPLE_BATCH, main launches of `main_batch` <=
- * sample_batch samples), with the small launches moved out of the way of the large ones: the
- * scout pass of the first batch runs on the library's second stream beside the row terms of the
- * rows it does not gather (as in mist_intra_stage_eval), and the scout pass of batch b + 1 beside
- * the main launches of batch b, into the other of two scout regions.  Same tables as the calls
- * it replaces (reference: the S samples of one compute_indices call per group,
- * mist/utils/pareto.py:124-144).  `ratios` and `sample_index` are HOST arrays of n_samples.
- * d_partial_cost / d_partial_index: [main_batch * n_reduce_blocks + 2 * sample_batch *
- * n_scout_blocks] slabs.  Without a scout pass (n_scout_blocks == 0 or
- * problem->max_scout_rows == 0) the calls it replaces run one after the other on `stream`. */
+ * number; batches of `sample_batch` <= MIST_MAX_SAMPLE_BATCH): the scout pass of the first batch
+ * runs on the library's second stream beside the row terms of the rows it does
+ * not gather.  Same tables as the calls it replaces (reference: the S samples of one
+ * compute_indices call per group, mist/utils/pareto.py:124-144).  `ratios` and `sample_index` are
+ * HOST arrays of n_samples.  Workspaces as for mist_eval_reduce_samples with `sample_batch`
+ * samples.  Without a scout pass (n_scout_blocks == 0 or problem->max_scout_rows == 0) everything
+ * runs on `stream`. */
 int mist_intra_stage_eval_samples(const MistProblem *problem, const MistGroupDesc *d_groups,
                                   int n_groups, const int32_t *d_terms_block_prefix,
                                   int n_terms_blocks, const int32_t *d_reduce_block_prefix,
@@ -306,15 +309,16 @@ int mist_intra_stage_eval_samples(const MistProblem *problem, const MistGroupDes
 /* mist_eval_reduce with every cell evaluated: each (row, layers, ckpt) through the latency and
  * memory model and each pre-saved micro-batch value through the reference's feasibility test
  * (batched_module_analyzer.py:2218-3106, pareto.py:124-144 as written, cell by cell), no scout
- * pass, no sieves.  Same workgroup decomposition (d_block_prefix, n_blocks) and slab layout as
- * the main launch of mist_eval_reduce; every slab is written.  The reference point the pruned
- * search is tested and measured against: identical tables, ~20x the time. */
+ * pass, no sieves.  Each of the n_blocks workgroups (decomposition as above) writes its minima to
+ * a slab of [2*MIST_P_TILE+2][MIST_LC_TILE] entries behind the reduce_cells entries of the table,
+ * which a second kernel combines into it.  The reference point the pruned search is tested and
+ * measured against: identical tables, ~30x the time. */
 int mist_eval_reduce_exhaustive(const MistProblem *problem, const MistGroupDesc *d_groups,
                                 int n_groups, const int32_t *d_block_prefix, int n_blocks,
                                 const double *d_row_terms, double ratio, double *d_partial_cost,
                                 int32_t *d_partial_index, void *stream);
 
-/* Combines the per-chunk partial minima (smallest cost, lowest row among equals),
+/* Takes the winners from the table of minima (smallest cost, lowest row among equals),
  * recomputes stable / delta of the winning row and scatters into the output tables at sample
  * position `sample_index`, reproducing which cells the reference leaves unwritten
  * (batched_module_analyzer.py:2819-2834, 2915-2923, 3021-3033, 3103-3106). */

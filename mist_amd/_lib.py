@@ -65,7 +65,10 @@ PROBLEM_DTYPE = np.dtype(
         ("incumbent_num_devices", "<i4"),
         ("incumbent_ckpt_rule", "<i4"),
         ("incumbent_first_estimate", "<i4"),
-        ("reserved0", "<i4"),
+        ("reduce_max_p", "<i4"),
+        ("reduce_cells", "<i8"),
+        ("reduce_supers", "<i8"),
+        ("reduce_items", "<i8"),
     ],
     align=True,
 )
@@ -80,7 +83,7 @@ GROUP_DTYPE = np.dtype(
         ("rows_per_chunk", "<i4"), ("n_chunks", "<i4"), ("n_lc_tiles", "<i4"),
         ("n_p_tiles", "<i4"), ("lc_tile_begin", "<i4"), ("scout_stride", "<i4"),
         ("scout_pair", "<i2", (MAX_SCOUT_PAIRS,)),
-        ("n_rows", "<i8"), ("row_offset", "<i8"), ("key_offset", "<i8"),
+        ("n_rows", "<i8"), ("row_offset", "<i8"), ("key_offset", "<i8"), ("cell_offset", "<i8"),
         ("par", "<f8", (MAX_PAR, PAR_FIELDS)),
         ("wo", "<f8", (MAX_RATIOS,)), ("go", "<f8", (MAX_RATIOS,)),
         ("oo", "<f8", (MAX_RATIOS,)), ("ao", "<f8", (MAX_RATIOS,)),
@@ -128,6 +131,8 @@ _SIGNATURES = {
     "mist_max_scout_pairs": (ctypes.c_int, []),
     "mist_stage_floor_doubles": (ctypes.c_int64, [ctypes.c_int64, ctypes.c_int]),
     "mist_key_terms_doubles": (ctypes.c_int64, [ctypes.c_int64]),
+    "mist_reduce_workspace_doubles": (
+        ctypes.c_int64, [ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_int]),
     "mist_row_terms": (ctypes.c_int, [_VP, _VP, ctypes.c_int, _VP, ctypes.c_int, _VP, _VP, _VP, _VP]),
     "mist_eval_reduce": (
         ctypes.c_int,

@@ -41,6 +41,7 @@ using mist::fail;
 constexpr int kTermsBlock = 128;  // rows per workgroup of the row-term kernel
 constexpr int kStageRows = 64;    // rows staged through LDS per step of the reduce kernel
 constexpr int kSlots = 2 * MIST_P_TILE + 2;  // per-thread running minima: base, with_pre, post, no_pp
+constexpr int kScoutSplit = 1;    // (mist_reduce_scout_split)
 constexpr double kIncumbentSlack = 0.25;  // relative room above MistProblem.stage_cost_incumbent / G
 // Stage summaries (written with the row terms, read by the reduce kernel): per stage of
 // kStageRows workspace rows the term-wise minimum of the latency and memory columns and the
@@ -928,52 +929,73 @@ __device__ __forceinline__ void take_min(double &best, int32_t &best_row, bool f
 }
 
 // ------------------------------------------------------------------------------------------
-// Kernel 2: evaluate + mask + running argmin.
-// Workgroup = one wavefront = one tile of 64 (l, c) pairs; it streams candidate rows through LDS
-// and each lane keeps the minima of MIST_P_TILE pre-saved micro-batch values for its own
-// (l, c).  No cross-lane reduction is needed: the reduction axis (rows) is the loop.
+// Kernels 2: evaluate + mask + argmin.
 //
 // Memory feasibility is monotone in p: the peaks are built from p * (non-negative) terms by
 // additions only, every floating-point add / multiply is monotone in each operand, and the
 // host rejects negative table values.  So per (row, l, c) the feasible p form a prefix
-// [0, count) and `count` is found by bisection with the exact peak formula at the probed p
-// (no closed-form shortcut: the comparison that decides is the reference's own expression).
-// The minima of a thread are therefore non-decreasing in p, and a row changes a slot iff it is
-// feasible at the lowest slot whose minimum it beats.
+// [0, count) and a row matters to one number per variant: its cost against the minimum of slot
+// count - 1 (the minima of a (l, c) pair do not decrease with p).
 //
-// Almost no row changes anything, so a stage of kStageRows rows goes through three sieves, each
-// keeping a per-lane bit mask of surviving rows so that a lane only pays for its own survivors
-// (a wave executes a sieve as often as its busiest lane, not once per row):
-//   A  objective value against the minimum of the highest slot the stage can reach (a bound
-//      from the term-wise minimum of the stage's memory terms); evaluated transposed, a lane
-//      holding one ROW and the loop running over the tile's pairs;
-//   B  lowest improvable slot and the exact memory test at that slot (minima as of stage start:
-//      they only decrease afterwards, so nothing that could matter later is dropped);
-//   C  survivors in row order against the live minima: bisection for `count`, update.
-// A scout pass runs the same code over a few gathered rows of a whole group first (those of the
-// group's scout offload pairs, see gathered_position); the
-// main pass starts every chunk from the scout's minima (real rows of the same group, hence valid
-// upper bounds), which removes the warm-up in which a fresh chunk lets most rows through.
+// The minima of every (group, (l, c) pair, variant, p, sample) live in one table in HBM
+// (ReduceTables.best) that all wavefronts lower by atomic minima on the bit patterns (costs are
+// not negative, so they order like integers).  Five launches:
+//   seed     the rows of the group's scout pairs against empty minima, in LDS: upper bounds made
+//            of real rows, final for most cells;
+//   filter   stage summaries (term-wise minima of 64 rows, and of 8 such stages) against the
+//            largest minimum of each pair; what some pair of a tile does not rule out becomes an
+//            item (group, tile, stage) of a queue;
+//   open     a wavefront per item: the summary with the minima of the slots the stage can reach;
+//   reduce   what is left, shared out by pairs: lane = row over the open pairs.  A row whose cost
+//            IS the minimum at its own slot (count - 1) offers its row number there (the lowest
+//            one stays, which is the reference's first-index-wins scan, pareto.py:134-142, in any
+//            processing order); a smaller cost lowers the minimum and marks the pair, whose row
+//            numbers no longer count.  The slots below take part in finalize, which takes each
+//            p's winner from the slots at and above it;
+//   resolve  the marked pairs of the items in which some row reached its minimum, again, with the
+//            final minima (the seeds are final for most cells: 19 changes for the 7B plan).
+// What this replaces kept 34 (cost, row) minima per lane in registers (253 of them, two
+// wavefronts per SIMD), one sample and 16 p values per pass over the rows, visited every stage
+// summary with every tile and p tile, and committed rows one by one per lane: 7B on 4x8, one
+// sample: 1.35 ms in the reduce kernels (seeds 0.42, main launch 0.92 of which 0.9 were visits
+// of summaries that close), now seeds 0.50 beside the row terms, filter 0.06, reduce 0.33, resolve
+// 0.07; 22B on 16x8: 37.8e6 visits for 0.1e6 stages whose rows were read, 3.7 -> 1.5 ms per batch
+// of groups; 30 samples of the 7B plan's tables for one tensor-parallel size: 24 -> 7.2 ms.
 // ------------------------------------------------------------------------------------------
-// kPow2G: the group's G is a power of two, so x / G == x * (1 / G) bit for bit (float32 and
-// float64) and the division leaves the inner loop; other G divide.  kFirstTile: this workgroup
-// owns p = 0 and therefore also the last-stage and single-stage variants.
-#ifndef MIST_REDUCE_MIN_WAVES
-#define MIST_REDUCE_MIN_WAVES 2
-#endif
-#ifndef MIST_SCOUT_SPLIT
-#define MIST_SCOUT_SPLIT 4
-#endif
-constexpr int kScoutSplit = MIST_SCOUT_SPLIT;  // scout workgroups per (group, (l, c) tile, p tile)
-constexpr int32_t kSlabUnchanged = -2;  // first row index of a slab that was not written (rows are >= -1)
-constexpr int kPairFields = 4;  // per-pair table of sieve A: thr_b, thr_o, n_ck, n_nock
-constexpr int kLdsRowStride = MIST_ROW_TERMS + 1;  // odd number of doubles: lanes reading the
-                                                   // same term of different rows hit different banks
-static_assert(kStageRows == 64, "the sieve masks are 64-bit");
-static_assert(MIST_ROW_TERMS % 2 == 0, "rows are staged as 16-byte pairs");
-static_assert(MIST_LC_TILE == 64, "one wavefront per workgroup: the stage minima use wave shuffles");
-static_assert(MIST_T_S_LAYER_CK == 0 && MIST_T_GCB < 32,
-              "latency and memory terms must be the first columns: one lane per term in the stage minima");
+constexpr int kSuperStages = 8;    // stages per second-level summary
+constexpr int kQueueShards = 64;   // counters of the item queue: one would serve an append in ~8 ns
+constexpr int kCounterPitch = 32;  // uint32 between counters: a cache line each
+constexpr int kNumXcd = 8;
+constexpr int kCounters = 2 * kQueueShards + kNumXcd;
+constexpr int kSeedThreads = 256;
+constexpr int kReduceThreads = 256;
+constexpr int kReduceBlocks = 2048;          // a multiple of kNumXcd
+constexpr int kSuperBlocks = 64;             // workgroups per group of the second-level summaries
+constexpr int kSeedLdsBytes = 40 * 1024;     // LDS aimed at per seed workgroup: four per CU
+constexpr int kSeedLdsMost = 160 * 1024;
+static_assert(kQueueShards == 64, "a lane per shard");
+constexpr uint32_t kUnresolved = 0x80000000u;
+constexpr double kSlack = 1e-9;
+// r x + d / G in float64 against a threshold of the base objective, whose second term is rounded to
+// float32 (one part in 2^24)
+constexpr double kBaseSlack = 1e-6;
+
+// (by value in the kernel arguments)
+struct ReduceTables {
+  // [pair][slot][sample] (slots_of(num_p) slots): bits of the smallest cost
+  unsigned long long *best;
+  // its lowest row, ~0 = none; kUnresolved + row from the reduce launch, row from the resolve launch
+  // (smaller than any of the former)
+  uint32_t *row;
+  uint32_t *changed;         // [pair's first cell / 4]: samples whose minima the reduce launch lowered
+  double *super_floor;       // [supers][kStageFloorPitch]
+  // [kQueueShards][capacity]: group << 48 | tile << 32 | stage, what the filter and then what the
+  // open launch left; pairs of the latter in which a row reached its minimum
+  unsigned long long *item, *opened, *hit;
+  uint32_t *counter;         // at kCounterPitch: [kQueueShards] items, [kQueueShards] opened, [kNumXcd] drawn
+  uint32_t capacity;
+  int n_samples;
+};
 
 struct LaneMemory {
   double fwd_states, bwd_states, cur_saved, mod_saved, ck_delta, fwd_pk, bwd_pk, out, gcb;
@@ -981,9 +1003,7 @@ struct LaneMemory {
 
   // Peaks of the middle-stage variant for p pre-saved micro-batches (:2755-2786).
   __device__ __forceinline__ void peaks(int p, double &peak_f, double &peak_b) const {
-    peaks_at((double)p, peak_f, peak_b);
-  }
-  __device__ __forceinline__ void peaks_at(double pf64, double &peak_f, double &peak_b) const {
+    const double pf64 = (double)p;
     const double pipe_saved = pf64 * mod_saved + cur_saved;
     const double outp2 = out * pf64 * 2.0;
     const double out2 = out * 2.0;
@@ -1012,14 +1032,10 @@ struct LaneMemory {
   }
 };
 
-// Distinct layer counts of one (l, c) tile up to which sieve A also drops rows by memory.
-constexpr int kTileLayerCounts = 12;
-
 // Workgroups are dealt round-robin to the 8 XCDs, each with its own L2.  Logical workgroups
-// that stream the same rows are consecutive, so runs of kXcdRun logical workgroups are given to
+// that read the same rows are consecutive, so runs of kXcdRun logical workgroups are given to
 // one XCD (and the runs round-robin, which keeps the XCDs evenly loaded).  The grid is padded to
 // a multiple of kNumXcd * kXcdRun; logical indices past the end do nothing.
-constexpr int kNumXcd = 8;
 constexpr int kXcdRun = 16;
 __device__ __forceinline__ int xcd_run_block(int physical) {
   const int xcd = physical % kNumXcd, slot = physical / kNumXcd;
@@ -1031,20 +1047,10 @@ __host__ __device__ constexpr int xcd_padded_grid(int n_blocks) {
 
 __device__ __forceinline__ LaneMemory cell_memory(const double *__restrict__ t, int l, int c);
 
-struct ReduceRange {
-  int64_t row_begin, row_end;  // rows of the group this workgroup covers (multiples of kStageRows)
-  int stage_step;              // visit every stage_step-th stage of the range
-  int skip_stride;             // > 0: skip stages whose index is a multiple (the scout did them)
-  int gathered;                // != 0 (scout pass): "stage" t is not a run of consecutive rows but
-                               // the rows number 64 t .. 64 t + 63 of the group's rows without
-                               // weight / gradient offloading, see gathered_position()
-};
-
 // The search's winners sit almost exclusively on rows whose (weight, gradient) offload pair is
 // the first one, (0, 0): 99.8 % of all cells of the GPT-7B plan, 95 % for LLaMA-13B.  In the
 // workspace order those rows are scattered (one per (parallelism row, activation ratio, optimizer
-// ratio)); the scout pass gathers them, n_par * n_oo * n_ao rows per group,
-// and so seeds every chunk with minima that are final for most cells.
+// ratio)); the seed launch gathers them, n_par * n_oo * n_ao rows per group.
 // With scout_stride = m > 1 the rows of the pairs scout_pair[1 .. m-1] follow.
 __device__ __forceinline__ int64_t gathered_position(const MistGroupDesc *g, int64_t q) {
   const int n_tail = g->n_oo * g->n_ao;
@@ -1065,627 +1071,1026 @@ struct SampleSlots {
   int32_t at[MIST_MAX_SAMPLE_BATCH];
 };
 
-template <bool kPow2G, bool kFirstTile>
-__device__ __forceinline__ void reduce_block(
-    const MistProblem &prob, const MistGroupDesc *__restrict__ g, const ReduceRange range,
-    int p_tile, int lc_tile, const double *__restrict__ row_terms,
-    const double *__restrict__ stage_floor /* of this group's stage 0 */, double ratio,
-    double *lds_terms, double *lds_min, double *lds_pair, int32_t *lds_rowpos,
-    const double *__restrict__ seed_cost,
-    const int32_t *__restrict__ seed_index, double *__restrict__ out_cost,
-    int32_t *__restrict__ out_index, bool skip_unchanged) {
-  const int L = prob.num_layers;
-  const int n_pairs = L * (L + 1) / 2 + L;  // sum over l = 1..L of (l + 1)
-  const int pair_idx = lc_tile * MIST_LC_TILE + threadIdx.x;
-  const bool active = pair_idx < n_pairs;
-  const PairIndex pc = decode_pair(active ? pair_idx : 0);
-  const int l = pc.l, c = pc.c;
-
-  const int p0 = p_tile * MIST_P_TILE;
-  const int n_tile_full = min(MIST_P_TILE, g->num_p - p0);  // p values of this tile
-  // Cells with c == l - 1 are only kept for p == 0 of the base / with_pre variants
-  // (batched_module_analyzer.py:3021-3023, 3103), so such a lane has at most one slot.
-  // Lanes past the last pair of the tile keep no slots; they still hold rows in sieve A.
-  const int n_tile =
-      !active ? 0 : (c == l - 1 ? (kFirstTile ? min(n_tile_full, 1) : 0) : n_tile_full);
-  int steps = 0;  // bisection steps that separate the n_tile + 1 possible counts
-  while ((1 << steps) < n_tile + 1) ++steps;
-  const bool do_post = kFirstTile && active && c != l - 1;
-  const bool do_nopp = kFirstTile && active && l == L && c != l - 1;
-  const GroupConsts k = group_consts(g);
-  const double cap = prob.mem_cap_mb;
-  const double G64 = (double)g->grad_accum;
-  const float G32 = (float)g->grad_accum;
-  const double inv_G64 = 1.0 / G64;
-  const float inv_G32 = 1.0f / G32;
-  // Stage costs the caller's search can use at all (MistProblem.stage_cost_incumbent): rows above
-  // it are not looked for.  (The scout pass reads the first estimate, which a few rows gave
-  // before it; the main launch reads the one the scout's seeds gave.)
-  const double cutoff = prob.stage_cost_incumbent == nullptr || prob.sample_size != 1
-                            ? (double)INFINITY
-                            : *prob.stage_cost_incumbent * inv_G64 * (1.0 + kIncumbentSlack);
-  const double pre_saved = g->pre_saved, pre_sas = g->pre_states_and_saved;
-  const double pre_states = g->pre_states;
-  const double post_states = g->post_states, post_fwd_peak = g->post_fwd_peak;
-  const double post_bwd_peak = g->post_bwd_peak, post_output = g->post_output;
-
-  double best_b[MIST_P_TILE], best_p[MIST_P_TILE];
-  int32_t row_b[MIST_P_TILE], row_p[MIST_P_TILE];
-  double best_post = INFINITY, best_pp = INFINITY;
-  int32_t row_post = -1, row_pp = -1;
-  // The minima of a tile are non-decreasing in p and finite on a prefix [0, fin); `top` is the
-  // largest finite one.  A row that does not reach `top` can only fill the first empty slot.
-  int fin_b = 0, fin_p = 0;
-  double top_b = -INFINITY, top_p = -INFINITY;
-  bool dirty = false;  // some slot of this lane differs from its seed
-#pragma unroll
-  for (int j = 0; j < MIST_P_TILE; ++j) {
-    best_b[j] = best_p[j] = INFINITY;
-    row_b[j] = row_p[j] = -1;
-  }
-  if (seed_cost != nullptr && active) {
-    {  // the first slab of the tile's scout workgroups holds their combined minima
-      const double *sc = seed_cost + threadIdx.x;
-      const int32_t *si = seed_index + threadIdx.x;
-#pragma unroll
-      for (int j = 0; j < MIST_P_TILE; ++j) {
-        const int32_t rb = si[j * MIST_LC_TILE], rp = si[(MIST_P_TILE + j) * MIST_LC_TILE];
-        take_min(best_b[j], row_b[j], rb >= 0, sc[j * MIST_LC_TILE], rb);
-        take_min(best_p[j], row_p[j], rp >= 0, sc[(MIST_P_TILE + j) * MIST_LC_TILE], rp);
-      }
-      const int32_t r2 = si[(2 * MIST_P_TILE) * MIST_LC_TILE];
-      const int32_t r3 = si[(2 * MIST_P_TILE + 1) * MIST_LC_TILE];
-      take_min(best_post, row_post, r2 >= 0, sc[(2 * MIST_P_TILE) * MIST_LC_TILE], r2);
-      take_min(best_pp, row_pp, r3 >= 0, sc[(2 * MIST_P_TILE + 1) * MIST_LC_TILE], r3);
-    }
-#pragma unroll
-    for (int j = 0; j < MIST_P_TILE; ++j) {
-      if (row_b[j] >= 0) { fin_b = j + 1; top_b = best_b[j]; }
-      if (row_p[j] >= 0) { fin_p = j + 1; top_p = best_p[j]; }
-    }
-  }
-
-  const double *__restrict__ src = row_terms + g->row_offset * MIST_ROW_TERMS;
-
-  // The tile's pairs are in (l, c) order, so its lanes hold a few consecutive l.  Per stage and
-  // per such l, one wave-wide test tells which ROWS cannot fit any (c, p) of this tile with that
-  // l (after sieve A's loops, below); it needs the group's pre / post terms to be non-negative.
-  const int l_lo = __shfl(l, 0);
-  const int n_active = __popcll((unsigned long long)__ballot(active));
-  const int n_tile_l = __shfl(l, max(n_active - 1, 0)) - l_lo + 1;
-  const bool rows_filtered = n_active > 0 && n_tile_l <= kTileLayerCounts && pre_saved >= 0.0 &&
-                             pre_sas >= 0.0 && pre_states >= 0.0 && post_states >= 0.0 &&
-                             post_output >= 0.0;
-
-  // Sieve A visits pairs class by class (which first / last family member the latency uses is
-  // fixed per class): 0 = 0 < c < l, 1 = c == 0, 2 = c == l.
-  const int pair_class = !active ? 3 : (c == 0 ? 1 : (c == l ? 2 : 0));
-  const uint64_t in_class0 = __ballot(pair_class == 0), in_class1 = __ballot(pair_class == 1);
-  const uint64_t in_class2 = __ballot(pair_class == 2);
-
-  const double lf = (double)l, lm1 = (double)max(l - 1, 0), cf = (double)c;
-  const double l_minus_c = (double)(l - c), l_minus_c_1 = (double)(l - c - 1);
-  const bool c_eq_l = c == l, c_ge_lm1 = c >= l - 1, c_eq_0 = c == 0;
-
-  // get_latencies (:2165-2216): which family member a lane needs is fixed by its (l, c), so the
-  // choice is made once as a column index instead of a per-row select.
-  const int lm2 = max(l - 2, 0);
-  const double n_ck = (double)min(max(c - 1, 0), lm2);
-  const double n_nock = (double)(lm2 - min(max(c - 1, 0), lm2));
-  const int first_col = c_eq_l ? 0 : 1, last_col = c_eq_0 ? 1 : 0;  // *_CK precedes *_NOCK
-  const int post_col = c > 0 ? 0 : 1;
-  lds_pair[threadIdx.x * kPairFields + 2] = n_ck;
-  lds_pair[threadIdx.x * kPairFields + 3] = n_nock;
-  auto div_G = [&](double v) { return kPow2G ? v * inv_G64 : v / G64; };
-  // Group-wide terms the composite objectives add to the base latency (see `examine`): with x, d
-  // the float32-rounded stable / delta latency,
-  //   with_pre  = r (x + pre_fwd + pre_bwd + w1 + w2) + (d + w1d + w2d) / G
-  //   with_post = r (x + post_fwd + [row terms >= 0]) + (d + [row terms >= 0]) / G
-  //   no_pp     = r (x + pre_fwd + pre_bwd + post_fwd + [..] + w1 + w2 + [..]) + (d + w1d + w2d + [..]) / G
-  // so each is at least r x + d / G plus the offset below, up to a few roundings of relative
-  // size 1e-16 (all terms are non-negative).  A row can beat a minimum `t` of such an objective
-  // only if r x + d / G <= t - offset; the offsets are taken 1e-9 short and `t` 1e-9 long, far
-  // more than the roundings and far less than anything that matters for pruning.
-  constexpr double kSlack = 1e-9;
-  const double off_pre =
-      (ratio * (k.pre_fwd + k.pre_bwd + k.w1 + k.w2) + div_G(k.w1d + k.w2d)) * (1.0 - kSlack);
-  const double off_post = ratio * k.post_fwd * (1.0 - kSlack);
-  const double off_pp = (ratio * (k.pre_fwd + k.pre_bwd + k.post_fwd + k.w1 + k.w2) +
-                         div_G(k.w1d + k.w2d)) * (1.0 - kSlack);
-  auto below = [&](double t, double offset) {
-    return fabs(t) == INFINITY ? t : (t - offset) + kSlack * fabs(t);
-  };
-
-  // Memory model of one candidate row for this lane's (l, c) (:2150-2162, 2358-2385, 2755-2786).
-  // `t` may also be the term-wise minimum of a stage: every operation below is monotone in
-  // every term, so the peaks of that pseudo row bound the peaks of each row of the stage from
-  // below.
-  auto lane_memory = [&](const double *__restrict__ t) {
-    LaneMemory mem;
-    const double S_ck = t[MIST_T_S_CK], S_nock = t[MIST_T_S_NOCK];
-    mem.fwd_states = t[MIST_T_FWD_STATES0] + lf * t[MIST_T_PWG] + lm1 * t[MIST_T_PO];
-    mem.bwd_states = t[MIST_T_BWD_STATES0] + lf * t[MIST_T_PWGO];
-    mem.cur_saved = c_eq_l ? (lf - 1.0) * S_ck : cf * S_ck + l_minus_c_1 * S_nock;
-    mem.mod_saved = S_ck * cf + S_nock * l_minus_c;
-    mem.ck_delta = c_ge_lm1 ? t[MIST_T_D_CK] : t[MIST_T_D_NOCK];
-    mem.fwd_pk = t[MIST_T_FWD_PEAK];
-    mem.bwd_pk = t[MIST_T_BWD_PEAK];
-    mem.out = t[MIST_T_OUT];
-    mem.gcb = t[MIST_T_GCB];
-    mem.mf_base = t[MIST_T_MF_BASE];
-    mem.mf_pp = t[MIST_T_MF_PP];
-    return mem;
-  };
-  // Number of feasible p of this tile, in [lo, n_tile], by bisection with the exact test.
-  auto feasible_count = [&](auto feasible, int lo) {
-    int hi = n_tile;
-    for (int it = 0; it < steps; ++it) {
-      const int mid = (lo + hi) >> 1;
-      const bool ok = feasible(p0 + mid);
-      const bool open = lo < hi;
-      lo = (open && ok) ? mid + 1 : lo;
-      hi = (open && !ok) ? mid : hi;
-    }
-    return lo;
-  };
-
-  // Upper bound of that number for the pseudo row of a stage.  The peaks are linear in p up to
-  // rounding, so the first infeasible slot is estimated from the values at the first two slots
-  // and confirmed with the exact test: any slot at which the pseudo row is infeasible bounds the
-  // count (monotonicity); an unconfirmed estimate falls back to the whole tile.
-  auto count_bound = [&](auto scaled) {
-    const double m0 = scaled(p0);
-    if (!(m0 <= cap)) return 0;
-    if (n_tile <= 1) return n_tile;
-    const float slope = (float)(scaled(p0 + 1) - m0);
-    if (!(slope > 0.0f)) return n_tile;
-    const float est = fminf((float)(cap - m0) * __frcp_rn(slope), (float)n_tile);
-    const int guess = (int)est + 1;  // slots 0 .. floor(est) are expected to be feasible
-    if (guess >= n_tile) return n_tile;
-    if (!(scaled(p0 + guess) <= cap)) return guess;
-    if (guess + 1 < n_tile && !(scaled(p0 + guess + 1) <= cap)) return guess + 1;
-    return n_tile;
-  };
-
-  // Stable / delta latency rounded to float32 (:2212-2213), the base objective r * x + y in
-  // float64 (pareto.py:138; y = float32 array / python int, :2815) and a lower bound of the three
-  // composite objectives: they add non-negative terms to x and d before the same monotone
-  // operations, so none of them can be below it.
-  auto objective = [&](const double *__restrict__ t, double &x, double &d, double &cost_base,
-                       double &bound) {
-    const double stable = n_ck * t[MIST_T_S_LAYER_CK] + n_nock * t[MIST_T_S_LAYER_NOCK] +
-                          t[MIST_T_S_FIRST_CK + first_col] + t[MIST_T_S_LAST_CK + last_col];
-    const double delta = n_ck * t[MIST_T_D_LAYER_CK] + n_nock * t[MIST_T_D_LAYER_NOCK] +
-                         t[MIST_T_D_FIRST_CK + first_col] + t[MIST_T_D_LAST_CK + last_col];
-    const float x32 = (float)stable, d32 = (float)delta;
-    x = (double)x32;
-    d = (double)d32;
-    const float y32 = kPow2G ? d32 * inv_G32 : d32 / G32;
-    const double rx = ratio * x;
-    cost_base = rx + (double)y32;
-    bound = rx + div_G(d);
-  };
-
-  // Sieves B (kCommit == false: would the row change anything, judged against the current
-  // minima) and C (kCommit == true: apply it).  Returns whether the row survives / changed a slot.
-  auto examine = [&](const double *__restrict__ t, int64_t pos, auto commit_tag) -> bool {
-    constexpr bool kCommit = decltype(commit_tag)::value;
-    double x, d, cost_base, bound;
-    objective(t, x, d, cost_base, bound);
-    const bool cand_b = (cost_base <= top_b || fin_b < n_tile) && cost_base <= cutoff;
-    const bool want_pre = (bound <= top_p || fin_p < n_tile) && bound <= cutoff;
-    const bool want_post = do_post && bound <= fmin(best_post, cutoff);
-    const bool want_pp = do_nopp && bound <= fmin(best_pp, cutoff);
-    if (!(cand_b || want_pre || want_post || want_pp)) return false;
-
-    double cost_pre = INFINITY, cost_post = INFINITY, cost_pp = INFINITY;
-    if (want_pre)
-      cost_pre = ratio * (x + k.pre_fwd + k.pre_bwd + k.w1 + k.w2) + div_G(d + k.w1d + k.w2d);
-    if (want_post || want_pp) {
-      const double nag = t[MIST_T_NAG_CK + post_col], nrs = t[MIST_T_NRS_CK + post_col];
-      const double ps1 = k.pp_wre ? nag : 0.0, ps2 = k.pp_gre ? nrs : 0.0;
-      const double pd1 = k.pp_wre ? 0.0 : nag, pd2 = k.pp_gre ? 0.0 : nrs;
-      const double opb = t[MIST_T_OPB];
-      cost_post = ratio * (x + k.post_fwd + opb + ps1 + ps2) + div_G(d + pd1 + pd2);
-      cost_pp = ratio * (x + k.pre_fwd + k.pre_bwd + k.post_fwd + opb + k.w1 + k.w2 + ps1 + ps2) +
-                div_G(d + k.w1d + k.w2d + pd1 + pd2);
-    }
-
-    // Lowest slot the row could change: the minima are non-decreasing in p, so it is the number
-    // of slots whose minimum is strictly below the row's value (empty slots hold +inf; a tie is
-    // decided by the row index when the slot is updated).
-    int lo_b = fin_b, lo_p = fin_p;
-    if (cost_base <= top_b) {
-      lo_b = 0;
-#pragma unroll
-      for (int j = 0; j < MIST_P_TILE; ++j) lo_b += best_b[j] < cost_base ? 1 : 0;
-    }
-    if (cost_pre <= top_p) {
-      lo_p = 0;
-#pragma unroll
-      for (int j = 0; j < MIST_P_TILE; ++j) lo_p += best_p[j] < cost_pre ? 1 : 0;
-    }
-    bool need_b = cand_b && lo_b < n_tile, need_p = want_pre && lo_p < n_tile && cost_pre <= cutoff;
-    bool need_post = want_post && cost_post <= fmin(best_post, cutoff);
-    bool need_pp = want_pp && cost_pp <= fmin(best_pp, cutoff);
-    if (!(need_b || need_p || need_post || need_pp)) return false;
-
-    const LaneMemory mem = lane_memory(t);
-    auto feasible_base = [&](int p) { return mem.feasible_base(p, cap); };
-    auto feasible_pre = [&](int p) { return mem.feasible_pre(p, cap, pre_saved, pre_sas); };
-
-    need_b = need_b && feasible_base(p0 + lo_b);
-    need_p = need_p && feasible_pre(p0 + lo_p);
-    bool ok_pp = false;
-    if (need_post || need_pp) {
-      // ---- last stage / single stage, p == 0 only (:2946-3106) ----
-      double peak_f, peak_b;
-      mem.peaks(0, peak_f, peak_b);
-      const double f_in = mem.fwd_states + post_states + mem.mod_saved + post_fwd_peak + mem.gcb;
-      const double b_in = mem.bwd_states + post_states + mem.mod_saved + post_bwd_peak +
-                          (c_eq_0 ? t[MIST_T_RD] : 0.0) + mem.gcb;
-      const double pf_post = fmax(f_in, peak_f + post_states);
-      const double pb_post = fmax(b_in, peak_b - mem.out + post_states) + post_output;
-      const bool ok_post = fmax(pf_post, pb_post) * mem.mf_pp <= cap;
-      if (need_pp) {
-        const double pf_pp = pf_post + pre_states + pre_saved;
-        const double pb_pp = pb_post + pre_states + pre_saved;
-        ok_pp = fmax(pf_pp, pb_pp) * t[MIST_T_MF] <= cap;
-      }
-      need_post = need_post && ok_post;
-      need_pp = need_pp && ok_pp;
-    }
-    if (!kCommit) return need_b || need_p || need_post || need_pp;
-
-    const int32_t row = row_of_position(g, pos);
-    bool changed = false;
-    if (need_b) {
-      const double cost = cost_base;
-      const int lo = feasible_count(feasible_base, lo_b + 1);  // slot lo_b is known feasible
-#pragma unroll
-      for (int j = 0; j < MIST_P_TILE; ++j) {
-        const bool better = j >= lo_b && j < lo && lex_less(cost, row, best_b[j], row_b[j]);
-        best_b[j] = better ? cost : best_b[j];
-        row_b[j] = better ? row : row_b[j];
-        changed |= better;
-      }
-      // Bookkeeping of (fin, top) without indexing the register array dynamically.
-      if (lo > fin_b) { fin_b = lo; top_b = cost; }
-      else if (lo == fin_b) top_b = fmin(top_b, cost);
-    }
-    if (need_p) {
-      const double cost = cost_pre;
-      const int lo = feasible_count(feasible_pre, lo_p + 1);
-#pragma unroll
-      for (int j = 0; j < MIST_P_TILE; ++j) {
-        const bool better = j >= lo_p && j < lo && lex_less(cost, row, best_p[j], row_p[j]);
-        best_p[j] = better ? cost : best_p[j];
-        row_p[j] = better ? row : row_p[j];
-        changed |= better;
-      }
-      if (lo > fin_p) { fin_p = lo; top_p = cost; }
-      else if (lo == fin_p) top_p = fmin(top_p, cost);
-    }
-    if (need_post) {
-      changed |= lex_less(cost_post, row, best_post, row_post);
-      take_min(best_post, row_post, true, cost_post, row);
-    }
-    if (need_pp) {
-      changed |= lex_less(cost_pp, row, best_pp, row_pp);
-      take_min(best_pp, row_pp, true, cost_pp, row);
-    }
-    return changed;
-  };
-
-  // Stages this workgroup visits: every stage_step-th one of its range, without those the scout
-  // pass has done.  (skip_stride > 1 goes with stage_step == 1: two skips are never adjacent.)
-  const bool gathered = range.gathered != 0;
-  const int64_t n_gather = (int64_t)g->n_par * g->n_oo * g->n_ao * max(g->scout_stride, 1);
-  const int64_t end_stage =
-      ((gathered ? n_gather : range.row_end) + kStageRows - 1) / kStageRows;
-  auto skipped = [&](int64_t st) { return range.skip_stride > 0 && st % range.skip_stride == 0; };
-  auto after = [&](int64_t st) {
-    st += range.stage_step;
-    return skipped(st) ? st + range.stage_step : st;
-  };
-  // The summary of a stage (term-wise minima of its rows, written with the row terms) is one
-  // 32-lane load; the next stage's is in flight while the current stage is processed.
-  // (Gathered rows have no summary: zero is a lower bound of every term, +inf an upper bound of
-  // the output term.)
-  auto load_floor = [&](int64_t st) {
-    if (gathered) return (int)threadIdx.x == kStageMaxOut ? (double)INFINITY : 0.0;
-    return threadIdx.x < kStageFloorPitch ? stage_floor[st * kStageFloorPitch + threadIdx.x] : 0.0;
-  };
-  int64_t stage = range.row_begin / kStageRows;
-  if (skipped(stage)) stage += range.stage_step;
-  double floor_v = stage < end_stage ? load_floor(stage) : 0.0;
-  for (; stage < end_stage; stage = after(stage)) {
-    const int64_t base = stage * kStageRows;
-    const int n_stage =
-        (int)min((int64_t)kStageRows, (gathered ? n_gather : range.row_end) - base);
-    __syncthreads();
-    // workspace position of row r of the stage
-    lds_rowpos[threadIdx.x] =
-        (int32_t)(gathered ? gathered_position(g, min(base + threadIdx.x, n_gather - 1))
-                           : base + threadIdx.x);
-    if (threadIdx.x < kStageFloorPitch) lds_min[threadIdx.x] = floor_v;
-    if (after(stage) < end_stage) floor_v = load_floor(after(stage));
-    __syncthreads();
-
-    // ---- the pseudo row (term-wise minimum of the stage) against the loosest thresholds, the
-    // largest minimum of each objective: the thresholds below are no larger, so a stage that
-    // no lane passes here is closed, and its memory bounds need not be formed ----
-    double floor_x, floor_d, floor_cost, floor_bound;
-    objective(lds_min, floor_x, floor_d, floor_cost, floor_bound);
-    // What the last-stage / single-stage objectives add to every row of this stage on top of
-    // their group-wide offsets: at least the stage's smallest post-layer terms (same slack).
-    const double nag_min = lds_min[kStageMinNag], nrs_min = lds_min[kStageMinNrs];
-    const double stage_post =
-        (ratio * (lds_min[kStageMinOpb] + (k.pp_wre ? nag_min : 0.0) + (k.pp_gre ? nrs_min : 0.0)) +
-         div_G((k.pp_wre ? 0.0 : nag_min) + (k.pp_gre ? 0.0 : nrs_min))) * (1.0 - kSlack);
-    {
-      const double loose_b = fmin(fin_b < n_tile ? (double)INFINITY : top_b, cutoff);
-      const double loose_p = fmin(fin_p < n_tile ? (double)INFINITY : top_p, cutoff);
-      double loose_o = below(loose_p, off_pre);
-      if (do_post) loose_o = fmax(loose_o, below(fmin(best_post, cutoff), off_post + stage_post));
-      if (do_nopp) loose_o = fmax(loose_o, below(fmin(best_pp, cutoff), off_pp + stage_post));
-      if (!__any(active && (floor_cost <= loose_b || floor_bound <= loose_o))) continue;
-    }
-
-    // ---- per-stage thresholds: no row of the stage is feasible beyond the pseudo row's count,
-    // so only the minima of the slots below it can be beaten ----
-    const LaneMemory floor_mem = lane_memory(lds_min);
-    const int cnt_b = count_bound([&](int p) { return floor_mem.scaled_base(p); });
-    const int cnt_p =
-        count_bound([&](int p) { return floor_mem.scaled_pre(p, pre_saved, pre_sas); });
-    double thr_b = -INFINITY, thr_p = -INFINITY;
-#pragma unroll
-    for (int j = 0; j < MIST_P_TILE; ++j) {  // minima are non-decreasing; empty slots hold +inf
-      thr_b = j < cnt_b ? best_b[j] : thr_b;
-      thr_p = j < cnt_p ? best_p[j] : thr_p;
-    }
-    thr_b = fmin(thr_b, cutoff);
-    thr_p = fmin(thr_p, cutoff);
-    // One threshold for the three composite objectives, expressed for `bound` (objective()):
-    // each of them exceeds `bound` by at least its group-wide offset.
-    double thr_o = below(thr_p, off_pre);
-    if (do_post) {
-      // Lower bounds of the last-stage / single-stage peaks (:2946-3106) from the pseudo row.
-      double peak_f, peak_b;
-      floor_mem.peaks(0, peak_f, peak_b);
-      const double f_in =
-          floor_mem.fwd_states + post_states + floor_mem.mod_saved + post_fwd_peak + floor_mem.gcb;
-      const double b_in =
-          floor_mem.bwd_states + post_states + floor_mem.mod_saved + post_bwd_peak + floor_mem.gcb;
-      const double pf_post = fmax(f_in, peak_f + post_states);
-      const double pb_post = fmax(b_in, peak_b - lds_min[kStageMaxOut] + post_states) + post_output;
-      if (fmax(pf_post, pb_post) * floor_mem.mf_pp <= cap)
-        thr_o = fmax(thr_o, below(fmin(best_post, cutoff), off_post + stage_post));
-      if (do_nopp) {
-        const double pf_pp = pf_post + pre_states + pre_saved;
-        const double pb_pp = pb_post + pre_states + pre_saved;
-        if (fmax(pf_pp, pb_pp) * lds_min[MIST_T_MF] <= cap)
-          thr_o = fmax(thr_o, below(fmin(best_pp, cutoff), off_pp + stage_post));
-      }
-    }
-
-    // ---- sieve A: the rows of the stage against those thresholds.  First the pseudo row of
-    // term-wise minima: the objective is monotone in every term, so a pair the pseudo row does
-    // not pass is passed by no row of the stage (two thirds of all stages end here).  For the
-    // other pairs the test runs transposed: a lane holds the latency terms of ONE ROW in
-    // registers and the loop runs over those pairs, whose constants and thresholds are
-    // wave-uniform reads of the per-pair table.  The wave-wide comparison result is exactly the
-    // 64-row survivor mask of that pair; it is handed to the pair's lane. ----
-    uint64_t sieve = 0;
-    uint64_t pairs_open;
-    pairs_open = __ballot(active && (floor_cost <= thr_b || floor_bound <= thr_o));
-    if (pairs_open != 0) {
-      lds_pair[threadIdx.x * kPairFields + 0] = thr_b;
-      lds_pair[threadIdx.x * kPairFields + 1] = thr_o;
-      if (!gathered) {  // 16-byte loads: a row is 17 such pairs and starts 16-byte aligned
-        const double2 *__restrict__ src2 =
-            reinterpret_cast<const double2 *>(src + base * MIST_ROW_TERMS);
-        for (int i = threadIdx.x; i < n_stage * (MIST_ROW_TERMS / 2); i += MIST_LC_TILE) {
-          const double2 v = src2[i];
-          const int at =
-              (i / (MIST_ROW_TERMS / 2)) * kLdsRowStride + 2 * (i % (MIST_ROW_TERMS / 2));
-          lds_terms[at] = v.x;
-          lds_terms[at + 1] = v.y;
-        }
-      } else {  // the same, row by row from the gathered positions
-        const double2 *__restrict__ src2 = reinterpret_cast<const double2 *>(src);
-        for (int i = threadIdx.x; i < n_stage * (MIST_ROW_TERMS / 2); i += MIST_LC_TILE) {
-          const int r = i / (MIST_ROW_TERMS / 2), c2 = i % (MIST_ROW_TERMS / 2);
-          const double2 v = src2[(int64_t)lds_rowpos[r] * (MIST_ROW_TERMS / 2) + c2];
-          lds_terms[r * kLdsRowStride + 2 * c2] = v.x;
-          lds_terms[r * kLdsRowStride + 2 * c2 + 1] = v.y;
-        }
-      }
-      __syncthreads();
-      double rt[MIST_T_D_LAST_NOCK + 1];
-#pragma unroll
-      for (int i = 0; i <= MIST_T_D_LAST_NOCK; ++i)
-        rt[i] = lds_terms[threadIdx.x * kLdsRowStride + i];  // stale beyond n_stage, masked below
-      __syncthreads();
-      const uint64_t valid_rows = n_stage < kStageRows ? (1ull << n_stage) - 1ull : ~0ull;
-      auto sieve_class = [&](uint64_t todo, auto first_col_tag, auto last_col_tag) {
-        constexpr int kFirstCol = decltype(first_col_tag)::value;
-        constexpr int kLastCol = decltype(last_col_tag)::value;
-        const double s_first = rt[MIST_T_S_FIRST_CK + kFirstCol];
-        const double s_last = rt[MIST_T_S_LAST_CK + kLastCol];
-        const double d_first = rt[MIST_T_D_FIRST_CK + kFirstCol];
-        const double d_last = rt[MIST_T_D_LAST_CK + kLastCol];
-        while (todo != 0) {
-          const int pair_lane = __ffsll((unsigned long long)todo) - 1;
-          todo &= todo - 1;
-          const double pair_thr_b = lds_pair[pair_lane * kPairFields + 0];
-          const double pair_thr_o = lds_pair[pair_lane * kPairFields + 1];
-          const double pair_n_ck = lds_pair[pair_lane * kPairFields + 2];
-          const double pair_n_nock = lds_pair[pair_lane * kPairFields + 3];
-          const double stable = pair_n_ck * rt[MIST_T_S_LAYER_CK] +
-                                pair_n_nock * rt[MIST_T_S_LAYER_NOCK] + s_first + s_last;
-          const double delta = pair_n_ck * rt[MIST_T_D_LAYER_CK] +
-                               pair_n_nock * rt[MIST_T_D_LAYER_NOCK] + d_first + d_last;
-          const float x32 = (float)stable, d32 = (float)delta;
-          const float y32 = kPow2G ? d32 * inv_G32 : d32 / G32;
-          const double rx = ratio * (double)x32;
-          const double cost_base = rx + (double)y32;
-          const double bound = rx + div_G((double)d32);
-          const uint64_t survivors =
-              __ballot(cost_base <= pair_thr_b || bound <= pair_thr_o) & valid_rows;
-          sieve = (int)threadIdx.x == pair_lane ? survivors : sieve;
-        }
-      };
-      sieve_class(pairs_open & in_class0, std::integral_constant<int, 1>{},
-                  std::integral_constant<int, 0>{});
-      sieve_class(pairs_open & in_class1, std::integral_constant<int, 1>{},
-                  std::integral_constant<int, 1>{});
-      sieve_class(pairs_open & in_class2, std::integral_constant<int, 0>{},
-                  std::integral_constant<int, 0>{});
-      // Rows that exceed the capacity with tile_l layers whatever c, p and variant: every
-      // variant's tested quantity is at least
-      //   max(fwd, bwd) * (smallest of the row's three memory factors),
-      //   fwd = fwd_states + (l - 1) min(S_ck, S_nock) + min(D_ck, D_nock) + fwd_peak + gcb
-      //         + p0 (l min(S_ck, S_nock) + 2 out),   bwd likewise with out counted once
-      // (cur_saved and mod_saved are sums of l - 1 and l saved terms; the last-stage variants
-      // take one output off the backward peak; pre / post terms only add).  The bound is taken
-      // 1e-9 short, far more than the roundings of the two evaluation orders.
-      if (rows_filtered && __any(sieve != 0)) {
-        uint64_t fits = ~0ull;
-        const double *mine = lds_terms + threadIdx.x * kLdsRowStride;
-        const double s_min = fmin(mine[MIST_T_S_CK], mine[MIST_T_S_NOCK]);
-        const double d_min = fmin(mine[MIST_T_D_CK], mine[MIST_T_D_NOCK]);
-        const double out = mine[MIST_T_OUT], gcb = mine[MIST_T_GCB];
-        const double mf_min =
-            fmin(fmin(mine[MIST_T_MF_BASE], mine[MIST_T_MF_PP]), mine[MIST_T_MF]);
-        const double fwd0 = mine[MIST_T_FWD_STATES0] + d_min + mine[MIST_T_FWD_PEAK] + gcb;
-        const double bwd0 = mine[MIST_T_BWD_STATES0] + d_min + mine[MIST_T_BWD_PEAK] + out + gcb;
-        const double pwg = mine[MIST_T_PWG], po = mine[MIST_T_PO], pwgo = mine[MIST_T_PWGO];
-#pragma unroll 1
-        for (int i = 0; i < n_tile_l; ++i) {
-          const double tl = (double)(l_lo + i), tl1 = (double)max(l_lo + i - 1, 0);
-          const double per_p = tl * s_min + 2.0 * out;
-          const double shared = tl1 * s_min + (double)p0 * per_p;
-          const double low = fmax(fwd0 + tl * pwg + tl1 * po + shared, bwd0 + tl * pwgo + shared);
-          const bool too_big = s_min >= 0.0 && out >= 0.0 && low >= 0.0 && mf_min >= 0.0 &&
-                               low * mf_min * (1.0 - 1e-9) > cap;
-          fits = l - l_lo == i ? ~__ballot(too_big) : fits;
-        }
-        sieve &= fits;
-      }
-    }
-
-    // ---- sieve B: lowest improvable slot and the memory test there, per-lane survivors.  It
-    // pays when it rejects most rows (the main pass: 96 %); the scout pass starts from empty
-    // minima and most of what reaches it also changes a slot, so there C takes the rows as they
-    // come (C repeats every test of B). ----
-    uint64_t keep = 0;
-    if (gathered) {
-      keep = sieve;
-      sieve = 0;
-    }
-    while (sieve != 0) {
-      const int r = __ffsll((unsigned long long)sieve) - 1;
-      sieve &= sieve - 1;
-      const bool hit = examine(lds_terms + r * kLdsRowStride, lds_rowpos[r], std::false_type{});
-      keep |= (uint64_t)(hit ? 1 : 0) << r;
-    }
-
-    // ---- sieve C: survivors in row order against the live minima ----
-    while (keep != 0) {
-      const int r = __ffsll((unsigned long long)keep) - 1;
-      keep &= keep - 1;
-      dirty |= examine(lds_terms + r * kLdsRowStride, lds_rowpos[r], std::true_type{});
-    }
-  }
-
-  // A chunk that changed no slot holds exactly its seeds, which the first chunk of the tile
-  // writes out anyway: it leaves a mark instead of its 26 KB slab, and the combining kernel
-  // skips it.
-  if (skip_unchanged && !__any(dirty)) {
-    if (threadIdx.x == 0) out_index[0] = kSlabUnchanged;
-    return;
-  }
-
-#pragma unroll
-  for (int j = 0; j < MIST_P_TILE; ++j) {
-    out_cost[j * MIST_LC_TILE + threadIdx.x] = best_b[j];
-    out_index[j * MIST_LC_TILE + threadIdx.x] = row_b[j];
-    out_cost[(MIST_P_TILE + j) * MIST_LC_TILE + threadIdx.x] = best_p[j];
-    out_index[(MIST_P_TILE + j) * MIST_LC_TILE + threadIdx.x] = row_p[j];
-  }
-  out_cost[(2 * MIST_P_TILE) * MIST_LC_TILE + threadIdx.x] = best_post;
-  out_index[(2 * MIST_P_TILE) * MIST_LC_TILE + threadIdx.x] = row_post;
-  out_cost[(2 * MIST_P_TILE + 1) * MIST_LC_TILE + threadIdx.x] = best_pp;
-  out_index[(2 * MIST_P_TILE + 1) * MIST_LC_TILE + threadIdx.x] = row_pp;
+__device__ __forceinline__ double from_lane(double v, int lane) {
+  const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+  const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)u, lane);
+  const uint32_t hi = __builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), lane);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+__device__ __forceinline__ int from_lane(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
+__device__ __forceinline__ float from_lane(float v, int lane) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+__device__ __forceinline__ uint64_t from_lane(uint64_t v, int lane) {
+  const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)v, lane);
+  const uint32_t hi = __builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), lane);
+  return ((uint64_t)hi << 32) | lo;
+}
+// Smallest of the wavefront's values, in every lane (rows of 16 lanes, then across the rows).
+__device__ __forceinline__ uint32_t wave_min(uint32_t v) {
+#define MIST_MIN_DPP(CTRL) \
+  v = min(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, 0xf, 0xf, false))
+  MIST_MIN_DPP(0x111);  // row_shr:1
+  MIST_MIN_DPP(0x112);
+  MIST_MIN_DPP(0x114);
+  MIST_MIN_DPP(0x118);
+  MIST_MIN_DPP(0x142);  // row_bcast:15
+  MIST_MIN_DPP(0x143);  // row_bcast:31
+#undef MIST_MIN_DPP
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+// A lane with `pending` whose cost is the smallest to float32 (costs are not negative).
+__device__ __forceinline__ int cheapest_lane(bool pending, double cost) {
+  const uint32_t key = pending ? __float_as_uint((float)cost) : ~0u;
+  return __ffsll((unsigned long long)__ballot(key == wave_min(key))) - 1;
+}
+__device__ __forceinline__ double cost_of_bits(unsigned long long bits) {
+  return __longlong_as_double((long long)bits);
 }
 
-// scout != 0: kScoutSplit workgroups per (group, (l, c) tile, p tile) share the gathered rows
-// of the whole group, results in slab n_blocks + logical workgroup.
-// scout == 0: one workgroup per row chunk of such a tile, seeded from the scout's slabs when the
-// group has them.
-__global__ __launch_bounds__(MIST_LC_TILE, MIST_REDUCE_MIN_WAVES) void eval_reduce_kernel(
+// Slots of a pair in ReduceTables: base p = 0.., with_pre p = 0.., with_post, no_pp.
+__host__ __device__ constexpr int slots_of(int num_p) { return 2 * num_p + 2; }
+
+// What is the same for all rows of one (l, c) pair; l and c may be wave-uniform or per lane.
+struct PairConsts {
+  double n_ck, n_nock, lf, lm1, cf, l_minus_c, l_minus_c_1;
+  bool all_ck, no_ck, ck_tail;
+};
+__device__ __forceinline__ PairConsts pair_consts(int l, int c) {
+  PairConsts k;
+  const int lm2 = max(l - 2, 0), n_ck = min(max(c - 1, 0), lm2);
+  k.n_ck = (double)n_ck;
+  k.n_nock = (double)(lm2 - n_ck);
+  k.lf = (double)l;
+  k.lm1 = (double)max(l - 1, 0);
+  k.cf = (double)c;
+  k.l_minus_c = (double)(l - c);
+  k.l_minus_c_1 = (double)(l - c - 1);
+  k.all_ck = c == l;
+  k.no_ck = c == 0;
+  k.ck_tail = c >= l - 1;
+  return k;
+}
+
+// Stable / delta latency rounded to float32 (get_latencies, :2165-2216).
+template <class Row>
+__device__ __forceinline__ void pair_latency(const Row &t, const PairConsts &k, float &x, float &d) {
+  const double stable = k.n_ck * t[MIST_T_S_LAYER_CK] + k.n_nock * t[MIST_T_S_LAYER_NOCK] +
+                        (k.all_ck ? t[MIST_T_S_FIRST_CK] : t[MIST_T_S_FIRST_NOCK]) +
+                        (k.no_ck ? t[MIST_T_S_LAST_NOCK] : t[MIST_T_S_LAST_CK]);
+  const double delta = k.n_ck * t[MIST_T_D_LAYER_CK] + k.n_nock * t[MIST_T_D_LAYER_NOCK] +
+                       (k.all_ck ? t[MIST_T_D_FIRST_CK] : t[MIST_T_D_FIRST_NOCK]) +
+                       (k.no_ck ? t[MIST_T_D_LAST_NOCK] : t[MIST_T_D_LAST_CK]);
+  x = (float)stable;
+  d = (float)delta;
+}
+
+// Memory model (:2150-2162, 2358-2385, 2755-2786).  `t` may also be the term-wise minimum of a
+// stage: every operation is monotone in every term, so the peaks of that pseudo row bound the
+// peaks of each row of the stage from below.
+template <class Row>
+__device__ __forceinline__ LaneMemory pair_memory(const Row &t, const PairConsts &k) {
+  LaneMemory mem;
+  const double S_ck = t[MIST_T_S_CK], S_nock = t[MIST_T_S_NOCK];
+  mem.fwd_states = t[MIST_T_FWD_STATES0] + k.lf * t[MIST_T_PWG] + k.lm1 * t[MIST_T_PO];
+  mem.bwd_states = t[MIST_T_BWD_STATES0] + k.lf * t[MIST_T_PWGO];
+  mem.cur_saved = k.all_ck ? (k.lf - 1.0) * S_ck : k.cf * S_ck + k.l_minus_c_1 * S_nock;
+  mem.mod_saved = S_ck * k.cf + S_nock * k.l_minus_c;
+  mem.ck_delta = k.ck_tail ? t[MIST_T_D_CK] : t[MIST_T_D_NOCK];
+  mem.fwd_pk = t[MIST_T_FWD_PEAK];
+  mem.bwd_pk = t[MIST_T_BWD_PEAK];
+  mem.out = t[MIST_T_OUT];
+  mem.gcb = t[MIST_T_GCB];
+  mem.mf_base = t[MIST_T_MF_BASE];
+  mem.mf_pp = t[MIST_T_MF_PP];
+  return mem;
+}
+
+// Upper bound of the number of feasible p in [0, n]: the scaled peaks are linear in p up to
+// rounding, so the first infeasible p is estimated from the first two and confirmed with the
+// exact test: any p at which the row is infeasible bounds the count (monotonicity); an
+// unconfirmed estimate falls back to n.
+template <class Scaled>
+__device__ __forceinline__ int count_bound(const Scaled &scaled, int n, double cap) {
+  const double m0 = scaled(0);
+  if (n <= 0 || !(m0 <= cap)) return 0;
+  if (n == 1) return 1;
+  const float slope = (float)(scaled(1) - m0);
+  if (!(slope > 0.0f)) return n;
+  const float est = fminf((float)(cap - m0) * __frcp_rn(slope), (float)n);
+  const int guess = (int)est + 1;  // 0 .. floor(est) are expected to be feasible
+  if (guess >= n) return n;
+  if (!(scaled(guess) <= cap)) return guess;
+  if (guess + 1 < n && !(scaled(guess + 1) <= cap)) return guess + 1;
+  return n;
+}
+// The number itself: from the bound down to the last p the exact test admits.
+template <class Scaled>
+__device__ __forceinline__ int count_exact(const Scaled &scaled, int n, double cap) {
+  int count = count_bound(scaled, n, cap);
+  while (count > 0 && !(scaled(count - 1) <= cap)) --count;
+  return count;
+}
+
+// Constants of a group, of one sample.
+struct GroupModel {
+  GroupConsts k;
+  double cap, G64, inv_G64;
+  float G32, inv_G32;
+  double pre_saved, pre_sas, pre_states, post_states, post_fwd_peak, post_bwd_peak, post_output;
+  bool pow2;  // x / G == x * (1 / G) bit for bit, and the division leaves the inner loop
+
+  __device__ __forceinline__ double div_G(double v) const { return pow2 ? v * inv_G64 : v / G64; }
+  __device__ __forceinline__ float div_G(float v) const { return pow2 ? v * inv_G32 : v / G32; }
+};
+__device__ __forceinline__ GroupModel group_model(const MistProblem &prob, const MistGroupDesc *g) {
+  GroupModel m;
+  m.k = group_consts(g);
+  m.cap = prob.mem_cap_mb;
+  m.G64 = (double)g->grad_accum;
+  m.G32 = (float)g->grad_accum;
+  m.inv_G64 = 1.0 / m.G64;
+  m.inv_G32 = 1.0f / m.G32;
+  m.pre_saved = g->pre_saved;
+  m.pre_sas = g->pre_states_and_saved;
+  m.pre_states = g->pre_states;
+  m.post_states = g->post_states;
+  m.post_fwd_peak = g->post_fwd_peak;
+  m.post_bwd_peak = g->post_bwd_peak;
+  m.post_output = g->post_output;
+  m.pow2 = (g->grad_accum & (g->grad_accum - 1)) == 0;
+  return m;
+}
+
+// Stage costs the caller's search can use at all (MistProblem.stage_cost_incumbent): rows above
+// it are not looked for.  (The seed launch reads the first estimate, which a few rows gave
+// before it; the later launches read the one the seeds gave.)
+__device__ __forceinline__ double stage_cost_cutoff(const MistProblem &prob, double inv_G64) {
+  return prob.stage_cost_incumbent == nullptr || prob.sample_size != 1
+             ? (double)INFINITY
+             : *prob.stage_cost_incumbent * inv_G64 * (1.0 + kIncumbentSlack);
+}
+
+// Group-wide terms the composite objectives add to the base latency: with x, d the
+// float32-rounded stable / delta latency,
+//   with_pre  = r (x + pre_fwd + pre_bwd + w1 + w2) + (d + w1d + w2d) / G
+//   with_post = r (x + post_fwd + [row terms >= 0]) + (d + [row terms >= 0]) / G
+//   no_pp     = r (x + pre_fwd + pre_bwd + post_fwd + [..] + w1 + w2 + [..]) + (d + w1d + w2d + [..]) / G
+// so each is at least `bound` = r x + d / G plus the offset below, up to a few roundings of
+// relative size 1e-16 (all terms are non-negative).  A row can beat a minimum `t` of such an
+// objective only if its bound <= t - offset; the offsets are taken 1e-9 short and `t` 1e-9 long, far
+// more than the roundings and far less than anything that matters for pruning.  The row terms of
+// the last two have their own minima over a stage (MIST_T_OPB, the NAG and NRS pairs).
+struct Offsets {
+  double pre, post, pp;
+};
+__device__ __forceinline__ Offsets composite_offsets(const GroupModel &m, double ratio, double opb_min,
+                                                     double nag_min, double nrs_min) {
+  const GroupConsts &k = m.k;
+  const double shared = m.div_G(k.w1d + k.w2d);
+  const double stage_post =
+      (ratio * (opb_min + (k.pp_wre ? nag_min : 0.0) + (k.pp_gre ? nrs_min : 0.0)) +
+       m.div_G((k.pp_wre ? 0.0 : nag_min) + (k.pp_gre ? 0.0 : nrs_min))) * (1.0 - kSlack);
+  Offsets o;
+  o.pre = (ratio * (k.pre_fwd + k.pre_bwd + k.w1 + k.w2) + shared) * (1.0 - kSlack);
+  o.post = ratio * k.post_fwd * (1.0 - kSlack) + stage_post;
+  o.pp = (ratio * (k.pre_fwd + k.pre_bwd + k.post_fwd + k.w1 + k.w2) + shared) * (1.0 - kSlack) +
+         stage_post;
+  return o;
+}
+__device__ __forceinline__ double below(double t, double offset) {
+  return fabs(t) == INFINITY ? t : (t - offset) + kSlack * fabs(t);
+}
+
+// The last-stage / single-stage memory tests, p == 0 only (:2946-3106); `smallest_out`: what the
+// backward peak may lose (the row's output; for a stage summary its largest).
+template <class Row>
+__device__ __forceinline__ void post_fits(const Row &t, const PairConsts &k, const LaneMemory &mem,
+                                          const GroupModel &m, double out, double rd, bool &post, bool &pp) {
+  double peak_f, peak_b;
+  mem.peaks(0, peak_f, peak_b);
+  const double f_in = mem.fwd_states + m.post_states + mem.mod_saved + m.post_fwd_peak + mem.gcb;
+  const double b_in = mem.bwd_states + m.post_states + mem.mod_saved + m.post_bwd_peak + rd + mem.gcb;
+  const double pf_post = fmax(f_in, peak_f + m.post_states);
+  const double pb_post = fmax(b_in, peak_b - out + m.post_states) + m.post_output;
+  post = fmax(pf_post, pb_post) * mem.mf_pp <= m.cap;
+  const double pf_pp = pf_post + m.pre_states + m.pre_saved;
+  const double pb_pp = pb_post + m.pre_states + m.pre_saved;
+  pp = fmax(pf_pp, pb_pp) * t[MIST_T_MF] <= m.cap;
+}
+
+// The four objectives of one row (pareto.py:138; base with y = float32 delta / G in float32,
+// :2815, the others in float64, :2898-2903, 3002-3007, 3084-3089).
+struct Objectives {
+  double base, pre, post, pp;
+};
+template <class Row>
+__device__ __forceinline__ Objectives objectives(const Row &t, float x32, float d32, bool no_ck, double ratio,
+                                                 const GroupModel &m, bool with_post) {
+  const GroupConsts &k = m.k;
+  const double x = (double)x32, d = (double)d32;
+  Objectives o;
+  o.base = ratio * x + (double)m.div_G(d32);
+  o.pre = ratio * (x + k.pre_fwd + k.pre_bwd + k.w1 + k.w2) + m.div_G(d + k.w1d + k.w2d);
+  o.post = o.pp = INFINITY;
+  if (with_post) {
+    const double nag = no_ck ? t[MIST_T_NAG_NOCK] : t[MIST_T_NAG_CK];
+    const double nrs = no_ck ? t[MIST_T_NRS_NOCK] : t[MIST_T_NRS_CK];
+    const double ps1 = k.pp_wre ? nag : 0.0, ps2 = k.pp_gre ? nrs : 0.0;
+    const double pd1 = k.pp_wre ? 0.0 : nag, pd2 = k.pp_gre ? 0.0 : nrs;
+    const double opb = t[MIST_T_OPB];
+    o.post = ratio * (x + k.post_fwd + opb + ps1 + ps2) + m.div_G(d + pd1 + pd2);
+    o.pp = ratio * (x + k.pre_fwd + k.pre_bwd + k.post_fwd + opb + k.w1 + k.w2 + ps1 + ps2) +
+           m.div_G(d + k.w1d + k.w2d + pd1 + pd2);
+  }
+  return o;
+}
+
+// One candidate row in registers.
+struct RowRegs {
+  double v[MIST_ROW_TERMS];
+  __device__ __forceinline__ double operator[](int i) const { return v[i]; }
+};
+template <int kFrom, int kTo>  // columns, even
+__device__ __forceinline__ void load_terms(RowRegs &r, const double *__restrict__ row) {
+  static_assert(kFrom % 2 == 0 && kTo % 2 == 0, "rows are read as 16-byte pairs");
+  const double2 *__restrict__ src = reinterpret_cast<const double2 *>(row);
+#pragma unroll
+  for (int i = kFrom / 2; i < kTo / 2; ++i) {
+    const double2 v = src[i];
+    r.v[2 * i] = v.x;
+    r.v[2 * i + 1] = v.y;
+  }
+}
+static_assert(MIST_T_S_LAYER_CK == 0 && MIST_T_D_LAST_NOCK == 11 && MIST_T_GCB < 32,
+              "latency terms, then memory terms, are the first columns");
+
+// ---- seeds ----
+__device__ __forceinline__ void clear_queue(const ReduceTables &tabs) {
+  if (blockIdx.x == 0 && blockIdx.y == 0)
+    for (int i = threadIdx.x; i < kCounters; i += blockDim.x) tabs.counter[i * kCounterPitch] = 0;
+}
+
+// One sample.  Workgroup = (`pair_split` consecutive pairs of a tile, group) with their minima in
+// LDS.  A wavefront takes 64 gathered rows, lane = row with all its terms in registers, and runs
+// over the pairs: per (pair, variant) one look-up of the minimum at each row's own count; of the
+// rows below it the cheapest lowers the slots up to its count (lane = slot) and drops the rows it
+// dominates, until none is left - a few steps from empty minima, none later.
+// (One LDS atomic per row at its own count, all rows of a stage at a few addresses: 0.96 ms for
+// the 7B plan; the register minima this replaced, one row after the other per lane: 0.42 ms.)
+__global__ __launch_bounds__(kSeedThreads) void seed_kernel(
+    const MistProblem prob, const MistGroupDesc *__restrict__ groups, const double *__restrict__ row_terms,
+    double ratio, ReduceTables tabs, int pair_split) {
+  extern __shared__ unsigned long long lds_best[];
+  const MistGroupDesc *g = groups + blockIdx.y;
+  const int parts = MIST_LC_TILE / pair_split;
+  const int tile_rel = (int)blockIdx.x / parts, part = (int)blockIdx.x % parts;
+  clear_queue(tabs);
+  if (tile_rel >= g->n_lc_tiles) return;
+  const int L = prob.num_layers, n_pairs = L * (L + 1) / 2 + L;
+  const int P = g->num_p, n_slots = slots_of(P);
+  const int first_pair = (g->lc_tile_begin + tile_rel) * MIST_LC_TILE + part * pair_split;
+  const int n_here = min(pair_split, n_pairs - first_pair);
+  const int n_entries = pair_split * n_slots;  // [pair][slot]
+  const unsigned long long kInf = (unsigned long long)__double_as_longlong((double)INFINITY);
+  for (int e = threadIdx.x; e < n_entries; e += kSeedThreads) lds_best[e] = kInf;
+  __syncthreads();
+  if (g->scout_stride > 0 && n_here > 0) {
+    constexpr int kWaves = kSeedThreads / 64;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const GroupModel m = group_model(prob, g);
+    const double cutoff = stage_cost_cutoff(prob, m.inv_G64);
+    const int n_gather = g->n_par * g->n_oo * g->n_ao * g->scout_stride;
+    const int n_stages = (n_gather + 63) / 64;
+    // units of work: (stage, share of the pairs), more than one share when there are few stages
+    const int shares = max(1, min(n_here, kWaves / n_stages)), per_share = (n_here + shares - 1) / shares;
+    const double *__restrict__ src = row_terms + g->row_offset * MIST_ROW_TERMS;
+    for (int unit = wave; unit < n_stages * shares; unit += kWaves) {
+      const int q = unit / shares * 64 + lane;
+      const int i0 = unit % shares * per_share, i1 = min(i0 + per_share, n_here);
+      const bool live = q < n_gather;
+      RowRegs t;
+      load_terms<0, MIST_ROW_TERMS>(t, src + gathered_position(g, min(q, n_gather - 1)) * MIST_ROW_TERMS);
+      const PairIndex pc = decode_pair(first_pair + min(i0, n_here - 1));
+      int l = __builtin_amdgcn_readfirstlane(pc.l), c = __builtin_amdgcn_readfirstlane(pc.c);
+      for (int i = i0; i < i1; ++i, c = c < l ? c + 1 : (++l, 0)) {
+        const PairConsts k = pair_consts(l, c);
+        // Cells with c == l - 1 are only kept for p == 0 of the base / with_pre variants
+        // (batched_module_analyzer.py:3021-3023, 3103).
+        const int np = c == l - 1 ? min(P, 1) : P;
+        const bool do_post = c != l - 1, do_pp = do_post && l == L;
+        float x, d;
+        pair_latency(t, k, x, d);
+        // (under a bound most rows are above it and need no memory model)
+        const bool wanted =
+            live && (cutoff == INFINITY || ratio * (double)x + m.div_G((double)d) <= cutoff * (1.0 + kBaseSlack));
+        if (!__any(wanted)) continue;
+        const LaneMemory mem = pair_memory(t, k);
+        const int cnt_b = count_exact([&](int p) { return mem.scaled_base(p); }, wanted ? np : 0, m.cap);
+        const int cnt_p =
+            count_exact([&](int p) { return mem.scaled_pre(p, m.pre_saved, m.pre_sas); }, wanted ? np : 0, m.cap);
+        bool ok_post = false, ok_pp = false;
+        if (do_post) post_fits(t, k, mem, m, mem.out, k.no_ck ? t[MIST_T_RD] : 0.0, ok_post, ok_pp);
+        unsigned long long *mine = lds_best + i * n_slots;
+        const Objectives o = objectives(t, x, d, k.no_ck, ratio, m, do_post);
+        auto offer = [&](int count, double cost, unsigned long long *slots) {
+          const unsigned long long bits = (unsigned long long)__double_as_longlong(cost);
+          bool pending = count > 0 && bits < slots[max(count - 1, 0)];
+          while (__any(pending)) {
+            const int r = cheapest_lane(pending, cost);
+            const double its_cost = from_lane(cost, r);
+            const int its_count = from_lane(count, r);
+            for (int j = lane; j < its_count; j += 64)
+              atomicMin(slots + j, (unsigned long long)__double_as_longlong(its_cost));
+            pending = pending && lane != r && (count > its_count || cost < its_cost);
+          }
+        };
+        offer(cnt_b, o.base, mine);
+        offer(cnt_p, o.pre, mine + P);
+        if (do_post) offer(wanted && ok_post ? 1 : 0, o.post, mine + 2 * P);
+        if (do_pp) offer(wanted && ok_pp ? 1 : 0, o.pp, mine + 2 * P + 1);
+      }
+    }
+  }
+  __syncthreads();
+  // (pairs past the last one of the list belong to the tile: they stay empty)
+  const int64_t cell0 = g->cell_offset + ((int64_t)tile_rel * MIST_LC_TILE + part * pair_split) * n_slots;
+  for (int e = threadIdx.x; e < n_entries; e += kSeedThreads) {
+    tabs.best[cell0 + e] = lds_best[e];
+    tabs.row[cell0 + e] = ~0u;
+  }
+  if ((int)threadIdx.x < pair_split) tabs.changed[(cell0 + threadIdx.x * n_slots) / 4] = 0;
+}
+
+// Several samples.  What the objectives of a row are made of, r X + Y per variant, and its counts,
+// for the lane = (row parity, sample) phases: a wavefront reads two rows at a time.
+struct SampleRows {
+  double2 xy[4][64];    // base, with_pre, with_post, no_pp: (X, Y)
+  uint32_t counts[64];  // feasible p: base | with_pre << 15 | with_post << 30 | no_pp << 31
+  uint32_t number[64];  // row number
+};
+static_assert(MIST_MAX_SAMPLE_BATCH <= 32, "half a wavefront per row");
+// Writes row `at` of the buffer.
+__device__ __forceinline__ void put_sample_row(SampleRows *rows, int at, const RowRegs &t, float x32, float d32, bool no_ck,
+                                               const GroupModel &m, int count_b, int count_p, bool post, bool pp,
+                                               bool do_post) {
+  const GroupConsts &k = m.k;
+  const double x = (double)x32, d = (double)d32;
+  rows->xy[0][at] = double2{x, (double)m.div_G(d32)};
+  rows->xy[1][at] = double2{x + k.pre_fwd + k.pre_bwd + k.w1 + k.w2, m.div_G(d + k.w1d + k.w2d)};
+  if (do_post) {
+    const double nag = no_ck ? t[MIST_T_NAG_NOCK] : t[MIST_T_NAG_CK];
+    const double nrs = no_ck ? t[MIST_T_NRS_NOCK] : t[MIST_T_NRS_CK];
+    const double ps1 = k.pp_wre ? nag : 0.0, ps2 = k.pp_gre ? nrs : 0.0;
+    const double pd1 = k.pp_wre ? 0.0 : nag, pd2 = k.pp_gre ? 0.0 : nrs;
+    const double opb = t[MIST_T_OPB];
+    rows->xy[2][at] = double2{x + k.post_fwd + opb + ps1 + ps2, m.div_G(d + pd1 + pd2)};
+    rows->xy[3][at] = double2{x + k.pre_fwd + k.pre_bwd + k.post_fwd + opb + k.w1 + k.w2 + ps1 + ps2,
+                              m.div_G(d + k.w1d + k.w2d + pd1 + pd2)};
+  }
+  rows->counts[at] = (uint32_t)count_b | (uint32_t)count_p << 15 | (post ? 1u << 30 : 0u) | (pp ? 1u << 31 : 0u);
+}
+
+// Workgroup = one wavefront = one pair of a group with the minima of all its samples in LDS, a
+// column per sample.  Lane = row for the latencies and counts of 64 gathered rows, then lane = (row
+// parity, sample): one LDS minimum per (row, variant, sample) at the row's own count, conflict-free
+// but for the two rows in flight.  The minima per p are the suffix minima of those buckets.
+// (30 samples one after the other through seed_kernel: 3.1 ms for the tables of one tensor-parallel
+// size of the 7B plan.)
+__global__ __launch_bounds__(64) void seed_samples_kernel(
+    const MistProblem prob, const MistGroupDesc *__restrict__ groups, const double *__restrict__ row_terms,
+    const RatioList ratios, ReduceTables tabs, int sample_split) {
+  extern __shared__ unsigned long long lds_best[];
+  const MistGroupDesc *g = groups + blockIdx.y;
+  clear_queue(tabs);
+  const int tile_rel = (int)blockIdx.x / MIST_LC_TILE, lane = threadIdx.x;
+  if (tile_rel >= g->n_lc_tiles) return;
+  const int L = prob.num_layers, n_pairs = L * (L + 1) / 2 + L;
+  const int P = g->num_p, n_slots = slots_of(P);
+  const int first_sample = (int)blockIdx.z * sample_split, S = min(sample_split, tabs.n_samples - first_sample);
+  const int pair = g->lc_tile_begin * MIST_LC_TILE + (int)blockIdx.x;
+  SampleRows *rows = reinterpret_cast<SampleRows *>(lds_best);
+  unsigned long long *mine = lds_best + sizeof(SampleRows) / 8;  // [slot][sample]
+  const unsigned long long kInf = (unsigned long long)__double_as_longlong((double)INFINITY);
+  for (int e = lane; e < n_slots * S; e += 64) mine[e] = kInf;
+  __syncthreads();
+  const int sample = lane & 31;
+  if (g->scout_stride > 0 && pair < n_pairs) {
+    const GroupModel m = group_model(prob, g);
+    const PairIndex pc = decode_pair(pair);
+    const int l = __builtin_amdgcn_readfirstlane(pc.l), c = __builtin_amdgcn_readfirstlane(pc.c);
+    const PairConsts k = pair_consts(l, c);
+    const int np = c == l - 1 ? min(P, 1) : P;
+    const bool do_post = c != l - 1, do_pp = do_post && l == L;
+    const double ratio = ratios.r[first_sample + min(sample, S - 1)];
+    const int n_gather = g->n_par * g->n_oo * g->n_ao * g->scout_stride;
+    const double *__restrict__ src = row_terms + g->row_offset * MIST_ROW_TERMS;
+    for (int q0 = 0; q0 < n_gather; q0 += 64) {
+      const int n_rows = min(64, n_gather - q0);
+      RowRegs t;
+      load_terms<0, MIST_ROW_TERMS>(t, src + gathered_position(g, min(q0 + lane, n_gather - 1)) * MIST_ROW_TERMS);
+      float x, d;
+      pair_latency(t, k, x, d);
+      const LaneMemory mem = pair_memory(t, k);
+      const int cnt_b = count_exact([&](int p) { return mem.scaled_base(p); }, lane < n_rows ? np : 0, m.cap);
+      const int cnt_p = count_exact([&](int p) { return mem.scaled_pre(p, m.pre_saved, m.pre_sas); },
+                                    lane < n_rows ? np : 0, m.cap);
+      bool ok_post = false, ok_pp = false;
+      if (do_post) post_fits(t, k, mem, m, mem.out, k.no_ck ? t[MIST_T_RD] : 0.0, ok_post, ok_pp);
+      ok_post = ok_post && lane < n_rows;
+      ok_pp = ok_pp && do_pp && lane < n_rows;
+      // (rows that fit nowhere are left out)
+      const uint64_t useful = __ballot(cnt_b > 0 || cnt_p > 0 || ok_post || ok_pp);
+      __syncthreads();
+      if (useful >> lane & 1ull)
+        put_sample_row(rows, __popcll(useful & ((1ull << lane) - 1ull)), t, x, d, k.no_ck, m, cnt_b, cnt_p, ok_post,
+                       ok_pp, do_post);
+      __syncthreads();
+      const int n_useful = __popcll(useful);
+      for (int r = lane >> 5; r < n_useful; r += 2) {
+        const uint32_t counts = rows->counts[r];
+        const int nb = (int)(counts & 0x7fff), npre = (int)(counts >> 15 & 0x7fff);
+        auto offer = [&](bool ok, int variant, int slot) {
+          const double2 xy = rows->xy[variant][r];
+          const double cost = ratio * xy.x + xy.y;
+          if (ok && sample < S && cost < INFINITY)
+            atomicMin(mine + slot * S + sample, (unsigned long long)__double_as_longlong(cost));
+        };
+        offer(nb > 0, 0, nb - 1);
+        offer(npre > 0, 1, P + npre - 1);
+        if (do_post) {
+          offer((counts >> 30 & 1u) != 0, 2, 2 * P);
+          if (do_pp) offer((counts >> 31) != 0, 3, 2 * P + 1);
+        }
+      }
+    }
+  }
+  __syncthreads();
+  const int64_t cell0 = g->cell_offset + (int64_t)blockIdx.x * n_slots;
+  if (sample < S) {
+    const int v = lane >> 5;  // base, with_pre
+    const int64_t at = cell0 * tabs.n_samples + first_sample + sample;
+    unsigned long long low = kInf;
+    for (int j = P - 1; j >= -1; --j) {
+      const int slot = j >= 0 ? v * P + j : 2 * P + v;
+      const unsigned long long held = mine[slot * S + sample];
+      low = j >= 0 ? min(low, held) : held;
+      tabs.best[at + (int64_t)slot * tabs.n_samples] = low;
+      tabs.row[at + (int64_t)slot * tabs.n_samples] = ~0u;
+    }
+  }
+  if (lane == 0 && first_sample == 0) tabs.changed[cell0 / 4] = 0;
+}
+
+// ---- summaries of kSuperStages stages ----
+__device__ __forceinline__ int64_t super_floor_slot(const MistGroupDesc *g, int group_index, int64_t super) {
+  return stage_floor_slot(g, group_index, 0) / kSuperStages + group_index + super;
+}
+__global__ __launch_bounds__(256) void super_floor_kernel(const MistGroupDesc *__restrict__ groups, int n_groups,
+                                                          const double *__restrict__ stage_floor,
+                                                          double *__restrict__ super_floor) {
+  const int gi = blockIdx.y;
+  const MistGroupDesc *g = groups + gi;
+  const int64_t n_stages = (g->n_rows + kStageRows - 1) / kStageRows;
+  const int col = threadIdx.x % kStageFloorPitch;
+  const int per_block = blockDim.x / kStageFloorPitch;
+  for (int64_t super = (int64_t)blockIdx.x * per_block + threadIdx.x / kStageFloorPitch;
+       super * kSuperStages < n_stages; super += (int64_t)gridDim.x * per_block) {
+    const double *__restrict__ src = stage_floor + (stage_floor_slot(g, gi, super * kSuperStages)) * kStageFloorPitch;
+    const int n = (int)min((int64_t)kSuperStages, n_stages - super * kSuperStages);
+    double v = src[col];
+    for (int i = 1; i < n; ++i) {
+      const double o = src[i * kStageFloorPitch + col];
+      v = col == kStageMaxOut ? fmax(v, o) : fmin(v, o);
+    }
+    super_floor[super_floor_slot(g, gi, super) * kStageFloorPitch + col] = v;
+  }
+}
+
+// The largest minimum of every variant of a lane's pair: a row above all of them changes nothing
+// (the minima do not decrease with p; +inf while a slot is empty).
+struct Loosest {
+  double base, pre, post, pp;
+};
+// (`slots`: the pair's slots of one sample, `pitch` apart)
+__device__ __forceinline__ Loosest loosest_minima(const double *slots, int pitch, int P, int count_b, int count_p,
+                                                  bool do_post, bool do_pp, double cutoff) {
+  const double base = slots[max(count_b - 1, 0) * pitch], pre = slots[(P + max(count_p - 1, 0)) * pitch];
+  const double post = slots[2 * P * pitch], pp = slots[(2 * P + 1) * pitch];
+  return Loosest{count_b > 0 ? fmin(base, cutoff) : -INFINITY, count_p > 0 ? fmin(pre, cutoff) : -INFINITY,
+                 do_post ? fmin(post, cutoff) : -INFINITY, do_pp ? fmin(pp, cutoff) : -INFINITY};
+}
+// One threshold for `bound` (see Offsets) that every row which could reach one of them passes.
+__device__ __forceinline__ double bound_threshold(const Loosest &t, const Offsets &o) {
+  return fmax(t.base + kBaseSlack * fabs(t.base),
+              fmax(below(t.pre, o.pre), fmax(below(t.post, o.post), below(t.pp, o.pp))));
+}
+
+// Lane = pair against a stage summary: the counts its pseudo row allows, hence which minima a row
+// of the stage can reach, and the bound that its objective gives.
+struct StageReach {
+  int count_b, count_p;  // base, with_pre
+  bool post, pp;
+  float x, d;            // of the pseudo row
+  __device__ __forceinline__ double threshold(const double *slots, int pitch, int P, double ratio, double cutoff,
+                                              const GroupModel &m, const double *__restrict__ floor) const {
+    return bound_threshold(loosest_minima(slots, pitch, P, count_b, count_p, post, pp, cutoff),
+                           composite_offsets(m, ratio, floor[kStageMinOpb], floor[kStageMinNag], floor[kStageMinNrs]));
+  }
+};
+__device__ __forceinline__ StageReach stage_reach(const double *__restrict__ f, const PairConsts &k, int np,
+                                                  bool do_post, bool do_pp, const GroupModel &m) {
+  StageReach r;
+  pair_latency(f, k, r.x, r.d);
+  const LaneMemory mem = pair_memory(f, k);
+  r.count_b = count_bound([&](int p) { return mem.scaled_base(p); }, np, m.cap);
+  r.count_p = count_bound([&](int p) { return mem.scaled_pre(p, m.pre_saved, m.pre_sas); }, np, m.cap);
+  bool post, pp;
+  post_fits(f, k, mem, m, f[kStageMaxOut], 0.0, post, pp);
+  r.post = do_post && post;
+  r.pp = do_pp && pp;
+  return r;
+}
+
+// ---- filter ----
+// Workgroup = one wavefront = (row chunk, tile, p tile as a share of the chunk's summaries), lane
+// = pair.  Summaries are wave-uniform and come through scalar loads; a visit is ~40 float64
+// instructions against the pair's loosest minima.
+__global__ __launch_bounds__(MIST_LC_TILE) void filter_kernel(
     const MistProblem prob, const MistGroupDesc *__restrict__ groups, int n_groups,
-    const int32_t *__restrict__ block_prefix, int n_blocks,
-    const int32_t *__restrict__ scout_prefix, int scout, const double *__restrict__ row_terms,
-    const double *__restrict__ stage_floor, const RatioList ratios, int first_sample,
-    int64_t scout_base, double *__restrict__ partial_cost, int32_t *__restrict__ partial_index) {
-  __shared__ double lds_terms[kStageRows * kLdsRowStride];
-  __shared__ double lds_min[kStageFloorPitch];
-  __shared__ double lds_pair[MIST_LC_TILE * kPairFields];
-  __shared__ int32_t lds_rowpos[kStageRows];
-  // blockIdx.y = sample first_sample + y of the ratio list.  Slabs: the main launch of its y-th
-  // sample writes slabs y * n_blocks + workgroup; the scout slabs of sample s (of the list) are
-  // scout_base + s * n_scout_total + workgroup, and seed the main launch of the same sample.
-  const int sample = first_sample + (int)blockIdx.y;
-  const double ratio = ratios.r[sample];
-  const int n_scout_total = scout_prefix != nullptr ? scout_prefix[n_groups] : 0;
+    const int32_t *__restrict__ block_prefix, int n_blocks, const double *__restrict__ stage_floor,
+    const double *__restrict__ super_floor, const RatioList ratios, ReduceTables tabs) {
   const int block = xcd_run_block(blockIdx.x);
-  if (block >= (scout ? n_scout_total : n_blocks)) return;
+  if (block >= n_blocks) return;
   int local_block;
-  const MistGroupDesc *g = find_group(groups, scout ? scout_prefix : block_prefix, n_groups,
-                                      block, &local_block);
-  const int gi = (int)(g - groups);
-  const bool seeded = scout_prefix != nullptr && g->scout_stride > 0;
-  int tile;
-  ReduceRange range;
-  int64_t out_slab;
-  bool skip_unchanged = false;  // only the chunks after the first of a tile may leave a mark
-  if (scout) {
-    if (g->scout_stride <= 0) return;
-    tile = local_block / kScoutSplit;
-    const int part = local_block % kScoutSplit;  // gathered stages part, part + split, ...
-    range = ReduceRange{(int64_t)part * kStageRows, g->n_rows, kScoutSplit, 0, 1};
-    out_slab = scout_base + (int64_t)sample * n_scout_total + block;
-  } else {
-    const int n_tiles = g->n_lc_tiles * g->n_p_tiles;
-    const int chunk = local_block / n_tiles;  // the tiles of one chunk are neighbours
-    tile = local_block % n_tiles;
-    const int64_t row_begin = (int64_t)chunk * g->rows_per_chunk;
-    range = ReduceRange{row_begin, min(row_begin + (int64_t)g->rows_per_chunk, g->n_rows), 1, 0, 0};
-    out_slab = (int64_t)blockIdx.y * n_blocks + block;
-    skip_unchanged = chunk > 0;
+  const MistGroupDesc *g = find_group(groups, block_prefix, n_groups, block, &local_block);
+  const int gi = __builtin_amdgcn_readfirstlane((int)(g - groups));
+  g = groups + gi;
+  local_block = __builtin_amdgcn_readfirstlane(local_block);
+  const int n_p = g->n_p_tiles, n_tiles = g->n_lc_tiles * n_p;
+  const int chunk = local_block / n_tiles, tile = local_block % n_tiles;
+  const int share = tile % n_p, tile_rel = tile / n_p;
+  const int n_stages = (int)((g->n_rows + kStageRows - 1) / kStageRows);
+  const int stage0 = (int)((int64_t)chunk * g->rows_per_chunk / kStageRows);
+  const int stage1 = min(stage0 + g->rows_per_chunk / kStageRows, n_stages);
+  const int super_first = stage0 / kSuperStages + share, super_last = (stage1 - 1) / kSuperStages;
+
+  const int L = prob.num_layers, n_pairs = L * (L + 1) / 2 + L, lane = threadIdx.x;
+  const int pair_idx = (g->lc_tile_begin + tile_rel) * MIST_LC_TILE + lane;
+  const bool active = pair_idx < n_pairs;
+  const PairIndex pc = decode_pair(active ? pair_idx : 0);
+  const PairConsts k = pair_consts(pc.l, pc.c);
+  const int P = g->num_p, S = tabs.n_samples;
+  const int np = !active ? 0 : (pc.c == pc.l - 1 ? min(P, 1) : P);
+  const bool do_post = active && pc.c != pc.l - 1, do_pp = do_post && pc.l == L;
+  const GroupModel m = group_model(prob, g);
+  const double cutoff = stage_cost_cutoff(prob, m.inv_G64);
+  const double *slots = reinterpret_cast<const double *>(tabs.best) +
+                        (g->cell_offset + ((int64_t)tile_rel * MIST_LC_TILE + lane) * slots_of(P)) * S;
+
+  // no lane's row can matter: the pseudo row against the loosest minima
+  auto closed = [&](const double *__restrict__ f, double ratio, const Loosest &t) {
+    float x, d;
+    pair_latency(f, k, x, d);
+    const Offsets o = composite_offsets(m, ratio, f[kStageMinOpb], f[kStageMinNag], f[kStageMinNrs]);
+    return !__any(ratio * (double)x + m.div_G((double)d) <= bound_threshold(t, o));
+  };
+  const double *__restrict__ supers = super_floor + super_floor_slot(g, gi, 0) * kStageFloorPitch;
+  const double *__restrict__ stages = stage_floor + stage_floor_slot(g, gi, 0) * kStageFloorPitch;
+  // batches of 64 summaries; lane i keeps the open stages of the batch's i-th
+  for (int first = super_first; first <= super_last; first += 64 * n_p) {
+    uint32_t open = 0;
+    for (int s = 0; s < S; ++s) {
+      const Loosest t = loosest_minima(slots + s, S, P, np, np, do_post, do_pp, cutoff);
+      const double ratio = ratios.r[s];
+      for (int i = 0; i < 64; ++i) {
+        const int super = first + i * n_p;
+        if (super > super_last) break;
+        const int st0 = max(super * kSuperStages, stage0), st1 = min((super + 1) * kSuperStages, stage1);
+        uint32_t seen = s > 0 ? (uint32_t)from_lane((int)open, i) : 0u;
+        if (seen == (1u << (st1 - st0)) - 1u) continue;
+        if (closed(supers + (int64_t)super * kStageFloorPitch, ratio, t)) continue;
+        for (int st = st0; st < st1; ++st)
+          if (!(seen >> (st - st0) & 1u) && !closed(stages + (int64_t)st * kStageFloorPitch, ratio, t))
+            seen |= 1u << (st - st0);
+        open = lane == i ? seen : open;
+      }
+    }
+    // append the open stages to the tile's shard of the queue (items of a tile read the same minima:
+    // its shard is worked off by one XCD), to the next ones if it is full (all shards together hold
+    // every (tile, stage) of the launch)
+    const int mine = __popc(open);
+    int end = mine;
+    for (int step = 1; step < 64; step <<= 1) {
+      const int o = __shfl_up(end, step);
+      if (lane >= step) end += o;
+    }
+    const int total = from_lane(end, 63);
+    int shard = (gi * 13 + tile_rel) % kQueueShards;
+    for (int done = 0; done < total; shard = (shard + 1) % kQueueShards) {
+      uint32_t base = 0;
+      if (lane == 0) base = atomicAdd(tabs.counter + shard * kCounterPitch, (uint32_t)(total - done));
+      base = (uint32_t)from_lane((int)base, 0);
+      const int room = base >= tabs.capacity ? 0 : (int)min((uint32_t)(total - done), tabs.capacity - base);
+      int at = end - mine;  // index of this lane's next item among the batch's
+      const int st0 = max((first + lane * n_p) * kSuperStages, stage0);
+      for (uint32_t rest = open; rest != 0; rest &= rest - 1, ++at) {
+        if (at < done || at >= done + room) continue;
+        const int st = st0 + __ffs(rest) - 1;
+        tabs.item[(int64_t)shard * tabs.capacity + base + (at - done)] =
+            (unsigned long long)gi << 48 | (unsigned long long)tile_rel << 32 | (uint32_t)st;
+      }
+      done += room;
+    }
   }
-  const int p_tile = tile % g->n_p_tiles;
-  const int lc_tile = g->lc_tile_begin + tile / g->n_p_tiles;  // position in the pair list
-  const int64_t slab = (int64_t)kSlots * MIST_LC_TILE;
-  const int64_t seed_slab = scout_base + (int64_t)sample * n_scout_total +
-                            (seeded ? scout_prefix[gi] + tile * kScoutSplit : 0);
-  const double *seed_cost = (!scout && seeded) ? partial_cost + seed_slab * slab : nullptr;
-  const int32_t *seed_index = (!scout && seeded) ? partial_index + seed_slab * slab : nullptr;
-  const bool pow2 = (g->grad_accum & (g->grad_accum - 1)) == 0;
-#define MIST_REDUCE(P2, FT)                                                                   \
-  reduce_block<P2, FT>(prob, g, range, p_tile, lc_tile, row_terms,                            \
-                       stage_floor + stage_floor_slot(g, gi, 0) * kStageFloorPitch, ratio,    \
-                       lds_terms, lds_min, lds_pair, lds_rowpos, seed_cost, seed_index,                   \
-                       partial_cost + out_slab * slab, partial_index + out_slab * slab,       \
-                       skip_unchanged)
-  if (pow2) {
-    if (p_tile == 0) MIST_REDUCE(true, true); else MIST_REDUCE(true, false);
-  } else {
-    if (p_tile == 0) MIST_REDUCE(false, true); else MIST_REDUCE(false, false);
+}
+
+// ---- open ----
+// Flat list over the shards of a queue, in shard order (lane = shard).
+struct FlatQueue {
+  uint32_t end;  // of this lane's shard
+  uint32_t total;
+  __device__ __forceinline__ int64_t at(uint32_t i, uint32_t capacity) const {
+    const int shard = __popcll((unsigned long long)__ballot(end <= i));
+    const uint32_t first = shard > 0 ? (uint32_t)from_lane((int)end, shard - 1) : 0u;
+    return (int64_t)shard * capacity + (i - first);
   }
-#undef MIST_REDUCE
+};
+__device__ __forceinline__ FlatQueue flat_queue(const ReduceTables &tabs, int queue) {
+  const int lane = threadIdx.x & 63;
+  FlatQueue q;
+  q.end = min(tabs.counter[(queue * kQueueShards + lane) * kCounterPitch], tabs.capacity);
+  for (int step = 1; step < 64; step <<= 1) {
+    const uint32_t o = (uint32_t)__shfl_up((int)q.end, step);
+    if (lane >= step) q.end += o;
+  }
+  q.total = (uint32_t)from_lane((int)q.end, 63);
+  return q;
+}
+
+// A lane's pair of a tile.
+struct TileLane {
+  PairIndex pc;
+  bool active, do_post, do_pp;
+  int np;
+};
+__device__ __forceinline__ TileLane tile_lane(const MistProblem &prob, const MistGroupDesc *__restrict__ g, int tile_rel) {
+  const int L = prob.num_layers, n_pairs = L * (L + 1) / 2 + L;
+  const int pair_idx = (g->lc_tile_begin + tile_rel) * MIST_LC_TILE + (int)(threadIdx.x & 63);
+  TileLane t;
+  t.active = pair_idx < n_pairs;
+  t.pc = decode_pair(t.active ? pair_idx : 0);
+  t.np = !t.active ? 0 : (t.pc.c == t.pc.l - 1 ? min(g->num_p, 1) : g->num_p);
+  t.do_post = t.active && t.pc.c != t.pc.l - 1;
+  t.do_pp = t.do_post && t.pc.l == L;
+  return t;
+}
+
+// A wavefront per item: only what its memory bounds leave open stays (7B on 4x8: 378000 stages x
+// tiles, 34000 pass the filter and 7800 of those are opened).
+__global__ __launch_bounds__(kReduceThreads) void open_kernel(const MistProblem prob,
+                                                              const MistGroupDesc *__restrict__ groups,
+                                                              const double *__restrict__ stage_floor,
+                                                              const RatioList ratios, const ReduceTables tabs) {
+  constexpr int kWaves = kReduceThreads / 64;
+  const int lane = threadIdx.x & 63, S = tabs.n_samples;
+  const FlatQueue queue = flat_queue(tabs, 0);
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * kWaves + (threadIdx.x >> 6)));
+  for (uint32_t i = wave; i < queue.total; i += gridDim.x * kWaves) {
+    const int64_t from = queue.at(i, tabs.capacity);
+    const uint64_t item = from_lane((uint64_t)tabs.item[from], 0);
+    const int gi = (int)(item >> 48), tile_rel = (int)(item >> 32 & 0xffff), stage = (int)(uint32_t)item;
+    const MistGroupDesc *g = groups + gi;
+    const TileLane p = tile_lane(prob, g, tile_rel);
+    const GroupModel m = group_model(prob, g);
+    const double cutoff = stage_cost_cutoff(prob, m.inv_G64);
+    const int P = g->num_p;
+    const double *__restrict__ f = stage_floor + stage_floor_slot(g, gi, stage) * kStageFloorPitch;
+    const StageReach reach = stage_reach(f, pair_consts(p.pc.l, p.pc.c), p.np, p.do_post, p.do_pp, m);
+    const double *slots = reinterpret_cast<const double *>(tabs.best) +
+                          (g->cell_offset + ((int64_t)tile_rel * MIST_LC_TILE + lane) * slots_of(P)) * S;
+    bool open = false;
+    for (int s = 0; s < S && !__any(open); ++s)
+      open = p.active && ratios.r[s] * (double)reach.x + m.div_G((double)reach.d) <=
+                             reach.threshold(slots + s, S, P, ratios.r[s], cutoff, m, f);
+    if (!__any(open)) continue;
+    const uint32_t shard = (uint32_t)(from / tabs.capacity);
+    if (lane == 0) {
+      // (no more than the shard's items are opened: it cannot overflow)
+      const uint32_t to = atomicAdd(tabs.counter + (kQueueShards + shard) * kCounterPitch, 1u);
+      tabs.opened[(int64_t)shard * tabs.capacity + to] = item;
+      tabs.hit[(int64_t)shard * tabs.capacity + to] = 0;
+    }
+  }
+}
+
+// ---- reduce / resolve ----
+// One item with the pairs in `pairs`, one sample.  Returns the pairs in which some row reached its
+// minimum (kResolve: unused).  `lds_row`: the wavefront's buffer for the minima of one pair, which
+// the rows look up at their own counts; the next pair's are on their way in registers meanwhile.
+template <bool kResolve>
+__device__ __forceinline__ uint64_t reduce_item(const MistProblem &prob, const MistGroupDesc *__restrict__ g, int gi,
+                                                int tile_rel, int stage, const double *__restrict__ row_terms,
+                                                const double *__restrict__ stage_floor, double ratio,
+                                                const ReduceTables &tabs, uint64_t pairs, double *lds_row) {
+  const int L = prob.num_layers, lane = threadIdx.x & 63;
+  const TileLane tl = tile_lane(prob, g, tile_rel);
+  const int P = g->num_p, n_slots = slots_of(P);
+  const GroupModel m = group_model(prob, g);
+  const double cutoff = stage_cost_cutoff(prob, m.inv_G64);
+  const int64_t tile_cell = g->cell_offset + (int64_t)tile_rel * MIST_LC_TILE * n_slots;
+  const double *best = reinterpret_cast<const double *>(tabs.best) + tile_cell;  // [pair][slot]
+
+  // ---- lane = pair: slots the pseudo row of the stage can reach, and the minima there ----
+  const double *__restrict__ f = stage_floor + stage_floor_slot(g, gi, stage) * kStageFloorPitch;
+  double thr;  // of this lane's pair
+  uint64_t todo;
+  {
+    const StageReach reach = stage_reach(f, pair_consts(tl.pc.l, tl.pc.c), tl.np, tl.do_post, tl.do_pp, m);
+    thr = reach.threshold(best + lane * n_slots, 1, P, ratio, cutoff, m, f);
+    todo = pairs & __ballot(tl.active && ratio * (double)reach.x + m.div_G((double)reach.d) <= thr);
+  }
+  if (todo == 0) return 0;
+
+  // ---- lane = row ----
+  const int64_t row0 = (int64_t)stage * kStageRows;
+  const int n_stage = (int)min((int64_t)kStageRows, g->n_rows - row0);
+  const double *__restrict__ my_row = row_terms + (g->row_offset + row0 + min(lane, n_stage - 1)) * MIST_ROW_TERMS;
+  const bool live = lane < n_stage;
+  RowRegs t;
+  load_terms<0, MIST_T_D_LAST_NOCK + 1>(t, my_row);
+  uint64_t sieve = 0;  // rows that pass the threshold of this lane's pair
+  for (uint64_t rest = todo; rest != 0; rest &= rest - 1) {
+    const int pl = __ffsll((unsigned long long)rest) - 1;
+    const PairConsts k = pair_consts(from_lane(tl.pc.l, pl), from_lane(tl.pc.c, pl));
+    float x, d;
+    pair_latency(t, k, x, d);
+    const uint64_t pass = __ballot(live && ratio * (double)x + m.div_G((double)d) <= from_lane(thr, pl));
+    sieve = lane == pl ? pass : sieve;
+  }
+  todo = __ballot(sieve != 0);
+  if (todo == 0) return 0;
+  load_terms<MIST_T_D_LAST_NOCK + 1, MIST_ROW_TERMS>(t, my_row);
+  // minima of one pair, a slot per lane and register
+  double ahead0 = 0.0, ahead1 = 0.0;
+  auto fetch = [&](int pair) {
+    const double *slots = best + pair * n_slots;
+    ahead0 = slots[min(lane, n_slots - 1)];
+    if (n_slots > 64) ahead1 = slots[min(lane + 64, n_slots - 1)];
+  };
+  auto settle = [&](int pair) {
+    __builtin_amdgcn_wave_barrier();
+    if (lane < n_slots) lds_row[lane] = ahead0;
+    if (lane + 64 < n_slots) lds_row[lane + 64] = ahead1;
+    for (int j = lane + 128; j < n_slots; j += 64) lds_row[j] = best[pair * n_slots + j];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+  fetch(__ffsll((unsigned long long)todo) - 1);
+  const uint32_t my_row_number =
+      (kResolve ? 0u : kUnresolved) + (uint32_t)row_of_position(g, row0 + min(lane, n_stage - 1));
+  uint64_t hits = 0;
+  for (uint64_t rest = todo; rest != 0; rest &= rest - 1) {
+    const int pl = __ffsll((unsigned long long)rest) - 1;
+    const int l = from_lane(tl.pc.l, pl), c = from_lane(tl.pc.c, pl);
+    const PairConsts k = pair_consts(l, c);
+    float x, d;
+    pair_latency(t, k, x, d);
+    const bool in = (from_lane(sieve, pl) >> lane & 1ull) != 0;
+    settle(pl);
+    const uint64_t later = rest & (rest - 1);
+    if (later != 0) fetch(__ffsll((unsigned long long)later) - 1);
+    const LaneMemory mem = pair_memory(t, k);
+    const int np = c == l - 1 ? min(P, 1) : P;
+    const bool do_post = c != l - 1, do_pp = do_post && l == L;
+    const int row_b = count_exact([&](int p) { return mem.scaled_base(p); }, in ? np : 0, m.cap);
+    const int row_p = count_exact([&](int p) { return mem.scaled_pre(p, m.pre_saved, m.pre_sas); }, in ? np : 0, m.cap);
+    bool ok_post = false, ok_pp = false;
+    if (do_post) post_fits(t, k, mem, m, mem.out, k.no_ck ? t[MIST_T_RD] : 0.0, ok_post, ok_pp);
+    const Objectives o = objectives(t, x, d, k.no_ck, ratio, m, do_post);
+    bool hit = false, lowered = false;
+    const int64_t cell = tile_cell + pl * n_slots;
+    // rows with `count` > 0 against the minimum of slot `slot` + count - 1
+    auto offer = [&](int count, double cost, int slot) {
+      const int own = slot + max(count - 1, 0);
+      const double now = in && count > 0 && cost <= cutoff && cost < INFINITY ? lds_row[own] : -INFINITY;
+      if (!kResolve && cost < now) {
+        atomicMin(tabs.best + cell + own, (unsigned long long)__double_as_longlong(cost));
+        lowered = true;
+      }
+      if (cost == now) atomicMin(tabs.row + cell + own, my_row_number);
+      hit = hit || cost <= now;
+    };
+    offer(row_b, o.base, 0);
+    offer(row_p, o.pre, P);
+    if (do_post) offer(ok_post ? 1 : 0, o.post, 2 * P);
+    if (do_pp) offer(ok_pp ? 1 : 0, o.pp, 2 * P + 1);
+    if (kResolve) continue;
+    if (__any(lowered) && lane == 0) tabs.changed[cell / 4] = 1u;
+    if (__any(hit)) hits |= 1ull << pl;
+  }
+  return hits;
+}
+
+// The same for several samples: lane = row for latencies, counts and the test against the samples'
+// thresholds, then lane = (row parity, sample) for the rows that pass some of them: the minima of a
+// slot lie side by side, so a row's look-up of all samples is one line.  (A wavefront that took the
+// samples one after the other, its minima through LDS: 14 ms for the tables of one tensor-parallel
+// size of the 7B plan, two thirds of it waiting for minima.)
+template <bool kResolve>
+__device__ __forceinline__ uint64_t reduce_item_samples(const MistProblem &prob, const MistGroupDesc *__restrict__ g,
+                                                        int gi, int tile_rel, int stage,
+                                                        const double *__restrict__ row_terms,
+                                                        const double *__restrict__ stage_floor, const RatioList &ratios,
+                                                        const ReduceTables &tabs, uint64_t pairs, SampleRows *rows) {
+  const int L = prob.num_layers, lane = threadIdx.x & 63, sample = lane & 31;
+  const TileLane tl = tile_lane(prob, g, tile_rel);
+  const int P = g->num_p, n_slots = slots_of(P), S = tabs.n_samples;
+  const GroupModel m = group_model(prob, g);
+  const int64_t tile_cell = g->cell_offset + (int64_t)tile_rel * MIST_LC_TILE * n_slots;
+  const double *best = reinterpret_cast<const double *>(tabs.best) + tile_cell * S;  // [pair][slot][sample]
+  const double *__restrict__ f = stage_floor + stage_floor_slot(g, gi, stage) * kStageFloorPitch;
+  const double ratio = ratios.r[min(sample, S - 1)];
+  const StageReach reach = stage_reach(f, pair_consts(tl.pc.l, tl.pc.c), tl.np, tl.do_post, tl.do_pp, m);
+  uint64_t todo = pairs & __ballot(tl.active && (reach.count_b > 0 || reach.count_p > 0 || reach.post || reach.pp));
+
+  const int64_t row0 = (int64_t)stage * kStageRows;
+  const int n_stage = (int)min((int64_t)kStageRows, g->n_rows - row0);
+  const double *__restrict__ my_row = row_terms + (g->row_offset + row0 + min(lane, n_stage - 1)) * MIST_ROW_TERMS;
+  const bool live = lane < n_stage;
+  const uint32_t my_row_number =
+      (kResolve ? 0u : kUnresolved) + (uint32_t)row_of_position(g, row0 + min(lane, n_stage - 1));
+  RowRegs t;
+  load_terms<0, MIST_T_D_LAST_NOCK + 1>(t, my_row);
+  bool have_rest = false;
+  uint64_t hits = 0;
+  for (uint64_t rest = todo; rest != 0; rest &= rest - 1) {
+    const int pl = __ffsll((unsigned long long)rest) - 1;
+    const int l = from_lane(tl.pc.l, pl), c = from_lane(tl.pc.c, pl);
+    const PairConsts k = pair_consts(l, c);
+    const double *slots = best + (int64_t)pl * n_slots * S;
+    // ---- lane = sample: thresholds ----
+    const StageReach its{from_lane(reach.count_b, pl), from_lane(reach.count_p, pl), from_lane((int)reach.post, pl) != 0,
+                         from_lane((int)reach.pp, pl) != 0, from_lane(reach.x, pl), from_lane(reach.d, pl)};
+    double thr = its.threshold(slots + min(sample, S - 1), S, P, ratio, INFINITY, m, f);
+    if (kResolve)  // only the samples whose minima changed
+      thr = tabs.changed[(tile_cell + pl * n_slots) / 4] >> sample & 1u ? thr : -INFINITY;
+    if (!__any(ratio * (double)its.x + m.div_G((double)its.d) <= thr)) continue;
+    // ---- lane = row ----
+    float x, d;
+    pair_latency(t, k, x, d);
+    const double xd = (double)x, dG = m.div_G((double)d);
+    bool pass = false;
+    for (int s = 0; s < S; ++s) pass = pass || ratios.r[s] * xd + dG <= from_lane(thr, s);
+    pass = pass && live;
+    if (!__any(pass)) continue;
+    if (!have_rest) {
+      load_terms<MIST_T_D_LAST_NOCK + 1, MIST_ROW_TERMS>(t, my_row);
+      have_rest = true;
+    }
+    const LaneMemory mem = pair_memory(t, k);
+    const int np = c == l - 1 ? min(P, 1) : P;
+    const bool do_post = c != l - 1, do_pp = do_post && l == L;
+    const int row_b = count_exact([&](int p) { return mem.scaled_base(p); }, pass ? np : 0, m.cap);
+    const int row_p = count_exact([&](int p) { return mem.scaled_pre(p, m.pre_saved, m.pre_sas); }, pass ? np : 0, m.cap);
+    bool ok_post = false, ok_pp = false;
+    if (do_post) post_fits(t, k, mem, m, mem.out, k.no_ck ? t[MIST_T_RD] : 0.0, ok_post, ok_pp);
+    ok_post = ok_post && pass;
+    ok_pp = ok_pp && do_pp && pass;
+    const uint64_t useful = __ballot(row_b > 0 || row_p > 0 || ok_post || ok_pp);
+    if (useful == 0) continue;
+    __builtin_amdgcn_wave_barrier();
+    const int at = __popcll(useful & ((1ull << lane) - 1ull));
+    if (useful >> lane & 1ull) {
+      put_sample_row(rows, at, t, x, d, k.no_ck, m, row_b, row_p, ok_post, ok_pp, do_post);
+      rows->number[at] = my_row_number;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    // ---- lane = (row parity, sample) ----
+    const int n_useful = __popcll(useful);
+    const int64_t at0 = (tile_cell + (int64_t)pl * n_slots) * S + sample;
+    bool hit = false, lowered = false;
+    const bool sampled = sample < S && (!kResolve || thr != -INFINITY);
+    // look-ups of a row, one iteration ahead of their use
+    double now_b, now_p, now_post = -INFINITY, now_pp = -INFINITY;
+    uint32_t counts;
+    auto look = [&](int r) {
+      counts = rows->counts[min(r, n_useful - 1)];
+      const int nb = (int)(counts & 0x7fff), npre = (int)(counts >> 15 & 0x7fff);
+      const double *mine = slots + min(sample, S - 1);
+      now_b = mine[max(nb - 1, 0) * S];
+      now_p = mine[(P + max(npre - 1, 0)) * S];
+      if (do_post) now_post = mine[2 * P * S];
+      if (do_pp) now_pp = mine[(2 * P + 1) * S];
+    };
+    look(lane >> 5);
+    for (int r0 = 0; r0 < n_useful; r0 += 2) {
+      const int r = min(r0 + (lane >> 5), n_useful - 1);
+      const bool on = sampled && r0 + (lane >> 5) < n_useful;
+      const uint32_t cn = counts;
+      const double nb_now = now_b, np_now = now_p, post_now = now_post, pp_now = now_pp;
+      if (r0 + 2 < n_useful) look(r0 + 2 + (lane >> 5));
+      auto offer = [&](bool ok, int variant, int own, double now) {
+        const double2 xy = rows->xy[variant][r];
+        const double cost = ratio * xy.x + xy.y;
+        if (!(on && ok && cost <= now && cost < INFINITY)) return;
+        hit = true;
+        const int64_t to = at0 + (int64_t)own * S;
+        if (cost == now) {
+          atomicMin(tabs.row + to, rows->number[r]);
+        } else if (!kResolve) {
+          atomicMin(tabs.best + to, (unsigned long long)__double_as_longlong(cost));
+          lowered = true;
+        }
+      };
+      const int nb = (int)(cn & 0x7fff), npre = (int)(cn >> 15 & 0x7fff);
+      offer(nb > 0, 0, nb - 1, nb_now);
+      offer(npre > 0, 1, P + npre - 1, np_now);
+      if (do_post) {
+        offer((cn >> 30 & 1u) != 0, 2, 2 * P, post_now);
+        if (do_pp) offer((cn >> 31) != 0, 3, 2 * P + 1, pp_now);
+      }
+    }
+    if (!kResolve) {
+      const uint64_t low = __ballot(lowered);
+      const uint32_t samples = (uint32_t)low | (uint32_t)(low >> 32);
+      if (samples != 0 && lane == 0) atomicOr(tabs.changed + (tile_cell + pl * n_slots) / 4, samples);
+      if (__any(hit)) hits |= 1ull << pl;
+    }
+  }
+  return hits;
+}
+
+// Every 2^k-th pair from the first on.
+__device__ __forceinline__ uint64_t every_pair(int k) {
+  return k == 0 ? ~0ull : k == 1 ? 0x5555555555555555ull : k == 2 ? 0x1111111111111111ull : k == 3 ? 0x0101010101010101ull
+                                                                                     : 0x0001000100010001ull;
+}
+
+// A unit of work is an opened item with every 2^split-th of its pairs: an item has 1 to 64 open
+// pairs at 1 - 3 us each, and a wavefront that drew several full ones was the launch's length (7B
+// on 4x8, whole items handed out in turn: 0.53 ms at one wavefront per SIMD on average).  The list
+// is in tile order; each XCD draws from its eighth of it, then from the next ones', and the next
+// draw is on its way while a unit is worked on.
+template <bool kResolve, bool kSamples>
+__global__ __launch_bounds__(kReduceThreads, 3) void reduce_kernel(
+    const MistProblem prob, const MistGroupDesc *__restrict__ groups, const double *__restrict__ row_terms,
+    const double *__restrict__ stage_floor, const RatioList ratios, const ReduceTables tabs, int row_pitch) {
+  extern __shared__ double lds_rows[];
+  constexpr int kWaves = kReduceThreads / 64;
+  const int local_wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+  const FlatQueue queue = flat_queue(tabs, 1);
+  int split = 0;  // enough units for every wavefront several times over
+  while (split < 4 && ((uint64_t)queue.total << split) < (uint64_t)gridDim.x * kWaves * 2) ++split;
+  const uint64_t units = (uint64_t)queue.total << split;
+  auto work = [&](uint32_t u) {
+    uint64_t pairs = every_pair(split) << (u & ((1u << split) - 1u));
+    const int64_t at = queue.at(u >> split, tabs.capacity);
+    if (kResolve) pairs &= from_lane((uint64_t)tabs.hit[at], 0);
+    if (pairs == 0) return;
+    const uint64_t item = from_lane((uint64_t)tabs.opened[at], 0);
+    const int gi = (int)(item >> 48), tile_rel = (int)(item >> 32 & 0xffff), stage = (int)(uint32_t)item;
+    const MistGroupDesc *g = groups + gi;
+    if (kResolve) {  // pairs whose minima changed
+      const int n_slots = slots_of(g->num_p);
+      const int64_t cell = g->cell_offset + ((int64_t)tile_rel * MIST_LC_TILE + lane) * n_slots;
+      pairs &= __ballot(tabs.changed[cell / 4] != 0);
+      if (pairs == 0) return;
+    }
+    uint64_t hit;
+    if constexpr (kSamples) {
+      __shared__ SampleRows lds_samples[kWaves];
+      hit = reduce_item_samples<kResolve>(prob, g, gi, tile_rel, stage, row_terms, stage_floor, ratios, tabs, pairs,
+                                          &lds_samples[local_wave]);
+    } else
+      hit = reduce_item<kResolve>(prob, g, gi, tile_rel, stage, row_terms, stage_floor, ratios.r[0], tabs, pairs,
+                                  lds_rows + local_wave * row_pitch);
+    if (!kResolve && hit != 0 && lane == 0) atomicOr(tabs.hit + at, (unsigned long long)hit);
+  };
+  if (kResolve) {  // few are left: handed out in turn
+    for (uint64_t u = (uint64_t)blockIdx.x * kWaves + local_wave; u < units; u += (uint64_t)gridDim.x * kWaves)
+      work((uint32_t)u);
+    return;
+  }
+  for (int k = 0; k < kNumXcd; ++k) {
+    const int part = ((int)blockIdx.x + k) % kNumXcd;
+    const uint32_t first = (uint32_t)(units * part / kNumXcd), n = (uint32_t)(units * (part + 1) / kNumXcd) - first;
+    uint32_t *drawn = tabs.counter + (2 * kQueueShards + part) * kCounterPitch;
+    if (k > 0 && *drawn >= n) continue;
+    auto draw = [&]() {
+      uint32_t u = 0;
+      if (lane == 0) u = atomicAdd(drawn, 1u);
+      return u;
+    };
+    uint32_t ahead = draw();
+    for (;;) {
+      const uint32_t u = (uint32_t)from_lane((int)ahead, 0);
+      if (u >= n) break;
+      ahead = draw();
+      work(first + u);
+    }
+  }
 }
 
 // Rows offered in ascending order: the first of equal costs stays (pareto.py:134-142 as written).
@@ -1704,6 +2109,8 @@ __device__ __forceinline__ void take_first(double &best, int32_t &best_row, bool
 // produce the same tables (tests) and is measured against it.  Same decomposition and slab
 // layout as eval_reduce_kernel's main launch, so finalize_kernel reads either.
 // ------------------------------------------------------------------------------------------
+constexpr int kLdsRowStride = MIST_ROW_TERMS + 1;  // odd number of doubles: lanes reading the
+                                                   // same term of different rows hit different banks
 template <bool kFirstTile>
 __device__ __forceinline__ void exhaustive_block(
     const MistProblem &prob, const MistGroupDesc *__restrict__ g, int64_t row_begin,
@@ -1860,28 +2267,25 @@ __device__ __forceinline__ int incumbent_stage_count(const MistProblem &prob,
 // Workgroup = group, its wavefronts take the stages in turn; lowers *incumbent.
 constexpr int kIncumbentWaves = 4;
 __global__ __launch_bounds__(64 * kIncumbentWaves) void incumbent_kernel(
-    const MistProblem prob, const MistGroupDesc *__restrict__ groups,
-    const int32_t *__restrict__ scout_prefix, int64_t scout_base,
-    const double *__restrict__ partial_cost, const int32_t *__restrict__ partial_index) {
+    const MistProblem prob, const MistGroupDesc *__restrict__ groups, const ReduceTables tabs) {
   const MistGroupDesc *g = groups + blockIdx.x;
   if (g->scout_stride <= 0) return;
   const int L = prob.num_layers;
   const int S = incumbent_stage_count(prob, g);
   if (S == 0) return;
-  const int l = L / S;
-  const int64_t slab = (int64_t)kSlots * MIST_LC_TILE;
-  // cheapest seed of the stage's (l, c) cells, c = 0..c_last, in slot `slot` of p tile `p_tile`
-  auto cheapest = [&](int slot, int p_tile, int c_last) {
+  const int l = L / S, P = g->num_p;
+  // seed of the stage's (l, c) cell in slot `slot` (one sample: bits of +inf where there is none)
+  auto seed_of = [&](int slot, int c) {
+    const int pair = l * (l + 1) / 2 - 1 + c;
+    const int lc_tile = pair / MIST_LC_TILE - g->lc_tile_begin;
+    if (lc_tile < 0 || lc_tile >= g->n_lc_tiles) return (double)INFINITY;
+    return cost_of_bits(tabs.best[g->cell_offset +
+                                  ((int64_t)lc_tile * MIST_LC_TILE + pair % MIST_LC_TILE) * slots_of(P) + slot]);
+  };
+  // cheapest one over c = 0..c_last
+  auto cheapest = [&](int slot, int c_last) {
     double best = INFINITY;
-    for (int c = threadIdx.x & 63; c <= c_last; c += 64) {
-      const int pair = l * (l + 1) / 2 - 1 + c;
-      const int lc_tile = pair / MIST_LC_TILE - g->lc_tile_begin;
-      if (lc_tile < 0 || lc_tile >= g->n_lc_tiles) continue;
-      const int64_t at = (scout_base + scout_prefix[blockIdx.x] +
-                          (int64_t)(lc_tile * g->n_p_tiles + p_tile) * kScoutSplit) * slab +
-                         slot * MIST_LC_TILE + pair % MIST_LC_TILE;
-      if (partial_index[at] >= 0) best = fmin(best, partial_cost[at]);
-    }
+    for (int c = threadIdx.x & 63; c <= c_last; c += 64) best = fmin(best, seed_of(slot, c));
     for (int step = 32; step > 0; step >>= 1) best = fmin(best, __shfl_xor(best, step));
     return best;
   };
@@ -1894,28 +2298,12 @@ __global__ __launch_bounds__(64 * kIncumbentWaves) void incumbent_kernel(
   for (int s = wave; s < S; s += kIncumbentWaves) {
     const int p = S - 1 - s, end_layer = (s + 1) * l - 1;
     int slot;
-    if (S == 1) slot = 2 * MIST_P_TILE + 1;
-    else if (s == 0) slot = MIST_P_TILE + p % MIST_P_TILE;
-    else if (s == S - 1) slot = 2 * MIST_P_TILE;
-    else slot = p % MIST_P_TILE;
-    const int p_tile = (S == 1 || s == S - 1) ? 0 : p / MIST_P_TILE;
-    double cost;
-    if (prob.incumbent_ckpt_rule == 2) {  // every layer of the stage checkpointed
-      cost = INFINITY;
-      if ((threadIdx.x & 63) == 0) {
-        const int pair = l * (l + 1) / 2 - 1 + l;
-        const int lc_tile = pair / MIST_LC_TILE - g->lc_tile_begin;
-        if (lc_tile >= 0 && lc_tile < g->n_lc_tiles) {
-          const int64_t at = (scout_base + scout_prefix[blockIdx.x] +
-                              (int64_t)(lc_tile * g->n_p_tiles + p_tile) * kScoutSplit) * slab +
-                             slot * MIST_LC_TILE + pair % MIST_LC_TILE;
-          if (partial_index[at] >= 0) cost = partial_cost[at];
-        }
-      }
-      cost = __shfl(cost, 0);
-    } else {
-      cost = cheapest(slot, p_tile, c_last_of(end_layer));
-    }
+    if (S == 1) slot = 2 * P + 1;
+    else if (s == 0) slot = P + p;
+    else if (s == S - 1) slot = 2 * P;
+    else slot = p;
+    // (rule 2: every layer of the stage checkpointed)
+    const double cost = prob.incumbent_ckpt_rule == 2 ? seed_of(slot, l) : cheapest(slot, c_last_of(end_layer));
     sum += cost;
     largest = fmax(largest, cost);
   }
@@ -1946,28 +2334,23 @@ __global__ __launch_bounds__(64 * kIncumbentWaves) void incumbent_kernel(
 // with_pre tables), and keeps per stage of the pipeline the cheapest feasible cost.  Minima over
 // fewer rows than the scout pass sees, so the estimate is no smaller than the scout's.
 // Grid (kEstimateSplit, group); workgroup k writes its S minima to doubles [k S, (k + 1) S) of
-// the group's first scout slab (free until the scout pass writes it).
+// the group's minima (the seed launch fills them afterwards).
 constexpr int kEstimateSplit = 16;
 constexpr int kEstimateRows = 1024;
 constexpr int kEstimateMaxStages = 256;
-static_assert(kEstimateSplit * kEstimateMaxStages <= kScoutSplit * kSlots * MIST_LC_TILE,
-              "the partial minima of a group fit the scout slabs of one tile");
-__device__ __forceinline__ bool estimate_runs(const MistProblem &prob, const MistGroupDesc *g,
-                                              const int32_t *__restrict__ scout_prefix, int gi,
-                                              int *stages) {
-  if (g->scout_stride <= 0 || scout_prefix[gi + 1] - scout_prefix[gi] < kScoutSplit) return false;
+static_assert(kEstimateSplit <= MIST_LC_TILE, "S <= num_p: the partial minima of a group fit one tile of its minima");
+__device__ __forceinline__ bool estimate_runs(const MistProblem &prob, const MistGroupDesc *g, int *stages) {
+  if (g->scout_stride <= 0) return false;
   *stages = incumbent_stage_count(prob, g);
   return *stages > 0 && *stages <= kEstimateMaxStages;
 }
 
 __global__ __launch_bounds__(256) void estimate_stage_minima_kernel(
     const MistProblem prob, const MistGroupDesc *__restrict__ groups,
-    const int32_t *__restrict__ scout_prefix, int64_t scout_base,
     const double *__restrict__ row_terms, double ratio, double *__restrict__ partial_cost) {
-  const int gi = (int)blockIdx.y;
-  const MistGroupDesc *g = groups + gi;
+  const MistGroupDesc *g = groups + blockIdx.y;
   int S;
-  if (!estimate_runs(prob, g, scout_prefix, gi, &S)) return;
+  if (!estimate_runs(prob, g, &S)) return;
   const int L = prob.num_layers, l = L / S, rule = prob.incumbent_ckpt_rule;
   __shared__ unsigned long long stage_min[kEstimateMaxStages];
   const unsigned long long kInf = (unsigned long long)__double_as_longlong((double)INFINITY);
@@ -2028,8 +2411,7 @@ __global__ __launch_bounds__(256) void estimate_stage_minima_kernel(
       offer(st, c <= c_last(st) && mem.feasible_base(S - 1 - st, cap), cost_base);
   }
   __syncthreads();
-  const int64_t slab = (int64_t)kSlots * MIST_LC_TILE;
-  double *out = partial_cost + (scout_base + scout_prefix[gi]) * slab + (int64_t)blockIdx.x * S;
+  double *out = partial_cost + g->cell_offset + (int64_t)blockIdx.x * S;
   for (int st = threadIdx.x; st < S; st += blockDim.x)
     out[st] = __longlong_as_double((long long)stage_min[st]);
 }
@@ -2037,14 +2419,11 @@ __global__ __launch_bounds__(256) void estimate_stage_minima_kernel(
 // Sum of a group's stage minima + (G - 1) x the largest (inter_tuning.py:342) into *incumbent.
 __global__ __launch_bounds__(64) void estimate_combine_kernel(
     const MistProblem prob, const MistGroupDesc *__restrict__ groups,
-    const int32_t *__restrict__ scout_prefix, int64_t scout_base,
     const double *__restrict__ partial_cost) {
-  const int gi = (int)blockIdx.x;
-  const MistGroupDesc *g = groups + gi;
+  const MistGroupDesc *g = groups + blockIdx.x;
   int S;
-  if (!estimate_runs(prob, g, scout_prefix, gi, &S)) return;
-  const int64_t slab = (int64_t)kSlots * MIST_LC_TILE;
-  const double *in = partial_cost + (scout_base + scout_prefix[gi]) * slab;
+  if (!estimate_runs(prob, g, &S)) return;
+  const double *in = partial_cost + g->cell_offset;
   double sum = 0.0, largest = 0.0;
   for (int st = threadIdx.x; st < S; st += 64) {
     double best = INFINITY;
@@ -2062,117 +2441,185 @@ __global__ __launch_bounds__(64) void estimate_combine_kernel(
               (unsigned long long)__double_as_longlong(total));
 }
 
-// Combines the slabs of the kScoutSplit scout workgroups of every tile into the first of them,
-// so that each chunk of the main launch reads one slab of seeds instead of kScoutSplit.
-// Workgroup = tile; the scout slabs of tile t are scout_base + t * kScoutSplit + k.
-__global__ __launch_bounds__(256) void merge_scout_kernel(int64_t scout_base, int n_scout_total,
-                                                          double *__restrict__ partial_cost,
-                                                          int32_t *__restrict__ partial_index) {
+// Combines the chunk slabs of the evaluate-every-cell kernel into the minima tables (one sample):
+// thread = (pair of a tile, slot of a p tile).
+__global__ __launch_bounds__(256) void combine_slabs_kernel(
+    const MistGroupDesc *__restrict__ groups, const int32_t *__restrict__ block_prefix,
+    const double *__restrict__ slab_cost, const int32_t *__restrict__ slab_index, const ReduceTables tabs) {
+  const int gi = blockIdx.y;
+  const MistGroupDesc *g = groups + gi;
+  const int n_tiles = g->n_lc_tiles * g->n_p_tiles, P = g->num_p;
   const int64_t slab = (int64_t)kSlots * MIST_LC_TILE;
-  const int64_t first = (scout_base + (int64_t)blockIdx.y * n_scout_total +
-                         (int64_t)blockIdx.x * kScoutSplit) * slab;
-  for (int e = threadIdx.x; e < (int)slab; e += blockDim.x) {
-    double best = INFINITY;
-    int32_t best_row = -1;
-    for (int k = 0; k < kScoutSplit; ++k) {
-      const int32_t row = partial_index[first + k * slab + e];
-      take_min(best, best_row, row >= 0, partial_cost[first + k * slab + e], row);
+  for (int tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
+    const int p_tile = tile % g->n_p_tiles, tile_rel = tile / g->n_p_tiles, p0 = p_tile * MIST_P_TILE;
+    for (int e = threadIdx.x; e < (int)slab; e += blockDim.x) {
+      const int kslot = e / MIST_LC_TILE, lane = e % MIST_LC_TILE, p = p0 + kslot % MIST_P_TILE;
+      int slot;
+      if (kslot >= 2 * MIST_P_TILE) {
+        if (p_tile != 0) continue;
+        slot = 2 * P + (kslot - 2 * MIST_P_TILE);
+      } else if (p >= P) {
+        continue;
+      } else {
+        slot = kslot < MIST_P_TILE ? p : P + p;
+      }
+      double best = INFINITY;
+      int32_t best_row = -1;
+      for (int ch = 0; ch < g->n_chunks; ++ch) {
+        const int64_t at = ((int64_t)block_prefix[gi] + (int64_t)ch * n_tiles + tile) * slab + e;
+        const int32_t row = slab_index[at];
+        take_min(best, best_row, row >= 0, slab_cost[at], row);
+      }
+      const int64_t cell = g->cell_offset + ((int64_t)tile_rel * MIST_LC_TILE + lane) * slots_of(P) + slot;
+      tabs.best[cell] = (unsigned long long)__double_as_longlong(best);
+      tabs.row[cell] = (uint32_t)best_row;
     }
-    partial_cost[first + e] = best;
-    partial_index[first + e] = best_row;
   }
 }
 
 // ------------------------------------------------------------------------------------------
-// Kernel 3: combine the chunks' (cost, row) minima, recompute the winner's stable / delta, scatter.
-// One thread per (group, (l, c) pair, slot); slots as in the reduce kernel but over all p.
+// Kernel 3: recompute the winners' stable / delta, scatter into the output tables.  The reduction
+// left each row's cost at the slot of its own count: a p's winner is the lexicographic minimum of
+// (cost, row) over the slots from it up.  Neighbouring p mostly share it, so a thread goes down the
+// slots and reads and prices a winner's terms once.
 // ------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void finalize_kernel(
-    const MistProblem prob, const MistGroupDesc *__restrict__ groups, int n_groups,
-    const int32_t *__restrict__ block_prefix, const double *__restrict__ row_terms,
-    const double *__restrict__ partial_cost, const int32_t *__restrict__ partial_index,
-    const SampleSlots samples, int n_blocks, MistOutTables tables) {
-  const int L = prob.num_layers;
-  const int n_pairs = L * (L + 1) / 2 + L;
-  const int gi = blockIdx.z;
-  const MistGroupDesc *g = groups + gi;
-  // blockIdx.x = (sample of the launch, block of 256 pairs); the slabs of the launch's m-th
-  // sample start at slab m * n_blocks
-  const int pair_blocks = (n_pairs + (int)blockDim.x - 1) / (int)blockDim.x;
-  const int m = blockIdx.x / pair_blocks;
-  const int sample_index = samples.at[m];
-  const int pair_idx = (blockIdx.x - m * pair_blocks) * blockDim.x + threadIdx.x;
-  // blockIdx.y: 0..p_dim-1 base, p_dim..2*p_dim-1 with_pre, 2*p_dim with_post, 2*p_dim+1 no_pp
-  const int P1 = prob.p_dim;
-  const int slot = blockIdx.y;
-  int variant, p;
-  if (slot < P1) { variant = 0; p = slot; }
-  else if (slot < 2 * P1) { variant = 1; p = slot - P1; }
-  else { variant = 2 + (slot - 2 * P1); p = 0; }
-  if (p >= g->num_p) return;
-  // A wavefront = the 64 pairs of one tile (the workgroup starts at a multiple of 256 pairs):
-  // what follows up to the chunk loop is the same for all its lanes.  The group's tiles are a
-  // window of the pair list; cells outside were not evaluated.
-  const int lc_tile = pair_idx / MIST_LC_TILE - g->lc_tile_begin, lane = pair_idx % MIST_LC_TILE;
-  if (lc_tile < 0 || lc_tile >= g->n_lc_tiles) return;
-  const PairIndex pc = decode_pair(min(pair_idx, n_pairs - 1));
-  const int l = pc.l, c = pc.c;
+// One (group, pair, variant) of the output.
+struct FinalCell {
+  double stable, delta;
+  uint32_t priced;  // row they are of
+  int64_t at, plane;  // element of p == 0, elements between p
   // Cells the reference never writes (batched_module_analyzer.py:3021-3023 rebinds the layer
   // mask inside the p == 0 branch, so it also governs base / with_pre for p >= 1; :3103).
-  const bool written = pair_idx < n_pairs && !(variant <= 1 && p >= 1 && c == l - 1) &&
-                       !(variant == 2 && c == l - 1) && !(variant == 3 && (l != L || c == L - 1));
-  const int p_tile = p / MIST_P_TILE;
-  int kslot;
-  if (variant == 0) kslot = p % MIST_P_TILE;
-  else if (variant == 1) kslot = MIST_P_TILE + p % MIST_P_TILE;
-  else kslot = 2 * MIST_P_TILE + (variant - 2);
-  const int n_tiles = g->n_lc_tiles * g->n_p_tiles;
-  const int64_t first_block =
-      (int64_t)m * n_blocks + (int64_t)block_prefix[gi] + (lc_tile * g->n_p_tiles + p_tile);
-  double best = INFINITY;
-  int32_t best_row = -1;
-  // Most chunks leave their seeds as they are and write a mark instead of a slab: the marks of
-  // 64 chunks are read at once, a lane each, and only the slabs that were written are visited
-  // (in chunk order, as a walk over all chunks would).
-  for (int ch0 = 0; ch0 < g->n_chunks; ch0 += 64) {
-    const int ch_mine = ch0 + (int)(threadIdx.x & 63);
-    bool has_slab = false;
-    if (ch_mine < g->n_chunks)
-      has_slab = ch_mine == 0 ||
-                 partial_index[(first_block + (int64_t)ch_mine * n_tiles) * kSlots * MIST_LC_TILE] !=
-                     kSlabUnchanged;
-    unsigned long long todo = __ballot(has_slab);
-    while (todo != 0) {
-      const int ch = ch0 + __ffsll(todo) - 1;
-      todo &= todo - 1;
-      const int64_t at = (first_block + (int64_t)ch * n_tiles) * kSlots * MIST_LC_TILE +
-                         (int64_t)kslot * MIST_LC_TILE + lane;
-      const double cost = partial_cost[at];
-      const int32_t row = partial_index[at];
-      take_min(best, best_row, row >= 0, cost, row);
+  int n_p;  // values of p written
+};
+__device__ __forceinline__ FinalCell final_cell(const MistProblem &prob, const MistGroupDesc *__restrict__ g, int variant,
+                                                PairIndex pc, int sample_at) {
+  const int L = prob.num_layers, P1 = prob.p_dim, S = prob.sample_size, l = pc.l, c = pc.c;
+  const int64_t gq = (int64_t)g->g_index * prob.num_mesh + g->q_index;
+  FinalCell f;
+  f.stable = f.delta = INFINITY;
+  f.priced = ~0u;
+  f.plane = (int64_t)L * (L + 1) * S;
+  f.at = (variant == 3 ? gq * (L + 1) + c : ((variant < 2 ? gq * P1 : gq) * L + (l - 1)) * (L + 1) + c) * S + sample_at;
+  f.n_p = variant < 2 ? (c == l - 1 ? 1 : g->num_p) : variant == 2 ? c != l - 1 : l == L && c != L - 1;
+  return f;
+}
+__device__ __forceinline__ void write_final(FinalCell &f, const MistGroupDesc *__restrict__ g, int variant, PairIndex pc,
+                                            const GroupConsts &k, const double *__restrict__ row_terms, uint32_t row,
+                                            int p, const MistOutTables &tables) {
+  if (row != f.priced) {
+    const double *t = row_terms + (g->row_offset + position_of_row(g, (int32_t)row)) * MIST_ROW_TERMS;
+    const CellLatency lat = cell_latency<true>(t, pc.l, pc.c, k);
+    if (variant == 0) { f.stable = (double)lat.x; f.delta = (double)lat.d; }
+    else if (variant == 1) { f.stable = lat.sp; f.delta = lat.dpre; }
+    else if (variant == 2) { f.stable = lat.spost; f.delta = lat.dpost; }
+    else { f.stable = lat.spp; f.delta = lat.dpp; }
+    f.priced = row;
+  }
+  const int64_t at = f.at + p * f.plane;
+  tables.stable[variant][at] = f.stable;
+  tables.delta[variant][at] = f.delta;
+  tables.index[variant][at] = (int32_t)row;
+}
+// (row as left by the reduction: ~0 none)
+__device__ __forceinline__ void take_lower(unsigned long long &cost, uint32_t &row, unsigned long long its_cost,
+                                           uint32_t its_row) {
+  row = its_cost < cost ? its_row : its_cost == cost ? min(row, its_row) : row;
+  cost = min(cost, its_cost);
+}
+__device__ __forceinline__ uint32_t row_number(uint32_t held) { return held == ~0u ? held : held & ~kUnresolved; }
+
+// One sample: workgroup = (tile, variant, group).  The slots of a pair lie side by side, the tables'
+// last axis is c: kFinalSlots slots at a time are read with lane = (pair parity, slot), scanned, and
+// left in LDS for the wavefronts to write with lane = pair.  (A thread per pair and variant that
+// walked the slots in memory: 3.6 ms for the 70B plan on 256 GPUs, a line per read.)
+constexpr int kFinalSlots = 32;
+__global__ __launch_bounds__(256) void finalize_kernel(
+    const MistProblem prob, const MistGroupDesc *__restrict__ groups, const double *__restrict__ row_terms,
+    const ReduceTables tabs, int sample_at, MistOutTables tables) {
+  __shared__ uint32_t winner[MIST_LC_TILE][kFinalSlots + 1];
+  __shared__ unsigned long long carry_cost[MIST_LC_TILE];
+  __shared__ uint32_t carry_row[MIST_LC_TILE];
+  const int L = prob.num_layers, n_pairs = L * (L + 1) / 2 + L;
+  const MistGroupDesc *g = groups + blockIdx.z;
+  const int tile_rel = blockIdx.x, variant = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (tile_rel >= g->n_lc_tiles) return;
+  const int P = variant < 2 ? g->num_p : 1, n_slots = slots_of(g->num_p);
+  const int first_pair = (g->lc_tile_begin + tile_rel) * MIST_LC_TILE;
+  const bool active = first_pair + lane < n_pairs;
+  const PairIndex pc = decode_pair(active ? first_pair + lane : 0);
+  FinalCell f = final_cell(prob, g, variant, pc, sample_at);
+  if (!active) f.n_p = 0;
+  const GroupConsts k = group_consts(g);
+  const int64_t first = g->cell_offset + (int64_t)tile_rel * MIST_LC_TILE * n_slots +
+                        (variant < 2 ? variant * P : 2 * g->num_p + variant - 2);
+  if (threadIdx.x < MIST_LC_TILE) {
+    carry_cost[threadIdx.x] = ~0ull;
+    carry_row[threadIdx.x] = ~0u;
+  }
+  for (int p0 = (P - 1) / kFinalSlots * kFinalSlots; p0 >= 0; p0 -= kFinalSlots) {
+    __syncthreads();
+    const int j = lane % kFinalSlots, p = p0 + j;
+#pragma unroll 2
+    for (int pair = wave * 2 + lane / kFinalSlots; pair < MIST_LC_TILE; pair += 8) {
+      const PairIndex its = decode_pair(min(first_pair + pair, n_pairs - 1));
+      const int np = its.c == its.l - 1 ? 1 : P;  // (later slots hold no minima)
+      const int64_t cell = first + (int64_t)pair * n_slots + p;
+      unsigned long long cost = ~0ull;
+      uint32_t row = ~0u;
+      if (p < np) {
+        cost = tabs.best[cell];
+        row = row_number(tabs.row[cell]);
+      }
+      for (int step = 1; step < kFinalSlots; step <<= 1) {
+        const unsigned long long its_cost = __shfl_down(cost, step, kFinalSlots);
+        const uint32_t its_row = __shfl_down(row, step, kFinalSlots);
+        if (j + step < kFinalSlots) take_lower(cost, row, its_cost, its_row);
+      }
+      take_lower(cost, row, carry_cost[pair], carry_row[pair]);
+      winner[pair][j] = row;
+      if (j == 0) {
+        carry_cost[pair] = cost;
+        carry_row[pair] = row;
+      }
+    }
+    __syncthreads();
+    for (int q = kFinalSlots / 4 - 1; q >= 0; --q) {
+      const int slot = wave * (kFinalSlots / 4) + q;
+      if (p0 + slot < f.n_p) write_final(f, g, variant, pc, k, row_terms, winner[lane][slot], p0 + slot, tables);
     }
   }
-  if (!written) return;
+}
 
-  double stable = INFINITY, delta = INFINITY;
-  if (best_row >= 0) {
-    const double *t = row_terms + (g->row_offset + position_of_row(g, best_row)) * MIST_ROW_TERMS;
-    const CellLatency lat = cell_latency<true>(t, l, c, group_consts(g));
-    if (variant == 0) { stable = (double)lat.x; delta = (double)lat.d; }
-    else if (variant == 1) { stable = lat.sp; delta = lat.dpre; }
-    else if (variant == 2) { stable = lat.spost; delta = lat.dpost; }
-    else { stable = lat.spp; delta = lat.dpp; }
+// Several samples (a slot's lie side by side, as in the tables): one thread per (group, pair,
+// sample, variant, kFinalRange values of p).
+constexpr int kFinalRange = 16;
+__global__ __launch_bounds__(256) void finalize_samples_kernel(
+    const MistProblem prob, const MistGroupDesc *__restrict__ groups, const double *__restrict__ row_terms,
+    const ReduceTables tabs, const SampleSlots samples, MistOutTables tables) {
+  const int L = prob.num_layers, n_pairs = L * (L + 1) / 2 + L;
+  const MistGroupDesc *g = groups + blockIdx.z;
+  const int P = g->num_p, n = tabs.n_samples;
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  const int s = e % n, pair_rel = e / n;
+  // blockIdx.y: ranges of p of base, then of with_pre; with_post; no_pp
+  const int ranges = (prob.p_dim + kFinalRange - 1) / kFinalRange, part = blockIdx.y;
+  const int variant = part < ranges ? 0 : part < 2 * ranges ? 1 : 2 + (part - 2 * ranges);
+  const int p_begin = variant < 2 ? part % ranges * kFinalRange : 0;
+  // The group's tiles are a window of the pair list; cells outside were not evaluated.
+  const int pair_idx = g->lc_tile_begin * MIST_LC_TILE + pair_rel;
+  if (pair_rel >= g->n_lc_tiles * MIST_LC_TILE || pair_idx >= n_pairs) return;
+  const PairIndex pc = decode_pair(pair_idx);
+  FinalCell f = final_cell(prob, g, variant, pc, samples.at[s]);
+  const int64_t first = (g->cell_offset + (int64_t)pair_rel * slots_of(P) +
+                         (variant < 2 ? variant * P : 2 * P + variant - 2)) * n + s;
+  const GroupConsts k = group_consts(g);
+  unsigned long long cost = ~0ull;
+  uint32_t row = ~0u;
+  for (int p = f.n_p - 1; p >= p_begin; --p) {
+    take_lower(cost, row, tabs.best[first + (int64_t)p * n], row_number(tabs.row[first + (int64_t)p * n]));
+    if (p < p_begin + kFinalRange) write_final(f, g, variant, pc, k, row_terms, row, p, tables);
   }
-
-  const int S = prob.sample_size;
-  const int64_t gq = (int64_t)g->g_index * prob.num_mesh + g->q_index;
-  int64_t at;
-  if (variant <= 1) at = (((gq * P1 + p) * L + (l - 1)) * (L + 1) + c) * S + sample_index;
-  else if (variant == 2) at = ((gq * L + (l - 1)) * (L + 1) + c) * S + sample_index;
-  else at = (gq * (L + 1) + c) * S + sample_index;
-  tables.stable[variant][at] = stable;
-  tables.delta[variant][at] = delta;
-  tables.index[variant][at] = best_row;
 }
 
 // ------------------------------------------------------------------------------------------
@@ -2447,52 +2894,157 @@ int64_t mist_stage_floor_doubles(int64_t total_rows, int n_groups) {
   return (total_rows / kStageRows + n_groups + 1) * kStageFloorPitch;
 }
 
-static int launch_first_estimate(const MistProblem *problem, const MistGroupDesc *d_groups,
-                                 int n_groups, const int32_t *scout_prefix, int64_t scout_base,
+// Sections of the reduce workspace in `d_partial_cost` (doubles): the minima of n_samples samples,
+// the second-level summaries, the three item arrays, the queue's counters and a word per pair.
+struct WorkspaceLayout {
+  int64_t best, supers, items, counters, changed, total;
+  int64_t capacity;  // items per shard
+};
+static WorkspaceLayout workspace_layout(int64_t cells, int64_t supers, int64_t items, int n_samples) {
+  WorkspaceLayout w;
+  w.capacity = (items + kQueueShards - 1) / kQueueShards + 1;
+  w.best = 0;
+  w.supers = cells * n_samples;
+  w.items = w.supers + supers * kStageFloorPitch;
+  w.counters = w.items + 3 * kQueueShards * w.capacity;
+  w.changed = w.counters + kCounters * kCounterPitch / 2;
+  w.total = w.changed + cells / 8 + 1;
+  return w;
+}
+int64_t mist_reduce_workspace_doubles(int64_t cells, int64_t supers, int64_t items, int n_samples) {
+  if (cells < 0 || supers < 0 || items < 0 || n_samples < 1) return -1;
+  return workspace_layout(cells, supers, items, n_samples).total;
+}
+static int reduce_tables(const MistProblem *problem, int n_samples, double *d_partial_cost, int32_t *d_partial_index,
+                         ReduceTables *out) {
+  if (problem->reduce_cells < 1 || problem->reduce_supers < 1 || problem->reduce_items < 1 ||
+      problem->reduce_max_p < 1)
+    return fail(MIST_E_INVALID, "MistProblem.reduce_* sizes of the workspace are not set");
+  const WorkspaceLayout w =
+      workspace_layout(problem->reduce_cells, problem->reduce_supers, problem->reduce_items, n_samples);
+  if (w.capacity >= (int64_t)1 << 31) return fail(MIST_E_INVALID, "too many (tile, stage) items");
+  out->best = reinterpret_cast<unsigned long long *>(d_partial_cost + w.best);
+  out->row = reinterpret_cast<uint32_t *>(d_partial_index);
+  out->super_floor = d_partial_cost + w.supers;
+  out->item = reinterpret_cast<unsigned long long *>(d_partial_cost + w.items);
+  out->opened = out->item + kQueueShards * w.capacity;
+  out->hit = out->opened + kQueueShards * w.capacity;
+  out->counter = reinterpret_cast<uint32_t *>(d_partial_cost + w.counters);
+  out->changed = reinterpret_cast<uint32_t *>(d_partial_cost + w.changed);
+  out->capacity = (uint32_t)w.capacity;
+  out->n_samples = n_samples;
+  return 0;
+}
+
+static int launch_first_estimate(const MistProblem *problem, const MistGroupDesc *d_groups, int n_groups,
                                  const double *d_row_terms, double ratio, double *d_partial_cost,
                                  void *stream) {
   hipLaunchKernelGGL(estimate_stage_minima_kernel, dim3(kEstimateSplit, n_groups), dim3(256), 0,
-                     (hipStream_t)stream, *problem, d_groups, scout_prefix, scout_base, d_row_terms,
-                     ratio, d_partial_cost);
+                     (hipStream_t)stream, *problem, d_groups, d_row_terms, ratio, d_partial_cost);
   MIST_HIP_CHECK(hipGetLastError());
   hipLaunchKernelGGL(estimate_combine_kernel, dim3(n_groups), dim3(64), 0, (hipStream_t)stream,
-                     *problem, d_groups, scout_prefix, scout_base, d_partial_cost);
+                     *problem, d_groups, d_partial_cost);
   MIST_HIP_CHECK(hipGetLastError());
   return 0;
 }
 
-// Scout launch + slab merge for n_samples ratios at once (grid.y = sample).
-static int launch_scout(const MistProblem *problem, const MistGroupDesc *d_groups, int n_groups,
-                        const int32_t *d_block_prefix, int n_blocks, const int32_t *scout_prefix,
-                        int n_scout_blocks, const double *d_row_terms, const double *d_stage_floor,
-                        const RatioList &ratios, int n_samples, int64_t scout_base,
-                        double *d_partial_cost, int32_t *d_partial_index, void *stream) {
-  if (n_scout_blocks % kScoutSplit != 0)
-    return fail(MIST_E_INVALID, "n_scout_blocks %d is not a multiple of the scout split %d",
-                n_scout_blocks, kScoutSplit);
-  if (problem->stage_cost_incumbent != nullptr && problem->incumbent_first_estimate != 0 &&
-      n_samples == 1 && n_groups <= 65535)
-    // a first estimate from a few rows, so that the scout pass itself runs under a bound
-    if (int rc = launch_first_estimate(problem, d_groups, n_groups, scout_prefix, scout_base,
-                                       d_row_terms, ratios.r[0], d_partial_cost, stream))
+// More than 64 KB of LDS per workgroup needs an opt-in, once per device.
+static int allow_large_lds() {
+  static std::mutex lock;
+  static bool done[64];
+  int device = 0;
+  MIST_HIP_CHECK(hipGetDevice(&device));
+  if (device < 0 || device >= 64) return fail(MIST_E_INVALID, "device ordinal %d outside [0, 64)", device);
+  std::lock_guard<std::mutex> guard(lock);
+  if (!done[device]) {
+    for (const void *kernel : {reinterpret_cast<const void *>(seed_kernel),
+                               reinterpret_cast<const void *>(seed_samples_kernel),
+                               reinterpret_cast<const void *>(reduce_kernel<false, false>),
+                               reinterpret_cast<const void *>(reduce_kernel<true, false>)})
+      MIST_HIP_CHECK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kSeedLdsMost));
+    done[device] = true;
+  }
+  return 0;
+}
+
+// Minima tables filled with what the rows of the scout pairs give (+inf where a group has none),
+// and the estimate of the best pipeline cost they allow.
+static int launch_seeds(const MistProblem *problem, const MistGroupDesc *d_groups, int n_groups,
+                        const double *d_row_terms, const RatioList &ratios, bool scouted,
+                        const ReduceTables &tabs, double *d_partial_cost, void *stream) {
+  if (scouted && problem->stage_cost_incumbent != nullptr && problem->incumbent_first_estimate != 0 &&
+      tabs.n_samples == 1)
+    // a first estimate from a few rows, so that the seed launch itself runs under a bound
+    if (int rc = launch_first_estimate(problem, d_groups, n_groups, d_row_terms, ratios.r[0], d_partial_cost, stream))
       return rc;
-  hipLaunchKernelGGL(eval_reduce_kernel, dim3(xcd_padded_grid(n_scout_blocks), n_samples),
-                     dim3(MIST_LC_TILE), 0, (hipStream_t)stream, *problem, d_groups, n_groups,
-                     d_block_prefix, n_blocks, scout_prefix, 1, d_row_terms, d_stage_floor, ratios,
-                     0, scout_base, d_partial_cost, d_partial_index);
+  const int L = problem->num_layers, n_pairs = L * (L + 1) / 2 + L;
+  const int tiles = (n_pairs + MIST_LC_TILE - 1) / MIST_LC_TILE;
+  if (tiles > 65535) return fail(MIST_E_INVALID, "at most 65535 tiles of (l, c) pairs, got %d", tiles);
+  const int64_t pair_bytes = 8 * (int64_t)slots_of(problem->reduce_max_p);
+  // fewer pairs, or samples, per workgroup when the slots are many, so that several stay resident
+  int pair_split = tabs.n_samples == 1 ? 16 : 1;
+  while (pair_split > 1 && pair_split * pair_bytes > kSeedLdsBytes) pair_split /= 2;
+  int sample_split = tabs.n_samples;
+  while (sample_split > 1 && pair_bytes * sample_split > kSeedLdsBytes) sample_split = (sample_split + 1) / 2;
+  const int64_t bytes =
+      pair_bytes * pair_split * sample_split + (tabs.n_samples == 1 ? 0 : (int64_t)sizeof(SampleRows));
+  if (bytes > kSeedLdsMost) return fail(MIST_E_INVALID, "%d pre-saved micro-batch values exceed the LDS", problem->reduce_max_p);
+  if (bytes > 64 * 1024)
+    if (int rc = allow_large_lds()) return rc;
+  const dim3 grid(tiles * (MIST_LC_TILE / pair_split), n_groups,
+                  (tabs.n_samples + sample_split - 1) / sample_split);
+  if (tabs.n_samples == 1)
+    hipLaunchKernelGGL(seed_kernel, grid, dim3(kSeedThreads), (size_t)bytes, (hipStream_t)stream, *problem, d_groups,
+                       d_row_terms, ratios.r[0], tabs, pair_split);
+  else
+    hipLaunchKernelGGL(seed_samples_kernel, grid, dim3(64), (size_t)bytes, (hipStream_t)stream, *problem, d_groups,
+                       d_row_terms, ratios, tabs, sample_split);
   MIST_HIP_CHECK(hipGetLastError());
-  if (kScoutSplit > 1) {
-    hipLaunchKernelGGL(merge_scout_kernel, dim3(n_scout_blocks / kScoutSplit, n_samples), dim3(256),
-                       0, (hipStream_t)stream, scout_base, n_scout_blocks, d_partial_cost,
-                       d_partial_index);
+  if (scouted && problem->stage_cost_incumbent != nullptr && tabs.n_samples == 1) {
+    hipLaunchKernelGGL(incumbent_kernel, dim3(n_groups), dim3(64 * kIncumbentWaves), 0, (hipStream_t)stream, *problem,
+                       d_groups, tabs);
     MIST_HIP_CHECK(hipGetLastError());
   }
-  if (problem->stage_cost_incumbent != nullptr && n_samples == 1) {
-    hipLaunchKernelGGL(incumbent_kernel, dim3(n_groups), dim3(64 * kIncumbentWaves), 0,
-                       (hipStream_t)stream, *problem,
-                       d_groups, scout_prefix, scout_base, d_partial_cost, d_partial_index);
+  return 0;
+}
+
+static int launch_super_floors(const MistGroupDesc *d_groups, int n_groups, const double *d_stage_floor,
+                               const ReduceTables &tabs, void *stream) {
+  hipLaunchKernelGGL(super_floor_kernel, dim3(kSuperBlocks, n_groups), dim3(256), 0, (hipStream_t)stream, d_groups,
+                     n_groups, d_stage_floor, tabs.super_floor);
+  MIST_HIP_CHECK(hipGetLastError());
+  return 0;
+}
+
+// filter + open + reduce + resolve on seeded tables.
+static int launch_reduce(const MistProblem *problem, const MistGroupDesc *d_groups, int n_groups,
+                         const int32_t *d_block_prefix, int n_blocks, const double *d_row_terms,
+                         const double *d_stage_floor, const RatioList &ratios, const ReduceTables &tabs, void *stream) {
+  hipLaunchKernelGGL(filter_kernel, dim3(xcd_padded_grid(n_blocks)), dim3(MIST_LC_TILE), 0, (hipStream_t)stream,
+                     *problem, d_groups, n_groups, d_block_prefix, n_blocks, d_stage_floor, tabs.super_floor, ratios, tabs);
+  MIST_HIP_CHECK(hipGetLastError());
+  hipLaunchKernelGGL(open_kernel, dim3(kReduceBlocks), dim3(kReduceThreads), 0, (hipStream_t)stream, *problem,
+                     d_groups, d_stage_floor, ratios, tabs);
+  MIST_HIP_CHECK(hipGetLastError());
+  const int row_pitch = slots_of(problem->reduce_max_p);
+  const size_t lds = tabs.n_samples == 1 ? sizeof(double) * row_pitch * (kReduceThreads / 64) : 0;
+  if (lds > kSeedLdsMost) return fail(MIST_E_INVALID, "%d pre-saved micro-batch values exceed the LDS", problem->reduce_max_p);
+  if (lds > 64 * 1024)
+    if (int rc = allow_large_lds()) return rc;
+#define MIST_REDUCE(RESOLVE, SAMPLES)                                                                       \
+  hipLaunchKernelGGL((reduce_kernel<RESOLVE, SAMPLES>), dim3(kReduceBlocks), dim3(kReduceThreads), lds,     \
+                     (hipStream_t)stream, *problem, d_groups, d_row_terms, d_stage_floor, ratios, tabs, row_pitch)
+  if (tabs.n_samples == 1) {
+    MIST_REDUCE(false, false);
     MIST_HIP_CHECK(hipGetLastError());
+    MIST_REDUCE(true, false);
+  } else {
+    MIST_REDUCE(false, true);
+    MIST_HIP_CHECK(hipGetLastError());
+    MIST_REDUCE(true, true);
   }
+#undef MIST_REDUCE
+  MIST_HIP_CHECK(hipGetLastError());
   return 0;
 }
 
@@ -2508,6 +3060,7 @@ static int check_reduce_arguments(const MistProblem *problem, const MistGroupDes
   if (n_scout_blocks < 0 || (n_scout_blocks > 0 && !d_scout_prefix))
     return fail(MIST_E_INVALID, "scout blocks need a scout prefix (n_scout_blocks=%d)",
                 n_scout_blocks);
+  if (n_groups > 65535) return fail(MIST_E_INVALID, "at most 65535 groups per call, got %d", n_groups);
   return 0;
 }
 
@@ -2521,20 +3074,16 @@ int mist_eval_reduce(const MistProblem *problem, const MistGroupDesc *d_groups, 
                                       d_partial_cost, d_partial_index))
     return rc;
   if (!(ratio >= 0.0)) return fail(MIST_E_INVALID, "ratio must be non-negative");
-  const int32_t *scout_prefix = n_scout_blocks > 0 ? d_scout_prefix : nullptr;
   RatioList ratios = {};
   ratios.r[0] = ratio;
-  if (scout_prefix)
-    if (int rc = launch_scout(problem, d_groups, n_groups, d_block_prefix, n_blocks, scout_prefix,
-                              n_scout_blocks, d_row_terms, d_stage_floor, ratios, 1, n_blocks,
-                              d_partial_cost, d_partial_index, stream))
-      return rc;
-  hipLaunchKernelGGL(eval_reduce_kernel, dim3(xcd_padded_grid(n_blocks)), dim3(MIST_LC_TILE), 0,
-                     (hipStream_t)stream, *problem, d_groups, n_groups, d_block_prefix, n_blocks,
-                     scout_prefix, 0, d_row_terms, d_stage_floor, ratios, 0, (int64_t)n_blocks,
-                     d_partial_cost, d_partial_index);
-  MIST_HIP_CHECK(hipGetLastError());
-  return 0;
+  ReduceTables tabs;
+  if (int rc = reduce_tables(problem, 1, d_partial_cost, d_partial_index, &tabs)) return rc;
+  if (int rc = launch_seeds(problem, d_groups, n_groups, d_row_terms, ratios, n_scout_blocks > 0, tabs, d_partial_cost,
+                            stream))
+    return rc;
+  if (int rc = launch_super_floors(d_groups, n_groups, d_stage_floor, tabs, stream)) return rc;
+  return launch_reduce(problem, d_groups, n_groups, d_block_prefix, n_blocks, d_row_terms, d_stage_floor, ratios, tabs,
+                       stream);
 }
 
 int mist_stage_cost_first_estimate(const MistProblem *problem, const MistGroupDesc *d_groups,
@@ -2549,15 +3098,39 @@ int mist_stage_cost_first_estimate(const MistProblem *problem, const MistGroupDe
     return fail(MIST_E_INVALID, "no stage-cost incumbent to lower");
   if (n_groups > 65535) return fail(MIST_E_INVALID, "at most 65535 groups per call, got %d", n_groups);
   if (!(ratio >= 0.0)) return fail(MIST_E_INVALID, "ratio must be non-negative");
-  return launch_first_estimate(problem, d_groups, n_groups, d_scout_prefix, (int64_t)n_blocks,
-                               d_row_terms, ratio, d_partial_cost, stream);
+  return launch_first_estimate(problem, d_groups, n_groups, d_row_terms, ratio, d_partial_cost, stream);
 }
 
 static int launch_finalize(const MistProblem *problem, const MistGroupDesc *d_groups, int n_groups,
-                           const int32_t *d_block_prefix, const double *d_row_terms,
-                           const double *d_partial_cost, const int32_t *d_partial_index,
-                           const int32_t *sample_index, int n_samples, int n_blocks,
-                           const MistOutTables *tables, void *stream);
+                           const double *d_row_terms, const ReduceTables &tabs, const int32_t *sample_index,
+                           const MistOutTables *tables, void *stream) {
+  if (!d_row_terms || !tables) return fail(MIST_E_INVALID, "null pointer argument");
+  for (int v = 0; v < 4; ++v)
+    if (!tables->stable[v] || !tables->delta[v] || !tables->index[v])
+      return fail(MIST_E_INVALID, "output table %d is null", v);
+  const MistProblem &prob = *problem;
+  const int L = prob.num_layers, P1 = prob.p_dim, n_samples = tabs.n_samples;
+  if (L <= 0 || P1 <= 0 || prob.sample_size <= 0)
+    return fail(MIST_E_INVALID, "bad problem extents L=%d P+1=%d S=%d", L, P1, prob.sample_size);
+  SampleSlots slots = {};
+  for (int i = 0; i < n_samples; ++i) {
+    if (sample_index[i] < 0 || sample_index[i] >= prob.sample_size)
+      return fail(MIST_E_INVALID, "sample_index %d outside [0, %d)", sample_index[i], prob.sample_size);
+    slots.at[i] = sample_index[i];
+  }
+  if (n_groups > 65535) return fail(MIST_E_INVALID, "too many groups for one launch: %d", n_groups);
+  const int64_t n_pairs = (int64_t)L * (L + 1) / 2 + L + MIST_LC_TILE;
+  if (n_samples == 1)
+    hipLaunchKernelGGL(finalize_kernel, dim3((unsigned)(n_pairs / MIST_LC_TILE), 4, n_groups), dim3(256), 0,
+                       (hipStream_t)stream, prob, d_groups, d_row_terms, tabs, slots.at[0], *tables);
+  else
+    hipLaunchKernelGGL(finalize_samples_kernel,
+                       dim3((unsigned)((n_pairs * n_samples + 255) / 256),
+                            2 * ((P1 + kFinalRange - 1) / kFinalRange) + 2, n_groups),
+                       dim3(256), 0, (hipStream_t)stream, prob, d_groups, d_row_terms, tabs, slots, *tables);
+  MIST_HIP_CHECK(hipGetLastError());
+  return 0;
+}
 
 int mist_eval_reduce_samples(const MistProblem *problem, const MistGroupDesc *d_groups,
                              int n_groups, const int32_t *d_block_prefix, int n_blocks,
@@ -2580,29 +3153,15 @@ int mist_eval_reduce_samples(const MistProblem *problem, const MistGroupDesc *d_
     if (!(ratios[i] >= 0.0)) return fail(MIST_E_INVALID, "ratio %d must be non-negative", i);
     all.r[i] = ratios[i];
   }
-  const int32_t *scout_prefix = n_scout_blocks > 0 ? d_scout_prefix : nullptr;
-  const int64_t scout_base = (int64_t)main_batch * n_blocks;
-  // the scout passes of all samples in one launch: a single one occupies a tenth of the GPU
-  if (scout_prefix)
-    if (int rc = launch_scout(problem, d_groups, n_groups, d_block_prefix, n_blocks, scout_prefix,
-                              n_scout_blocks, d_row_terms, d_stage_floor, all, n_samples, scout_base,
-                              d_partial_cost, d_partial_index, stream))
-      return rc;
-  // main launches and finalize launches of main_batch samples at a time (grid.y = sample): the
-  // tail of one sample's wavefronts runs beside the next sample's
-  for (int first = 0; first < n_samples; first += main_batch) {
-    const int count = std::min(main_batch, n_samples - first);
-    hipLaunchKernelGGL(eval_reduce_kernel, dim3(xcd_padded_grid(n_blocks), count), dim3(MIST_LC_TILE),
-                       0, (hipStream_t)stream, *problem, d_groups, n_groups, d_block_prefix, n_blocks,
-                       scout_prefix, 0, d_row_terms, d_stage_floor, all, first, scout_base,
-                       d_partial_cost, d_partial_index);
-    MIST_HIP_CHECK(hipGetLastError());
-    if (int rc = launch_finalize(problem, d_groups, n_groups, d_block_prefix, d_row_terms,
-                                 d_partial_cost, d_partial_index, sample_index + first, count,
-                                 n_blocks, tables, stream))
-      return rc;
-  }
-  return 0;
+  ReduceTables tabs;
+  if (int rc = reduce_tables(problem, n_samples, d_partial_cost, d_partial_index, &tabs)) return rc;
+  if (int rc = launch_seeds(problem, d_groups, n_groups, d_row_terms, all, n_scout_blocks > 0, tabs, d_partial_cost, stream))
+    return rc;
+  if (int rc = launch_super_floors(d_groups, n_groups, d_stage_floor, tabs, stream)) return rc;
+  if (int rc = launch_reduce(problem, d_groups, n_groups, d_block_prefix, n_blocks, d_row_terms, d_stage_floor, all, tabs,
+                             stream))
+    return rc;
+  return launch_finalize(problem, d_groups, n_groups, d_row_terms, tabs, sample_index, tables, stream);
 }
 
 int mist_eval_reduce_exhaustive(const MistProblem *problem, const MistGroupDesc *d_groups,
@@ -2614,40 +3173,18 @@ int mist_eval_reduce_exhaustive(const MistProblem *problem, const MistGroupDesc 
     return fail(MIST_E_INVALID, "null workspace pointer");
   if (n_blocks <= 0) return fail(MIST_E_INVALID, "n_blocks must be positive, got %d", n_blocks);
   if (!(ratio >= 0.0)) return fail(MIST_E_INVALID, "ratio must be non-negative");
+  if (n_groups > 65535) return fail(MIST_E_INVALID, "at most 65535 groups per call, got %d", n_groups);
+  ReduceTables tabs;
+  if (int rc = reduce_tables(problem, 1, d_partial_cost, d_partial_index, &tabs)) return rc;
+  // the chunks' slabs lie behind the minima
+  double *slab_cost = d_partial_cost + problem->reduce_cells;
+  int32_t *slab_index = d_partial_index + problem->reduce_cells;
   hipLaunchKernelGGL(eval_reduce_exhaustive_kernel, dim3(xcd_padded_grid(n_blocks)),
                      dim3(MIST_LC_TILE), 0, (hipStream_t)stream, *problem, d_groups, n_groups,
-                     d_block_prefix, n_blocks, d_row_terms, ratio, d_partial_cost, d_partial_index);
+                     d_block_prefix, n_blocks, d_row_terms, ratio, slab_cost, slab_index);
   MIST_HIP_CHECK(hipGetLastError());
-  return 0;
-}
-
-static int launch_finalize(const MistProblem *problem, const MistGroupDesc *d_groups, int n_groups,
-                           const int32_t *d_block_prefix, const double *d_row_terms,
-                           const double *d_partial_cost, const int32_t *d_partial_index,
-                           const int32_t *sample_index, int n_samples, int n_blocks,
-                           const MistOutTables *tables, void *stream) {
-  if (int rc = check_common(problem, d_groups, n_groups)) return rc;
-  if (!d_block_prefix || !d_row_terms || !d_partial_cost || !d_partial_index || !tables)
-    return fail(MIST_E_INVALID, "null pointer argument");
-  for (int v = 0; v < 4; ++v)
-    if (!tables->stable[v] || !tables->delta[v] || !tables->index[v])
-      return fail(MIST_E_INVALID, "output table %d is null", v);
-  const MistProblem &prob = *problem;
-  const int L = prob.num_layers, P1 = prob.p_dim;
-  if (L <= 0 || P1 <= 0 || prob.sample_size <= 0)
-    return fail(MIST_E_INVALID, "bad problem extents L=%d P+1=%d S=%d", L, P1, prob.sample_size);
-  SampleSlots slots = {};
-  for (int i = 0; i < n_samples; ++i) {
-    if (sample_index[i] < 0 || sample_index[i] >= prob.sample_size)
-      return fail(MIST_E_INVALID, "sample_index %d outside [0, %d)", sample_index[i], prob.sample_size);
-    slots.at[i] = sample_index[i];
-  }
-  if (n_groups > 65535) return fail(MIST_E_INVALID, "too many groups for one launch: %d", n_groups);
-  const int n_pairs = L * (L + 1) / 2 + L;
-  dim3 grid((n_pairs + 255) / 256 * n_samples, 2 * P1 + 2, n_groups);
-  hipLaunchKernelGGL(finalize_kernel, grid, dim3(256), 0, (hipStream_t)stream, prob, d_groups,
-                     n_groups, d_block_prefix, d_row_terms, d_partial_cost, d_partial_index, slots,
-                     n_blocks, *tables);
+  hipLaunchKernelGGL(combine_slabs_kernel, dim3(64, n_groups), dim3(256), 0, (hipStream_t)stream, d_groups,
+                     d_block_prefix, slab_cost, slab_index, tabs);
   MIST_HIP_CHECK(hipGetLastError());
   return 0;
 }
@@ -2656,8 +3193,13 @@ int mist_finalize(const MistProblem *problem, const MistGroupDesc *d_groups, int
                   const int32_t *d_block_prefix, const double *d_row_terms,
                   const double *d_partial_cost, const int32_t *d_partial_index,
                   int sample_index, const MistOutTables *tables, void *stream) {
-  return launch_finalize(problem, d_groups, n_groups, d_block_prefix, d_row_terms, d_partial_cost,
-                         d_partial_index, &sample_index, 1, 0, tables, stream);
+  if (int rc = check_common(problem, d_groups, n_groups)) return rc;
+  if (!d_block_prefix || !d_partial_cost || !d_partial_index) return fail(MIST_E_INVALID, "null pointer argument");
+  ReduceTables tabs;
+  if (int rc = reduce_tables(problem, 1, const_cast<double *>(d_partial_cost),
+                             const_cast<int32_t *>(d_partial_index), &tabs))
+    return rc;
+  return launch_finalize(problem, d_groups, n_groups, d_row_terms, tabs, &sample_index, tables, stream);
 }
 
 // Second stream and events of mist_intra_stage_eval, one set per device, kept for the life of
@@ -2665,7 +3207,7 @@ int mist_finalize(const MistProblem *problem, const MistGroupDesc *d_groups, int
 namespace {
 struct OverlapStreams {
   hipStream_t side = nullptr;
-  hipEvent_t rows_ready = nullptr, scout_done = nullptr, main_done = nullptr;
+  hipEvent_t rows_ready = nullptr, seeds_done = nullptr;
 };
 std::mutex g_enqueue_lock;  // one call's records and waits on the shared events are a unit
 int overlap_streams(OverlapStreams **out) {
@@ -2679,90 +3221,12 @@ int overlap_streams(OverlapStreams **out) {
   if (s.side == nullptr) {
     MIST_HIP_CHECK(hipStreamCreateWithFlags(&s.side, hipStreamNonBlocking));  // default priority
     MIST_HIP_CHECK(hipEventCreateWithFlags(&s.rows_ready, hipEventDisableTiming));
-    MIST_HIP_CHECK(hipEventCreateWithFlags(&s.scout_done, hipEventDisableTiming));
-    MIST_HIP_CHECK(hipEventCreateWithFlags(&s.main_done, hipEventDisableTiming));
+    MIST_HIP_CHECK(hipEventCreateWithFlags(&s.seeds_done, hipEventDisableTiming));
   }
   *out = &s;
   return 0;
 }
 }  // namespace
-
-int mist_intra_stage_eval(const MistProblem *problem, const MistGroupDesc *d_groups,
-                          int n_groups, const int32_t *d_terms_block_prefix, int n_terms_blocks,
-                          const int32_t *d_reduce_block_prefix, int n_reduce_blocks,
-                          const int32_t *d_scout_prefix, int n_scout_blocks, double *d_row_terms,
-                          double *d_stage_floor, double *d_key_terms, double *d_partial_cost,
-                          int32_t *d_partial_index, double ratio, int sample_index,
-                          int compute_terms, const MistOutTables *tables, void *stream) {
-  if (compute_terms && n_scout_blocks > 0 && problem != nullptr && problem->max_scout_rows > 0 &&
-      n_groups > 0 && n_groups <= 65535) {
-    // The scout pass reads a few hundred rows per group and leaves most of the GPU idle; the row
-    // terms of everything else are computed beside it.  Stream order: [terms of the gathered
-    // rows] -> side stream: scout pass + merge || this stream: all other row terms -> main
-    // launch -> finalize.
-    if (int rc = check_reduce_arguments(problem, d_groups, n_groups, d_reduce_block_prefix,
-                                        n_reduce_blocks, d_scout_prefix, n_scout_blocks,
-                                        d_row_terms, d_stage_floor, d_partial_cost, d_partial_index))
-      return rc;
-    if (!d_terms_block_prefix || n_terms_blocks <= 0)
-      return fail(MIST_E_INVALID, "null / empty row-term decomposition");
-    if (int rc = check_factors(problem)) return rc;
-    if (!(ratio >= 0.0)) return fail(MIST_E_INVALID, "ratio must be non-negative");
-    OverlapStreams *os = nullptr;
-    if (int rc = overlap_streams(&os)) return rc;
-    // the second stream and its events are shared by all callers: one call's records and waits
-    // are enqueued as a unit
-    std::lock_guard<std::mutex> enqueue_guard(g_enqueue_lock);
-    hipStream_t main_stream = (hipStream_t)stream;
-    const unsigned scout_term_blocks = (unsigned)((problem->max_scout_rows + kTermsBlock - 1) / kTermsBlock);
-    hipLaunchKernelGGL((row_terms_kernel<1, false>), dim3(scout_term_blocks, n_groups),
-                       dim3(kTermsBlock), 0, main_stream, *problem, d_groups, n_groups,
-                       d_terms_block_prefix, d_row_terms, d_stage_floor, nullptr);
-    MIST_HIP_CHECK(hipGetLastError());
-    MIST_HIP_CHECK(hipEventRecord(os->rows_ready, main_stream));
-    MIST_HIP_CHECK(hipStreamWaitEvent(os->side, os->rows_ready, 0));
-    // (the other row terms are queued first: the scout pass is five launches, and this stream
-    // would idle while they are made)
-    bool from_keys = false;
-    if (int rc = launch_key_terms(problem, d_groups, n_groups, d_key_terms, main_stream, &from_keys))
-      return rc;
-    if (from_keys)
-      hipLaunchKernelGGL((row_terms_kernel<2, true>), dim3(n_terms_blocks), dim3(kTermsBlock), 0,
-                         main_stream, *problem, d_groups, n_groups, d_terms_block_prefix, d_row_terms,
-                         d_stage_floor, d_key_terms);
-    else
-      hipLaunchKernelGGL((row_terms_kernel<2, false>), dim3(n_terms_blocks), dim3(kTermsBlock), 0,
-                         main_stream, *problem, d_groups, n_groups, d_terms_block_prefix, d_row_terms,
-                         d_stage_floor, nullptr);
-    MIST_HIP_CHECK(hipGetLastError());
-    RatioList ratios = {};
-    ratios.r[0] = ratio;
-    if (int rc = launch_scout(problem, d_groups, n_groups, d_reduce_block_prefix, n_reduce_blocks,
-                              d_scout_prefix, n_scout_blocks, d_row_terms, d_stage_floor, ratios, 1,
-                              n_reduce_blocks, d_partial_cost, d_partial_index, os->side))
-      return rc;
-    MIST_HIP_CHECK(hipEventRecord(os->scout_done, os->side));
-    MIST_HIP_CHECK(hipStreamWaitEvent(main_stream, os->scout_done, 0));
-    hipLaunchKernelGGL(eval_reduce_kernel, dim3(xcd_padded_grid(n_reduce_blocks)), dim3(MIST_LC_TILE),
-                       0, main_stream, *problem, d_groups, n_groups, d_reduce_block_prefix,
-                       n_reduce_blocks, d_scout_prefix, 0, d_row_terms, d_stage_floor, ratios, 0,
-                       (int64_t)n_reduce_blocks, d_partial_cost, d_partial_index);
-    MIST_HIP_CHECK(hipGetLastError());
-    return mist_finalize(problem, d_groups, n_groups, d_reduce_block_prefix, d_row_terms,
-                         d_partial_cost, d_partial_index, sample_index, tables, stream);
-  }
-  if (compute_terms) {
-    if (int rc = mist_row_terms(problem, d_groups, n_groups, d_terms_block_prefix,
-                                n_terms_blocks, d_row_terms, d_stage_floor, d_key_terms, stream))
-      return rc;
-  }
-  if (int rc = mist_eval_reduce(problem, d_groups, n_groups, d_reduce_block_prefix,
-                                n_reduce_blocks, d_scout_prefix, n_scout_blocks, d_row_terms,
-                                d_stage_floor, ratio, d_partial_cost, d_partial_index, stream))
-    return rc;
-  return mist_finalize(problem, d_groups, n_groups, d_reduce_block_prefix, d_row_terms,
-                       d_partial_cost, d_partial_index, sample_index, tables, stream);
-}
 
 int mist_intra_stage_eval_samples(const MistProblem *problem, const MistGroupDesc *d_groups,
                                   int n_groups, const int32_t *d_terms_block_prefix,
@@ -2779,107 +3243,95 @@ int mist_intra_stage_eval_samples(const MistProblem *problem, const MistGroupDes
     return fail(MIST_E_INVALID, "sample_batch %d outside [1, %d]", sample_batch, MIST_MAX_SAMPLE_BATCH);
   if (main_batch < 1 || main_batch > sample_batch)
     return fail(MIST_E_INVALID, "main_batch %d outside [1, sample_batch = %d]", main_batch, sample_batch);
-  const bool overlap = n_scout_blocks > 0 && problem != nullptr && problem->max_scout_rows > 0 &&
-                       n_groups > 0 && n_groups <= 65535;
-  if (!overlap) {
-    if (int rc = mist_row_terms(problem, d_groups, n_groups, d_terms_block_prefix, n_terms_blocks,
-                                d_row_terms, d_stage_floor, d_key_terms, stream))
-      return rc;
-    for (int first = 0; first < n_samples; first += sample_batch) {
-      const int count = std::min(sample_batch, n_samples - first);
-      if (int rc = mist_eval_reduce_samples(problem, d_groups, n_groups, d_reduce_block_prefix,
-                                            n_reduce_blocks, d_scout_prefix, n_scout_blocks,
-                                            d_row_terms, d_stage_floor, ratios + first,
-                                            sample_index + first, count, std::min(main_batch, count),
-                                            d_partial_cost, d_partial_index, tables, stream))
-        return rc;
-    }
-    return 0;
-  }
-  // Stream order: [terms of the gathered rows] -> side stream: scout pass of the first batch of
-  // samples || this stream: all other row terms -> per batch b: side stream: scout pass of batch
-  // b + 1 (into the other scout region, once the main launches of batch b - 1, which read it,
-  // are through) || this stream: main launches and finalize of batch b.
   if (int rc = check_reduce_arguments(problem, d_groups, n_groups, d_reduce_block_prefix,
-                                      n_reduce_blocks, d_scout_prefix, n_scout_blocks, d_row_terms,
-                                      d_stage_floor, d_partial_cost, d_partial_index))
+                                      n_reduce_blocks, d_scout_prefix, n_scout_blocks,
+                                      d_row_terms, d_stage_floor, d_partial_cost, d_partial_index))
     return rc;
   if (!d_terms_block_prefix || n_terms_blocks <= 0)
     return fail(MIST_E_INVALID, "null / empty row-term decomposition");
   if (int rc = check_factors(problem)) return rc;
   for (int i = 0; i < n_samples; ++i)
     if (!(ratios[i] >= 0.0)) return fail(MIST_E_INVALID, "ratio %d must be non-negative", i);
-  OverlapStreams *os = nullptr;
-  if (int rc = overlap_streams(&os)) return rc;
-  std::lock_guard<std::mutex> enqueue_guard(g_enqueue_lock);
   hipStream_t main_stream = (hipStream_t)stream;
-  const int n_batches = (n_samples + sample_batch - 1) / sample_batch;
-  const int64_t main_slabs = (int64_t)main_batch * n_reduce_blocks;
-  const int64_t scout_slabs = (int64_t)sample_batch * n_scout_blocks;
-  auto batch_ratios = [&](int b, int *count) {
-    RatioList list = {};
-    const int first = b * sample_batch;
-    *count = std::min(sample_batch, n_samples - first);
-    for (int i = 0; i < *count; ++i) list.r[i] = ratios[first + i];
-    return list;
-  };
-  auto scout_of = [&](int b) -> int {  // on the side stream
-    int count = 0;
-    const RatioList list = batch_ratios(b, &count);
-    if (int rc = launch_scout(problem, d_groups, n_groups, d_reduce_block_prefix, n_reduce_blocks,
-                              d_scout_prefix, n_scout_blocks, d_row_terms, d_stage_floor, list, count,
-                              main_slabs + (b % 2) * scout_slabs, d_partial_cost, d_partial_index,
-                              os->side))
+  // The seeds read a few hundred rows per group and leave most of the GPU idle; the row terms of
+  // everything else are computed beside them.  Stream order: [terms of the gathered rows] -> side
+  // stream: seeds of the first batch of samples || this stream: all other row terms, second-level
+  // summaries -> filter, reduce, resolve, finalize; further batches one after the other.
+  const bool overlap = n_scout_blocks > 0 && problem->max_scout_rows > 0;
+  OverlapStreams *os = nullptr;
+  std::unique_lock<std::mutex> enqueue_guard;
+  if (overlap) {
+    if (int rc = overlap_streams(&os)) return rc;
+    // the second stream and its events are shared by all callers: one call's records and waits
+    // are enqueued as a unit
+    enqueue_guard = std::unique_lock<std::mutex>(g_enqueue_lock);
+    const unsigned scout_term_blocks = (unsigned)((problem->max_scout_rows + kTermsBlock - 1) / kTermsBlock);
+    hipLaunchKernelGGL((row_terms_kernel<1, false>), dim3(scout_term_blocks, n_groups),
+                       dim3(kTermsBlock), 0, main_stream, *problem, d_groups, n_groups,
+                       d_terms_block_prefix, d_row_terms, d_stage_floor, nullptr);
+    MIST_HIP_CHECK(hipGetLastError());
+    MIST_HIP_CHECK(hipEventRecord(os->rows_ready, main_stream));
+    MIST_HIP_CHECK(hipStreamWaitEvent(os->side, os->rows_ready, 0));
+    // (the other row terms are queued first: the seeds are several launches, and this stream would
+    // idle while they are made)
+    bool from_keys = false;
+    if (int rc = launch_key_terms(problem, d_groups, n_groups, d_key_terms, main_stream, &from_keys))
       return rc;
-    MIST_HIP_CHECK(hipEventRecord(os->scout_done, os->side));
-    return 0;
-  };
-  const unsigned scout_term_blocks = (unsigned)((problem->max_scout_rows + kTermsBlock - 1) / kTermsBlock);
-  hipLaunchKernelGGL((row_terms_kernel<1, false>), dim3(scout_term_blocks, n_groups),
-                     dim3(kTermsBlock), 0, main_stream, *problem, d_groups, n_groups,
-                     d_terms_block_prefix, d_row_terms, d_stage_floor, nullptr);
-  MIST_HIP_CHECK(hipGetLastError());
-  MIST_HIP_CHECK(hipEventRecord(os->rows_ready, main_stream));
-  MIST_HIP_CHECK(hipStreamWaitEvent(os->side, os->rows_ready, 0));
-  if (int rc = scout_of(0)) return rc;
-  bool from_keys = false;
-  if (int rc = launch_key_terms(problem, d_groups, n_groups, d_key_terms, main_stream, &from_keys))
-    return rc;
-  if (from_keys)
-    hipLaunchKernelGGL((row_terms_kernel<2, true>), dim3(n_terms_blocks), dim3(kTermsBlock), 0,
-                       main_stream, *problem, d_groups, n_groups, d_terms_block_prefix, d_row_terms,
-                       d_stage_floor, d_key_terms);
-  else
-    hipLaunchKernelGGL((row_terms_kernel<2, false>), dim3(n_terms_blocks), dim3(kTermsBlock), 0,
-                       main_stream, *problem, d_groups, n_groups, d_terms_block_prefix, d_row_terms,
-                       d_stage_floor, nullptr);
-  MIST_HIP_CHECK(hipGetLastError());
-  for (int b = 0; b < n_batches; ++b) {
-    // (a wait takes the event's latest record at the time of the call: the scout pass of batch b)
-    MIST_HIP_CHECK(hipStreamWaitEvent(main_stream, os->scout_done, 0));
-    if (b + 1 < n_batches) {
-      if (b >= 1) MIST_HIP_CHECK(hipStreamWaitEvent(os->side, os->main_done, 0));  // batch b - 1
-      if (int rc = scout_of(b + 1)) return rc;
-    }
-    int count = 0;
-    const RatioList list = batch_ratios(b, &count);
-    for (int first = 0; first < count; first += main_batch) {
-      const int n = std::min(main_batch, count - first);
-      hipLaunchKernelGGL(eval_reduce_kernel, dim3(xcd_padded_grid(n_reduce_blocks), n),
-                         dim3(MIST_LC_TILE), 0, main_stream, *problem, d_groups, n_groups,
-                         d_reduce_block_prefix, n_reduce_blocks, d_scout_prefix, 0, d_row_terms,
-                         d_stage_floor, list, first, main_slabs + (b % 2) * scout_slabs, d_partial_cost,
-                         d_partial_index);
-      MIST_HIP_CHECK(hipGetLastError());
-      if (int rc = launch_finalize(problem, d_groups, n_groups, d_reduce_block_prefix, d_row_terms,
-                                   d_partial_cost, d_partial_index,
-                                   sample_index + b * sample_batch + first, n, n_reduce_blocks, tables,
-                                   stream))
-        return rc;
-    }
-    MIST_HIP_CHECK(hipEventRecord(os->main_done, main_stream));
+    if (from_keys)
+      hipLaunchKernelGGL((row_terms_kernel<2, true>), dim3(n_terms_blocks), dim3(kTermsBlock), 0,
+                         main_stream, *problem, d_groups, n_groups, d_terms_block_prefix, d_row_terms,
+                         d_stage_floor, d_key_terms);
+    else
+      hipLaunchKernelGGL((row_terms_kernel<2, false>), dim3(n_terms_blocks), dim3(kTermsBlock), 0,
+                         main_stream, *problem, d_groups, n_groups, d_terms_block_prefix, d_row_terms,
+                         d_stage_floor, nullptr);
+    MIST_HIP_CHECK(hipGetLastError());
+  } else {
+    if (int rc = mist_row_terms(problem, d_groups, n_groups, d_terms_block_prefix, n_terms_blocks,
+                                d_row_terms, d_stage_floor, d_key_terms, stream))
+      return rc;
+  }
+  for (int first = 0; first < n_samples; first += sample_batch) {
+    const int count = std::min(sample_batch, n_samples - first);
+    ReduceTables tabs;
+    if (int rc = reduce_tables(problem, count, d_partial_cost, d_partial_index, &tabs)) return rc;
+    RatioList list = {};
+    for (int i = 0; i < count; ++i) list.r[i] = ratios[first + i];
+    const bool aside = overlap && first == 0;
+    if (int rc = launch_seeds(problem, d_groups, n_groups, d_row_terms, list, n_scout_blocks > 0, tabs, d_partial_cost,
+                              aside ? (void *)os->side : stream))
+      return rc;
+    if (aside) MIST_HIP_CHECK(hipEventRecord(os->seeds_done, os->side));
+    // (the summaries' place depends on the number of samples)
+    if (int rc = launch_super_floors(d_groups, n_groups, d_stage_floor, tabs, stream)) return rc;
+    if (aside) MIST_HIP_CHECK(hipStreamWaitEvent(main_stream, os->seeds_done, 0));
+    if (int rc = launch_reduce(problem, d_groups, n_groups, d_reduce_block_prefix, n_reduce_blocks, d_row_terms,
+                               d_stage_floor, list, tabs, stream))
+      return rc;
+    if (int rc = launch_finalize(problem, d_groups, n_groups, d_row_terms, tabs, sample_index + first, tables, stream))
+      return rc;
   }
   return 0;
+}
+
+int mist_intra_stage_eval(const MistProblem *problem, const MistGroupDesc *d_groups,
+                          int n_groups, const int32_t *d_terms_block_prefix, int n_terms_blocks,
+                          const int32_t *d_reduce_block_prefix, int n_reduce_blocks,
+                          const int32_t *d_scout_prefix, int n_scout_blocks, double *d_row_terms,
+                          double *d_stage_floor, double *d_key_terms, double *d_partial_cost,
+                          int32_t *d_partial_index, double ratio, int sample_index,
+                          int compute_terms, const MistOutTables *tables, void *stream) {
+  if (compute_terms)
+    return mist_intra_stage_eval_samples(problem, d_groups, n_groups, d_terms_block_prefix, n_terms_blocks,
+                                         d_reduce_block_prefix, n_reduce_blocks, d_scout_prefix, n_scout_blocks,
+                                         d_row_terms, d_stage_floor, d_key_terms, d_partial_cost, d_partial_index,
+                                         &ratio, &sample_index, 1, 1, 1, tables, stream);
+  if (int rc = mist_eval_reduce(problem, d_groups, n_groups, d_reduce_block_prefix,
+                                n_reduce_blocks, d_scout_prefix, n_scout_blocks, d_row_terms,
+                                d_stage_floor, ratio, d_partial_cost, d_partial_index, stream))
+    return rc;
+  return mist_finalize(problem, d_groups, n_groups, d_reduce_block_prefix, d_row_terms,
+                       d_partial_cost, d_partial_index, sample_index, tables, stream);
 }
 
 int mist_row_diagnostics(const MistProblem *problem, const MistGroupDesc *d_groups, int n_groups,

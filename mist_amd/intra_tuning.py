@@ -26,11 +26,10 @@ from .stage_inputs import GroupInputBuilder, make_problem
 
 SAMPLE_SIZE = 30  # reference default (batched_module_analyzer.py:67)
 VARIANTS = ("", "_with_pre", "_with_post", "_no_pp")
-# wavefronts of the reduce kernel the row chunks are sized for: 64 per SIMD, so that the tail of
-# the launch is short; a chunk that changes no slot writes no slab, which keeps small chunks cheap
-TARGET_REDUCE_WAVES = 65536
-SCOUT_MIN_STAGES = 128  # groups with fewer stages get no scout pass (0 = never scout)
-SCOUT_MIN_PAIRS = 4     # ... and so do groups with fewer (weight, gradient) offload pairs
+# wavefronts of the filter launch the row chunks are sized for: 16 per SIMD
+TARGET_REDUCE_WAVES = 16384
+SCOUT_MIN_STAGES = 1    # groups with fewer stages get no seeds (0 = never seed)
+SCOUT_MIN_PAIRS = 1     # ... and so do groups with fewer (weight, gradient) offload pairs
 SCOUT_PAIRS = 1         # offload pairs whose rows the scout pass gathers: the first, (0, 0), then evenly spread ones
 SCOUT_PAIR_SPAN = 200   # ... one more for every so many pairs of the group (GPT-22B: 421 pairs, 3 gathered)
 # ... and three for a group none of whose parallelism rows can hold this fraction of the model's
@@ -47,9 +46,9 @@ SCOUT_TIGHT_PAIRS = 3
 # the bound is a batch of its own).  GPT-7B (0.88 GB) and LLaMA-13B (1.4 GB) are one batch,
 # GPT-22B (18.4 GB of row terms) ten; with more than one batch two such workspaces alternate.
 ROW_TERMS_BUDGET_BYTES = 2 << 30
-# Partial-minima slabs the main launches of a multi-sample call may hold at once: samples in
-# flight = this / (workgroups of the launch x 26 KB); GPT-7B (63 232 workgroups): 4.
-MAIN_BATCH_SLAB_BYTES = 8 << 30
+# Minima tables (12 bytes per (l, c) pair, variant, p and sample) the launches of a multi-sample call
+# may hold: more samples go through them in batches.
+MINIMA_BYTES = 8 << 30
 
 
 _SIDE_STREAMS: Dict[str, "torch.cuda.Stream"] = {}
@@ -679,6 +678,29 @@ class IntraStageTuner:
         def to_dev(a: np.ndarray) -> torch.Tensor:
             return torch.from_numpy(np.ascontiguousarray(a).view(np.uint8).reshape(-1)).to(dev)
         lib = _lib.load()
+        # sizes of the reduce workspace: the minima of every (tile, slot) of a batch's groups, the
+        # second-level summaries, a queue that holds every (tile, stage)
+        most = dict(reduce_cells=1, reduce_supers=1, reduce_items=1, reduce_max_p=1)
+        for b in plan["batches"]:
+            g = b["groups"]
+            cells = g["n_lc_tiles"].astype(np.int64) * (_lib.LC_TILE * 2) * (g["num_p"] + 1)
+            g["cell_offset"] = np.concatenate(([0], np.cumsum(cells)[:-1]))
+            stages = -(-g["n_rows"] // _lib.STAGE_ROWS)
+            for key, value in (("reduce_cells", cells.sum()), ("reduce_items", (stages * g["n_lc_tiles"]).sum()),
+                               ("reduce_supers", b["total_rows"] // 512 + 2 * len(g) + 2),
+                               ("reduce_max_p", g["num_p"].max())):
+                most[key] = max(most[key], int(value))
+        for key, value in most.items():
+            plan["problem"][key] = value
+        self._sample_batch = min(len(self.sample_slots), _lib.MAX_SAMPLE_BATCH,
+                                 max(1, MINIMA_BYTES // (12 * most["reduce_cells"])))
+        n_index = self._sample_batch * most["reduce_cells"]
+        n_cost = lib.mist_reduce_workspace_doubles(most["reduce_cells"], most["reduce_supers"],
+                                                   most["reduce_items"], self._sample_batch)
+        if self.exhaustive:  # its chunks' minima behind the table
+            slabs = max([int(b["reduce_prefix"][-1]) for b in plan["batches"]] + [1]) * _lib.SLOTS * _lib.LC_TILE
+            n_index += slabs
+            n_cost = max(n_cost, most["reduce_cells"] + slabs)
         batches = []
         for b in plan["batches"]:
             batches.append(dict(
@@ -692,17 +714,6 @@ class IntraStageTuner:
         max_rows = max([b["total_rows"] for b in batches], default=0)
         max_groups = max([b["n_groups"] for b in batches], default=0)
         max_keys = max([b["total_keys"] for b in batches], default=0)
-        # several samples share one scout launch: their scout slabs lie behind one another; the
-        # main launches take as many samples at a time as their slabs (26 KB per workgroup and
-        # sample, written only where a chunk changes a minimum) fit MAIN_BATCH_SLAB_BYTES
-        self._sample_batch = min(len(self.sample_slots), _lib.MAX_SAMPLE_BATCH)
-        slab_bytes = _lib.SLOTS * _lib.LC_TILE * 12
-        most = max([b["n_reduce_blocks"] for b in batches] + [1])
-        self._main_batch = int(max(1, min(self._sample_batch, MAIN_BATCH_SLAB_BYTES // (most * slab_bytes))))
-        # (two scout regions: the scout pass of the next batch of samples runs beside the main
-        # launches of the current one)
-        n_slabs = max([self._main_batch * b["n_reduce_blocks"] + 2 * self._sample_batch * b["n_scout_blocks"]
-                       for b in batches] + [1])
         def workspace():
             return dict(
                 row_terms=torch.empty(max(max_rows, 1) * _lib.ROW_TERMS, dtype=torch.float64, device=dev),
@@ -710,8 +721,8 @@ class IntraStageTuner:
                                         dtype=torch.float64, device=dev),
                 key_terms=torch.empty(max(lib.mist_key_terms_doubles(max_keys), 1),
                                       dtype=torch.float64, device=dev),
-                partial_cost=torch.empty(n_slabs * _lib.SLOTS * _lib.LC_TILE, dtype=torch.float64, device=dev),
-                partial_index=torch.empty(n_slabs * _lib.SLOTS * _lib.LC_TILE, dtype=torch.int32, device=dev),
+                partial_cost=torch.empty(n_cost, dtype=torch.float64, device=dev),
+                partial_index=torch.empty(n_index, dtype=torch.int32, device=dev),
             )
         # several batches alternate between two workspaces on two streams, so that the tail of
         # one batch's launches overlaps the start of the next
@@ -793,7 +804,7 @@ class IntraStageTuner:
                     _ptr(w["stage_floor"]), _ptr(w["key_terms"]), _ptr(w["partial_cost"]),
                     _ptr(w["partial_index"]), ctypes.c_void_p(all_ratios.ctypes.data),
                     ctypes.c_void_p(slots.ctypes.data), len(slots), self._sample_batch,
-                    min(self._main_batch, self._sample_batch), ctypes.byref(out), stream)
+                    self._sample_batch, ctypes.byref(out), stream)
                 _lib.check(rc, "mist_intra_stage_eval_samples")
                 continue
             for i, slot in enumerate(self.sample_slots):

@@ -1,0 +1,40 @@
+"""The pruned reduction against the kernel that evaluates every cell, at the edges of its tiles."""
+import pytest
+
+from tests.util import tiny_plan
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("layers, nodes, gpus, batch, samples, seeded", [
+    (1, 1, 1, 2, 1, True),      # one layer: two pairs, one value of p
+    (9, 1, 4, 16, 1, False),    # 54 pairs, empty minima at the start of the reduce launch
+    (10, 1, 4, 16, 33, True),   # 65 pairs: a tile of one; a batch of 32 samples and one of 1
+    (10, 1, 4, 16, 31, False),
+    (66, 8, 8, 128, 1, True),   # 64 values of p: the minima of a pair are more than two per lane
+    (66, 8, 8, 128, 5, True),
+    (130, 2, 64, 128, 32, True),  # 128 of them: the samples of a pair do not fit the seeds' LDS at once
+])
+def test_pruned_tables_equal_every_cell_evaluated(layers, nodes, gpus, batch, samples, seeded, monkeypatch):
+    import torch
+
+    from mist_amd import intra_tuning
+    from mist_amd.config import tp_candidates
+    from mist_amd.intra_tuning import IntraStageTuner
+
+    if not seeded:
+        monkeypatch.setattr(intra_tuning, "SCOUT_MIN_STAGES", 0)
+    cfg, tables = tiny_plan(1, layers=layers, hardware__num_nodes=nodes, hardware__num_gpus_per_node=gpus,
+                            training__global_batch_size=batch, hardware__memory_capacity=8.0)
+    devices = nodes * gpus
+    meshes = [(1, 1)] if devices == 1 else [(1, 1), (1, 2), (nodes, gpus)]
+    tp, Gs = tp_candidates(cfg)[0], [batch // 2, batch]
+    got, want = [IntraStageTuner(tables, layers, meshes, Gs, tp, cfg, sample_size=samples, exhaustive=exhaustive).tune()
+                 for exhaustive in (False, True)]
+    finite = 0
+    for v in range(4):
+        for kind in ("index", "stable", "delta"):
+            a, b = getattr(got.device, kind)[v], getattr(want.device, kind)[v]
+            assert torch.equal(a, b), f"{kind} of variant {v}: {int((a != b).sum())} of {a.numel()} differ"
+        finite += int(torch.isfinite(want.device.stable[v]).sum())
+    assert finite > 0
