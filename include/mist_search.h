@@ -26,7 +26,7 @@ extern "C" {
 #define MIST_MAX_PAIRS (MIST_MAX_RATIOS * MIST_MAX_RATIOS)
 #define MIST_PAR_FIELDS 20
 #define MIST_ROW_TERMS 34   /* doubles per candidate row produced by mist_row_terms */
-#define MIST_KEY_TERMS 28   /* doubles per (parallelism row, activation ratio, offload pair) of the
+#define MIST_KEY_TERMS 56   /* doubles per (parallelism row, activation ratio, offload pair) of the
                              * key-term workspace of mist_row_terms */
 #define MIST_LC_TILE 64     /* (layers, ckpt) pairs per workgroup (one wavefront) of the reduce kernel */
 #ifndef MIST_P_TILE
@@ -329,7 +329,9 @@ int mist_finalize(const MistProblem *problem, const MistGroupDesc *d_groups, int
 
 /* mist_row_terms (when `compute_terms` != 0) + mist_eval_reduce + mist_finalize for one ratio:
  * the device side of IntraStageTuner.tune (mist/analyzer/intra_tuning.py:169-282) for one tp
- * candidate and one sample.  d_key_terms: as for mist_row_terms, may be NULL. */
+ * candidate and one sample.  d_key_terms: as for mist_row_terms, may be NULL.  With it and a scout
+ * pass only the stage summaries of all rows are computed first, and the row terms of the stages
+ * that the search opens when it does: d_row_terms then holds those and the scout pass's rows. */
 int mist_intra_stage_eval(const MistProblem *problem, const MistGroupDesc *d_groups,
                           int n_groups, const int32_t *d_terms_block_prefix, int n_terms_blocks,
                           const int32_t *d_reduce_block_prefix, int n_reduce_blocks,

@@ -25,7 +25,7 @@ TERMS_BLOCK = 128  # replaced by the library's own value in load()
 MAX_MESH = 16
 MAX_SAMPLE_BATCH = 16  # MIST_MAX_SAMPLE_BATCH; replaced by the library's own value in load()
 MAX_SCOUT_PAIRS = 8  # MIST_MAX_SCOUT_PAIRS (sizes a field of GROUP_DTYPE; checked in load())
-KEY_TERMS = 28  # MIST_KEY_TERMS; replaced by the library's own value in load()
+KEY_TERMS = 56  # MIST_KEY_TERMS; replaced by the library's own value in load()
 DP_NO_START = -3
 DP_CKPT_TAIL, DP_CKPT_STAGE, DP_CKPT_ALL = 0, 1, 2
 DP_THRESHOLD, DP_BOTTLENECK = 0, 1

@@ -56,6 +56,23 @@ static_assert(kStageMinNrs < kStageFloorPitch, "a stage summary is one 32-lane l
 static_assert(MIST_T_NAG_NOCK == MIST_T_NAG_CK + 1 && MIST_T_NRS_NOCK == MIST_T_NRS_CK + 1, "ck / nock pairs");
 static_assert(kStageRows == 2 * kStageFloorPitch, "lane = (column, half of the rows)");
 
+// Value of one lane (wave-uniform index) for the whole wavefront.
+__device__ __forceinline__ double from_lane(double v, int lane) {
+  const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+  const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)u, lane);
+  const uint32_t hi = __builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), lane);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+__device__ __forceinline__ int from_lane(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
+__device__ __forceinline__ float from_lane(float v, int lane) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+__device__ __forceinline__ uint64_t from_lane(uint64_t v, int lane) {
+  const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)v, lane);
+  const uint32_t hi = __builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), lane);
+  return ((uint64_t)hi << 32) | lo;
+}
+
 // ------------------------------------------------------------------------------------------
 // Communication models (mist/tools/optimize.py:257-303, 459-470).
 // ------------------------------------------------------------------------------------------
@@ -344,10 +361,11 @@ __device__ __forceinline__ int tile_position(const MistGroupDesc *g, int oo, int
   return tile * kOoTile * g->n_pair + pair * width + (oo - tile * kOoTile);
 }
 
-__device__ __forceinline__ RowParts parts_of_position(const MistGroupDesc *g, int64_t pos) {
+// (positions fit 32 bits: the tables hold row numbers as int32)
+__device__ __forceinline__ RowParts parts_of_position(const MistGroupDesc *g, uint32_t pos) {
   RowParts r;
-  r.par = (int)(pos / g->n_off);
-  int rem = (int)(pos % g->n_off);
+  r.par = (int)(pos / (uint32_t)g->n_off);
+  int rem = (int)(pos - (uint32_t)r.par * (uint32_t)g->n_off);
   const int per_ao = g->n_oo * g->n_pair;
   r.ao = rem / per_ao;
   rem -= r.ao * per_ao;
@@ -360,7 +378,7 @@ __device__ __forceinline__ RowParts parts_of_position(const MistGroupDesc *g, in
 }
 
 __device__ __forceinline__ int32_t row_of_position(const MistGroupDesc *g, int64_t pos) {
-  const RowParts r = parts_of_position(g, pos);
+  const RowParts r = parts_of_position(g, (uint32_t)pos);
   return (int32_t)((int64_t)r.par * g->n_off + (r.pair * g->n_oo + r.oo) * g->n_ao + r.ao);
 }
 
@@ -388,7 +406,19 @@ constexpr int kKeyBwd = 0;        // [last?0:1 micro-batch][nock, ck] x (layer, 
 constexpr int kKeyFwd = 20;       // forward, not the first micro-batch: [nock, ck] x (layer, last, extra_post)
 constexpr int kKeyFwdFirst = 26;  //   its `first` and `extra_pre`, which do not depend on ckpt
 constexpr int kKeyFwdExtraPre = 27;
-static_assert(MIST_KEY_TERMS == 28 && MIST_KEY_TERMS % 2 == 0, "key terms are read as 16-byte pairs");
+constexpr int kKeyRow = 28;       // terms up to here are what row_terms reads of a key
+// ... and for the stage summaries the columns that are the same for the n_oo rows of the key,
+constexpr int kKeyCols = 28;      // S_LAYER_CK .. S_LAST_NOCK (of G > 1), then
+constexpr int kKeyState0 = 34;    // FWD_STATES0, BWD_STATES0, PWG, S_CK, S_NOCK, D_CK, D_NOCK,
+constexpr int kKeyPeaks = 41;     // FWD_PEAK, BWD_PEAK, OUT, GCB,
+constexpr int kKeyPost = 45;      // OPB, the smaller NAG, the smaller NRS;
+constexpr int kKeyColsEnd = 48;
+// what the rows' first forward phase and memory factor take from the key
+constexpr int kKeySoW = 48, kKeySiG = 49, kKeySoA = 50;  // so_W, si_G, so_A_ck, so_A_nock
+constexpr int kKeyFactor = 52;    // memory factor without / with optimizer offloading
+constexpr int kKeyGather = 54;    // AG_w * ore
+static_assert(MIST_KEY_TERMS == 56 && MIST_KEY_TERMS % 2 == 0, "key terms are read as 16-byte pairs");
+constexpr int kKeyPitch = MIST_KEY_TERMS + 1;  // of a key in LDS
 
 // Model tables of a workgroup in LDS (tables indexed at run time: indexing the by-value kernel
 // argument would make every lane keep a private copy of the whole struct in scratch memory).
@@ -405,6 +435,51 @@ __device__ __forceinline__ bool load_model_tables(const MistProblem &prob,
   }
   if (threadIdx.x >= 64 && threadIdx.x < 96) lds_gpu_gpu[threadIdx.x - 64] = prob.gpu_gpu[threadIdx.x - 64];
   return __syncthreads_and(factors_tame) != 0;
+}
+
+// batched_module_analyzer.py:1181-1199
+__device__ __forceinline__ double memory_factor(const MistProblem &prob, const double *par, double wo, double go,
+                                                double oo, double ao) {
+  double mf = 1.0;
+  mf += prob.frag_factor;
+  mf += wo > 0.0 ? 0.025 : 0.0;
+  mf += go > 0.0 ? 0.025 : 0.0;
+  mf += oo > 0.0 ? 0.03 : 0.0;
+  mf += ao > 0.0 ? 0.04 : 0.0;
+  mf += par[MIST_PAR_WRE] != 0.0 ? 0.025 : 0.0;
+  mf += par[MIST_PAR_GRE] != 0.0 ? 0.025 : 0.0;
+  mf += par[MIST_PAR_TP] > 1.0 ? 0.04 : 0.0;
+  mf += par[MIST_PAR_B] >= 4.0 ? 0.01 : 0.0;
+  return mf;
+}
+
+// Memory pieces of a row that do not depend on the optimizer ratio (:1216-1272, 2091-2162).
+struct KeyMemory {
+  double pWG, S_ck, S_nock, D_ck, D_nock, two_buf, fwd_states0;
+};
+__device__ __forceinline__ KeyMemory key_memory(const MistGroupDesc *g, const double *par, double wo, double go,
+                                                double ao) {
+  const double dp = par[MIST_PAR_DP];
+  const double W = par[MIST_PAR_W], Gr = par[MIST_PAR_G], O = par[MIST_PAR_O];
+  const double raw_ck = par[MIST_PAR_RAW_CK], raw_nock = par[MIST_PAR_RAW_NOCK];
+  const double wre_size = par[MIST_PAR_WRE] == 1.0 ? dp : 1.0;
+  const double gre_size = par[MIST_PAR_GRE] == 1.0 ? dp : 1.0;
+  const double ore_size = par[MIST_PAR_ORE] == 1.0 ? dp : 1.0;
+  KeyMemory m;
+  const double pW = W / wre_size * (1.0 - wo);
+  const double pG = Gr / gre_size * (1.0 - go);
+  m.pWG = pW + pG;
+  m.S_ck = raw_ck * (1.0 - ao);
+  m.D_ck = raw_ck * ao;
+  m.S_nock = raw_nock * (1.0 - ao);
+  m.D_nock = raw_nock * ao;
+  const bool wbuf_on = wre_size > 1.0 || g->pp_wre == 1 || wo > 0.0;
+  const bool gbuf_on = gre_size > 1.0 || g->pp_gre == 1 || go > 0.0;
+  const double Wbuf = wbuf_on ? fmax(fmax(g->pre_full_w, g->post_full_w), W) : 0.0;
+  const double Gbuf = gbuf_on ? fmax(fmax(g->pre_full_g, g->post_full_g), Gr) : 0.0;
+  m.two_buf = 2.0 * (Wbuf + Gbuf);
+  m.fwd_states0 = m.two_buf + np_floor_divide(O, ore_size);
+  return m;
 }
 
 // Operands of the interference evaluations that do not depend on the optimizer ratio: swap and
@@ -458,6 +533,23 @@ __device__ __forceinline__ KeyInputs key_inputs(const MistProblem &prob, const d
   in.extra_fb = in.extra_fwd + in.extra_bwd;
   in.exec_bwd_ck = in.exec_fwd + in.exec_bwd_nock;
   return in;
+}
+
+// Post-layer collectives left over beside the last layer (:2251-2292).
+struct PostTerms {
+  double nag_ck, nag_nock, nrs_ck, nrs_nock;
+};
+__device__ __forceinline__ PostTerms post_terms(const MistGroupDesc *g, const KeyInputs &in) {
+  PostTerms p;
+  const double ovw_ck = fmax(in.exec_fwd - 0.0 - in.so_A_ck, 0.0);
+  const double ovw_nock = fmax(in.exec_fwd - 0.0 - in.so_A_nock, 0.0);
+  p.nag_ck = fmax(g->post_ag - ovw_ck, 0.0);
+  p.nag_nock = fmax(g->post_ag - ovw_nock, 0.0);
+  const double ovg_ck = fmax(in.exec_bwd_ck - in.ag_wre - in.c2g_B - in.si_A_ck, 0.0);
+  const double ovg_nock = fmax(in.exec_bwd_nock - in.ag_wre - in.c2g_B - in.si_A_nock, 0.0);
+  p.nrs_ck = fmax(g->post_rs - ovg_ck, 0.0);
+  p.nrs_nock = fmax(g->post_rs - ovg_nock, 0.0);
+  return p;
 }
 
 // Forward phases (:1432-1621): phase 0 = first micro-batch (the optimizer-state swaps so_O /
@@ -525,6 +617,7 @@ __global__ __launch_bounds__(kTermsBlock) void key_terms_kernel(
   if ((int)blockIdx.x * kKeysPerBlock >= n_keys) return;
   __shared__ __align__(16) double lds_factor[11][kFactorPitch];
   __shared__ double lds_gpu_gpu[32];
+  __shared__ double lds_out[kKeysPerBlock][kKeyPitch];
   InterferenceModel<false> I;
   I.factors_tame = load_model_tables(prob, lds_factor, lds_gpu_gpu);
   I.table = (LdsDouble *)&lds_factor[0][0];
@@ -534,15 +627,15 @@ __global__ __launch_bounds__(kTermsBlock) void key_terms_kernel(
   const int pair = key % g->n_pair;
   const int ao_i = (key / g->n_pair) % g->n_ao;
   const int par_i = key / (g->n_pair * g->n_ao);
-  const KeyInputs in = key_inputs(prob, lds_gpu_gpu, g, g->par[par_i], g->wo[g->pair_wo[pair]],
-                                  g->go[g->pair_go[pair]], g->ao[ao_i]);
+  const double *par = g->par[par_i];
+  const double wo = g->wo[g->pair_wo[pair]], go = g->go[g->pair_go[pair]], ao = g->ao[ao_i];
+  const KeyInputs in = key_inputs(prob, lds_gpu_gpu, g, par, wo, go, ao);
   const Family back = bwd_family(I, in, (j & 2) != 0, (j & 1) != 0);
   const FwdOperands op = fwd_operands(in, false, 0.0, 0.0);
   double first, extra_pre, layer, last, extra_post;
   fwd_common(I, in, op, false, prob.adv_first_block != 0, first, extra_pre);
   fwd_of_ckpt(I, in, op, (j & 1) != 0, layer, last, extra_post);
-  if (key_here >= n_keys) return;
-  double *out = key_terms + (g->key_offset + key) * MIST_KEY_TERMS;
+  double *out = lds_out[threadIdx.x / 4];
   double *b = out + kKeyBwd + j * 5;
   b[0] = back.layer;
   b[1] = back.first;
@@ -554,61 +647,62 @@ __global__ __launch_bounds__(kTermsBlock) void key_terms_kernel(
     f[0] = layer;
     f[1] = last;
     f[2] = extra_post;
+  } else {
+    // (with ckpt in front of without)
+    double *c = out + kKeyCols + (1 - (j & 1));
+    c[0] = layer + back.layer;
+    c[2] = extra_pre + back.extra_post + first + back.first;
+    c[4] = extra_post + back.extra_pre + last + back.last;
+    if (j == 3) out[kKeyPost] = fmax(g->post_bwd - back.extra_pre, 0.0);
   }
   if (j == 0) {
     out[kKeyFwdFirst] = first;
     out[kKeyFwdExtraPre] = extra_pre;
-  }
-}
-
-// kMode 0: every row of every group.  kMode 1: only the rows the scout pass gathers (workgroup
-// = (128 gathered rows, group); no stage summaries), so that the scout pass can start while
-// kMode 2 computes everything: that one leaves the stores of the gathered rows out (the scout
-// pass may be reading them) and is otherwise kMode 0.  kFromKeys: the key terms are read from
-// `key_terms` (written by key_terms_kernel) instead of evaluated per row.
-__device__ __forceinline__ int64_t gathered_position(const MistGroupDesc *g, int64_t q);
-__device__ __forceinline__ bool is_scout_pair(const MistGroupDesc *g, int pair) {
-  for (int k = 0; k < g->scout_stride; ++k)
-    if (pair == g->scout_pair[k]) return true;
-  return false;
-}
-
-template <int kMode, bool kFromKeys>
-__global__ __launch_bounds__(kTermsBlock) void row_terms_kernel(
-    const MistProblem prob, const MistGroupDesc *__restrict__ groups, int n_groups,
-    const int32_t *__restrict__ block_prefix, double *__restrict__ row_terms,
-    double *__restrict__ stage_floor, const double *__restrict__ key_terms) {
-  int local_block;
-  const MistGroupDesc *g;
-  int64_t n_here_total;  // rows this launch computes for the group
-  if (kMode == 1) {
-    g = groups + blockIdx.y;
-    local_block = blockIdx.x;
-    n_here_total = g->scout_stride > 0 ? (int64_t)g->n_par * g->n_oo * g->n_ao * g->scout_stride : 0;
-    if ((int64_t)local_block * kTermsBlock >= n_here_total) return;
+    const PostTerms post = post_terms(g, in);
+    out[kKeyPost + 1] = fmin(post.nag_ck, post.nag_nock);
+    out[kKeyPost + 2] = fmin(post.nrs_ck, post.nrs_nock);
+    out[kKeyFactor] = memory_factor(prob, par, wo, go, 0.0, ao);
+    out[kKeyFactor + 1] = memory_factor(prob, par, wo, go, 1.0, ao);
+  } else if (j == 1) {
+    const KeyMemory m = key_memory(g, par, wo, go, ao);
+    double *c = out + kKeyState0;
+    c[0] = m.fwd_states0;
+    c[1] = m.two_buf;
+    c[2] = m.pWG;
+    c[3] = m.S_ck;
+    c[4] = m.S_nock;
+    c[5] = m.D_ck;
+    c[6] = m.D_nock;
+  } else if (j == 2) {
+    double *c = out + kKeyPeaks;
+    c[0] = par[MIST_PAR_FWD_PEAK];
+    c[1] = par[MIST_PAR_BWD_PEAK];
+    c[2] = par[MIST_PAR_OUT];
+    c[3] = par[MIST_PAR_GCB];
   } else {
-    g = find_group(groups, block_prefix, n_groups, blockIdx.x, &local_block);
-    n_here_total = g->n_rows;
+    out[kKeySoW] = in.so_W;
+    out[kKeySiG] = in.si_G;
+    out[kKeySoA] = in.so_A_ck;
+    out[kKeySoA + 1] = in.so_A_nock;
+    out[kKeyGather] = in.AG_w * in.ore;
+    out[kKeyGather + 1] = 0.0;
   }
-  // The block's terms are written out as one contiguous, fully coalesced range (a lane writing
-  // its own 272-byte row would touch 34 partial cache lines): wavefront by wavefront through one
-  // LDS buffer of kStageRows rows (row pitch 35 doubles: conflict-free).  One buffer for the
-  // block, not one per wavefront: LDS is what bounds the number of resident wavefronts here, and
-  // the kernel is a chain of dependent loads and evaluations that needs them.
-  __shared__ double lds_out[kStageRows * (MIST_ROW_TERMS + 1)];
-  __shared__ __align__(16) double lds_factor[11][kFactorPitch];
-  __shared__ double lds_gpu_gpu[32];
-  __shared__ unsigned char lds_skip[kTermsBlock];
-  __shared__ double lds_part[kTermsBlock / kStageRows - 1][2][kStageFloorPitch];  // stage summaries
-  InterferenceModel<kFromKeys> I;  // with key terms only the first forward phase is evaluated here
-  I.factors_tame = load_model_tables(prob, lds_factor, lds_gpu_gpu);
-  I.table = (LdsDouble *)&lds_factor[0][0];
-  const int64_t block_first = (int64_t)local_block * kTermsBlock;
-  const int rows_here = (int)min((int64_t)kTermsBlock, n_here_total - block_first);
-  // Lanes past the end recompute the last row (no divergent barrier); their result is dropped.
-  const int64_t nth = block_first + min((int)threadIdx.x, rows_here - 1);
-  const int64_t row = kMode == 1 ? gathered_position(g, nth) : nth;  // workspace position
+  __syncthreads();
+  double *__restrict__ dst =
+      key_terms + (g->key_offset + (int64_t)blockIdx.x * kKeysPerBlock) * MIST_KEY_TERMS;
+  const int n_out = min(kKeysPerBlock, n_keys - (int)blockIdx.x * kKeysPerBlock) * MIST_KEY_TERMS;
+  for (int i = threadIdx.x; i < n_out; i += kTermsBlock)
+    dst[i] = lds_out[i / MIST_KEY_TERMS][i % MIST_KEY_TERMS];
+}
 
+__device__ __forceinline__ int64_t gathered_position(const MistGroupDesc *g, int64_t q);
+
+// Terms of the row at workspace position `row` of a group.  kFromKeys: what is the same for the
+// n_oo rows of its key is read from `key_terms` (written by key_terms_kernel) instead of evaluated.
+template <bool kFromKeys>
+__device__ __forceinline__ void row_terms_of(const MistProblem &prob, const MistGroupDesc *__restrict__ g, uint32_t row,
+                                             const double *__restrict__ key_terms, const double *lds_gpu_gpu,
+                                             const InterferenceModel<kFromKeys> &I, double (&t)[MIST_ROW_TERMS]) {
   // ---- index decomposition (batched_module_analyzer.py:490-534) ----
   const RowParts parts = parts_of_position(g, row);
   const int par_i = parts.par, pair = parts.pair, oo_i = parts.oo, ao_i = parts.ao;
@@ -619,13 +713,13 @@ __global__ __launch_bounds__(kTermsBlock) void row_terms_kernel(
 
   // the key terms are fetched first and used last: the loads are in flight across everything
   // computed here
-  double v[kFromKeys ? MIST_KEY_TERMS : 2];
+  double v[kFromKeys ? kKeyRow : 2];
   if (kFromKeys) {
     const int64_t key = (int64_t)(par_i * g->n_ao + ao_i) * g->n_pair + pair;
     const double2 *__restrict__ kt =
         reinterpret_cast<const double2 *>(key_terms + (g->key_offset + key) * MIST_KEY_TERMS);
 #pragma unroll
-    for (int i = 0; i < MIST_KEY_TERMS / 2; ++i) {
+    for (int i = 0; i < kKeyRow / 2; ++i) {
       const double2 two = kt[i];
       v[2 * i] = two.x;
       v[2 * i + 1] = two.y;
@@ -633,38 +727,12 @@ __global__ __launch_bounds__(kTermsBlock) void row_terms_kernel(
   }
 
   const double *par = g->par[par_i];
-  const double b = par[MIST_PAR_B], dp = par[MIST_PAR_DP], tp = par[MIST_PAR_TP];
-  const double wre = par[MIST_PAR_WRE], gre = par[MIST_PAR_GRE], ore = par[MIST_PAR_ORE];
-  const double W = par[MIST_PAR_W], Gr = par[MIST_PAR_G], O = par[MIST_PAR_O];
-  const double raw_ck = par[MIST_PAR_RAW_CK], raw_nock = par[MIST_PAR_RAW_NOCK];
-  const double wre_size = wre == 1.0 ? dp : 1.0;
-  const double gre_size = gre == 1.0 ? dp : 1.0;
-  const double ore_size = ore == 1.0 ? dp : 1.0;
-
-  // ---- memory factor (:1181-1199) ----
-  double mf = 1.0;
-  mf += prob.frag_factor;
-  mf += wo > 0.0 ? 0.025 : 0.0;
-  mf += go > 0.0 ? 0.025 : 0.0;
-  mf += oo > 0.0 ? 0.03 : 0.0;
-  mf += ao > 0.0 ? 0.04 : 0.0;
-  mf += wre != 0.0 ? 0.025 : 0.0;
-  mf += gre != 0.0 ? 0.025 : 0.0;
-  mf += tp > 1.0 ? 0.04 : 0.0;
-  mf += b >= 4.0 ? 0.01 : 0.0;
+  const double ore_size = par[MIST_PAR_ORE] == 1.0 ? par[MIST_PAR_DP] : 1.0;
+  const double O = par[MIST_PAR_O], raw_nock = par[MIST_PAR_RAW_NOCK];
+  const double mf = memory_factor(prob, par, wo, go, oo, ao);
   const double mf_pp = mf + 0.025;
-
-  // ---- memory pieces (:1216-1272, 2091-2162) ----
-  const double pW = W / wre_size * (1.0 - wo);
-  const double pG = Gr / gre_size * (1.0 - go);
+  const KeyMemory mem = key_memory(g, par, wo, go, ao);
   const double pO = O / ore_size * (1.0 - oo);
-  const double S_ck = raw_ck * (1.0 - ao), D_ck = raw_ck * ao;
-  const double S_nock = raw_nock * (1.0 - ao), D_nock = raw_nock * ao;
-  const bool wbuf_on = wre_size > 1.0 || g->pp_wre == 1 || wo > 0.0;
-  const bool gbuf_on = gre_size > 1.0 || g->pp_gre == 1 || go > 0.0;
-  const double Wbuf = wbuf_on ? fmax(fmax(g->pre_full_w, g->post_full_w), W) : 0.0;
-  const double Gbuf = gbuf_on ? fmax(fmax(g->pre_full_g, g->post_full_g), Gr) : 0.0;
-  const double two_buf = 2.0 * (Wbuf + Gbuf);
 
   // ---- swap and collective latencies (:1362-1408) ----
   const KeyInputs in = key_inputs(prob, lds_gpu_gpu, g, par, wo, go, ao);
@@ -712,7 +780,6 @@ __global__ __launch_bounds__(kTermsBlock) void row_terms_kernel(
   }
 
   // ---- stable / delta families (:1910-2028) ----
-  double t[MIST_ROW_TERMS];  // compile-time indices only: registers
   const int st = g->grad_accum == 1 ? 0 : 1;  // phase index that forms the stable part
 #pragma unroll
   for (int k = 0; k < 2; ++k) {
@@ -739,15 +806,15 @@ __global__ __launch_bounds__(kTermsBlock) void row_terms_kernel(
     t[MIST_T_D_LAST_CK + (1 - k)] = d_last;
   }
 
-  t[MIST_T_FWD_STATES0] = two_buf + np_floor_divide(O, ore_size);
-  t[MIST_T_BWD_STATES0] = two_buf;
-  t[MIST_T_PWG] = pW + pG;
+  t[MIST_T_FWD_STATES0] = mem.fwd_states0;
+  t[MIST_T_BWD_STATES0] = mem.two_buf;
+  t[MIST_T_PWG] = mem.pWG;
   t[MIST_T_PO] = pO;
-  t[MIST_T_PWGO] = pW + pG + pO;
-  t[MIST_T_S_CK] = S_ck;
-  t[MIST_T_S_NOCK] = S_nock;
-  t[MIST_T_D_CK] = D_ck;
-  t[MIST_T_D_NOCK] = D_nock;
+  t[MIST_T_PWGO] = mem.pWG + pO;
+  t[MIST_T_S_CK] = mem.S_ck;
+  t[MIST_T_S_NOCK] = mem.S_nock;
+  t[MIST_T_D_CK] = mem.D_ck;
+  t[MIST_T_D_NOCK] = mem.D_nock;
   t[MIST_T_MF_BASE] = mf_pp + 0.01;
   t[MIST_T_MF_PP] = mf_pp;
   t[MIST_T_MF] = mf;
@@ -756,17 +823,62 @@ __global__ __launch_bounds__(kTermsBlock) void row_terms_kernel(
   t[MIST_T_OUT] = par[MIST_PAR_OUT];
   t[MIST_T_GCB] = par[MIST_PAR_GCB];
 
-  // ---- post-layer overlap pieces (:2251-2292) ----
-  const double ovw_ck = fmax(in.exec_fwd - 0.0 - in.so_A_ck, 0.0);
-  const double ovw_nock = fmax(in.exec_fwd - 0.0 - in.so_A_nock, 0.0);
-  t[MIST_T_NAG_CK] = fmax(g->post_ag - ovw_ck, 0.0);
-  t[MIST_T_NAG_NOCK] = fmax(g->post_ag - ovw_nock, 0.0);
-  const double ovg_ck = fmax(in.exec_bwd_ck - in.ag_wre - in.c2g_B - in.si_A_ck, 0.0);
-  const double ovg_nock = fmax(in.exec_bwd_nock - in.ag_wre - in.c2g_B - in.si_A_nock, 0.0);
-  t[MIST_T_NRS_CK] = fmax(g->post_rs - ovg_ck, 0.0);
-  t[MIST_T_NRS_NOCK] = fmax(g->post_rs - ovg_nock, 0.0);
+  const PostTerms post = post_terms(g, in);
+  t[MIST_T_NAG_CK] = post.nag_ck;
+  t[MIST_T_NAG_NOCK] = post.nag_nock;
+  t[MIST_T_NRS_CK] = post.nrs_ck;
+  t[MIST_T_NRS_NOCK] = post.nrs_nock;
   t[MIST_T_OPB] = fmax(g->post_bwd - bwd[1][1].extra_pre, 0.0);
-  t[MIST_T_RD] = raw_nock - S_nock;
+  t[MIST_T_RD] = raw_nock - mem.S_nock;
+}
+
+// Rows leave a workgroup as contiguous, fully coalesced ranges (a lane writing its own 272-byte row
+// would touch 34 partial cache lines): wavefront by wavefront through one LDS buffer of kStageRows
+// rows (row pitch 35 doubles: conflict-free).  One buffer for the block, not one per wavefront: LDS
+// is what bounds the number of resident wavefronts here.
+__device__ __forceinline__ void store_rows(const double *lds_rows, int n, double *__restrict__ out) {
+  double2 *__restrict__ dst = reinterpret_cast<double2 *>(out);
+  for (int i = threadIdx.x; i < n * (MIST_ROW_TERMS / 2); i += kTermsBlock) {
+    const int at = i / (MIST_ROW_TERMS / 2) * (MIST_ROW_TERMS + 1) + 2 * (i % (MIST_ROW_TERMS / 2));
+    dst[i] = make_double2(lds_rows[at], lds_rows[at + 1]);
+  }
+}
+
+// kMode 0: every row of every group, and without key terms (kFromKeys) their stage summaries.
+// kMode 1: only the rows the scout pass gathers (workgroup = (128 gathered rows, group)), so that
+// it can start before anything else is there.
+template <int kMode, bool kFromKeys>
+__global__ __launch_bounds__(kTermsBlock) void row_terms_kernel(
+    const MistProblem prob, const MistGroupDesc *__restrict__ groups, int n_groups,
+    const int32_t *__restrict__ block_prefix, double *__restrict__ row_terms,
+    double *__restrict__ stage_floor, const double *__restrict__ key_terms) {
+  constexpr bool kFloors = kMode == 0 && !kFromKeys;
+  int local_block;
+  const MistGroupDesc *g;
+  int64_t n_here_total;  // rows this launch computes for the group
+  if (kMode == 1) {
+    g = groups + blockIdx.y;
+    local_block = blockIdx.x;
+    n_here_total = g->scout_stride > 0 ? (int64_t)g->n_par * g->n_oo * g->n_ao * g->scout_stride : 0;
+    if ((int64_t)local_block * kTermsBlock >= n_here_total) return;
+  } else {
+    g = find_group(groups, block_prefix, n_groups, blockIdx.x, &local_block);
+    n_here_total = g->n_rows;
+  }
+  __shared__ double lds_out[kMode == 1 ? 1 : kStageRows * (MIST_ROW_TERMS + 1)];
+  __shared__ __align__(16) double lds_factor[11][kFactorPitch];
+  __shared__ double lds_gpu_gpu[32];
+  __shared__ double lds_part[kFloors ? kTermsBlock / kStageRows - 1 : 1][2][kFloors ? kStageFloorPitch : 1];
+  InterferenceModel<kFromKeys> I;  // with key terms only the first forward phase is evaluated here
+  I.factors_tame = load_model_tables(prob, lds_factor, lds_gpu_gpu);
+  I.table = (LdsDouble *)&lds_factor[0][0];
+  const int64_t block_first = (int64_t)local_block * kTermsBlock;
+  const int rows_here = (int)min((int64_t)kTermsBlock, n_here_total - block_first);
+  // Lanes past the end recompute the last row (no divergent barrier); their result is dropped.
+  const int64_t nth = block_first + min((int)threadIdx.x, rows_here - 1);
+  const int64_t row = kMode == 1 ? gathered_position(g, nth) : nth;  // workspace position
+  double t[MIST_ROW_TERMS];  // compile-time indices only: registers
+  row_terms_of<kFromKeys>(prob, g, (uint32_t)row, key_terms, lds_gpu_gpu, I, t);
 
   if (kMode == 1) {  // scattered rows: every lane writes its own
     if ((int)threadIdx.x < rows_here) {
@@ -777,7 +889,6 @@ __global__ __launch_bounds__(kTermsBlock) void row_terms_kernel(
     }
     return;
   }
-  if (kMode == 2) lds_skip[threadIdx.x] = is_scout_pair(g, pair) ? 1 : 0;
   static_assert(kTermsBlock % kStageRows == 0 && kStageRows == 64, "a wavefront's rows are one stage");
   const int wave = threadIdx.x / kStageRows, lane = threadIdx.x % kStageRows;
   for (int stage_here = 0; stage_here < kTermsBlock / kStageRows; ++stage_here) {
@@ -788,17 +899,15 @@ __global__ __launch_bounds__(kTermsBlock) void row_terms_kernel(
     __syncthreads();
     const int stage_first = stage_here * kStageRows;
     const int stage_rows = min(kStageRows, rows_here - stage_first);  // <= 0: nothing left
-    double2 *__restrict__ dst = reinterpret_cast<double2 *>(
-        row_terms + (g->row_offset + block_first + stage_first) * MIST_ROW_TERMS);
-    for (int i = threadIdx.x; i < stage_rows * (MIST_ROW_TERMS / 2); i += kTermsBlock) {
-      const int r = i / (MIST_ROW_TERMS / 2);
-      if (kMode == 2 && lds_skip[stage_first + r]) continue;  // written by the kMode 1 launch
-      const int at = r * (MIST_ROW_TERMS + 1) + 2 * (i % (MIST_ROW_TERMS / 2));
-      dst[i] = make_double2(lds_out[at], lds_out[at + 1]);
+    store_rows(lds_out, stage_rows, row_terms + (g->row_offset + block_first + stage_first) * MIST_ROW_TERMS);
+    if (!kFloors) {
+      __syncthreads();
+      continue;
     }
     // Summary of the stage for the reduce kernel: thread = (column, one of kTermsBlock / 32
     // runs of the stage's rows); columns 0 .. MIST_T_GCB hold the minimum, column kStageMaxOut
-    // the maximum of MIST_T_OUT, the three behind it minima of post-layer terms.  The runs of a wavefront meet by shuffle, the wavefronts in LDS.
+    // the maximum of MIST_T_OUT, the three behind it minima of post-layer terms.  The runs of a
+    // wavefront meet by shuffle, the wavefronts in LDS.
     constexpr int kRuns = kTermsBlock / kStageFloorPitch, kRunRows = kStageRows / kRuns;
     const int col = threadIdx.x & (kStageFloorPitch - 1), run = threadIdx.x / kStageFloorPitch;
     const int src_col = col == kStageMaxOut ? MIST_T_OUT
@@ -820,20 +929,162 @@ __global__ __launch_bounds__(kTermsBlock) void row_terms_kernel(
     lo_v = fmin(lo_v, __shfl_xor(lo_v, kStageFloorPitch));
     hi_v = fmax(hi_v, __shfl_xor(hi_v, kStageFloorPitch));
     if (wave > 0 && lane < kStageFloorPitch) {
-      lds_part[wave - 1][0][col] = lo_v;
-      lds_part[wave - 1][1][col] = hi_v;
+      lds_part[wave - 1][0][kFloors ? col : 0] = lo_v;
+      lds_part[wave - 1][1][kFloors ? col : 0] = hi_v;
     }
     __syncthreads();  // every read of this stage is done; the other wavefronts' parts are in LDS
     if (wave == 0 && lane < kStageFloorPitch && stage_rows > 0) {
 #pragma unroll
       for (int w = 0; w < kTermsBlock / kStageRows - 1; ++w) {
-        lo_v = fmin(lo_v, lds_part[w][0][col]);
-        hi_v = fmax(hi_v, lds_part[w][1][col]);
+        lo_v = fmin(lo_v, lds_part[w][0][kFloors ? col : 0]);
+        hi_v = fmax(hi_v, lds_part[w][1][kFloors ? col : 0]);
       }
       const int64_t slot = stage_floor_slot(g, (int)(g - groups), block_first / kStageRows + stage_here);
       stage_floor[slot * kStageFloorPitch + col] = col == kStageMaxOut ? hi_v : lo_v;
     }
   }
+}
+
+// Stage summaries of every row, from the key terms and without the rows themselves: the search
+// reads the rows of a few stages (22B on 16x8: 67e6 rows, 18 GB, of which a tenth is read), which
+// are computed when it is known which (stage_rows_kernel).  Wavefront = stage, lane = row.  The columns a key decides are
+// taken from the stage's keys (16 of them as a rule), the six latencies and three memory columns
+// that see the optimizer ratio are evaluated per row and meet through LDS.  Bound by the float64
+// VALU: 8 evaluations of the interference model per row.
+constexpr int kFloorCols = 9;               // 6 latencies, PO, PWGO, MF
+constexpr int kFloorPitch = kStageRows + 1;
+__global__ __launch_bounds__(kTermsBlock) void stage_floor_kernel(
+    const MistProblem prob, const MistGroupDesc *__restrict__ groups, int n_groups,
+    const int32_t *__restrict__ block_prefix, double *__restrict__ stage_floor,
+    const double *__restrict__ key_terms) {
+  __shared__ __align__(16) double lds_factor[11][kFactorPitch];
+  __shared__ double lds_gpu_gpu[32];  // (of the tables, not read here)
+  __shared__ double lds_cols[kTermsBlock / kStageRows][kFloorCols * kFloorPitch];
+  __shared__ int lds_keys[kTermsBlock / kStageRows][kStageRows];
+  int local_block;
+  const MistGroupDesc *g = find_group(groups, block_prefix, n_groups, blockIdx.x, &local_block);
+  const int gi = __builtin_amdgcn_readfirstlane((int)(g - groups));
+  g = groups + gi;
+  InterferenceModel<true> I;
+  I.factors_tame = load_model_tables(prob, lds_factor, lds_gpu_gpu);
+  I.table = (LdsDouble *)&lds_factor[0][0];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kStageRows);
+  const int64_t stage = (int64_t)local_block * (kTermsBlock / kStageRows) + wave;
+  if (stage * kStageRows >= g->n_rows) return;
+  // (lanes past the end repeat the last row: minima do not change)
+  const uint32_t row = (uint32_t)min(stage * kStageRows + lane, g->n_rows - 1);
+  const RowParts at = parts_of_position(g, row);
+  const int key = (at.par * g->n_ao + at.ao) * g->n_pair + at.pair;
+  const double2 *__restrict__ kt =
+      reinterpret_cast<const double2 *>(key_terms + (g->key_offset + key) * MIST_KEY_TERMS);
+  double2 bwd[5], cols[3], links[3];
+#pragma unroll
+  for (int i = 0; i < 5; ++i) bwd[i] = kt[kKeyBwd / 2 + i];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) links[i] = kt[kKeySoW / 2 + i];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) cols[i] = kt[kKeyCols / 2 + i];
+  const double pWG = reinterpret_cast<const double *>(kt)[kKeyState0 + 2];
+  const double gather = reinterpret_cast<const double *>(kt)[kKeyGather];
+
+  const double *par = g->par[at.par];
+  const double oo = g->oo[at.oo];
+  const double O_shard = par[MIST_PAR_O] / (par[MIST_PAR_ORE] == 1.0 ? par[MIST_PAR_DP] : 1.0);
+  const double so_O = host_link_latency(prob.gpu_cpu, O_shard * oo);
+  const double si_O = host_link_latency(prob.cpu_gpu, O_shard * oo);
+  KeyInputs in = {};  // what the first forward phase reads of it
+  in.exec_fwd = par[MIST_PAR_EXEC_FWD];
+  in.extra_fwd = par[MIST_PAR_EXTRA_FWD];
+  in.E_f = in.exec_fwd - in.extra_fwd;
+  in.ore = 1.0;
+  in.AG_w = gather;
+  in.so_W = links[0].x;
+  in.si_G = links[0].y;
+  in.so_A_ck = links[1].x;
+  in.so_A_nock = links[1].y;
+  const FwdOperands op = fwd_operands(in, true, so_O, si_O);
+  double first, extra_pre;
+  fwd_common(I, in, op, true, prob.adv_first_block != 0, first, extra_pre);
+  double *mine = lds_cols[wave];
+  const bool accumulates = g->grad_accum != 1;
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    double layer, last, extra_post;
+    fwd_of_ckpt(I, in, op, k != 0, layer, last, extra_post);
+    // backward family of the last micro-batch: layer, first, last, extra_pre, extra_post
+    const double b_layer = k ? bwd[2].y : bwd[0].x, b_first = k ? bwd[3].x : bwd[0].y;
+    const double b_last = k ? bwd[3].y : bwd[1].x, b_pre = k ? bwd[4].x : bwd[1].y;
+    const double b_post = k ? bwd[4].y : bwd[2].x;
+    double v_layer = layer + b_layer;
+    double v_first = extra_pre + b_post + first + b_first;
+    double v_last = extra_post + b_pre + last + b_last;
+    if (accumulates) {  // the delta part
+      v_layer = v_layer - (k ? cols[0].x : cols[0].y);
+      v_first = v_first - (k ? cols[1].x : cols[1].y);
+      v_last = v_last - (k ? cols[2].x : cols[2].y);
+    }
+    mine[(0 + (1 - k)) * kFloorPitch + lane] = v_layer;
+    mine[(2 + (1 - k)) * kFloorPitch + lane] = v_first;
+    mine[(4 + (1 - k)) * kFloorPitch + lane] = v_last;
+  }
+  const double pO = O_shard * (1.0 - oo);
+  mine[6 * kFloorPitch + lane] = pO;
+  mine[7 * kFloorPitch + lane] = pWG + pO;
+  mine[8 * kFloorPitch + lane] = oo > 0.0 ? links[2].y : links[2].x;
+  // the stage's keys, each once
+  const bool new_key = lane == 0 || key != __shfl_up(key, 1);
+  const uint64_t new_keys = __ballot(new_key);
+  if (new_key) lds_keys[wave][__popcll(new_keys & ((1ull << lane) - 1ull))] = key;
+  const int n_keys = __popcll(new_keys);
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+
+  // ---- lane = (column of the keys, parity) ----
+  double lo = INFINITY, hi = 0.0;
+  {
+    const int col = lane & 31, parity = lane >> 5;
+    const double *__restrict__ src =
+        key_terms + g->key_offset * MIST_KEY_TERMS + kKeyCols + min(col, kKeyColsEnd - kKeyCols - 1);
+#pragma unroll 8
+    for (int i = parity; i < n_keys; i += 2) {
+      const double v = src[(int64_t)lds_keys[wave][i] * MIST_KEY_TERMS];
+      lo = fmin(lo, v);
+      hi = fmax(hi, v);
+    }
+    lo = fmin(lo, __shfl_xor(lo, 32));
+    hi = fmax(hi, __shfl_xor(hi, 32));
+  }
+  // ---- lane = (column of the rows, a quarter of them) ----
+  double row_lo = INFINITY;
+  {
+    const double *src = mine + min(lane & 15, kFloorCols - 1) * kFloorPitch + (lane >> 4) * 16;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) row_lo = fmin(row_lo, src[i]);
+    row_lo = fmin(row_lo, __shfl_xor(row_lo, 16));
+    row_lo = fmin(row_lo, __shfl_xor(row_lo, 32));
+  }
+  double *__restrict__ out = stage_floor + stage_floor_slot(g, gi, stage) * kStageFloorPitch;
+  // summary column `lane`: from which of the two, and from which column of it
+  const double mf = from_lane(row_lo, 8);
+  const bool latency_of_rows = accumulates ? (lane >= 6 && lane < 12) : lane < 6;
+  const int key_col = lane < 6 ? lane
+                      : lane <= MIST_T_BWD_STATES0 ? kKeyState0 - kKeyCols + (lane - MIST_T_FWD_STATES0)
+                      : lane == MIST_T_PWG ? kKeyState0 - kKeyCols + 2
+                      : lane <= MIST_T_D_NOCK ? kKeyState0 - kKeyCols + 3 + (lane - MIST_T_S_CK)
+                      : lane <= MIST_T_GCB ? kKeyPeaks - kKeyCols + (lane - MIST_T_FWD_PEAK)
+                      : lane == kStageMaxOut ? kKeyPeaks - kKeyCols + 2
+                                             : kKeyPost - kKeyCols + (lane - kStageMinOpb);
+  const double of_keys = __shfl(lo, max(key_col, 0));
+  const double max_out = from_lane(hi, kKeyPeaks - kKeyCols + 2);
+  const double of_rows = __shfl(row_lo, lane == MIST_T_PO ? 6 : lane == MIST_T_PWGO ? 7 : lane % 6);
+  double v = of_keys;
+  if (latency_of_rows || lane == MIST_T_PO || lane == MIST_T_PWGO) v = of_rows;
+  else if (lane >= 6 && lane < 12) v = 0.0;  // one micro-batch: no delta part
+  else if (lane == MIST_T_MF) v = mf;
+  else if (lane == MIST_T_MF_PP) v = mf + 0.025;
+  else if (lane == MIST_T_MF_BASE) v = mf + 0.025 + 0.01;
+  else if (lane == kStageMaxOut) v = max_out;
+  if (lane < kStageFloorPitch) out[lane] = v;
 }
 
 // ------------------------------------------------------------------------------------------
@@ -966,10 +1217,11 @@ constexpr int kSuperStages = 8;    // stages per second-level summary
 constexpr int kQueueShards = 64;   // counters of the item queue: one would serve an append in ~8 ns
 constexpr int kCounterPitch = 32;  // uint32 between counters: a cache line each
 constexpr int kNumXcd = 8;
-constexpr int kCounters = 2 * kQueueShards + kNumXcd;
+constexpr int kCounters = 3 * kQueueShards + kNumXcd;
 constexpr int kSeedThreads = 256;
 constexpr int kReduceThreads = 256;
 constexpr int kReduceBlocks = 2048;          // a multiple of kNumXcd
+constexpr int kStageRowsBlocks = 1024;       // four per CU, two stages at a time each
 constexpr int kSuperBlocks = 64;             // workgroups per group of the second-level summaries
 constexpr int kSeedLdsBytes = 40 * 1024;     // LDS aimed at per seed workgroup: four per CU
 constexpr int kSeedLdsMost = 160 * 1024;
@@ -992,7 +1244,12 @@ struct ReduceTables {
   // [kQueueShards][capacity]: group << 48 | tile << 32 | stage, what the filter and then what the
   // open launch left; pairs of the latter in which a row reached its minimum
   unsigned long long *item, *opened, *hit;
-  uint32_t *counter;         // at kCounterPitch: [kQueueShards] items, [kQueueShards] opened, [kNumXcd] drawn
+  // [kQueueShards][capacity]: group << 32 | stage of the stages opened, each once; stage_flag (one
+  // per stage summary) tells whether one is listed.  Null: the rows of all stages are there.
+  unsigned long long *listed;
+  uint32_t *stage_flag;
+  // at kCounterPitch: [kQueueShards] items, [kQueueShards] opened, [kQueueShards] listed, [kNumXcd] drawn
+  uint32_t *counter;
   uint32_t capacity;
   int n_samples;
 };
@@ -1071,21 +1328,6 @@ struct SampleSlots {
   int32_t at[MIST_MAX_SAMPLE_BATCH];
 };
 
-__device__ __forceinline__ double from_lane(double v, int lane) {
-  const unsigned long long u = (unsigned long long)__double_as_longlong(v);
-  const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)u, lane);
-  const uint32_t hi = __builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), lane);
-  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-__device__ __forceinline__ int from_lane(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
-__device__ __forceinline__ float from_lane(float v, int lane) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
-}
-__device__ __forceinline__ uint64_t from_lane(uint64_t v, int lane) {
-  const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)v, lane);
-  const uint32_t hi = __builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), lane);
-  return ((uint64_t)hi << 32) | lo;
-}
 // Smallest of the wavefront's values, in every lane (rows of 16 lanes, then across the rows).
 __device__ __forceinline__ uint32_t wave_min(uint32_t v) {
 #define MIST_MIN_DPP(CTRL) \
@@ -1548,7 +1790,7 @@ __device__ __forceinline__ int64_t super_floor_slot(const MistGroupDesc *g, int 
 }
 __global__ __launch_bounds__(256) void super_floor_kernel(const MistGroupDesc *__restrict__ groups, int n_groups,
                                                           const double *__restrict__ stage_floor,
-                                                          double *__restrict__ super_floor) {
+                                                          const ReduceTables tabs) {
   const int gi = blockIdx.y;
   const MistGroupDesc *g = groups + gi;
   const int64_t n_stages = (g->n_rows + kStageRows - 1) / kStageRows;
@@ -1563,7 +1805,8 @@ __global__ __launch_bounds__(256) void super_floor_kernel(const MistGroupDesc *_
       const double o = src[i * kStageFloorPitch + col];
       v = col == kStageMaxOut ? fmax(v, o) : fmin(v, o);
     }
-    super_floor[super_floor_slot(g, gi, super) * kStageFloorPitch + col] = v;
+    tabs.super_floor[super_floor_slot(g, gi, super) * kStageFloorPitch + col] = v;
+    if (tabs.listed != nullptr && col < n) tabs.stage_flag[stage_floor_slot(g, gi, super * kSuperStages) + col] = 0;
   }
 }
 
@@ -1780,6 +2023,53 @@ __global__ __launch_bounds__(kReduceThreads) void open_kernel(const MistProblem 
       const uint32_t to = atomicAdd(tabs.counter + (kQueueShards + shard) * kCounterPitch, 1u);
       tabs.opened[(int64_t)shard * tabs.capacity + to] = item;
       tabs.hit[(int64_t)shard * tabs.capacity + to] = 0;
+      if (tabs.listed != nullptr && atomicExch(tabs.stage_flag + stage_floor_slot(g, gi, stage), 1u) == 0) {
+        const uint32_t row_to = atomicAdd(tabs.counter + (2 * kQueueShards + shard) * kCounterPitch, 1u);
+        tabs.listed[(int64_t)shard * tabs.capacity + row_to] = (unsigned long long)gi << 32 | (uint32_t)stage;
+      }
+    }
+  }
+}
+
+// ---- rows of the opened stages ----
+// Workgroup = two stages of the list at a time.
+__global__ __launch_bounds__(kTermsBlock) void stage_rows_kernel(
+    const MistProblem prob, const MistGroupDesc *__restrict__ groups, double *__restrict__ row_terms,
+    const double *__restrict__ key_terms, const ReduceTables tabs) {
+  constexpr int kStages = kTermsBlock / kStageRows;
+  __shared__ double lds_out[kStageRows * (MIST_ROW_TERMS + 1)];
+  __shared__ __align__(16) double lds_factor[11][kFactorPitch];
+  __shared__ double lds_gpu_gpu[32];
+  const FlatQueue queue = flat_queue(tabs, 2);
+  if (blockIdx.x * kStages >= queue.total) return;
+  InterferenceModel<true> I;
+  I.factors_tame = load_model_tables(prob, lds_factor, lds_gpu_gpu);
+  I.table = (LdsDouble *)&lds_factor[0][0];
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kStageRows), lane = threadIdx.x % kStageRows;
+  for (uint32_t first = blockIdx.x * kStages; first < queue.total; first += gridDim.x * kStages) {
+    auto stage_of = [&](int k) {
+      return from_lane((uint64_t)tabs.listed[queue.at(min(first + k, queue.total - 1), tabs.capacity)], 0);
+    };
+    double t[MIST_ROW_TERMS];
+    {
+      const uint64_t its = stage_of(wave);
+      const MistGroupDesc *g = groups + (int)(its >> 32);
+      const int64_t row0 = (int64_t)(uint32_t)its * kStageRows;
+      row_terms_of<true>(prob, g, (uint32_t)min(row0 + lane, g->n_rows - 1), key_terms, lds_gpu_gpu, I, t);
+    }
+    for (int k = 0; k < kStages; ++k) {
+      __syncthreads();
+      if (wave == k) {
+#pragma unroll
+        for (int i = 0; i < MIST_ROW_TERMS; ++i) lds_out[lane * (MIST_ROW_TERMS + 1) + i] = t[i];
+      }
+      __syncthreads();
+      if (first + k >= queue.total) continue;
+      const uint64_t its = stage_of(k);
+      const MistGroupDesc *g = groups + (int)(its >> 32);
+      const int64_t row0 = (int64_t)(uint32_t)its * kStageRows;
+      store_rows(lds_out, (int)min((int64_t)kStageRows, g->n_rows - row0),
+                 row_terms + (g->row_offset + row0) * MIST_ROW_TERMS);
     }
   }
 }
@@ -2076,7 +2366,7 @@ __global__ __launch_bounds__(kReduceThreads, 3) void reduce_kernel(
   for (int k = 0; k < kNumXcd; ++k) {
     const int part = ((int)blockIdx.x + k) % kNumXcd;
     const uint32_t first = (uint32_t)(units * part / kNumXcd), n = (uint32_t)(units * (part + 1) / kNumXcd) - first;
-    uint32_t *drawn = tabs.counter + (2 * kQueueShards + part) * kCounterPitch;
+    uint32_t *drawn = tabs.counter + (3 * kQueueShards + part) * kCounterPitch;
     if (k > 0 && *drawn >= n) continue;
     auto draw = [&]() {
       uint32_t u = 0;
@@ -2840,11 +3130,14 @@ int mist_sizeof_group(void) { return (int)sizeof(MistGroupDesc); }
 int mist_reduce_p_tile(void) { return MIST_P_TILE; }
 double mist_incumbent_slack(void) { return kIncumbentSlack; }
 
+static bool has_key_terms(const MistProblem *problem, int n_groups, const double *d_key_terms) {
+  return d_key_terms != nullptr && problem->max_group_keys > 0 && n_groups <= 65535;
+}
 // key_terms_kernel over every group when the caller gave a key-term workspace and the bound the
 // grid needs; *launched tells whether the row-term kernel can read key terms.
 static int launch_key_terms(const MistProblem *problem, const MistGroupDesc *d_groups, int n_groups,
                             double *d_key_terms, hipStream_t stream, bool *launched) {
-  *launched = d_key_terms != nullptr && problem->max_group_keys > 0 && n_groups <= 65535;
+  *launched = has_key_terms(problem, n_groups, d_key_terms);
   if (!*launched) return 0;
   constexpr int kKeysPerBlock = kTermsBlock / 4;
   const unsigned blocks = (unsigned)((problem->max_group_keys + kKeysPerBlock - 1) / kKeysPerBlock);
@@ -2865,11 +3158,14 @@ int mist_row_terms(const MistProblem *problem, const MistGroupDesc *d_groups, in
   bool from_keys = false;
   if (int rc = launch_key_terms(problem, d_groups, n_groups, d_key_terms, (hipStream_t)stream, &from_keys))
     return rc;
-  if (from_keys)
+  if (from_keys) {
+    hipLaunchKernelGGL(stage_floor_kernel, dim3(n_blocks), dim3(kTermsBlock), 0, (hipStream_t)stream, *problem,
+                       d_groups, n_groups, d_block_prefix, d_stage_floor, d_key_terms);
+    MIST_HIP_CHECK(hipGetLastError());
     hipLaunchKernelGGL((row_terms_kernel<0, true>), dim3(n_blocks), dim3(kTermsBlock), 0,
                        (hipStream_t)stream, *problem, d_groups, n_groups, d_block_prefix, d_row_terms,
                        d_stage_floor, d_key_terms);
-  else
+  } else
     hipLaunchKernelGGL((row_terms_kernel<0, false>), dim3(n_blocks), dim3(kTermsBlock), 0,
                        (hipStream_t)stream, *problem, d_groups, n_groups, d_block_prefix, d_row_terms,
                        d_stage_floor, nullptr);
@@ -2895,9 +3191,9 @@ int64_t mist_stage_floor_doubles(int64_t total_rows, int n_groups) {
 }
 
 // Sections of the reduce workspace in `d_partial_cost` (doubles): the minima of n_samples samples,
-// the second-level summaries, the three item arrays, the queue's counters and a word per pair.
+// the second-level summaries, the four lists, their counters, a word per stage and one per pair.
 struct WorkspaceLayout {
-  int64_t best, supers, items, counters, changed, total;
+  int64_t best, supers, items, counters, flags, changed, total;
   int64_t capacity;  // items per shard
 };
 static WorkspaceLayout workspace_layout(int64_t cells, int64_t supers, int64_t items, int n_samples) {
@@ -2906,8 +3202,9 @@ static WorkspaceLayout workspace_layout(int64_t cells, int64_t supers, int64_t i
   w.best = 0;
   w.supers = cells * n_samples;
   w.items = w.supers + supers * kStageFloorPitch;
-  w.counters = w.items + 3 * kQueueShards * w.capacity;
-  w.changed = w.counters + kCounters * kCounterPitch / 2;
+  w.counters = w.items + 4 * kQueueShards * w.capacity;
+  w.flags = w.counters + kCounters * kCounterPitch / 2;
+  w.changed = w.flags + supers * kSuperStages / 2;
   w.total = w.changed + cells / 8 + 1;
   return w;
 }
@@ -2915,8 +3212,9 @@ int64_t mist_reduce_workspace_doubles(int64_t cells, int64_t supers, int64_t ite
   if (cells < 0 || supers < 0 || items < 0 || n_samples < 1) return -1;
   return workspace_layout(cells, supers, items, n_samples).total;
 }
+// rows_present: false = only the rows the scout pass gathers are, the others follow by need
 static int reduce_tables(const MistProblem *problem, int n_samples, double *d_partial_cost, int32_t *d_partial_index,
-                         ReduceTables *out) {
+                         ReduceTables *out, bool rows_present = true) {
   if (problem->reduce_cells < 1 || problem->reduce_supers < 1 || problem->reduce_items < 1 ||
       problem->reduce_max_p < 1)
     return fail(MIST_E_INVALID, "MistProblem.reduce_* sizes of the workspace are not set");
@@ -2929,6 +3227,8 @@ static int reduce_tables(const MistProblem *problem, int n_samples, double *d_pa
   out->item = reinterpret_cast<unsigned long long *>(d_partial_cost + w.items);
   out->opened = out->item + kQueueShards * w.capacity;
   out->hit = out->opened + kQueueShards * w.capacity;
+  out->listed = rows_present ? nullptr : out->hit + kQueueShards * w.capacity;
+  out->stage_flag = reinterpret_cast<uint32_t *>(d_partial_cost + w.flags);
   out->counter = reinterpret_cast<uint32_t *>(d_partial_cost + w.counters);
   out->changed = reinterpret_cast<uint32_t *>(d_partial_cost + w.changed);
   out->capacity = (uint32_t)w.capacity;
@@ -3011,7 +3311,7 @@ static int launch_seeds(const MistProblem *problem, const MistGroupDesc *d_group
 static int launch_super_floors(const MistGroupDesc *d_groups, int n_groups, const double *d_stage_floor,
                                const ReduceTables &tabs, void *stream) {
   hipLaunchKernelGGL(super_floor_kernel, dim3(kSuperBlocks, n_groups), dim3(256), 0, (hipStream_t)stream, d_groups,
-                     n_groups, d_stage_floor, tabs.super_floor);
+                     n_groups, d_stage_floor, tabs);
   MIST_HIP_CHECK(hipGetLastError());
   return 0;
 }
@@ -3019,13 +3319,19 @@ static int launch_super_floors(const MistGroupDesc *d_groups, int n_groups, cons
 // filter + open + reduce + resolve on seeded tables.
 static int launch_reduce(const MistProblem *problem, const MistGroupDesc *d_groups, int n_groups,
                          const int32_t *d_block_prefix, int n_blocks, const double *d_row_terms,
-                         const double *d_stage_floor, const RatioList &ratios, const ReduceTables &tabs, void *stream) {
+                         const double *d_stage_floor, const double *d_key_terms, const RatioList &ratios,
+                         const ReduceTables &tabs, void *stream) {
   hipLaunchKernelGGL(filter_kernel, dim3(xcd_padded_grid(n_blocks)), dim3(MIST_LC_TILE), 0, (hipStream_t)stream,
                      *problem, d_groups, n_groups, d_block_prefix, n_blocks, d_stage_floor, tabs.super_floor, ratios, tabs);
   MIST_HIP_CHECK(hipGetLastError());
   hipLaunchKernelGGL(open_kernel, dim3(kReduceBlocks), dim3(kReduceThreads), 0, (hipStream_t)stream, *problem,
                      d_groups, d_stage_floor, ratios, tabs);
   MIST_HIP_CHECK(hipGetLastError());
+  if (tabs.listed != nullptr) {
+    hipLaunchKernelGGL(stage_rows_kernel, dim3(kStageRowsBlocks), dim3(kTermsBlock), 0, (hipStream_t)stream, *problem,
+                       d_groups, const_cast<double *>(d_row_terms), d_key_terms, tabs);
+    MIST_HIP_CHECK(hipGetLastError());
+  }
   const int row_pitch = slots_of(problem->reduce_max_p);
   const size_t lds = tabs.n_samples == 1 ? sizeof(double) * row_pitch * (kReduceThreads / 64) : 0;
   if (lds > kSeedLdsMost) return fail(MIST_E_INVALID, "%d pre-saved micro-batch values exceed the LDS", problem->reduce_max_p);
@@ -3082,7 +3388,7 @@ int mist_eval_reduce(const MistProblem *problem, const MistGroupDesc *d_groups, 
                             stream))
     return rc;
   if (int rc = launch_super_floors(d_groups, n_groups, d_stage_floor, tabs, stream)) return rc;
-  return launch_reduce(problem, d_groups, n_groups, d_block_prefix, n_blocks, d_row_terms, d_stage_floor, ratios, tabs,
+  return launch_reduce(problem, d_groups, n_groups, d_block_prefix, n_blocks, d_row_terms, d_stage_floor, nullptr, ratios, tabs,
                        stream);
 }
 
@@ -3158,8 +3464,8 @@ int mist_eval_reduce_samples(const MistProblem *problem, const MistGroupDesc *d_
   if (int rc = launch_seeds(problem, d_groups, n_groups, d_row_terms, all, n_scout_blocks > 0, tabs, d_partial_cost, stream))
     return rc;
   if (int rc = launch_super_floors(d_groups, n_groups, d_stage_floor, tabs, stream)) return rc;
-  if (int rc = launch_reduce(problem, d_groups, n_groups, d_block_prefix, n_blocks, d_row_terms, d_stage_floor, all, tabs,
-                             stream))
+  if (int rc = launch_reduce(problem, d_groups, n_groups, d_block_prefix, n_blocks, d_row_terms, d_stage_floor, nullptr, all,
+                             tabs, stream))
     return rc;
   return launch_finalize(problem, d_groups, n_groups, d_row_terms, tabs, sample_index, tables, stream);
 }
@@ -3253,11 +3559,12 @@ int mist_intra_stage_eval_samples(const MistProblem *problem, const MistGroupDes
   for (int i = 0; i < n_samples; ++i)
     if (!(ratios[i] >= 0.0)) return fail(MIST_E_INVALID, "ratio %d must be non-negative", i);
   hipStream_t main_stream = (hipStream_t)stream;
-  // The seeds read a few hundred rows per group and leave most of the GPU idle; the row terms of
-  // everything else are computed beside them.  Stream order: [terms of the gathered rows] -> side
-  // stream: seeds of the first batch of samples || this stream: all other row terms, second-level
-  // summaries -> filter, reduce, resolve, finalize; further batches one after the other.
-  const bool overlap = n_scout_blocks > 0 && problem->max_scout_rows > 0;
+  // The seeds read a few hundred rows per group and leave most of the GPU idle; the stage summaries
+  // are computed beside them.  Stream order: [terms of the gathered rows] -> side stream: seeds of
+  // the first batch of samples || this stream: key terms, summaries -> filter, open, rows of the
+  // opened stages, reduce, resolve, finalize; further batches one after the other.
+  const bool overlap = n_scout_blocks > 0 && problem->max_scout_rows > 0 && has_key_terms(problem, n_groups, d_key_terms);
+  const bool by_need = overlap;
   OverlapStreams *os = nullptr;
   std::unique_lock<std::mutex> enqueue_guard;
   if (overlap) {
@@ -3272,19 +3579,13 @@ int mist_intra_stage_eval_samples(const MistProblem *problem, const MistGroupDes
     MIST_HIP_CHECK(hipGetLastError());
     MIST_HIP_CHECK(hipEventRecord(os->rows_ready, main_stream));
     MIST_HIP_CHECK(hipStreamWaitEvent(os->side, os->rows_ready, 0));
-    // (the other row terms are queued first: the seeds are several launches, and this stream would
-    // idle while they are made)
+    // (the summaries are queued first: the seeds are several launches, and this stream would idle
+    // while they are made)
     bool from_keys = false;
     if (int rc = launch_key_terms(problem, d_groups, n_groups, d_key_terms, main_stream, &from_keys))
       return rc;
-    if (from_keys)
-      hipLaunchKernelGGL((row_terms_kernel<2, true>), dim3(n_terms_blocks), dim3(kTermsBlock), 0,
-                         main_stream, *problem, d_groups, n_groups, d_terms_block_prefix, d_row_terms,
-                         d_stage_floor, d_key_terms);
-    else
-      hipLaunchKernelGGL((row_terms_kernel<2, false>), dim3(n_terms_blocks), dim3(kTermsBlock), 0,
-                         main_stream, *problem, d_groups, n_groups, d_terms_block_prefix, d_row_terms,
-                         d_stage_floor, nullptr);
+    hipLaunchKernelGGL(stage_floor_kernel, dim3(n_terms_blocks), dim3(kTermsBlock), 0, main_stream, *problem, d_groups,
+                       n_groups, d_terms_block_prefix, d_stage_floor, d_key_terms);
     MIST_HIP_CHECK(hipGetLastError());
   } else {
     if (int rc = mist_row_terms(problem, d_groups, n_groups, d_terms_block_prefix, n_terms_blocks,
@@ -3294,7 +3595,7 @@ int mist_intra_stage_eval_samples(const MistProblem *problem, const MistGroupDes
   for (int first = 0; first < n_samples; first += sample_batch) {
     const int count = std::min(sample_batch, n_samples - first);
     ReduceTables tabs;
-    if (int rc = reduce_tables(problem, count, d_partial_cost, d_partial_index, &tabs)) return rc;
+    if (int rc = reduce_tables(problem, count, d_partial_cost, d_partial_index, &tabs, !by_need)) return rc;
     RatioList list = {};
     for (int i = 0; i < count; ++i) list.r[i] = ratios[first + i];
     const bool aside = overlap && first == 0;
@@ -3306,7 +3607,7 @@ int mist_intra_stage_eval_samples(const MistProblem *problem, const MistGroupDes
     if (int rc = launch_super_floors(d_groups, n_groups, d_stage_floor, tabs, stream)) return rc;
     if (aside) MIST_HIP_CHECK(hipStreamWaitEvent(main_stream, os->seeds_done, 0));
     if (int rc = launch_reduce(problem, d_groups, n_groups, d_reduce_block_prefix, n_reduce_blocks, d_row_terms,
-                               d_stage_floor, list, tabs, stream))
+                               d_stage_floor, d_key_terms, list, tabs, stream))
       return rc;
     if (int rc = launch_finalize(problem, d_groups, n_groups, d_row_terms, tabs, sample_index + first, tables, stream))
       return rc;

@@ -43,9 +43,10 @@ SCOUT_TIGHT_FRACTION = 0.3
 SCOUT_TIGHT_PAIRS = 3
 # Upper bound of the row-term workspace (272 bytes per candidate row): the groups of a tuner call
 # go through the kernels in batches of consecutive groups whose rows fit it (a group larger than
-# the bound is a batch of its own).  GPT-7B (0.88 GB) and LLaMA-13B (1.4 GB) are one batch,
-# GPT-22B (18.4 GB of row terms) ten; with more than one batch two such workspaces alternate.
-ROW_TERMS_BUDGET_BYTES = 2 << 30
+# the bound is a batch of its own); with more than one batch two such workspaces alternate.  Only
+# the rows that the search opens are written, and a launch per plan keeps the GPU fuller than ten
+# of them: GPT-22B (18.4 GB) as nine batches of 2 GB takes 23.4 ms, as one 19.9 ms.
+ROW_TERMS_BUDGET_BYTES = 24 << 30
 # Minima tables (12 bytes per (l, c) pair, variant, p and sample) the launches of a multi-sample call
 # may hold: more samples go through them in batches.
 MINIMA_BYTES = 8 << 30
