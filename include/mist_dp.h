@@ -175,13 +175,23 @@ int mist_dp_first_batch_index(int k, int n_avail, int first_chunk, int first_lea
  *   (end layer, n, m, ckpt), pre-filled with -1 by the caller.
  * d_scratch: mist_dp_scratch_floats() floats (four (L+1)(D+1) state planes per instance plus the
  * reachable row range of every device column).
- * For tests the environment variable MIST_DP_FORCE_SCHEDULE (step | fused | plane) overrides the
- * choice of schedule; a shape the forced schedule does not support fails with MIST_E_INVALID. */
+ * For tests the environment variable MIST_DP_FORCE_SCHEDULE (step | fused | plane | history) overrides
+ * the choice of schedule; a shape the forced schedule does not support fails with MIST_E_INVALID. */
 int64_t mist_dp_scratch_floats(const MistDpShape *shape, int n_tmax);
 int mist_dp_run(const MistDpShape *shape, const MistDpCosts *costs, const float *d_tmax,
                 const int32_t *d_g_index, int n_tmax, int mode, int32_t *d_best_s,
                 float *d_best_sum, float *d_stage_max, int32_t *d_argmin, float *d_scratch,
                 void *stream);
+
+/* mist_dp_run() with a scratch whose size is given: with the mist_dp_scratch_floats_sized() floats
+ * of a batch (at least mist_dp_scratch_floats() and, beyond that, at most 1 GiB), one without
+ * back-pointers may keep the planes of all stage counts and look the winners up on the answer's
+ * path alone.  Same arguments and results otherwise. */
+int64_t mist_dp_scratch_floats_sized(const MistDpShape *shape, int n_tmax);
+int mist_dp_run_sized(const MistDpShape *shape, const MistDpCosts *costs, const float *d_tmax,
+                      const int32_t *d_g_index, int n_tmax, int mode, int32_t *d_best_s,
+                      float *d_best_sum, float *d_stage_max, int32_t *d_argmin, float *d_scratch,
+                      int64_t scratch_floats, void *stream);
 
 /* mist_dp_run() for callers that cannot allocate device memory (code under HIP graph capture,
  * serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  Same

@@ -4,9 +4,10 @@
 // of one s are independent; each is scanned by one thread (or a team of lanes) that walks its
 // (mesh, end layer, ckpt) candidates in the reference's order with float32 adds and strict "<",
 // so ties resolve exactly as in the reference loop nest (mist/analyzer/inter_tuning.py:298-333).
-// Two schedules: one launch per s with the states of all instances spread over the GPU
-// (dp_step_kernel), or one workgroup per instance that keeps its state planes in LDS and loops
-// over s itself (dp_fused_kernel).
+// Schedules: one launch per s with the states of all instances spread over the GPU
+// (dp_step_kernel); one workgroup per instance that loops over s itself, with its state planes in
+// LDS (dp_fused_kernel) or only the one it reads at random (dp_plane_kernel); and, where no
+// back-pointers are asked for, dp_history_kernel, which finds winners on the answer's path alone.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -15,6 +16,7 @@
 #include <cstring>
 #include <cstdlib>
 #include <map>
+#include <tuple>
 #include <mutex>
 #include <utility>
 
@@ -1204,6 +1206,236 @@ __global__ __launch_bounds__(kDpPlaneThreads) void dp_plane_kernel(
   }
 }
 
+// ------------------------------------------------------------------------------------------
+// The recurrence without per-state winners.  A caller of a scan batch wants three numbers per
+// instance (stage count, sum, stage maximum), so only the winners on ONE path matter; the kernels
+// above find the winner of every state, carry it through a plane of maxima and walk its ckpt row
+// in the tables (a gather of up to 64 cache lines per load: about half of their time).  Here a
+// state is only the minimum (add + min per candidate, any order), every plane F(s) is kept in the
+// workgroup's history, and the answer's path is read back from it at the end: per stage the first
+// (mesh, end layer) in the reference's order that attains the value, then the first ckpt count.
+// One workgroup takes instance after instance, so the history is per workgroup and not per
+// instance.  A wavefront owns a start layer with all device counts; F(s - 1) lies in LDS without
+// what no scan can read (row 0, row L, column D), which lets two workgroups of 80 layers x 256
+// devices share a compute unit (bound: LDS reads and the add + min behind them, 13 instructions per
+// admissible candidate of 256 states).  Column 0 is +inf: F(s - 1) of zero devices is reachable for
+// s = 1 only, which has a step of its own, and lanes with d < n m read it.
+// Threshold batches of one search, dp_plane / dp_fused -> here: 80 x 256 (four batches, 1100
+// instances) 13.2 -> 5.2 ms, 48 x 128 (600) 2.9 -> 0.7 ms, 40 x 64 1.06 -> 0.40 ms, 32 x 32 0.32 ->
+// 0.20 ms; bottleneck batches of 40-48 instances 2.2 -> 1.65, 0.67 -> 0.26, 0.33 -> 0.16 and 0.16 ->
+// 0.11 ms.
+// ------------------------------------------------------------------------------------------
+constexpr int kDpHistoryThreads = 1024;
+constexpr int kDpHistoryBatch = 8;   // meshes whose row minima a lane has in flight
+constexpr int kDpUnreached = 1 << 20;
+// LDS of a workgroup: F(s - 1), the smallest reached device count per row (two steps), the stage
+// values of the answer's path, three flags
+inline size_t dp_history_lds(int L, int D, int max_stages) {
+  const size_t f = std::max((size_t)(L - 1) * D, (size_t)(kDpHistoryThreads / 64) * 2 * (L + 1));
+  return (f + 2 * (size_t)L + (size_t)max_stages + 3) * sizeof(float);
+}
+
+template <bool kBottleneck, int kCols>
+__global__ __launch_bounds__(kDpHistoryThreads, 8) void dp_history_kernel(
+    const MistDpShape shape, const MistDpCosts tabs, const float *__restrict__ tmax_list,
+    const int32_t *__restrict__ g_list, int n_instances, float *__restrict__ histories,
+    int32_t *__restrict__ best_s_out, float *__restrict__ best_sum_out,
+    float *__restrict__ stage_max_out) {
+  extern __shared__ float dp_lds[];
+  const int L = shape.num_layers, D = shape.num_devices, Q = shape.num_mesh;
+  const int S = shape.max_stages, plane = L * D, tri = dp_triangle(L);
+  const int n_waves = kDpHistoryThreads / 64;
+  const int n_f = max((L - 1) * D, n_waves * 2 * (L + 1));
+  float *f = dp_lds;  // F(s - 1) of row r >= 1, column c < D: f[(r - 1) * D + c]
+  int32_t *first_col = reinterpret_cast<int32_t *>(dp_lds + n_f);  // [2][L]
+  float *path_value = dp_lds + n_f + 2 * L;                        // [S]
+  int32_t *reached = first_col + 2 * L + S;                        // [3]
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // F(s) of start layer k, d devices: history[(s - 1) * plane + k * D + d - 1]
+  float *history = histories + (int64_t)blockIdx.x * S * plane;
+  for (int t = blockIdx.x; t < n_instances; t += gridDim.x) {
+    const int64_t g = g_list[t];
+    if (g < 0) {  // an empty slot of the batch
+      if (threadIdx.x == 0) {
+        best_s_out[t] = -1;
+        best_sum_out[t] = INFINITY;
+        stage_max_out[t] = 0.0f;
+      }
+      continue;
+    }
+    const float *__restrict__ relaid = tabs.stage_min + g * tabs.stage_min_g_stride;
+    // the bottleneck DP has no threshold of its own: an upper bound of its answer serves as one
+    const float t_max = kBottleneck
+                            ? fminf(kDpNoThreshold, dp_uniform_mesh_bound(shape, relaid, f, n_f, reached))
+                            : tmax_list[t];
+    __syncthreads();  // (the bound was read by every wavefront)
+    if (threadIdx.x < 3) reached[threadIdx.x] = 0;
+    __syncthreads();
+    float answer_sum = INFINITY;  // of the lane that owns (k = 0, d = D): wavefront 0's first task
+    int answer_s = -1;
+    for (int s = 1; s <= S; ++s) {
+      const float *__restrict__ block = relaid + (int64_t)(s - 1) * Q * tri;
+      float *__restrict__ out = history + (int64_t)(s - 1) * plane;
+      const int32_t *col_prev = first_col + (s & 1) * L;
+      int32_t *col_cur = first_col + ((s & 1) ^ 1) * L;
+      // the last stage count has one state anybody reads
+      const int n_tasks = s == S ? 1 : L - s + 1;
+      if (threadIdx.x == 0) reached[(s + 1) % 3] = 0;
+      for (int k_up = wave, round = 0; k_up < n_tasks; k_up += n_waves, ++round) {
+        // snake order: the cost of a task falls with k
+        int k = (round & 1) ? round * n_waves + n_waves - 1 - wave : k_up;
+        if ((round + 1) * n_waves > n_tasks) k = k_up;  // the last, partial round
+        const float *__restrict__ row = block + dp_triangle_row(L, k) - k;  // row[q * tri + i]
+        float best[kCols];
+#pragma unroll
+        for (int j = 0; j < kCols; ++j) best[j] = INFINITY;
+        if (s == 1) {
+          for (int q = 0; q < Q; ++q) {
+            const int nm = shape.mesh_n[q] * shape.mesh_m[q];
+            const float rmin = row[q * tri + L - 1];
+            const float target = kBottleneck ? fmaxf(rmin, 0.0f) : rmin + 0.0f;
+#pragma unroll
+            for (int j = 0; j < kCols; ++j)
+              if (1 + lane + 64 * j == nm && rmin <= t_max) best[j] = fminf(best[j], target);
+          }
+        } else {
+          for (int i0 = k; i0 <= L - s; i0 += 64) {  // end layers behind which s - 1 stages fit
+            const int i_mine = i0 + lane;
+            const bool in_row = i_mine <= L - s;
+            const int col = in_row ? col_prev[i_mine + 1] : kDpUnreached;
+            for (int q0 = 0; q0 < Q; q0 += kDpHistoryBatch) {
+              float r[kDpHistoryBatch];
+#pragma unroll
+              for (int u = 0; u < kDpHistoryBatch; ++u)
+                r[u] = in_row && q0 + u < Q ? row[(q0 + u) * tri + i_mine] : INFINITY;
+#pragma unroll
+              for (int u = 0; u < kDpHistoryBatch; ++u) {
+                if (q0 + u >= Q) break;
+                const int nm = shape.mesh_n[q0 + u] * shape.mesh_m[q0 + u];
+                // admissible, and its successor reached on what the mesh leaves: the same for
+                // every lane
+                unsigned long long todo = __ballot(r[u] <= t_max && col + nm <= D);
+                if (todo == 0) continue;
+                const float *from[kCols];
+#pragma unroll
+                for (int j = 0; j < kCols; ++j) {
+                  const int d = 1 + lane + 64 * j;
+                  from[j] = f + (d <= D && d > nm ? d - nm : 0);
+                }
+                while (todo != 0) {
+                  const int bit = __ffsll(todo) - 1;
+                  todo &= todo - 1;
+                  const float rmin = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r[u]), bit));
+                  const int at = (i0 + bit) * D;  // row i + 1
+#pragma unroll
+                  for (int j = 0; j < kCols; ++j) {
+                    const float prev = from[j][at];
+                    best[j] = fminf(best[j], kBottleneck ? fmaxf(rmin, prev) : rmin + prev);
+                  }
+                }
+              }
+            }
+          }
+        }
+        int col = kDpUnreached;
+#pragma unroll
+        for (int j = kCols - 1; j >= 0; --j) {
+          const int d = 1 + lane + 64 * j;
+          if (d <= D) out[k * D + d - 1] = best[j];
+          const unsigned long long finite = __ballot(d <= D && best[j] < INFINITY);
+          if (finite != 0) col = 64 * j + __ffsll(finite);
+          // first s wins ties (inter_tuning.py:335-340)
+          if (k == 0 && d == D && best[j] < answer_sum) {
+            answer_sum = best[j];
+            answer_s = s;
+          }
+        }
+        if (lane == 0) {
+          col_cur[k] = col;
+          if (col != kDpUnreached) reached[s % 3] = 1;
+        }
+      }
+      __syncthreads();  // every scan of F(s - 1) is done, F(s) is in the history
+      if (s == S || reached[s % 3] == 0) break;  // (no state: none behind it either)
+      for (int k = 1 + wave; k <= L - s; k += n_waves) {
+        if (col_cur[k] == kDpUnreached) continue;
+        for (int c = lane; c < D; c += 64) f[(k - 1) * D + c] = c == 0 ? INFINITY : out[k * D + c - 1];
+      }
+      __syncthreads();
+    }
+    if (wave == 0) {
+      const int owner = (D - 1) & 63;
+      answer_s = __builtin_amdgcn_readlane(answer_s, owner);
+      answer_sum = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(answer_sum), owner));
+      const int64_t off[4] = {g * tabs.g_stride[0], g * tabs.g_stride[1], g * tabs.g_stride[2],
+                              g * tabs.g_stride[3]};
+      float best = answer_sum;
+      int k = 0, d = D;
+      for (int s = answer_s; s >= 1; --s) {
+        const float *__restrict__ block =
+            relaid + (int64_t)(s - 1) * Q * tri + dp_triangle_row(L, k) - k;
+        int arg_q = -1, arg_i = -1;
+        float arg_rmin = 0.0f, arg_prev = 0.0f;
+        for (int q = 0; q < Q && arg_q < 0; ++q) {
+          const int left = d - shape.mesh_n[q] * shape.mesh_m[q];
+          if (left < (s == 1 ? 0 : 1) || (s == 1 && left != 0)) continue;
+          for (int i0 = s == 1 ? L - 1 : k; i0 <= L - s; i0 += 64) {
+            const int i = i0 + lane;
+            float rmin = INFINITY, prev = INFINITY;
+            if (i <= L - s) {
+              rmin = block[q * tri + i];
+              prev = s == 1 ? 0.0f : history[(int64_t)(s - 2) * plane + (i + 1) * D + left - 1];
+            }
+            const float target = kBottleneck ? fmaxf(rmin, prev) : rmin + prev;
+            const unsigned long long hit = __ballot(rmin <= t_max && target == best);
+            if (hit != 0) {
+              const int bit = __ffsll(hit) - 1;
+              arg_q = q;
+              arg_i = i0 + bit;
+              arg_rmin = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(rmin), bit));
+              arg_prev = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(prev), bit));
+              break;
+            }
+          }
+        }
+        if (arg_q < 0) break;  // (a reached state has a candidate that attains its value)
+        float value = arg_rmin;
+        if (!kBottleneck) {
+          const DpRowRef ref = dp_row_ref(shape, off, s - 1, k, arg_q, arg_i);
+          const float *__restrict__ costs = dp_table(tabs, ref.v, false) + ref.at;
+          const int j_begin = shape.ckpt_rule == MIST_DP_CKPT_ALL ? arg_i - k + 1 : 0;
+          const int j_end = dp_j_last(shape, k, arg_i);
+          value = 0.0f;
+          for (int j0 = j_begin; j0 <= j_end; j0 += 64) {
+            const float cost = j0 + lane <= j_end ? costs[j0 + lane] : INFINITY;
+            const unsigned long long hit = __ballot(cost <= t_max && cost + arg_prev == best);
+            if (hit != 0) {
+              value = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cost), __ffsll(hit) - 1));
+              break;
+            }
+          }
+        }
+        if (lane == 0) path_value[s - 1] = value;
+        d -= shape.mesh_n[arg_q] * shape.mesh_m[arg_q];
+        k = arg_i + 1;
+        best = arg_prev;
+      }
+      if (lane == 0) {
+        // threshold: largest stage cost; bottleneck: the sum, added from the last stage on as the
+        // threshold DP adds it
+        float value = 0.0f;
+        for (int s = 0; s < answer_s; ++s)
+          value = kBottleneck ? path_value[s] + value : fmaxf(value, path_value[s]);
+        best_s_out[t] = answer_s;
+        best_sum_out[t] = answer_sum;
+        stage_max_out[t] = value;
+      }
+    }
+    __syncthreads();  // the next instance writes the history and LDS
+  }
+}
+
 // Follows the back-pointers of each instance from (best_s, layer 0, all devices) and writes its
 // stages in pipeline order (inter_tuning.py:341-355); one thread per instance.  Only entries the
 // DP wrote are read: a state with a finite value has a winner, and so has every successor on
@@ -1302,6 +1534,50 @@ size_t fused_lds_limit(int mode) {
   if (it == known.end())
     it = known.emplace(key, mode == MIST_DP_BOTTLENECK ? fused_lds_limit_of<true>()
                                                        : fused_lds_limit_of<false>()).first;
+  return it->second;
+}
+
+// Workgroups, floats of history and LDS of dp_history_kernel for a batch; n_wg 0: not this shape.
+// Two workgroups per compute unit; a history that would take more than a GiB for one workgroup
+// per compute unit is left to the schedules that keep two planes.
+struct HistoryPlan {
+  int n_wg = 0;
+  int64_t floats = 0;
+  size_t lds = 0;
+};
+constexpr int64_t kDpHistoryMaxFloats = (int64_t)256 << 20;
+constexpr int kDpComputeUnits = 256;
+HistoryPlan history_plan(const MistDpShape &shape, int n_tmax) {
+  HistoryPlan plan;
+  if (shape.free_devices != 0 || shape.num_devices > 256 || shape.max_stages < 1) return plan;
+  plan.lds = dp_history_lds(shape.num_layers, shape.num_devices, shape.max_stages);
+  if (plan.lds > kDpLdsPerCu) return plan;
+  const int64_t each = (int64_t)shape.max_stages * shape.num_layers * shape.num_devices;
+  const int64_t n_wg = std::min<int64_t>(std::min(n_tmax, 2 * kDpComputeUnits), kDpHistoryMaxFloats / each);
+  if (n_wg < std::min(n_tmax, kDpComputeUnits)) return plan;
+  plan.n_wg = (int)n_wg;
+  plan.floats = n_wg * each;
+  return plan;
+}
+template <bool kBottleneck>
+const void *history_kernel(int cols) {
+  return cols == 1   ? reinterpret_cast<const void *>(&dp_history_kernel<kBottleneck, 1>)
+         : cols == 2 ? reinterpret_cast<const void *>(&dp_history_kernel<kBottleneck, 2>)
+         : cols == 3 ? reinterpret_cast<const void *>(&dp_history_kernel<kBottleneck, 3>)
+                     : reinterpret_cast<const void *>(&dp_history_kernel<kBottleneck, 4>);
+}
+size_t history_lds_limit(int mode, int cols) {
+  // per device: the attribute belongs to the device's copy of the kernel
+  static std::mutex lock;
+  static std::map<std::tuple<int, int, int>, size_t> known;
+  int device = 0;
+  if (hipGetDevice(&device) != hipSuccess) return 0;
+  std::lock_guard<std::mutex> guard(lock);
+  const auto key = std::make_tuple(device, mode, cols);
+  auto it = known.find(key);
+  if (it == known.end())
+    it = known.emplace(key, lds_limit_of(mode == MIST_DP_BOTTLENECK ? history_kernel<true>(cols)
+                                                                    : history_kernel<false>(cols))).first;
   return it->second;
 }
 
@@ -1600,10 +1876,24 @@ int64_t mist_dp_scratch_floats(const MistDpShape *shape, int n_tmax) {
          (int64_t)6 * n_tmax * (shape->num_devices + 1);
 }
 
+int64_t mist_dp_scratch_floats_sized(const MistDpShape *shape, int n_tmax) {
+  const int64_t least = mist_dp_scratch_floats(shape, n_tmax);
+  return least < 0 ? least : std::max(least, history_plan(*shape, n_tmax).floats);
+}
+
 int mist_dp_run(const MistDpShape *shape, const MistDpCosts *costs, const float *d_tmax,
                 const int32_t *d_g_index, int n_tmax, int mode, int32_t *d_best_s,
                 float *d_best_sum, float *d_stage_max, int32_t *d_argmin, float *d_scratch,
                 void *stream) {
+  return mist_dp_run_sized(shape, costs, d_tmax, d_g_index, n_tmax, mode, d_best_s, d_best_sum,
+                           d_stage_max, d_argmin, d_scratch, mist_dp_scratch_floats(shape, n_tmax),
+                           stream);
+}
+
+int mist_dp_run_sized(const MistDpShape *shape, const MistDpCosts *costs, const float *d_tmax,
+                const int32_t *d_g_index, int n_tmax, int mode, int32_t *d_best_s,
+                float *d_best_sum, float *d_stage_max, int32_t *d_argmin, float *d_scratch,
+                int64_t scratch_floats, void *stream) {
   if (int rc = check_run_arguments(shape, costs, d_tmax, d_g_index, n_tmax, mode, d_best_s,
                                    d_best_sum, d_stage_max))
     return rc;
@@ -1631,8 +1921,33 @@ int mist_dp_run(const MistDpShape *shape, const MistDpCosts *costs, const float 
   const bool force_step = forced && !strcmp(forced, "step");
   const bool force_fused = forced && !strcmp(forced, "fused");
   const bool force_plane = forced && !strcmp(forced, "plane");
-  if (forced && *forced && !force_step && !force_fused && !force_plane)
-    return fail(MIST_E_INVALID, "MIST_DP_FORCE_SCHEDULE=%s: expected step, fused or plane", forced);
+  const bool force_history = forced && !strcmp(forced, "history");
+  if (forced && *forced && !force_step && !force_fused && !force_plane && !force_history)
+    return fail(MIST_E_INVALID, "MIST_DP_FORCE_SCHEDULE=%s: expected step, fused, plane or history", forced);
+  // Without back-pointers and with room for the history that schedule runs: it was the fastest at
+  // every shape and batch size measured (33 x 33 to 81 x 257 states, 28 to 2304 instances).
+  if (!(force_step || force_fused || force_plane)) {
+    const HistoryPlan plan = history_plan(*shape, n_tmax);
+    const int cols = (shape->num_devices + 63) / 64;
+    const bool possible = plan.n_wg > 0 && d_argmin == nullptr && costs->stage_min != nullptr &&
+                          plan.floats <= scratch_floats && plan.lds <= history_lds_limit(mode, cols);
+    if (force_history && !possible)
+      return fail(MIST_E_INVALID, "forced history schedule: needs stage_min, consumed devices, D <= 256, no "
+                  "back-pointers, %lld scratch floats and %zu B of LDS", (long long)plan.floats, plan.lds);
+    if (possible) {
+      const MistDpShape shape_arg = *shape;
+      const MistDpCosts costs_arg = *costs;
+      int n_arg = n_tmax;
+      void *args[] = {(void *)&shape_arg, (void *)&costs_arg, &d_tmax, &d_g_index, &n_arg,
+                      &d_scratch, &d_best_s, &d_best_sum, &d_stage_max};
+      MIST_HIP_CHECK(hipLaunchKernel(mode == MIST_DP_BOTTLENECK ? history_kernel<true>(cols)
+                                                                : history_kernel<false>(cols),
+                                     dim3(plan.n_wg), dim3(kDpHistoryThreads), args, plan.lds,
+                                     (hipStream_t)stream));
+      MIST_HIP_CHECK(hipGetLastError());
+      return 0;
+    }
+  }
   if (force_fused) {
     if (costs->stage_min == nullptr || fused_lds > fused_lds_limit(mode))
       return fail(MIST_E_INVALID, "forced fused schedule: needs stage_min and %zu B of LDS", fused_lds);

@@ -13,7 +13,7 @@
 // families of a batch run back to back on the stream and come back with one synchronisation.
 //
 // Everything that decides a result is shared with the Python driver through the C ABI:
-// mist_dp_run, mist_dp_select_candidates, mist_dp_window_begin, mist_dp_filter_tmax,
+// mist_dp_run_sized, mist_dp_select_candidates, mist_dp_window_begin, mist_dp_filter_tmax,
 // mist_dp_backtrack (mist_dp_windows_first_batch walks the windows with the code of
 // mist_dp_window_begin, and a window it cannot decide sends the search down the host route).
 // How far a window is fetched or how many thresholds a batch speculates on
@@ -353,7 +353,7 @@ struct Search {
     int64_t n_scratch = 1;
     size_t slab = 0;
     for (int f = 0; f < n_families; ++f) {
-      const int64_t want = mist_dp_scratch_floats(&shapes[f], n);
+      const int64_t want = mist_dp_scratch_floats_sized(&shapes[f], n);
       if (want < 0) return MIST_E_INVALID;
       n_scratch = std::max(n_scratch, want);
       slab = std::max(slab, (size_t)(shapes[f].max_stages + 1) * (shapes[f].num_layers + 1) *
@@ -376,9 +376,9 @@ struct Search {
       int32_t *d_argmin = want_path ? ws->d_argmin.as<int32_t>() : nullptr;  // no fill: the
                                                      // walk reads what the DP wrote
       const MistDpShape shape = shape_of(f);
-      if (int rc = mist_dp_run(&shape, &costs[f], d_in, d_g, n, mode,
-                               reinterpret_cast<int32_t *>(d_out), d_out + n, d_out + 2 * n,
-                               d_argmin, ws->d_scratch.as<float>(), stream))
+      if (int rc = mist_dp_run_sized(&shape, &costs[f], d_in, d_g, n, mode,
+                                     reinterpret_cast<int32_t *>(d_out), d_out + n, d_out + 2 * n,
+                                     d_argmin, ws->d_scratch.as<float>(), n_scratch, stream))
         return rc;
       if (want_path) {
         int32_t *d_path = d_paths + path_offset(f, n);
@@ -509,7 +509,7 @@ struct Search {
     // the state planes of the batch are the larger need: sized before anything is queued
     int64_t n_scratch = 1;
     for (int f = 0; f < n_families; ++f) {
-      const int64_t want = mist_dp_scratch_floats(&shapes[f], n_inst);
+      const int64_t want = mist_dp_scratch_floats_sized(&shapes[f], n_inst);
       if (want < 0) return MIST_E_INVALID;
       n_scratch = std::max(n_scratch, want);
     }
@@ -535,10 +535,11 @@ struct Search {
       return rc;
     for (int f = 0; f < n_families; ++f) {
       float *d_out = d_first + at_out + (size_t)f * 3 * n_inst;
-      if (int rc = mist_dp_run(&shapes[f], &costs[f], ws->d_inst_t.as<float>(),
-                               ws->d_inst_row.as<int32_t>(), n_inst, MIST_DP_THRESHOLD,
-                               reinterpret_cast<int32_t *>(d_out), d_out + n_inst, d_out + 2 * n_inst,
-                               nullptr, ws->d_scratch.as<float>(), stream))
+      if (int rc = mist_dp_run_sized(&shapes[f], &costs[f], ws->d_inst_t.as<float>(),
+                                     ws->d_inst_row.as<int32_t>(), n_inst, MIST_DP_THRESHOLD,
+                                     reinterpret_cast<int32_t *>(d_out), d_out + n_inst,
+                                     d_out + 2 * n_inst, nullptr, ws->d_scratch.as<float>(), n_scratch,
+                                     stream))
         return rc;
     }
     MIST_HIP_CHECK(hipMemcpyAsync(h_first, d_first, sizeof(float) * (at_kept + kKeptHead),

@@ -1,0 +1,89 @@
+"""The DP schedule that keeps every plane and looks winners up on the answer's path
+(``dp_history_kernel``) against the one-launch-per-stage-count schedule, bit by bit."""
+import ctypes
+import os
+
+import numpy as np
+import pytest
+
+from tests.test_gpu_inter import _random_tables
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(meshes, L, D, P1, S, rule, tabs, g_index, tmax, mode, schedule):
+    import torch
+
+    from mist_amd import _lib
+
+    lib = _lib.load()
+    Q, n = len(meshes), len(tmax)
+    shape = np.zeros(1, dtype=_lib.DP_SHAPE_DTYPE)
+    shape["num_layers"], shape["num_devices"], shape["num_mesh"], shape["p_dim"] = L, D, Q, P1
+    shape["max_stages"], shape["ckpt_rule"] = S, rule
+    shape["mesh_n"][0, :Q] = [a for a, _ in meshes]
+    shape["mesh_m"][0, :Q] = [b for _, b in meshes]
+    sp = ctypes.c_void_p(shape.ctypes.data)
+    dev = [torch.from_numpy(np.stack([t[v] for t in tabs])).cuda() for v in range(4)]
+    dev += [torch.cummin(t, dim=-1).values.contiguous() for t in dev]
+    costs = _lib.DpCosts(*[t.data_ptr() for t in dev])
+    for v in range(4):
+        costs.g_stride[v] = dev[v][0].numel()
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    per_g = lib.mist_dp_stage_minima_floats(sp)
+    stage_min = torch.empty(per_g * len(tabs), dtype=torch.float32).cuda()
+    _lib.check(lib.mist_dp_stage_minima(sp, ctypes.byref(costs), len(tabs), stage_min.data_ptr(), stream),
+               "mist_dp_stage_minima")
+    costs.stage_min, costs.stage_min_g_stride = stage_min.data_ptr(), per_g
+    d_t = torch.tensor(np.asarray(tmax, dtype=np.float32)).cuda()
+    d_g = torch.tensor(np.asarray(g_index, dtype=np.int32)).cuda()
+    out = torch.full((3, n), -9.0, dtype=torch.float32).cuda()
+    floats = lib.mist_dp_scratch_floats_sized(sp, n)
+    scratch = torch.empty(floats, dtype=torch.float32).cuda()
+    old = os.environ.get("MIST_DP_FORCE_SCHEDULE")
+    os.environ["MIST_DP_FORCE_SCHEDULE"] = schedule
+    try:
+        rc = lib.mist_dp_run_sized(sp, ctypes.byref(costs), d_t.data_ptr(), d_g.data_ptr(), n, mode, out[0].data_ptr(),
+                                   out[1].data_ptr(), out[2].data_ptr(), None, scratch.data_ptr(), floats, stream)
+    finally:
+        if old is None:
+            del os.environ["MIST_DP_FORCE_SCHEDULE"]
+        else:
+            os.environ["MIST_DP_FORCE_SCHEDULE"] = old
+    _lib.check(rc, schedule)
+    torch.cuda.synchronize()
+    return out.cpu().numpy().view(np.int32)
+
+
+@pytest.mark.parametrize(
+    "L,D,meshes,S,n,quantum,rule",
+    [
+        (1, 1, [(1, 1)], 1, 3, None, 0),                                                     # one state
+        (1, 4, [(1, 2), (1, 4)], 1, 3, None, 0),
+        (5, 1, [(1, 1)], 2, 3, None, 0),                                                     # more stages than devices
+        (9, 8, [(1, 1), (1, 2), (1, 4), (2, 4)], 9, 600, 0.125, 0),                          # more instances than workgroups
+        (16, 64, [(1, 1), (1, 8), (2, 8), (4, 8), (8, 8)], 8, 40, 0.0625, 1),                # D a multiple of 64
+        (33, 65, [(1, 1), (1, 5), (5, 5), (5, 13)], 12, 40, 0.0625, 2),                      # and one above
+        (66, 33, [(1, k) for k in range(1, 17)], 9, 30, 0.03125, 0),                         # rows above 64, the most meshes
+        (48, 128, [(1, 1), (1, 2), (1, 8), (2, 8), (16, 8)], 16, 30, 0.03125, 0),
+        (80, 256, [(1, 4), (1, 8), (2, 8), (4, 8), (8, 8), (16, 8), (32, 8)], 16, 24, 0.03125, 0),
+    ],
+)
+@pytest.mark.parametrize("mode", [0, 1], ids=["threshold", "bottleneck"])
+def test_history_schedule_gives_what_the_step_schedule_gives(L, D, meshes, S, n, quantum, rule, mode):
+    rng = np.random.default_rng(L * 1000 + D + mode)
+    tabs = [_random_tables(rng, len(meshes), S, L, quantum=quantum) for _ in range(3)]
+    tmax = rng.uniform(0.05, 1.1, size=n).astype(np.float32)
+    g_index = rng.integers(0, 3, size=n).astype(np.int32)
+    args = (meshes, L, D, S, S, rule, tabs, g_index, tmax, mode)
+    want, got = _run(*args, "step"), _run(*args, "history")
+    feasible = want[0] >= 0
+    assert feasible.any() or L * D <= 5
+    assert np.array_equal(want[0], got[0])
+    assert np.array_equal(want[1], got[1])
+    assert np.array_equal(want[2][feasible], got[2][feasible])
+    # empty slots of a batch are infeasible and leave the others as they are
+    g_index[::2] = -1
+    again = _run(meshes, L, D, S, S, rule, tabs, g_index, tmax, mode, "history")
+    assert (again[0][::2] == -1).all()
+    assert np.array_equal(again[:, 1::2], got[:, 1::2])
