@@ -1235,6 +1235,36 @@ inline size_t dp_history_lds(int L, int D, int max_stages) {
   return (f + 2 * (size_t)L + (size_t)max_stages + 3) * sizeof(float);
 }
 
+// Cost of the stage k..i on mesh q, p pre-saved micro-batches, whose state has the value `best`
+// behind a successor of value `prev`: the first ckpt candidate that attains it (one wavefront).
+__device__ __forceinline__ float dp_stage_value(const MistDpShape &shape, const MistDpCosts &tabs,
+                                                const int64_t (&off)[4], float t_max, int p, int k,
+                                                int q, int i, float prev, float best) {
+  const int lane = threadIdx.x & 63;
+  const DpRowRef ref = dp_row_ref(shape, off, p, k, q, i);
+  const float *__restrict__ costs = dp_table(tabs, ref.v, false) + ref.at;
+  const int j_begin = shape.ckpt_rule == MIST_DP_CKPT_ALL ? i - k + 1 : 0;
+  const int j_end = dp_j_last(shape, k, i);
+  for (int j0 = j_begin; j0 <= j_end; j0 += 64) {
+    const float cost = j0 + lane <= j_end ? costs[j0 + lane] : INFINITY;
+    const unsigned long long hit = __ballot(cost <= t_max && cost + prev == best);
+    if (hit != 0)
+      return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cost), __ffsll(hit) - 1));
+  }
+  return 0.0f;
+}
+
+// Third output of an instance from the stage values of its path (stage count s at s - 1).
+// Threshold: the largest; bottleneck: the sum, added from the last stage on as the threshold DP
+// adds it.
+template <bool kBottleneck>
+__device__ __forceinline__ float dp_fold_path(const float *path_value, int n_stages) {
+  float value = 0.0f;
+  for (int s = 0; s < n_stages; ++s)
+    value = kBottleneck ? path_value[s] + value : fmaxf(value, path_value[s]);
+  return value;
+}
+
 template <bool kBottleneck, int kCols>
 __global__ __launch_bounds__(kDpHistoryThreads, 8) void dp_history_kernel(
     const MistDpShape shape, const MistDpCosts tabs, const float *__restrict__ tmax_list,
@@ -1400,39 +1430,142 @@ __global__ __launch_bounds__(kDpHistoryThreads, 8) void dp_history_kernel(
           }
         }
         if (arg_q < 0) break;  // (a reached state has a candidate that attains its value)
-        float value = arg_rmin;
-        if (!kBottleneck) {
-          const DpRowRef ref = dp_row_ref(shape, off, s - 1, k, arg_q, arg_i);
-          const float *__restrict__ costs = dp_table(tabs, ref.v, false) + ref.at;
-          const int j_begin = shape.ckpt_rule == MIST_DP_CKPT_ALL ? arg_i - k + 1 : 0;
-          const int j_end = dp_j_last(shape, k, arg_i);
-          value = 0.0f;
-          for (int j0 = j_begin; j0 <= j_end; j0 += 64) {
-            const float cost = j0 + lane <= j_end ? costs[j0 + lane] : INFINITY;
-            const unsigned long long hit = __ballot(cost <= t_max && cost + arg_prev == best);
-            if (hit != 0) {
-              value = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cost), __ffsll(hit) - 1));
-              break;
-            }
-          }
-        }
+        const float value = kBottleneck ? arg_rmin
+                                        : dp_stage_value(shape, tabs, off, t_max, s - 1, k, arg_q,
+                                                         arg_i, arg_prev, best);
         if (lane == 0) path_value[s - 1] = value;
         d -= shape.mesh_n[arg_q] * shape.mesh_m[arg_q];
         k = arg_i + 1;
         best = arg_prev;
       }
       if (lane == 0) {
-        // threshold: largest stage cost; bottleneck: the sum, added from the last stage on as the
-        // threshold DP adds it
-        float value = 0.0f;
-        for (int s = 0; s < answer_s; ++s)
-          value = kBottleneck ? path_value[s] + value : fmaxf(value, path_value[s]);
         best_s_out[t] = answer_s;
         best_sum_out[t] = answer_sum;
-        stage_max_out[t] = value;
+        stage_max_out[t] = dp_fold_path<kBottleneck>(path_value, answer_s);
       }
     }
     __syncthreads();  // the next instance writes the history and LDS
+  }
+}
+
+// ------------------------------------------------------------------------------------------
+// The recurrence of one mesh for all stages (free_devices): a state is a start layer, F(s) has
+// L + 1 values, and all of them stay in LDS.  With a launch per stage count a search of 6 stage
+// counts (1, 2, .. 32) in four batches made 250 launches of 3 to 8 us with as long a gap behind
+// each.  Here a workgroup runs an instance through all stage counts: per count it gathers the row
+// minima (consecutive end layers of a stage length are neighbours in the tables; up to
+// kDpFreeLoads reads of a lane in flight), then a wavefront takes a start layer with its lanes on
+// the end layers.  Bound: latency of that gather and two barriers, 2.5 us per stage count at 37
+// layers.  Six families of that plan: 250 launches, 3.3 ms from the first to the last -> 18, 0.75.
+// ------------------------------------------------------------------------------------------
+constexpr int kDpFreeThreads = 512;
+constexpr int kDpFreeLoads = 4;
+inline size_t dp_free_lds(int L, int S) {
+  return ((size_t)L * L + (size_t)(S + 1) * (L + 1) + S) * sizeof(float);
+}
+
+template <bool kBottleneck>
+__global__ __launch_bounds__(kDpFreeThreads) void dp_free_kernel(
+    const MistDpShape shape, const MistDpCosts tabs, const float *__restrict__ tmax_list,
+    const int32_t *__restrict__ g_list, int32_t *__restrict__ best_s_out,
+    float *__restrict__ best_sum_out, float *__restrict__ stage_max_out) {
+  extern __shared__ float dp_lds[];
+  const int L = shape.num_layers, S = shape.max_stages;
+  float *rows = dp_lds;                             // [L][L] (stage layers - 1, end layer)
+  float *history = rows + L * L;                    // [S + 1][L + 1]
+  float *path_value = history + (S + 1) * (L + 1);  // [S]
+  const int t = blockIdx.x;
+  const int64_t g = g_list[t];
+  if (g < 0) {  // an empty slot of the batch
+    if (threadIdx.x == 0) {
+      best_s_out[t] = -1;
+      best_sum_out[t] = INFINITY;
+      stage_max_out[t] = 0.0f;
+    }
+    return;
+  }
+  const int64_t off[4] = {g * tabs.g_stride[0], g * tabs.g_stride[1], g * tabs.g_stride[2],
+                          g * tabs.g_stride[3]};
+  const float t_max = kBottleneck ? kDpNoThreshold : tmax_list[t];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  constexpr int kWaves = kDpFreeThreads / 64;
+  for (int k = threadIdx.x; k <= L; k += kDpFreeThreads) history[k] = k == L ? 0.0f : INFINITY;
+  for (int s = 1; s <= S; ++s) {
+    const float *f_prev = history + (s - 1) * (L + 1);
+    float *f_cur = history + s * (L + 1);
+    // row minima of the stages (k, i) behind which s - 1 layers are left (s = 1: none)
+    for (int x0 = threadIdx.x; x0 < L * L; x0 += kDpFreeLoads * kDpFreeThreads) {
+      float value[kDpFreeLoads];
+#pragma unroll
+      for (int u = 0; u < kDpFreeLoads; ++u) {
+        const int x = x0 + u * kDpFreeThreads;
+        const int i = x % L, k = i - x / L;
+        const bool wanted = x < L * L && k >= 0 && i <= L - s && (s > 1 || i == L - 1);
+        value[u] = wanted ? dp_row_min(shape, tabs, off, s - 1, k, 0, i) : INFINITY;
+      }
+#pragma unroll
+      for (int u = 0; u < kDpFreeLoads; ++u) {
+        const int x = x0 + u * kDpFreeThreads;
+        if (x < L * L) rows[x] = value[u] <= t_max ? value[u] : INFINITY;
+      }
+    }
+    __syncthreads();
+    for (int k = wave; k <= L; k += kWaves) {
+      float best = INFINITY;
+      for (int i = k + lane; i <= L - s; i += 64) {
+        const float rmin = rows[(i - k) * L + i], prev = f_prev[i + 1];
+        // (an inadmissible row is +inf here, and so is its target)
+        best = fminf(best, kBottleneck ? fmaxf(rmin, prev) : rmin + prev);
+      }
+#pragma unroll
+      for (int step = 32; step >= 1; step >>= 1) best = fminf(best, __shfl_xor(best, step));
+      if (lane == 0) f_cur[k] = best;
+    }
+    __syncthreads();
+  }
+  if (wave != 0) return;
+  // first s wins ties (inter_tuning_uniform_device.py:335-340)
+  float answer_sum = INFINITY;
+  int answer_s = -1;
+  for (int s = 1; s <= S; ++s) {
+    const float sum = history[s * (L + 1)];
+    if (sum < answer_sum) {
+      answer_sum = sum;
+      answer_s = s;
+    }
+  }
+  int k = 0;
+  for (int s = answer_s; s >= 1; --s) {
+    const float *f_prev = history + (s - 1) * (L + 1);
+    const float best = history[s * (L + 1) + k];
+    int arg_i = -1;
+    float arg_rmin = 0.0f;
+    for (int i0 = k; i0 <= L - s && arg_i < 0; i0 += 64) {
+      const int i = i0 + lane;
+      float rmin = INFINITY, target = INFINITY;
+      if (i <= L - s && f_prev[i + 1] < INFINITY) {
+        rmin = dp_row_min(shape, tabs, off, s - 1, k, 0, i);
+        target = kBottleneck ? fmaxf(rmin, f_prev[i + 1]) : rmin + f_prev[i + 1];
+      }
+      const unsigned long long hit = __ballot(rmin <= t_max && target == best);
+      if (hit != 0) {
+        const int bit = __ffsll(hit) - 1;
+        arg_i = i0 + bit;
+        arg_rmin = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(rmin), bit));
+      }
+    }
+    if (arg_i < 0) break;  // (a reached state has a candidate that attains its value)
+    const float value = kBottleneck ? arg_rmin
+                                    : dp_stage_value(shape, tabs, off, t_max, s - 1, k, 0, arg_i,
+                                                     f_prev[arg_i + 1], best);
+    if (lane == 0) path_value[s - 1] = value;
+    k = arg_i + 1;
+  }
+  if (lane == 0) {
+    best_s_out[t] = answer_s;
+    best_sum_out[t] = answer_sum;
+    stage_max_out[t] = dp_fold_path<kBottleneck>(path_value, answer_s);
   }
 }
 
@@ -1927,6 +2060,19 @@ int mist_dp_run_sized(const MistDpShape *shape, const MistDpCosts *costs, const 
   // Without back-pointers and with room for the history that schedule runs: it was the fastest at
   // every shape and batch size measured (33 x 33 to 81 x 257 states, 28 to 2304 instances).
   if (!(force_step || force_fused || force_plane)) {
+    const size_t free_lds = dp_free_lds(shape->num_layers, shape->max_stages);
+    if (shape->free_devices != 0 && d_argmin == nullptr && free_lds <= 64 * 1024) {
+      if (mode == MIST_DP_BOTTLENECK)
+        hipLaunchKernelGGL(dp_free_kernel<true>, dim3(n_tmax), dim3(kDpFreeThreads), free_lds,
+                           (hipStream_t)stream, *shape, *costs, d_tmax, d_g_index, d_best_s,
+                           d_best_sum, d_stage_max);
+      else
+        hipLaunchKernelGGL(dp_free_kernel<false>, dim3(n_tmax), dim3(kDpFreeThreads), free_lds,
+                           (hipStream_t)stream, *shape, *costs, d_tmax, d_g_index, d_best_s,
+                           d_best_sum, d_stage_max);
+      MIST_HIP_CHECK(hipGetLastError());
+      return 0;
+    }
     const HistoryPlan plan = history_plan(*shape, n_tmax);
     const int cols = (shape->num_devices + 63) / 64;
     const bool possible = plan.n_wg > 0 && d_argmin == nullptr && costs->stage_min != nullptr &&

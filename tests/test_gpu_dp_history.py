@@ -1,5 +1,5 @@
-"""The DP schedule that keeps every plane and looks winners up on the answer's path
-(``dp_history_kernel``) against the one-launch-per-stage-count schedule, bit by bit."""
+"""The DP schedules that keep every plane and look winners up on the answer's path
+(``dp_history_kernel``, ``dp_free_kernel``) against the one-launch-per-stage-count schedule, bit by bit."""
 import ctypes
 import os
 
@@ -11,7 +11,7 @@ from tests.test_gpu_inter import _random_tables
 pytestmark = pytest.mark.gpu
 
 
-def _run(meshes, L, D, P1, S, rule, tabs, g_index, tmax, mode, schedule):
+def _run(meshes, L, D, P1, S, rule, tabs, g_index, tmax, mode, schedule, free=False):
     import torch
 
     from mist_amd import _lib
@@ -21,6 +21,7 @@ def _run(meshes, L, D, P1, S, rule, tabs, g_index, tmax, mode, schedule):
     shape = np.zeros(1, dtype=_lib.DP_SHAPE_DTYPE)
     shape["num_layers"], shape["num_devices"], shape["num_mesh"], shape["p_dim"] = L, D, Q, P1
     shape["max_stages"], shape["ckpt_rule"] = S, rule
+    shape["free_devices"] = free
     shape["mesh_n"][0, :Q] = [a for a, _ in meshes]
     shape["mesh_m"][0, :Q] = [b for _, b in meshes]
     sp = ctypes.c_void_p(shape.ctypes.data)
@@ -87,3 +88,23 @@ def test_history_schedule_gives_what_the_step_schedule_gives(L, D, meshes, S, n,
     again = _run(meshes, L, D, S, S, rule, tabs, g_index, tmax, mode, "history")
     assert (again[0][::2] == -1).all()
     assert np.array_equal(again[:, 1::2], got[:, 1::2])
+
+
+@pytest.mark.parametrize("L,S,n,quantum", [(1, 1, 3, None), (9, 9, 40, 0.125), (37, 16, 30, 0.0625), (64, 3, 9, 0.0625),
+                                           (65, 32, 70, 0.03125), (100, 8, 20, 0.03125)])
+@pytest.mark.parametrize("rule", [0, 1, 2])
+@pytest.mark.parametrize("mode", [0, 1], ids=["threshold", "bottleneck"])
+def test_one_mesh_schedule_gives_what_the_step_schedule_gives(L, S, n, quantum, rule, mode):
+    rng = np.random.default_rng(L * 1000 + rule + mode)
+    tabs = [_random_tables(rng, 1, S, L, quantum=quantum) for _ in range(3)]
+    tmax = rng.uniform(0.05, 1.1, size=n).astype(np.float32)
+    g_index = rng.integers(0, 3, size=n).astype(np.int32)
+    g_index[-1] = -1
+    args = ([(2, 4)], L, 0, S, S, rule, tabs, g_index, tmax, mode)
+    want, got = _run(*args, "step", free=True)[:, :-1], _run(*args, "", free=True)
+    feasible = want[0] >= 0
+    assert got[0, -1] == -1
+    got = got[:, :-1]
+    assert np.array_equal(want[0], got[0])
+    assert np.array_equal(want[1], got[1])
+    assert np.array_equal(want[2][feasible], got[2][feasible])
