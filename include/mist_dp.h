@@ -186,12 +186,14 @@ int mist_dp_run(const MistDpShape *shape, const MistDpCosts *costs, const float 
 /* mist_dp_run() with a scratch whose size is given: with the mist_dp_scratch_floats_sized() floats
  * of a batch (at least mist_dp_scratch_floats() and, beyond that, at most 1 GiB), one without
  * back-pointers may keep the planes of all stage counts and look the winners up on the answer's
- * path alone.  Same arguments and results otherwise. */
+ * path alone.  d_path (may be NULL): the partition of every instance, as mist_dp_backtrack() writes
+ * it; d_argmin is then only its workspace (same size, contents undefined, no fill needed).  Same
+ * arguments and results otherwise. */
 int64_t mist_dp_scratch_floats_sized(const MistDpShape *shape, int n_tmax);
 int mist_dp_run_sized(const MistDpShape *shape, const MistDpCosts *costs, const float *d_tmax,
                       const int32_t *d_g_index, int n_tmax, int mode, int32_t *d_best_s,
-                      float *d_best_sum, float *d_stage_max, int32_t *d_argmin, float *d_scratch,
-                      int64_t scratch_floats, void *stream);
+                      float *d_best_sum, float *d_stage_max, int32_t *d_argmin, int32_t *d_path,
+                      float *d_scratch, int64_t scratch_floats, void *stream);
 
 /* mist_dp_run() for callers that cannot allocate device memory (code under HIP graph capture,
  * serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  Same

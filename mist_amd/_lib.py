@@ -256,7 +256,7 @@ _DP_SIGNATURES = {
     "mist_dp_run_sized": (
         ctypes.c_int,
         [_VP, ctypes.POINTER(DpCosts), _VP, _VP, ctypes.c_int, ctypes.c_int, _VP, _VP, _VP, _VP, _VP,
-         ctypes.c_int64, _VP],
+         _VP, ctypes.c_int64, _VP],
     ),
     "mist_dp_static_scratch_floats": (ctypes.c_int64, []),
     "mist_dp_run_static": (

@@ -1239,7 +1239,7 @@ inline size_t dp_history_lds(int L, int D, int max_stages) {
 // behind a successor of value `prev`: the first ckpt candidate that attains it (one wavefront).
 __device__ __forceinline__ float dp_stage_value(const MistDpShape &shape, const MistDpCosts &tabs,
                                                 const int64_t (&off)[4], float t_max, int p, int k,
-                                                int q, int i, float prev, float best) {
+                                                int q, int i, float prev, float best, int *arg_j) {
   const int lane = threadIdx.x & 63;
   const DpRowRef ref = dp_row_ref(shape, off, p, k, q, i);
   const float *__restrict__ costs = dp_table(tabs, ref.v, false) + ref.at;
@@ -1248,8 +1248,11 @@ __device__ __forceinline__ float dp_stage_value(const MistDpShape &shape, const 
   for (int j0 = j_begin; j0 <= j_end; j0 += 64) {
     const float cost = j0 + lane <= j_end ? costs[j0 + lane] : INFINITY;
     const unsigned long long hit = __ballot(cost <= t_max && cost + prev == best);
-    if (hit != 0)
-      return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cost), __ffsll(hit) - 1));
+    if (hit != 0) {
+      const int bit = __ffsll(hit) - 1;
+      *arg_j = j0 + bit;
+      return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cost), bit));
+    }
   }
   return 0.0f;
 }
@@ -1265,12 +1268,20 @@ __device__ __forceinline__ float dp_fold_path(const float *path_value, int n_sta
   return value;
 }
 
+// A stage of an instance's partition, as backtrack_kernel writes it.
+__device__ __forceinline__ void dp_write_stage(int32_t *at, int end, int n, int m, int ckpt) {
+  at[0] = end;
+  at[1] = n;
+  at[2] = m;
+  at[3] = ckpt;
+}
+
 template <bool kBottleneck, int kCols>
 __global__ __launch_bounds__(kDpHistoryThreads, 8) void dp_history_kernel(
     const MistDpShape shape, const MistDpCosts tabs, const float *__restrict__ tmax_list,
     const int32_t *__restrict__ g_list, int n_instances, float *__restrict__ histories,
     int32_t *__restrict__ best_s_out, float *__restrict__ best_sum_out,
-    float *__restrict__ stage_max_out) {
+    float *__restrict__ stage_max_out, int32_t *__restrict__ path_out) {
   extern __shared__ float dp_lds[];
   const int L = shape.num_layers, D = shape.num_devices, Q = shape.num_mesh;
   const int S = shape.max_stages, plane = L * D, tri = dp_triangle(L);
@@ -1286,6 +1297,8 @@ __global__ __launch_bounds__(kDpHistoryThreads, 8) void dp_history_kernel(
   float *history = histories + (int64_t)blockIdx.x * S * plane;
   for (int t = blockIdx.x; t < n_instances; t += gridDim.x) {
     const int64_t g = g_list[t];
+    for (int x = threadIdx.x; path_out != nullptr && x < 4 * S; x += kDpHistoryThreads)
+      path_out[(int64_t)t * S * 4 + x] = -1;
     if (g < 0) {  // an empty slot of the batch
       if (threadIdx.x == 0) {
         best_s_out[t] = -1;
@@ -1430,10 +1443,16 @@ __global__ __launch_bounds__(kDpHistoryThreads, 8) void dp_history_kernel(
           }
         }
         if (arg_q < 0) break;  // (a reached state has a candidate that attains its value)
+        int arg_j = -1;
         const float value = kBottleneck ? arg_rmin
                                         : dp_stage_value(shape, tabs, off, t_max, s - 1, k, arg_q,
-                                                         arg_i, arg_prev, best);
-        if (lane == 0) path_value[s - 1] = value;
+                                                         arg_i, arg_prev, best, &arg_j);
+        if (lane == 0) {
+          path_value[s - 1] = value;
+          if (path_out != nullptr)
+            dp_write_stage(path_out + ((int64_t)t * S + answer_s - s) * 4, arg_i,
+                           shape.mesh_n[arg_q], shape.mesh_m[arg_q], arg_j);
+        }
         d -= shape.mesh_n[arg_q] * shape.mesh_m[arg_q];
         k = arg_i + 1;
         best = arg_prev;
@@ -1468,7 +1487,8 @@ template <bool kBottleneck>
 __global__ __launch_bounds__(kDpFreeThreads) void dp_free_kernel(
     const MistDpShape shape, const MistDpCosts tabs, const float *__restrict__ tmax_list,
     const int32_t *__restrict__ g_list, int32_t *__restrict__ best_s_out,
-    float *__restrict__ best_sum_out, float *__restrict__ stage_max_out) {
+    float *__restrict__ best_sum_out, float *__restrict__ stage_max_out,
+    int32_t *__restrict__ path_out) {
   extern __shared__ float dp_lds[];
   const int L = shape.num_layers, S = shape.max_stages;
   float *rows = dp_lds;                             // [L][L] (stage layers - 1, end layer)
@@ -1476,6 +1496,8 @@ __global__ __launch_bounds__(kDpFreeThreads) void dp_free_kernel(
   float *path_value = history + (S + 1) * (L + 1);  // [S]
   const int t = blockIdx.x;
   const int64_t g = g_list[t];
+  for (int x = threadIdx.x; path_out != nullptr && x < 4 * S; x += kDpFreeThreads)
+    path_out[(int64_t)t * S * 4 + x] = -1;
   if (g < 0) {  // an empty slot of the batch
     if (threadIdx.x == 0) {
       best_s_out[t] = -1;
@@ -1556,10 +1578,16 @@ __global__ __launch_bounds__(kDpFreeThreads) void dp_free_kernel(
       }
     }
     if (arg_i < 0) break;  // (a reached state has a candidate that attains its value)
+    int arg_j = -1;
     const float value = kBottleneck ? arg_rmin
                                     : dp_stage_value(shape, tabs, off, t_max, s - 1, k, 0, arg_i,
-                                                     f_prev[arg_i + 1], best);
-    if (lane == 0) path_value[s - 1] = value;
+                                                     f_prev[arg_i + 1], best, &arg_j);
+    if (lane == 0) {
+      path_value[s - 1] = value;
+      if (path_out != nullptr)
+        dp_write_stage(path_out + ((int64_t)t * S + answer_s - s) * 4, arg_i, shape.mesh_n[0],
+                       shape.mesh_m[0], arg_j);
+    }
     k = arg_i + 1;
   }
   if (lane == 0) {
@@ -1591,10 +1619,7 @@ __global__ __launch_bounds__(64) void backtrack_kernel(const MistDpShape shape,
     // a path that does not cover the layers
     if (end < k || end >= L || mesh_n < 1 || mesh_m < 1) break;
     if (shape.free_devices == 0 && mesh_n * mesh_m > d) break;
-    out[stage * 4 + 0] = end;
-    out[stage * 4 + 1] = mesh_n;
-    out[stage * 4 + 2] = mesh_m;
-    out[stage * 4 + 3] = a[3];
+    dp_write_stage(out + stage * 4, end, mesh_n, mesh_m, a[3]);
     ++stage;
     --s;
     k = end + 1;
@@ -2019,18 +2044,20 @@ int mist_dp_run(const MistDpShape *shape, const MistDpCosts *costs, const float 
                 float *d_best_sum, float *d_stage_max, int32_t *d_argmin, float *d_scratch,
                 void *stream) {
   return mist_dp_run_sized(shape, costs, d_tmax, d_g_index, n_tmax, mode, d_best_s, d_best_sum,
-                           d_stage_max, d_argmin, d_scratch, mist_dp_scratch_floats(shape, n_tmax),
-                           stream);
+                           d_stage_max, d_argmin, nullptr, d_scratch,
+                           mist_dp_scratch_floats(shape, n_tmax), stream);
 }
 
 int mist_dp_run_sized(const MistDpShape *shape, const MistDpCosts *costs, const float *d_tmax,
-                const int32_t *d_g_index, int n_tmax, int mode, int32_t *d_best_s,
-                float *d_best_sum, float *d_stage_max, int32_t *d_argmin, float *d_scratch,
-                int64_t scratch_floats, void *stream) {
+                      const int32_t *d_g_index, int n_tmax, int mode, int32_t *d_best_s,
+                      float *d_best_sum, float *d_stage_max, int32_t *d_argmin, int32_t *d_path,
+                      float *d_scratch, int64_t scratch_floats, void *stream) {
   if (int rc = check_run_arguments(shape, costs, d_tmax, d_g_index, n_tmax, mode, d_best_s,
                                    d_best_sum, d_stage_max))
     return rc;
   if (!d_scratch) return fail(MIST_E_INVALID, "null scratch pointer");
+  if (d_path && !d_argmin) return fail(MIST_E_INVALID, "d_path needs d_argmin");
+  const bool whole_argmin = d_argmin != nullptr && d_path == nullptr;
   const int plane = (shape->num_layers + 1) * (shape->num_devices + 1);
   const bool wide = dp_wide_teams(n_tmax, plane);
   // Larger ones: one workgroup per instance with its planes in LDS when they fit and the caller
@@ -2061,21 +2088,21 @@ int mist_dp_run_sized(const MistDpShape *shape, const MistDpCosts *costs, const 
   // every shape and batch size measured (33 x 33 to 81 x 257 states, 28 to 2304 instances).
   if (!(force_step || force_fused || force_plane)) {
     const size_t free_lds = dp_free_lds(shape->num_layers, shape->max_stages);
-    if (shape->free_devices != 0 && d_argmin == nullptr && free_lds <= 64 * 1024) {
+    if (shape->free_devices != 0 && !whole_argmin && free_lds <= 64 * 1024) {
       if (mode == MIST_DP_BOTTLENECK)
         hipLaunchKernelGGL(dp_free_kernel<true>, dim3(n_tmax), dim3(kDpFreeThreads), free_lds,
                            (hipStream_t)stream, *shape, *costs, d_tmax, d_g_index, d_best_s,
-                           d_best_sum, d_stage_max);
+                           d_best_sum, d_stage_max, d_path);
       else
         hipLaunchKernelGGL(dp_free_kernel<false>, dim3(n_tmax), dim3(kDpFreeThreads), free_lds,
                            (hipStream_t)stream, *shape, *costs, d_tmax, d_g_index, d_best_s,
-                           d_best_sum, d_stage_max);
+                           d_best_sum, d_stage_max, d_path);
       MIST_HIP_CHECK(hipGetLastError());
       return 0;
     }
     const HistoryPlan plan = history_plan(*shape, n_tmax);
     const int cols = (shape->num_devices + 63) / 64;
-    const bool possible = plan.n_wg > 0 && d_argmin == nullptr && costs->stage_min != nullptr &&
+    const bool possible = plan.n_wg > 0 && !whole_argmin && costs->stage_min != nullptr &&
                           plan.floats <= scratch_floats && plan.lds <= history_lds_limit(mode, cols);
     if (force_history && !possible)
       return fail(MIST_E_INVALID, "forced history schedule: needs stage_min, consumed devices, D <= 256, no "
@@ -2085,7 +2112,7 @@ int mist_dp_run_sized(const MistDpShape *shape, const MistDpCosts *costs, const 
       const MistDpCosts costs_arg = *costs;
       int n_arg = n_tmax;
       void *args[] = {(void *)&shape_arg, (void *)&costs_arg, &d_tmax, &d_g_index, &n_arg,
-                      &d_scratch, &d_best_s, &d_best_sum, &d_stage_max};
+                      &d_scratch, &d_best_s, &d_best_sum, &d_stage_max, &d_path};
       MIST_HIP_CHECK(hipLaunchKernel(mode == MIST_DP_BOTTLENECK ? history_kernel<true>(cols)
                                                                 : history_kernel<false>(cols),
                                      dim3(plan.n_wg), dim3(kDpHistoryThreads), args, plan.lds,
@@ -2093,6 +2120,12 @@ int mist_dp_run_sized(const MistDpShape *shape, const MistDpCosts *costs, const 
       MIST_HIP_CHECK(hipGetLastError());
       return 0;
     }
+  }
+  if (d_path) {
+    if (int rc = mist_dp_run_sized(shape, costs, d_tmax, d_g_index, n_tmax, mode, d_best_s, d_best_sum,
+                                   d_stage_max, d_argmin, nullptr, d_scratch, scratch_floats, stream))
+      return rc;
+    return mist_dp_backtrack(shape, d_argmin, d_best_s, n_tmax, d_path, stream);
   }
   if (force_fused) {
     if (costs->stage_min == nullptr || fused_lds > fused_lds_limit(mode))

@@ -375,16 +375,13 @@ struct Search {
       float *d_out = ws->d_out.as<float>() + (size_t)f * 3 * n;
       int32_t *d_argmin = want_path ? ws->d_argmin.as<int32_t>() : nullptr;  // no fill: the
                                                      // walk reads what the DP wrote
+      int32_t *d_path = want_path ? d_paths + path_offset(f, n) : nullptr;
       const MistDpShape shape = shape_of(f);
       if (int rc = mist_dp_run_sized(&shape, &costs[f], d_in, d_g, n, mode,
                                      reinterpret_cast<int32_t *>(d_out), d_out + n, d_out + 2 * n,
-                                     d_argmin, ws->d_scratch.as<float>(), n_scratch, stream))
+                                     d_argmin, d_path, ws->d_scratch.as<float>(), n_scratch, stream))
         return rc;
       if (want_path) {
-        int32_t *d_path = d_paths + path_offset(f, n);
-        if (int rc = mist_dp_backtrack(&shape, d_argmin, reinterpret_cast<int32_t *>(d_out), n,
-                                       d_path, stream))
-          return rc;
         if (strategy) {
           const int cells = n * shape.max_stages;
           hipLaunchKernelGGL(strategy_rows_kernel, dim3((cells + 63) / 64), dim3(64), 0, stream,
@@ -538,7 +535,7 @@ struct Search {
       if (int rc = mist_dp_run_sized(&shapes[f], &costs[f], ws->d_inst_t.as<float>(),
                                      ws->d_inst_row.as<int32_t>(), n_inst, MIST_DP_THRESHOLD,
                                      reinterpret_cast<int32_t *>(d_out), d_out + n_inst,
-                                     d_out + 2 * n_inst, nullptr, ws->d_scratch.as<float>(), n_scratch,
+                                     d_out + 2 * n_inst, nullptr, nullptr, ws->d_scratch.as<float>(), n_scratch,
                                      stream))
         return rc;
     }

@@ -11,7 +11,7 @@ from tests.test_gpu_inter import _random_tables
 pytestmark = pytest.mark.gpu
 
 
-def _run(meshes, L, D, P1, S, rule, tabs, g_index, tmax, mode, schedule, free=False):
+def _run(meshes, L, D, P1, S, rule, tabs, g_index, tmax, mode, schedule, free=False, want_path=False):
     import torch
 
     from mist_amd import _lib
@@ -39,13 +39,16 @@ def _run(meshes, L, D, P1, S, rule, tabs, g_index, tmax, mode, schedule, free=Fa
     d_t = torch.tensor(np.asarray(tmax, dtype=np.float32)).cuda()
     d_g = torch.tensor(np.asarray(g_index, dtype=np.int32)).cuda()
     out = torch.full((3, n), -9.0, dtype=torch.float32).cuda()
+    path = torch.full((n, S, 4), -9, dtype=torch.int32).cuda()
+    argmin = torch.empty((n, S + 1, L + 1, D + 1, 4), dtype=torch.int32).cuda()
     floats = lib.mist_dp_scratch_floats_sized(sp, n)
     scratch = torch.empty(floats, dtype=torch.float32).cuda()
     old = os.environ.get("MIST_DP_FORCE_SCHEDULE")
     os.environ["MIST_DP_FORCE_SCHEDULE"] = schedule
     try:
         rc = lib.mist_dp_run_sized(sp, ctypes.byref(costs), d_t.data_ptr(), d_g.data_ptr(), n, mode, out[0].data_ptr(),
-                                   out[1].data_ptr(), out[2].data_ptr(), None, scratch.data_ptr(), floats, stream)
+                                   out[1].data_ptr(), out[2].data_ptr(), argmin.data_ptr() if want_path else None,
+                                   path.data_ptr() if want_path else None, scratch.data_ptr(), floats, stream)
     finally:
         if old is None:
             del os.environ["MIST_DP_FORCE_SCHEDULE"]
@@ -53,7 +56,8 @@ def _run(meshes, L, D, P1, S, rule, tabs, g_index, tmax, mode, schedule, free=Fa
             os.environ["MIST_DP_FORCE_SCHEDULE"] = old
     _lib.check(rc, schedule)
     torch.cuda.synchronize()
-    return out.cpu().numpy().view(np.int32)
+    out = out.cpu().numpy().view(np.int32)
+    return (out, path.cpu().numpy()) if want_path else out
 
 
 @pytest.mark.parametrize(
@@ -83,6 +87,10 @@ def test_history_schedule_gives_what_the_step_schedule_gives(L, D, meshes, S, n,
     assert np.array_equal(want[0], got[0])
     assert np.array_equal(want[1], got[1])
     assert np.array_equal(want[2][feasible], got[2][feasible])
+    # the partitions: the other schedule's back-pointers, walked
+    with_path, path = _run(*args, "history", want_path=True)
+    assert np.array_equal(with_path, got)
+    assert np.array_equal(path, _run(*args, "step", want_path=True)[1])
     # empty slots of a batch are infeasible and leave the others as they are
     g_index[::2] = -1
     again = _run(meshes, L, D, S, S, rule, tabs, g_index, tmax, mode, "history")
@@ -101,7 +109,12 @@ def test_one_mesh_schedule_gives_what_the_step_schedule_gives(L, S, n, quantum, 
     g_index = rng.integers(0, 3, size=n).astype(np.int32)
     g_index[-1] = -1
     args = ([(2, 4)], L, 0, S, S, rule, tabs, g_index, tmax, mode)
-    want, got = _run(*args, "step", free=True)[:, :-1], _run(*args, "", free=True)
+    want, want_path = _run(*args, "step", free=True, want_path=True)
+    want = want[:, :-1]
+    got, path = _run(*args, "", free=True, want_path=True)
+    assert np.array_equal(got, _run(*args, "", free=True))
+    assert np.array_equal(path[:-1], want_path[:-1])
+    assert (path[-1] == -1).all()
     feasible = want[0] >= 0
     assert got[0, -1] == -1
     got = got[:, :-1]
