@@ -1408,28 +1408,20 @@ __device__ __forceinline__ LaneMemory pair_memory(const Row &t, const PairConsts
   return mem;
 }
 
-// Upper bound of the number of feasible p in [0, n]: the scaled peaks are linear in p up to
-// rounding, so the first infeasible p is estimated from the first two and confirmed with the
-// exact test: any p at which the row is infeasible bounds the count (monotonicity); an
-// unconfirmed estimate falls back to n.
-template <class Scaled>
-__device__ __forceinline__ int count_bound(const Scaled &scaled, int n, double cap) {
-  const double m0 = scaled(0);
+// Upper bound of the number of feasible p in [0, n): both peaks are a value at p = 0 plus p times the
+// same step, so what p admits is a quotient.  Rounding moves a scaled peak by a few 1e-16 of itself,
+// at most 1e-15 of the capacity while it fits, hence the quotient by less than 1e-5 where a step
+// counts for more than 1e-9 of the capacity; the quotient is taken 1e-4 and 0.01 long.  (`m0`, the
+// scaled peak at p = 0, is the reference's value.)
+__device__ __forceinline__ int count_upper(double m0, double step, int n, double cap) {
   if (n <= 0 || !(m0 <= cap)) return 0;
-  if (n == 1) return 1;
-  const float slope = (float)(scaled(1) - m0);
-  if (!(slope > 0.0f)) return n;
-  const float est = fminf((float)(cap - m0) * __frcp_rn(slope), (float)n);
-  const int guess = (int)est + 1;  // 0 .. floor(est) are expected to be feasible
-  if (guess >= n) return n;
-  if (!(scaled(guess) <= cap)) return guess;
-  if (guess + 1 < n && !(scaled(guess + 1) <= cap)) return guess + 1;
-  return n;
+  if (!(step > 1e-9 * cap)) return n;
+  const float most = (float)(cap - m0) * __frcp_rn((float)step) * 1.0001f + 0.01f;
+  return most < (float)(n - 1) ? (int)most + 1 : n;
 }
 // The number itself: from the bound down to the last p the exact test admits.
 template <class Scaled>
-__device__ __forceinline__ int count_exact(const Scaled &scaled, int n, double cap) {
-  int count = count_bound(scaled, n, cap);
+__device__ __forceinline__ int count_exact(const Scaled &scaled, int count, double cap) {
   while (count > 0 && !(scaled(count - 1) <= cap)) --count;
   return count;
 }
@@ -1462,6 +1454,26 @@ __device__ __forceinline__ GroupModel group_model(const MistProblem &prob, const
   m.post_output = g->post_output;
   m.pow2 = (g->grad_accum & (g->grad_accum - 1)) == 0;
   return m;
+}
+
+// count_upper of the base and with_pre variants.
+struct UpperCounts {
+  int b, p;
+};
+__device__ __forceinline__ UpperCounts upper_counts(const LaneMemory &mem, const GroupModel &m, int n) {
+  double peak_f, peak_b;
+  mem.peaks(0, peak_f, peak_b);
+  const double peak = fmax(peak_f, peak_b), step = mem.mod_saved + 2.0 * mem.out;
+  return UpperCounts{count_upper(peak * mem.mf_base, step * mem.mf_base, n, m.cap),
+                     count_upper((peak + m.pre_sas) * mem.mf_pp, (step + m.pre_saved) * mem.mf_pp, n, m.cap)};
+}
+struct RowCounts {
+  int b, p;
+};
+__device__ __forceinline__ RowCounts exact_counts(const LaneMemory &mem, const GroupModel &m, int upper_b, int upper_p) {
+  return RowCounts{
+      count_exact([&](int p) { return mem.scaled_base(p); }, upper_b, m.cap),
+      count_exact([&](int p) { return mem.scaled_pre(p, m.pre_saved, m.pre_sas); }, upper_p, m.cap)};
 }
 
 // Stage costs the caller's search can use at all (MistProblem.stage_cost_incumbent): rows above
@@ -1628,13 +1640,21 @@ __global__ __launch_bounds__(kSeedThreads) void seed_kernel(
             live && (cutoff == INFINITY || ratio * (double)x + m.div_G((double)d) <= cutoff * (1.0 + kBaseSlack));
         if (!__any(wanted)) continue;
         const LaneMemory mem = pair_memory(t, k);
-        const int cnt_b = count_exact([&](int p) { return mem.scaled_base(p); }, wanted ? np : 0, m.cap);
-        const int cnt_p =
-            count_exact([&](int p) { return mem.scaled_pre(p, m.pre_saved, m.pre_sas); }, wanted ? np : 0, m.cap);
-        bool ok_post = false, ok_pp = false;
-        if (do_post) post_fits(t, k, mem, m, mem.out, k.no_ck ? t[MIST_T_RD] : 0.0, ok_post, ok_pp);
         unsigned long long *mine = lds_best + i * n_slots;
         const Objectives o = objectives(t, x, d, k.no_ck, ratio, m, do_post);
+        // the minima do not decrease with p: at the bound of its count a row meets the largest one
+        // it could beat
+        const UpperCounts upper = upper_counts(mem, m, wanted ? np : 0);
+        auto may = [&](int count, double cost, const unsigned long long *slots) {
+          return count > 0 && (unsigned long long)__double_as_longlong(cost) < slots[max(count - 1, 0)];
+        };
+        const bool may_b = may(upper.b, o.base, mine), may_p = may(upper.p, o.pre, mine + P);
+        const bool may_post = do_post && may(wanted, o.post, mine + 2 * P);
+        const bool may_pp = do_pp && may(wanted, o.pp, mine + 2 * P + 1);
+        if (!__any(may_b || may_p || may_post || may_pp)) continue;
+        const RowCounts cnt = exact_counts(mem, m, may_b ? upper.b : 0, may_p ? upper.p : 0);
+        bool ok_post = false, ok_pp = false;
+        if (do_post) post_fits(t, k, mem, m, mem.out, k.no_ck ? t[MIST_T_RD] : 0.0, ok_post, ok_pp);
         auto offer = [&](int count, double cost, unsigned long long *slots) {
           const unsigned long long bits = (unsigned long long)__double_as_longlong(cost);
           bool pending = count > 0 && bits < slots[max(count - 1, 0)];
@@ -1647,8 +1667,8 @@ __global__ __launch_bounds__(kSeedThreads) void seed_kernel(
             pending = pending && lane != r && (count > its_count || cost < its_cost);
           }
         };
-        offer(cnt_b, o.base, mine);
-        offer(cnt_p, o.pre, mine + P);
+        offer(cnt.b, o.base, mine);
+        offer(cnt.p, o.pre, mine + P);
         if (do_post) offer(wanted && ok_post ? 1 : 0, o.post, mine + 2 * P);
         if (do_pp) offer(wanted && ok_pp ? 1 : 0, o.pp, mine + 2 * P + 1);
       }
@@ -1734,18 +1754,17 @@ __global__ __launch_bounds__(64) void seed_samples_kernel(
       float x, d;
       pair_latency(t, k, x, d);
       const LaneMemory mem = pair_memory(t, k);
-      const int cnt_b = count_exact([&](int p) { return mem.scaled_base(p); }, lane < n_rows ? np : 0, m.cap);
-      const int cnt_p = count_exact([&](int p) { return mem.scaled_pre(p, m.pre_saved, m.pre_sas); },
-                                    lane < n_rows ? np : 0, m.cap);
+      const UpperCounts upper = upper_counts(mem, m, lane < n_rows ? np : 0);
+      const RowCounts cnt = exact_counts(mem, m, upper.b, upper.p);
       bool ok_post = false, ok_pp = false;
       if (do_post) post_fits(t, k, mem, m, mem.out, k.no_ck ? t[MIST_T_RD] : 0.0, ok_post, ok_pp);
       ok_post = ok_post && lane < n_rows;
       ok_pp = ok_pp && do_pp && lane < n_rows;
       // (rows that fit nowhere are left out)
-      const uint64_t useful = __ballot(cnt_b > 0 || cnt_p > 0 || ok_post || ok_pp);
+      const uint64_t useful = __ballot(cnt.b > 0 || cnt.p > 0 || ok_post || ok_pp);
       __syncthreads();
       if (useful >> lane & 1ull)
-        put_sample_row(rows, __popcll(useful & ((1ull << lane) - 1ull)), t, x, d, k.no_ck, m, cnt_b, cnt_p, ok_post,
+        put_sample_row(rows, __popcll(useful & ((1ull << lane) - 1ull)), t, x, d, k.no_ck, m, cnt.b, cnt.p, ok_post,
                        ok_pp, do_post);
       __syncthreads();
       const int n_useful = __popcll(useful);
@@ -1846,8 +1865,9 @@ __device__ __forceinline__ StageReach stage_reach(const double *__restrict__ f, 
   StageReach r;
   pair_latency(f, k, r.x, r.d);
   const LaneMemory mem = pair_memory(f, k);
-  r.count_b = count_bound([&](int p) { return mem.scaled_base(p); }, np, m.cap);
-  r.count_p = count_bound([&](int p) { return mem.scaled_pre(p, m.pre_saved, m.pre_sas); }, np, m.cap);
+  const UpperCounts upper = upper_counts(mem, m, np);
+  r.count_b = upper.b;
+  r.count_p = upper.p;
   bool post, pp;
   post_fits(f, k, mem, m, f[kStageMaxOut], 0.0, post, pp);
   r.post = do_post && post;
@@ -2153,11 +2173,20 @@ __device__ __forceinline__ uint64_t reduce_item(const MistProblem &prob, const M
     const LaneMemory mem = pair_memory(t, k);
     const int np = c == l - 1 ? min(P, 1) : P;
     const bool do_post = c != l - 1, do_pp = do_post && l == L;
-    const int row_b = count_exact([&](int p) { return mem.scaled_base(p); }, in ? np : 0, m.cap);
-    const int row_p = count_exact([&](int p) { return mem.scaled_pre(p, m.pre_saved, m.pre_sas); }, in ? np : 0, m.cap);
+    const Objectives o = objectives(t, x, d, k.no_ck, ratio, m, do_post);
+    // Rows that reach the minimum at the bound of their count: one pair in eight has any, and only
+    // these pay for the exact tests.  (A lowered slot may lie below the slots under it; a row above
+    // it is above the winner of its own slot too, which finalize takes from the slots at and above.)
+    const UpperCounts upper = upper_counts(mem, m, in ? np : 0);
+    auto may = [&](int count, double cost, int slot) {
+      return in && count > 0 && cost <= cutoff && cost < INFINITY && cost <= lds_row[slot + max(count - 1, 0)];
+    };
+    const bool may_b = may(upper.b, o.base, 0), may_p = may(upper.p, o.pre, P);
+    const bool may_post = do_post && may(1, o.post, 2 * P), may_pp = do_pp && may(1, o.pp, 2 * P + 1);
+    if (!__any(may_b || may_p || may_post || may_pp)) continue;
+    const RowCounts cnt = exact_counts(mem, m, may_b ? upper.b : 0, may_p ? upper.p : 0);
     bool ok_post = false, ok_pp = false;
     if (do_post) post_fits(t, k, mem, m, mem.out, k.no_ck ? t[MIST_T_RD] : 0.0, ok_post, ok_pp);
-    const Objectives o = objectives(t, x, d, k.no_ck, ratio, m, do_post);
     bool hit = false, lowered = false;
     const int64_t cell = tile_cell + pl * n_slots;
     // rows with `count` > 0 against the minimum of slot `slot` + count - 1
@@ -2171,8 +2200,8 @@ __device__ __forceinline__ uint64_t reduce_item(const MistProblem &prob, const M
       if (cost == now) atomicMin(tabs.row + cell + own, my_row_number);
       hit = hit || cost <= now;
     };
-    offer(row_b, o.base, 0);
-    offer(row_p, o.pre, P);
+    offer(cnt.b, o.base, 0);
+    offer(cnt.p, o.pre, P);
     if (do_post) offer(ok_post ? 1 : 0, o.post, 2 * P);
     if (do_pp) offer(ok_pp ? 1 : 0, o.pp, 2 * P + 1);
     if (kResolve) continue;
@@ -2241,18 +2270,18 @@ __device__ __forceinline__ uint64_t reduce_item_samples(const MistProblem &prob,
     const LaneMemory mem = pair_memory(t, k);
     const int np = c == l - 1 ? min(P, 1) : P;
     const bool do_post = c != l - 1, do_pp = do_post && l == L;
-    const int row_b = count_exact([&](int p) { return mem.scaled_base(p); }, pass ? np : 0, m.cap);
-    const int row_p = count_exact([&](int p) { return mem.scaled_pre(p, m.pre_saved, m.pre_sas); }, pass ? np : 0, m.cap);
+    const UpperCounts upper = upper_counts(mem, m, pass ? np : 0);
+    const RowCounts cnt = exact_counts(mem, m, upper.b, upper.p);
     bool ok_post = false, ok_pp = false;
     if (do_post) post_fits(t, k, mem, m, mem.out, k.no_ck ? t[MIST_T_RD] : 0.0, ok_post, ok_pp);
     ok_post = ok_post && pass;
     ok_pp = ok_pp && do_pp && pass;
-    const uint64_t useful = __ballot(row_b > 0 || row_p > 0 || ok_post || ok_pp);
+    const uint64_t useful = __ballot(cnt.b > 0 || cnt.p > 0 || ok_post || ok_pp);
     if (useful == 0) continue;
     __builtin_amdgcn_wave_barrier();
     const int at = __popcll(useful & ((1ull << lane) - 1ull));
     if (useful >> lane & 1ull) {
-      put_sample_row(rows, at, t, x, d, k.no_ck, m, row_b, row_p, ok_post, ok_pp, do_post);
+      put_sample_row(rows, at, t, x, d, k.no_ck, m, cnt.b, cnt.p, ok_post, ok_pp, do_post);
       rows->number[at] = my_row_number;
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
