@@ -47,12 +47,17 @@ constexpr int kDpBatch = 4;  // end layers whose reads a lane of the one-lane-pe
 // takes as many whole rows as fit its 256 lanes, one lane per entry, so that loads and stores
 // are contiguous; the running minimum is a segmented scan (wavefront shuffles, LDS between the
 // wavefronts a row spans).  Rows longer than the workgroup are walked in passes of 256 entries
-// with the minimum of the earlier passes carried along.
+// with the minimum of the earlier passes carried along.  A workgroup takes kCostRuns such sets of
+// rows: with one each, 1.85e6 workgroups of a few hundred instructions per lane were bound by their
+// own start and by a 64-bit division per lane (70B on 32x8, 4.5e8 cells: 2.70 ms; division per
+// workgroup and lane shifts instead of shuffles through LDS 2.52, eight sets 2.02; 7B on 4x8 0.104
+// -> 0.083).  Bound: 12 bytes a cell and 16 more where it holds a row, at 3.5 TB/s.
 // Most cells of a plan hold no strategy (no group for that (g, mesh), or nothing fits): their
 // row index is -1 and their costs +inf, so with the index table (may be null) the 16 bytes of
 // such a cell's costs are not read.
 // The four tables of a call (base, with_pre, with_post, no_pp) go through one launch: table v
 // owns the workgroups first_block[v] .. first_block[v + 1] - 1.
+constexpr int kCostRuns = 8;
 struct CostTableJob {
   const double *stable[4], *delta[4];
   const int32_t *index[4];
@@ -73,41 +78,60 @@ __global__ __launch_bounds__(256) void cost_table_kernel(const CostTableJob job,
   const int seg = min(row_len, 256);  // entries of a row per pass
   const int rows_here = 256 / seg;
   const int local_row = threadIdx.x / seg, j0 = threadIdx.x % seg;
-  const int64_t r = (int64_t)(blockIdx.x - job.first_block[v]) * rows_here + local_row;
-  const bool live_row = local_row < rows_here && r < n_rows;
-  const float G = live_row ? (float)grad_accum[r / rows_per_g] : 1.0f;
-  float carry = INFINITY;
-  for (int base = 0; base < row_len; base += seg) {
-    const int j = base + j0;
-    const bool live = live_row && j < row_len;
-    const int64_t i = r * row_len + j;
-    float c = INFINITY;
-    if (live) {
-      if (index == nullptr || index[i * sample_size + slot] >= 0) {
-        const float s = (float)stable[i * sample_size + slot];
-        const float d = (float)delta[i * sample_size + slot];
-        c = s + d / G;
+  // (rows_per_g is the size of one g: 32 bits)
+  const uint32_t per_g = (uint32_t)rows_per_g;
+  const int64_t row0 = (int64_t)(blockIdx.x - job.first_block[v]) * rows_here * kCostRuns;
+  const int64_t g0 = row0 >> 32 == 0 ? (int64_t)((uint32_t)row0 / per_g) : row0 / rows_per_g;
+  const uint32_t in_g0 = (uint32_t)(row0 - g0 * rows_per_g);
+  for (int turn = 0; turn < kCostRuns; ++turn) {
+    const uint32_t ahead = (uint32_t)(turn * rows_here + local_row);
+    const int64_t r = row0 + ahead;
+    if (row0 + turn * rows_here >= n_rows) break;
+    const bool live_row = local_row < rows_here && r < n_rows;
+    const float G = live_row ? (float)grad_accum[g0 + (in_g0 + ahead) / per_g] : 1.0f;
+    float carry = INFINITY;
+    for (int base = 0; base < row_len; base += seg) {
+      const int j = base + j0;
+      const bool live = live_row && j < row_len;
+      const int64_t i = r * row_len + j;
+      float c = INFINITY;
+      if (live) {
+        if (index == nullptr || index[i * sample_size + slot] >= 0) {
+          const float s = (float)stable[i * sample_size + slot];
+          const float d = (float)delta[i * sample_size + slot];
+          c = s + d / G;
+        }
+        out[i] = c;
       }
-      out[i] = c;
+      // running minimum over the row's lanes of this pass: inside a wavefront by lane shifts that stop
+      // at the row's first lane, then the part of the row that lies in earlier wavefronts (their
+      // last lanes hold it)
+      float run = c;
+      const int lane = threadIdx.x & 63;
+      // `run` of the lane `control` names, where it is `distance` back in the same row of the table;
+      // a lane without a source keeps its own
+#define MIST_RUN_DPP(control, rows, distance)                                                    \
+    {                                                                                              \
+      const int other = __builtin_amdgcn_update_dpp(__float_as_int(run), __float_as_int(run),      \
+                                                    control, rows, 0xf, false);                    \
+      run = j0 >= (distance) ? fminf(run, __int_as_float(other)) : run;                            \
     }
-    // running minimum over the row's lanes of this pass: inside a wavefront by shuffles that stop
-    // at the row's first lane, then the part of the row that lies in earlier wavefronts (their
-    // last lanes hold it)
-    float run = c;
-    const int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int step = 1; step < 64; step <<= 1) {
-      const float other = __shfl_up(run, step);
-      if (lane >= step && j0 >= step) run = fminf(run, other);
+      MIST_RUN_DPP(0x111, 0xf, 1)  // row_shr:1
+      MIST_RUN_DPP(0x112, 0xf, 2)
+      MIST_RUN_DPP(0x114, 0xf, 4)
+      MIST_RUN_DPP(0x118, 0xf, 8)
+      MIST_RUN_DPP(0x142, 0xa, (lane & 15) + 1)  // row_bcast:15 into the odd rows of 16 lanes
+      MIST_RUN_DPP(0x143, 0xc, lane - 31)        // row_bcast:31 into the upper half
+#undef MIST_RUN_DPP
+      lds[threadIdx.x] = run;
+      __syncthreads();
+      const int row_first = (int)threadIdx.x - j0;
+      for (int at = (int)(threadIdx.x & ~63u) - 1; at >= row_first; at -= 64) run = fminf(run, lds[at]);
+      if (live) pmin[i] = fminf(run, carry);
+      if (base + seg < row_len)  // only rows longer than one pass: then the row is the workgroup
+        carry = fminf(carry, fminf(fminf(lds[63], lds[127]), fminf(lds[191], lds[255])));
+      __syncthreads();
     }
-    lds[threadIdx.x] = run;
-    __syncthreads();
-    const int row_first = (int)threadIdx.x - j0;
-    for (int at = (int)(threadIdx.x & ~63u) - 1; at >= row_first; at -= 64) run = fminf(run, lds[at]);
-    if (live) pmin[i] = fminf(run, carry);
-    if (base + seg < row_len)  // only rows longer than one pass: then the row is the workgroup
-      carry = fminf(carry, fminf(fminf(lds[63], lds[127]), fminf(lds[191], lds[255])));
-    __syncthreads();
   }
 }
 
@@ -1861,7 +1885,7 @@ int mist_dp_cost_tables(const MistProblem *problem, const MistOutTables *tables,
     return fail(MIST_E_INVALID, "bad problem extents");
   if (slot < 0 || slot >= S) return fail(MIST_E_INVALID, "slot %d outside [0, %d)", slot, (int)S);
   const int64_t rows_per_g[4] = {Q * P1 * L, Q * P1 * L, Q * L, Q};
-  const int64_t rows_per_block = 256 / std::min<int64_t>(L + 1, 256);
+  const int64_t rows_per_block = 256 / std::min<int64_t>(L + 1, 256) * kCostRuns;
   CostTableJob job = {};
   int64_t blocks = 0;
   for (int v = 0; v < 4; ++v) {
