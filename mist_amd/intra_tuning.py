@@ -613,17 +613,20 @@ class IntraStageTuner:
             starts.append(starts[-1] + int(np.prod(shape)))
         return shapes, starts
 
-    def _allocate_flat(self, plan: Optional[dict] = None):
+    def _allocate_flat(self, plan: Optional[dict] = None, fill_costs: bool = True):
         """The output tables as two flat allocations (float64 costs: stable then delta; int32
         row indices) with their pre-fill queued on the current stream, and the ``MistOutTables``
         of pointers into them.  Pre-filled with +inf / -1: everywhere, or (``plan`` of a tuner
-        with ``prefill_wanted_cells_only``) in the cells ``cells_wanted`` names."""
+        with ``prefill_wanted_cells_only``) in the cells ``cells_wanted`` names.  ``fill_costs``
+        False: the costs are defined where an index is not -1."""
         shapes, starts = self._table_layout()
         total, dev = starts[-1], self.device
         wanted = plan.get("wanted") if plan is not None and self.prefill_wanted_cells_only else None
         if wanted is None:
             # one allocation and one fill per element type
-            costs = torch.full((2 * total,), float("inf"), dtype=torch.float64, device=dev)
+            costs = torch.empty((2 * total,), dtype=torch.float64, device=dev)
+            if fill_costs:
+                costs.fill_(float("inf"))
             index = torch.full((total,), -1, dtype=torch.int32, device=dev)
         else:
             costs = torch.empty((2 * total,), dtype=torch.float64, device=dev)
@@ -853,7 +856,8 @@ class IntraStageTuner:
         return outs
 
     def run_prepared(self, plan, dev_plan,
-                     stage_cost_cutoff: Optional[dict] = None) -> List[IntraStageTunerOutput]:
+                     stage_cost_cutoff: Optional[dict] = None,
+                     fill_costs: bool = True) -> List[IntraStageTunerOutput]:
         """Device part only: fresh output tables + kernel launches for an uploaded plan; one
         output per tp size, all resident in the same tables.
 
@@ -861,7 +865,10 @@ class IntraStageTuner:
         whose inter-stage search is all that reads the tables: the scout pass turns its seeds
         into an upper bound of the best pipeline cost (``MistProblem.stage_cost_incumbent``),
         and the main launch does not look for stage costs that no threshold of that search can
-        admit.  Cells above that bound then hold some value above it, not their minimum."""
+        admit.  Cells above that bound then hold some value above it, not their minimum.
+
+        ``fill_costs`` False is for a caller that reads the costs of cells with a row index only:
+        the tables are not pre-filled with +inf."""
         problem = plan["problem"]
         problem["stage_cost_incumbent"] = 0
         if stage_cost_cutoff is not None and self.sample_size == 1 and not self.exhaustive:
@@ -873,7 +880,7 @@ class IntraStageTuner:
             problem["incumbent_num_devices"] = int(stage_cost_cutoff["num_devices"])
             problem["incumbent_ckpt_rule"] = int(stage_cost_cutoff["ckpt_rule"])
         with torch.cuda.device(self.device):
-            costs, index, struct = self._allocate_flat(plan)
+            costs, index, struct = self._allocate_flat(plan, fill_costs)
             self.launch(plan, dev_plan, struct)
             # (the tensor views of the tables are made while the kernels run)
             tables = self._table_views(costs, index)
