@@ -1991,6 +1991,32 @@ __device__ __forceinline__ FlatQueue flat_queue(const ReduceTables &tabs, int qu
   return q;
 }
 
+// The same in chunks of up to 64 items of one shard.
+struct ChunkQueue {
+  uint32_t end, items;  // of this lane's shard: chunks up to it, items in it
+  uint32_t chunks;
+  // first item of chunk u, number of its items
+  __device__ __forceinline__ int64_t at(uint32_t u, uint32_t capacity, int *n) const {
+    const int shard = __popcll((unsigned long long)__ballot(end <= u));
+    const uint32_t before = shard > 0 ? (uint32_t)from_lane((int)end, shard - 1) : 0u;
+    const uint32_t first = (u - before) * 64u;
+    *n = (int)min(64u, (uint32_t)from_lane((int)items, shard) - first);
+    return (int64_t)shard * capacity + first;
+  }
+};
+__device__ __forceinline__ ChunkQueue chunk_queue(const ReduceTables &tabs, int queue) {
+  const int lane = threadIdx.x & 63;
+  ChunkQueue q;
+  q.items = min(tabs.counter[(queue * kQueueShards + lane) * kCounterPitch], tabs.capacity);
+  q.end = (q.items + 63u) / 64u;
+  for (int step = 1; step < 64; step <<= 1) {
+    const uint32_t o = (uint32_t)__shfl_up((int)q.end, step);
+    if (lane >= step) q.end += o;
+  }
+  q.chunks = (uint32_t)from_lane((int)q.end, 63);
+  return q;
+}
+
 // A lane's pair of a tile.
 struct TileLane {
   PairIndex pc;
@@ -2359,24 +2385,10 @@ __global__ __launch_bounds__(kReduceThreads, 3) void reduce_kernel(
   extern __shared__ double lds_rows[];
   constexpr int kWaves = kReduceThreads / 64;
   const int local_wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
-  const FlatQueue queue = flat_queue(tabs, 1);
-  int split = 0;  // enough units for every wavefront several times over
-  while (split < 4 && ((uint64_t)queue.total << split) < (uint64_t)gridDim.x * kWaves * 2) ++split;
-  const uint64_t units = (uint64_t)queue.total << split;
-  auto work = [&](uint32_t u) {
-    uint64_t pairs = every_pair(split) << (u & ((1u << split) - 1u));
-    const int64_t at = queue.at(u >> split, tabs.capacity);
-    if (kResolve) pairs &= from_lane((uint64_t)tabs.hit[at], 0);
-    if (pairs == 0) return;
-    const uint64_t item = from_lane((uint64_t)tabs.opened[at], 0);
+  const uint32_t n_waves = gridDim.x * kWaves;
+  auto work = [&](int64_t at, uint64_t item, uint64_t pairs) {
     const int gi = (int)(item >> 48), tile_rel = (int)(item >> 32 & 0xffff), stage = (int)(uint32_t)item;
     const MistGroupDesc *g = groups + gi;
-    if (kResolve) {  // pairs whose minima changed
-      const int n_slots = slots_of(g->num_p);
-      const int64_t cell = g->cell_offset + ((int64_t)tile_rel * MIST_LC_TILE + lane) * n_slots;
-      pairs &= __ballot(tabs.changed[cell / 4] != 0);
-      if (pairs == 0) return;
-    }
     uint64_t hit;
     if constexpr (kSamples) {
       __shared__ SampleRows lds_samples[kWaves];
@@ -2387,11 +2399,30 @@ __global__ __launch_bounds__(kReduceThreads, 3) void reduce_kernel(
                                   lds_rows + local_wave * row_pitch);
     if (!kResolve && hit != 0 && lane == 0) atomicOr(tabs.hit + at, (unsigned long long)hit);
   };
+  constexpr bool kListed = kResolve && kSamples;
+  const FlatQueue queue = flat_queue(tabs, kListed ? 0 : 1);
+  int split = 0;  // enough units for every wavefront several times over
+  while (split < 4 && ((uint64_t)queue.total << split) < (uint64_t)n_waves * 2) ++split;
+  const uint64_t units = (uint64_t)queue.total << split;
   if (kResolve) {  // few are left: handed out in turn
-    for (uint64_t u = (uint64_t)blockIdx.x * kWaves + local_wave; u < units; u += (uint64_t)gridDim.x * kWaves)
-      work((uint32_t)u);
+    for (uint64_t u = (uint64_t)blockIdx.x * kWaves + local_wave; u < units; u += n_waves) {
+      int64_t at = queue.at((uint32_t)(u >> split), tabs.capacity);
+      if (kListed) at = (int64_t)from_lane((uint64_t)tabs.item[at], 0);
+      uint64_t pairs = from_lane((uint64_t)tabs.hit[at], 0) & (every_pair(split) << (u & ((1u << split) - 1u)));
+      if (pairs == 0) continue;
+      const uint64_t item = from_lane((uint64_t)tabs.opened[at], 0);
+      if (!kListed) {  // pairs whose minima changed
+        const MistGroupDesc *g = groups + (item >> 48);
+        const int64_t tile_cell = g->cell_offset + (int64_t)(item >> 32 & 0xffff) * MIST_LC_TILE * slots_of(g->num_p);
+        pairs &= __ballot(tabs.changed[(tile_cell + lane * slots_of(g->num_p)) / 4] != 0);
+        if (pairs == 0) continue;
+      }
+      work(at, item, pairs);
+    }
     return;
   }
+  // (the resolve list goes where the filter's items were)
+  if (kSamples && blockIdx.x == 0 && threadIdx.x < kQueueShards) tabs.counter[threadIdx.x * kCounterPitch] = 0;
   for (int k = 0; k < kNumXcd; ++k) {
     const int part = ((int)blockIdx.x + k) % kNumXcd;
     const uint32_t first = (uint32_t)(units * part / kNumXcd), n = (uint32_t)(units * (part + 1) / kNumXcd) - first;
@@ -2407,7 +2438,47 @@ __global__ __launch_bounds__(kReduceThreads, 3) void reduce_kernel(
       const uint32_t u = (uint32_t)from_lane((int)ahead, 0);
       if (u >= n) break;
       ahead = draw();
-      work(first + u);
+      const int64_t at = queue.at((first + u) >> split, tabs.capacity);
+      work(at, from_lane((uint64_t)tabs.opened[at], 0), every_pair(split) << ((first + u) & ((1u << split) - 1u)));
+    }
+  }
+}
+
+// ---- resolve list (several samples) ----
+// A wavefront takes 64 neighbouring items of a shard, lane = item: of the pairs in which some row
+// reached its minimum those whose minima changed stay in `hit`, and the items that have any are
+// listed (places in `opened`).  (The resolve launch looked for them itself, a wavefront and four
+// dependent reads per item, and the few that were left sat with few wavefronts: 30 samples of one
+// tensor-parallel size of the 7B plan 2.03 ms, 1.37 with the list; the whole of 7B on 4x8 0.59 -> 0.27.)
+__global__ __launch_bounds__(kReduceThreads) void resolve_list_kernel(const MistGroupDesc *__restrict__ groups,
+                                                                      const ReduceTables tabs) {
+  constexpr int kWaves = kReduceThreads / 64;
+  const int lane = threadIdx.x & 63;
+  const ChunkQueue queue = chunk_queue(tabs, 1);
+  for (uint32_t u = (uint32_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * kWaves + (threadIdx.x >> 6)));
+       u < queue.chunks; u += gridDim.x * kWaves) {
+    int n_here;
+    const int64_t first = queue.at(u, tabs.capacity, &n_here);
+    const int64_t at = first + min(lane, n_here - 1);
+    uint64_t left = lane < n_here ? tabs.hit[at] : 0, mine = 0;
+    if (!__any(left != 0)) continue;
+    const uint64_t item = tabs.opened[at];
+    const MistGroupDesc *g = groups + (item >> 48);
+    const int n_slots = slots_of(g->num_p);
+    const int64_t cell0 = g->cell_offset + (int64_t)(item >> 32 & 0xffff) * MIST_LC_TILE * n_slots;
+    for (; left != 0; left &= left - 1) {
+      const int pair = __ffsll((unsigned long long)left) - 1;
+      if (tabs.changed[(cell0 + pair * n_slots) / 4] != 0) mine |= 1ull << pair;
+    }
+    const uint64_t found = (uint64_t)__ballot(mine != 0);
+    if (found == 0) continue;
+    const int shard = (int)(first / tabs.capacity);  // (no more than the shard's items: it cannot overflow)
+    uint32_t base = 0;
+    if (lane == 0) base = atomicAdd(tabs.counter + shard * kCounterPitch, (uint32_t)__popcll(found));
+    base = (uint32_t)from_lane((int)base, 0);
+    if (mine != 0) {
+      tabs.hit[at] = mine;
+      tabs.item[(int64_t)shard * tabs.capacity + base + __popcll(found & ((1ull << lane) - 1ull))] = (unsigned long long)at;
     }
   }
 }
@@ -3369,15 +3440,18 @@ static int launch_reduce(const MistProblem *problem, const MistGroupDesc *d_grou
 #define MIST_REDUCE(RESOLVE, SAMPLES)                                                                       \
   hipLaunchKernelGGL((reduce_kernel<RESOLVE, SAMPLES>), dim3(kReduceBlocks), dim3(kReduceThreads), lds,     \
                      (hipStream_t)stream, *problem, d_groups, d_row_terms, d_stage_floor, ratios, tabs, row_pitch)
-  if (tabs.n_samples == 1) {
-    MIST_REDUCE(false, false);
+  const bool one = tabs.n_samples == 1;
+  if (one) MIST_REDUCE(false, false);
+  else MIST_REDUCE(false, true);
+  MIST_HIP_CHECK(hipGetLastError());
+  // (with one sample the list costs what it saves, 15 us of 1.3B on 1x2, and 70B on 32x8 gains 0.06 ms)
+  if (!one) {
+    hipLaunchKernelGGL(resolve_list_kernel, dim3(kReduceBlocks / 4), dim3(kReduceThreads), 0, (hipStream_t)stream,
+                       d_groups, tabs);
     MIST_HIP_CHECK(hipGetLastError());
-    MIST_REDUCE(true, false);
-  } else {
-    MIST_REDUCE(false, true);
-    MIST_HIP_CHECK(hipGetLastError());
-    MIST_REDUCE(true, true);
   }
+  if (one) MIST_REDUCE(true, false);
+  else MIST_REDUCE(true, true);
 #undef MIST_REDUCE
   MIST_HIP_CHECK(hipGetLastError());
   return 0;
