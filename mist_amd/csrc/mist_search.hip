@@ -1189,8 +1189,10 @@ __device__ __forceinline__ void take_min(double &best, int32_t &best_row, bool f
 // count - 1 (the minima of a (l, c) pair do not decrease with p).
 //
 // The minima of every (group, (l, c) pair, variant, p, sample) live in one table in HBM
-// (ReduceTables.best) that all wavefronts lower by atomic minima on the bit patterns (costs are
-// not negative, so they order like integers).  Five launches:
+// (ReduceTables.best) that all wavefronts lower by float64 atomic minima (an objective can be
+// negative: the first micro-batch may be cheaper than the later ones, which swap weights in, and
+// with a small alpha and few accumulation steps its share of the difference outweighs the rest).
+// Five launches:
 //   seed     the rows of the group's scout pairs against empty minima, in LDS: upper bounds made
 //            of real rows, final for most cells;
 //   filter   stage summaries (term-wise minima of 64 rows, and of 8 such stages) against the
@@ -1234,8 +1236,7 @@ constexpr double kBaseSlack = 1e-6;
 
 // (by value in the kernel arguments)
 struct ReduceTables {
-  // [pair][slot][sample] (slots_of(num_p) slots): bits of the smallest cost
-  unsigned long long *best;
+  double *best;  // [pair][slot][sample] (slots_of(num_p) slots): the smallest cost
   // its lowest row, ~0 = none; kUnresolved + row from the reduce launch, row from the resolve launch
   // (smaller than any of the former)
   uint32_t *row;
@@ -1341,13 +1342,19 @@ __device__ __forceinline__ uint32_t wave_min(uint32_t v) {
 #undef MIST_MIN_DPP
   return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
-// A lane with `pending` whose cost is the smallest to float32 (costs are not negative).
+// A lane with `pending` whose cost is the smallest to float32.  (Keys of floats in their order: all
+// bits flipped under a sign, else the sign bit.)
 __device__ __forceinline__ int cheapest_lane(bool pending, double cost) {
-  const uint32_t key = pending ? __float_as_uint((float)cost) : ~0u;
+  const int bits = __float_as_int((float)cost);
+  const uint32_t key = pending ? (uint32_t)bits ^ ((uint32_t)(bits >> 31) | 0x80000000u) : ~0u;
   return __ffsll((unsigned long long)__ballot(key == wave_min(key))) - 1;
 }
-__device__ __forceinline__ double cost_of_bits(unsigned long long bits) {
-  return __longlong_as_double((long long)bits);
+// One entry of the minima in device memory / in LDS (global_atomic_min_f64, ds_min_f64).
+__device__ __forceinline__ void lower_minimum(double *entry, double cost) {
+  __hip_atomic_fetch_min(entry, cost, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void lower_minimum_in_lds(double *entry, double cost) {
+  __hip_atomic_fetch_min(entry, cost, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
 // Slots of a pair in ReduceTables: base p = 0.., with_pre p = 0.., with_post, no_pp.
@@ -1595,7 +1602,7 @@ __device__ __forceinline__ void clear_queue(const ReduceTables &tabs) {
 __global__ __launch_bounds__(kSeedThreads) void seed_kernel(
     const MistProblem prob, const MistGroupDesc *__restrict__ groups, const double *__restrict__ row_terms,
     double ratio, ReduceTables tabs, int pair_split) {
-  extern __shared__ unsigned long long lds_best[];
+  extern __shared__ double lds_best[];
   const MistGroupDesc *g = groups + blockIdx.y;
   const int parts = MIST_LC_TILE / pair_split;
   const int tile_rel = (int)blockIdx.x / parts, part = (int)blockIdx.x % parts;
@@ -1606,8 +1613,7 @@ __global__ __launch_bounds__(kSeedThreads) void seed_kernel(
   const int first_pair = (g->lc_tile_begin + tile_rel) * MIST_LC_TILE + part * pair_split;
   const int n_here = min(pair_split, n_pairs - first_pair);
   const int n_entries = pair_split * n_slots;  // [pair][slot]
-  const unsigned long long kInf = (unsigned long long)__double_as_longlong((double)INFINITY);
-  for (int e = threadIdx.x; e < n_entries; e += kSeedThreads) lds_best[e] = kInf;
+  for (int e = threadIdx.x; e < n_entries; e += kSeedThreads) lds_best[e] = INFINITY;
   __syncthreads();
   if (g->scout_stride > 0 && n_here > 0) {
     constexpr int kWaves = kSeedThreads / 64;
@@ -1640,13 +1646,13 @@ __global__ __launch_bounds__(kSeedThreads) void seed_kernel(
             live && (cutoff == INFINITY || ratio * (double)x + m.div_G((double)d) <= cutoff * (1.0 + kBaseSlack));
         if (!__any(wanted)) continue;
         const LaneMemory mem = pair_memory(t, k);
-        unsigned long long *mine = lds_best + i * n_slots;
+        double *mine = lds_best + i * n_slots;
         const Objectives o = objectives(t, x, d, k.no_ck, ratio, m, do_post);
         // the minima do not decrease with p: at the bound of its count a row meets the largest one
         // it could beat
         const UpperCounts upper = upper_counts(mem, m, wanted ? np : 0);
-        auto may = [&](int count, double cost, const unsigned long long *slots) {
-          return count > 0 && (unsigned long long)__double_as_longlong(cost) < slots[max(count - 1, 0)];
+        auto may = [&](int count, double cost, const double *slots) {
+          return count > 0 && cost < slots[max(count - 1, 0)];
         };
         const bool may_b = may(upper.b, o.base, mine), may_p = may(upper.p, o.pre, mine + P);
         const bool may_post = do_post && may(wanted, o.post, mine + 2 * P);
@@ -1655,15 +1661,13 @@ __global__ __launch_bounds__(kSeedThreads) void seed_kernel(
         const RowCounts cnt = exact_counts(mem, m, may_b ? upper.b : 0, may_p ? upper.p : 0);
         bool ok_post = false, ok_pp = false;
         if (do_post) post_fits(t, k, mem, m, mem.out, k.no_ck ? t[MIST_T_RD] : 0.0, ok_post, ok_pp);
-        auto offer = [&](int count, double cost, unsigned long long *slots) {
-          const unsigned long long bits = (unsigned long long)__double_as_longlong(cost);
-          bool pending = count > 0 && bits < slots[max(count - 1, 0)];
+        auto offer = [&](int count, double cost, double *slots) {
+          bool pending = count > 0 && cost < slots[max(count - 1, 0)];
           while (__any(pending)) {
             const int r = cheapest_lane(pending, cost);
             const double its_cost = from_lane(cost, r);
             const int its_count = from_lane(count, r);
-            for (int j = lane; j < its_count; j += 64)
-              atomicMin(slots + j, (unsigned long long)__double_as_longlong(its_cost));
+            for (int j = lane; j < its_count; j += 64) lower_minimum_in_lds(slots + j, its_cost);
             pending = pending && lane != r && (count > its_count || cost < its_cost);
           }
         };
@@ -1722,7 +1726,7 @@ __device__ __forceinline__ void put_sample_row(SampleRows *rows, int at, const R
 __global__ __launch_bounds__(64) void seed_samples_kernel(
     const MistProblem prob, const MistGroupDesc *__restrict__ groups, const double *__restrict__ row_terms,
     const RatioList ratios, ReduceTables tabs, int sample_split) {
-  extern __shared__ unsigned long long lds_best[];
+  extern __shared__ double lds_best[];
   const MistGroupDesc *g = groups + blockIdx.y;
   clear_queue(tabs);
   const int tile_rel = (int)blockIdx.x / MIST_LC_TILE, lane = threadIdx.x;
@@ -1732,9 +1736,8 @@ __global__ __launch_bounds__(64) void seed_samples_kernel(
   const int first_sample = (int)blockIdx.z * sample_split, S = min(sample_split, tabs.n_samples - first_sample);
   const int pair = g->lc_tile_begin * MIST_LC_TILE + (int)blockIdx.x;
   SampleRows *rows = reinterpret_cast<SampleRows *>(lds_best);
-  unsigned long long *mine = lds_best + sizeof(SampleRows) / 8;  // [slot][sample]
-  const unsigned long long kInf = (unsigned long long)__double_as_longlong((double)INFINITY);
-  for (int e = lane; e < n_slots * S; e += 64) mine[e] = kInf;
+  double *mine = lds_best + sizeof(SampleRows) / 8;  // [slot][sample]
+  for (int e = lane; e < n_slots * S; e += 64) mine[e] = INFINITY;
   __syncthreads();
   const int sample = lane & 31;
   if (g->scout_stride > 0 && pair < n_pairs) {
@@ -1774,8 +1777,7 @@ __global__ __launch_bounds__(64) void seed_samples_kernel(
         auto offer = [&](bool ok, int variant, int slot) {
           const double2 xy = rows->xy[variant][r];
           const double cost = ratio * xy.x + xy.y;
-          if (ok && sample < S && cost < INFINITY)
-            atomicMin(mine + slot * S + sample, (unsigned long long)__double_as_longlong(cost));
+          if (ok && sample < S && cost < INFINITY) lower_minimum_in_lds(mine + slot * S + sample, cost);
         };
         offer(nb > 0, 0, nb - 1);
         offer(npre > 0, 1, P + npre - 1);
@@ -1791,11 +1793,11 @@ __global__ __launch_bounds__(64) void seed_samples_kernel(
   if (sample < S) {
     const int v = lane >> 5;  // base, with_pre
     const int64_t at = cell0 * tabs.n_samples + first_sample + sample;
-    unsigned long long low = kInf;
+    double low = INFINITY;
     for (int j = P - 1; j >= -1; --j) {
       const int slot = j >= 0 ? v * P + j : 2 * P + v;
-      const unsigned long long held = mine[slot * S + sample];
-      low = j >= 0 ? min(low, held) : held;
+      const double held = mine[slot * S + sample];
+      low = j >= 0 ? fmin(low, held) : held;
       tabs.best[at + (int64_t)slot * tabs.n_samples] = low;
       tabs.row[at + (int64_t)slot * tabs.n_samples] = ~0u;
     }
@@ -1908,7 +1910,7 @@ __global__ __launch_bounds__(MIST_LC_TILE) void filter_kernel(
   const bool do_post = active && pc.c != pc.l - 1, do_pp = do_post && pc.l == L;
   const GroupModel m = group_model(prob, g);
   const double cutoff = stage_cost_cutoff(prob, m.inv_G64);
-  const double *slots = reinterpret_cast<const double *>(tabs.best) +
+  const double *slots = tabs.best +
                         (g->cell_offset + ((int64_t)tile_rel * MIST_LC_TILE + lane) * slots_of(P)) * S;
 
   // no lane's row can matter: the pseudo row against the loosest minima
@@ -2056,7 +2058,7 @@ __global__ __launch_bounds__(kReduceThreads) void open_kernel(const MistProblem 
     const int P = g->num_p;
     const double *__restrict__ f = stage_floor + stage_floor_slot(g, gi, stage) * kStageFloorPitch;
     const StageReach reach = stage_reach(f, pair_consts(p.pc.l, p.pc.c), p.np, p.do_post, p.do_pp, m);
-    const double *slots = reinterpret_cast<const double *>(tabs.best) +
+    const double *slots = tabs.best +
                           (g->cell_offset + ((int64_t)tile_rel * MIST_LC_TILE + lane) * slots_of(P)) * S;
     bool open = false;
     for (int s = 0; s < S && !__any(open); ++s)
@@ -2135,7 +2137,7 @@ __device__ __forceinline__ uint64_t reduce_item(const MistProblem &prob, const M
   const GroupModel m = group_model(prob, g);
   const double cutoff = stage_cost_cutoff(prob, m.inv_G64);
   const int64_t tile_cell = g->cell_offset + (int64_t)tile_rel * MIST_LC_TILE * n_slots;
-  const double *best = reinterpret_cast<const double *>(tabs.best) + tile_cell;  // [pair][slot]
+  const double *best = tabs.best + tile_cell;  // [pair][slot]
 
   // ---- lane = pair: slots the pseudo row of the stage can reach, and the minima there ----
   const double *__restrict__ f = stage_floor + stage_floor_slot(g, gi, stage) * kStageFloorPitch;
@@ -2220,7 +2222,7 @@ __device__ __forceinline__ uint64_t reduce_item(const MistProblem &prob, const M
       const int own = slot + max(count - 1, 0);
       const double now = in && count > 0 && cost <= cutoff && cost < INFINITY ? lds_row[own] : -INFINITY;
       if (!kResolve && cost < now) {
-        atomicMin(tabs.best + cell + own, (unsigned long long)__double_as_longlong(cost));
+        lower_minimum(tabs.best + cell + own, cost);
         lowered = true;
       }
       if (cost == now) atomicMin(tabs.row + cell + own, my_row_number);
@@ -2253,7 +2255,7 @@ __device__ __forceinline__ uint64_t reduce_item_samples(const MistProblem &prob,
   const int P = g->num_p, n_slots = slots_of(P), S = tabs.n_samples;
   const GroupModel m = group_model(prob, g);
   const int64_t tile_cell = g->cell_offset + (int64_t)tile_rel * MIST_LC_TILE * n_slots;
-  const double *best = reinterpret_cast<const double *>(tabs.best) + tile_cell * S;  // [pair][slot][sample]
+  const double *best = tabs.best + tile_cell * S;  // [pair][slot][sample]
   const double *__restrict__ f = stage_floor + stage_floor_slot(g, gi, stage) * kStageFloorPitch;
   const double ratio = ratios.r[min(sample, S - 1)];
   const StageReach reach = stage_reach(f, pair_consts(tl.pc.l, tl.pc.c), tl.np, tl.do_post, tl.do_pp, m);
@@ -2345,7 +2347,7 @@ __device__ __forceinline__ uint64_t reduce_item_samples(const MistProblem &prob,
         if (cost == now) {
           atomicMin(tabs.row + to, rows->number[r]);
         } else if (!kResolve) {
-          atomicMin(tabs.best + to, (unsigned long long)__double_as_longlong(cost));
+          lower_minimum(tabs.best + to, cost);
           lowered = true;
         }
       };
@@ -2664,13 +2666,13 @@ __global__ __launch_bounds__(64 * kIncumbentWaves) void incumbent_kernel(
   const int S = incumbent_stage_count(prob, g);
   if (S == 0) return;
   const int l = L / S, P = g->num_p;
-  // seed of the stage's (l, c) cell in slot `slot` (one sample: bits of +inf where there is none)
+  // seed of the stage's (l, c) cell in slot `slot` (one sample; +inf where there is none)
   auto seed_of = [&](int slot, int c) {
     const int pair = l * (l + 1) / 2 - 1 + c;
     const int lc_tile = pair / MIST_LC_TILE - g->lc_tile_begin;
     if (lc_tile < 0 || lc_tile >= g->n_lc_tiles) return (double)INFINITY;
-    return cost_of_bits(tabs.best[g->cell_offset +
-                                  ((int64_t)lc_tile * MIST_LC_TILE + pair % MIST_LC_TILE) * slots_of(P) + slot]);
+    return tabs.best[g->cell_offset +
+                     ((int64_t)lc_tile * MIST_LC_TILE + pair % MIST_LC_TILE) * slots_of(P) + slot];
   };
   // cheapest one over c = 0..c_last
   auto cheapest = [&](int slot, int c_last) {
@@ -2709,7 +2711,7 @@ __global__ __launch_bounds__(64 * kIncumbentWaves) void incumbent_kernel(
     largest = fmax(largest, wave_largest[w]);
   }
   const double total = sum + (double)(g->grad_accum - 1) * largest;
-  // costs are not negative, and non-negative doubles order like their bit patterns
+  // (a pipeline's cost, unlike an objective of another alpha, is not negative: its bits order)
   if (threadIdx.x == 0 && total >= 0.0 && total < INFINITY)
     atomicMin(reinterpret_cast<unsigned long long *>(prob.stage_cost_incumbent),
               (unsigned long long)__double_as_longlong(total));
@@ -2757,7 +2759,7 @@ __global__ __launch_bounds__(256) void estimate_stage_minima_kernel(
   const float G32 = (float)g->grad_accum;
   const double *__restrict__ src = row_terms + g->row_offset * MIST_ROW_TERMS;
   auto offer = [&](int st, bool ok, double cost) {
-    // costs are not negative, and non-negative doubles order like their bit patterns
+    // (stage costs, unlike objectives of another alpha, are not negative: their bits order)
     if (ok && cost >= 0.0 && cost < INFINITY)
       atomicMin(&stage_min[st], (unsigned long long)__double_as_longlong(cost));
   };
@@ -2861,7 +2863,7 @@ __global__ __launch_bounds__(256) void combine_slabs_kernel(
         take_min(best, best_row, row >= 0, slab_cost[at], row);
       }
       const int64_t cell = g->cell_offset + ((int64_t)tile_rel * MIST_LC_TILE + lane) * slots_of(P) + slot;
-      tabs.best[cell] = (unsigned long long)__double_as_longlong(best);
+      tabs.best[cell] = best;
       tabs.row[cell] = (uint32_t)best_row;
     }
   }
@@ -2912,10 +2914,9 @@ __device__ __forceinline__ void write_final(FinalCell &f, const MistGroupDesc *_
   tables.index[variant][at] = (int32_t)row;
 }
 // (row as left by the reduction: ~0 none)
-__device__ __forceinline__ void take_lower(unsigned long long &cost, uint32_t &row, unsigned long long its_cost,
-                                           uint32_t its_row) {
+__device__ __forceinline__ void take_lower(double &cost, uint32_t &row, double its_cost, uint32_t its_row) {
   row = its_cost < cost ? its_row : its_cost == cost ? min(row, its_row) : row;
-  cost = min(cost, its_cost);
+  cost = fmin(cost, its_cost);
 }
 __device__ __forceinline__ uint32_t row_number(uint32_t held) { return held == ~0u ? held : held & ~kUnresolved; }
 
@@ -2928,7 +2929,7 @@ __global__ __launch_bounds__(256) void finalize_kernel(
     const MistProblem prob, const MistGroupDesc *__restrict__ groups, const double *__restrict__ row_terms,
     const ReduceTables tabs, int sample_at, MistOutTables tables) {
   __shared__ uint32_t winner[MIST_LC_TILE][kFinalSlots + 1];
-  __shared__ unsigned long long carry_cost[MIST_LC_TILE];
+  __shared__ double carry_cost[MIST_LC_TILE];
   __shared__ uint32_t carry_row[MIST_LC_TILE];
   const int L = prob.num_layers, n_pairs = L * (L + 1) / 2 + L;
   const MistGroupDesc *g = groups + blockIdx.z;
@@ -2944,7 +2945,7 @@ __global__ __launch_bounds__(256) void finalize_kernel(
   const int64_t first = g->cell_offset + (int64_t)tile_rel * MIST_LC_TILE * n_slots +
                         (variant < 2 ? variant * P : 2 * g->num_p + variant - 2);
   if (threadIdx.x < MIST_LC_TILE) {
-    carry_cost[threadIdx.x] = ~0ull;
+    carry_cost[threadIdx.x] = INFINITY;
     carry_row[threadIdx.x] = ~0u;
   }
   for (int p0 = (P - 1) / kFinalSlots * kFinalSlots; p0 >= 0; p0 -= kFinalSlots) {
@@ -2955,14 +2956,14 @@ __global__ __launch_bounds__(256) void finalize_kernel(
       const PairIndex its = decode_pair(min(first_pair + pair, n_pairs - 1));
       const int np = its.c == its.l - 1 ? 1 : P;  // (later slots hold no minima)
       const int64_t cell = first + (int64_t)pair * n_slots + p;
-      unsigned long long cost = ~0ull;
+      double cost = INFINITY;
       uint32_t row = ~0u;
       if (p < np) {
         cost = tabs.best[cell];
         row = row_number(tabs.row[cell]);
       }
       for (int step = 1; step < kFinalSlots; step <<= 1) {
-        const unsigned long long its_cost = __shfl_down(cost, step, kFinalSlots);
+        const double its_cost = __shfl_down(cost, step, kFinalSlots);
         const uint32_t its_row = __shfl_down(row, step, kFinalSlots);
         if (j + step < kFinalSlots) take_lower(cost, row, its_cost, its_row);
       }
@@ -3004,7 +3005,7 @@ __global__ __launch_bounds__(256) void finalize_samples_kernel(
   const int64_t first = (g->cell_offset + (int64_t)pair_rel * slots_of(P) +
                          (variant < 2 ? variant * P : 2 * P + variant - 2)) * n + s;
   const GroupConsts k = group_consts(g);
-  unsigned long long cost = ~0ull;
+  double cost = INFINITY;
   uint32_t row = ~0u;
   for (int p = f.n_p - 1; p >= p_begin; --p) {
     take_lower(cost, row, tabs.best[first + (int64_t)p * n], row_number(tabs.row[first + (int64_t)p * n]));
@@ -3321,7 +3322,7 @@ static int reduce_tables(const MistProblem *problem, int n_samples, double *d_pa
   const WorkspaceLayout w =
       workspace_layout(problem->reduce_cells, problem->reduce_supers, problem->reduce_items, n_samples);
   if (w.capacity >= (int64_t)1 << 31) return fail(MIST_E_INVALID, "too many (tile, stage) items");
-  out->best = reinterpret_cast<unsigned long long *>(d_partial_cost + w.best);
+  out->best = d_partial_cost + w.best;
   out->row = reinterpret_cast<uint32_t *>(d_partial_index);
   out->super_floor = d_partial_cost + w.supers;
   out->item = reinterpret_cast<unsigned long long *>(d_partial_cost + w.items);
