@@ -1229,10 +1229,12 @@ constexpr int kSeedLdsBytes = 40 * 1024;     // LDS aimed at per seed workgroup:
 constexpr int kSeedLdsMost = 160 * 1024;
 static_assert(kQueueShards == 64, "a lane per shard");
 constexpr uint32_t kUnresolved = 0x80000000u;
+// Room below r x and below the terms the composite objectives add (their roundings: a few 1e-16) ...
 constexpr double kSlack = 1e-9;
-// r x + d / G in float64 against a threshold of the base objective, whose second term is rounded to
-// float32 (one part in 2^24)
-constexpr double kBaseSlack = 1e-6;
+// ... and below d / G, which the base objective rounds to float32 (one part in 2^24).  Relative to
+// the operands, not to their sum: d can be negative, and where r x and d / G cancel the sum is far
+// smaller than what was rounded.
+constexpr double kShareSlack = 1e-7;
 
 // (by value in the kernel arguments)
 struct ReduceTables {
@@ -1437,12 +1439,23 @@ __device__ __forceinline__ int count_exact(const Scaled &scaled, int count, doub
 struct GroupModel {
   GroupConsts k;
   double cap, G64, inv_G64;
+  double inv_G_down, inv_G_up;  // 1 / G, kShareSlack short and long
   float G32, inv_G32;
   double pre_saved, pre_sas, pre_states, post_states, post_fwd_peak, post_bwd_peak, post_output;
   bool pow2;  // x / G == x * (1 / G) bit for bit, and the division leaves the inner loop
 
   __device__ __forceinline__ double div_G(double v) const { return pow2 ? v * inv_G64 : v / G64; }
   __device__ __forceinline__ float div_G(float v) const { return pow2 ? v * inv_G32 : v / G32; }
+
+  // At most d / G, and r * lower_x(x) + lower_share(d) at most the base objective of a row, by the
+  // slacks.  Monotone in x and d, so that of a stage's pseudo row bounds its rows' from below.
+  __device__ __forceinline__ double lower_share(float d) const {
+    return (double)d * (d < 0.0f ? inv_G_up : inv_G_down);
+  }
+  __device__ __forceinline__ double lower_x(float x) const { return (double)x * (1.0 - kSlack); }
+  __device__ __forceinline__ double bound(double ratio, float x, float d) const {
+    return ratio * lower_x(x) + lower_share(d);
+  }
 };
 __device__ __forceinline__ GroupModel group_model(const MistProblem &prob, const MistGroupDesc *g) {
   GroupModel m;
@@ -1452,6 +1465,8 @@ __device__ __forceinline__ GroupModel group_model(const MistProblem &prob, const
   m.G32 = (float)g->grad_accum;
   m.inv_G64 = 1.0 / m.G64;
   m.inv_G32 = 1.0f / m.G32;
+  m.inv_G_down = m.inv_G64 * (1.0 - kShareSlack);
+  m.inv_G_up = m.inv_G64 * (1.0 + kShareSlack);
   m.pre_saved = g->pre_saved;
   m.pre_sas = g->pre_states_and_saved;
   m.pre_states = g->pre_states;
@@ -1497,11 +1512,12 @@ __device__ __forceinline__ double stage_cost_cutoff(const MistProblem &prob, dou
 //   with_pre  = r (x + pre_fwd + pre_bwd + w1 + w2) + (d + w1d + w2d) / G
 //   with_post = r (x + post_fwd + [row terms >= 0]) + (d + [row terms >= 0]) / G
 //   no_pp     = r (x + pre_fwd + pre_bwd + post_fwd + [..] + w1 + w2 + [..]) + (d + w1d + w2d + [..]) / G
-// so each is at least `bound` = r x + d / G plus the offset below, up to a few roundings of
-// relative size 1e-16 (all terms are non-negative).  A row can beat a minimum `t` of such an
-// objective only if its bound <= t - offset; the offsets are taken 1e-9 short and `t` 1e-9 long, far
-// more than the roundings and far less than anything that matters for pruning.  The row terms of
-// the last two have their own minima over a stage (MIST_T_OPB, the NAG and NRS pairs).
+// so each is at least r x + d / G plus the offset below, up to a few roundings of relative size
+// 1e-16 of the operands (of which only d can be negative).  A row can reach a minimum `t` of such an
+// objective only if GroupModel::bound <= t - offset: the bound is short by the slacks of r x and
+// d / G, the offsets are taken 1e-9 short, so every operand has room for its roundings a million
+// times over, and it is far less than anything that matters for pruning.  The row terms of the
+// last two have their own minima over a stage (MIST_T_OPB, the NAG and NRS pairs).
 struct Offsets {
   double pre, post, pp;
 };
@@ -1518,9 +1534,6 @@ __device__ __forceinline__ Offsets composite_offsets(const GroupModel &m, double
   o.pp = (ratio * (k.pre_fwd + k.pre_bwd + k.post_fwd + k.w1 + k.w2) + shared) * (1.0 - kSlack) +
          stage_post;
   return o;
-}
-__device__ __forceinline__ double below(double t, double offset) {
-  return fabs(t) == INFINITY ? t : (t - offset) + kSlack * fabs(t);
 }
 
 // The last-stage / single-stage memory tests, p == 0 only (:2946-3106); `smallest_out`: what the
@@ -1643,7 +1656,7 @@ __global__ __launch_bounds__(kSeedThreads) void seed_kernel(
         pair_latency(t, k, x, d);
         // (under a bound most rows are above it and need no memory model)
         const bool wanted =
-            live && (cutoff == INFINITY || ratio * (double)x + m.div_G((double)d) <= cutoff * (1.0 + kBaseSlack));
+            live && (cutoff == INFINITY || m.bound(ratio, x, d) <= cutoff);
         if (!__any(wanted)) continue;
         const LaneMemory mem = pair_memory(t, k);
         double *mine = lds_best + i * n_slots;
@@ -1844,10 +1857,9 @@ __device__ __forceinline__ Loosest loosest_minima(const double *slots, int pitch
   return Loosest{count_b > 0 ? fmin(base, cutoff) : -INFINITY, count_p > 0 ? fmin(pre, cutoff) : -INFINITY,
                  do_post ? fmin(post, cutoff) : -INFINITY, do_pp ? fmin(pp, cutoff) : -INFINITY};
 }
-// One threshold for `bound` (see Offsets) that every row which could reach one of them passes.
+// One threshold for GroupModel::bound that every row which could reach one of them passes.
 __device__ __forceinline__ double bound_threshold(const Loosest &t, const Offsets &o) {
-  return fmax(t.base + kBaseSlack * fabs(t.base),
-              fmax(below(t.pre, o.pre), fmax(below(t.post, o.post), below(t.pp, o.pp))));
+  return fmax(t.base, fmax(t.pre - o.pre, fmax(t.post - o.post, t.pp - o.pp)));
 }
 
 // Lane = pair against a stage summary: the counts its pseudo row allows, hence which minima a row
@@ -1918,7 +1930,7 @@ __global__ __launch_bounds__(MIST_LC_TILE) void filter_kernel(
     float x, d;
     pair_latency(f, k, x, d);
     const Offsets o = composite_offsets(m, ratio, f[kStageMinOpb], f[kStageMinNag], f[kStageMinNrs]);
-    return !__any(ratio * (double)x + m.div_G((double)d) <= bound_threshold(t, o));
+    return !__any(m.bound(ratio, x, d) <= bound_threshold(t, o));
   };
   const double *__restrict__ supers = super_floor + super_floor_slot(g, gi, 0) * kStageFloorPitch;
   const double *__restrict__ stages = stage_floor + stage_floor_slot(g, gi, 0) * kStageFloorPitch;
@@ -2062,7 +2074,7 @@ __global__ __launch_bounds__(kReduceThreads) void open_kernel(const MistProblem 
                           (g->cell_offset + ((int64_t)tile_rel * MIST_LC_TILE + lane) * slots_of(P)) * S;
     bool open = false;
     for (int s = 0; s < S && !__any(open); ++s)
-      open = p.active && ratios.r[s] * (double)reach.x + m.div_G((double)reach.d) <=
+      open = p.active && m.bound(ratios.r[s], reach.x, reach.d) <=
                              reach.threshold(slots + s, S, P, ratios.r[s], cutoff, m, f);
     if (!__any(open)) continue;
     const uint32_t shard = (uint32_t)(from / tabs.capacity);
@@ -2146,7 +2158,7 @@ __device__ __forceinline__ uint64_t reduce_item(const MistProblem &prob, const M
   {
     const StageReach reach = stage_reach(f, pair_consts(tl.pc.l, tl.pc.c), tl.np, tl.do_post, tl.do_pp, m);
     thr = reach.threshold(best + lane * n_slots, 1, P, ratio, cutoff, m, f);
-    todo = pairs & __ballot(tl.active && ratio * (double)reach.x + m.div_G((double)reach.d) <= thr);
+    todo = pairs & __ballot(tl.active && m.bound(ratio, reach.x, reach.d) <= thr);
   }
   if (todo == 0) return 0;
 
@@ -2163,7 +2175,7 @@ __device__ __forceinline__ uint64_t reduce_item(const MistProblem &prob, const M
     const PairConsts k = pair_consts(from_lane(tl.pc.l, pl), from_lane(tl.pc.c, pl));
     float x, d;
     pair_latency(t, k, x, d);
-    const uint64_t pass = __ballot(live && ratio * (double)x + m.div_G((double)d) <= from_lane(thr, pl));
+    const uint64_t pass = __ballot(live && m.bound(ratio, x, d) <= from_lane(thr, pl));
     sieve = lane == pl ? pass : sieve;
   }
   todo = __ballot(sieve != 0);
@@ -2282,13 +2294,13 @@ __device__ __forceinline__ uint64_t reduce_item_samples(const MistProblem &prob,
     double thr = its.threshold(slots + min(sample, S - 1), S, P, ratio, INFINITY, m, f);
     if (kResolve)  // only the samples whose minima changed
       thr = tabs.changed[(tile_cell + pl * n_slots) / 4] >> sample & 1u ? thr : -INFINITY;
-    if (!__any(ratio * (double)its.x + m.div_G((double)its.d) <= thr)) continue;
+    if (!__any(m.bound(ratio, its.x, its.d) <= thr)) continue;
     // ---- lane = row ----
     float x, d;
     pair_latency(t, k, x, d);
-    const double xd = (double)x, dG = m.div_G((double)d);
+    const double low_x = m.lower_x(x), low_share = m.lower_share(d);
     bool pass = false;
-    for (int s = 0; s < S; ++s) pass = pass || ratios.r[s] * xd + dG <= from_lane(thr, s);
+    for (int s = 0; s < S; ++s) pass = pass || ratios.r[s] * low_x + low_share <= from_lane(thr, s);
     pass = pass && live;
     if (!__any(pass)) continue;
     if (!have_rest) {
@@ -2899,7 +2911,10 @@ __device__ __forceinline__ FinalCell final_cell(const MistProblem &prob, const M
 __device__ __forceinline__ void write_final(FinalCell &f, const MistGroupDesc *__restrict__ g, int variant, PairIndex pc,
                                             const GroupConsts &k, const double *__restrict__ row_terms, uint32_t row,
                                             int p, const MistOutTables &tables) {
-  if (row != f.priced) {
+  if (row == ~0u) {
+    f.stable = f.delta = INFINITY;
+    f.priced = row;
+  } else if (row != f.priced) {
     const double *t = row_terms + (g->row_offset + position_of_row(g, (int32_t)row)) * MIST_ROW_TERMS;
     const CellLatency lat = cell_latency<true>(t, pc.l, pc.c, k);
     if (variant == 0) { f.stable = (double)lat.x; f.delta = (double)lat.d; }

@@ -103,3 +103,43 @@ def test_tune_whose_answer_has_a_negative_objective(seed, base, layers, gpus, ba
     want = oracle_tune(cfg, tables)
     assert want[1] is not None
     assert tune(cfg) == want
+
+
+@pytest.mark.parametrize("exhaustive", [False, True], ids=["pruned", "every-cell"])
+@pytest.mark.parametrize("seed, layers, capacity, vocab", [(601, 8, 33.9, 622444), (2027, 7, 36.4, 774180)])
+def test_minima_far_smaller_than_their_operands(seed, layers, capacity, vocab, exhaustive):
+    """G = 3: the base objective rounds ``delta / G`` to float32.  Where it nearly cancels
+    ``r stable``, that rounding is more than a millionth of the minimum: a winner whose exact sum
+    lies above the minimum by more than such a share of it must not be pruned.  (Picked so that no
+    first-stage minimum keeps those cells open.)"""
+    from mist_amd.intra_tuning import IntraStageTuner
+    from oracle.pareto import alpha_ratios
+
+    mesh, G, samples, batch = (1, 2), 3, 30, 12
+    cfg, tables = _plan(seed, 2, layers, mesh, batch, capacity, vocab=vocab)
+    want, negative = _oracle(cfg, tables, mesh, G, 1, samples)
+    (index, stable, delta), pre_index = want[0], want[1][0]
+    ratio = alpha_ratios(samples)
+    with np.errstate(invalid="ignore"):
+        cost = ratio * stable + (delta.astype(np.float32) / np.float32(G)).astype(np.float64)
+        cancels = (index >= 0) & (pre_index < 0) & (ratio * stable + delta / G > cost + 1e-6 * np.abs(cost))
+    assert cancels.any() and negative[0] > 0
+    got = IntraStageTuner(tables, layers, [mesh], [G], 1, cfg, sample_size=samples, exhaustive=exhaustive).tune()
+    _hold(got, want, list(range(samples)))
+
+
+@pytest.mark.parametrize("seed, base, layers, mesh, G, batch, capacity", [
+    (326, 2, 7, (1, 4), 3, 24, 28.0), (299, 3, 8, (1, 2), 3, 12, 48.0), (318, 2, 7, (1, 4), 7, 28, 42.0),
+])
+def test_stage_operator_with_a_count_that_is_no_power_of_two(seed, base, layers, mesh, G, batch, capacity):
+    from mist_amd.batched_module_analyzer import batched_tune_best_latency_for_stage as on_gpu
+    from oracle.stage import batched_tune_best_latency_for_stage as on_cpu
+
+    cfg, tables = _plan(seed, base, layers, mesh, batch, capacity)
+    shape = (range(2), range(1, layers + 1), range(layers + 1), *mesh, G)
+    for samples in (1, 30):
+        got = on_gpu(tables, None, None, *shape, cfg, tp_size=1, sample_size=samples)
+        want = on_cpu(tables, cfg, *map(list, shape[:3]), *mesh, G, tp_size=1, sample_size=samples, inner="c")
+        for v in range(4):
+            for i in range(3):
+                assert_same_f64(got[v][i], want[v][i], f"{samples} samples, result {i} of table {v}")
