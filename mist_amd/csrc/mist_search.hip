@@ -1439,7 +1439,6 @@ __device__ __forceinline__ int count_exact(const Scaled &scaled, int count, doub
 struct GroupModel {
   GroupConsts k;
   double cap, G64, inv_G64;
-  double inv_G_down, inv_G_up;  // 1 / G, kShareSlack short and long
   float G32, inv_G32;
   double pre_saved, pre_sas, pre_states, post_states, post_fwd_peak, post_bwd_peak, post_output;
   bool pow2;  // x / G == x * (1 / G) bit for bit, and the division leaves the inner loop
@@ -1450,7 +1449,7 @@ struct GroupModel {
   // At most d / G, and r * lower_x(x) + lower_share(d) at most the base objective of a row, by the
   // slacks.  Monotone in x and d, so that of a stage's pseudo row bounds its rows' from below.
   __device__ __forceinline__ double lower_share(float d) const {
-    return (double)d * (d < 0.0f ? inv_G_up : inv_G_down);
+    return (double)d * inv_G64 * (d < 0.0f ? 1.0 + kShareSlack : 1.0 - kShareSlack);
   }
   __device__ __forceinline__ double lower_x(float x) const { return (double)x * (1.0 - kSlack); }
   __device__ __forceinline__ double bound(double ratio, float x, float d) const {
@@ -1465,8 +1464,6 @@ __device__ __forceinline__ GroupModel group_model(const MistProblem &prob, const
   m.G32 = (float)g->grad_accum;
   m.inv_G64 = 1.0 / m.G64;
   m.inv_G32 = 1.0f / m.G32;
-  m.inv_G_down = m.inv_G64 * (1.0 - kShareSlack);
-  m.inv_G_up = m.inv_G64 * (1.0 + kShareSlack);
   m.pre_saved = g->pre_saved;
   m.pre_sas = g->pre_states_and_saved;
   m.pre_states = g->pre_states;
