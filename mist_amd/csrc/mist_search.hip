@@ -1227,6 +1227,8 @@ constexpr int kStageRowsBlocks = 1024;       // four per CU, two stages at a tim
 constexpr int kSuperBlocks = 64;             // workgroups per group of the second-level summaries
 constexpr int kSeedLdsBytes = 40 * 1024;     // LDS aimed at per seed workgroup: four per CU
 constexpr int kSeedLdsMost = 160 * 1024;
+// Minima of one pair that every wavefront of a reduce workgroup can hold in LDS: 2559 values of p.
+constexpr int kMostBufferedSlots = kSeedLdsMost / (8 * (kReduceThreads / 64));
 static_assert(kQueueShards == 64, "a lane per shard");
 constexpr uint32_t kUnresolved = 0x80000000u;
 // Room below r x and below the terms the composite objectives add (their roundings: a few 1e-16) ...
@@ -1698,6 +1700,17 @@ __global__ __launch_bounds__(kSeedThreads) void seed_kernel(
   if ((int)threadIdx.x < pair_split) tabs.changed[(cell0 + threadIdx.x * n_slots) / 4] = 0;
 }
 
+// No seeds (the minima of one pair exceed the LDS): the tables of the launch, empty.
+__global__ __launch_bounds__(256) void empty_minima_kernel(ReduceTables tabs, int64_t cells) {
+  clear_queue(tabs);
+  const int64_t first = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, step = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = first; i < cells * tabs.n_samples; i += step) {
+    tabs.best[i] = INFINITY;
+    tabs.row[i] = ~0u;
+  }
+  for (int64_t i = first; i < cells / 4; i += step) tabs.changed[i] = 0;
+}
+
 // Several samples.  What the objectives of a row are made of, r X + Y per variant, and its counts,
 // for the lane = (row parity, sample) phases: a wavefront reads two rows at a time.
 struct SampleRows {
@@ -1705,6 +1718,9 @@ struct SampleRows {
   uint32_t counts[64];  // feasible p: base | with_pre << 15 | with_post << 30 | no_pp << 31
   uint32_t number[64];  // row number
 };
+// (counts of two words cost 30 samples of 7B on 1x8 5 %; calls with more values of p take their
+// samples one by one)
+constexpr int kMostCountedP = 0x7fff;
 static_assert(MIST_MAX_SAMPLE_BATCH <= 32, "half a wavefront per row");
 // Writes row `at` of the buffer.
 __device__ __forceinline__ void put_sample_row(SampleRows *rows, int at, const RowRegs &t, float x32, float d32, bool no_ck,
@@ -2135,7 +2151,8 @@ __global__ __launch_bounds__(kTermsBlock) void stage_rows_kernel(
 // One item with the pairs in `pairs`, one sample.  Returns the pairs in which some row reached its
 // minimum (kResolve: unused).  `lds_row`: the wavefront's buffer for the minima of one pair, which
 // the rows look up at their own counts; the next pair's are on their way in registers meanwhile.
-template <bool kResolve>
+// kInLds false: there are too many for it (see kMostBufferedSlots), rows look them up in memory.
+template <bool kResolve, bool kInLds>
 __device__ __forceinline__ uint64_t reduce_item(const MistProblem &prob, const MistGroupDesc *__restrict__ g, int gi,
                                                 int tile_rel, int stage, const double *__restrict__ row_terms,
                                                 const double *__restrict__ stage_floor, double ratio,
@@ -2181,11 +2198,13 @@ __device__ __forceinline__ uint64_t reduce_item(const MistProblem &prob, const M
   // minima of one pair, a slot per lane and register
   double ahead0 = 0.0, ahead1 = 0.0;
   auto fetch = [&](int pair) {
+    if (!kInLds) return;
     const double *slots = best + pair * n_slots;
     ahead0 = slots[min(lane, n_slots - 1)];
     if (n_slots > 64) ahead1 = slots[min(lane + 64, n_slots - 1)];
   };
   auto settle = [&](int pair) {
+    if (!kInLds) return;
     __builtin_amdgcn_wave_barrier();
     if (lane < n_slots) lds_row[lane] = ahead0;
     if (lane + 64 < n_slots) lds_row[lane + 64] = ahead1;
@@ -2215,8 +2234,9 @@ __device__ __forceinline__ uint64_t reduce_item(const MistProblem &prob, const M
     // these pay for the exact tests.  (A lowered slot may lie below the slots under it; a row above
     // it is above the winner of its own slot too, which finalize takes from the slots at and above.)
     const UpperCounts upper = upper_counts(mem, m, in ? np : 0);
+    auto minimum = [&](int slot) { return kInLds ? lds_row[slot] : best[(int64_t)pl * n_slots + slot]; };
     auto may = [&](int count, double cost, int slot) {
-      return in && count > 0 && cost <= cutoff && cost < INFINITY && cost <= lds_row[slot + max(count - 1, 0)];
+      return in && count > 0 && cost <= cutoff && cost < INFINITY && cost <= minimum(slot + max(count - 1, 0));
     };
     const bool may_b = may(upper.b, o.base, 0), may_p = may(upper.p, o.pre, P);
     const bool may_post = do_post && may(1, o.post, 2 * P), may_pp = do_pp && may(1, o.pp, 2 * P + 1);
@@ -2229,7 +2249,7 @@ __device__ __forceinline__ uint64_t reduce_item(const MistProblem &prob, const M
     // rows with `count` > 0 against the minimum of slot `slot` + count - 1
     auto offer = [&](int count, double cost, int slot) {
       const int own = slot + max(count - 1, 0);
-      const double now = in && count > 0 && cost <= cutoff && cost < INFINITY ? lds_row[own] : -INFINITY;
+      const double now = in && count > 0 && cost <= cutoff && cost < INFINITY ? minimum(own) : -INFINITY;
       if (!kResolve && cost < now) {
         lower_minimum(tabs.best + cell + own, cost);
         lowered = true;
@@ -2389,7 +2409,7 @@ __device__ __forceinline__ uint64_t every_pair(int k) {
 // on 4x8, whole items handed out in turn: 0.53 ms at one wavefront per SIMD on average).  The list
 // is in tile order; each XCD draws from its eighth of it, then from the next ones', and the next
 // draw is on its way while a unit is worked on.
-template <bool kResolve, bool kSamples>
+template <bool kResolve, bool kSamples, bool kInLds>
 __global__ __launch_bounds__(kReduceThreads, 3) void reduce_kernel(
     const MistProblem prob, const MistGroupDesc *__restrict__ groups, const double *__restrict__ row_terms,
     const double *__restrict__ stage_floor, const RatioList ratios, const ReduceTables tabs, int row_pitch) {
@@ -2406,8 +2426,8 @@ __global__ __launch_bounds__(kReduceThreads, 3) void reduce_kernel(
       hit = reduce_item_samples<kResolve>(prob, g, gi, tile_rel, stage, row_terms, stage_floor, ratios, tabs, pairs,
                                           &lds_samples[local_wave]);
     } else
-      hit = reduce_item<kResolve>(prob, g, gi, tile_rel, stage, row_terms, stage_floor, ratios.r[0], tabs, pairs,
-                                  lds_rows + local_wave * row_pitch);
+      hit = reduce_item<kResolve, kInLds>(prob, g, gi, tile_rel, stage, row_terms, stage_floor, ratios.r[0], tabs,
+                                          pairs, lds_rows + local_wave * row_pitch);
     if (!kResolve && hit != 0 && lane == 0) atomicOr(tabs.hit + at, (unsigned long long)hit);
   };
   constexpr bool kListed = kResolve && kSamples;
@@ -3361,6 +3381,11 @@ static int launch_first_estimate(const MistProblem *problem, const MistGroupDesc
   return 0;
 }
 
+// Samples of a batch that one set of launches takes (see kMostCountedP).
+static int samples_together(const MistProblem *problem, int n_samples) {
+  return problem->reduce_max_p > kMostCountedP ? 1 : n_samples;
+}
+
 // More than 64 KB of LDS per workgroup needs an opt-in, once per device.
 static int allow_large_lds() {
   static std::mutex lock;
@@ -3372,8 +3397,8 @@ static int allow_large_lds() {
   if (!done[device]) {
     for (const void *kernel : {reinterpret_cast<const void *>(seed_kernel),
                                reinterpret_cast<const void *>(seed_samples_kernel),
-                               reinterpret_cast<const void *>(reduce_kernel<false, false>),
-                               reinterpret_cast<const void *>(reduce_kernel<true, false>)})
+                               reinterpret_cast<const void *>(reduce_kernel<false, false, true>),
+                               reinterpret_cast<const void *>(reduce_kernel<true, false, true>)})
       MIST_HIP_CHECK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kSeedLdsMost));
     done[device] = true;
   }
@@ -3401,7 +3426,12 @@ static int launch_seeds(const MistProblem *problem, const MistGroupDesc *d_group
   while (sample_split > 1 && pair_bytes * sample_split > kSeedLdsBytes) sample_split = (sample_split + 1) / 2;
   const int64_t bytes =
       pair_bytes * pair_split * sample_split + (tabs.n_samples == 1 ? 0 : (int64_t)sizeof(SampleRows));
-  if (bytes > kSeedLdsMost) return fail(MIST_E_INVALID, "%d pre-saved micro-batch values exceed the LDS", problem->reduce_max_p);
+  if (bytes > kSeedLdsMost) {  // some 10000 values of p
+    hipLaunchKernelGGL(empty_minima_kernel, dim3(kReduceBlocks), dim3(256), 0, (hipStream_t)stream, tabs,
+                       problem->reduce_cells);
+    MIST_HIP_CHECK(hipGetLastError());
+    return 0;
+  }
   if (bytes > 64 * 1024)
     if (int rc = allow_large_lds()) return rc;
   const dim3 grid(tiles * (MIST_LC_TILE / pair_split), n_groups,
@@ -3445,17 +3475,17 @@ static int launch_reduce(const MistProblem *problem, const MistGroupDesc *d_grou
                        d_groups, const_cast<double *>(d_row_terms), d_key_terms, tabs);
     MIST_HIP_CHECK(hipGetLastError());
   }
-  const int row_pitch = slots_of(problem->reduce_max_p);
-  const size_t lds = tabs.n_samples == 1 ? sizeof(double) * row_pitch * (kReduceThreads / 64) : 0;
-  if (lds > kSeedLdsMost) return fail(MIST_E_INVALID, "%d pre-saved micro-batch values exceed the LDS", problem->reduce_max_p);
+  const bool one = tabs.n_samples == 1, buffered = one && slots_of(problem->reduce_max_p) <= kMostBufferedSlots;
+  const int row_pitch = buffered ? slots_of(problem->reduce_max_p) : 0;
+  const size_t lds = sizeof(double) * row_pitch * (kReduceThreads / 64);
   if (lds > 64 * 1024)
     if (int rc = allow_large_lds()) return rc;
-#define MIST_REDUCE(RESOLVE, SAMPLES)                                                                       \
-  hipLaunchKernelGGL((reduce_kernel<RESOLVE, SAMPLES>), dim3(kReduceBlocks), dim3(kReduceThreads), lds,     \
+#define MIST_REDUCE(RESOLVE, SAMPLES, IN_LDS)                                                               \
+  hipLaunchKernelGGL((reduce_kernel<RESOLVE, SAMPLES, IN_LDS>), dim3(kReduceBlocks), dim3(kReduceThreads), lds, \
                      (hipStream_t)stream, *problem, d_groups, d_row_terms, d_stage_floor, ratios, tabs, row_pitch)
-  const bool one = tabs.n_samples == 1;
-  if (one) MIST_REDUCE(false, false);
-  else MIST_REDUCE(false, true);
+  if (!one) MIST_REDUCE(false, true, false);
+  else if (buffered) MIST_REDUCE(false, false, true);
+  else MIST_REDUCE(false, false, false);
   MIST_HIP_CHECK(hipGetLastError());
   // (with one sample the list costs what it saves, 15 us of 1.3B on 1x2, and 70B on 32x8 gains 0.06 ms)
   if (!one) {
@@ -3463,8 +3493,9 @@ static int launch_reduce(const MistProblem *problem, const MistGroupDesc *d_grou
                        d_groups, tabs);
     MIST_HIP_CHECK(hipGetLastError());
   }
-  if (one) MIST_REDUCE(true, false);
-  else MIST_REDUCE(true, true);
+  if (!one) MIST_REDUCE(true, true, false);
+  else if (buffered) MIST_REDUCE(true, false, true);
+  else MIST_REDUCE(true, false, false);
 #undef MIST_REDUCE
   MIST_HIP_CHECK(hipGetLastError());
   return 0;
@@ -3570,20 +3601,26 @@ int mist_eval_reduce_samples(const MistProblem *problem, const MistGroupDesc *d_
                 MIST_MAX_SAMPLE_BATCH);
   if (main_batch < 1 || main_batch > n_samples)
     return fail(MIST_E_INVALID, "main_batch %d outside [1, n_samples = %d]", main_batch, n_samples);
-  RatioList all = {};
-  for (int i = 0; i < n_samples; ++i) {
+  for (int i = 0; i < n_samples; ++i)
     if (!(ratios[i] >= 0.0)) return fail(MIST_E_INVALID, "ratio %d must be non-negative", i);
-    all.r[i] = ratios[i];
+  const int batch = samples_together(problem, n_samples);
+  for (int first = 0; first < n_samples; first += batch) {
+    const int count = std::min(batch, n_samples - first);
+    RatioList list = {};
+    for (int i = 0; i < count; ++i) list.r[i] = ratios[first + i];
+    ReduceTables tabs;
+    if (int rc = reduce_tables(problem, count, d_partial_cost, d_partial_index, &tabs)) return rc;
+    if (int rc = launch_seeds(problem, d_groups, n_groups, d_row_terms, list, n_scout_blocks > 0, tabs, d_partial_cost,
+                              stream))
+      return rc;
+    if (int rc = launch_super_floors(d_groups, n_groups, d_stage_floor, tabs, stream)) return rc;
+    if (int rc = launch_reduce(problem, d_groups, n_groups, d_block_prefix, n_blocks, d_row_terms, d_stage_floor, nullptr,
+                               list, tabs, stream))
+      return rc;
+    if (int rc = launch_finalize(problem, d_groups, n_groups, d_row_terms, tabs, sample_index + first, tables, stream))
+      return rc;
   }
-  ReduceTables tabs;
-  if (int rc = reduce_tables(problem, n_samples, d_partial_cost, d_partial_index, &tabs)) return rc;
-  if (int rc = launch_seeds(problem, d_groups, n_groups, d_row_terms, all, n_scout_blocks > 0, tabs, d_partial_cost, stream))
-    return rc;
-  if (int rc = launch_super_floors(d_groups, n_groups, d_stage_floor, tabs, stream)) return rc;
-  if (int rc = launch_reduce(problem, d_groups, n_groups, d_block_prefix, n_blocks, d_row_terms, d_stage_floor, nullptr, all,
-                             tabs, stream))
-    return rc;
-  return launch_finalize(problem, d_groups, n_groups, d_row_terms, tabs, sample_index, tables, stream);
+  return 0;
 }
 
 int mist_eval_reduce_exhaustive(const MistProblem *problem, const MistGroupDesc *d_groups,
@@ -3708,8 +3745,9 @@ int mist_intra_stage_eval_samples(const MistProblem *problem, const MistGroupDes
                                 d_row_terms, d_stage_floor, d_key_terms, stream))
       return rc;
   }
-  for (int first = 0; first < n_samples; first += sample_batch) {
-    const int count = std::min(sample_batch, n_samples - first);
+  const int batch = samples_together(problem, sample_batch);
+  for (int first = 0; first < n_samples; first += batch) {
+    const int count = std::min(batch, n_samples - first);
     ReduceTables tabs;
     if (int rc = reduce_tables(problem, count, d_partial_cost, d_partial_index, &tabs, !by_need)) return rc;
     RatioList list = {};

@@ -1,7 +1,8 @@
 """The pruned reduction against the kernel that evaluates every cell, at the edges of its tiles."""
+import numpy as np
 import pytest
 
-from tests.util import tiny_plan
+from tests.util import assert_same_f64, tiny_plan
 
 pytestmark = pytest.mark.gpu
 
@@ -38,3 +39,28 @@ def test_pruned_tables_equal_every_cell_evaluated(layers, nodes, gpus, batch, sa
             assert torch.equal(a, b), f"{kind} of variant {v}: {int((a != b).sum())} of {a.numel()} differ"
         finite += int(torch.isfinite(want.device.stable[v]).sum())
     assert finite > 0
+
+
+@pytest.mark.parametrize("n_p, capacity, samples", [
+    (2559, 90.0, 1), (2560, 90.0, 1),         # the minima of a pair in every wavefront's LDS, and not
+    (10400, 300.0, 1), (10400, 300.0, 2),     # more than a workgroup's LDS: no seeds
+    (36000, 1345.0, 1), (36000, 1345.0, 2),   # counts of more than 15 bits
+])
+def test_many_pre_saved_micro_batch_values(n_p, capacity, samples):
+    """The stage operator takes the values of p from its caller."""
+    from mist_amd.batched_module_analyzer import batched_tune_best_latency_for_stage as on_gpu
+    from oracle.stage import batched_tune_best_latency_for_stage as on_cpu
+
+    grid = [0.0, 0.5, 1.0]
+    cfg, tables = tiny_plan(2, layers=2, hardware__num_nodes=1, hardware__num_gpus_per_node=2,
+                            training__global_batch_size=16, hardware__memory_capacity=capacity,
+                            tuning__search_space__offloading_ratio_candidates=grid,
+                            tuning__search_space__sparse_offloading_ratio_candidates=grid)
+    shape = (range(n_p), range(1, 3), range(3), 1, 2, 8)
+    got = on_gpu(tables, None, None, *shape, cfg, tp_size=1, sample_size=samples)
+    want = on_cpu(tables, cfg, *map(list, shape[:3]), *shape[3:], tp_size=1, sample_size=samples, inner="c")
+    last = np.isfinite(want[0][0]).reshape(n_p, -1).any(axis=1).nonzero()[0].max()
+    assert last > 0.6 * n_p, last
+    for v in range(4):
+        for i in range(3):
+            assert_same_f64(got[v][i], want[v][i], f"result {i} of table {v}")
