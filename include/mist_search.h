@@ -249,7 +249,7 @@ int mist_row_terms(const MistProblem *problem, const MistGroupDesc *d_groups, in
  * n_lc_tiles*n_p_tiles*n_chunks workgroups ordered (chunk, lc_tile, p_tile), p_tile fastest.
  * d_scout_prefix[n_groups+1]: n_lc_tiles*n_p_tiles*mist_reduce_scout_split() per group.
  * d_partial_cost: mist_reduce_workspace_doubles(reduce_cells, .., 1) doubles (any contents on
- * entry), d_partial_index: reduce_cells int32.  At most 65535 groups and 65535 tiles of the (l, c)
+ * entry), d_partial_index: reduce_cells int32.  At most 65535 groups and 2^23 tiles of the (l, c)
  * list. */
 int mist_eval_reduce(const MistProblem *problem, const MistGroupDesc *d_groups, int n_groups,
                      const int32_t *d_block_prefix, int n_blocks,

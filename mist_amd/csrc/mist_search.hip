@@ -1238,6 +1238,24 @@ constexpr double kSlack = 1e-9;
 // smaller than what was rounded.
 constexpr double kShareSlack = 1e-7;
 
+// A (group, tile, stage) of the queues in one word: 65535 groups, stages of fewer than 2^31 rows, and
+// the rest for the tiles of the pair list (32765 layers).
+constexpr int kItemStageBits = 25, kItemTileBits = 23;
+static_assert((((int64_t)1 << 31) + kStageRows - 1) / kStageRows <= (int64_t)1 << kItemStageBits, "stages of a group");
+struct Item {
+  int group, tile, stage;
+  __device__ __forceinline__ explicit Item(uint64_t word)
+      : group((int)(word >> (kItemTileBits + kItemStageBits))),
+        tile((int)(word >> kItemStageBits & ((1u << kItemTileBits) - 1u))),
+        stage((int)(word & ((1u << kItemStageBits) - 1u))) {}
+  __device__ __forceinline__ Item(int its_group, int its_tile, int its_stage)
+      : group(its_group), tile(its_tile), stage(its_stage) {}
+  __device__ __forceinline__ unsigned long long word() const {
+    return (unsigned long long)group << (kItemTileBits + kItemStageBits) | (unsigned long long)tile << kItemStageBits |
+           (unsigned long long)stage;
+  }
+};
+
 // (by value in the kernel arguments)
 struct ReduceTables {
   double *best;  // [pair][slot][sample] (slots_of(num_p) slots): the smallest cost
@@ -1246,8 +1264,8 @@ struct ReduceTables {
   uint32_t *row;
   uint32_t *changed;         // [pair's first cell / 4]: samples whose minima the reduce launch lowered
   double *super_floor;       // [supers][kStageFloorPitch]
-  // [kQueueShards][capacity]: group << 48 | tile << 32 | stage, what the filter and then what the
-  // open launch left; pairs of the latter in which a row reached its minimum
+  // [kQueueShards][capacity]: Item, what the filter and then what the open launch left; pairs of the
+  // latter in which a row reached its minimum
   unsigned long long *item, *opened, *hit;
   // [kQueueShards][capacity]: group << 32 | stage of the stages opened, each once; stage_flag (one
   // per stage summary) tells whether one is listed.  Null: the rows of all stages are there.
@@ -1987,8 +2005,7 @@ __global__ __launch_bounds__(MIST_LC_TILE) void filter_kernel(
       for (uint32_t rest = open; rest != 0; rest &= rest - 1, ++at) {
         if (at < done || at >= done + room) continue;
         const int st = st0 + __ffs(rest) - 1;
-        tabs.item[(int64_t)shard * tabs.capacity + base + (at - done)] =
-            (unsigned long long)gi << 48 | (unsigned long long)tile_rel << 32 | (uint32_t)st;
+        tabs.item[(int64_t)shard * tabs.capacity + base + (at - done)] = Item(gi, tile_rel, st).word();
       }
       done += room;
     }
@@ -2074,8 +2091,9 @@ __global__ __launch_bounds__(kReduceThreads) void open_kernel(const MistProblem 
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * kWaves + (threadIdx.x >> 6)));
   for (uint32_t i = wave; i < queue.total; i += gridDim.x * kWaves) {
     const int64_t from = queue.at(i, tabs.capacity);
-    const uint64_t item = from_lane((uint64_t)tabs.item[from], 0);
-    const int gi = (int)(item >> 48), tile_rel = (int)(item >> 32 & 0xffff), stage = (int)(uint32_t)item;
+    const uint64_t word = from_lane((uint64_t)tabs.item[from], 0);
+    const Item item(word);
+    const int gi = item.group, tile_rel = item.tile, stage = item.stage;
     const MistGroupDesc *g = groups + gi;
     const TileLane p = tile_lane(prob, g, tile_rel);
     const GroupModel m = group_model(prob, g);
@@ -2094,7 +2112,7 @@ __global__ __launch_bounds__(kReduceThreads) void open_kernel(const MistProblem 
     if (lane == 0) {
       // (no more than the shard's items are opened: it cannot overflow)
       const uint32_t to = atomicAdd(tabs.counter + (kQueueShards + shard) * kCounterPitch, 1u);
-      tabs.opened[(int64_t)shard * tabs.capacity + to] = item;
+      tabs.opened[(int64_t)shard * tabs.capacity + to] = word;
       tabs.hit[(int64_t)shard * tabs.capacity + to] = 0;
       if (tabs.listed != nullptr && atomicExch(tabs.stage_flag + stage_floor_slot(g, gi, stage), 1u) == 0) {
         const uint32_t row_to = atomicAdd(tabs.counter + (2 * kQueueShards + shard) * kCounterPitch, 1u);
@@ -2417,8 +2435,9 @@ __global__ __launch_bounds__(kReduceThreads, 3) void reduce_kernel(
   constexpr int kWaves = kReduceThreads / 64;
   const int local_wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
   const uint32_t n_waves = gridDim.x * kWaves;
-  auto work = [&](int64_t at, uint64_t item, uint64_t pairs) {
-    const int gi = (int)(item >> 48), tile_rel = (int)(item >> 32 & 0xffff), stage = (int)(uint32_t)item;
+  auto work = [&](int64_t at, uint64_t word, uint64_t pairs) {
+    const Item item(word);
+    const int gi = item.group, tile_rel = item.tile, stage = item.stage;
     const MistGroupDesc *g = groups + gi;
     uint64_t hit;
     if constexpr (kSamples) {
@@ -2441,14 +2460,15 @@ __global__ __launch_bounds__(kReduceThreads, 3) void reduce_kernel(
       if (kListed) at = (int64_t)from_lane((uint64_t)tabs.item[at], 0);
       uint64_t pairs = from_lane((uint64_t)tabs.hit[at], 0) & (every_pair(split) << (u & ((1u << split) - 1u)));
       if (pairs == 0) continue;
-      const uint64_t item = from_lane((uint64_t)tabs.opened[at], 0);
+      const uint64_t word = from_lane((uint64_t)tabs.opened[at], 0);
       if (!kListed) {  // pairs whose minima changed
-        const MistGroupDesc *g = groups + (item >> 48);
-        const int64_t tile_cell = g->cell_offset + (int64_t)(item >> 32 & 0xffff) * MIST_LC_TILE * slots_of(g->num_p);
+        const Item item(word);
+        const MistGroupDesc *g = groups + item.group;
+        const int64_t tile_cell = g->cell_offset + (int64_t)item.tile * MIST_LC_TILE * slots_of(g->num_p);
         pairs &= __ballot(tabs.changed[(tile_cell + lane * slots_of(g->num_p)) / 4] != 0);
         if (pairs == 0) continue;
       }
-      work(at, item, pairs);
+      work(at, word, pairs);
     }
     return;
   }
@@ -2493,10 +2513,10 @@ __global__ __launch_bounds__(kReduceThreads) void resolve_list_kernel(const Mist
     const int64_t at = first + min(lane, n_here - 1);
     uint64_t left = lane < n_here ? tabs.hit[at] : 0, mine = 0;
     if (!__any(left != 0)) continue;
-    const uint64_t item = tabs.opened[at];
-    const MistGroupDesc *g = groups + (item >> 48);
+    const Item item((uint64_t)tabs.opened[at]);
+    const MistGroupDesc *g = groups + item.group;
     const int n_slots = slots_of(g->num_p);
-    const int64_t cell0 = g->cell_offset + (int64_t)(item >> 32 & 0xffff) * MIST_LC_TILE * n_slots;
+    const int64_t cell0 = g->cell_offset + (int64_t)item.tile * MIST_LC_TILE * n_slots;
     for (; left != 0; left &= left - 1) {
       const int pair = __ffsll((unsigned long long)left) - 1;
       if (tabs.changed[(cell0 + pair * n_slots) / 4] != 0) mine |= 1ull << pair;
@@ -3417,7 +3437,8 @@ static int launch_seeds(const MistProblem *problem, const MistGroupDesc *d_group
       return rc;
   const int L = problem->num_layers, n_pairs = L * (L + 1) / 2 + L;
   const int tiles = (n_pairs + MIST_LC_TILE - 1) / MIST_LC_TILE;
-  if (tiles > 65535) return fail(MIST_E_INVALID, "at most 65535 tiles of (l, c) pairs, got %d", tiles);
+  if (tiles > 1 << kItemTileBits)
+    return fail(MIST_E_INVALID, "at most %d tiles of (l, c) pairs, got %d", 1 << kItemTileBits, tiles);
   const int64_t pair_bytes = 8 * (int64_t)slots_of(problem->reduce_max_p);
   // fewer pairs, or samples, per workgroup when the slots are many, so that several stay resident
   int pair_split = tabs.n_samples == 1 ? 16 : 1;

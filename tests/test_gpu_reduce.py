@@ -64,3 +64,24 @@ def test_many_pre_saved_micro_batch_values(n_p, capacity, samples):
     for v in range(4):
         for i in range(3):
             assert_same_f64(got[v][i], want[v][i], f"result {i} of table {v}")
+
+
+def test_more_than_65535_tiles_of_pairs():
+    """2900 layers: 4.2e6 (l, c) pairs."""
+    import torch
+
+    from mist_amd.intra_tuning import IntraStageTuner
+
+    layers = 2900
+    cfg, tables = tiny_plan(2, layers=layers, hardware__num_nodes=1, hardware__num_gpus_per_node=2,
+                            training__global_batch_size=4, hardware__memory_capacity=1500.0,
+                            tuning__search_space__offloading_ratio_candidates=[0.0, 1.0],
+                            tuning__search_space__sparse_offloading_ratio_candidates=[0.0, 1.0])
+    got, want = [IntraStageTuner(tables, layers, [(1, 2)], [2], 1, cfg, sample_size=1, exhaustive=exhaustive).tune()
+                 for exhaustive in (False, True)]
+    for v in range(4):
+        for kind in ("index", "stable", "delta"):
+            a, b = getattr(got.device, kind)[v], getattr(want.device, kind)[v]
+            assert torch.equal(a, b), f"{kind} of variant {v}: {int((a != b).sum())} of {a.numel()} differ"
+    assert 0 < int(torch.isfinite(want.device.stable[0]).sum()) < want.device.stable[0].numel()
+    assert bool(torch.isfinite(want.device.stable[0][0, 0, 0, 2890]).any())
