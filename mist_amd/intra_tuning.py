@@ -47,9 +47,20 @@ SCOUT_TIGHT_PAIRS = 3
 # the rows that the search opens are written, and a launch per plan keeps the GPU fuller than ten
 # of them: GPT-22B (18.4 GB) as nine batches of 2 GB takes 23.4 ms, as one 19.9 ms.
 ROW_TERMS_BUDGET_BYTES = 24 << 30
+# ... or this share of the memory that is free, where that is less, down to the second bound.
+ROW_TERMS_FREE_SHARE = 0.25
+ROW_TERMS_LEAST_BYTES = 2 << 30
 # Minima tables (12 bytes per (l, c) pair, variant, p and sample) the launches of a multi-sample call
 # may hold: more samples go through them in batches.
 MINIMA_BYTES = 8 << 30
+
+
+def _free_device_bytes(device: torch.device) -> Optional[int]:
+    """Memory an allocation can still get: free on the GPU, or held by torch and not in use."""
+    if device.type != "cuda" or not torch.cuda.is_available():
+        return None
+    return (torch.cuda.mem_get_info(device)[0] + torch.cuda.memory_reserved(device)
+            - torch.cuda.memory_allocated(device))
 
 
 _SIDE_STREAMS: Dict[str, "torch.cuda.Stream"] = {}
@@ -320,14 +331,25 @@ class IntraStageTuner:
         otherwise and when ``MIST_PYTHON_PLAN_BUILDER`` is set; the two give the same bytes."""
         _lib.load()  # the tile sizes of the decomposition are the library's
         wanted = self._wanted_cells()
-        built = None
-        if not os.environ.get("MIST_PYTHON_PLAN_BUILDER"):
-            built = self._build_groups_native(wanted)
-        if built is None:
-            built = self._build_groups_python(wanted)
+        most, least = ROW_TERMS_BUDGET_BYTES, min(ROW_TERMS_BUDGET_BYTES, ROW_TERMS_LEAST_BYTES)
+        built = self._build_groups(wanted, most)
+        if int(built[0]["n_rows"].sum()) * 8 * _lib.ROW_TERMS > least:
+            free = _free_device_bytes(self.device)
+            budget = most if free is None else max(min(most, int(free * ROW_TERMS_FREE_SHARE)), least)
+            if budget < most:
+                built = self._build_groups(wanted, budget)
         plan = self._finish_plan(*built)
         plan["wanted"] = wanted
         return plan
+
+    def _build_groups(self, wanted: Optional[np.ndarray], budget_bytes: int):
+        """Groups and decomposition of the call, in batches of at most ``budget_bytes`` of row terms."""
+        built = None
+        if not os.environ.get("MIST_PYTHON_PLAN_BUILDER"):
+            built = self._build_groups_native(wanted, budget_bytes)
+        if built is None:
+            built = self._build_groups_python(wanted, budget_bytes)
+        return built
 
     def _wanted_cells(self) -> Optional[np.ndarray]:
         """``cells_wanted`` of every (G, mesh) as int32 ``[G][mesh][3]`` = (smallest layer count,
@@ -356,7 +378,7 @@ class IntraStageTuner:
             return None
         return l_min, l_max, int(p_count)
 
-    def _build_groups_native(self, wanted: Optional[np.ndarray] = None):
+    def _build_groups_native(self, wanted: Optional[np.ndarray] = None, budget_bytes: Optional[int] = None):
         """The groups of this call from ``mist_plan_groups``, or None when the plan is outside
         what it covers or fails one of its checks (the python builder then words the error)."""
         cfg, tables, L = self.config, self.layer_tables, self.num_layers
@@ -402,7 +424,7 @@ class IntraStageTuner:
         req.pp_mode = pp_mode
         req.scout_tight_fraction = SCOUT_TIGHT_FRACTION
         req.global_batch_size = cfg.training.global_batch_size
-        req.workspace_rows = max(ROW_TERMS_BUDGET_BYTES // (8 * _lib.ROW_TERMS), 1)
+        req.workspace_rows = self._workspace_rows(budget_bytes)
         req.model_heads, req.model_seq_len = cfg.model.num_attention_heads, cfg.training.max_sequence_length
         req.model_flash = bool(cfg.model.use_flash_attn)
         req.num_layers, req.max_pre_saved = L, self.max_possible_pre_saved_micro_batches
@@ -447,7 +469,7 @@ class IntraStageTuner:
         return (groups[:n], spaces, prefixes[0, :n + 1], prefixes[1, :n + 1], prefixes[2, :n + 1], bounds,
                 result.max_scout_rows, result.max_group_keys)
 
-    def _build_groups_python(self, wanted: Optional[np.ndarray] = None):
+    def _build_groups_python(self, wanted: Optional[np.ndarray] = None, budget_bytes: Optional[int] = None):
         cfg, L = self.config, self.num_layers
         Gs, Q = self.gradient_accumulation_steps_candidates, self.device_mesh_candidates
         P = self.max_possible_pre_saved_micro_batches
@@ -488,7 +510,7 @@ class IntraStageTuner:
         builder.fill_many(groups, pending)
         builder.validate(groups)
 
-        bounds = self._batch_bounds(groups["n_rows"]) if len(pending) else []
+        bounds = self._batch_bounds(groups["n_rows"], self._workspace_rows(budget_bytes)) if len(pending) else []
         max_scout_rows = max_group_keys = 0
         if len(pending):
             groups["lc_tile_begin"] = [w[0] for w in tile_window]
@@ -583,10 +605,14 @@ class IntraStageTuner:
         )
 
     @staticmethod
-    def _batch_bounds(n_rows) -> List[Tuple[int, int]]:
+    def _workspace_rows(budget_bytes: Optional[int]) -> int:
+        budget_bytes = ROW_TERMS_BUDGET_BYTES if budget_bytes is None else budget_bytes
+        return max(budget_bytes // (8 * _lib.ROW_TERMS), 1)
+
+    @staticmethod
+    def _batch_bounds(n_rows, budget_rows: int) -> List[Tuple[int, int]]:
         """Runs of consecutive groups whose rows fit the row-term workspace bound (a larger
         group is a run of its own)."""
-        budget_rows = max(ROW_TERMS_BUDGET_BYTES // (8 * _lib.ROW_TERMS), 1)
         bounds, first = [], 0
         while first < len(n_rows):
             last, rows = first, 0

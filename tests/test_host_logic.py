@@ -844,3 +844,33 @@ def test_inputs_outside_the_kernels_preconditions_are_rejected():
     tuner = IntraStageTuner(broken, 4, [(1, 1), (1, 2)], [1, 2, 4, 8], 1, cfg, sample_size=1)
     with pytest.raises(ValueError, match="non-negative"):
         tuner.prepare()
+
+
+@pytest.mark.parametrize("builder", ["library", "python"])
+def test_row_term_batches_follow_the_free_memory(builder, monkeypatch):
+    """GPT-22B's rows are 18.4 GB: one batch where memory is plenty, batches of a quarter of what
+    is free (two of them alternate) where it is not, 2 GB ones at the least; plans under 2 GB and
+    a CPU without a GPU do not ask."""
+    from mist_amd import intra_tuning
+
+    if builder == "python":
+        monkeypatch.setenv("MIST_PYTHON_PLAN_BUILDER", "1")
+    cfg, tables = load_plan(4)
+    hw = cfg.hardware
+    meshes = _get_device_mesh_candidates(hw.num_nodes, hw.num_gpus_per_node, False)
+    Gs = _get_grad_accumu_steps_candidates(cfg.training.global_batch_size)
+    tuner = IntraStageTuner(tables, cfg.model.num_hidden_layers, meshes, Gs, tp_candidates(cfg), cfg, sample_size=1)
+    row_bytes, gib = 8 * _lib.ROW_TERMS, 1 << 30
+    for free, most in ((None, 24), (280 * gib, 24), (40 * gib, 10), (20 * gib, 5), (3 * gib, 2)):
+        monkeypatch.setattr(intra_tuning, "_free_device_bytes", lambda device: free)
+        batches = tuner.prepare()["batches"]
+        assert (len(batches) == 1) == (most == 24)
+        assert all(b["total_rows"] * row_bytes <= most * gib for b in batches)
+        assert sum(b["total_rows"] for b in batches) * row_bytes > 17 * gib
+
+    def unexpected(device):
+        raise AssertionError("asked for the free memory")
+
+    monkeypatch.setattr(intra_tuning, "_free_device_bytes", unexpected)
+    small = load_plan(2)
+    assert len(IntraStageTuner(small[1], 32, [(1, 8), (4, 8)], [8, 16], 1, small[0], sample_size=1).prepare()["batches"]) == 1
