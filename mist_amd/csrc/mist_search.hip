@@ -1718,7 +1718,7 @@ __global__ __launch_bounds__(kSeedThreads) void seed_kernel(
   if ((int)threadIdx.x < pair_split) tabs.changed[(cell0 + threadIdx.x * n_slots) / 4] = 0;
 }
 
-// No seeds (the minima of one pair exceed the LDS): the tables of the launch, empty.
+// No seeds (none asked for, or the minima of one pair exceed the LDS): the tables of the launch, empty.
 __global__ __launch_bounds__(256) void empty_minima_kernel(ReduceTables tabs, int64_t cells) {
   clear_queue(tabs);
   const int64_t first = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, step = (int64_t)gridDim.x * blockDim.x;
@@ -3425,8 +3425,8 @@ static int allow_large_lds() {
   return 0;
 }
 
-// Minima tables filled with what the rows of the scout pairs give (+inf where a group has none),
-// and the estimate of the best pipeline cost they allow.
+// Minima tables filled with what the rows of the scout pairs give (+inf where a group has none and
+// with `scouted` false), and the estimate of the best pipeline cost they allow.
 static int launch_seeds(const MistProblem *problem, const MistGroupDesc *d_groups, int n_groups,
                         const double *d_row_terms, const RatioList &ratios, bool scouted,
                         const ReduceTables &tabs, double *d_partial_cost, void *stream) {
@@ -3447,7 +3447,7 @@ static int launch_seeds(const MistProblem *problem, const MistGroupDesc *d_group
   while (sample_split > 1 && pair_bytes * sample_split > kSeedLdsBytes) sample_split = (sample_split + 1) / 2;
   const int64_t bytes =
       pair_bytes * pair_split * sample_split + (tabs.n_samples == 1 ? 0 : (int64_t)sizeof(SampleRows));
-  if (bytes > kSeedLdsMost) {  // some 10000 values of p
+  if (!scouted || bytes > kSeedLdsMost) {  // (some 10000 values of p)
     hipLaunchKernelGGL(empty_minima_kernel, dim3(kReduceBlocks), dim3(256), 0, (hipStream_t)stream, tabs,
                        problem->reduce_cells);
     MIST_HIP_CHECK(hipGetLastError());
