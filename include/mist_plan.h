@@ -80,7 +80,7 @@ typedef struct MistPlanRequest {
   int32_t num_layers;            /* L */
   int32_t max_pre_saved;         /* P: largest number of pre-saved micro-batches (intra_tuning.py:117-126) */
   int32_t evaluate_all_p;        /* every p of 0..P for every G */
-  int32_t exhaustive;            /* the evaluate-every-cell kernel: no scout pass */
+  int32_t exhaustive;            /* the evaluate-every-cell kernel: no seeds */
   int32_t n_tp, tp_size[MIST_PLAN_MAX_LIST]; /* 0 = none given: the first feasible batch size decides */
   int32_t n_grad_accum, grad_accum[MIST_PLAN_MAX_LIST];
   int32_t n_mesh, mesh_n[MIST_MAX_MESH], mesh_m[MIST_MAX_MESH];
@@ -92,7 +92,7 @@ typedef struct MistPlanRequest {
   int32_t n_wo, n_go, n_oo, n_ao, n_pair;
   uint8_t pair_wo[MIST_MAX_PAIRS], pair_go[MIST_MAX_PAIRS];
   int32_t pp_mode;
-  /* sizing of the reduce launches and of the scout pass */
+  /* sizing of the filter launch and of the seeds */
   int32_t target_reduce_waves, scout_min_stages, scout_min_pairs, scout_pairs, scout_pair_span,
       scout_tight_pairs;
   /* optional [n_grad_accum][n_mesh][3] = (smallest layer count, largest layer count, number of
@@ -117,8 +117,9 @@ int mist_sizeof_plan_request(void);
  *   space_offset[entries+1], space_rows[entries * MIST_MAX_PAR][6]: the parallelism rows
  *     (b, dp, tp, wre, gre, ore) of every entry, also of those without a group
  *   group_of_entry[entries]: index into groups, -1 = none
- *   terms_prefix, reduce_prefix, scout_prefix [group_capacity+1]: first workgroup of each group
- *     in the row-term, reduce and scout launches
+ *   terms_prefix, reduce_prefix [group_capacity+1]: first workgroup of each group in the row-term
+ *     (summary) and filter launches; scout_prefix [group_capacity+1]: what mist_eval_reduce asks for,
+ *     all zero when no group has seeds
  *   batch_bounds[group_capacity+1]: first group of each batch, then n_groups
  * Returns 0, MIST_E_INVALID (bad sizes) or MIST_E_PLAN_UNSUPPORTED. */
 int mist_plan_groups(const MistPlanRequest *request, MistGroupDesc *groups, int32_t group_capacity,

@@ -28,12 +28,12 @@ extern "C" {
 #define MIST_ROW_TERMS 34   /* doubles per candidate row produced by mist_row_terms */
 #define MIST_KEY_TERMS 56   /* doubles per (parallelism row, activation ratio, offload pair) of the
                              * key-term workspace of mist_row_terms */
-#define MIST_LC_TILE 64     /* (layers, ckpt) pairs per workgroup (one wavefront) of the reduce kernel */
+#define MIST_LC_TILE 64     /* (layers, ckpt) pairs of a tile: one wavefront, lane = pair */
 #ifndef MIST_P_TILE
-#define MIST_P_TILE 16      /* pre-saved micro-batch values per thread of the reduce kernel */
+#define MIST_P_TILE 16      /* pre-saved micro-batch values per thread of the evaluate-every-cell kernel */
 #endif
 #define MIST_MAX_MESH 16    /* device-mesh candidates of the inter-stage DP */
-#define MIST_MAX_SCOUT_PAIRS 8 /* offload pairs whose rows the scout pass of a group gathers */
+#define MIST_MAX_SCOUT_PAIRS 8 /* offload pairs whose rows the scout pass (the seed launch) of a group gathers */
 #define MIST_MAX_SAMPLE_BATCH 32 /* alpha samples per mist_eval_reduce_samples call */
 
 #define MIST_E_INVALID (-1) /* argument / shape check failed, nothing was launched */
@@ -91,15 +91,15 @@ typedef struct MistProblem {
   int32_t num_mesh;        /* extent of the q axis */
   int32_t adv_first_block; /* enable_advanced_opt_in_first_block */
   int32_t max_scout_rows;  /* largest n_par * n_oo * n_ao * scout_stride of the call's groups with a
-                            * scout pass; 0 = unknown (mist_intra_stage_eval then runs the row
-                            * terms and the scout pass one after the other) */
+                            * scout pass; 0 = unknown (mist_intra_stage_eval then computes all row
+                            * terms first and the scout pass after them) */
   int32_t max_group_keys;  /* largest n_par * n_ao * n_pair of the call's groups; 0 = unknown
                             * (mist_row_terms then evaluates every row on its own) */
   /* Optional (NULL = none; sample_size 1 only, where a cell's objective is its stage cost): one
    * double in device memory, an estimate of the cost of the best pipeline the caller's
    * inter-stage search returns (+inf before the first call).  The scout pass lowers it to the
-   * cost of the best partition into equal stages on equal meshes that its seeds allow; the main
-   * launch (and the scout pass itself, with the value it finds) then does not look for stage
+   * cost of the best partition into equal stages on equal meshes that its seeds allow; the launches
+   * behind it (and the scout pass itself, with the value it finds) then do not look for stage
    * costs above
    *     bound(G) = incumbent / G * (1 + mist_incumbent_slack()).
    * A cell whose minimum is not above bound(G) holds its minimum and row as always; any other
@@ -191,10 +191,10 @@ double mist_incumbent_slack(void); /* see MistProblem.stage_cost_incumbent */
 int mist_sizeof_group(void);
 int mist_reduce_p_tile(void); /* MIST_P_TILE the library was built with */
 int mist_reduce_lc_tile(void); /* MIST_LC_TILE the library was built with */
-int mist_reduce_scout_split(void); /* scout workgroups per (group, (l, c) tile, p tile) */
+int mist_reduce_scout_split(void); /* 1: factor of d_scout_prefix (see mist_eval_reduce) */
 int mist_workspace_oo_tile(void);  /* optimizer-ratio tile T of the workspace order (mist_row_terms) */
 int mist_terms_block_rows(void); /* candidate rows per workgroup of mist_row_terms */
-int mist_reduce_stage_rows(void); /* rows per LDS stage; rows_per_chunk must be a multiple */
+int mist_reduce_stage_rows(void); /* rows per stage; rows_per_chunk must be a multiple */
 int mist_max_sample_batch(void); /* MIST_MAX_SAMPLE_BATCH the library was built with */
 int mist_key_terms_per_key(void); /* MIST_KEY_TERMS the library was built with */
 int mist_max_scout_pairs(void);  /* MIST_MAX_SCOUT_PAIRS the library was built with */
@@ -219,7 +219,7 @@ int64_t mist_reduce_workspace_doubles(int64_t cells, int64_t supers, int64_t ite
  *   position = (par * n_ao + ao) * n_oo * n_pair + t * T * n_pair + pair * w + oo % T
  * with T = mist_workspace_oo_tile(), t = oo / T and w = min(T, n_oo - t * T): per (par, ao) the
  * optimizer ratios in tiles of T, pair by pair inside a tile (rows of similar latency and memory
- * footprint next to each other, which the reduce kernel's per-stage bound relies on for speed,
+ * footprint next to each other, which the bounds per stage rely on for speed,
  * not for correctness); all results carry reference row numbers.
  * d_stage_floor: mist_stage_floor_doubles() float64, written here and read by mist_eval_reduce:
  * per stage of mist_reduce_stage_rows() workspace rows the term-wise minimum of the latency and
@@ -247,10 +247,13 @@ int mist_row_terms(const MistProblem *problem, const MistGroupDesc *d_groups, in
  * what is left, *resolve* finds the rows of the minima that were lowered meanwhile.
  * d_block_prefix[n_groups+1]: first workgroup of each group in the filter launch; a group owns
  * n_lc_tiles*n_p_tiles*n_chunks workgroups ordered (chunk, lc_tile, p_tile), p_tile fastest.
- * d_scout_prefix[n_groups+1]: n_lc_tiles*n_p_tiles*mist_reduce_scout_split() per group.
+ * n_scout_blocks > 0 asks for the seeds; d_scout_prefix[n_groups+1] (n_lc_tiles * n_p_tiles *
+ * mist_reduce_scout_split() per group, n_scout_blocks in all) must then be given, but no launch
+ * reads it: the seed launch takes its grid from the groups.
  * d_partial_cost: mist_reduce_workspace_doubles(reduce_cells, .., 1) doubles (any contents on
- * entry), d_partial_index: reduce_cells int32.  At most 65535 groups and 2^23 tiles of the (l, c)
- * list. */
+ * entry; memory of the GPU itself, as hipMalloc gives it: the minima are lowered by float64
+ * atomics), d_partial_index: reduce_cells int32.  At most 65535 groups and 2^23 tiles of the
+ * (l, c) list. */
 int mist_eval_reduce(const MistProblem *problem, const MistGroupDesc *d_groups, int n_groups,
                      const int32_t *d_block_prefix, int n_blocks,
                      const int32_t *d_scout_prefix, int n_scout_blocks,
@@ -278,6 +281,7 @@ int mist_stage_cost_first_estimate(const MistProblem *problem, const MistGroupDe
  * latency, memory and feasibility once for all of them (`main_batch`, 1 .. n_samples, is the
  * number of samples a caller of the launches one by one would take together; it is checked and
  * does not change anything here).  `ratios` and `sample_index` are HOST arrays.
+ * With more than 32767 values of p the samples are taken one by one.
  * d_partial_cost: mist_reduce_workspace_doubles(reduce_cells, .., n_samples) doubles,
  * d_partial_index: reduce_cells * n_samples int32. */
 int mist_eval_reduce_samples(const MistProblem *problem, const MistGroupDesc *d_groups,
@@ -290,8 +294,8 @@ int mist_eval_reduce_samples(const MistProblem *problem, const MistGroupDesc *d_
 
 /* mist_row_terms + mist_eval_reduce_samples for ALL n_samples ratios of a tuner call (any
  * number; batches of `sample_batch` <= MIST_MAX_SAMPLE_BATCH): the scout pass of the first batch
- * runs on the library's second stream beside the row terms of the rows it does
- * not gather.  Same tables as the calls it replaces (reference: the S samples of one
+ * runs on the library's second stream beside the key terms and the stage summaries.  Same
+ * tables as the calls it replaces (reference: the S samples of one
  * compute_indices call per group, mist/utils/pareto.py:124-144).  `ratios` and `sample_index` are
  * HOST arrays of n_samples.  Workspaces as for mist_eval_reduce_samples with `sample_batch`
  * samples.  Without a scout pass (n_scout_blocks == 0 or problem->max_scout_rows == 0) everything
@@ -308,11 +312,11 @@ int mist_intra_stage_eval_samples(const MistProblem *problem, const MistGroupDes
 
 /* mist_eval_reduce with every cell evaluated: each (row, layers, ckpt) through the latency and
  * memory model and each pre-saved micro-batch value through the reference's feasibility test
- * (batched_module_analyzer.py:2218-3106, pareto.py:124-144 as written, cell by cell), no scout
- * pass, no sieves.  Each of the n_blocks workgroups (decomposition as above) writes its minima to
+ * (batched_module_analyzer.py:2218-3106, pareto.py:124-144 as written, cell by cell), no seeds,
+ * no bounds.  Each of the n_blocks workgroups (decomposition as above) writes its minima to
  * a slab of [2*MIST_P_TILE+2][MIST_LC_TILE] entries behind the reduce_cells entries of the table,
  * which a second kernel combines into it.  The reference point the pruned search is tested and
- * measured against: identical tables, ~30x the time. */
+ * measured against: identical tables (GPT-7B: 59 ms). */
 int mist_eval_reduce_exhaustive(const MistProblem *problem, const MistGroupDesc *d_groups,
                                 int n_groups, const int32_t *d_block_prefix, int n_blocks,
                                 const double *d_row_terms, double ratio, double *d_partial_cost,

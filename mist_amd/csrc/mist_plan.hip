@@ -502,7 +502,7 @@ extern "C" int mist_plan_groups(const MistPlanRequest *request, MistGroupDesc *g
       reduce_prefix[i] = (int32_t)reduce;
       terms += (d->n_rows + kTermsBlock - 1) / kTermsBlock;
       reduce += (int64_t)d->n_chunks * n_lc_tiles[i] * p_tiles;
-      // Scout pass: the rows of a few (weight, gradient) offload pairs seed the group's chunks;
+      // Seeds: the rows of a few (weight, gradient) offload pairs give the group's first minima;
       // groups that are small or have few offload pairs go without.
       const int64_t n_stages = (d->n_rows + kStageRows - 1) / kStageRows;
       const bool scout = n_stages >= r.scout_min_stages && d->n_pair >= r.scout_min_pairs &&

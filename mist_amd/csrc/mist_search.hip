@@ -1,6 +1,6 @@
-// Intra-stage configuration search on MI355X (gfx950): row terms, fused evaluate+mask+argmin,
-// finalize.  Everything is float64 VALU work with float32 rounding points where the reference
-// has them; there is no dense contraction here, so no MFMA.
+// Intra-stage configuration search on MI355X (gfx950): row terms and stage summaries, the pruned
+// reduction to one table of minima, finalize.  Everything is float64 VALU work with float32
+// rounding points where the reference has them; there is no dense contraction here, so no MFMA.
 //
 // Bit-exactness rules for this file (results must equal the numpy formulation operation for
 // operation): compile with -ffp-contract=off, keep the operand order of every sum exactly as
@@ -39,11 +39,11 @@ namespace {
 using mist::fail;
 
 constexpr int kTermsBlock = 128;  // rows per workgroup of the row-term kernel
-constexpr int kStageRows = 64;    // rows staged through LDS per step of the reduce kernel
+constexpr int kStageRows = 64;    // rows of a stage: one summary, one item of the reduction
 constexpr int kSlots = 2 * MIST_P_TILE + 2;  // per-thread running minima: base, with_pre, post, no_pp
-constexpr int kScoutSplit = 1;    // (mist_reduce_scout_split)
+constexpr int kScoutSplit = 1;    // (mist_reduce_scout_split: workgroups of a decomposition no launch has any more)
 constexpr double kIncumbentSlack = 0.25;  // relative room above MistProblem.stage_cost_incumbent / G
-// Stage summaries (written with the row terms, read by the reduce kernel): per stage of
+// Stage summaries (written with or ahead of the row terms, read by filter, open and reduce): per stage of
 // kStageRows workspace rows the term-wise minimum of the latency and memory columns and the
 // maximum of MIST_T_OUT, kStageFloorPitch doubles per stage.
 constexpr int kStageFloorPitch = 32;
@@ -343,7 +343,7 @@ __device__ __forceinline__ const MistGroupDesc *find_group(const MistGroupDesc *
 // pair by pair:
 //   position = (par * n_ao + ao) * n_oo * n_pair + tile * kOoTile * n_pair + pair * width + oo % kOoTile
 // with tile = oo / kOoTile and width = ratios in that tile (kOoTile, fewer in the last one).  A
-// stage of the reduce kernel (64 consecutive positions) then covers 16 neighbouring (weight,
+// stage (64 consecutive positions) then covers 16 neighbouring (weight,
 // gradient) pairs at 4 neighbouring optimizer ratios: rows of similar latency AND footprint, so
 // the stage's term-wise minimum is close to a real row and its bounds prune.  (With all pairs of
 // one optimizer ratio in a run, a stage spanned half of the pair list: its minimum was as fast as
@@ -400,8 +400,8 @@ __device__ __forceinline__ int64_t position_of_row(const MistGroupDesc *g, int64
 // are the same for the n_oo rows of one "key" = (parallelism, activation ratio, offload pair).
 // key_terms_kernel evaluates those once per key into MIST_KEY_TERMS doubles, row_terms_kernel
 // reads them: the same operations on the same operands as when every row evaluates everything
-// (which it does when the caller passes no key-term workspace, and for the rows of the scout
-// pass, which are computed ahead of all others).
+// (which it does when the caller passes no key-term workspace, and for the gathered rows of the seed
+// launch, which are computed ahead of all others).
 constexpr int kKeyBwd = 0;        // [last?0:1 micro-batch][nock, ck] x (layer, first, last, extra_pre, extra_post)
 constexpr int kKeyFwd = 20;       // forward, not the first micro-batch: [nock, ck] x (layer, last, extra_post)
 constexpr int kKeyFwdFirst = 26;  //   its `first` and `extra_pre`, which do not depend on ckpt
@@ -845,7 +845,7 @@ __device__ __forceinline__ void store_rows(const double *lds_rows, int n, double
 }
 
 // kMode 0: every row of every group, and without key terms (kFromKeys) their stage summaries.
-// kMode 1: only the rows the scout pass gathers (workgroup = (128 gathered rows, group)), so that
+// kMode 1: only the rows the seed launch gathers (workgroup = (128 gathered rows, group)), so that
 // it can start before anything else is there.
 template <int kMode, bool kFromKeys>
 __global__ __launch_bounds__(kTermsBlock) void row_terms_kernel(
@@ -904,7 +904,7 @@ __global__ __launch_bounds__(kTermsBlock) void row_terms_kernel(
       __syncthreads();
       continue;
     }
-    // Summary of the stage for the reduce kernel: thread = (column, one of kTermsBlock / 32
+    // Summary of the stage: thread = (column, one of kTermsBlock / 32
     // runs of the stage's rows); columns 0 .. MIST_T_GCB hold the minimum, column kStageMaxOut
     // the maximum of MIST_T_OUT, the three behind it minima of post-layer terms.  The runs of a
     // wavefront meet by shuffle, the wavefronts in LDS.
@@ -946,7 +946,7 @@ __global__ __launch_bounds__(kTermsBlock) void row_terms_kernel(
 }
 
 // Stage summaries of every row, from the key terms and without the rows themselves: the search
-// reads the rows of a few stages (22B on 16x8: 67e6 rows, 18 GB, of which a tenth is read), which
+// reads the rows of a few stages (22B on 16x8: 67e6 rows, 18 GB, of which 9 % is read), which
 // are computed when it is known which (stage_rows_kernel).  Wavefront = stage, lane = row.  The columns a key decides are
 // taken from the stage's keys (16 of them as a rule), the six latencies and three memory columns
 // that see the optimizer ratio are evaluated per row and meet through LDS.  Bound by the float64
@@ -1088,7 +1088,7 @@ __global__ __launch_bounds__(kTermsBlock) void stage_floor_kernel(
 }
 
 // ------------------------------------------------------------------------------------------
-// Per-cell evaluation shared by the reduce and finalize kernels.
+// Per-cell evaluation of the evaluate-every-cell, first-estimate, finalize and analysis kernels.
 // ------------------------------------------------------------------------------------------
 struct PairIndex {
   int l, c;  // layers in the stage (1..L), checkpointed layers (0..l)
@@ -1210,10 +1210,9 @@ __device__ __forceinline__ void take_min(double &best, int32_t &best_row, bool f
 // What this replaces kept 34 (cost, row) minima per lane in registers (253 of them, two
 // wavefronts per SIMD), one sample and 16 p values per pass over the rows, visited every stage
 // summary with every tile and p tile, and committed rows one by one per lane: 7B on 4x8, one
-// sample: 1.35 ms in the reduce kernels (seeds 0.42, main launch 0.92 of which 0.9 were visits
-// of summaries that close), now seeds 0.50 beside the row terms, filter 0.06, reduce 0.33, resolve
-// 0.07; 22B on 16x8: 37.8e6 visits for 0.1e6 stages whose rows were read, 3.7 -> 1.5 ms per batch
-// of groups; 30 samples of the 7B plan's tables for one tensor-parallel size: 24 -> 7.2 ms.
+// sample: 1.35 ms (0.42 of it seeds); now seeds 0.29 beside key terms and summaries, filter 0.06, open 0.05,
+// reduce 0.27, resolve 0.05.  30 samples of the 7B plan's tables for one tensor-parallel size: 24 ms;
+// now 8.0 (reduce 4.2, open 1.4, resolve 1.3, filter 0.65, seeds 0.47).
 // ------------------------------------------------------------------------------------------
 constexpr int kSuperStages = 8;    // stages per second-level summary
 constexpr int kQueueShards = 64;   // counters of the item queue: one would serve an append in ~8 ns
@@ -2079,8 +2078,8 @@ __device__ __forceinline__ TileLane tile_lane(const MistProblem &prob, const Mis
   return t;
 }
 
-// A wavefront per item: only what its memory bounds leave open stays (7B on 4x8: 378000 stages x
-// tiles, 34000 pass the filter and 7800 of those are opened).
+// A wavefront per item: only what its memory bounds leave open stays (7B on 4x8: 454000 stages x
+// tiles, 36300 pass the filter and 13700 of those are opened; 22B on 16x8: 21.1e6, 2.1e6, 0.45e6).
 __global__ __launch_bounds__(kReduceThreads) void open_kernel(const MistProblem prob,
                                                               const MistGroupDesc *__restrict__ groups,
                                                               const double *__restrict__ stage_floor,
@@ -2543,12 +2542,13 @@ __device__ __forceinline__ void take_first(double &best, int32_t &best_row, bool
 }
 
 // ------------------------------------------------------------------------------------------
-// Kernel 2x: the same reduction with every cell evaluated.  No scout pass, no sieves, no bounds,
-// no bisection: each (row, l, c) goes through the latency model and the memory model, and each
-// of its p values through the reference's feasibility test and the (cost, row) comparison.  This
-// is the work the reference's formulas describe cell by cell; the pruned kernel above must
-// produce the same tables (tests) and is measured against it.  Same decomposition and slab
-// layout as eval_reduce_kernel's main launch, so finalize_kernel reads either.
+// Kernel 2x: the same reduction with every cell evaluated.  No seeds, no summaries, no bounds: each
+// (row, l, c) goes through the latency model and the memory model, and each of its p values
+// through the reference's feasibility test and the (cost, row) comparison.  This is the work the
+// reference's formulas describe cell by cell; the pruned launches above must produce the same
+// tables (tests) and are measured against it.  Workgroup = (row chunk, tile, p tile) of the
+// filter launch's decomposition; it leaves its minima in a slab of its own, and
+// combine_slabs_kernel takes the slabs into the table of minima, which finalize_kernel reads.
 // ------------------------------------------------------------------------------------------
 constexpr int kLdsRowStride = MIST_ROW_TERMS + 1;  // odd number of doubles: lanes reading the
                                                    // same term of different rows hit different banks
@@ -2694,7 +2694,7 @@ __device__ __forceinline__ int incumbent_stage_count(const MistProblem &prob,
   return S;
 }
 
-// Cost of the best pipeline of equal stages on equal meshes that the scout pass's seeds allow
+// Cost of the best pipeline of equal stages on equal meshes that the seeds allow
 // (sample 0 of a call with one sample, whose objective is the stage cost): group (G, mesh (n, m))
 // offers S = devices / (n m) stages of L / S layers each, the first one from the with_pre table
 // at S - 1 pre-saved micro-batches, the last one from the with_post table, those between from
@@ -2766,14 +2766,14 @@ __global__ __launch_bounds__(64 * kIncumbentWaves) void incumbent_kernel(
               (unsigned long long)__double_as_longlong(total));
 }
 
-// First estimate of the same pipeline cost, formed before the scout pass so that the scout pass
+// First estimate of the same pipeline cost, formed before the seeds so that the seed launch
 // can already leave out stage costs the caller's search cannot use.  Each group evaluates about
 // kEstimateRows of its gathered rows - every parallelism row of every scout pair without
 // activation / optimizer offloading first, then with the next ratios - for the layer count
 // l = L / S and every ckpt count, exactly as the tables would (same latency and memory code as
 // the evaluate-every-cell kernel, same cells kept: c == l - 1 only at p == 0 of the base /
 // with_pre tables), and keeps per stage of the pipeline the cheapest feasible cost.  Minima over
-// fewer rows than the scout pass sees, so the estimate is no smaller than the scout's.
+// fewer rows than the seeds see, so the estimate is no smaller than theirs.
 // Grid (kEstimateSplit, group); workgroup k writes its S minima to doubles [k S, (k + 1) S) of
 // the group's minima (the seed launch fills them afterwards).
 constexpr int kEstimateSplit = 16;
@@ -3365,7 +3365,7 @@ int64_t mist_reduce_workspace_doubles(int64_t cells, int64_t supers, int64_t ite
   if (cells < 0 || supers < 0 || items < 0 || n_samples < 1) return -1;
   return workspace_layout(cells, supers, items, n_samples).total;
 }
-// rows_present: false = only the rows the scout pass gathers are, the others follow by need
+// rows_present: false = only the rows the seed launch gathers are, the others follow by need
 static int reduce_tables(const MistProblem *problem, int n_samples, double *d_partial_cost, int32_t *d_partial_index,
                          ReduceTables *out, bool rows_present = true) {
   if (problem->reduce_cells < 1 || problem->reduce_supers < 1 || problem->reduce_items < 1 ||

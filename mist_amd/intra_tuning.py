@@ -2,9 +2,10 @@
 
 ``IntraStageTuner.tune()`` (reference :169-282) loops the gradient-accumulation candidates and
 device meshes and calls the numpy evaluation once per (G, mesh).  Here the host only prepares
-one small descriptor per (G, mesh) group; all groups of a tuner call are then evaluated by three
-kernel launches on the GPU (row terms, evaluate+mask+argmin, finalize) and the result tables
-stay resident in HBM for the inter-stage search.  ``IntraStageTunerOutput`` exposes the same
+one small descriptor per (G, mesh) group; all groups of a tuner call are then evaluated by one
+chain of kernel launches on the GPU (key terms, stage summaries and seeds, the pruned reduction,
+finalize) and the result tables stay resident in HBM for the inter-stage search.
+``IntraStageTunerOutput`` exposes the same
 fields and layouts as the reference (:59-82); numpy copies are made lazily on first access.
 """
 from __future__ import annotations
@@ -35,10 +36,11 @@ SCOUT_PAIR_SPAN = 200   # ... one more for every so many pairs of the group (GPT
 # ... and three for a group none of whose parallelism rows can hold this fraction of the model's
 # layers (weights, gradients and optimizer states of a layer at the group's tensor parallelism,
 # unsharded, nothing offloaded) within the memory capacity: such stages need sharding or
-# offloading, and the winners spread over the weight / gradient offload pairs.  (Speed only,
-# set from four plans: LLaMA-70B has 0.07 - 0.28 there for tp 1 - 4 and 0.55 for tp 8 and runs
-# 140 -> 98 ms with the two further pairs; GPT-7B has 0.73 - 5.9 and LLaMA-13B 0.37 - 3.0, and
-# they run 17 - 20 % slower with further pairs for every group, 2 % with them for tp 1.)
+# offloading, and the winners spread over the weight / gradient offload pairs.  (Speed only.
+# LLaMA-70B has 0.07 - 0.28 there for tp 1 - 4 and 0.55 for tp 8: tune 21.1 - 21.5 ms, 21.9 without
+# the two further pairs.  GPT-7B has 0.73 - 5.9 and LLaMA-13B 0.37 - 3.0: 2.14 and 4.08 ms, 2.25 and
+# 4.32 with further pairs for every group.  The span makes no difference on GPT-22B: 18.4 ms
+# with one pair, 18.7 - 19.4 with three.)
 SCOUT_TIGHT_FRACTION = 0.3
 SCOUT_TIGHT_PAIRS = 3
 # Upper bound of the row-term workspace (272 bytes per candidate row): the groups of a tuner call
@@ -70,7 +72,7 @@ def _side_stream(device) -> "torch.cuda.Stream":
     """The second stream that plans of several batches alternate with, one per device for the
     life of the process.  A stream per tuner would take another hardware queue each time (there
     are four): sooner or later one shared with the caller's stream or with the library's own
-    scout stream, whose kernels then no longer overlap (GPT-22B: 150 ms became 164 to 187 ms,
+    second stream, whose kernels then no longer overlap (GPT-22B, when it took 150 ms: 164 to 187 ms,
     depending on how many tuners the process had created before)."""
     key = str(torch.device(device))
     if key not in _SIDE_STREAMS:
@@ -280,7 +282,7 @@ class IntraStageTuner:
         device: str = "cuda:0",
         exhaustive: bool = False,
     ):
-        # exhaustive: evaluate every cell (no scout pass, no sieves) with
+        # exhaustive: evaluate every cell (no seeds, no bounds) with
         # mist_eval_reduce_exhaustive; same tables, the reference point for tests and bench
         self.exhaustive = bool(exhaustive)
         self.layer_tables = layer_tables
@@ -533,8 +535,8 @@ class IntraStageTuner:
             groups["key_offset"] = np.concatenate(([0], np.cumsum(n_keys)[:-1]))
             terms_blocks = -(-groups["n_rows"] // _lib.TERMS_BLOCK)
             reduce_blocks = groups["n_chunks"].astype(np.int64) * n_lc_tiles * n_p_tiles
-            # Scout pass: the rows of a group without weight / gradient offloading (one in n_pair)
-            # seed its chunks; groups that are small or have few offload pairs go without.
+            # Seeds: the rows of a group without weight / gradient offloading (one in n_pair) give
+            # its first minima; groups that are small or have few offload pairs go without.
             n_stages = -(-groups["n_rows"] // _lib.STAGE_ROWS)
             scout = (n_stages >= SCOUT_MIN_STAGES) & (groups["n_pair"] >= SCOUT_MIN_PAIRS) & (SCOUT_MIN_STAGES > 0)
             scout &= not self.exhaustive
@@ -774,8 +776,8 @@ class IntraStageTuner:
     def launch(self, plan, dev_plan, tables, events: Optional[list] = None) -> None:
         """Enqueues the kernels for every requested sample on the current stream; ``tables`` are
         the output tables (``DeviceTables``) or the ``MistOutTables`` of their pointers.  With
-        ``events`` (a list) the three kernels are launched through their own entry points and
-        ``(name, start_event, end_event)`` triples recorded on that stream are appended."""
+        ``events`` (a list) row terms, reduction and finalize are launched through their own entry
+        points and ``(name, start_event, end_event)`` triples recorded on that stream are appended."""
         if not dev_plan["batches"]:
             return
         lib = _lib.load()
@@ -890,7 +892,7 @@ class IntraStageTuner:
         ``stage_cost_cutoff`` (``num_devices``, ``ckpt_rule``; one sample only) is for a caller
         whose inter-stage search is all that reads the tables: the scout pass turns its seeds
         into an upper bound of the best pipeline cost (``MistProblem.stage_cost_incumbent``),
-        and the main launch does not look for stage costs that no threshold of that search can
+        and the launches behind it do not look for stage costs that no threshold of that search can
         admit.  Cells above that bound then hold some value above it, not their minimum.
 
         ``fill_costs`` False is for a caller that reads the costs of cells with a row index only:
