@@ -1470,7 +1470,10 @@ struct GroupModel {
   __device__ __forceinline__ double lower_share(float d) const {
     return (double)d * inv_G64 * (d < 0.0f ? 1.0 + kShareSlack : 1.0 - kShareSlack);
   }
-  __device__ __forceinline__ double lower_x(float x) const { return (double)x * (1.0 - kSlack); }
+  // (|x|: nothing checks that a provider's extra share of a latency is no larger than the whole)
+  __device__ __forceinline__ double lower_x(float x) const {
+    return (double)x - kSlack * fabs((double)x);
+  }
   __device__ __forceinline__ double bound(double ratio, float x, float d) const {
     return ratio * lower_x(x) + lower_share(d);
   }
@@ -1529,7 +1532,7 @@ __device__ __forceinline__ double stage_cost_cutoff(const MistProblem &prob, dou
 //   with_post = r (x + post_fwd + [row terms >= 0]) + (d + [row terms >= 0]) / G
 //   no_pp     = r (x + pre_fwd + pre_bwd + post_fwd + [..] + w1 + w2 + [..]) + (d + w1d + w2d + [..]) / G
 // so each is at least r x + d / G plus the offset below, up to a few roundings of relative size
-// 1e-16 of the operands (of which only d can be negative).  A row can reach a minimum `t` of such an
+// 1e-16 of the operands (the added terms are not negative).  A row can reach a minimum `t` of such an
 // objective only if GroupModel::bound <= t - offset: the bound is short by the slacks of r x and
 // d / G, the offsets are taken 1e-9 short, so every operand has room for its roundings a million
 // times over, and it is far less than anything that matters for pruning.  The row terms of the
