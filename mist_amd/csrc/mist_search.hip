@@ -1226,8 +1226,12 @@ constexpr int kStageRowsBlocks = 1024;       // four per CU, two stages at a tim
 constexpr int kSuperBlocks = 64;             // workgroups per group of the second-level summaries
 constexpr int kSeedLdsBytes = 40 * 1024;     // LDS aimed at per seed workgroup: four per CU
 constexpr int kSeedLdsMost = 160 * 1024;
-// Minima of one pair that every wavefront of a reduce workgroup can hold in LDS: 2559 values of p.
-constexpr int kMostBufferedSlots = kSeedLdsMost / (8 * (kReduceThreads / 64));
+// (row, pair) candidates a reduce wavefront collects: 64 that wait, and a pair's 64.
+constexpr int kCandidates = 128;
+constexpr int kCandidateDoubles = kCandidates * 2 / 8;
+// Minima of one pair that every wavefront of a reduce workgroup can hold in LDS beside them: 2543
+// values of p.
+constexpr int kMostBufferedSlots = kSeedLdsMost / (8 * (kReduceThreads / 64)) - kCandidateDoubles;
 static_assert(kQueueShards == 64, "a lane per shard");
 constexpr uint32_t kUnresolved = 0x80000000u;
 // Room below r x and below the terms the composite objectives add (their roundings: a few 1e-16) ...
@@ -1444,7 +1448,7 @@ __device__ __forceinline__ LaneMemory pair_memory(const Row &t, const PairConsts
 __device__ __forceinline__ int count_upper(double m0, double step, int n, double cap) {
   if (n <= 0 || !(m0 <= cap)) return 0;
   if (!(step > 1e-9 * cap)) return n;
-  const float most = (float)(cap - m0) * __frcp_rn((float)step) * 1.0001f + 0.01f;
+  const float most = (float)(cap - m0) * __builtin_amdgcn_rcpf((float)step) * 1.0001f + 0.01f;
   return most < (float)(n - 1) ? (int)most + 1 : n;
 }
 // The number itself: from the bound down to the last p the exact test admits.
@@ -1540,19 +1544,22 @@ __device__ __forceinline__ double stage_cost_cutoff(const MistProblem &prob, dou
 struct Offsets {
   double pre, post, pp;
 };
-__device__ __forceinline__ Offsets composite_offsets(const GroupModel &m, double ratio, double opb_min,
-                                                     double nag_min, double nrs_min) {
+// what is the same for the whole group ...
+__device__ __forceinline__ Offsets group_offsets(const GroupModel &m, double ratio) {
   const GroupConsts &k = m.k;
   const double shared = m.div_G(k.w1d + k.w2d);
-  const double stage_post =
-      (ratio * (opb_min + (k.pp_wre ? nag_min : 0.0) + (k.pp_gre ? nrs_min : 0.0)) +
-       m.div_G((k.pp_wre ? 0.0 : nag_min) + (k.pp_gre ? 0.0 : nrs_min))) * (1.0 - kSlack);
   Offsets o;
   o.pre = (ratio * (k.pre_fwd + k.pre_bwd + k.w1 + k.w2) + shared) * (1.0 - kSlack);
-  o.post = ratio * k.post_fwd * (1.0 - kSlack) + stage_post;
-  o.pp = (ratio * (k.pre_fwd + k.pre_bwd + k.post_fwd + k.w1 + k.w2) + shared) * (1.0 - kSlack) +
-         stage_post;
+  o.post = ratio * k.post_fwd * (1.0 - kSlack);
+  o.pp = (ratio * (k.pre_fwd + k.pre_bwd + k.post_fwd + k.w1 + k.w2) + shared) * (1.0 - kSlack);
   return o;
+}
+// ... and what the minima of a stage summary's post-layer terms add to the last two
+__device__ __forceinline__ double post_layer_offset(const GroupModel &m, double ratio, const double *__restrict__ floor) {
+  const GroupConsts &k = m.k;
+  const double opb = floor[kStageMinOpb], nag = floor[kStageMinNag], nrs = floor[kStageMinNrs];
+  return (ratio * (opb + (k.pp_wre ? nag : 0.0) + (k.pp_gre ? nrs : 0.0)) +
+          m.div_G((k.pp_wre ? 0.0 : nag) + (k.pp_gre ? 0.0 : nrs))) * (1.0 - kSlack);
 }
 
 // The last-stage / single-stage memory tests, p == 0 only (:2946-3106); `smallest_out`: what the
@@ -1882,18 +1889,27 @@ __global__ __launch_bounds__(256) void super_floor_kernel(const MistGroupDesc *_
 struct Loosest {
   double base, pre, post, pp;
 };
-// (`slots`: the pair's slots of one sample, `pitch` apart)
-__device__ __forceinline__ Loosest loosest_minima(const double *slots, int pitch, int P, int count_b, int count_p,
-                                                  bool do_post, bool do_pp, double cutoff) {
+// (`slots`: the pair's slots of one sample, `pitch` apart; a pair that is not `wanted` reads none)
+__device__ __forceinline__ Loosest loosest_minima(bool wanted, const double *slots, int pitch, int P, int count_b,
+                                                  int count_p, bool do_post, bool do_pp, double cutoff) {
+  Loosest t{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+  if (!wanted) return t;
   const double base = slots[max(count_b - 1, 0) * pitch], pre = slots[(P + max(count_p - 1, 0)) * pitch];
   const double post = slots[2 * P * pitch], pp = slots[(2 * P + 1) * pitch];
-  return Loosest{count_b > 0 ? fmin(base, cutoff) : -INFINITY, count_p > 0 ? fmin(pre, cutoff) : -INFINITY,
-                 do_post ? fmin(post, cutoff) : -INFINITY, do_pp ? fmin(pp, cutoff) : -INFINITY};
+  if (count_b > 0) t.base = fmin(base, cutoff);
+  if (count_p > 0) t.pre = fmin(pre, cutoff);
+  if (do_post) t.post = fmin(post, cutoff);
+  if (do_pp) t.pp = fmin(pp, cutoff);
+  return t;
 }
-// One threshold for GroupModel::bound that every row which could reach one of them passes.
-__device__ __forceinline__ double bound_threshold(const Loosest &t, const Offsets &o) {
-  return fmax(t.base, fmax(t.pre - o.pre, fmax(t.post - o.post, t.pp - o.pp)));
-}
+// One threshold for GroupModel::bound that every row which could reach one of them passes: in two
+// parts, from the offsets of the group and with what a stage's post-layer terms add to the second.
+struct Threshold {
+  double front, post;  // base and with_pre; with_post and no_pp
+  __device__ __forceinline__ Threshold(const Loosest &t, const Offsets &group)
+      : front(fmax(t.base, t.pre - group.pre)), post(fmax(t.post - group.post, t.pp - group.pp)) {}
+  __device__ __forceinline__ double at(double post_layer) const { return fmax(front, post - post_layer); }
+};
 
 // Lane = pair against a stage summary: the counts its pseudo row allows, hence which minima a row
 // of the stage can reach, and the bound that its objective gives.
@@ -1903,8 +1919,8 @@ struct StageReach {
   float x, d;            // of the pseudo row
   __device__ __forceinline__ double threshold(const double *slots, int pitch, int P, double ratio, double cutoff,
                                               const GroupModel &m, const double *__restrict__ floor) const {
-    return bound_threshold(loosest_minima(slots, pitch, P, count_b, count_p, post, pp, cutoff),
-                           composite_offsets(m, ratio, floor[kStageMinOpb], floor[kStageMinNag], floor[kStageMinNrs]));
+    return Threshold(loosest_minima(true, slots, pitch, P, count_b, count_p, post, pp, cutoff), group_offsets(m, ratio))
+        .at(post_layer_offset(m, ratio, floor));
   }
 };
 __device__ __forceinline__ StageReach stage_reach(const double *__restrict__ f, const PairConsts &k, int np,
@@ -1959,11 +1975,10 @@ __global__ __launch_bounds__(MIST_LC_TILE) void filter_kernel(
                         (g->cell_offset + ((int64_t)tile_rel * MIST_LC_TILE + lane) * slots_of(P)) * S;
 
   // no lane's row can matter: the pseudo row against the loosest minima
-  auto closed = [&](const double *__restrict__ f, double ratio, const Loosest &t) {
+  auto closed = [&](const double *__restrict__ f, double ratio, const Threshold &t) {
     float x, d;
     pair_latency(f, k, x, d);
-    const Offsets o = composite_offsets(m, ratio, f[kStageMinOpb], f[kStageMinNag], f[kStageMinNrs]);
-    return !__any(m.bound(ratio, x, d) <= bound_threshold(t, o));
+    return !__any(m.bound(ratio, x, d) <= t.at(post_layer_offset(m, ratio, f)));
   };
   const double *__restrict__ supers = super_floor + super_floor_slot(g, gi, 0) * kStageFloorPitch;
   const double *__restrict__ stages = stage_floor + stage_floor_slot(g, gi, 0) * kStageFloorPitch;
@@ -1971,8 +1986,8 @@ __global__ __launch_bounds__(MIST_LC_TILE) void filter_kernel(
   for (int first = super_first; first <= super_last; first += 64 * n_p) {
     uint32_t open = 0;
     for (int s = 0; s < S; ++s) {
-      const Loosest t = loosest_minima(slots + s, S, P, np, np, do_post, do_pp, cutoff);
       const double ratio = ratios.r[s];
+      const Threshold t(loosest_minima(true, slots + s, S, P, np, np, do_post, do_pp, cutoff), group_offsets(m, ratio));
       for (int i = 0; i < 64; ++i) {
         const int super = first + i * n_p;
         if (super > super_last) break;
@@ -1986,9 +2001,12 @@ __global__ __launch_bounds__(MIST_LC_TILE) void filter_kernel(
         open = lane == i ? seen : open;
       }
     }
-    // append the open stages to the tile's shard of the queue (items of a tile read the same minima:
-    // its shard is worked off by one XCD), to the next ones if it is full (all shards together hold
-    // every (tile, stage) of the launch)
+    // append the open stages to a shard of the queue, which one XCD works off, to the next ones if it is
+    // full (all shards together hold every (tile, stage) of the launch).  One sample: the shard of the
+    // chunk, so that the tiles which open a stage read its 17 KB of rows while they are in the L2 (the
+    // shard of the tile, for the minima: six times the rows from memory, 10.6 GB of 22B on 16x8 and 3.8
+    // instead of 3.2 ms of the reduce launch).  Several: the shard of the tile, whose minima are the
+    // larger part (1 MB with 30 samples).
     const int mine = __popc(open);
     int end = mine;
     for (int step = 1; step < 64; step <<= 1) {
@@ -1996,7 +2014,7 @@ __global__ __launch_bounds__(MIST_LC_TILE) void filter_kernel(
       if (lane >= step) end += o;
     }
     const int total = from_lane(end, 63);
-    int shard = (gi * 13 + tile_rel) % kQueueShards;
+    int shard = (gi * 13 + (S > 1 ? tile_rel : chunk)) % kQueueShards;
     for (int done = 0; done < total; shard = (shard + 1) % kQueueShards) {
       uint32_t base = 0;
       if (lane == 0) base = atomicAdd(tabs.counter + shard * kCounterPitch, (uint32_t)(total - done));
@@ -2168,53 +2186,157 @@ __global__ __launch_bounds__(kTermsBlock) void stage_rows_kernel(
 }
 
 // ---- reduce / resolve ----
+// A row's part of GroupModel::bound as a linear form of a pair's layer counts, unrounded: 0.2 ppm of
+// every operand short, so that float32 rounding of x (6e-8 of the operands, with what the sums and
+// products lose) and of d / G (twice that) leave it below every objective of the row.
+// (values in, not references to members: a choice between those would put the struct into memory)
+__device__ __forceinline__ double choose(bool first, double a, double b) { return first ? a : b; }
+struct LinearBound {
+  double ck, nock;          // per checkpointed / other layer
+  double all_ck, none, mid; // first and last layer of a stage with c == l, c == 0, other c
+  __device__ __forceinline__ double at(double n_ck, double n_nock, bool is_all, bool is_none) const {
+    return __builtin_fma(n_ck, ck, __builtin_fma(n_nock, nock, choose(is_all, all_ck, choose(is_none, none, mid))));
+  }
+};
+constexpr double kLinearSlack = 2e-7;
+__device__ __forceinline__ LinearBound linear_bound(const RowRegs &t, double ratio, double inv_G) {
+  auto term = [&](int stable, int delta) {
+    const double x = ratio * t[stable], d = t[delta] * inv_G;
+    return __builtin_fma(-kLinearSlack, fabs(x), x) + __builtin_fma(-kLinearSlack, fabs(d), d);
+  };
+  const double first_ck = term(MIST_T_S_FIRST_CK, MIST_T_D_FIRST_CK), last_ck = term(MIST_T_S_LAST_CK, MIST_T_D_LAST_CK);
+  const double first_nock = term(MIST_T_S_FIRST_NOCK, MIST_T_D_FIRST_NOCK);
+  LinearBound b;
+  b.ck = term(MIST_T_S_LAYER_CK, MIST_T_D_LAYER_CK);
+  b.nock = term(MIST_T_S_LAYER_NOCK, MIST_T_D_LAYER_NOCK);
+  // (1e-40: float32 values below the normal range are rounded by up to 1e-45)
+  b.all_ck = first_ck + last_ck - 1e-40;
+  b.none = first_nock + term(MIST_T_S_LAST_NOCK, MIST_T_D_LAST_NOCK) - 1e-40;
+  b.mid = first_nock + last_ck - 1e-40;
+  return b;
+}
+
+// The scaled peaks at p = 0 and their steps in another order of operations than pair_memory (a few
+// 1e-16 off), for bounds of the counts: 1e-12 of the capacity of room covers that for every step, the
+// quotient is taken 1e-4 and 0.01 long as in count_upper.
+struct LinearMemory {
+  double fwd, bwd, pwg, po, pwgo, s_ck, s_nock, d_ck, d_nock, out2, mf_base, mf_pp;
+};
+__device__ __forceinline__ LinearMemory linear_memory(const RowRegs &t) {
+  LinearMemory r;
+  r.out2 = 2.0 * t[MIST_T_OUT];
+  r.fwd = t[MIST_T_FWD_STATES0] + t[MIST_T_FWD_PEAK] + t[MIST_T_GCB];
+  r.bwd = t[MIST_T_BWD_STATES0] + t[MIST_T_BWD_PEAK] + t[MIST_T_GCB] + r.out2;
+  r.pwg = t[MIST_T_PWG];
+  r.po = t[MIST_T_PO];
+  r.pwgo = t[MIST_T_PWGO];
+  r.s_ck = t[MIST_T_S_CK];
+  r.s_nock = t[MIST_T_S_NOCK];
+  r.d_ck = t[MIST_T_D_CK];
+  r.d_nock = t[MIST_T_D_NOCK];
+  r.mf_base = t[MIST_T_MF_BASE];
+  r.mf_pp = t[MIST_T_MF_PP];
+  return r;
+}
+__device__ __forceinline__ int count_bound(double m0, double step, int n, double cap_and_room) {
+  const double room = cap_and_room - m0;
+  const float most = __builtin_fmaf((float)room * __builtin_amdgcn_rcpf((float)step), 1.0001f, 0.01f);
+  const int count = most < (float)(n - 1) ? (int)most + 1 : n;  // (a step of 0: infinite, or not a number)
+  return room >= 0.0 ? count : 0;
+}
+
 // One item with the pairs in `pairs`, one sample.  Returns the pairs in which some row reached its
-// minimum (kResolve: unused).  `lds_row`: the wavefront's buffer for the minima of one pair, which
-// the rows look up at their own counts; the next pair's are on their way in registers meanwhile.
-// kInLds false: there are too many for it (see kMostBufferedSlots), rows look them up in memory.
+// minimum (kResolve: unused).
+//   lane = pair   the slots the stage's pseudo row can reach, and with their minima a threshold;
+//   lane = row    the rows below it, by their linear bounds: two FMAs and a compare per pair;
+//   lane = row    of the pairs that have any: a bound of each row's count and the minimum there (one
+//                 pair's minima at a time in `lds_row`, the next ones on their way in registers);
+//   lane = (row, pair) of what is left, collected in `queue`: the reference's arithmetic.
+// VALU issue bounds it: of 22B on 16x8's 12.6e6 pairs with an open stage 4.9e6 hold rows below the
+// threshold, 23 of 64 rows each, and 0.9e6 a row that may reach a minimum.  (Every pair's rows through
+// the reference's latencies, then memory, counts and objectives for all of them as soon as one was
+// below the threshold: 1.9e9 wave instructions and 5.1 ms; now 1.05e9 and 3.2.  70B on 32x8 4.2 -> 2.6,
+// 7B on 4x8 0.28 -> 0.19.  Four wavefronts per SIMD, with 128 registers, are no faster than three.)
+// kInLds false: there are too many minima for the buffer (see kMostBufferedSlots), rows look them up in memory.
 template <bool kResolve, bool kInLds>
 __device__ __forceinline__ uint64_t reduce_item(const MistProblem &prob, const MistGroupDesc *__restrict__ g, int gi,
                                                 int tile_rel, int stage, const double *__restrict__ row_terms,
                                                 const double *__restrict__ stage_floor, double ratio,
-                                                const ReduceTables &tabs, uint64_t pairs, double *lds_row) {
+                                                const ReduceTables &tabs, uint64_t pairs, double *lds) {
   const int L = prob.num_layers, lane = threadIdx.x & 63;
-  const TileLane tl = tile_lane(prob, g, tile_rel);
   const int P = g->num_p, n_slots = slots_of(P);
   const GroupModel m = group_model(prob, g);
   const double cutoff = stage_cost_cutoff(prob, m.inv_G64);
   const int64_t tile_cell = g->cell_offset + (int64_t)tile_rel * MIST_LC_TILE * n_slots;
   const double *best = tabs.best + tile_cell;  // [pair][slot]
 
-  // ---- lane = pair: slots the pseudo row of the stage can reach, and the minima there ----
+  uint16_t *queue = reinterpret_cast<uint16_t *>(lds);  // pair << 6 | row
+  double *lds_row = lds + kCandidateDoubles;
+  // ---- lane = pair ----
   const double *__restrict__ f = stage_floor + stage_floor_slot(g, gi, stage) * kStageFloorPitch;
-  double thr;  // of this lane's pair
+  double thr, thr_post;  // of this lane's pair: of any variant, of with_post and no_pp
+  double off_pre;
+  int lc;  // l | c << 15
   uint64_t todo;
   {
+    const TileLane tl = tile_lane(prob, g, tile_rel);
+    lc = tl.pc.l | tl.pc.c << 15;
     const StageReach reach = stage_reach(f, pair_consts(tl.pc.l, tl.pc.c), tl.np, tl.do_post, tl.do_pp, m);
-    thr = reach.threshold(best + lane * n_slots, 1, P, ratio, cutoff, m, f);
-    todo = pairs & __ballot(tl.active && m.bound(ratio, reach.x, reach.d) <= thr);
+    const double bound = m.bound(ratio, reach.x, reach.d);
+    const Loosest low = loosest_minima(tl.active && bound <= cutoff, best + lane * n_slots, 1, P,
+                                       reach.count_b, reach.count_p, reach.post, reach.pp, cutoff);
+    const Offsets off = group_offsets(m, ratio);
+    const Threshold its(low, off);
+    const double post_layer = post_layer_offset(m, ratio, f);
+    thr = its.at(post_layer);
+    thr_post = its.post - post_layer;
+    off_pre = off.pre;
+    todo = pairs & __ballot(bound <= thr);
   }
   if (todo == 0) return 0;
 
   // ---- lane = row ----
   const int64_t row0 = (int64_t)stage * kStageRows;
   const int n_stage = (int)min((int64_t)kStageRows, g->n_rows - row0);
-  const double *__restrict__ my_row = row_terms + (g->row_offset + row0 + min(lane, n_stage - 1)) * MIST_ROW_TERMS;
-  const bool live = lane < n_stage;
-  RowRegs t;
-  load_terms<0, MIST_T_D_LAST_NOCK + 1>(t, my_row);
-  uint64_t sieve = 0;  // rows that pass the threshold of this lane's pair
+  const double *__restrict__ rows = row_terms + (g->row_offset + row0) * MIST_ROW_TERMS;
+  const uint64_t live = ~0ull >> (64 - n_stage);
+  LinearBound bound;
+  {
+    RowRegs t;
+    load_terms<0, MIST_T_D_LAST_NOCK + 1>(t, rows + min(lane, n_stage - 1) * MIST_ROW_TERMS);
+    bound = linear_bound(t, ratio, m.inv_G64);
+  }
+  struct Pair {  // wave-uniform
+    int l, c;
+    bool all_ck, none;
+    double n_ck, n_nock;
+  };
+  auto pair_at = [&](int pl) {
+    Pair p;
+    const int its = from_lane(lc, pl);
+    p.l = its & 0x7fff;
+    p.c = its >> 15;
+    const int lm2 = max(p.l - 2, 0), n_ck = min(max(p.c - 1, 0), lm2);
+    p.n_ck = (double)n_ck;
+    p.n_nock = (double)(lm2 - n_ck);
+    p.all_ck = p.c == p.l;
+    p.none = p.c == 0;
+    return p;
+  };
+  uint64_t left = 0;  // pairs with rows below their threshold
   for (uint64_t rest = todo; rest != 0; rest &= rest - 1) {
     const int pl = __ffsll((unsigned long long)rest) - 1;
-    const PairConsts k = pair_consts(from_lane(tl.pc.l, pl), from_lane(tl.pc.c, pl));
-    float x, d;
-    pair_latency(t, k, x, d);
-    const uint64_t pass = __ballot(live && m.bound(ratio, x, d) <= from_lane(thr, pl));
-    sieve = lane == pl ? pass : sieve;
+    const Pair p = pair_at(pl);
+    const uint64_t pass = live & __ballot(bound.at(p.n_ck, p.n_nock, p.all_ck, p.none) <= from_lane(thr, pl));
+    left |= pass != 0 ? 1ull << pl : 0ull;
   }
-  todo = __ballot(sieve != 0);
-  if (todo == 0) return 0;
-  load_terms<MIST_T_D_LAST_NOCK + 1, MIST_ROW_TERMS>(t, my_row);
+  if (left == 0) return 0;
+  LinearMemory mem;
+  {
+    RowRegs t;
+    load_terms<MIST_T_D_LAST_NOCK + 1, MIST_T_GCB + 1>(t, rows + min(lane, n_stage - 1) * MIST_ROW_TERMS);
+    mem = linear_memory(t);
+  }
   // minima of one pair, a slot per lane and register
   double ahead0 = 0.0, ahead1 = 0.0;
   auto fetch = [&](int pair) {
@@ -2232,58 +2354,110 @@ __device__ __forceinline__ uint64_t reduce_item(const MistProblem &prob, const M
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
   };
-  fetch(__ffsll((unsigned long long)todo) - 1);
-  const uint32_t my_row_number =
-      (kResolve ? 0u : kUnresolved) + (uint32_t)row_of_position(g, row0 + min(lane, n_stage - 1));
+
+  // ---- lane = (row, pair): the first `n` of the queue ----
   uint64_t hits = 0;
-  for (uint64_t rest = todo; rest != 0; rest &= rest - 1) {
-    const int pl = __ffsll((unsigned long long)rest) - 1;
-    const int l = from_lane(tl.pc.l, pl), c = from_lane(tl.pc.c, pl);
+  auto settle_candidates = [&](int n) {
+    const uint32_t entry = queue[min(lane, n - 1)];
+    const int pl = (int)(entry >> 6), its_row = (int)(entry & 63u);
+    const int its = __shfl(lc, pl), l = its & 0x7fff, c = its >> 15;
+    const bool in = lane < n;
+    RowRegs t;
+    load_terms<0, MIST_T_D_LAST_NOCK + 1>(t, rows + its_row * MIST_ROW_TERMS);
     const PairConsts k = pair_consts(l, c);
     float x, d;
     pair_latency(t, k, x, d);
-    const bool in = (from_lane(sieve, pl) >> lane & 1ull) != 0;
-    settle(pl);
-    const uint64_t later = rest & (rest - 1);
-    if (later != 0) fetch(__ffsll((unsigned long long)later) - 1);
-    const LaneMemory mem = pair_memory(t, k);
+    asm volatile("" : "+v"(x), "+v"(d)::"memory");
+    load_terms<MIST_T_NAG_CK, MIST_ROW_TERMS>(t, rows + its_row * MIST_ROW_TERMS);
     const int np = c == l - 1 ? min(P, 1) : P;
-    const bool do_post = c != l - 1, do_pp = do_post && l == L;
-    const Objectives o = objectives(t, x, d, k.no_ck, ratio, m, do_post);
-    // Rows that reach the minimum at the bound of their count: one pair in eight has any, and only
-    // these pay for the exact tests.  (A lowered slot may lie below the slots under it; a row above
-    // it is above the winner of its own slot too, which finalize takes from the slots at and above.)
-    const UpperCounts upper = upper_counts(mem, m, in ? np : 0);
-    auto minimum = [&](int slot) { return kInLds ? lds_row[slot] : best[(int64_t)pl * n_slots + slot]; };
-    auto may = [&](int count, double cost, int slot) {
-      return in && count > 0 && cost <= cutoff && cost < INFINITY && cost <= minimum(slot + max(count - 1, 0));
-    };
-    const bool may_b = may(upper.b, o.base, 0), may_p = may(upper.p, o.pre, P);
-    const bool may_post = do_post && may(1, o.post, 2 * P), may_pp = do_pp && may(1, o.pp, 2 * P + 1);
-    if (!__any(may_b || may_p || may_post || may_pp)) continue;
-    const RowCounts cnt = exact_counts(mem, m, may_b ? upper.b : 0, may_p ? upper.p : 0);
-    bool ok_post = false, ok_pp = false;
-    if (do_post) post_fits(t, k, mem, m, mem.out, k.no_ck ? t[MIST_T_RD] : 0.0, ok_post, ok_pp);
-    bool hit = false, lowered = false;
+    const bool do_post = in && c != l - 1, do_pp = do_post && l == L;
+    Objectives o = objectives(t, x, d, k.no_ck, ratio, m, true);
+    asm volatile("" : "+v"(o.base), "+v"(o.pre), "+v"(o.post), "+v"(o.pp)::"memory");
+    load_terms<MIST_T_D_LAST_NOCK + 1, MIST_T_NAG_CK>(t, rows + its_row * MIST_ROW_TERMS);
+    const LaneMemory lm = pair_memory(t, k);
+    const UpperCounts upper = upper_counts(lm, m, in ? np : 0);
+    const RowCounts cnt = exact_counts(lm, m, upper.b, upper.p);
+    bool ok_post, ok_pp;
+    post_fits(t, k, lm, m, lm.out, k.no_ck ? t[MIST_T_RD] : 0.0, ok_post, ok_pp);
     const int64_t cell = tile_cell + pl * n_slots;
-    // rows with `count` > 0 against the minimum of slot `slot` + count - 1
-    auto offer = [&](int count, double cost, int slot) {
-      const int own = slot + max(count - 1, 0);
-      const double now = in && count > 0 && cost <= cutoff && cost < INFINITY ? minimum(own) : -INFINITY;
-      if (!kResolve && cost < now) {
+    const int own_b = max(cnt.b - 1, 0), own_p = P + max(cnt.p - 1, 0);
+    const double *slots = tabs.best + cell;
+    const double now_b = slots[own_b], now_p = slots[own_p], now_post = slots[2 * P], now_pp = slots[2 * P + 1];
+    const uint32_t number = (kResolve ? 0u : kUnresolved) + (uint32_t)row_of_position(g, row0 + its_row);
+    bool hit = false, lowered = false;
+    // A lowered slot may lie below the slots under it; a row above it is above the winner of its own
+    // slot too, which finalize takes from the slots at and above.
+    auto offer = [&](bool ok, double cost, int own, double now) {
+      if (!(ok && cost <= now && cost <= cutoff && cost < INFINITY)) return;
+      hit = true;
+      if (cost == now) {
+        atomicMin(tabs.row + cell + own, number);
+      } else if (!kResolve) {
         lower_minimum(tabs.best + cell + own, cost);
         lowered = true;
       }
-      if (cost == now) atomicMin(tabs.row + cell + own, my_row_number);
-      hit = hit || cost <= now;
     };
-    offer(cnt.b, o.base, 0);
-    offer(cnt.p, o.pre, P);
-    if (do_post) offer(ok_post ? 1 : 0, o.post, 2 * P);
-    if (do_pp) offer(ok_pp ? 1 : 0, o.pp, 2 * P + 1);
-    if (kResolve) continue;
-    if (__any(lowered) && lane == 0) tabs.changed[cell / 4] = 1u;
-    if (__any(hit)) hits |= 1ull << pl;
+    offer(cnt.b > 0, o.base, own_b, now_b);
+    offer(cnt.p > 0, o.pre, own_p, now_p);
+    offer(do_post && ok_post, o.post, 2 * P, now_post);
+    offer(do_pp && ok_pp, o.pp, 2 * P + 1, now_pp);
+    if (kResolve) return;
+    if (lowered) tabs.changed[cell / 4] = 1u;
+    for (uint64_t some = __ballot(hit); some != 0;) {  // a few pairs of the 64 candidates
+      const int first = from_lane(pl, __ffsll((unsigned long long)some) - 1);
+      hits |= 1ull << first;
+      some &= ~(uint64_t)__ballot(pl == first);
+    }
+  };
+
+  const double cap_and_room = m.cap * (1.0 + 1e-12);
+  int waiting = 0;
+  fetch(__ffsll((unsigned long long)left) - 1);
+  uint64_t rest = left;
+  while (rest != 0 || waiting > 0) {
+    if (rest != 0) {
+      const int pl = __ffsll((unsigned long long)rest) - 1;
+      settle(pl);
+      rest &= rest - 1;
+      if (rest != 0) fetch(__ffsll((unsigned long long)rest) - 1);
+      const Pair p = pair_at(pl);
+      const double low = bound.at(p.n_ck, p.n_nock, p.all_ck, p.none);
+      const double lf = (double)p.l, lm1 = (double)(p.l - 1);
+      double saved_now = lm1 * mem.s_ck, next = mem.s_ck, ck_delta = mem.d_ck;
+      if (!p.all_ck) {
+        saved_now = __builtin_fma((double)p.c, mem.s_ck, (double)(p.l - p.c - 1) * mem.s_nock);
+        next = mem.s_nock;
+      }
+      if (p.c < p.l - 1) ck_delta = mem.d_nock;
+      const double shared = saved_now + ck_delta, step = saved_now + next + mem.out2;
+      const double fwd = __builtin_fma(lf, mem.pwg, __builtin_fma(lm1, mem.po, mem.fwd));
+      const double bwd = __builtin_fma(lf, mem.pwgo, mem.bwd), peak = shared + fmax(fwd, bwd);
+      const int np = p.c == p.l - 1 ? min(P, 1) : P;
+      const int upper_b = count_bound(peak * mem.mf_base, step * mem.mf_base, np, cap_and_room);
+      const int upper_p = count_bound((peak + m.pre_sas) * mem.mf_pp, (step + m.pre_saved) * mem.mf_pp, np, cap_and_room);
+      auto minimum = [&](int slot) { return kInLds ? lds_row[slot] : best[(int64_t)pl * n_slots + slot]; };
+      const double now_b = minimum(max(upper_b - 1, 0)), now_p = minimum(P + max(upper_p - 1, 0));
+      bool may = (upper_b > 0 && low <= fmin(now_b, cutoff)) || (upper_p > 0 && low <= fmin(now_p, cutoff) - off_pre);
+      const bool may_post = low <= from_lane(thr_post, pl);
+      if (__any(may_post)) {  // a pair in seven
+        // the larger ones of post_fits' sums (a single stage's factor is the smaller one, MIST_T_MF)
+        const double post = shared + fmax(fwd, bwd - 0.5 * mem.out2 + m.post_output);
+        const double factor = p.l == L ? mem.mf_pp - (0.025 + 1e-9) : mem.mf_pp;
+        may = may || (may_post && (post + m.post_states) * factor <= cap_and_room);
+      }
+      const uint64_t found = live & __ballot(may && low <= from_lane(thr, pl));
+      if (found >> lane & 1ull)
+        queue[waiting + __popcll(found & ((1ull << lane) - 1ull))] = (uint16_t)(pl << 6 | lane);
+      waiting += __popcll(found);
+      if (waiting == 0 || (waiting < 64 && rest != 0)) continue;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    settle_candidates(min(waiting, 64));
+    waiting = max(waiting - 64, 0);
+    const uint16_t moved = queue[64 + lane];
+    __builtin_amdgcn_wave_barrier();
+    queue[lane] = moved;
   }
   return hits;
 }
@@ -2432,7 +2606,7 @@ __device__ __forceinline__ uint64_t every_pair(int k) {
 template <bool kResolve, bool kSamples, bool kInLds>
 __global__ __launch_bounds__(kReduceThreads, 3) void reduce_kernel(
     const MistProblem prob, const MistGroupDesc *__restrict__ groups, const double *__restrict__ row_terms,
-    const double *__restrict__ stage_floor, const RatioList ratios, const ReduceTables tabs, int row_pitch) {
+    const double *__restrict__ stage_floor, const RatioList ratios, const ReduceTables tabs, int wave_pitch) {
   extern __shared__ double lds_rows[];
   constexpr int kWaves = kReduceThreads / 64;
   const int local_wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
@@ -2448,7 +2622,7 @@ __global__ __launch_bounds__(kReduceThreads, 3) void reduce_kernel(
                                           &lds_samples[local_wave]);
     } else
       hit = reduce_item<kResolve, kInLds>(prob, g, gi, tile_rel, stage, row_terms, stage_floor, ratios.r[0], tabs,
-                                          pairs, lds_rows + local_wave * row_pitch);
+                                          pairs, lds_rows + local_wave * wave_pitch);
     if (!kResolve && hit != 0 && lane == 0) atomicOr(tabs.hit + at, (unsigned long long)hit);
   };
   constexpr bool kListed = kResolve && kSamples;
@@ -3491,22 +3665,22 @@ static int launch_reduce(const MistProblem *problem, const MistGroupDesc *d_grou
   hipLaunchKernelGGL(filter_kernel, dim3(xcd_padded_grid(n_blocks)), dim3(MIST_LC_TILE), 0, (hipStream_t)stream,
                      *problem, d_groups, n_groups, d_block_prefix, n_blocks, d_stage_floor, tabs.super_floor, ratios, tabs);
   MIST_HIP_CHECK(hipGetLastError());
-  hipLaunchKernelGGL(open_kernel, dim3(kReduceBlocks), dim3(kReduceThreads), 0, (hipStream_t)stream, *problem,
-                     d_groups, d_stage_floor, ratios, tabs);
+  const bool one = tabs.n_samples == 1, buffered = one && slots_of(problem->reduce_max_p) <= kMostBufferedSlots;
+  hipLaunchKernelGGL(open_kernel, dim3(kReduceBlocks), dim3(kReduceThreads), 0,
+                     (hipStream_t)stream, *problem, d_groups, d_stage_floor, ratios, tabs);
   MIST_HIP_CHECK(hipGetLastError());
   if (tabs.listed != nullptr) {
     hipLaunchKernelGGL(stage_rows_kernel, dim3(kStageRowsBlocks), dim3(kTermsBlock), 0, (hipStream_t)stream, *problem,
                        d_groups, const_cast<double *>(d_row_terms), d_key_terms, tabs);
     MIST_HIP_CHECK(hipGetLastError());
   }
-  const bool one = tabs.n_samples == 1, buffered = one && slots_of(problem->reduce_max_p) <= kMostBufferedSlots;
-  const int row_pitch = buffered ? slots_of(problem->reduce_max_p) : 0;
-  const size_t lds = sizeof(double) * row_pitch * (kReduceThreads / 64);
+  const int wave_pitch = one ? kCandidateDoubles + (buffered ? slots_of(problem->reduce_max_p) : 0) : 0;
+  const size_t lds = sizeof(double) * wave_pitch * (kReduceThreads / 64);
   if (lds > 64 * 1024)
     if (int rc = allow_large_lds()) return rc;
 #define MIST_REDUCE(RESOLVE, SAMPLES, IN_LDS)                                                               \
   hipLaunchKernelGGL((reduce_kernel<RESOLVE, SAMPLES, IN_LDS>), dim3(kReduceBlocks), dim3(kReduceThreads), lds, \
-                     (hipStream_t)stream, *problem, d_groups, d_row_terms, d_stage_floor, ratios, tabs, row_pitch)
+                     (hipStream_t)stream, *problem, d_groups, d_row_terms, d_stage_floor, ratios, tabs, wave_pitch)
   if (!one) MIST_REDUCE(false, true, false);
   else if (buffered) MIST_REDUCE(false, false, true);
   else MIST_REDUCE(false, false, false);
