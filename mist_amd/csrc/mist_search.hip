@@ -1268,7 +1268,7 @@ struct ReduceTables {
   uint32_t *changed;         // [pair's first cell / 4]: samples whose minima the reduce launch lowered
   double *super_floor;       // [supers][kStageFloorPitch]
   // [kQueueShards][capacity]: Item, what the filter and then what the open launch left; pairs of the
-  // latter in which a row reached its minimum
+  // latter, first the open ones, then those in which a row reached its minimum
   unsigned long long *item, *opened, *hit;
   // [kQueueShards][capacity]: group << 32 | stage of the stages opened, each once; stage_flag (one
   // per stage summary) tells whether one is listed.  Null: the rows of all stages are there.
@@ -2099,44 +2099,101 @@ __device__ __forceinline__ TileLane tile_lane(const MistProblem &prob, const Mis
   return t;
 }
 
-// A wavefront per item: only what its memory bounds leave open stays (7B on 4x8: 454000 stages x
-// tiles, 36300 pass the filter and 13700 of those are opened; 22B on 16x8: 21.1e6, 2.1e6, 0.45e6).
+// A wavefront takes runs of neighbouring items: only what the memory bounds of their stages leave open
+// stays, with a word of its open pairs (7B on 4x8: 454000 stages x tiles, 36300 pass the filter and
+// 13700 of those are opened; 22B on 16x8: 21.1e6, 2.1e6, 0.45e6).  Items of a run are mostly the
+// stages of one tile, whose pairs, constants and offsets stay in registers.
+//   One sample: lane = pair; VALU issue and the gather of minima, a line per lane and load, bound it (an
+//   item of its own per wavefront, everything computed again for each, 540 VALU instructions: 22B
+//   2.9 ms; now 2.2).
+//   Several: lane = pair for what the stage can reach, then lane = (pair parity, sample): the minima of a
+//   slot lie side by side, two lines per load (lane = pair through all samples, a line per lane and load,
+//   kept the address units busy 82 % of the time: 30 samples of 7B for one tensor-parallel size 1.41 ms;
+//   now 0.45, and it knows every open pair: the reduce launch tries 1.4e6 instead of 2.9e6).
+constexpr int kOpenRun = 16;
+template <bool kSamples>
 __global__ __launch_bounds__(kReduceThreads) void open_kernel(const MistProblem prob,
                                                               const MistGroupDesc *__restrict__ groups,
                                                               const double *__restrict__ stage_floor,
                                                               const RatioList ratios, const ReduceTables tabs) {
   constexpr int kWaves = kReduceThreads / 64;
-  const int lane = threadIdx.x & 63, S = tabs.n_samples;
+  const int lane = threadIdx.x & 63, S = kSamples ? tabs.n_samples : 1;
+  const int sample = kSamples ? min(lane & 31, S - 1) : 0;
   const FlatQueue queue = flat_queue(tabs, 0);
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * kWaves + (threadIdx.x >> 6)));
-  for (uint32_t i = wave; i < queue.total; i += gridDim.x * kWaves) {
-    const int64_t from = queue.at(i, tabs.capacity);
-    const uint64_t word = from_lane((uint64_t)tabs.item[from], 0);
-    const Item item(word);
-    const int gi = item.group, tile_rel = item.tile, stage = item.stage;
-    const MistGroupDesc *g = groups + gi;
-    const TileLane p = tile_lane(prob, g, tile_rel);
-    const GroupModel m = group_model(prob, g);
-    const double cutoff = stage_cost_cutoff(prob, m.inv_G64);
-    const int P = g->num_p;
-    const double *__restrict__ f = stage_floor + stage_floor_slot(g, gi, stage) * kStageFloorPitch;
-    const StageReach reach = stage_reach(f, pair_consts(p.pc.l, p.pc.c), p.np, p.do_post, p.do_pp, m);
-    const double *slots = tabs.best +
-                          (g->cell_offset + ((int64_t)tile_rel * MIST_LC_TILE + lane) * slots_of(P)) * S;
-    bool open = false;
-    for (int s = 0; s < S && !__any(open); ++s)
-      open = p.active && m.bound(ratios.r[s], reach.x, reach.d) <=
-                             reach.threshold(slots + s, S, P, ratios.r[s], cutoff, m, f);
-    if (!__any(open)) continue;
-    const uint32_t shard = (uint32_t)(from / tabs.capacity);
-    if (lane == 0) {
-      // (no more than the shard's items are opened: it cannot overflow)
-      const uint32_t to = atomicAdd(tabs.counter + (kQueueShards + shard) * kCounterPitch, 1u);
-      tabs.opened[(int64_t)shard * tabs.capacity + to] = word;
-      tabs.hit[(int64_t)shard * tabs.capacity + to] = 0;
-      if (tabs.listed != nullptr && atomicExch(tabs.stage_flag + stage_floor_slot(g, gi, stage), 1u) == 0) {
-        const uint32_t row_to = atomicAdd(tabs.counter + (2 * kQueueShards + shard) * kCounterPitch, 1u);
-        tabs.listed[(int64_t)shard * tabs.capacity + row_to] = (unsigned long long)gi << 32 | (uint32_t)stage;
+  const uint32_t n_waves = gridDim.x * kWaves, run = max(1u, min((uint32_t)kOpenRun, queue.total / (2 * n_waves)));
+  const double ratio = ratios.r[sample];
+  // of the tile the last item was of
+  uint64_t tile_word = ~0ull;
+  const MistGroupDesc *g = groups;
+  TileLane p = {};
+  PairConsts k = {};
+  GroupModel m = {};
+  Offsets group = {};
+  double cutoff = INFINITY;
+  int P = 1;
+  const double *best = tabs.best;
+  for (uint32_t first = wave * run; first < queue.total; first += n_waves * run) {
+    const uint32_t end = min(first + run, queue.total);
+    int64_t from = queue.at(first, tabs.capacity);
+    uint64_t ahead = tabs.item[from];
+    for (uint32_t i = first; i < end; ++i) {
+      const uint64_t word = from_lane(ahead, 0);
+      const uint32_t shard = (uint32_t)(from / tabs.capacity);
+      if (i + 1 < end) {
+        from = queue.at(i + 1, tabs.capacity);
+        ahead = tabs.item[from];
+      }
+      const Item item(word);
+      const int gi = item.group, stage = item.stage;
+      if (word >> kItemStageBits != tile_word) {
+        tile_word = word >> kItemStageBits;
+        g = groups + gi;
+        p = tile_lane(prob, g, item.tile);
+        k = pair_consts(p.pc.l, p.pc.c);
+        m = group_model(prob, g);
+        group = group_offsets(m, ratio);
+        cutoff = stage_cost_cutoff(prob, m.inv_G64);
+        P = g->num_p;
+        best = tabs.best + (g->cell_offset + (int64_t)item.tile * MIST_LC_TILE * slots_of(P)) * S;
+      }
+      const double *__restrict__ f = stage_floor + stage_floor_slot(g, gi, stage) * kStageFloorPitch;
+      const StageReach reach = stage_reach(f, k, p.np, p.do_post, p.do_pp, m);
+      const double post_layer = post_layer_offset(m, ratio, f);
+      uint64_t open = 0;
+      if (!kSamples) {
+        // (what lies above the cutoff needs no minima)
+        const double bound = m.bound(ratio, reach.x, reach.d);
+        const Loosest low = loosest_minima(p.active && bound <= cutoff, best + lane * slots_of(P), 1, P, reach.count_b,
+                                           reach.count_p, reach.post, reach.pp, cutoff);
+        open = __ballot(bound <= Threshold(low, group).at(post_layer));
+      } else {
+        const int parts = reach.count_b | reach.count_p << 15 | (int)reach.post << 30 | (int)((unsigned)reach.pp << 31);
+        // two pairs at a time
+        for (uint64_t rest = __ballot(p.active && parts != 0); rest != 0;) {
+          const int even = __ffsll((unsigned long long)rest) - 1;
+          rest &= rest - 1;
+          const int odd = rest != 0 ? __ffsll((unsigned long long)rest) - 1 : even;
+          rest &= rest - 1;
+          const int mine = lane < 32 ? even : odd;
+          const uint32_t its = (uint32_t)__shfl(parts, mine);
+          const Loosest low = loosest_minima(true, best + (int64_t)mine * slots_of(P) * S + sample, S, P, (int)(its & 0x7fff),
+                                             (int)(its >> 15 & 0x7fff), (its >> 30 & 1u) != 0, its >> 31 != 0, INFINITY);
+          const uint64_t pass =
+              __ballot(m.bound(ratio, __shfl(reach.x, mine), __shfl(reach.d, mine)) <= Threshold(low, group).at(post_layer));
+          open |= ((uint32_t)pass != 0 ? 1ull << even : 0ull) | (pass >> 32 != 0 ? 1ull << odd : 0ull);
+        }
+      }
+      if (open == 0) continue;
+      if (lane == 0) {
+        // (no more than the shard's items are opened: it cannot overflow)
+        const uint32_t to = atomicAdd(tabs.counter + (kQueueShards + shard) * kCounterPitch, 1u);
+        tabs.opened[(int64_t)shard * tabs.capacity + to] = word;
+        tabs.hit[(int64_t)shard * tabs.capacity + to] = open;
+        if (tabs.listed != nullptr && atomicExch(tabs.stage_flag + stage_floor_slot(g, gi, stage), 1u) == 0) {
+          const uint32_t row_to = atomicAdd(tabs.counter + (2 * kQueueShards + shard) * kCounterPitch, 1u);
+          tabs.listed[(int64_t)shard * tabs.capacity + row_to] = (unsigned long long)gi << 32 | (uint32_t)stage;
+        }
       }
     }
   }
@@ -2283,7 +2340,7 @@ __device__ __forceinline__ uint64_t reduce_item(const MistProblem &prob, const M
     lc = tl.pc.l | tl.pc.c << 15;
     const StageReach reach = stage_reach(f, pair_consts(tl.pc.l, tl.pc.c), tl.np, tl.do_post, tl.do_pp, m);
     const double bound = m.bound(ratio, reach.x, reach.d);
-    const Loosest low = loosest_minima(tl.active && bound <= cutoff, best + lane * n_slots, 1, P,
+    const Loosest low = loosest_minima((pairs >> lane & 1ull) != 0 && bound <= cutoff, best + lane * n_slots, 1, P,
                                        reach.count_b, reach.count_p, reach.post, reach.pp, cutoff);
     const Offsets off = group_offsets(m, ratio);
     const Threshold its(low, off);
@@ -2623,7 +2680,8 @@ __global__ __launch_bounds__(kReduceThreads, 3) void reduce_kernel(
     } else
       hit = reduce_item<kResolve, kInLds>(prob, g, gi, tile_rel, stage, row_terms, stage_floor, ratios.r[0], tabs,
                                           pairs, lds_rows + local_wave * wave_pitch);
-    if (!kResolve && hit != 0 && lane == 0) atomicOr(tabs.hit + at, (unsigned long long)hit);
+    // (the other units of the item read and write other bits)
+    if (!kResolve && hit != pairs && lane == 0) atomicAnd(tabs.hit + at, (unsigned long long)~(pairs & ~hit));
   };
   constexpr bool kListed = kResolve && kSamples;
   const FlatQueue queue = flat_queue(tabs, kListed ? 0 : 1);
@@ -2666,7 +2724,9 @@ __global__ __launch_bounds__(kReduceThreads, 3) void reduce_kernel(
       if (u >= n) break;
       ahead = draw();
       const int64_t at = queue.at((first + u) >> split, tabs.capacity);
-      work(at, from_lane((uint64_t)tabs.opened[at], 0), every_pair(split) << ((first + u) & ((1u << split) - 1u)));
+      const uint64_t pairs = tabs.hit[at] & every_pair(split) << ((first + u) & ((1u << split) - 1u));
+      const uint64_t word = tabs.opened[at];
+      if (from_lane(pairs, 0) != 0) work(at, from_lane(word, 0), from_lane(pairs, 0));
     }
   }
 }
@@ -3666,7 +3726,7 @@ static int launch_reduce(const MistProblem *problem, const MistGroupDesc *d_grou
                      *problem, d_groups, n_groups, d_block_prefix, n_blocks, d_stage_floor, tabs.super_floor, ratios, tabs);
   MIST_HIP_CHECK(hipGetLastError());
   const bool one = tabs.n_samples == 1, buffered = one && slots_of(problem->reduce_max_p) <= kMostBufferedSlots;
-  hipLaunchKernelGGL(open_kernel, dim3(kReduceBlocks), dim3(kReduceThreads), 0,
+  hipLaunchKernelGGL(one ? open_kernel<false> : open_kernel<true>, dim3(kReduceBlocks), dim3(kReduceThreads), 0,
                      (hipStream_t)stream, *problem, d_groups, d_stage_floor, ratios, tabs);
   MIST_HIP_CHECK(hipGetLastError());
   if (tabs.listed != nullptr) {
