@@ -695,7 +695,7 @@ __global__ __launch_bounds__(kTermsBlock) void key_terms_kernel(
     dst[i] = lds_out[i / MIST_KEY_TERMS][i % MIST_KEY_TERMS];
 }
 
-__device__ __forceinline__ int64_t gathered_position(const MistGroupDesc *g, int64_t q);
+__device__ __forceinline__ int64_t gathered_position(const MistGroupDesc *g, uint32_t q);
 
 // Terms of the row at workspace position `row` of a group.  kFromKeys: what is the same for the
 // n_oo rows of its key is read from `key_terms` (written by key_terms_kernel) instead of evaluated.
@@ -876,7 +876,7 @@ __global__ __launch_bounds__(kTermsBlock) void row_terms_kernel(
   const int rows_here = (int)min((int64_t)kTermsBlock, n_here_total - block_first);
   // Lanes past the end recompute the last row (no divergent barrier); their result is dropped.
   const int64_t nth = block_first + min((int)threadIdx.x, rows_here - 1);
-  const int64_t row = kMode == 1 ? gathered_position(g, nth) : nth;  // workspace position
+  const int64_t row = kMode == 1 ? gathered_position(g, (uint32_t)nth) : nth;  // workspace position
   double t[MIST_ROW_TERMS];  // compile-time indices only: registers
   row_terms_of<kFromKeys>(prob, g, (uint32_t)row, key_terms, lds_gpu_gpu, I, t);
 
@@ -1096,7 +1096,8 @@ struct PairIndex {
 
 // Valid (l, c <= l) pairs are numbered l-major: index(l, c) = l*(l+1)/2 - 1 + c.
 __device__ __forceinline__ PairIndex decode_pair(int idx) {
-  int l = (int)((sqrt(8.0 * (double)idx + 9.0) - 1.0) * 0.5);
+  // (the float32 root is off by less than 1 up to 32765 layers; the loops settle it)
+  int l = (int)((__builtin_amdgcn_sqrtf(__builtin_fmaf(8.0f, (float)idx, 9.0f)) - 1.0f) * 0.5f);
   while (l * (l + 1) / 2 - 1 > idx) --l;
   while ((l + 1) * (l + 2) / 2 - 1 <= idx) ++l;
   return PairIndex{l, idx - (l * (l + 1) / 2 - 1)};
@@ -1215,6 +1216,7 @@ __device__ __forceinline__ void take_min(double &best, int32_t &best_row, bool f
 // now 8.0 (reduce 4.2, open 1.4, resolve 1.3, filter 0.65, seeds 0.47).
 // ------------------------------------------------------------------------------------------
 constexpr int kSuperStages = 8;    // stages per second-level summary
+constexpr int kGatherFloor = 5;    // linear bounds of 64 gathered rows
 constexpr int kQueueShards = 64;   // counters of the item queue: one would serve an append in ~8 ns
 constexpr int kCounterPitch = 32;  // uint32 between counters: a cache line each
 constexpr int kNumXcd = 8;
@@ -1225,6 +1227,7 @@ constexpr int kReduceBlocks = 2048;          // a multiple of kNumXcd
 constexpr int kStageRowsBlocks = 1024;       // four per CU, two stages at a time each
 constexpr int kSuperBlocks = 64;             // workgroups per group of the second-level summaries
 constexpr int kSeedLdsBytes = 40 * 1024;     // LDS aimed at per seed workgroup: four per CU
+constexpr int kSeedWorkgroups = 2048;
 constexpr int kSeedLdsMost = 160 * 1024;
 // (row, pair) candidates a reduce wavefront collects: 64 that wait, and a pair's 64.
 constexpr int kCandidates = 128;
@@ -1267,6 +1270,7 @@ struct ReduceTables {
   uint32_t *row;
   uint32_t *changed;         // [pair's first cell / 4]: samples whose minima the reduce launch lowered
   double *super_floor;       // [supers][kStageFloorPitch]
+  double *gather_floor;      // [stage][kGatherFloor]: what the seed launch asks of 64 gathered rows (one sample)
   // [kQueueShards][capacity]: Item, what the filter and then what the open launch left; pairs of the
   // latter, first the open ones, then those in which a row reached its minimum
   unsigned long long *item, *opened, *hit;
@@ -1335,14 +1339,15 @@ __device__ __forceinline__ LaneMemory cell_memory(const double *__restrict__ t, 
 // workspace order those rows are scattered (one per (parallelism row, activation ratio, optimizer
 // ratio)); the seed launch gathers them, n_par * n_oo * n_ao rows per group.
 // With scout_stride = m > 1 the rows of the pairs scout_pair[1 .. m-1] follow.
-__device__ __forceinline__ int64_t gathered_position(const MistGroupDesc *g, int64_t q) {
-  const int n_tail = g->n_oo * g->n_ao;
-  const int64_t per_pair = (int64_t)g->n_par * n_tail;
-  const int64_t k = q / per_pair, rest = q - k * per_pair;
-  const int64_t par = rest / n_tail, tail = rest - par * n_tail;
-  const int64_t pair = g->scout_pair[k];
-  const int ao = (int)(tail / g->n_oo), oo = (int)(tail - (int64_t)ao * g->n_oo);
-  return par * g->n_off + (int64_t)ao * g->n_oo * g->n_pair + tile_position(g, oo, (int)pair);
+// (32-bit arithmetic: q and positions are below the number of rows)
+__device__ __forceinline__ int64_t gathered_position(const MistGroupDesc *g, uint32_t q) {
+  const uint32_t n_ao = (uint32_t)g->n_ao, n_oo = (uint32_t)g->n_oo, n_tail = n_oo * n_ao;
+  const uint32_t per_pair = (uint32_t)g->n_par * n_tail;
+  const uint32_t k = q / per_pair, rest = q - k * per_pair;
+  const uint32_t par = rest / n_tail, tail = rest - par * n_tail;
+  const uint32_t ao = tail / n_oo, oo = tail - ao * n_oo;
+  const int pair = g->scout_pair[k];
+  return (int64_t)(par * (uint32_t)g->n_off + ao * n_oo * (uint32_t)g->n_pair) + tile_position(g, (int)oo, pair);
 }
 
 // alpha / (1 - alpha) of the samples of one launch (by value in the kernel arguments)
@@ -1625,20 +1630,183 @@ __device__ __forceinline__ void load_terms(RowRegs &r, const double *__restrict_
 static_assert(MIST_T_S_LAYER_CK == 0 && MIST_T_D_LAST_NOCK == 11 && MIST_T_GCB < 32,
               "latency terms, then memory terms, are the first columns");
 
+// A row's part of GroupModel::bound as a linear form of a pair's layer counts, unrounded: 0.2 ppm of
+// every operand short, so that float32 rounding of x (6e-8 of the operands, with what the sums and
+// products lose) and of d / G (twice that) leave it below every objective of the row.
+// (values in, not references to members: a choice between those would put the struct into memory)
+__device__ __forceinline__ double choose(bool first, double a, double b) { return first ? a : b; }
+struct LinearBound {
+  double ck, nock;          // per checkpointed / other layer
+  double all_ck, none, mid; // first and last layer of a stage with c == l, c == 0, other c
+  __device__ __forceinline__ double at(double n_ck, double n_nock, bool is_all, bool is_none) const {
+    return __builtin_fma(n_ck, ck, __builtin_fma(n_nock, nock, choose(is_all, all_ck, choose(is_none, none, mid))));
+  }
+};
+constexpr double kLinearSlack = 2e-7;
+__device__ __forceinline__ LinearBound linear_bound(const RowRegs &t, double ratio, double inv_G) {
+  auto term = [&](int stable, int delta) {
+    const double x = ratio * t[stable], d = t[delta] * inv_G;
+    return __builtin_fma(-kLinearSlack, fabs(x), x) + __builtin_fma(-kLinearSlack, fabs(d), d);
+  };
+  const double first_ck = term(MIST_T_S_FIRST_CK, MIST_T_D_FIRST_CK), last_ck = term(MIST_T_S_LAST_CK, MIST_T_D_LAST_CK);
+  const double first_nock = term(MIST_T_S_FIRST_NOCK, MIST_T_D_FIRST_NOCK);
+  LinearBound b;
+  b.ck = term(MIST_T_S_LAYER_CK, MIST_T_D_LAYER_CK);
+  b.nock = term(MIST_T_S_LAYER_NOCK, MIST_T_D_LAYER_NOCK);
+  // (1e-40: float32 values below the normal range are rounded by up to 1e-45)
+  b.all_ck = first_ck + last_ck - 1e-40;
+  b.none = first_nock + term(MIST_T_S_LAST_NOCK, MIST_T_D_LAST_NOCK) - 1e-40;
+  b.mid = first_nock + last_ck - 1e-40;
+  return b;
+}
+
+// The scaled peaks at p = 0 and their steps in another order of operations than pair_memory (a few
+// 1e-16 off), for bounds of the counts: 1e-12 of the capacity of room covers that for every step, the
+// quotient is taken 1e-4 and 0.01 long as in count_upper.
+struct LinearMemory {
+  double fwd, bwd, pwg, po, pwgo, s_ck, s_nock, d_ck, d_nock, out2, mf_base, mf_pp;
+};
+__device__ __forceinline__ LinearMemory linear_memory(const RowRegs &t) {
+  LinearMemory r;
+  r.out2 = 2.0 * t[MIST_T_OUT];
+  r.fwd = t[MIST_T_FWD_STATES0] + t[MIST_T_FWD_PEAK] + t[MIST_T_GCB];
+  r.bwd = t[MIST_T_BWD_STATES0] + t[MIST_T_BWD_PEAK] + t[MIST_T_GCB] + r.out2;
+  r.pwg = t[MIST_T_PWG];
+  r.po = t[MIST_T_PO];
+  r.pwgo = t[MIST_T_PWGO];
+  r.s_ck = t[MIST_T_S_CK];
+  r.s_nock = t[MIST_T_S_NOCK];
+  r.d_ck = t[MIST_T_D_CK];
+  r.d_nock = t[MIST_T_D_NOCK];
+  r.mf_base = t[MIST_T_MF_BASE];
+  r.mf_pp = t[MIST_T_MF_PP];
+  return r;
+}
+__device__ __forceinline__ int count_bound(double m0, double step, int n, double cap_and_room) {
+  const double room = cap_and_room - m0;
+  const float most = __builtin_fmaf((float)room * __builtin_amdgcn_rcpf((float)step), 1.0001f, 0.01f);
+  const int count = most < (float)(n - 1) ? (int)most + 1 : n;  // (a step of 0: infinite, or not a number)
+  return room >= 0.0 ? count : 0;
+}
+// A pair's constants for them; wave-uniform.
+struct LinearPair {
+  int l, c;
+  bool all_ck, none;
+  double n_ck, n_nock;
+  __device__ __forceinline__ LinearPair(int layers, int ckpt) : l(layers), c(ckpt), all_ck(ckpt == layers), none(ckpt == 0) {
+    const int lm2 = max(l - 2, 0), ck = min(max(c - 1, 0), lm2);
+    n_ck = (double)ck;
+    n_nock = (double)(lm2 - ck);
+  }
+};
+// What they give of a row and a pair: bounds of the counts of base and with_pre, and the larger sums of
+// post_fits without the states of the post layer.
+struct LinearReach {
+  int count_b, count_p;
+  double post;
+};
+__device__ __forceinline__ LinearReach linear_reach(const LinearMemory &mem, const LinearPair &p, const GroupModel &m,
+                                                    int np, double cap_and_room) {
+  const double lf = (double)p.l, lm1 = (double)(p.l - 1);
+  double saved_now = lm1 * mem.s_ck, next = mem.s_ck, ck_delta = mem.d_ck;
+  if (!p.all_ck) {
+    saved_now = __builtin_fma((double)p.c, mem.s_ck, (double)(p.l - p.c - 1) * mem.s_nock);
+    next = mem.s_nock;
+  }
+  if (p.c < p.l - 1) ck_delta = mem.d_nock;
+  const double shared = saved_now + ck_delta, step = saved_now + next + mem.out2;
+  const double fwd = __builtin_fma(lf, mem.pwg, __builtin_fma(lm1, mem.po, mem.fwd));
+  const double bwd = __builtin_fma(lf, mem.pwgo, mem.bwd), peak = shared + fmax(fwd, bwd);
+  LinearReach r;
+  r.count_b = count_bound(peak * mem.mf_base, step * mem.mf_base, np, cap_and_room);
+  r.count_p = count_bound((peak + m.pre_sas) * mem.mf_pp, (step + m.pre_saved) * mem.mf_pp, np, cap_and_room);
+  r.post = shared + fmax(fwd, bwd - 0.5 * mem.out2 + m.post_output);
+  return r;
+}
+// Whether with_post or, in a pair of all layers, no_pp may fit (the latter's factor is the smaller one, MIST_T_MF).
+__device__ __forceinline__ bool post_may_fit(const LinearReach &r, const LinearMemory &mem, const LinearPair &p, int num_layers,
+                                             const GroupModel &m, double cap_and_room) {
+  const double factor = p.l == num_layers ? mem.mf_pp - (0.025 + 1e-9) : mem.mf_pp;
+  return (r.post + m.post_states) * factor <= cap_and_room;
+}
+
+// The largest minimum of every variant of a lane's pair: a row above all of them changes nothing
+// (the minima do not decrease with p; +inf while a slot is empty).
+struct Loosest {
+  double base, pre, post, pp;
+};
+// (`slots`: the pair's slots of one sample, `pitch` apart; a pair that is not `wanted` reads none)
+__device__ __forceinline__ Loosest loosest_minima(bool wanted, const double *slots, int pitch, int P, int count_b,
+                                                  int count_p, bool do_post, bool do_pp, double cutoff) {
+  Loosest t{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+  if (!wanted) return t;
+  const double base = slots[max(count_b - 1, 0) * pitch], pre = slots[(P + max(count_p - 1, 0)) * pitch];
+  const double post = slots[2 * P * pitch], pp = slots[(2 * P + 1) * pitch];
+  if (count_b > 0) t.base = fmin(base, cutoff);
+  if (count_p > 0) t.pre = fmin(pre, cutoff);
+  if (do_post) t.post = fmin(post, cutoff);
+  if (do_pp) t.pp = fmin(pp, cutoff);
+  return t;
+}
+// One threshold for GroupModel::bound that every row which could reach one of them passes: in two
+// parts, from the offsets of the group and with what a stage's post-layer terms add to the second.
+struct Threshold {
+  double front, post;  // base and with_pre; with_post and no_pp
+  __device__ __forceinline__ Threshold(const Loosest &t, const Offsets &group)
+      : front(fmax(t.base, t.pre - group.pre)), post(fmax(t.post - group.post, t.pp - group.pp)) {}
+  __device__ __forceinline__ double at(double post_layer) const { return fmax(front, post - post_layer); }
+};
+
 // ---- seeds ----
 __device__ __forceinline__ void clear_queue(const ReduceTables &tabs) {
   if (blockIdx.x == 0 && blockIdx.y == 0)
     for (int i = threadIdx.x; i < kCounters; i += blockDim.x) tabs.counter[i * kCounterPitch] = 0;
 }
 
+// Smallest linear bounds of 64 gathered rows at a time, for the seed launch: workgroup `part` of
+// `n_parts` of a group, a wavefront per 64 rows.
+__device__ __forceinline__ void gather_floors(const MistProblem &prob, const MistGroupDesc *__restrict__ g, int gi,
+                                              const double *__restrict__ row_terms, double ratio, double *gather_floor,
+                                              int part, int n_parts) {
+  if (g->scout_stride <= 0) return;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int waves = (int)blockDim.x / 64, n_gather = g->n_par * g->n_oo * g->n_ao * g->scout_stride;
+  const double inv_G = 1.0 / (double)g->grad_accum;
+  const double *__restrict__ src = row_terms + g->row_offset * MIST_ROW_TERMS;
+  for (int stage = part * waves + wave; stage < (n_gather + 63) / 64; stage += n_parts * waves) {
+    RowRegs t;
+    load_terms<0, MIST_T_D_LAST_NOCK + 1>(
+        t, src + gathered_position(g, (uint32_t)min(stage * 64 + lane, n_gather - 1)) * MIST_ROW_TERMS);
+    const LinearBound b = linear_bound(t, ratio, inv_G);
+    double low[kGatherFloor] = {b.ck, b.nock, b.all_ck, b.none, b.mid}, mine = 0.0;
+#pragma unroll
+    for (int i = 0; i < kGatherFloor; ++i) {
+      for (int step = 1; step < 64; step <<= 1) low[i] = fmin(low[i], __shfl_xor(low[i], step));
+      if (lane == i) mine = low[i];
+    }
+    if (lane < kGatherFloor) gather_floor[stage_floor_slot(g, gi, stage) * kGatherFloor + lane] = mine;
+  }
+}
+constexpr int kGatherBlocks = 16;  // workgroups per group
+__global__ __launch_bounds__(256) void gather_floor_kernel(const MistProblem prob, const MistGroupDesc *__restrict__ groups,
+                                                           const double *__restrict__ row_terms, double ratio,
+                                                           double *gather_floor) {
+  gather_floors(prob, groups + blockIdx.y, blockIdx.y, row_terms, ratio, gather_floor, blockIdx.x, gridDim.x);
+}
+
 // One sample.  Workgroup = (`pair_split` consecutive pairs of a tile, group) with their minima in
-// LDS.  A wavefront takes 64 gathered rows, lane = row with all its terms in registers, and runs
-// over the pairs: per (pair, variant) one look-up of the minimum at each row's own count; of the
-// rows below it the cheapest lowers the slots up to its count (lane = slot) and drops the rows it
+// LDS.  A wavefront takes 64 gathered rows: lane = pair, the smallest of their linear bounds against the
+// pair's loosest minima and the cutoff (of 22B on 16x8's 582000 times 16 pairs 86000 have one left, 0.9e6
+// pairs in all); then lane = row over those: the row's own bound, bounds of its counts against the minima
+// there, the reference's arithmetic.  Of the rows below the minimum at their
+// own count the cheapest lowers the slots up to its count (lane = slot) and drops the rows it
 // dominates, until none is left - a few steps from empty minima, none later.
 // (One LDS atomic per row at its own count, all rows of a stage at a few addresses: 0.96 ms for
-// the 7B plan; the register minima this replaced, one row after the other per lane: 0.42 ms.)
-__global__ __launch_bounds__(kSeedThreads) void seed_kernel(
+// the 7B plan; the register minima this replaced, one row after the other per lane: 0.42 ms; the
+// reference's latencies for every row and pair and its memory model below the cutoff, every row loaded
+// for every 16 pairs: 22B on 16x8 7.5e8 wave instructions, 5.7 ms beside the summaries, 70B on 32x8 1.95 ms; now
+// 2.4e8, 4.7 and 1.25.)
+__global__ __launch_bounds__(kSeedThreads, 3) void seed_kernel(
     const MistProblem prob, const MistGroupDesc *__restrict__ groups, const double *__restrict__ row_terms,
     double ratio, ReduceTables tabs, int pair_split) {
   extern __shared__ double lds_best[];
@@ -1658,46 +1826,73 @@ __global__ __launch_bounds__(kSeedThreads) void seed_kernel(
     constexpr int kWaves = kSeedThreads / 64;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const GroupModel m = group_model(prob, g);
-    const double cutoff = stage_cost_cutoff(prob, m.inv_G64);
+    const Offsets group = group_offsets(m, ratio);
+    const double cutoff = stage_cost_cutoff(prob, m.inv_G64), cap_and_room = m.cap * (1.0 + 1e-12);
     const int n_gather = g->n_par * g->n_oo * g->n_ao * g->scout_stride;
     const int n_stages = (n_gather + 63) / 64;
     // units of work: (stage, share of the pairs), more than one share when there are few stages
     const int shares = max(1, min(n_here, kWaves / n_stages)), per_share = (n_here + shares - 1) / shares;
     const double *__restrict__ src = row_terms + g->row_offset * MIST_ROW_TERMS;
+    // lane = pair of the workgroup
+    const int my_pair = min(lane, n_here - 1);
+    const PairIndex pc = decode_pair(first_pair + my_pair);
+    const int lc = pc.l | pc.c << 15, my_np = pc.c == pc.l - 1 ? min(P, 1) : P;
+    const LinearPair my_lp(pc.l, pc.c);
+    const int64_t floor_slot = stage_floor_slot(g, blockIdx.y, 0);
     for (int unit = wave; unit < n_stages * shares; unit += kWaves) {
       const int q = unit / shares * 64 + lane;
       const int i0 = unit % shares * per_share, i1 = min(i0 + per_share, n_here);
       const bool live = q < n_gather;
+      // what a row has to reach of the lane's pair (they fall while the loop runs), against the rows' bounds
+      const bool its_post = pc.c != pc.l - 1;
+      const double thr = Threshold(loosest_minima(true, lds_best + my_pair * n_slots, 1, P, my_np, my_np, its_post,
+                                                  its_post && pc.l == L, cutoff), group).at(0.0);
+      const double *__restrict__ f = tabs.gather_floor + (floor_slot + unit / shares) * kGatherFloor;
+      const LinearBound floor{f[0], f[1], f[2], f[3], f[4]};
+      uint64_t open = __ballot(lane >= i0 && lane < i1 &&
+                               floor.at(my_lp.n_ck, my_lp.n_nock, my_lp.all_ck, my_lp.none) <= thr);
+      if (open == 0) continue;
+      const double *__restrict__ my_row = src + gathered_position(g, (uint32_t)min(q, n_gather - 1)) * MIST_ROW_TERMS;
       RowRegs t;
-      load_terms<0, MIST_ROW_TERMS>(t, src + gathered_position(g, min(q, n_gather - 1)) * MIST_ROW_TERMS);
-      const PairIndex pc = decode_pair(first_pair + min(i0, n_here - 1));
-      int l = __builtin_amdgcn_readfirstlane(pc.l), c = __builtin_amdgcn_readfirstlane(pc.c);
-      for (int i = i0; i < i1; ++i, c = c < l ? c + 1 : (++l, 0)) {
-        const PairConsts k = pair_consts(l, c);
+      load_terms<0, MIST_T_D_LAST_NOCK + 1>(t, my_row);
+      const LinearBound bound = linear_bound(t, ratio, m.inv_G64);
+      LinearMemory memory = {};
+      bool have_rest = false;
+      for (; open != 0; open &= open - 1) {
+        const int i = __ffsll((unsigned long long)open) - 1;
+        const int its = from_lane(lc, i), l = its & 0x7fff, c = its >> 15;
+        const LinearPair p(l, c);
+        const double low = bound.at(p.n_ck, p.n_nock, p.all_ck, p.none);
+        const bool wanted = live && low <= from_lane(thr, i);
+        if (!__any(wanted)) continue;
+        if (!have_rest) {
+          load_terms<MIST_T_D_LAST_NOCK + 1, MIST_ROW_TERMS>(t, my_row);
+          memory = linear_memory(t);
+          have_rest = true;
+        }
         // Cells with c == l - 1 are only kept for p == 0 of the base / with_pre variants
         // (batched_module_analyzer.py:3021-3023, 3103).
         const int np = c == l - 1 ? min(P, 1) : P;
         const bool do_post = c != l - 1, do_pp = do_post && l == L;
-        float x, d;
-        pair_latency(t, k, x, d);
-        // (under a bound most rows are above it and need no memory model)
-        const bool wanted =
-            live && (cutoff == INFINITY || m.bound(ratio, x, d) <= cutoff);
-        if (!__any(wanted)) continue;
-        const LaneMemory mem = pair_memory(t, k);
         double *mine = lds_best + i * n_slots;
-        const Objectives o = objectives(t, x, d, k.no_ck, ratio, m, do_post);
         // the minima do not decrease with p: at the bound of its count a row meets the largest one
         // it could beat
-        const UpperCounts upper = upper_counts(mem, m, wanted ? np : 0);
-        auto may = [&](int count, double cost, const double *slots) {
-          return count > 0 && cost < slots[max(count - 1, 0)];
-        };
-        const bool may_b = may(upper.b, o.base, mine), may_p = may(upper.p, o.pre, mine + P);
-        const bool may_post = do_post && may(wanted, o.post, mine + 2 * P);
-        const bool may_pp = do_pp && may(wanted, o.pp, mine + 2 * P + 1);
-        if (!__any(may_b || may_p || may_post || may_pp)) continue;
-        const RowCounts cnt = exact_counts(mem, m, may_b ? upper.b : 0, may_p ? upper.p : 0);
+        const LinearReach reach = linear_reach(memory, p, m, np, cap_and_room);
+        bool may = (reach.count_b > 0 && low < mine[max(reach.count_b - 1, 0)]) ||
+                   (reach.count_p > 0 && low + group.pre < mine[P + max(reach.count_p - 1, 0)]);
+        if (do_post) {
+          const double post = do_pp ? fmax(mine[2 * P] - group.post, mine[2 * P + 1] - group.pp) : mine[2 * P] - group.post;
+          may = may || (low < post && post_may_fit(reach, memory, p, L, m, cap_and_room));
+        }
+        may = may && wanted;
+        if (!__any(may)) continue;
+        const PairConsts k = pair_consts(l, c);
+        float x, d;
+        pair_latency(t, k, x, d);
+        const LaneMemory mem = pair_memory(t, k);
+        const Objectives o = objectives(t, x, d, k.no_ck, ratio, m, do_post);
+        const UpperCounts upper = upper_counts(mem, m, may ? np : 0);
+        const RowCounts cnt = exact_counts(mem, m, upper.b, upper.p);
         bool ok_post = false, ok_pp = false;
         if (do_post) post_fits(t, k, mem, m, mem.out, k.no_ck ? t[MIST_T_RD] : 0.0, ok_post, ok_pp);
         auto offer = [&](int count, double cost, double *slots) {
@@ -1712,8 +1907,8 @@ __global__ __launch_bounds__(kSeedThreads) void seed_kernel(
         };
         offer(cnt.b, o.base, mine);
         offer(cnt.p, o.pre, mine + P);
-        if (do_post) offer(wanted && ok_post ? 1 : 0, o.post, mine + 2 * P);
-        if (do_pp) offer(wanted && ok_pp ? 1 : 0, o.pp, mine + 2 * P + 1);
+        if (do_post) offer(may && ok_post ? 1 : 0, o.post, mine + 2 * P);
+        if (do_pp) offer(may && ok_pp ? 1 : 0, o.pp, mine + 2 * P + 1);
       }
     }
   }
@@ -1806,7 +2001,7 @@ __global__ __launch_bounds__(64) void seed_samples_kernel(
     for (int q0 = 0; q0 < n_gather; q0 += 64) {
       const int n_rows = min(64, n_gather - q0);
       RowRegs t;
-      load_terms<0, MIST_ROW_TERMS>(t, src + gathered_position(g, min(q0 + lane, n_gather - 1)) * MIST_ROW_TERMS);
+      load_terms<0, MIST_ROW_TERMS>(t, src + gathered_position(g, (uint32_t)min(q0 + lane, n_gather - 1)) * MIST_ROW_TERMS);
       float x, d;
       pair_latency(t, k, x, d);
       const LaneMemory mem = pair_memory(t, k);
@@ -1883,33 +2078,6 @@ __global__ __launch_bounds__(256) void super_floor_kernel(const MistGroupDesc *_
     if (tabs.listed != nullptr && col < n) tabs.stage_flag[stage_floor_slot(g, gi, super * kSuperStages) + col] = 0;
   }
 }
-
-// The largest minimum of every variant of a lane's pair: a row above all of them changes nothing
-// (the minima do not decrease with p; +inf while a slot is empty).
-struct Loosest {
-  double base, pre, post, pp;
-};
-// (`slots`: the pair's slots of one sample, `pitch` apart; a pair that is not `wanted` reads none)
-__device__ __forceinline__ Loosest loosest_minima(bool wanted, const double *slots, int pitch, int P, int count_b,
-                                                  int count_p, bool do_post, bool do_pp, double cutoff) {
-  Loosest t{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
-  if (!wanted) return t;
-  const double base = slots[max(count_b - 1, 0) * pitch], pre = slots[(P + max(count_p - 1, 0)) * pitch];
-  const double post = slots[2 * P * pitch], pp = slots[(2 * P + 1) * pitch];
-  if (count_b > 0) t.base = fmin(base, cutoff);
-  if (count_p > 0) t.pre = fmin(pre, cutoff);
-  if (do_post) t.post = fmin(post, cutoff);
-  if (do_pp) t.pp = fmin(pp, cutoff);
-  return t;
-}
-// One threshold for GroupModel::bound that every row which could reach one of them passes: in two
-// parts, from the offsets of the group and with what a stage's post-layer terms add to the second.
-struct Threshold {
-  double front, post;  // base and with_pre; with_post and no_pp
-  __device__ __forceinline__ Threshold(const Loosest &t, const Offsets &group)
-      : front(fmax(t.base, t.pre - group.pre)), post(fmax(t.post - group.post, t.pp - group.pp)) {}
-  __device__ __forceinline__ double at(double post_layer) const { return fmax(front, post - post_layer); }
-};
 
 // Lane = pair against a stage summary: the counts its pseudo row allows, hence which minima a row
 // of the stage can reach, and the bound that its objective gives.
@@ -2243,65 +2411,6 @@ __global__ __launch_bounds__(kTermsBlock) void stage_rows_kernel(
 }
 
 // ---- reduce / resolve ----
-// A row's part of GroupModel::bound as a linear form of a pair's layer counts, unrounded: 0.2 ppm of
-// every operand short, so that float32 rounding of x (6e-8 of the operands, with what the sums and
-// products lose) and of d / G (twice that) leave it below every objective of the row.
-// (values in, not references to members: a choice between those would put the struct into memory)
-__device__ __forceinline__ double choose(bool first, double a, double b) { return first ? a : b; }
-struct LinearBound {
-  double ck, nock;          // per checkpointed / other layer
-  double all_ck, none, mid; // first and last layer of a stage with c == l, c == 0, other c
-  __device__ __forceinline__ double at(double n_ck, double n_nock, bool is_all, bool is_none) const {
-    return __builtin_fma(n_ck, ck, __builtin_fma(n_nock, nock, choose(is_all, all_ck, choose(is_none, none, mid))));
-  }
-};
-constexpr double kLinearSlack = 2e-7;
-__device__ __forceinline__ LinearBound linear_bound(const RowRegs &t, double ratio, double inv_G) {
-  auto term = [&](int stable, int delta) {
-    const double x = ratio * t[stable], d = t[delta] * inv_G;
-    return __builtin_fma(-kLinearSlack, fabs(x), x) + __builtin_fma(-kLinearSlack, fabs(d), d);
-  };
-  const double first_ck = term(MIST_T_S_FIRST_CK, MIST_T_D_FIRST_CK), last_ck = term(MIST_T_S_LAST_CK, MIST_T_D_LAST_CK);
-  const double first_nock = term(MIST_T_S_FIRST_NOCK, MIST_T_D_FIRST_NOCK);
-  LinearBound b;
-  b.ck = term(MIST_T_S_LAYER_CK, MIST_T_D_LAYER_CK);
-  b.nock = term(MIST_T_S_LAYER_NOCK, MIST_T_D_LAYER_NOCK);
-  // (1e-40: float32 values below the normal range are rounded by up to 1e-45)
-  b.all_ck = first_ck + last_ck - 1e-40;
-  b.none = first_nock + term(MIST_T_S_LAST_NOCK, MIST_T_D_LAST_NOCK) - 1e-40;
-  b.mid = first_nock + last_ck - 1e-40;
-  return b;
-}
-
-// The scaled peaks at p = 0 and their steps in another order of operations than pair_memory (a few
-// 1e-16 off), for bounds of the counts: 1e-12 of the capacity of room covers that for every step, the
-// quotient is taken 1e-4 and 0.01 long as in count_upper.
-struct LinearMemory {
-  double fwd, bwd, pwg, po, pwgo, s_ck, s_nock, d_ck, d_nock, out2, mf_base, mf_pp;
-};
-__device__ __forceinline__ LinearMemory linear_memory(const RowRegs &t) {
-  LinearMemory r;
-  r.out2 = 2.0 * t[MIST_T_OUT];
-  r.fwd = t[MIST_T_FWD_STATES0] + t[MIST_T_FWD_PEAK] + t[MIST_T_GCB];
-  r.bwd = t[MIST_T_BWD_STATES0] + t[MIST_T_BWD_PEAK] + t[MIST_T_GCB] + r.out2;
-  r.pwg = t[MIST_T_PWG];
-  r.po = t[MIST_T_PO];
-  r.pwgo = t[MIST_T_PWGO];
-  r.s_ck = t[MIST_T_S_CK];
-  r.s_nock = t[MIST_T_S_NOCK];
-  r.d_ck = t[MIST_T_D_CK];
-  r.d_nock = t[MIST_T_D_NOCK];
-  r.mf_base = t[MIST_T_MF_BASE];
-  r.mf_pp = t[MIST_T_MF_PP];
-  return r;
-}
-__device__ __forceinline__ int count_bound(double m0, double step, int n, double cap_and_room) {
-  const double room = cap_and_room - m0;
-  const float most = __builtin_fmaf((float)room * __builtin_amdgcn_rcpf((float)step), 1.0001f, 0.01f);
-  const int count = most < (float)(n - 1) ? (int)most + 1 : n;  // (a step of 0: infinite, or not a number)
-  return room >= 0.0 ? count : 0;
-}
-
 // One item with the pairs in `pairs`, one sample.  Returns the pairs in which some row reached its
 // minimum (kResolve: unused).
 //   lane = pair   the slots the stage's pseudo row can reach, and with their minima a threshold;
@@ -2363,27 +2472,14 @@ __device__ __forceinline__ uint64_t reduce_item(const MistProblem &prob, const M
     load_terms<0, MIST_T_D_LAST_NOCK + 1>(t, rows + min(lane, n_stage - 1) * MIST_ROW_TERMS);
     bound = linear_bound(t, ratio, m.inv_G64);
   }
-  struct Pair {  // wave-uniform
-    int l, c;
-    bool all_ck, none;
-    double n_ck, n_nock;
-  };
   auto pair_at = [&](int pl) {
-    Pair p;
     const int its = from_lane(lc, pl);
-    p.l = its & 0x7fff;
-    p.c = its >> 15;
-    const int lm2 = max(p.l - 2, 0), n_ck = min(max(p.c - 1, 0), lm2);
-    p.n_ck = (double)n_ck;
-    p.n_nock = (double)(lm2 - n_ck);
-    p.all_ck = p.c == p.l;
-    p.none = p.c == 0;
-    return p;
+    return LinearPair(its & 0x7fff, its >> 15);
   };
   uint64_t left = 0;  // pairs with rows below their threshold
   for (uint64_t rest = todo; rest != 0; rest &= rest - 1) {
     const int pl = __ffsll((unsigned long long)rest) - 1;
-    const Pair p = pair_at(pl);
+    const LinearPair p = pair_at(pl);
     const uint64_t pass = live & __ballot(bound.at(p.n_ck, p.n_nock, p.all_ck, p.none) <= from_lane(thr, pl));
     left |= pass != 0 ? 1ull << pl : 0ull;
   }
@@ -2477,31 +2573,15 @@ __device__ __forceinline__ uint64_t reduce_item(const MistProblem &prob, const M
       settle(pl);
       rest &= rest - 1;
       if (rest != 0) fetch(__ffsll((unsigned long long)rest) - 1);
-      const Pair p = pair_at(pl);
+      const LinearPair p = pair_at(pl);
       const double low = bound.at(p.n_ck, p.n_nock, p.all_ck, p.none);
-      const double lf = (double)p.l, lm1 = (double)(p.l - 1);
-      double saved_now = lm1 * mem.s_ck, next = mem.s_ck, ck_delta = mem.d_ck;
-      if (!p.all_ck) {
-        saved_now = __builtin_fma((double)p.c, mem.s_ck, (double)(p.l - p.c - 1) * mem.s_nock);
-        next = mem.s_nock;
-      }
-      if (p.c < p.l - 1) ck_delta = mem.d_nock;
-      const double shared = saved_now + ck_delta, step = saved_now + next + mem.out2;
-      const double fwd = __builtin_fma(lf, mem.pwg, __builtin_fma(lm1, mem.po, mem.fwd));
-      const double bwd = __builtin_fma(lf, mem.pwgo, mem.bwd), peak = shared + fmax(fwd, bwd);
-      const int np = p.c == p.l - 1 ? min(P, 1) : P;
-      const int upper_b = count_bound(peak * mem.mf_base, step * mem.mf_base, np, cap_and_room);
-      const int upper_p = count_bound((peak + m.pre_sas) * mem.mf_pp, (step + m.pre_saved) * mem.mf_pp, np, cap_and_room);
+      const LinearReach reach = linear_reach(mem, p, m, p.c == p.l - 1 ? min(P, 1) : P, cap_and_room);
       auto minimum = [&](int slot) { return kInLds ? lds_row[slot] : best[(int64_t)pl * n_slots + slot]; };
-      const double now_b = minimum(max(upper_b - 1, 0)), now_p = minimum(P + max(upper_p - 1, 0));
-      bool may = (upper_b > 0 && low <= fmin(now_b, cutoff)) || (upper_p > 0 && low <= fmin(now_p, cutoff) - off_pre);
+      const double now_b = minimum(max(reach.count_b - 1, 0)), now_p = minimum(P + max(reach.count_p - 1, 0));
+      bool may = (reach.count_b > 0 && low <= fmin(now_b, cutoff)) ||
+                 (reach.count_p > 0 && low <= fmin(now_p, cutoff) - off_pre);
       const bool may_post = low <= from_lane(thr_post, pl);
-      if (__any(may_post)) {  // a pair in seven
-        // the larger ones of post_fits' sums (a single stage's factor is the smaller one, MIST_T_MF)
-        const double post = shared + fmax(fwd, bwd - 0.5 * mem.out2 + m.post_output);
-        const double factor = p.l == L ? mem.mf_pp - (0.025 + 1e-9) : mem.mf_pp;
-        may = may || (may_post && (post + m.post_states) * factor <= cap_and_room);
-      }
+      if (__any(may_post)) may = may || (may_post && post_may_fit(reach, mem, p, L, m, cap_and_room));  // a pair in seven
       const uint64_t found = live & __ballot(may && low <= from_lane(thr, pl));
       if (found >> lane & 1ull)
         queue[waiting + __popcll(found & ((1ull << lane) - 1ull))] = (uint16_t)(pl << 6 | lane);
@@ -3025,8 +3105,12 @@ __device__ __forceinline__ bool estimate_runs(const MistProblem &prob, const Mis
 
 __global__ __launch_bounds__(256) void estimate_stage_minima_kernel(
     const MistProblem prob, const MistGroupDesc *__restrict__ groups,
-    const double *__restrict__ row_terms, double ratio, double *__restrict__ partial_cost) {
+    const double *__restrict__ row_terms, double ratio, double *__restrict__ partial_cost, double *gather_floor) {
   const MistGroupDesc *g = groups + blockIdx.y;
+  if (blockIdx.x >= kEstimateSplit) {  // (what the seed launch wants next needs no launch of its own)
+    gather_floors(prob, g, blockIdx.y, row_terms, ratio, gather_floor, blockIdx.x - kEstimateSplit, kGatherBlocks);
+    return;
+  }
   int S;
   if (!estimate_runs(prob, g, &S)) return;
   const int L = prob.num_layers, l = L / S, rule = prob.incumbent_ckpt_rule;
@@ -3050,7 +3134,7 @@ __global__ __launch_bounds__(256) void estimate_stage_minima_kernel(
       atomicMin(&stage_min[st], (unsigned long long)__double_as_longlong(cost));
   };
   for (int64_t item = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; item < n_items;
-       item += (int64_t)gridDim.x * blockDim.x) {
+       item += (int64_t)kEstimateSplit * blockDim.x) {
     const int c = (int)(item % (l + 1));
     const int64_t q = item / (l + 1);
     const int64_t tail = q / per_tail, rest = q - tail * per_tail;
@@ -3058,7 +3142,7 @@ __global__ __launch_bounds__(256) void estimate_stage_minima_kernel(
     if (rule == 2 && c != l) continue;  // every layer of a stage checkpointed
     if (c == l - 1) continue;  // kept at p == 0 of base / with_pre only, which no stage below reads
     const double *__restrict__ t =
-        src + gathered_position(g, pair * per_pair + par * n_tail + tail) * MIST_ROW_TERMS;
+        src + gathered_position(g, (uint32_t)(pair * per_pair + par * n_tail + tail)) * MIST_ROW_TERMS;
     const CellLatency lat = cell_latency<true>(t, l, c, k);
     const LaneMemory mem = cell_memory(t, l, c);
     // largest ckpt count of the stage that ends with layer end_layer (rule of the caller's search)
@@ -3581,9 +3665,10 @@ int64_t mist_stage_floor_doubles(int64_t total_rows, int n_groups) {
 }
 
 // Sections of the reduce workspace in `d_partial_cost` (doubles): the minima of n_samples samples,
-// the second-level summaries, the four lists, their counters, a word per stage and one per pair.
+// the second-level summaries, the four lists, their counters, a word per stage and one per pair, the
+// bounds of the gathered rows.
 struct WorkspaceLayout {
-  int64_t best, supers, items, counters, flags, changed, total;
+  int64_t best, supers, items, counters, flags, changed, gathered, total;
   int64_t capacity;  // items per shard
 };
 static WorkspaceLayout workspace_layout(int64_t cells, int64_t supers, int64_t items, int n_samples) {
@@ -3595,7 +3680,8 @@ static WorkspaceLayout workspace_layout(int64_t cells, int64_t supers, int64_t i
   w.counters = w.items + 4 * kQueueShards * w.capacity;
   w.flags = w.counters + kCounters * kCounterPitch / 2;
   w.changed = w.flags + supers * kSuperStages / 2;
-  w.total = w.changed + cells / 8 + 1;
+  w.gathered = w.changed + cells / 8 + 1;
+  w.total = w.gathered + supers * kSuperStages * kGatherFloor;  // (a batch of samples may end with one alone)
   return w;
 }
 int64_t mist_reduce_workspace_doubles(int64_t cells, int64_t supers, int64_t items, int n_samples) {
@@ -3621,6 +3707,7 @@ static int reduce_tables(const MistProblem *problem, int n_samples, double *d_pa
   out->stage_flag = reinterpret_cast<uint32_t *>(d_partial_cost + w.flags);
   out->counter = reinterpret_cast<uint32_t *>(d_partial_cost + w.counters);
   out->changed = reinterpret_cast<uint32_t *>(d_partial_cost + w.changed);
+  out->gather_floor = d_partial_cost + w.gathered;
   out->capacity = (uint32_t)w.capacity;
   out->n_samples = n_samples;
   return 0;
@@ -3628,9 +3715,9 @@ static int reduce_tables(const MistProblem *problem, int n_samples, double *d_pa
 
 static int launch_first_estimate(const MistProblem *problem, const MistGroupDesc *d_groups, int n_groups,
                                  const double *d_row_terms, double ratio, double *d_partial_cost,
-                                 void *stream) {
-  hipLaunchKernelGGL(estimate_stage_minima_kernel, dim3(kEstimateSplit, n_groups), dim3(256), 0,
-                     (hipStream_t)stream, *problem, d_groups, d_row_terms, ratio, d_partial_cost);
+                                 double *gather_floor, void *stream) {
+  hipLaunchKernelGGL(estimate_stage_minima_kernel, dim3(kEstimateSplit + (gather_floor ? kGatherBlocks : 0), n_groups),
+                     dim3(256), 0, (hipStream_t)stream, *problem, d_groups, d_row_terms, ratio, d_partial_cost, gather_floor);
   MIST_HIP_CHECK(hipGetLastError());
   hipLaunchKernelGGL(estimate_combine_kernel, dim3(n_groups), dim3(64), 0, (hipStream_t)stream,
                      *problem, d_groups, d_partial_cost);
@@ -3667,11 +3754,6 @@ static int allow_large_lds() {
 static int launch_seeds(const MistProblem *problem, const MistGroupDesc *d_groups, int n_groups,
                         const double *d_row_terms, const RatioList &ratios, bool scouted,
                         const ReduceTables &tabs, double *d_partial_cost, void *stream) {
-  if (scouted && problem->stage_cost_incumbent != nullptr && problem->incumbent_first_estimate != 0 &&
-      tabs.n_samples == 1)
-    // a first estimate from a few rows, so that the seed launch itself runs under a bound
-    if (int rc = launch_first_estimate(problem, d_groups, n_groups, d_row_terms, ratios.r[0], d_partial_cost, stream))
-      return rc;
   const int L = problem->num_layers, n_pairs = L * (L + 1) / 2 + L;
   const int tiles = (n_pairs + MIST_LC_TILE - 1) / MIST_LC_TILE;
   if (tiles > 1 << kItemTileBits)
@@ -3680,11 +3762,23 @@ static int launch_seeds(const MistProblem *problem, const MistGroupDesc *d_group
   // fewer pairs, or samples, per workgroup when the slots are many, so that several stay resident
   int pair_split = tabs.n_samples == 1 ? 16 : 1;
   while (pair_split > 1 && pair_split * pair_bytes > kSeedLdsBytes) pair_split /= 2;
+  // ... and where there would be fewer than eight workgroups per CU (16, 8 and 4 pairs: stage operator of 7B on
+  // 2x8, one group, 106, 65, 40 us; uniform-pp of 7B on 2x8 beside the summaries 123, 85, 146; the 7B plan on
+  // 4x8, 72 groups, 257, 255, 259; 70B on 32x8, 120 groups, 1250, 1490, 1930)
+  while (pair_split > 4 && (int64_t)tiles * (MIST_LC_TILE / pair_split) * n_groups < kSeedWorkgroups) pair_split /= 2;
   int sample_split = tabs.n_samples;
   while (sample_split > 1 && pair_bytes * sample_split > kSeedLdsBytes) sample_split = (sample_split + 1) / 2;
   const int64_t bytes =
       pair_bytes * pair_split * sample_split + (tabs.n_samples == 1 ? 0 : (int64_t)sizeof(SampleRows));
-  if (!scouted || bytes > kSeedLdsMost) {  // (some 10000 values of p)
+  const bool seeds = scouted && bytes <= kSeedLdsMost;  // (some 10000 values of p)
+  const bool estimate = scouted && problem->stage_cost_incumbent != nullptr && problem->incumbent_first_estimate != 0 &&
+                        tabs.n_samples == 1;
+  // a first estimate from a few rows, so that the seed launch itself runs under a bound
+  if (estimate)
+    if (int rc = launch_first_estimate(problem, d_groups, n_groups, d_row_terms, ratios.r[0], d_partial_cost,
+                                       seeds ? tabs.gather_floor : nullptr, stream))
+      return rc;
+  if (!seeds) {
     hipLaunchKernelGGL(empty_minima_kernel, dim3(kReduceBlocks), dim3(256), 0, (hipStream_t)stream, tabs,
                        problem->reduce_cells);
     MIST_HIP_CHECK(hipGetLastError());
@@ -3692,6 +3786,11 @@ static int launch_seeds(const MistProblem *problem, const MistGroupDesc *d_group
   }
   if (bytes > 64 * 1024)
     if (int rc = allow_large_lds()) return rc;
+  if (tabs.n_samples == 1 && !estimate) {
+    hipLaunchKernelGGL(gather_floor_kernel, dim3(kGatherBlocks, n_groups), dim3(256), 0, (hipStream_t)stream, *problem,
+                       d_groups, d_row_terms, ratios.r[0], tabs.gather_floor);
+    MIST_HIP_CHECK(hipGetLastError());
+  }
   const dim3 grid(tiles * (MIST_LC_TILE / pair_split), n_groups,
                   (tabs.n_samples + sample_split - 1) / sample_split);
   if (tabs.n_samples == 1)
@@ -3809,7 +3908,7 @@ int mist_stage_cost_first_estimate(const MistProblem *problem, const MistGroupDe
     return fail(MIST_E_INVALID, "no stage-cost incumbent to lower");
   if (n_groups > 65535) return fail(MIST_E_INVALID, "at most 65535 groups per call, got %d", n_groups);
   if (!(ratio >= 0.0)) return fail(MIST_E_INVALID, "ratio must be non-negative");
-  return launch_first_estimate(problem, d_groups, n_groups, d_row_terms, ratio, d_partial_cost, stream);
+  return launch_first_estimate(problem, d_groups, n_groups, d_row_terms, ratio, d_partial_cost, nullptr, stream);
 }
 
 static int launch_finalize(const MistProblem *problem, const MistGroupDesc *d_groups, int n_groups,
