@@ -18,10 +18,12 @@
 #include <map>
 #include <tuple>
 #include <mutex>
+#include <type_traits>
 #include <utility>
 
 #include "mist_common.h"
 #include "mist_dp.h"
+#include "mist_dp_rates.h"
 
 namespace {
 
@@ -606,8 +608,10 @@ __device__ __forceinline__ void dp_finish_winner(DpBest &w, const MistDpShape &s
 // with the layers split freely: a recurrence over (stage count, start layer) alone,
 //   B(s, k) = min over i >= k of max(cost(s, k, i, q), B(s - 1, i + 1)),
 // one wavefront per mesh, its two rows of B in `rows` (LDS, 2 (L + 1) of its `n_rows` floats per
-// wavefront).  Called by the whole workgroup; `slot` is one int of LDS.  +inf when no such
+// wavefront), kDpBoundLoads costs of a lane in flight (one at a time: 34 us of a bottleneck instance
+// of the 7B plan, 364 of 70B on 32x8; 16 at a time about half of it).  Called by the whole workgroup; `slot` is one int of LDS.  +inf when no such
 // partition is feasible (or L > 128: a lane holds two start layers; or `rows` is too small).
+constexpr int kDpBoundLoads = 16;
 __device__ __forceinline__ float dp_uniform_mesh_bound(const MistDpShape &shape,
                                                        const float *__restrict__ relaid,
                                                        float *rows, int n_rows, int32_t *slot) {
@@ -638,7 +642,14 @@ __device__ __forceinline__ float dp_uniform_mesh_bound(const MistDpShape &shape,
           if (k <= L - s) {
             const float *__restrict__ row = block + dp_triangle_row(L, k) - k;  // row[i]
             // the s - 1 stages behind this one take a layer each at least
-            for (int i = k; i <= L - s; ++i) best = fminf(best, fmaxf(row[i], prev[i + 1]));
+            for (int i0 = k; i0 <= L - s; i0 += kDpBoundLoads) {
+              float cost[kDpBoundLoads];
+#pragma unroll
+              for (int u = 0; u < kDpBoundLoads; ++u) cost[u] = row[min(i0 + u, L - s)];
+#pragma unroll
+              for (int u = 0; u < kDpBoundLoads; ++u)
+                best = fminf(best, fmaxf(cost[u], prev[min(i0 + u, L - s) + 1]));
+            }
           }
           cur[k] = best;
         }
@@ -1248,15 +1259,75 @@ __global__ __launch_bounds__(kDpPlaneThreads) void dp_plane_kernel(
 // instances) 13.2 -> 5.2 ms, 48 x 128 (600) 2.9 -> 0.7 ms, 40 x 64 1.06 -> 0.40 ms, 32 x 32 0.32 ->
 // 0.20 ms; bottleneck batches of 40-48 instances 2.2 -> 1.65, 0.67 -> 0.26, 0.33 -> 0.16 and 0.16 ->
 // 0.11 ms.
+//   An instance ends when no larger stage count can improve its answer (`rates` given, no cost of its
+// g negative): a pipeline of more than s stages ends with s stages that are some state (k, d) of
+// F(s), and those in front of it put k >= 1 layers on D - d devices.  With rate = the smallest cost x
+// devices / layers of a stage they sum to no less than rate k / (D - d), and the largest of them is
+// no less than that either.  float32 additions of costs that are not negative lose at most 2^-24 of the
+// sum each, the bound is taken 1.2e-7 short for every layer.  Stage counts of all instances of a search,
+// without -> with: 40 x 64 10700 -> 3000, 48 x 128 15300 -> 6300.  And columns of F(s) are the multiples of
+// the greatest common divisor of the meshes that hold an admissible stage (80 x 256: 64 or fewer columns
+// for most instances, a quarter of the LDS reads).  Threshold batches of a search 80 x 256 5.6 -> 2.1 ms, 48 x
+// 128 0.85 -> 0.44, 40 x 64 0.42 -> 0.29; what is left are instances whose answer has many stages (16 or 32
+// steps in turn, of 300 VALU instructions per start layer), and their launches end with the longest.
 // ------------------------------------------------------------------------------------------
 constexpr int kDpHistoryThreads = 1024;
-constexpr int kDpHistoryBatch = 8;   // meshes whose row minima a lane has in flight
+constexpr int kDpHistoryBatch = 10;  // meshes whose row minima a lane has in flight
 constexpr int kDpUnreached = 1 << 20;
 // LDS of a workgroup: F(s - 1), the smallest reached device count per row (two steps), the stage
-// values of the answer's path, three flags
+// values of the answer's path, three flags, three bounds, the answer
 inline size_t dp_history_lds(int L, int D, int max_stages) {
   const size_t f = std::max((size_t)(L - 1) * D, (size_t)(kDpHistoryThreads / 64) * 2 * (L + 1));
-  return (f + 2 * (size_t)L + (size_t)max_stages + 3) * sizeof(float);
+  return (f + 2 * (size_t)L + (size_t)max_stages + 7) * sizeof(float);
+}
+
+// Over the re-laid row minima of every g, for dp_history_kernel: the smallest stage cost x devices / layers,
+// negative where some cost is, and the smallest cost on every mesh.  out[g][1 + Q], +inf before the
+// launch; workgroup = (share of the stage counts, mesh, g).
+constexpr int kRateShares = 4;
+__global__ __launch_bounds__(256) void stage_rate_kernel(const MistDpShape shape, const float *__restrict__ stage_min,
+                                                         int64_t g_stride, float *__restrict__ out) {
+  __shared__ float lds[2][4];
+  const int L = shape.num_layers, tri = dp_triangle(L), q = blockIdx.y;
+  const float *__restrict__ in = stage_min + blockIdx.z * g_stride + (int64_t)q * tri;
+  const float rows = 2.0f * (float)L + 1.0f;
+  float per_layer = INFINITY, least = INFINITY;
+  for (int x = threadIdx.x; x < tri; x += 256) {
+    int k = (int)((rows - __builtin_amdgcn_sqrtf(fmaxf(rows * rows - 8.0f * (float)x, 0.0f))) * 0.5f);
+    k = min(max(k, 0), L - 1);
+    while (dp_triangle_row(L, k) > x) --k;
+    while (k < L - 1 && dp_triangle_row(L, k + 1) <= x) ++k;
+    float cost = INFINITY;
+#pragma unroll 4
+    for (int p = blockIdx.x; p < shape.max_stages; p += kRateShares) cost = fminf(cost, in[(int64_t)p * shape.num_mesh * tri + x]);
+    least = fminf(least, cost);
+    per_layer = fminf(per_layer, cost / (float)(x - dp_triangle_row(L, k) + 1));
+  }
+  for (int step = 1; step < 64; step <<= 1) {
+    per_layer = fminf(per_layer, __shfl_xor(per_layer, step));
+    least = fminf(least, __shfl_xor(least, step));
+  }
+  if ((threadIdx.x & 63) == 0) {
+    lds[0][threadIdx.x >> 6] = per_layer;
+    lds[1][threadIdx.x >> 6] = least;
+  }
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    float low = fminf(fminf(lds[threadIdx.x][0], lds[threadIdx.x][1]), fminf(lds[threadIdx.x][2], lds[threadIdx.x][3]));
+    if (threadIdx.x == 0) low *= (float)(shape.mesh_n[q] * shape.mesh_m[q]);
+    // (as integers: those of positive floats are in their order, and a negative one is below them all)
+    if (low < INFINITY)
+      atomicMin(reinterpret_cast<int *>(out) + (int64_t)blockIdx.z * (1 + shape.num_mesh) + (threadIdx.x == 0 ? 0 : 1 + q),
+                __float_as_int(low));
+  }
+}
+__device__ __forceinline__ int greatest_common_divisor(int a, int b) {
+  while (b != 0) {
+    const int rest = a % b;
+    a = b;
+    b = rest;
+  }
+  return a;
 }
 
 // Cost of the stage k..i on mesh q, p pre-saved micro-batches, whose state has the value `best`
@@ -1303,21 +1374,23 @@ __device__ __forceinline__ void dp_write_stage(int32_t *at, int end, int n, int 
 template <bool kBottleneck, int kCols>
 __global__ __launch_bounds__(kDpHistoryThreads, 8) void dp_history_kernel(
     const MistDpShape shape, const MistDpCosts tabs, const float *__restrict__ tmax_list,
-    const int32_t *__restrict__ g_list, int n_instances, float *__restrict__ histories,
-    int32_t *__restrict__ best_s_out, float *__restrict__ best_sum_out,
+    const int32_t *__restrict__ g_list, int n_instances, const float *__restrict__ rates,
+    float *__restrict__ histories, int32_t *__restrict__ best_s_out, float *__restrict__ best_sum_out,
     float *__restrict__ stage_max_out, int32_t *__restrict__ path_out) {
   extern __shared__ float dp_lds[];
   const int L = shape.num_layers, D = shape.num_devices, Q = shape.num_mesh;
   const int S = shape.max_stages, plane = L * D, tri = dp_triangle(L);
   const int n_waves = kDpHistoryThreads / 64;
   const int n_f = max((L - 1) * D, n_waves * 2 * (L + 1));
-  float *f = dp_lds;  // F(s - 1) of row r >= 1, column c < D: f[(r - 1) * D + c]
+  float *f = dp_lds;  // F(s - 1) of row r >= 1, column c < W: f[(r - 1) * W + c]
   int32_t *first_col = reinterpret_cast<int32_t *>(dp_lds + n_f);  // [2][L]
   float *path_value = dp_lds + n_f + 2 * L;                        // [S]
   int32_t *reached = first_col + 2 * L + S;                        // [3]
+  int32_t *bound = reached + 3;  // [3]: float bits of the smallest bound of a state
+  float *answer = path_value + S + 6;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // F(s) of start layer k, d devices: history[(s - 1) * plane + k * D + d - 1]
+  // F(s) of start layer k, column c (from 1): history[(s - 1) * plane + k * W + c - 1]
   float *history = histories + (int64_t)blockIdx.x * S * plane;
   for (int t = blockIdx.x; t < n_instances; t += gridDim.x) {
     const int64_t g = g_list[t];
@@ -1337,7 +1410,22 @@ __global__ __launch_bounds__(kDpHistoryThreads, 8) void dp_history_kernel(
                             ? fminf(kDpNoThreshold, dp_uniform_mesh_bound(shape, relaid, f, n_f, reached))
                             : tmax_list[t];
     __syncthreads();  // (the bound was read by every wavefront)
-    if (threadIdx.x < 3) reached[threadIdx.x] = 0;
+    if (threadIdx.x < 3) {
+      reached[threadIdx.x] = 0;
+      bound[threadIdx.x] = __float_as_int(INFINITY);
+      *answer = INFINITY;
+    }
+    const float rate = rates != nullptr ? rates[g * (1 + Q)] : -1.0f;
+    const bool bounded = rate >= 0.0f && rate < INFINITY;
+    const float short_by = 1.0f - 1.2e-7f * (float)(L + 8);
+    // stages take whole multiples of `unit` devices: a state's column is d / unit - 1, of W
+    int unit = rates != nullptr ? D : 1;
+    for (int q = 0; rates != nullptr && q < Q; ++q)
+      if (rates[g * (1 + Q) + 1 + q] <= t_max) unit = greatest_common_divisor(unit, shape.mesh_n[q] * shape.mesh_m[q]);
+    const int W = D / unit;
+    // lane = mesh: columns a stage on it takes; more than there are where none of its stages is admissible
+    const int its_devices = lane < Q ? shape.mesh_n[min(lane, Q - 1)] * shape.mesh_m[min(lane, Q - 1)] : 0;
+    const int mesh_columns = its_devices % unit == 0 ? its_devices / unit : W + 1;
     __syncthreads();
     float answer_sum = INFINITY;  // of the lane that owns (k = 0, d = D): wavefront 0's first task
     int answer_s = -1;
@@ -1348,23 +1436,27 @@ __global__ __launch_bounds__(kDpHistoryThreads, 8) void dp_history_kernel(
       int32_t *col_cur = first_col + ((s & 1) ^ 1) * L;
       // the last stage count has one state anybody reads
       const int n_tasks = s == S ? 1 : L - s + 1;
-      if (threadIdx.x == 0) reached[(s + 1) % 3] = 0;
-      for (int k_up = wave, round = 0; k_up < n_tasks; k_up += n_waves, ++round) {
-        // snake order: the cost of a task falls with k
-        int k = (round & 1) ? round * n_waves + n_waves - 1 - wave : k_up;
-        if ((round + 1) * n_waves > n_tasks) k = k_up;  // the last, partial round
+      if (threadIdx.x == 0) {
+        reached[(s + 1) % 3] = 0;
+        bound[(s + 1) % 3] = __float_as_int(INFINITY);
+      }
+      float low = INFINITY;
+      auto task = [&](auto columns, int k) {  // one start layer with all its columns, 64 at a time
+        constexpr int kC = decltype(columns)::value;
         const float *__restrict__ row = block + dp_triangle_row(L, k) - k;  // row[q * tri + i]
-        float best[kCols];
+        float best[kC];
 #pragma unroll
-        for (int j = 0; j < kCols; ++j) best[j] = INFINITY;
+        for (int j = 0; j < kC; ++j) best[j] = INFINITY;
         if (s == 1) {
-          for (int q = 0; q < Q; ++q) {
-            const int nm = shape.mesh_n[q] * shape.mesh_m[q];
-            const float rmin = row[q * tri + L - 1];
-            const float target = kBottleneck ? fmaxf(rmin, 0.0f) : rmin + 0.0f;
+          // the stage up to the last layer, lane = mesh
+          const float mine = row[min(lane, Q - 1) * tri + L - 1];
+          for (unsigned long long todo = __ballot(lane < Q && mine <= t_max); todo != 0; todo &= todo - 1) {
+            const int q = __ffsll(todo) - 1;
+            const float rmin = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mine), q));
+            const int nm = __builtin_amdgcn_readlane(mesh_columns, q);
 #pragma unroll
-            for (int j = 0; j < kCols; ++j)
-              if (1 + lane + 64 * j == nm && rmin <= t_max) best[j] = fminf(best[j], target);
+            for (int j = 0; j < kC; ++j)
+              if (1 + lane + 64 * j == nm) best[j] = fminf(best[j], kBottleneck ? fmaxf(rmin, 0.0f) : rmin + 0.0f);
           }
         } else {
           for (int i0 = k; i0 <= L - s; i0 += 64) {  // end layers behind which s - 1 stages fit
@@ -1379,24 +1471,24 @@ __global__ __launch_bounds__(kDpHistoryThreads, 8) void dp_history_kernel(
 #pragma unroll
               for (int u = 0; u < kDpHistoryBatch; ++u) {
                 if (q0 + u >= Q) break;
-                const int nm = shape.mesh_n[q0 + u] * shape.mesh_m[q0 + u];
                 // admissible, and its successor reached on what the mesh leaves: the same for
                 // every lane
-                unsigned long long todo = __ballot(r[u] <= t_max && col + nm <= D);
+                const int nm = __builtin_amdgcn_readlane(mesh_columns, q0 + u);
+                unsigned long long todo = __ballot(r[u] <= t_max && col + nm <= W);
                 if (todo == 0) continue;
-                const float *from[kCols];
+                const float *from[kC];
 #pragma unroll
-                for (int j = 0; j < kCols; ++j) {
-                  const int d = 1 + lane + 64 * j;
-                  from[j] = f + (d <= D && d > nm ? d - nm : 0);
+                for (int j = 0; j < kC; ++j) {
+                  const int c = 1 + lane + 64 * j;
+                  from[j] = f + (c <= W && c > nm ? c - nm : 0);
                 }
                 while (todo != 0) {
                   const int bit = __ffsll(todo) - 1;
                   todo &= todo - 1;
                   const float rmin = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r[u]), bit));
-                  const int at = (i0 + bit) * D;  // row i + 1
+                  const int at = (i0 + bit) * W;  // row i + 1
 #pragma unroll
-                  for (int j = 0; j < kCols; ++j) {
+                  for (int j = 0; j < kC; ++j) {
                     const float prev = from[j][at];
                     best[j] = fminf(best[j], kBottleneck ? fmaxf(rmin, prev) : rmin + prev);
                   }
@@ -1407,85 +1499,126 @@ __global__ __launch_bounds__(kDpHistoryThreads, 8) void dp_history_kernel(
         }
         int col = kDpUnreached;
 #pragma unroll
-        for (int j = kCols - 1; j >= 0; --j) {
-          const int d = 1 + lane + 64 * j;
-          if (d <= D) out[k * D + d - 1] = best[j];
-          const unsigned long long finite = __ballot(d <= D && best[j] < INFINITY);
+        for (int j = kC - 1; j >= 0; --j) {
+          const int c = 1 + lane + 64 * j;
+          if (c <= W) out[k * W + c - 1] = best[j];
+          const unsigned long long finite = __ballot(c <= W && best[j] < INFINITY);
           if (finite != 0) col = 64 * j + __ffsll(finite);
+          if (k > 0 && c < W) {  // with what the layers in front cost on the devices left, at least
+            const float front = (float)k * rate * __builtin_amdgcn_rcpf((float)((W - c) * unit));
+            low = fminf(low, kBottleneck ? fmaxf(best[j], front) : best[j] + front);
+          }
           // first s wins ties (inter_tuning.py:335-340)
-          if (k == 0 && d == D && best[j] < answer_sum) {
+          if (k == 0 && c == W && best[j] < answer_sum) {
             answer_sum = best[j];
             answer_s = s;
+            *answer = best[j];
           }
         }
         if (lane == 0) {
           col_cur[k] = col;
           if (col != kDpUnreached) reached[s % 3] = 1;
         }
+      };
+      for (int k_up = wave, round = 0; k_up < n_tasks; k_up += n_waves, ++round) {
+        // snake order: the cost of a task falls with k
+        int k = (round & 1) ? round * n_waves + n_waves - 1 - wave : k_up;
+        if ((round + 1) * n_waves > n_tasks) k = k_up;  // the last, partial round
+        if (kCols > 1 && W <= 64) task(std::integral_constant<int, 1>(), k);
+        else if (kCols > 2 && W <= 128) task(std::integral_constant<int, 2>(), k);
+        else task(std::integral_constant<int, kCols>(), k);
+      }
+      if (bounded) {
+        for (int step = 1; step < 64; step <<= 1) low = fminf(low, __shfl_xor(low, step));
+        if (lane == 0) atomicMin(&bound[s % 3], __float_as_int(low));
       }
       __syncthreads();  // every scan of F(s - 1) is done, F(s) is in the history
       if (s == S || reached[s % 3] == 0) break;  // (no state: none behind it either)
+      if (bounded && __int_as_float(bound[s % 3]) * short_by >= *answer) break;
       for (int k = 1 + wave; k <= L - s; k += n_waves) {
         if (col_cur[k] == kDpUnreached) continue;
-        for (int c = lane; c < D; c += 64) f[(k - 1) * D + c] = c == 0 ? INFINITY : out[k * D + c - 1];
+        for (int c = lane; c < W; c += 64) f[(k - 1) * W + c] = c == 0 ? INFINITY : out[k * W + c - 1];
       }
       __syncthreads();
     }
+    // the answer's path: per stage the first (mesh, end layer) that attains the value, all meshes' reads of
+    // 64 end layers in flight ...
+    int32_t *path = reinterpret_cast<int32_t *>(f);  // [stage count - 1][4]: start layer, end layer, mesh, value behind
     if (wave == 0) {
-      const int owner = (D - 1) & 63;
+      const int owner = (W - 1) & 63;
       answer_s = __builtin_amdgcn_readlane(answer_s, owner);
       answer_sum = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(answer_sum), owner));
-      const int64_t off[4] = {g * tabs.g_stride[0], g * tabs.g_stride[1], g * tabs.g_stride[2],
-                              g * tabs.g_stride[3]};
       float best = answer_sum;
-      int k = 0, d = D;
+      int k = 0, columns = W, missing = 0;
       for (int s = answer_s; s >= 1; --s) {
-        const float *__restrict__ block =
-            relaid + (int64_t)(s - 1) * Q * tri + dp_triangle_row(L, k) - k;
-        int arg_q = -1, arg_i = -1;
+        const float *__restrict__ block = relaid + (int64_t)(s - 1) * Q * tri + dp_triangle_row(L, k) - k;
+        int arg_q = Q, arg_i = -1;
         float arg_rmin = 0.0f, arg_prev = 0.0f;
-        for (int q = 0; q < Q && arg_q < 0; ++q) {
-          const int left = d - shape.mesh_n[q] * shape.mesh_m[q];
-          if (left < (s == 1 ? 0 : 1) || (s == 1 && left != 0)) continue;
-          for (int i0 = s == 1 ? L - 1 : k; i0 <= L - s; i0 += 64) {
-            const int i = i0 + lane;
-            float rmin = INFINITY, prev = INFINITY;
-            if (i <= L - s) {
-              rmin = block[q * tri + i];
-              prev = s == 1 ? 0.0f : history[(int64_t)(s - 2) * plane + (i + 1) * D + left - 1];
+        for (int i0 = s == 1 ? L - 1 : k; i0 <= L - s; i0 += 64) {
+          const int i = i0 + lane;
+          for (int q0 = 0; q0 < arg_q; q0 += kDpHistoryBatch) {
+            float rmin[kDpHistoryBatch], prev[kDpHistoryBatch];
+#pragma unroll
+            for (int u = 0; u < kDpHistoryBatch; ++u) {
+              const int left = q0 + u < Q ? columns - __builtin_amdgcn_readlane(mesh_columns, q0 + u) : -1;
+              const bool on = i <= L - s && (s == 1 ? left == 0 : left >= 1);
+              rmin[u] = on ? block[(q0 + u) * tri + i] : INFINITY;
+              prev[u] = !on ? INFINITY : s == 1 ? 0.0f : history[(int64_t)(s - 2) * plane + (i + 1) * W + left - 1];
             }
-            const float target = kBottleneck ? fmaxf(rmin, prev) : rmin + prev;
-            const unsigned long long hit = __ballot(rmin <= t_max && target == best);
-            if (hit != 0) {
+#pragma unroll
+            for (int u = 0; u < kDpHistoryBatch; ++u) {
+              if (q0 + u >= arg_q) continue;
+              const float target = kBottleneck ? fmaxf(rmin[u], prev[u]) : rmin[u] + prev[u];
+              const unsigned long long hit = __ballot(rmin[u] <= t_max && target == best);
+              if (hit == 0) continue;
               const int bit = __ffsll(hit) - 1;
-              arg_q = q;
+              arg_q = q0 + u;
               arg_i = i0 + bit;
-              arg_rmin = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(rmin), bit));
-              arg_prev = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(prev), bit));
-              break;
+              arg_rmin = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(rmin[u]), bit));
+              arg_prev = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(prev[u]), bit));
             }
           }
         }
-        if (arg_q < 0) break;  // (a reached state has a candidate that attains its value)
-        int arg_j = -1;
-        const float value = kBottleneck ? arg_rmin
-                                        : dp_stage_value(shape, tabs, off, t_max, s - 1, k, arg_q,
-                                                         arg_i, arg_prev, best, &arg_j);
-        if (lane == 0) {
-          path_value[s - 1] = value;
-          if (path_out != nullptr)
-            dp_write_stage(path_out + ((int64_t)t * S + answer_s - s) * 4, arg_i,
-                           shape.mesh_n[arg_q], shape.mesh_m[arg_q], arg_j);
+        if (arg_q >= Q) {  // (a reached state has a candidate that attains its value)
+          missing = s;
+          break;
         }
-        d -= shape.mesh_n[arg_q] * shape.mesh_m[arg_q];
+        if (lane == 0) {
+          path[4 * (s - 1)] = k;
+          path[4 * (s - 1) + 1] = arg_i;
+          path[4 * (s - 1) + 2] = arg_q;
+          path[4 * (s - 1) + 3] = __float_as_int(arg_prev);
+          path_value[s - 1] = kBottleneck ? arg_rmin : best;
+        }
+        columns -= __builtin_amdgcn_readlane(mesh_columns, arg_q);
         k = arg_i + 1;
         best = arg_prev;
       }
       if (lane == 0) {
-        best_s_out[t] = answer_s;
-        best_sum_out[t] = answer_sum;
-        stage_max_out[t] = dp_fold_path<kBottleneck>(path_value, answer_s);
+        reached[0] = answer_s;
+        reached[1] = missing;
       }
+    }
+    __syncthreads();
+    // ... then the first ckpt count of every stage, a wavefront each
+    const int its_s = reached[0];
+    const int64_t off[4] = {g * tabs.g_stride[0], g * tabs.g_stride[1], g * tabs.g_stride[2], g * tabs.g_stride[3]};
+    for (int s = reached[1] + 1 + wave; s <= its_s; s += n_waves) {
+      const int k = path[4 * (s - 1)], i = path[4 * (s - 1) + 1], q = path[4 * (s - 1) + 2];
+      int arg_j = -1;
+      if (!kBottleneck) {
+        const float value = dp_stage_value(shape, tabs, off, t_max, s - 1, k, q, i, __int_as_float(path[4 * (s - 1) + 3]),
+                                           path_value[s - 1], &arg_j);
+        if (lane == 0) path_value[s - 1] = value;
+      }
+      if (lane == 0 && path_out != nullptr)
+        dp_write_stage(path_out + ((int64_t)t * S + its_s - s) * 4, i, shape.mesh_n[q], shape.mesh_m[q], arg_j);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      best_s_out[t] = answer_s;
+      best_sum_out[t] = answer_sum;
+      stage_max_out[t] = dp_fold_path<kBottleneck>(path_value, answer_s);
     }
     __syncthreads();  // the next instance writes the history and LDS
   }
@@ -2072,10 +2205,20 @@ int mist_dp_run(const MistDpShape *shape, const MistDpCosts *costs, const float 
                            mist_dp_scratch_floats(shape, n_tmax), stream);
 }
 
-int mist_dp_run_sized(const MistDpShape *shape, const MistDpCosts *costs, const float *d_tmax,
-                      const int32_t *d_g_index, int n_tmax, int mode, int32_t *d_best_s,
-                      float *d_best_sum, float *d_stage_max, int32_t *d_argmin, int32_t *d_path,
-                      float *d_scratch, int64_t scratch_floats, void *stream) {
+}  // extern "C"
+
+int mist::dp_stage_rates(const MistDpShape &shape, const MistDpCosts &costs, int n_g, float *d_rates, hipStream_t stream) {
+  if (costs.stage_min == nullptr || n_g < 1 || n_g > 65535) return fail(MIST_E_INVALID, "no row minima or %d tables", n_g);
+  hipLaunchKernelGGL(stage_rate_kernel, dim3(kRateShares, shape.num_mesh, n_g), dim3(256), 0, stream, shape,
+                     costs.stage_min, costs.stage_min_g_stride, d_rates);
+  MIST_HIP_CHECK(hipGetLastError());
+  return 0;
+}
+
+int mist::dp_run(const MistDpShape *shape, const MistDpCosts *costs, const float *d_rates, const float *d_tmax,
+                 const int32_t *d_g_index, int n_tmax, int mode, int32_t *d_best_s, float *d_best_sum,
+                 float *d_stage_max, int32_t *d_argmin, int32_t *d_path, float *d_scratch, int64_t scratch_floats,
+                 void *stream) {
   if (int rc = check_run_arguments(shape, costs, d_tmax, d_g_index, n_tmax, mode, d_best_s,
                                    d_best_sum, d_stage_max))
     return rc;
@@ -2135,7 +2278,7 @@ int mist_dp_run_sized(const MistDpShape *shape, const MistDpCosts *costs, const 
       const MistDpShape shape_arg = *shape;
       const MistDpCosts costs_arg = *costs;
       int n_arg = n_tmax;
-      void *args[] = {(void *)&shape_arg, (void *)&costs_arg, &d_tmax, &d_g_index, &n_arg,
+      void *args[] = {(void *)&shape_arg, (void *)&costs_arg, &d_tmax, &d_g_index, &n_arg, &d_rates,
                       &d_scratch, &d_best_s, &d_best_sum, &d_stage_max, &d_path};
       MIST_HIP_CHECK(hipLaunchKernel(mode == MIST_DP_BOTTLENECK ? history_kernel<true>(cols)
                                                                 : history_kernel<false>(cols),
@@ -2146,8 +2289,8 @@ int mist_dp_run_sized(const MistDpShape *shape, const MistDpCosts *costs, const 
     }
   }
   if (d_path) {
-    if (int rc = mist_dp_run_sized(shape, costs, d_tmax, d_g_index, n_tmax, mode, d_best_s, d_best_sum,
-                                   d_stage_max, d_argmin, nullptr, d_scratch, scratch_floats, stream))
+    if (int rc = dp_run(shape, costs, d_rates, d_tmax, d_g_index, n_tmax, mode, d_best_s, d_best_sum,
+                        d_stage_max, d_argmin, nullptr, d_scratch, scratch_floats, stream))
       return rc;
     return mist_dp_backtrack(shape, d_argmin, d_best_s, n_tmax, d_path, stream);
   }
@@ -2200,6 +2343,16 @@ int mist_dp_run_sized(const MistDpShape *shape, const MistDpCosts *costs, const 
   }
   return run_step_schedule(shape, costs, d_tmax, d_g_index, n_tmax, mode, d_best_s, d_best_sum,
                            d_stage_max, d_argmin, d_scratch, stream);
+}
+
+extern "C" {
+
+int mist_dp_run_sized(const MistDpShape *shape, const MistDpCosts *costs, const float *d_tmax,
+                      const int32_t *d_g_index, int n_tmax, int mode, int32_t *d_best_s,
+                      float *d_best_sum, float *d_stage_max, int32_t *d_argmin, int32_t *d_path,
+                      float *d_scratch, int64_t scratch_floats, void *stream) {
+  return mist::dp_run(shape, costs, nullptr, d_tmax, d_g_index, n_tmax, mode, d_best_s, d_best_sum, d_stage_max,
+                      d_argmin, d_path, d_scratch, scratch_floats, stream);
 }
 
 int64_t mist_dp_static_scratch_floats(void) { return kStaticScratchFloats; }

@@ -1,0 +1,18 @@
+// Between the DP and the search driver: mist_dp_run_sized with what ends an instance early.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+
+#include "mist_dp.h"
+
+namespace mist {
+// d_rates[n_g][1 + num_mesh], +inf before the call: over costs.stage_min of every g the smallest stage
+// cost x devices / layers (negative where a cost is), and the smallest cost on every mesh.
+int dp_stage_rates(const MistDpShape &shape, const MistDpCosts &costs, int n_g, float *d_rates, hipStream_t stream);
+
+// mist_dp_run_sized; `d_rates` (may be null) holds what dp_stage_rates left for every g the instances name.
+int dp_run(const MistDpShape *shape, const MistDpCosts *costs, const float *d_rates, const float *d_tmax,
+           const int32_t *d_g_index, int n_tmax, int mode, int32_t *d_best_s, float *d_best_sum, float *d_stage_max,
+           int32_t *d_argmin, int32_t *d_path, float *d_scratch, int64_t scratch_floats, void *stream);
+}  // namespace mist

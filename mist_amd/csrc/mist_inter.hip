@@ -34,6 +34,7 @@
 
 #include "mist_common.h"
 #include "mist_dp.h"
+#include "mist_dp_rates.h"
 #include "mist_inter.h"
 
 using mist::fail;
@@ -300,6 +301,8 @@ __global__ __launch_bounds__(64) void uniform_search_kernel(
   if (lane == 0) out_total[g * n_problems + k] = total;
 }
 
+constexpr int64_t kRatesMinStates = 1024;
+
 struct Search {
   int n_families;
   const MistDpShape *shapes;  // [n_families]
@@ -316,6 +319,42 @@ struct Search {
   // the stage counts 1..s is the same, no smaller count reaches its sum (the first count wins
   // ties), so the result and the back-pointers on its path are those of the full run.
   int stage_limit = 0;
+
+  // Accumulation counts of the window requests, and behind them per family the rates that end a DP
+  // instance early (of the table rows below n_rates).  Not for planes of a few states, which end after
+  // a few short steps anyway (two batches and the bottleneck of 32 x 32 0.31 ms with them and 0.30
+  // without, of 24 x 2 0.04 and 0.03; of 40 x 64 0.44 and 0.58, of 80 x 256 2.7 and 7.2).  For tests
+  // MIST_DP_RATES = 0 | 1 decides.
+  int n_rates = 0, at_rates = 0;
+  int upload_grad_accum(const std::vector<int32_t> &rows, const int32_t *grad_accum, int n_grad_accum) {
+    n_rates = 0;
+    at_rates = n_grad_accum;
+    int n_g = 0;
+    for (const int32_t row : rows) n_g = std::max(n_g, row + 1);
+    size_t words = n_grad_accum;
+    for (int f = 0; f < n_families; ++f) words += (size_t)n_g * (1 + shapes[f].num_mesh);
+    if (int rc = ws->h_grad.reserve(sizeof(int32_t) * words)) return rc;
+    if (int rc = ws->d_grad.reserve(sizeof(int32_t) * words)) return rc;
+    std::memcpy(ws->h_grad.ptr, grad_accum, sizeof(int32_t) * n_grad_accum);
+    std::fill_n(ws->h_grad.as<float>() + n_grad_accum, words - n_grad_accum, std::numeric_limits<float>::infinity());
+    MIST_HIP_CHECK(hipMemcpyAsync(ws->d_grad.ptr, ws->h_grad.ptr, sizeof(int32_t) * words, hipMemcpyHostToDevice, stream));
+    if (n_g == 0 || n_g > 65535) return 0;
+    n_rates = n_g;
+    for (int f = 0; f < n_families; ++f)
+      if (rates_of(f) != nullptr)
+        if (int rc = mist::dp_stage_rates(shapes[f], costs[f], n_g, rates_of(f), stream)) return rc;
+    return 0;
+  }
+  float *rates_of(int f) const {
+    if (n_rates == 0 || shapes[f].free_devices != 0 || costs[f].stage_min == nullptr) return nullptr;
+    const char *decided = getenv("MIST_DP_RATES");
+    if (decided && *decided ? *decided == '0' : (int64_t)shapes[f].num_layers * shapes[f].num_devices <= kRatesMinStates)
+      return nullptr;
+    size_t at = at_rates;
+    for (int before = 0; before < f; ++before) at += (size_t)n_rates * (1 + shapes[before].num_mesh);
+    return ws->d_grad.as<float>() + at;
+  }
+
   MistDpShape shape_of(int f) const {
     MistDpShape shape = shapes[f];
     if (n_families == 1 && stage_limit > 0) shape.max_stages = std::min(shape.max_stages, stage_limit);
@@ -369,6 +408,7 @@ struct Search {
                                   stream));
     float *d_in = ws->d_in.as<float>();
     const int32_t *d_g = reinterpret_cast<int32_t *>(d_in + n);
+    const bool known = *std::max_element(g_index.begin(), g_index.end()) < n_rates;
     // the families share the state planes and the back-pointer slab: they run one after the
     // other on the stream
     for (int f = 0; f < n_families; ++f) {
@@ -377,9 +417,9 @@ struct Search {
                                                      // walk reads what the DP wrote
       int32_t *d_path = want_path ? d_paths + path_offset(f, n) : nullptr;
       const MistDpShape shape = shape_of(f);
-      if (int rc = mist_dp_run_sized(&shape, &costs[f], d_in, d_g, n, mode,
-                                     reinterpret_cast<int32_t *>(d_out), d_out + n, d_out + 2 * n,
-                                     d_argmin, d_path, ws->d_scratch.as<float>(), n_scratch, stream))
+      if (int rc = mist::dp_run(&shape, &costs[f], known ? rates_of(f) : nullptr, d_in, d_g, n, mode,
+                                reinterpret_cast<int32_t *>(d_out), d_out + n, d_out + 2 * n, d_argmin,
+                                d_path, ws->d_scratch.as<float>(), n_scratch, stream))
         return rc;
       if (want_path) {
         if (strategy) {
@@ -453,13 +493,9 @@ struct Search {
   int bottleneck_and_fetch(const std::vector<int32_t> &rows, const int32_t *grad_accum,
                            int n_grad_accum, std::vector<Fetched> *out) {
     const int n = (int)rows.size();
-    if (int rc = ws->h_grad.reserve(sizeof(int32_t) * n_grad_accum)) return rc;
-    if (int rc = ws->d_grad.reserve(sizeof(int32_t) * n_grad_accum)) return rc;
     if (int rc = ws->h_req.reserve(sizeof(float) * 4 * n)) return rc;
     if (int rc = ws->d_req.reserve(sizeof(float) * 4 * n)) return rc;
-    std::memcpy(ws->h_grad.ptr, grad_accum, sizeof(int32_t) * n_grad_accum);
-    MIST_HIP_CHECK(hipMemcpyAsync(ws->d_grad.ptr, ws->h_grad.ptr, sizeof(int32_t) * n_grad_accum,
-                                  hipMemcpyHostToDevice, stream));
+    if (int rc = upload_grad_accum(rows, grad_accum, n_grad_accum)) return rc;
     const std::vector<float> zeros(n, 0.0f);
     if (int rc = run(rows, zeros, MIST_DP_BOTTLENECK, false, /*sync=*/false)) return rc;
     hipLaunchKernelGGL(window_request_kernel, dim3((n + 63) / 64), dim3(64), 0, stream,
@@ -486,8 +522,6 @@ struct Search {
   int bottleneck_windows_first_batch(const std::vector<int32_t> &rows, const int32_t *grad_accum,
                                      int n_grad_accum, int window_capacity, int first_chunk) {
     const int n = (int)rows.size(), n_inst = n * first_chunk;
-    if (int rc = ws->h_grad.reserve(sizeof(int32_t) * n_grad_accum)) return rc;
-    if (int rc = ws->d_grad.reserve(sizeof(int32_t) * n_grad_accum)) return rc;
     if (int rc = ws->d_win_values.reserve(sizeof(float) * (size_t)n * window_capacity)) return rc;
     if (int rc = ws->d_win_counts.reserve(sizeof(int32_t) * (2 + 2 * (size_t)n))) return rc;
     if (int rc = ws->d_inst_t.reserve(sizeof(float) * n_inst)) return rc;
@@ -511,9 +545,7 @@ struct Search {
       n_scratch = std::max(n_scratch, want);
     }
     if (int rc = ws->d_scratch.reserve(sizeof(float) * (size_t)n_scratch)) return rc;
-    std::memcpy(ws->h_grad.ptr, grad_accum, sizeof(int32_t) * n_grad_accum);
-    MIST_HIP_CHECK(hipMemcpyAsync(ws->d_grad.ptr, ws->h_grad.ptr, sizeof(int32_t) * n_grad_accum,
-                                  hipMemcpyHostToDevice, stream));
+    if (int rc = upload_grad_accum(rows, grad_accum, n_grad_accum)) return rc;
     const std::vector<float> zeros(n, 0.0f);
     if (int rc = run(rows, zeros, MIST_DP_BOTTLENECK, false, /*sync=*/false)) return rc;
     float *d_req = d_first;
@@ -532,11 +564,10 @@ struct Search {
       return rc;
     for (int f = 0; f < n_families; ++f) {
       float *d_out = d_first + at_out + (size_t)f * 3 * n_inst;
-      if (int rc = mist_dp_run_sized(&shapes[f], &costs[f], ws->d_inst_t.as<float>(),
-                                     ws->d_inst_row.as<int32_t>(), n_inst, MIST_DP_THRESHOLD,
-                                     reinterpret_cast<int32_t *>(d_out), d_out + n_inst,
-                                     d_out + 2 * n_inst, nullptr, nullptr, ws->d_scratch.as<float>(), n_scratch,
-                                     stream))
+      if (int rc = mist::dp_run(&shapes[f], &costs[f], rates_of(f), ws->d_inst_t.as<float>(),
+                                ws->d_inst_row.as<int32_t>(), n_inst, MIST_DP_THRESHOLD,
+                                reinterpret_cast<int32_t *>(d_out), d_out + n_inst, d_out + 2 * n_inst,
+                                nullptr, nullptr, ws->d_scratch.as<float>(), n_scratch, stream))
         return rc;
     }
     MIST_HIP_CHECK(hipMemcpyAsync(h_first, d_first, sizeof(float) * (at_kept + kKeptHead),
