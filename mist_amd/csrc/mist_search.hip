@@ -1643,11 +1643,8 @@ struct LinearBound {
   }
 };
 constexpr double kLinearSlack = 2e-7;
-__device__ __forceinline__ LinearBound linear_bound(const RowRegs &t, double ratio, double inv_G) {
-  auto term = [&](int stable, int delta) {
-    const double x = ratio * t[stable], d = t[delta] * inv_G;
-    return __builtin_fma(-kLinearSlack, fabs(x), x) + __builtin_fma(-kLinearSlack, fabs(d), d);
-  };
+template <class Term>
+__device__ __forceinline__ LinearBound linear_form(const Term &term) {
   const double first_ck = term(MIST_T_S_FIRST_CK, MIST_T_D_FIRST_CK), last_ck = term(MIST_T_S_LAST_CK, MIST_T_D_LAST_CK);
   const double first_nock = term(MIST_T_S_FIRST_NOCK, MIST_T_D_FIRST_NOCK);
   LinearBound b;
@@ -1658,6 +1655,10 @@ __device__ __forceinline__ LinearBound linear_bound(const RowRegs &t, double rat
   b.none = first_nock + term(MIST_T_S_LAST_NOCK, MIST_T_D_LAST_NOCK) - 1e-40;
   b.mid = first_nock + last_ck - 1e-40;
   return b;
+}
+__device__ __forceinline__ double less_slack(double v) { return __builtin_fma(-kLinearSlack, fabs(v), v); }
+__device__ __forceinline__ LinearBound linear_bound(const RowRegs &t, double ratio, double inv_G) {
+  return linear_form([&](int stable, int delta) { return less_slack(ratio * t[stable]) + less_slack(t[delta] * inv_G); });
 }
 
 // The scaled peaks at p = 0 and their steps in another order of operations than pair_memory (a few
@@ -2599,113 +2600,176 @@ __device__ __forceinline__ uint64_t reduce_item(const MistProblem &prob, const M
   return hits;
 }
 
-// The same for several samples: lane = row for latencies, counts and the test against the samples'
-// thresholds, then lane = (row parity, sample) for the rows that pass some of them: the minima of a
-// slot lie side by side, so a row's look-up of all samples is one line.  (A wavefront that took the
-// samples one after the other, its minima through LDS: 14 ms for the tables of one tensor-parallel
-// size of the 7B plan, two thirds of it waiting for minima.)
+// The same for several samples.  The linear bounds of a row are those of its stable and of its delta part,
+// so that a sample's is one FMA.  Per pair
+//   lane = (one of two pairs, sample)  thresholds, and the samples that the stage's pseudo row passes (they
+//                   lie side by side, 4 to 12 of 30 on the 7B plans);
+//   lane = row      the rows below the threshold of some of them, and bounds of their counts;
+//   lane = (row, sample)  as many rows side by side as the samples leave room for: bounds against the minima at
+//                   the rows' counts, kRowLooks look-ups per slot in flight;
+//   lane = (row, pair), then (row, sample)  of what is left, collected in `queue`: the reference's arithmetic,
+//                   and a minimum per row, variant and sample.
+// (A wavefront that took the samples one after the other, its minima through LDS: 14 ms for the tables of one
+// tensor-parallel size of the 7B plan; lane = row for the reference's latencies and counts, then two rows by 32
+// samples: 3.95 ms, 1160 vector instructions a pair; now 2.1 ms and 370, which wait for the look-ups most of
+// the time.  Four wavefronts per SIMD spill, 4.0 ms; the next pairs' thresholds fetched ahead: 2.3, they are
+// older by then.  30 samples of 7B on 4x8 1.65 -> 0.81 ms.)
+constexpr int kRowLooks = 4;
+constexpr int kLinearMemoryTerms = sizeof(LinearMemory) / 8;
+struct SampleQueue {
+  union {
+    struct {
+      double2 low[64], post[64];  // of a pair's rows: stable and delta part of the bounds
+      uint32_t counts[64];        // bounds of the counts: base | with_pre << 15 | with_post or no_pp << 30
+      uint8_t row[64];
+    };
+    SampleRows exact;  // of the candidates
+  };
+  double mem[kLinearMemoryTerms][64];  // of the stage's rows (24 registers through the whole item otherwise)
+  double2 post_terms[64];
+  uint32_t entry[kCandidates];         // pair | row << 6 | first sample << 12 | samples << 17
+  uint32_t useful[64];                 // the same of the candidates that have a count
+  uint32_t changed[64];                // their pairs' samples
+};
+// `n` items of `width` lanes each, side by side.
+struct LaneGroups {
+  int width, n, item, offset;
+  __device__ __forceinline__ LaneGroups(int lane, int w) : width(w) {
+    const int inverse = (65536 + w - 1) / w;  // (exact for 64 lanes)
+    n = 64 * inverse >> 16;
+    item = lane * inverse >> 16;
+    offset = lane - item * w;
+  }
+  // lane `item` = the lanes of `of` that are its
+  __device__ __forceinline__ uint32_t bits(uint64_t of, int its) const {
+    return (uint32_t)(of >> (its * width & 63)) & (uint32_t)((1ull << width) - 1ull);
+  }
+};
 template <bool kResolve>
 __device__ __forceinline__ uint64_t reduce_item_samples(const MistProblem &prob, const MistGroupDesc *__restrict__ g,
                                                         int gi, int tile_rel, int stage,
                                                         const double *__restrict__ row_terms,
                                                         const double *__restrict__ stage_floor, const RatioList &ratios,
-                                                        const ReduceTables &tabs, uint64_t pairs, SampleRows *rows) {
-  const int L = prob.num_layers, lane = threadIdx.x & 63, sample = lane & 31;
-  const TileLane tl = tile_lane(prob, g, tile_rel);
-  const int P = g->num_p, n_slots = slots_of(P), S = tabs.n_samples;
+                                                        const ReduceTables &tabs, uint64_t pairs, SampleQueue *queue) {
+  SampleRows *const exact = &queue->exact;
+  const int L = prob.num_layers, lane = threadIdx.x & 63, S = tabs.n_samples;
+  const int my_sample = min(lane & 31, S - 1);
+  const int P = g->num_p, n_slots = slots_of(P);
   const GroupModel m = group_model(prob, g);
   const int64_t tile_cell = g->cell_offset + (int64_t)tile_rel * MIST_LC_TILE * n_slots;
   const double *best = tabs.best + tile_cell * S;  // [pair][slot][sample]
   const double *__restrict__ f = stage_floor + stage_floor_slot(g, gi, stage) * kStageFloorPitch;
-  const double ratio = ratios.r[min(sample, S - 1)];
-  const StageReach reach = stage_reach(f, pair_consts(tl.pc.l, tl.pc.c), tl.np, tl.do_post, tl.do_pp, m);
-  uint64_t todo = pairs & __ballot(tl.active && (reach.count_b > 0 || reach.count_p > 0 || reach.post || reach.pp));
+  const double ratio = ratios.r[my_sample];
+  const Offsets off = group_offsets(m, ratio);
+  const double post_layer = post_layer_offset(m, ratio, f);
+  // ---- lane = pair: what the pseudo row of the stage can reach ----
+  int lc, parts;  // l | c << 15; counts as in SampleRows
+  float floor_x, floor_d;
+  {
+    const TileLane tl = tile_lane(prob, g, tile_rel);
+    lc = tl.pc.l | tl.pc.c << 15;
+    const StageReach reach = stage_reach(f, pair_consts(tl.pc.l, tl.pc.c), tl.np, tl.do_post, tl.do_pp, m);
+    parts = reach.count_b | reach.count_p << 15 | (int)reach.post << 30 | (int)((unsigned)reach.pp << 31);
+    floor_x = reach.x;
+    floor_d = reach.d;
+    pairs &= __ballot(tl.active && parts != 0);
+  }
+  if (pairs == 0) return 0;
 
+  // ---- lane = row ----
   const int64_t row0 = (int64_t)stage * kStageRows;
   const int n_stage = (int)min((int64_t)kStageRows, g->n_rows - row0);
-  const double *__restrict__ my_row = row_terms + (g->row_offset + row0 + min(lane, n_stage - 1)) * MIST_ROW_TERMS;
-  const bool live = lane < n_stage;
-  const uint32_t my_row_number =
-      (kResolve ? 0u : kUnresolved) + (uint32_t)row_of_position(g, row0 + min(lane, n_stage - 1));
-  RowRegs t;
-  load_terms<0, MIST_T_D_LAST_NOCK + 1>(t, my_row);
-  bool have_rest = false;
-  uint64_t hits = 0;
-  for (uint64_t rest = todo; rest != 0; rest &= rest - 1) {
-    const int pl = __ffsll((unsigned long long)rest) - 1;
-    const int l = from_lane(tl.pc.l, pl), c = from_lane(tl.pc.c, pl);
-    const PairConsts k = pair_consts(l, c);
-    const double *slots = best + (int64_t)pl * n_slots * S;
-    // ---- lane = sample: thresholds ----
-    const StageReach its{from_lane(reach.count_b, pl), from_lane(reach.count_p, pl), from_lane((int)reach.post, pl) != 0,
-                         from_lane((int)reach.pp, pl) != 0, from_lane(reach.x, pl), from_lane(reach.d, pl)};
-    double thr = its.threshold(slots + min(sample, S - 1), S, P, ratio, INFINITY, m, f);
-    if (kResolve)  // only the samples whose minima changed
-      thr = tabs.changed[(tile_cell + pl * n_slots) / 4] >> sample & 1u ? thr : -INFINITY;
-    if (!__any(m.bound(ratio, its.x, its.d) <= thr)) continue;
-    // ---- lane = row ----
-    float x, d;
-    pair_latency(t, k, x, d);
-    const double low_x = m.lower_x(x), low_share = m.lower_share(d);
-    bool pass = false;
-    for (int s = 0; s < S; ++s) pass = pass || ratios.r[s] * low_x + low_share <= from_lane(thr, s);
-    pass = pass && live;
-    if (!__any(pass)) continue;
-    if (!have_rest) {
-      load_terms<MIST_T_D_LAST_NOCK + 1, MIST_ROW_TERMS>(t, my_row);
-      have_rest = true;
+  const double *__restrict__ rows = row_terms + (g->row_offset + row0) * MIST_ROW_TERMS;
+  const uint64_t live = ~0ull >> (64 - n_stage);
+  LinearBound stable, delta;
+  __builtin_amdgcn_wave_barrier();
+  {
+    RowRegs t;
+    load_terms<0, MIST_ROW_TERMS>(t, rows + min(lane, n_stage - 1) * MIST_ROW_TERMS);
+    stable = linear_form([&](int its, int) { return less_slack(t[its]); });
+    delta = linear_form([&](int, int its) { return less_slack(t[its] * m.inv_G64); });
+    const LinearMemory mem = linear_memory(t);
+#pragma unroll
+    for (int i = 0; i < kLinearMemoryTerms; ++i) queue->mem[i][lane] = reinterpret_cast<const double *>(&mem)[i];
+    const double opb = t[MIST_T_OPB], nag = fmin(t[MIST_T_NAG_NOCK], t[MIST_T_NAG_CK]),
+                 nrs = fmin(t[MIST_T_NRS_NOCK], t[MIST_T_NRS_CK]);
+    double2 post_terms;
+    post_terms.x = less_slack(opb) + less_slack(m.k.pp_wre ? nag : 0.0) + less_slack(m.k.pp_gre ? nrs : 0.0);
+    post_terms.y = less_slack(m.div_G(m.k.pp_wre ? 0.0 : nag)) + less_slack(m.div_G(m.k.pp_gre ? 0.0 : nrs));
+    queue->post_terms[lane] = post_terms;
+  }
+  const double cap_and_room = m.cap * (1.0 + 1e-12);
+  uint64_t hits = 0;  // of the lane's items
+
+  // ---- lane = (row, pair): the first `n` of the queue; then lane = (row, sample) ----
+  auto settle_candidates = [&](int n) {
+    const uint32_t entry = queue->entry[min(lane, n - 1)];
+    const int pl = (int)(entry & 63u), its_row = (int)(entry >> 6 & 63u);
+    int width = (int)(entry >> 17);
+    {
+      const int its = __shfl(lc, pl), l = its & 0x7fff, c = its >> 15;
+      const bool in = lane < n;
+      RowRegs t;
+      load_terms<0, MIST_ROW_TERMS>(t, rows + its_row * MIST_ROW_TERMS);
+      const PairConsts k = pair_consts(l, c);
+      float x, d;
+      pair_latency(t, k, x, d);
+      const LaneMemory lm = pair_memory(t, k);
+      const bool do_post = in && c != l - 1;
+      const UpperCounts upper = upper_counts(lm, m, in ? (c == l - 1 ? min(P, 1) : P) : 0);
+      const RowCounts cnt = exact_counts(lm, m, upper.b, upper.p);
+      bool ok_post, ok_pp;
+      post_fits(t, k, lm, m, lm.out, k.no_ck ? t[MIST_T_RD] : 0.0, ok_post, ok_pp);
+      ok_post = ok_post && do_post;
+      ok_pp = ok_pp && do_post && l == L;
+      const bool useful = cnt.b > 0 || cnt.p > 0 || ok_post || ok_pp;
+      const uint64_t some = __ballot(useful);
+      const int at = __popcll(some & ((1ull << lane) - 1ull));
+      if (useful) {
+        put_sample_row(exact, at, t, x, d, k.no_ck, m, cnt.b, cnt.p, ok_post, ok_pp, true);
+        exact->number[at] = (kResolve ? 0u : kUnresolved) + (uint32_t)row_of_position(g, row0 + its_row);
+        queue->useful[at] = entry;
+        if (kResolve) queue->changed[at] = tabs.changed[(tile_cell + pl * n_slots) / 4];
+      }
+      n = __popcll(some);
     }
-    const LaneMemory mem = pair_memory(t, k);
-    const int np = c == l - 1 ? min(P, 1) : P;
-    const bool do_post = c != l - 1, do_pp = do_post && l == L;
-    const UpperCounts upper = upper_counts(mem, m, pass ? np : 0);
-    const RowCounts cnt = exact_counts(mem, m, upper.b, upper.p);
-    bool ok_post = false, ok_pp = false;
-    if (do_post) post_fits(t, k, mem, m, mem.out, k.no_ck ? t[MIST_T_RD] : 0.0, ok_post, ok_pp);
-    ok_post = ok_post && pass;
-    ok_pp = ok_pp && do_pp && pass;
-    const uint64_t useful = __ballot(cnt.b > 0 || cnt.p > 0 || ok_post || ok_pp);
-    if (useful == 0) continue;
-    __builtin_amdgcn_wave_barrier();
-    const int at = __popcll(useful & ((1ull << lane) - 1ull));
-    if (useful >> lane & 1ull) {
-      put_sample_row(rows, at, t, x, d, k.no_ck, m, cnt.b, cnt.p, ok_post, ok_pp, do_post);
-      rows->number[at] = my_row_number;
-    }
+    if (n == 0) return;
+    for (int step = 1; step < 64; step *= 2) width = max(width, __shfl_xor(width, step));
+    const LaneGroups slot(lane, __builtin_amdgcn_readfirstlane(width));
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
-    // ---- lane = (row parity, sample) ----
-    const int n_useful = __popcll(useful);
-    const int64_t at0 = (tile_cell + (int64_t)pl * n_slots) * S + sample;
-    bool hit = false, lowered = false;
-    const bool sampled = sample < S && (!kResolve || thr != -INFINITY);
     // look-ups of a row, one iteration ahead of their use
-    double now_b, now_p, now_post = -INFINITY, now_pp = -INFINITY;
-    uint32_t counts;
+    double now_b, now_p, now_post, now_pp;
+    uint32_t counts, place;
     auto look = [&](int r) {
-      counts = rows->counts[min(r, n_useful - 1)];
+      counts = exact->counts[r];
+      place = queue->useful[r];
       const int nb = (int)(counts & 0x7fff), npre = (int)(counts >> 15 & 0x7fff);
-      const double *mine = slots + min(sample, S - 1);
+      const double *mine = best + (int64_t)(place & 63u) * n_slots * S + min((int)(place >> 12 & 31u) + slot.offset, S - 1);
       now_b = mine[max(nb - 1, 0) * S];
       now_p = mine[(P + max(npre - 1, 0)) * S];
-      if (do_post) now_post = mine[2 * P * S];
-      if (do_pp) now_pp = mine[(2 * P + 1) * S];
+      now_post = mine[2 * P * S];
+      now_pp = mine[(2 * P + 1) * S];
     };
-    look(lane >> 5);
-    for (int r0 = 0; r0 < n_useful; r0 += 2) {
-      const int r = min(r0 + (lane >> 5), n_useful - 1);
-      const bool on = sampled && r0 + (lane >> 5) < n_useful;
+    look(min(slot.item, n - 1));
+    for (int r0 = 0; r0 < n; r0 += slot.n) {
+      const int r = min(r0 + slot.item, n - 1), its_pair = (int)(place & 63u), first = (int)(place >> 12 & 31u);
+      const int sample = min(first + slot.offset, S - 1);
+      const bool on = slot.item < slot.n && r0 + slot.item < n && first + slot.offset < S &&
+                      (!kResolve || (queue->changed[r] >> sample & 1u) != 0);
+      const double its_ratio = __shfl(ratio, sample);
       const uint32_t cn = counts;
       const double nb_now = now_b, np_now = now_p, post_now = now_post, pp_now = now_pp;
-      if (r0 + 2 < n_useful) look(r0 + 2 + (lane >> 5));
+      if (r0 + slot.n < n) look(min(r0 + slot.n + slot.item, n - 1));
+      bool hit = false, lowered = false;
       auto offer = [&](bool ok, int variant, int own, double now) {
-        const double2 xy = rows->xy[variant][r];
-        const double cost = ratio * xy.x + xy.y;
+        const double2 xy = exact->xy[variant][r];
+        const double cost = its_ratio * xy.x + xy.y;
         if (!(on && ok && cost <= now && cost < INFINITY)) return;
         hit = true;
-        const int64_t to = at0 + (int64_t)own * S;
+        const int64_t to = (tile_cell + its_pair * n_slots + own) * S + sample;
         if (cost == now) {
-          atomicMin(tabs.row + to, rows->number[r]);
+          atomicMin(tabs.row + to, exact->number[r]);
         } else if (!kResolve) {
           lower_minimum(tabs.best + to, cost);
           lowered = true;
@@ -2714,19 +2778,128 @@ __device__ __forceinline__ uint64_t reduce_item_samples(const MistProblem &prob,
       const int nb = (int)(cn & 0x7fff), npre = (int)(cn >> 15 & 0x7fff);
       offer(nb > 0, 0, nb - 1, nb_now);
       offer(npre > 0, 1, P + npre - 1, np_now);
-      if (do_post) {
-        offer((cn >> 30 & 1u) != 0, 2, 2 * P, post_now);
-        if (do_pp) offer((cn >> 31) != 0, 3, 2 * P + 1, pp_now);
+      offer((cn >> 30 & 1u) != 0, 2, 2 * P, post_now);
+      offer((cn >> 31) != 0, 3, 2 * P + 1, pp_now);
+      if (kResolve) continue;
+      const uint64_t some = __ballot(hit), low = __ballot(lowered);
+      if (some == 0 || slot.offset != 0 || slot.item >= slot.n) continue;
+      const uint32_t samples = slot.bits(low, slot.item);
+      if (samples != 0) atomicOr(tabs.changed + (tile_cell + its_pair * n_slots) / 4, samples << first);
+      if (slot.bits(some, slot.item) != 0) hits |= 1ull << its_pair;
+    }
+  };
+
+  int waiting = 0;
+  // A pair's rows; `thr_post` of sample `lane & 31`, `samples` that may pass.
+  auto visit = [&](int pl, double thr, double thr_post, int half, uint32_t samples) {
+    const int its_lc = from_lane(lc, pl);
+    const LinearPair p(its_lc & 0x7fff, its_lc >> 15);
+    const double low_x = stable.at(p.n_ck, p.n_nock, p.all_ck, p.none), low_y = delta.at(p.n_ck, p.n_nock, p.all_ck, p.none);
+    uint64_t found = 0;
+    for (uint32_t left = samples; left != 0; left &= left - 1) {
+      const int s = __ffs(left) - 1;
+      found |= __ballot(__builtin_fma(from_lane(ratio, s), low_x, low_y) <= from_lane(thr, half + s));
+    }
+    found &= live;
+    if (found == 0) return;
+    LinearMemory mem;
+#pragma unroll
+    for (int i = 0; i < kLinearMemoryTerms; ++i) reinterpret_cast<double *>(&mem)[i] = queue->mem[i][lane];
+    const LinearReach reach = linear_reach(mem, p, m, p.c == p.l - 1 ? min(P, 1) : P, cap_and_room);
+    const bool post = p.c != p.l - 1 && post_may_fit(reach, mem, p, L, m, cap_and_room);
+    found &= __ballot(reach.count_b > 0 || reach.count_p > 0 || post);
+    if (found == 0) return;
+    const int n_found = __popcll(found);
+    __builtin_amdgcn_wave_barrier();
+    if (found >> lane & 1ull) {
+      const int at = __popcll(found & ((1ull << lane) - 1ull));
+      queue->low[at] = double2{low_x, low_y};
+      const double2 post_terms = queue->post_terms[lane];
+      queue->post[at] = double2{low_x + post_terms.x, low_y + post_terms.y};
+      queue->counts[at] = (uint32_t)reach.count_b | (uint32_t)reach.count_p << 15 | (post ? 1u << 30 : 0u);
+      queue->row[at] = (uint8_t)lane;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    // ---- lane = (row, sample) ----
+    const int first = __ffs(samples) - 1;
+    const LaneGroups slot(lane, 32 - __clz(samples) - first);
+    const int sample = min(first + slot.offset, S - 1);
+    const double its_ratio = __shfl(ratio, sample), its_post = __shfl(thr_post, half + sample),
+                 its_pre = __shfl(off.pre, sample);
+    const bool on = slot.item < slot.n && first + slot.offset < S;
+    const double *mine = best + (int64_t)pl * n_slots * S + sample;
+    uint64_t may = 0;
+    for (int r0 = 0; r0 < n_found; r0 += kRowLooks * slot.n) {
+      double now_b[kRowLooks], now_p[kRowLooks];
+      uint32_t counts[kRowLooks];
+#pragma unroll
+      for (int u = 0; u < kRowLooks; ++u) {
+        counts[u] = queue->counts[min(r0 + u * slot.n + slot.item, n_found - 1)];
+        now_b[u] = mine[max((int)(counts[u] & 0x7fff) - 1, 0) * S];
+        now_p[u] = mine[(P + max((int)(counts[u] >> 15 & 0x7fff) - 1, 0)) * S];
+      }
+#pragma unroll
+      for (int u = 0; u < kRowLooks; ++u) {
+        const int first_row = r0 + u * slot.n, r = min(first_row + slot.item, n_found - 1);
+        if (first_row >= n_found) break;
+        const double2 xy = queue->low[r], post_xy = queue->post[r];
+        const double low = __builtin_fma(its_ratio, xy.x, xy.y);
+        const bool reached = ((low <= now_b[u]) & ((counts[u] & 0x7fff) != 0)) |
+                             ((low <= now_p[u] - its_pre) & ((counts[u] >> 15 & 0x7fff) != 0)) |
+                             ((__builtin_fma(its_ratio, post_xy.x, post_xy.y) <= its_post) & ((counts[u] >> 30 & 1u) != 0));
+        const uint64_t some = __ballot(reached && on);
+        if (some == 0) continue;
+        const uint64_t its = __ballot(lane < slot.n && first_row + lane < n_found && slot.bits(some, lane) != 0);
+        may |= its << first_row;
       }
     }
-    if (!kResolve) {
-      const uint64_t low = __ballot(lowered);
-      const uint32_t samples = (uint32_t)low | (uint32_t)(low >> 32);
-      if (samples != 0 && lane == 0) atomicOr(tabs.changed + (tile_cell + pl * n_slots) / 4, samples);
-      if (__any(hit)) hits |= 1ull << pl;
+    if (may == 0) return;
+    if (may >> lane & 1ull)
+      queue->entry[waiting + __popcll(may & ((1ull << lane) - 1ull))] =
+          (uint32_t)pl | (uint32_t)queue->row[lane] << 6 | (uint32_t)first << 12 | (uint32_t)slot.width << 17;
+    waiting += __popcll(may);
+  };
+  double thr, thr_post;
+  uint64_t may = 0;  // samples of the two pairs
+  int pair_a = 0, pair_b = 0;
+  for (uint64_t rest = pairs; rest != 0 || may != 0 || waiting > 0;) {
+    if (may != 0) {
+      const int half = (uint32_t)may != 0 ? 0 : 32;
+      const uint32_t samples = (uint32_t)(may >> half);
+      may &= ~(0xffffffffull << half);
+      visit(half == 0 ? pair_a : pair_b, thr, thr_post, half, samples);
+    } else if (rest != 0) {
+      pair_a = __ffsll((unsigned long long)rest) - 1;
+      rest &= rest - 1;
+      const uint64_t second = rest != 0 ? ~0ull : 0xffffffffull;
+      pair_b = rest != 0 ? __ffsll((unsigned long long)rest) - 1 : pair_a;
+      rest &= rest - 1;
+      // ---- lane = (pair, sample): thresholds ----
+      const int pl = lane < 32 ? pair_a : pair_b;
+      const uint32_t its_parts = (uint32_t)__shfl(parts, pl);
+      const Threshold its(loosest_minima(true, best + (int64_t)pl * n_slots * S + my_sample, S, P, (int)(its_parts & 0x7fff),
+                                         (int)(its_parts >> 15 & 0x7fff), (its_parts >> 30 & 1u) != 0, its_parts >> 31 != 0,
+                                         INFINITY), off);
+      thr = its.at(post_layer);
+      thr_post = its.post;
+      const double low = m.bound(ratio, __shfl(floor_x, pl), __shfl(floor_d, pl));
+      bool on = (lane & 31) < S;
+      if (kResolve) on = on && (tabs.changed[(tile_cell + pl * n_slots) / 4] >> (lane & 31) & 1u) != 0;
+      may = second & __ballot(on && low <= thr);
     }
+    if (waiting < 64 && (waiting == 0 || rest != 0 || may != 0)) continue;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    settle_candidates(min(waiting, 64));
+    waiting = max(waiting - 64, 0);
+    const uint32_t moved = queue->entry[64 + lane];
+    __builtin_amdgcn_wave_barrier();
+    queue->entry[lane] = moved;
   }
-  return hits;
+  if (kResolve) return 0;
+  for (int step = 1; step < 64; step *= 2) hits |= __shfl_xor((unsigned long long)hits, step);
+  return from_lane(hits, 0);
 }
 
 // Every 2^k-th pair from the first on.
@@ -2754,9 +2927,9 @@ __global__ __launch_bounds__(kReduceThreads, 3) void reduce_kernel(
     const MistGroupDesc *g = groups + gi;
     uint64_t hit;
     if constexpr (kSamples) {
-      __shared__ SampleRows lds_samples[kWaves];
+      __shared__ SampleQueue lds_queues[kWaves];
       hit = reduce_item_samples<kResolve>(prob, g, gi, tile_rel, stage, row_terms, stage_floor, ratios, tabs, pairs,
-                                          &lds_samples[local_wave]);
+                                          &lds_queues[local_wave]);
     } else
       hit = reduce_item<kResolve, kInLds>(prob, g, gi, tile_rel, stage, row_terms, stage_floor, ratios.r[0], tabs,
                                           pairs, lds_rows + local_wave * wave_pitch);
@@ -2765,7 +2938,9 @@ __global__ __launch_bounds__(kReduceThreads, 3) void reduce_kernel(
   };
   constexpr bool kListed = kResolve && kSamples;
   const FlatQueue queue = flat_queue(tabs, kListed ? 0 : 1);
-  int split = 0;  // enough units for every wavefront several times over
+  // enough units for every wavefront several times over; a pair of several samples takes longer (30 samples
+  // of one tensor-parallel size of the 7B plan: 64 pairs a unit 2.36 ms, 32 2.12, 16 2.09)
+  int split = kSamples ? 2 : 0;
   while (split < 4 && ((uint64_t)queue.total << split) < (uint64_t)n_waves * 2) ++split;
   const uint64_t units = (uint64_t)queue.total << split;
   if (kResolve) {  // few are left: handed out in turn

@@ -13,7 +13,7 @@ def test_minima_and_candidates_in_lds(n_p):
     hold_against_the_oracle(n_p, 90.0, 1)
 
 
-@pytest.mark.parametrize("samples", [1, 2, 31])
+@pytest.mark.parametrize("samples", [1, 2, 7, 32])
 @pytest.mark.parametrize("base, capacity", [(1, 3.0), (1, 3.9), (1, 5.0), (2, 9.0), (2, 12.0), (2, 20.0)])
 def test_where_memory_decides(base, capacity, samples):
     """From plans of which a few cells fit to plans with most of them: counts at their edges, last and
