@@ -46,19 +46,15 @@ constexpr int kDpBatch = 4;  // end layers whose reads a lane of the one-lane-pe
 // ------------------------------------------------------------------------------------------
 // Table rows (fixed g, mesh, p, layers) hold the L+1 ckpt entries: cost = (float)stable +
 // (float)delta / G, and alongside its running minimum pmin[j] = min(cost[0..j]).  A workgroup
-// takes as many whole rows as fit its 256 lanes, one lane per entry, so that loads and stores
-// are contiguous; the running minimum is a segmented scan (wavefront shuffles, LDS between the
-// wavefronts a row spans).  Rows longer than the workgroup are walked in passes of 256 entries
-// with the minimum of the earlier passes carried along.  A workgroup takes kCostRuns such sets of
-// rows: with one each, 1.85e6 workgroups of a few hundred instructions per lane were bound by their
-// own start and by a 64-bit division per lane (70B on 32x8, 4.5e8 cells: 2.70 ms; division per
-// workgroup and lane shifts instead of shuffles through LDS 2.52, eight sets 2.02; 7B on 4x8 0.104
-// -> 0.083).  Bound: 12 bytes a cell and 16 more where it holds a row, at 3.5 TB/s.
+// takes sets of whole rows, so that loads and stores are contiguous; the running minimum is a
+// segmented scan (lane shifts, LDS between the wavefronts a row spans).
 // Most cells of a plan hold no strategy (no group for that (g, mesh), or nothing fits): their
 // row index is -1 and their costs +inf, so with the index table (may be null) the 16 bytes of
 // such a cell's costs are not read.
 // The four tables of a call (base, with_pre, with_post, no_pp) go through one launch: table v
-// owns the workgroups first_block[v] .. first_block[v + 1] - 1.
+// owns the workgroups first_block[v] .. first_block[v + 1] - 1.  A workgroup takes kCostRuns sets
+// of rows one after the other: with one each, its own start and a division per lane were the bound.
+// Bound: 12 bytes a cell and 16 more where it holds a row.
 constexpr int kCostRuns = 8;
 struct CostTableJob {
   const double *stable[4], *delta[4];
@@ -67,6 +63,141 @@ struct CostTableJob {
   int64_t n_rows[4], rows_per_g[4];
   unsigned first_block[5];
 };
+// `run` of the lane `control` names, where it is `distance` back in the same row of the table;
+// a lane without a source keeps its own
+#define MIST_RUN_DPP(run, back, control, rows, distance)                                          \
+  {                                                                                               \
+    const int other = __builtin_amdgcn_update_dpp(__float_as_int(run), __float_as_int(run),       \
+                                                  control, rows, 0xf, false);                     \
+    run = (back) >= (distance) ? fminf(run, __int_as_float(other)) : run;                         \
+  }
+// running minimum over the lanes of a wavefront; `back`: lanes since the row's first
+__device__ __forceinline__ float running_minimum(float run, int back) {
+  const int lane = threadIdx.x & 63;
+  MIST_RUN_DPP(run, back, 0x111, 0xf, 1)  // row_shr:1
+  MIST_RUN_DPP(run, back, 0x112, 0xf, 2)
+  MIST_RUN_DPP(run, back, 0x114, 0xf, 4)
+  MIST_RUN_DPP(run, back, 0x118, 0xf, 8)
+  MIST_RUN_DPP(run, back, 0x142, 0xa, (lane & 15) + 1)  // row_bcast:15 into the odd rows of 16 lanes
+  MIST_RUN_DPP(run, back, 0x143, 0xc, lane - 31)        // row_bcast:31 into the upper half
+  return run;
+}
+#undef MIST_RUN_DPP
+
+// Four neighbouring cells per lane, in as many rows (a multiple of four, so that each set begins at
+// 16 bytes) as 1024 cells hold; one sample, rows of up to 256 cells: a row lies in two wavefronts at
+// most.  (A cell per lane: 95 vector instructions for 64 cells and the stores of 4 bytes, 70B on 32x8
+// with its 4.5e8 cells 2.03 ms; now 1.06, 5.1 TB/s; 7B on 4x8 0.084 -> 0.047.)
+constexpr int kCostCells = 1024;
+// (a table may begin at any of its elements; loads and stores of 16 bytes need 4)
+typedef int AnyInt4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef float AnyFloat4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef double AnyDouble2 __attribute__((ext_vector_type(2), aligned(8)));
+__global__ __launch_bounds__(256) void cost_rows_kernel(const CostTableJob job, const int32_t *__restrict__ grad_accum,
+                                                        int row_len) {
+  __shared__ float ends[2][4];
+  const int v = (blockIdx.x >= job.first_block[1]) + (blockIdx.x >= job.first_block[2]) +
+                (blockIdx.x >= job.first_block[3]);
+  const double *__restrict__ stable = job.stable[v], *__restrict__ delta = job.delta[v];
+  const int32_t *__restrict__ index = job.index[v];
+  float *__restrict__ out = job.out[v], *__restrict__ pmin = job.pmin[v];
+  const int64_t n_rows = job.n_rows[v], per_g = job.rows_per_g[v];
+  const int rows_here = (kCostCells / row_len) & ~3, cells_here = rows_here * row_len;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, cell0 = (int)threadIdx.x * 4;
+  int its_row[4], j[4];
+  its_row[0] = cell0 / row_len;
+  j[0] = cell0 - its_row[0] * row_len;
+#pragma unroll
+  for (int u = 1; u < 4; ++u) {
+    const bool next = j[u - 1] + 1 == row_len;
+    its_row[u] = its_row[u - 1] + next;
+    j[u] = next ? 0 : j[u - 1] + 1;
+  }
+  const int back = min((int)threadIdx.x - ((cell0 + 3 - j[3]) >> 2), lane);  // to where the last cell's row begins
+  const bool spills = cell0 - j[0] < wave * 256;  // the first cell's begins in an earlier wavefront
+  const int64_t row0 = (int64_t)(blockIdx.x - job.first_block[v]) * rows_here * kCostRuns;
+  int64_t g = row0 / per_g, in_g = row0 - g * per_g;
+  for (int turn = 0; turn < kCostRuns; ++turn) {
+    const int64_t row = row0 + turn * rows_here;
+    if (row >= n_rows) break;
+    const int n_cells = (int)min((int64_t)cells_here, (n_rows - row) * row_len);
+    const int n_mine = min(n_cells - cell0, 4);
+    const int64_t i = row * row_len + cell0;
+    const int until = (int)min(per_g - in_g, (int64_t)rows_here);  // rows of g
+    float c[4];
+    bool holds[4];
+    if (n_mine == 4) {
+      const AnyInt4 at = index == nullptr ? AnyInt4{0, 0, 0, 0} : *reinterpret_cast<const AnyInt4 *>(index + i);
+      holds[0] = at.x >= 0;
+      holds[1] = at.y >= 0;
+      holds[2] = at.z >= 0;
+      holds[3] = at.w >= 0;
+    } else {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) holds[u] = u < n_mine && (index == nullptr || index[i + u] >= 0);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) c[u] = INFINITY;
+    if (holds[0] || holds[1] || holds[2] || holds[3]) {
+      double its_stable[4], its_delta[4];
+      if (n_mine == 4) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const AnyDouble2 s = reinterpret_cast<const AnyDouble2 *>(stable + i)[h];
+          const AnyDouble2 d = reinterpret_cast<const AnyDouble2 *>(delta + i)[h];
+          its_stable[2 * h] = s.x;
+          its_stable[2 * h + 1] = s.y;
+          its_delta[2 * h] = d.x;
+          its_delta[2 * h + 1] = d.y;
+        }
+      } else {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          its_stable[u] = holds[u] ? stable[i + u] : 0.0;
+          its_delta[u] = holds[u] ? delta[i + u] : 0.0;
+        }
+      }
+      const float first_G = (float)grad_accum[g];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        float G = first_G;
+        if (holds[u] && its_row[u] >= until) {
+          int64_t its_g = g + 1;
+          for (int64_t past = its_row[u] - until; past >= per_g; past -= per_g) ++its_g;
+          G = (float)grad_accum[its_g];
+        }
+        const float cost = (float)its_stable[u] + (float)its_delta[u] / G;
+        c[u] = holds[u] ? cost : INFINITY;
+      }
+    }
+    for (in_g += rows_here; in_g >= per_g; in_g -= per_g) ++g;
+    float run = INFINITY;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) run = fminf(c[u], j[u] == 0 ? INFINITY : run);
+    run = running_minimum(run, back);
+    if (lane == 63) ends[turn & 1][wave] = run;
+    __syncthreads();
+    run = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(INFINITY), __float_as_int(run), 0x138, 0xf, 0xf,
+                                                     false));  // wave_shr:1
+    if (spills) run = fminf(run, ends[turn & 1][wave - 1]);
+    float m[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) m[u] = run = fminf(c[u], j[u] == 0 ? INFINITY : run);
+    if (n_mine == 4) {
+      *reinterpret_cast<AnyFloat4 *>(out + i) = AnyFloat4{c[0], c[1], c[2], c[3]};
+      *reinterpret_cast<AnyFloat4 *>(pmin + i) = AnyFloat4{m[0], m[1], m[2], m[3]};
+    } else {
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (u < n_mine) {
+          out[i + u] = c[u];
+          pmin[i + u] = m[u];
+        }
+    }
+  }
+}
+
+// Any row length and sample position: a cell per lane.
 __global__ __launch_bounds__(256) void cost_table_kernel(const CostTableJob job,
                                                          const int32_t *__restrict__ grad_accum,
                                                          int row_len, int sample_size, int slot) {
@@ -108,23 +239,7 @@ __global__ __launch_bounds__(256) void cost_table_kernel(const CostTableJob job,
       // running minimum over the row's lanes of this pass: inside a wavefront by lane shifts that stop
       // at the row's first lane, then the part of the row that lies in earlier wavefronts (their
       // last lanes hold it)
-      float run = c;
-      const int lane = threadIdx.x & 63;
-      // `run` of the lane `control` names, where it is `distance` back in the same row of the table;
-      // a lane without a source keeps its own
-#define MIST_RUN_DPP(control, rows, distance)                                                    \
-    {                                                                                              \
-      const int other = __builtin_amdgcn_update_dpp(__float_as_int(run), __float_as_int(run),      \
-                                                    control, rows, 0xf, false);                    \
-      run = j0 >= (distance) ? fminf(run, __int_as_float(other)) : run;                            \
-    }
-      MIST_RUN_DPP(0x111, 0xf, 1)  // row_shr:1
-      MIST_RUN_DPP(0x112, 0xf, 2)
-      MIST_RUN_DPP(0x114, 0xf, 4)
-      MIST_RUN_DPP(0x118, 0xf, 8)
-      MIST_RUN_DPP(0x142, 0xa, (lane & 15) + 1)  // row_bcast:15 into the odd rows of 16 lanes
-      MIST_RUN_DPP(0x143, 0xc, lane - 31)        // row_bcast:31 into the upper half
-#undef MIST_RUN_DPP
+      float run = running_minimum(c, j0);
       lds[threadIdx.x] = run;
       __syncthreads();
       const int row_first = (int)threadIdx.x - j0;
@@ -2018,7 +2133,9 @@ int mist_dp_cost_tables(const MistProblem *problem, const MistOutTables *tables,
     return fail(MIST_E_INVALID, "bad problem extents");
   if (slot < 0 || slot >= S) return fail(MIST_E_INVALID, "slot %d outside [0, %d)", slot, (int)S);
   const int64_t rows_per_g[4] = {Q * P1 * L, Q * P1 * L, Q * L, Q};
-  const int64_t rows_per_block = 256 / std::min<int64_t>(L + 1, 256) * kCostRuns;
+  const bool wide = S == 1 && L + 1 <= 256;  // four neighbouring cells a lane, rows of a wavefront's cells at most
+  const int64_t rows_per_block =
+      (wide ? (kCostCells / (L + 1)) & ~3ll : 256 / std::min<int64_t>(L + 1, 256)) * kCostRuns;
   CostTableJob job = {};
   int64_t blocks = 0;
   for (int v = 0; v < 4; ++v) {
@@ -2036,8 +2153,12 @@ int mist_dp_cost_tables(const MistProblem *problem, const MistOutTables *tables,
   }
   if (blocks >= (int64_t)1 << 31) return fail(MIST_E_INVALID, "cost tables too large for one launch");
   job.first_block[4] = (unsigned)blocks;
-  hipLaunchKernelGGL(cost_table_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, job,
-                     d_grad_accum, (int)(L + 1), (int)S, slot);
+  if (wide)
+    hipLaunchKernelGGL(cost_rows_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, job, d_grad_accum,
+                       (int)(L + 1));
+  else
+    hipLaunchKernelGGL(cost_table_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, job,
+                       d_grad_accum, (int)(L + 1), (int)S, slot);
   MIST_HIP_CHECK(hipGetLastError());
   return 0;
 }
