@@ -1753,6 +1753,7 @@ __device__ __forceinline__ Loosest loosest_minima(bool wanted, const double *slo
 // parts, from the offsets of the group and with what a stage's post-layer terms add to the second.
 struct Threshold {
   double front, post;  // base and with_pre; with_post and no_pp
+  __device__ __forceinline__ Threshold(double its_front, double its_post) : front(its_front), post(its_post) {}
   __device__ __forceinline__ Threshold(const Loosest &t, const Offsets &group)
       : front(fmax(t.base, t.pre - group.pre)), post(fmax(t.post - group.post, t.pp - group.pp)) {}
   __device__ __forceinline__ double at(double post_layer) const { return fmax(front, post - post_layer); }
@@ -2111,7 +2112,16 @@ __device__ __forceinline__ StageReach stage_reach(const double *__restrict__ f, 
 // Workgroup = one wavefront = (row chunk, tile, p tile as a share of the chunk's summaries), lane
 // = pair.  Summaries are wave-uniform and come through scalar loads; a visit is ~40 float64
 // instructions against the pair's loosest minima.
-__global__ __launch_bounds__(MIST_LC_TILE) void filter_kernel(
+// Several samples: kFilterShares wavefronts of a workgroup take as many shares of a tile and its thresholds
+// at every sample from LDS, where they get them with lane = (pair parity, sample): the minima of a slot lie
+// side by side.  A summary is tried at the sample that the last one passed first.  (A wavefront a share and
+// its samples one after the other, a line per lane, slot and sample, kept the address units busy 84 % of the
+// time: 30 samples of 7B on 4x8 0.55 ms; 0.33 with the thresholds from LDS, 0.16 with a summary's latency
+// computed once for all samples.)
+constexpr int kFilterShares = 4;
+constexpr int kFilterPitch = MIST_LC_TILE + 1;  // doubles; front and post of a sample
+template <bool kSamples>
+__global__ __launch_bounds__(kSamples ? kFilterShares * 64 : 64) void filter_kernel(
     const MistProblem prob, const MistGroupDesc *__restrict__ groups, int n_groups,
     const int32_t *__restrict__ block_prefix, int n_blocks, const double *__restrict__ stage_floor,
     const double *__restrict__ super_floor, const RatioList ratios, ReduceTables tabs) {
@@ -2126,11 +2136,23 @@ __global__ __launch_bounds__(MIST_LC_TILE) void filter_kernel(
   const int chunk = local_block / n_tiles, tile = local_block % n_tiles;
   const int share = tile % n_p, tile_rel = tile / n_p;
   const int n_stages = (int)((g->n_rows + kStageRows - 1) / kStageRows);
-  const int stage0 = (int)((int64_t)chunk * g->rows_per_chunk / kStageRows);
-  const int stage1 = min(stage0 + g->rows_per_chunk / kStageRows, n_stages);
-  const int super_first = stage0 / kSuperStages + share, super_last = (stage1 - 1) / kSuperStages;
+  int stage0 = (int)((int64_t)chunk * g->rows_per_chunk / kStageRows);
+  int stage1 = min(stage0 + g->rows_per_chunk / kStageRows, n_stages);
+  int super_first = stage0 / kSuperStages + share, super_last = (stage1 - 1) / kSuperStages, stride = n_p;
+  if (kSamples) {
+    const int64_t mine = (int64_t)chunk * n_p + share;  // the workgroups of the other shares have nothing to do
+    if (mine % kFilterShares != 0) return;
+    const int64_t all = ((int64_t)g->n_chunks * n_p + kFilterShares - 1) / kFilterShares * kFilterShares;
+    const int64_t at = mine + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int64_t n_supers = (n_stages + kSuperStages - 1) / kSuperStages;
+    super_first = (int)(n_supers * at / all);
+    super_last = (int)(n_supers * (at + 1) / all) - 1;
+    stride = 1;
+    stage0 = 0;
+    stage1 = n_stages;
+  }
 
-  const int L = prob.num_layers, n_pairs = L * (L + 1) / 2 + L, lane = threadIdx.x;
+  const int L = prob.num_layers, n_pairs = L * (L + 1) / 2 + L, lane = threadIdx.x & 63;
   const int pair_idx = (g->lc_tile_begin + tile_rel) * MIST_LC_TILE + lane;
   const bool active = pair_idx < n_pairs;
   const PairIndex pc = decode_pair(active ? pair_idx : 0);
@@ -2140,35 +2162,60 @@ __global__ __launch_bounds__(MIST_LC_TILE) void filter_kernel(
   const bool do_post = active && pc.c != pc.l - 1, do_pp = do_post && pc.l == L;
   const GroupModel m = group_model(prob, g);
   const double cutoff = stage_cost_cutoff(prob, m.inv_G64);
-  const double *slots = tabs.best +
-                        (g->cell_offset + ((int64_t)tile_rel * MIST_LC_TILE + lane) * slots_of(P)) * S;
+  const double *best = tabs.best + (g->cell_offset + (int64_t)tile_rel * MIST_LC_TILE * slots_of(P)) * S;
+  extern __shared__ double lds_thresholds[];  // [sample][front, post][pair]
+  if (kSamples) {
+    const int sample = min(lane & 31, S - 1), parts = np | (int)do_post << 30 | (int)((unsigned)do_pp << 31);
+    const Offsets offsets = group_offsets(m, ratios.r[sample]);
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    constexpr int kPairs = MIST_LC_TILE / kFilterShares;
+#pragma unroll
+    for (int i = 0; i < kPairs; i += 2) {
+      const int pair = wave * kPairs + i + (lane >> 5);
+      const uint32_t its = (uint32_t)__shfl(parts, pair);
+      const int n = (int)(its & 0x7fff);
+      const Threshold t(loosest_minima(true, best + (int64_t)pair * slots_of(P) * S + sample, S, P, n, n,
+                                       (its >> 30 & 1u) != 0, its >> 31 != 0, cutoff), offsets);
+      lds_thresholds[2 * sample * kFilterPitch + pair] = t.front;
+      lds_thresholds[(2 * sample + 1) * kFilterPitch + pair] = t.post;
+    }
+    __syncthreads();
+  }
 
-  // no lane's row can matter: the pseudo row against the loosest minima
-  auto closed = [&](const double *__restrict__ f, double ratio, const Threshold &t) {
+  // whether any lane's row can matter: the pseudo row against the loosest minima, of the sample before first
+  const double loosest_ratio = ratios.r[kSamples ? min(lane & 31, S - 1) : 0];
+  const Threshold loosest =
+      kSamples ? Threshold(0.0, 0.0)
+               : Threshold(loosest_minima(true, best + (int64_t)lane * slots_of(P), 1, P, np, np, do_post, do_pp, cutoff),
+                           group_offsets(m, loosest_ratio));
+  int s = 0;
+  auto passes = [&](const double *__restrict__ f) {
     float x, d;
     pair_latency(f, k, x, d);
-    return !__any(m.bound(ratio, x, d) <= t.at(post_layer_offset(m, ratio, f)));
+    if (!kSamples) return (bool)__any(m.bound(loosest_ratio, x, d) <= loosest.at(post_layer_offset(m, loosest_ratio, f)));
+    const double low_x = m.lower_x(x), low_share = m.lower_share(d);
+    for (int n = 0; n < S; ++n) {
+      const double ratio = from_lane(loosest_ratio, s);
+      const Threshold t(lds_thresholds[2 * s * kFilterPitch + lane], lds_thresholds[(2 * s + 1) * kFilterPitch + lane]);
+      if (__any(ratio * low_x + low_share <= t.at(post_layer_offset(m, ratio, f)))) return true;
+      s = s + 1 == S ? 0 : s + 1;
+    }
+    return false;
   };
   const double *__restrict__ supers = super_floor + super_floor_slot(g, gi, 0) * kStageFloorPitch;
   const double *__restrict__ stages = stage_floor + stage_floor_slot(g, gi, 0) * kStageFloorPitch;
   // batches of 64 summaries; lane i keeps the open stages of the batch's i-th
-  for (int first = super_first; first <= super_last; first += 64 * n_p) {
+  for (int first = super_first; first <= super_last; first += 64 * stride) {
     uint32_t open = 0;
-    for (int s = 0; s < S; ++s) {
-      const double ratio = ratios.r[s];
-      const Threshold t(loosest_minima(true, slots + s, S, P, np, np, do_post, do_pp, cutoff), group_offsets(m, ratio));
-      for (int i = 0; i < 64; ++i) {
-        const int super = first + i * n_p;
-        if (super > super_last) break;
-        const int st0 = max(super * kSuperStages, stage0), st1 = min((super + 1) * kSuperStages, stage1);
-        uint32_t seen = s > 0 ? (uint32_t)from_lane((int)open, i) : 0u;
-        if (seen == (1u << (st1 - st0)) - 1u) continue;
-        if (closed(supers + (int64_t)super * kStageFloorPitch, ratio, t)) continue;
-        for (int st = st0; st < st1; ++st)
-          if (!(seen >> (st - st0) & 1u) && !closed(stages + (int64_t)st * kStageFloorPitch, ratio, t))
-            seen |= 1u << (st - st0);
-        open = lane == i ? seen : open;
-      }
+    for (int i = 0; i < 64; ++i) {
+      const int super = first + i * stride;
+      if (super > super_last) break;
+      if (!passes(supers + (int64_t)super * kStageFloorPitch)) continue;
+      const int st0 = max(super * kSuperStages, stage0), st1 = min((super + 1) * kSuperStages, stage1);
+      uint32_t seen = 0;
+      for (int st = st0; st < st1; ++st)
+        if (passes(stages + (int64_t)st * kStageFloorPitch)) seen |= 1u << (st - st0);
+      open = lane == i ? seen : open;
     }
     // append the open stages to a shard of the queue, which one XCD works off, to the next ones if it is
     // full (all shards together hold every (tile, stage) of the launch).  One sample: the shard of the
@@ -2190,7 +2237,7 @@ __global__ __launch_bounds__(MIST_LC_TILE) void filter_kernel(
       base = (uint32_t)from_lane((int)base, 0);
       const int room = base >= tabs.capacity ? 0 : (int)min((uint32_t)(total - done), tabs.capacity - base);
       int at = end - mine;  // index of this lane's next item among the batch's
-      const int st0 = max((first + lane * n_p) * kSuperStages, stage0);
+      const int st0 = max((first + lane * stride) * kSuperStages, stage0);
       for (uint32_t rest = open; rest != 0; rest &= rest - 1, ++at) {
         if (at < done || at >= done + room) continue;
         const int st = st0 + __ffs(rest) - 1;
@@ -3996,10 +4043,13 @@ static int launch_reduce(const MistProblem *problem, const MistGroupDesc *d_grou
                          const int32_t *d_block_prefix, int n_blocks, const double *d_row_terms,
                          const double *d_stage_floor, const double *d_key_terms, const RatioList &ratios,
                          const ReduceTables &tabs, void *stream) {
-  hipLaunchKernelGGL(filter_kernel, dim3(xcd_padded_grid(n_blocks)), dim3(MIST_LC_TILE), 0, (hipStream_t)stream,
-                     *problem, d_groups, n_groups, d_block_prefix, n_blocks, d_stage_floor, tabs.super_floor, ratios, tabs);
+  const bool one = tabs.n_samples == 1;
+  hipLaunchKernelGGL(one ? filter_kernel<false> : filter_kernel<true>, dim3(xcd_padded_grid(n_blocks)),
+                     dim3(one ? 64 : kFilterShares * 64), one ? 0 : tabs.n_samples * 2 * kFilterPitch * sizeof(double),
+                     (hipStream_t)stream, *problem, d_groups, n_groups, d_block_prefix, n_blocks, d_stage_floor,
+                     tabs.super_floor, ratios, tabs);
   MIST_HIP_CHECK(hipGetLastError());
-  const bool one = tabs.n_samples == 1, buffered = one && slots_of(problem->reduce_max_p) <= kMostBufferedSlots;
+  const bool buffered = one && slots_of(problem->reduce_max_p) <= kMostBufferedSlots;
   hipLaunchKernelGGL(one ? open_kernel<false> : open_kernel<true>, dim3(kReduceBlocks), dim3(kReduceThreads), 0,
                      (hipStream_t)stream, *problem, d_groups, d_stage_floor, ratios, tabs);
   MIST_HIP_CHECK(hipGetLastError());
