@@ -1967,27 +1967,31 @@ __device__ __forceinline__ void put_sample_row(SampleRows *rows, int at, const R
   rows->counts[at] = (uint32_t)count_b | (uint32_t)count_p << 15 | (post ? 1u << 30 : 0u) | (pp ? 1u << 31 : 0u);
 }
 
-// Workgroup = one wavefront = one pair of a group with the minima of all its samples in LDS, a
-// column per sample.  Lane = row for the latencies and counts of 64 gathered rows, then lane = (row
+// Workgroup = one pair of a group with the minima of all its samples in LDS, a column per sample; its
+// wavefronts take 64 gathered rows each: lane = row for their latencies and counts, then lane = (row
 // parity, sample): one LDS minimum per (row, variant, sample) at the row's own count, conflict-free
-// but for the two rows in flight.  The minima per p are the suffix minima of those buckets.
+// but for the rows in flight.  The minima per p are the suffix minima of those buckets, a range of p
+// per wavefront.
 // (30 samples one after the other through seed_kernel: 3.1 ms for the tables of one tensor-parallel
-// size of the 7B plan.)
-__global__ __launch_bounds__(64) void seed_samples_kernel(
+// size of the 7B plan.  One wavefront a pair: its minima leave room for four on a CU, 0.47 ms; now 0.33. 7B on
+// 4x8 0.43 -> 0.38, on 1x8 0.096 -> 0.075; eight wavefronts 0.39, 0.43, 0.11.)
+constexpr int kSeedSampleWaves = 4;
+__global__ __launch_bounds__(64 * kSeedSampleWaves) void seed_samples_kernel(
     const MistProblem prob, const MistGroupDesc *__restrict__ groups, const double *__restrict__ row_terms,
     const RatioList ratios, ReduceTables tabs, int sample_split) {
   extern __shared__ double lds_best[];
   const MistGroupDesc *g = groups + blockIdx.y;
   clear_queue(tabs);
-  const int tile_rel = (int)blockIdx.x / MIST_LC_TILE, lane = threadIdx.x;
+  const int tile_rel = (int)blockIdx.x / MIST_LC_TILE, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), n_waves = blockDim.x >> 6;
   if (tile_rel >= g->n_lc_tiles) return;
   const int L = prob.num_layers, n_pairs = L * (L + 1) / 2 + L;
   const int P = g->num_p, n_slots = slots_of(P);
   const int first_sample = (int)blockIdx.z * sample_split, S = min(sample_split, tabs.n_samples - first_sample);
   const int pair = g->lc_tile_begin * MIST_LC_TILE + (int)blockIdx.x;
-  SampleRows *rows = reinterpret_cast<SampleRows *>(lds_best);
-  double *mine = lds_best + sizeof(SampleRows) / 8;  // [slot][sample]
-  for (int e = lane; e < n_slots * S; e += 64) mine[e] = INFINITY;
+  SampleRows *rows = reinterpret_cast<SampleRows *>(lds_best) + wave;
+  double *mine = lds_best + sizeof(SampleRows) / 8 * n_waves;  // [slot][sample]
+  for (int e = threadIdx.x; e < n_slots * S; e += blockDim.x) mine[e] = INFINITY;
   __syncthreads();
   const int sample = lane & 31;
   if (g->scout_stride > 0 && pair < n_pairs) {
@@ -2000,7 +2004,7 @@ __global__ __launch_bounds__(64) void seed_samples_kernel(
     const double ratio = ratios.r[first_sample + min(sample, S - 1)];
     const int n_gather = g->n_par * g->n_oo * g->n_ao * g->scout_stride;
     const double *__restrict__ src = row_terms + g->row_offset * MIST_ROW_TERMS;
-    for (int q0 = 0; q0 < n_gather; q0 += 64) {
+    for (int q0 = wave * 64; q0 < n_gather; q0 += 64 * n_waves) {
       const int n_rows = min(64, n_gather - q0);
       RowRegs t;
       load_terms<0, MIST_ROW_TERMS>(t, src + gathered_position(g, (uint32_t)min(q0 + lane, n_gather - 1)) * MIST_ROW_TERMS);
@@ -2015,11 +2019,12 @@ __global__ __launch_bounds__(64) void seed_samples_kernel(
       ok_pp = ok_pp && do_pp && lane < n_rows;
       // (rows that fit nowhere are left out)
       const uint64_t useful = __ballot(cnt.b > 0 || cnt.p > 0 || ok_post || ok_pp);
-      __syncthreads();
+      __builtin_amdgcn_wave_barrier();
       if (useful >> lane & 1ull)
         put_sample_row(rows, __popcll(useful & ((1ull << lane) - 1ull)), t, x, d, k.no_ck, m, cnt.b, cnt.p, ok_post,
                        ok_pp, do_post);
-      __syncthreads();
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
       const int n_useful = __popcll(useful);
       for (int r = lane >> 5; r < n_useful; r += 2) {
         const uint32_t counts = rows->counts[r];
@@ -2040,19 +2045,24 @@ __global__ __launch_bounds__(64) void seed_samples_kernel(
   }
   __syncthreads();
   const int64_t cell0 = g->cell_offset + (int64_t)blockIdx.x * n_slots;
+  const int v = lane >> 5;  // base, with_pre
+  const int first_p = P * wave / n_waves, end_p = P * (wave + 1) / n_waves;
+  double low = INFINITY;
+  if (sample < S)
+    for (int j = end_p; j < P; ++j) low = fmin(low, mine[(v * P + j) * S + sample]);
   if (sample < S) {
-    const int v = lane >> 5;  // base, with_pre
     const int64_t at = cell0 * tabs.n_samples + first_sample + sample;
-    double low = INFINITY;
-    for (int j = P - 1; j >= -1; --j) {
-      const int slot = j >= 0 ? v * P + j : 2 * P + v;
-      const double held = mine[slot * S + sample];
-      low = j >= 0 ? fmin(low, held) : held;
-      tabs.best[at + (int64_t)slot * tabs.n_samples] = low;
+    auto put = [&](int slot, double value) {
+      tabs.best[at + (int64_t)slot * tabs.n_samples] = value;
       tabs.row[at + (int64_t)slot * tabs.n_samples] = ~0u;
+    };
+    for (int j = end_p - 1; j >= first_p; --j) {
+      low = fmin(low, mine[(v * P + j) * S + sample]);
+      put(v * P + j, low);
     }
+    if (wave == 0) put(2 * P + v, mine[(2 * P + v) * S + sample]);
   }
-  if (lane == 0 && first_sample == 0) tabs.changed[cell0 / 4] = 0;
+  if (threadIdx.x == 0 && first_sample == 0) tabs.changed[cell0 / 4] = 0;
 }
 
 // ---- summaries of kSuperStages stages ----
@@ -3990,8 +4000,9 @@ static int launch_seeds(const MistProblem *problem, const MistGroupDesc *d_group
   while (pair_split > 4 && (int64_t)tiles * (MIST_LC_TILE / pair_split) * n_groups < kSeedWorkgroups) pair_split /= 2;
   int sample_split = tabs.n_samples;
   while (sample_split > 1 && pair_bytes * sample_split > kSeedLdsBytes) sample_split = (sample_split + 1) / 2;
-  const int64_t bytes =
-      pair_bytes * pair_split * sample_split + (tabs.n_samples == 1 ? 0 : (int64_t)sizeof(SampleRows));
+  int sample_waves = tabs.n_samples == 1 ? 0 : kSeedSampleWaves;
+  while (sample_waves > 1 && pair_bytes + sample_waves * (int64_t)sizeof(SampleRows) > kSeedLdsMost) sample_waves /= 2;
+  const int64_t bytes = pair_bytes * pair_split * sample_split + sample_waves * (int64_t)sizeof(SampleRows);
   const bool seeds = scouted && bytes <= kSeedLdsMost;  // (some 10000 values of p)
   const bool estimate = scouted && problem->stage_cost_incumbent != nullptr && problem->incumbent_first_estimate != 0 &&
                         tabs.n_samples == 1;
@@ -4019,7 +4030,7 @@ static int launch_seeds(const MistProblem *problem, const MistGroupDesc *d_group
     hipLaunchKernelGGL(seed_kernel, grid, dim3(kSeedThreads), (size_t)bytes, (hipStream_t)stream, *problem, d_groups,
                        d_row_terms, ratios.r[0], tabs, pair_split);
   else
-    hipLaunchKernelGGL(seed_samples_kernel, grid, dim3(64), (size_t)bytes, (hipStream_t)stream, *problem, d_groups,
+    hipLaunchKernelGGL(seed_samples_kernel, grid, dim3(64 * sample_waves), (size_t)bytes, (hipStream_t)stream, *problem, d_groups,
                        d_row_terms, ratios, tabs, sample_split);
   MIST_HIP_CHECK(hipGetLastError());
   if (scouted && problem->stage_cost_incumbent != nullptr && tabs.n_samples == 1) {
