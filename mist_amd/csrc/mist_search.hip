@@ -2329,14 +2329,15 @@ __device__ __forceinline__ TileLane tile_lane(const MistProblem &prob, const Mis
 // stays, with a word of its open pairs (7B on 4x8: 454000 stages x tiles, 36300 pass the filter and
 // 13700 of those are opened; 22B on 16x8: 21.1e6, 2.1e6, 0.45e6).  Items of a run are mostly the
 // stages of one tile, whose pairs, constants and offsets stay in registers.
-//   One sample: lane = pair; VALU issue and the gather of minima, a line per lane and load, bound it (an
-//   item of its own per wavefront, everything computed again for each, 540 VALU instructions: 22B
-//   2.9 ms; now 2.2).
+//   One sample: lane = pair; the latency of an item bounds it (an item of its own per wavefront, everything
+//   computed again for each, 540 VALU instructions: 22B 2.9 ms; constants of the tile kept 2.2; the next
+//   item's summary through LDS 1.9; one append a run instead of three dependent atomics an opened item 1.5;
+//   70B on 32x8 0.92 -> 0.38.  Gathering minima only for pairs below the filter's thresholds: no change).
 //   Several: lane = pair for what the stage can reach, then lane = (pair parity, sample): the minima of a
 //   slot lie side by side, two lines per load (lane = pair through all samples, a line per lane and load,
 //   kept the address units busy 82 % of the time: 30 samples of 7B for one tensor-parallel size 1.41 ms;
 //   now 0.45, and it knows every open pair: the reduce launch tries 1.4e6 instead of 2.9e6).
-constexpr int kOpenRun = 16;
+constexpr int kOpenRun = 16;  // (items kept by lanes)
 template <bool kSamples>
 __global__ __launch_bounds__(kReduceThreads) void open_kernel(const MistProblem prob,
                                                               const MistGroupDesc *__restrict__ groups,
@@ -2359,21 +2360,67 @@ __global__ __launch_bounds__(kReduceThreads) void open_kernel(const MistProblem 
   double cutoff = INFINITY;
   int P = 1;
   const double *best = tabs.best;
+  // (the next item's summary is on its way to LDS while one is worked on, and the word of the one after it)
+  __shared__ double lds_floor[kWaves][2][kStageFloorPitch];
+  double(*const floor_of)[kStageFloorPitch] = lds_floor[threadIdx.x >> 6];
+  auto floor_term = [&](uint64_t word) {
+    const Item item(word);
+    return stage_floor[stage_floor_slot(groups + item.group, item.group, item.stage) * kStageFloorPitch +
+                       lane % kStageFloorPitch];
+  };
+  // what a run opens is appended together, lane = item
+  uint64_t kept_word = 0, kept_open = 0;
+  uint32_t kept_shard = 0;
+  int n_kept = 0;
+  auto append = [&]() {
+    if (n_kept == 0) return;
+    const bool mine = lane < n_kept;
+    const int64_t shard0 = (int64_t)kept_shard * tabs.capacity;
+    // (no more than the shard's items are opened: it cannot overflow)
+    uint32_t base = 0;
+    if (lane == 0) base = atomicAdd(tabs.counter + (kQueueShards + kept_shard) * kCounterPitch, (uint32_t)n_kept);
+    base = (uint32_t)from_lane((int)base, 0);
+    if (mine) {
+      tabs.opened[shard0 + base + lane] = kept_word;
+      tabs.hit[shard0 + base + lane] = kept_open;
+    }
+    n_kept = 0;
+    if (tabs.listed == nullptr) return;
+    const Item item(kept_word);
+    bool fresh = false;
+    if (mine)
+      fresh = atomicExch(tabs.stage_flag + stage_floor_slot(groups + item.group, item.group, item.stage), 1u) == 0;
+    const uint64_t listed = __ballot(fresh);
+    if (listed == 0) return;
+    if (lane == 0)
+      base = atomicAdd(tabs.counter + (2 * kQueueShards + kept_shard) * kCounterPitch, (uint32_t)__popcll(listed));
+    base = (uint32_t)from_lane((int)base, 0);
+    if (fresh)
+      tabs.listed[shard0 + base + __popcll(listed & ((1ull << lane) - 1ull))] =
+          (unsigned long long)item.group << 32 | (uint32_t)item.stage;
+  };
   for (uint32_t first = wave * run; first < queue.total; first += n_waves * run) {
     const uint32_t end = min(first + run, queue.total);
-    int64_t from = queue.at(first, tabs.capacity);
-    uint64_t ahead = tabs.item[from];
+    int64_t from = queue.at(first, tabs.capacity), from_next = queue.at(min(first + 1, end - 1), tabs.capacity);
+    uint64_t word = from_lane((uint64_t)tabs.item[from], 0), ahead = tabs.item[from_next];
+    double term = floor_term(word);
     for (uint32_t i = first; i < end; ++i) {
-      const uint64_t word = from_lane(ahead, 0);
+      double *const f = floor_of[i & 1];
+      __builtin_amdgcn_wave_barrier();
+      if (lane < kStageFloorPitch) f[lane] = term;
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
       const uint32_t shard = (uint32_t)(from / tabs.capacity);
-      if (i + 1 < end) {
-        from = queue.at(i + 1, tabs.capacity);
-        ahead = tabs.item[from];
-      }
       const Item item(word);
+      const uint64_t its_word = word;
+      from = from_next;
+      word = from_lane(ahead, 0);
+      term = floor_term(word);
+      from_next = queue.at(min(i + 2, end - 1), tabs.capacity);
+      ahead = tabs.item[from_next];
       const int gi = item.group, stage = item.stage;
-      if (word >> kItemStageBits != tile_word) {
-        tile_word = word >> kItemStageBits;
+      if (its_word >> kItemStageBits != tile_word) {
+        tile_word = its_word >> kItemStageBits;
         g = groups + gi;
         p = tile_lane(prob, g, item.tile);
         k = pair_consts(p.pc.l, p.pc.c);
@@ -2383,7 +2430,6 @@ __global__ __launch_bounds__(kReduceThreads) void open_kernel(const MistProblem 
         P = g->num_p;
         best = tabs.best + (g->cell_offset + (int64_t)item.tile * MIST_LC_TILE * slots_of(P)) * S;
       }
-      const double *__restrict__ f = stage_floor + stage_floor_slot(g, gi, stage) * kStageFloorPitch;
       const StageReach reach = stage_reach(f, k, p.np, p.do_post, p.do_pp, m);
       const double post_layer = post_layer_offset(m, ratio, f);
       uint64_t open = 0;
@@ -2411,17 +2457,15 @@ __global__ __launch_bounds__(kReduceThreads) void open_kernel(const MistProblem 
         }
       }
       if (open == 0) continue;
-      if (lane == 0) {
-        // (no more than the shard's items are opened: it cannot overflow)
-        const uint32_t to = atomicAdd(tabs.counter + (kQueueShards + shard) * kCounterPitch, 1u);
-        tabs.opened[(int64_t)shard * tabs.capacity + to] = word;
-        tabs.hit[(int64_t)shard * tabs.capacity + to] = open;
-        if (tabs.listed != nullptr && atomicExch(tabs.stage_flag + stage_floor_slot(g, gi, stage), 1u) == 0) {
-          const uint32_t row_to = atomicAdd(tabs.counter + (2 * kQueueShards + shard) * kCounterPitch, 1u);
-          tabs.listed[(int64_t)shard * tabs.capacity + row_to] = (unsigned long long)gi << 32 | (uint32_t)stage;
-        }
+      if (n_kept > 0 && shard != kept_shard) append();
+      kept_shard = shard;
+      if (lane == n_kept) {
+        kept_word = its_word;
+        kept_open = open;
       }
+      ++n_kept;
     }
+    append();
   }
 }
 
