@@ -1748,20 +1748,45 @@ __global__ __launch_bounds__(kDpHistoryThreads, 8) void dp_history_kernel(
 // kDpFreeLoads reads of a lane in flight), then a wavefront takes a start layer with its lanes on
 // the end layers.  Bound: latency of that gather and two barriers, 2.5 us per stage count at 37
 // layers.  Six families of that plan: 250 launches, 3.3 ms from the first to the last -> 18, 0.75.
+// The families of a search wait for nothing of each other: up to kDpFreeFamilies go through one
+// launch, workgroup = (instance, family), the ones given last (more stage counts as a rule) first:
+// 24 launches, 0.89 ms of 13B on 4x8 -> 4, 0.50.
 // ------------------------------------------------------------------------------------------
 constexpr int kDpFreeThreads = 512;
 constexpr int kDpFreeLoads = 4;
+constexpr int kDpFreeFamilies = 8;
+struct DpFreeFamily {
+  MistDpCosts costs;
+  int32_t max_stages, p_dim, ckpt_rule, mesh_n, mesh_m;
+  int32_t *best_s, *path;
+  float *best_sum, *stage_max;
+};
+struct DpFreeFamilies {
+  DpFreeFamily family[kDpFreeFamilies];
+};
 inline size_t dp_free_lds(int L, int S) {
   return ((size_t)L * L + (size_t)(S + 1) * (L + 1) + S) * sizeof(float);
 }
 
 template <bool kBottleneck>
 __global__ __launch_bounds__(kDpFreeThreads) void dp_free_kernel(
-    const MistDpShape shape, const MistDpCosts tabs, const float *__restrict__ tmax_list,
-    const int32_t *__restrict__ g_list, int32_t *__restrict__ best_s_out,
-    float *__restrict__ best_sum_out, float *__restrict__ stage_max_out,
-    int32_t *__restrict__ path_out) {
+    const DpFreeFamilies families, int num_layers, const float *__restrict__ tmax_list,
+    const int32_t *__restrict__ g_list) {
   extern __shared__ float dp_lds[];
+  const DpFreeFamily &its = families.family[gridDim.y - 1 - blockIdx.y];
+  const MistDpCosts tabs = its.costs;
+  int32_t *__restrict__ best_s_out = its.best_s, *__restrict__ path_out = its.path;
+  float *__restrict__ best_sum_out = its.best_sum, *__restrict__ stage_max_out = its.stage_max;
+  MistDpShape shape;  // (of one mesh)
+  shape.num_layers = num_layers;
+  shape.num_devices = 0;
+  shape.num_mesh = 1;
+  shape.p_dim = its.p_dim;
+  shape.max_stages = its.max_stages;
+  shape.ckpt_rule = its.ckpt_rule;
+  shape.free_devices = 1;
+  shape.mesh_n[0] = its.mesh_n;
+  shape.mesh_m[0] = its.mesh_m;
   const int L = shape.num_layers, S = shape.max_stages;
   float *rows = dp_lds;                             // [L][L] (stage layers - 1, end layer)
   float *history = rows + L * L;                    // [S + 1][L + 1]
@@ -2336,6 +2361,47 @@ int mist::dp_stage_rates(const MistDpShape &shape, const MistDpCosts &costs, int
   return 0;
 }
 
+// Whether the whole recurrence of one mesh fits a workgroup.
+static bool dp_free_runs(const MistDpShape &shape) {
+  return shape.free_devices != 0 && dp_free_lds(shape.num_layers, shape.max_stages) <= 64 * 1024;
+}
+static int launch_dp_free(const mist::DpFreeRun *runs, int n, const float *d_tmax, const int32_t *d_g_index, int n_tmax,
+                          int mode, hipStream_t stream) {
+  for (int first = 0; first < n; first += kDpFreeFamilies) {
+    const int here = std::min(n - first, kDpFreeFamilies), L = runs[first].shape->num_layers;
+    DpFreeFamilies families = {};
+    size_t lds = 0;
+    for (int f = 0; f < here; ++f) {
+      const mist::DpFreeRun &run = runs[first + f];
+      const MistDpShape &shape = *run.shape;
+      families.family[f] = {*run.costs, shape.max_stages, shape.p_dim, shape.ckpt_rule, shape.mesh_n[0], shape.mesh_m[0],
+                            run.d_best_s, run.d_path, run.d_best_sum, run.d_stage_max};
+      lds = std::max(lds, dp_free_lds(L, shape.max_stages));
+    }
+    if (mode == MIST_DP_BOTTLENECK)
+      hipLaunchKernelGGL(dp_free_kernel<true>, dim3(n_tmax, here), dim3(kDpFreeThreads), lds, stream, families, L, d_tmax,
+                         d_g_index);
+    else
+      hipLaunchKernelGGL(dp_free_kernel<false>, dim3(n_tmax, here), dim3(kDpFreeThreads), lds, stream, families, L, d_tmax,
+                         d_g_index);
+    MIST_HIP_CHECK(hipGetLastError());
+  }
+  return 0;
+}
+
+int mist::dp_run_free(const DpFreeRun *runs, int n, const float *d_tmax, const int32_t *d_g_index, int n_tmax, int mode,
+                      hipStream_t stream) {
+  const char *forced = getenv("MIST_DP_FORCE_SCHEDULE");
+  if (forced && *forced) return 1;
+  for (int f = 0; f < n; ++f)
+    if (!dp_free_runs(*runs[f].shape) || runs[f].shape->num_layers != runs[0].shape->num_layers) return 1;
+  for (int f = 0; f < n; ++f)
+    if (int rc = check_run_arguments(runs[f].shape, runs[f].costs, d_tmax, d_g_index, n_tmax, mode, runs[f].d_best_s,
+                                     runs[f].d_best_sum, runs[f].d_stage_max))
+      return rc;
+  return launch_dp_free(runs, n, d_tmax, d_g_index, n_tmax, mode, stream);
+}
+
 int mist::dp_run(const MistDpShape *shape, const MistDpCosts *costs, const float *d_rates, const float *d_tmax,
                  const int32_t *d_g_index, int n_tmax, int mode, int32_t *d_best_s, float *d_best_sum,
                  float *d_stage_max, int32_t *d_argmin, int32_t *d_path, float *d_scratch, int64_t scratch_floats,
@@ -2375,18 +2441,9 @@ int mist::dp_run(const MistDpShape *shape, const MistDpCosts *costs, const float
   // Without back-pointers and with room for the history that schedule runs: it was the fastest at
   // every shape and batch size measured (33 x 33 to 81 x 257 states, 28 to 2304 instances).
   if (!(force_step || force_fused || force_plane)) {
-    const size_t free_lds = dp_free_lds(shape->num_layers, shape->max_stages);
-    if (shape->free_devices != 0 && !whole_argmin && free_lds <= 64 * 1024) {
-      if (mode == MIST_DP_BOTTLENECK)
-        hipLaunchKernelGGL(dp_free_kernel<true>, dim3(n_tmax), dim3(kDpFreeThreads), free_lds,
-                           (hipStream_t)stream, *shape, *costs, d_tmax, d_g_index, d_best_s,
-                           d_best_sum, d_stage_max, d_path);
-      else
-        hipLaunchKernelGGL(dp_free_kernel<false>, dim3(n_tmax), dim3(kDpFreeThreads), free_lds,
-                           (hipStream_t)stream, *shape, *costs, d_tmax, d_g_index, d_best_s,
-                           d_best_sum, d_stage_max, d_path);
-      MIST_HIP_CHECK(hipGetLastError());
-      return 0;
+    if (!whole_argmin && dp_free_runs(*shape)) {
+      const mist::DpFreeRun run = {shape, costs, d_best_s, d_best_sum, d_stage_max, d_path};
+      return launch_dp_free(&run, 1, d_tmax, d_g_index, n_tmax, mode, (hipStream_t)stream);
     }
     const HistoryPlan plan = history_plan(*shape, n_tmax);
     const int cols = (shape->num_devices + 63) / 64;

@@ -1,4 +1,5 @@
-// Between the DP and the search driver: mist_dp_run_sized with what ends an instance early.
+// Between the DP and the search driver: mist_dp_run_sized with what ends an instance early, and several
+// families of one mesh at a time.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -15,4 +16,16 @@ int dp_stage_rates(const MistDpShape &shape, const MistDpCosts &costs, int n_g, 
 int dp_run(const MistDpShape *shape, const MistDpCosts *costs, const float *d_rates, const float *d_tmax,
            const int32_t *d_g_index, int n_tmax, int mode, int32_t *d_best_s, float *d_best_sum, float *d_stage_max,
            int32_t *d_argmin, int32_t *d_path, float *d_scratch, int64_t scratch_floats, void *stream);
+
+struct DpFreeRun {
+  const MistDpShape *shape;
+  const MistDpCosts *costs;
+  int32_t *d_best_s;
+  float *d_best_sum, *d_stage_max;
+  int32_t *d_path;  // may be null
+};
+// dp_run of the same instances for every family, all on one mesh, without a launch per family; > 0 and nothing
+// is done where a family needs another schedule.
+int dp_run_free(const DpFreeRun *runs, int n, const float *d_tmax, const int32_t *d_g_index, int n_tmax, int mode,
+                hipStream_t stream);
 }  // namespace mist

@@ -409,15 +409,25 @@ struct Search {
     float *d_in = ws->d_in.as<float>();
     const int32_t *d_g = reinterpret_cast<int32_t *>(d_in + n);
     const bool known = *std::max_element(g_index.begin(), g_index.end()) < n_rates;
-    // the families share the state planes and the back-pointer slab: they run one after the
-    // other on the stream
+    std::vector<mist::DpFreeRun> together;
+    std::vector<MistDpShape> its_shapes;
+    for (int f = 0; f < n_families; ++f) its_shapes.push_back(shape_of(f));
+    for (int f = 0; f < n_families; ++f) {
+      float *d_out = ws->d_out.as<float>() + (size_t)f * 3 * n;
+      together.push_back({&its_shapes[f], &costs[f], reinterpret_cast<int32_t *>(d_out), d_out + n, d_out + 2 * n,
+                          want_path ? d_paths + path_offset(f, n) : nullptr});
+    }
+    const int apart = mist::dp_run_free(together.data(), n_families, d_in, d_g, n, mode, stream);
+    if (apart < 0) return apart;
+    // otherwise the families share the state planes and the back-pointer slab: they run one after
+    // the other on the stream
     for (int f = 0; f < n_families; ++f) {
       float *d_out = ws->d_out.as<float>() + (size_t)f * 3 * n;
       int32_t *d_argmin = want_path ? ws->d_argmin.as<int32_t>() : nullptr;  // no fill: the
                                                      // walk reads what the DP wrote
       int32_t *d_path = want_path ? d_paths + path_offset(f, n) : nullptr;
-      const MistDpShape shape = shape_of(f);
-      if (int rc = mist::dp_run(&shape, &costs[f], known ? rates_of(f) : nullptr, d_in, d_g, n, mode,
+      const MistDpShape &shape = its_shapes[f];
+      if (int rc = apart == 0 ? 0 : mist::dp_run(&shape, &costs[f], known ? rates_of(f) : nullptr, d_in, d_g, n, mode,
                                 reinterpret_cast<int32_t *>(d_out), d_out + n, d_out + 2 * n, d_argmin,
                                 d_path, ws->d_scratch.as<float>(), n_scratch, stream))
         return rc;
@@ -562,7 +572,16 @@ struct Search {
             reinterpret_cast<int32_t *>(d_first + at_meta), ws->d_inst_t.as<float>(),
             ws->d_inst_row.as<int32_t>(), stream))
       return rc;
+    std::vector<mist::DpFreeRun> together;
     for (int f = 0; f < n_families; ++f) {
+      float *d_out = d_first + at_out + (size_t)f * 3 * n_inst;
+      together.push_back({&shapes[f], &costs[f], reinterpret_cast<int32_t *>(d_out), d_out + n_inst, d_out + 2 * n_inst,
+                          nullptr});
+    }
+    const int apart = mist::dp_run_free(together.data(), n_families, ws->d_inst_t.as<float>(),
+                                        ws->d_inst_row.as<int32_t>(), n_inst, MIST_DP_THRESHOLD, stream);
+    if (apart < 0) return apart;
+    for (int f = 0; f < n_families && apart != 0; ++f) {
       float *d_out = d_first + at_out + (size_t)f * 3 * n_inst;
       if (int rc = mist::dp_run(&shapes[f], &costs[f], rates_of(f), ws->d_inst_t.as<float>(),
                                 ws->d_inst_row.as<int32_t>(), n_inst, MIST_DP_THRESHOLD,
