@@ -52,16 +52,19 @@ constexpr int kDpBatch = 4;  // end layers whose reads a lane of the one-lane-pe
 // row index is -1 and their costs +inf, so with the index table (may be null) the 16 bytes of
 // such a cell's costs are not read.
 // The four tables of a call (base, with_pre, with_post, no_pp) go through one launch: table v
-// owns the workgroups first_block[v] .. first_block[v + 1] - 1.  A workgroup takes kCostRuns sets
+// owns the workgroups first_block[v] .. first_block[v + 1] - 1.  A workgroup takes up to kCostRuns sets
 // of rows one after the other: with one each, its own start and a division per lane were the bound.
+// Small tables, whose workgroups are all resident, take fewer (1.3B on 1x2: eight 14.4 us, one 5.3).
 // Bound: 12 bytes a cell and 16 more where it holds a row.
 constexpr int kCostRuns = 8;
+constexpr int kCostResident = 2048;  // workgroups at a time, eight per CU
 struct CostTableJob {
   const double *stable[4], *delta[4];
   const int32_t *index[4];
   float *out[4], *pmin[4];
   int64_t n_rows[4], rows_per_g[4];
   unsigned first_block[5];
+  int runs;  // sets of rows per workgroup
 };
 // `run` of the lane `control` names, where it is `distance` back in the same row of the table;
 // a lane without a source keeps its own
@@ -115,9 +118,9 @@ __global__ __launch_bounds__(256) void cost_rows_kernel(const CostTableJob job, 
   }
   const int back = min((int)threadIdx.x - ((cell0 + 3 - j[3]) >> 2), lane);  // to where the last cell's row begins
   const bool spills = cell0 - j[0] < wave * 256;  // the first cell's begins in an earlier wavefront
-  const int64_t row0 = (int64_t)(blockIdx.x - job.first_block[v]) * rows_here * kCostRuns;
+  const int64_t row0 = (int64_t)(blockIdx.x - job.first_block[v]) * rows_here * job.runs;
   int64_t g = row0 / per_g, in_g = row0 - g * per_g;
-  for (int turn = 0; turn < kCostRuns; ++turn) {
+  for (int turn = 0; turn < job.runs; ++turn) {
     const int64_t row = row0 + turn * rows_here;
     if (row >= n_rows) break;
     const int n_cells = (int)min((int64_t)cells_here, (n_rows - row) * row_len);
@@ -213,10 +216,10 @@ __global__ __launch_bounds__(256) void cost_table_kernel(const CostTableJob job,
   const int local_row = threadIdx.x / seg, j0 = threadIdx.x % seg;
   // (rows_per_g is the size of one g: 32 bits)
   const uint32_t per_g = (uint32_t)rows_per_g;
-  const int64_t row0 = (int64_t)(blockIdx.x - job.first_block[v]) * rows_here * kCostRuns;
+  const int64_t row0 = (int64_t)(blockIdx.x - job.first_block[v]) * rows_here * job.runs;
   const int64_t g0 = row0 >> 32 == 0 ? (int64_t)((uint32_t)row0 / per_g) : row0 / rows_per_g;
   const uint32_t in_g0 = (uint32_t)(row0 - g0 * rows_per_g);
-  for (int turn = 0; turn < kCostRuns; ++turn) {
+  for (int turn = 0; turn < job.runs; ++turn) {
     const uint32_t ahead = (uint32_t)(turn * rows_here + local_row);
     const int64_t r = row0 + ahead;
     if (row0 + turn * rows_here >= n_rows) break;
@@ -2159,9 +2162,12 @@ int mist_dp_cost_tables(const MistProblem *problem, const MistOutTables *tables,
   if (slot < 0 || slot >= S) return fail(MIST_E_INVALID, "slot %d outside [0, %d)", slot, (int)S);
   const int64_t rows_per_g[4] = {Q * P1 * L, Q * P1 * L, Q * L, Q};
   const bool wide = S == 1 && L + 1 <= 256;  // four neighbouring cells a lane, rows of a wavefront's cells at most
-  const int64_t rows_per_block =
-      (wide ? (kCostCells / (L + 1)) & ~3ll : 256 / std::min<int64_t>(L + 1, 256)) * kCostRuns;
+  const int64_t rows_per_set = wide ? (kCostCells / (L + 1)) & ~3ll : 256 / std::min<int64_t>(L + 1, 256);
+  int64_t sets = 0;
+  for (int v = 0; v < 4; ++v) sets += Gn * rows_per_g[v] / rows_per_set;
   CostTableJob job = {};
+  job.runs = (int)std::max<int64_t>(1, std::min<int64_t>(kCostRuns, sets / kCostResident));
+  const int64_t rows_per_block = rows_per_set * job.runs;
   int64_t blocks = 0;
   for (int v = 0; v < 4; ++v) {
     if (!tables->stable[v] || !tables->delta[v] || !d_out[v] || !d_out_pmin[v])

@@ -1199,8 +1199,10 @@ __device__ __forceinline__ void take_min(double &best, int32_t &best_row, bool f
 //   filter   stage summaries (term-wise minima of 64 rows, and of 8 such stages) against the
 //            largest minimum of each pair; what some pair of a tile does not rule out becomes an
 //            item (group, tile, stage) of a queue;
-//   open     a wavefront per item: the summary with the minima of the slots the stage can reach;
-//   reduce   what is left, shared out by pairs: lane = row over the open pairs.  A row whose cost
+//   open     runs of items per wavefront: the summary with the minima of the slots the stage can reach;
+//            which pairs stay open goes along;
+//   reduce   what is left, shared out by pairs: linear bounds of 64 rows against a pair's minima, then
+//            the reference's arithmetic for the candidates of several pairs.  A row whose cost
 //            IS the minimum at its own slot (count - 1) offers its row number there (the lowest
 //            one stays, which is the reference's first-index-wins scan, pareto.py:134-142, in any
 //            processing order); a smaller cost lowers the minimum and marks the pair, whose row
@@ -1211,9 +1213,9 @@ __device__ __forceinline__ void take_min(double &best, int32_t &best_row, bool f
 // What this replaces kept 34 (cost, row) minima per lane in registers (253 of them, two
 // wavefronts per SIMD), one sample and 16 p values per pass over the rows, visited every stage
 // summary with every tile and p tile, and committed rows one by one per lane: 7B on 4x8, one
-// sample: 1.35 ms (0.42 of it seeds); now seeds 0.29 beside key terms and summaries, filter 0.06, open 0.05,
-// reduce 0.27, resolve 0.05.  30 samples of the 7B plan's tables for one tensor-parallel size: 24 ms;
-// now 8.0 (reduce 4.2, open 1.4, resolve 1.3, filter 0.65, seeds 0.47).
+// sample: 1.35 ms (0.42 of it seeds); now seeds 0.26 beside key terms and summaries, filter 0.04, open 0.04,
+// reduce 0.19, resolve 0.03.  30 samples of the 7B plan's tables for one tensor-parallel size: 24 ms;
+// now 3.7 (reduce 2.1, resolve 0.57, open 0.42, seeds 0.33, filter 0.17).
 // ------------------------------------------------------------------------------------------
 constexpr int kSuperStages = 8;    // stages per second-level summary
 constexpr int kGatherFloor = 5;    // linear bounds of 64 gathered rows
