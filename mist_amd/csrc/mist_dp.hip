@@ -255,6 +255,15 @@ __global__ __launch_bounds__(256) void cost_table_kernel(const CostTableJob job,
   }
 }
 
+// Counters and instance slots of a first batch before it: one launch (two fills of the runtime take three, 5 us
+// of the chain each).
+__global__ __launch_bounds__(256) void window_clear_kernel(int32_t *__restrict__ counts, int n_counts,
+                                                           int32_t *__restrict__ inst_row, int n_inst) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n_counts) counts[i] = 0;
+  if (i < n_inst) inst_row[i] = -1;
+}
+
 // ------------------------------------------------------------------------------------------
 // t_max candidates of a value window: one pass over the three cost tables of a table row g
 // (costs, with_pre, with_post; inter_tuning.py:180-186).  Request r selects the finite values v
@@ -2319,8 +2328,10 @@ int mist_dp_windows_first_batch(const MistDpCosts *costs, int n_requests, const 
                 first_chunk, n_requests);
   if (first_lead < 1) return fail(MIST_E_INVALID, "first_lead %d < 1", first_lead);
   hipStream_t st = (hipStream_t)stream;
-  MIST_HIP_CHECK(hipMemsetAsync(d_counts, 0, sizeof(int32_t) * (2 + 2 * (size_t)n_requests), st));
-  MIST_HIP_CHECK(hipMemsetAsync(d_inst_row, 0xFF, sizeof(int32_t) * (size_t)n_requests * first_chunk, st));
+  const int n_counts = 2 + 2 * n_requests, n_inst = n_requests * first_chunk;
+  hipLaunchKernelGGL(window_clear_kernel, dim3((unsigned)((std::max(n_counts, n_inst) + 255) / 256)), dim3(256), 0, st,
+                     d_counts, n_counts, d_inst_row, n_inst);
+  MIST_HIP_CHECK(hipGetLastError());
   const int64_t per_row = costs->g_stride[0] + costs->g_stride[1] + costs->g_stride[2];
   const unsigned blocks = (unsigned)std::min<int64_t>((per_row + 16383) / 16384, 64);
   hipLaunchKernelGGL(select_candidates_kernel, dim3(blocks, n_requests), dim3(256), 0, st, *costs,
