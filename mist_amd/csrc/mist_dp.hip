@@ -1668,6 +1668,7 @@ __global__ __launch_bounds__(kDpHistoryThreads, 8) void dp_history_kernel(
       }
       __syncthreads();
     }
+    __syncthreads();  // every wavefront has left the loop: `reached` is free for what the path hands over
     // the answer's path: per stage the first (mesh, end layer) that attains the value, all meshes' reads of
     // 64 end layers in flight ...
     int32_t *path = reinterpret_cast<int32_t *>(f);  // [stage count - 1][4]: start layer, end layer, mesh, value behind

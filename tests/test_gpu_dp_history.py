@@ -121,3 +121,24 @@ def test_one_mesh_schedule_gives_what_the_step_schedule_gives(L, S, n, quantum, 
     assert np.array_equal(want[0], got[0])
     assert np.array_equal(want[1], got[1])
     assert np.array_equal(want[2][feasible], got[2][feasible])
+
+
+@pytest.mark.parametrize("L, D, S", [(40, 5, 8), (40, 11, 12), (40, 4, 8), (40, 10, 12), (7, 5, 7), (70, 17, 16)])
+@pytest.mark.parametrize("mode", [0, 1], ids=["threshold", "bottleneck"])
+def test_instances_whose_states_run_out(L, D, S, mode):
+    """Stages take two devices each: with the third, sixth or ninth stage count no state is left, behind an
+    answer (D even) or without one, while further instances wait for the same workgroups."""
+    rng = np.random.default_rng(L + D + mode)
+    meshes, n = [(1, 2), (2, 1)], 600
+    tabs = [_random_tables(rng, len(meshes), S, L, quantum=0.0625) for _ in range(2)]
+    tmax = rng.choice([0.0, 0.5, 2.0], size=n).astype(np.float32)
+    g_index = rng.integers(-1, 2, size=n).astype(np.int32)
+    args = (meshes, L, D, S, S, 0, tabs, g_index, tmax, mode)
+    want = _run(meshes, L, D, S, S, 0, tabs, np.maximum(g_index, 0), tmax, mode, "step")
+    feasible = (want[0] >= 0) & (g_index >= 0)
+    assert feasible.any() == (D % 2 == 0)
+    got, path = _run(*args, "history", want_path=True)
+    assert np.array_equal(got[0], np.where(g_index >= 0, want[0], -1))
+    assert np.array_equal(got[1:, feasible], want[1:, feasible])
+    assert ((path[:, 0, 0] >= 0) == feasible).all()
+    assert np.array_equal(got, _run(*args, "history"))
