@@ -1408,12 +1408,21 @@ inline size_t dp_history_lds(int L, int D, int max_stages) {
   return (f + 2 * (size_t)L + (size_t)max_stages + 7) * sizeof(float);
 }
 
+// A float's bits as an integer in the order of the values, either zero as +0; and back.
+__device__ __forceinline__ int32_t ordered_bits(float v) {
+  const int32_t bits = __float_as_int(v + 0.0f);
+  return bits ^ (bits >> 31 & 0x7fffffff);
+}
+__device__ __forceinline__ float from_ordered_bits(int32_t bits) {
+  return __int_as_float(bits ^ (bits >> 31 & 0x7fffffff));
+}
+
 // Over the re-laid row minima of every g, for dp_history_kernel: the smallest stage cost x devices / layers,
-// negative where some cost is, and the smallest cost on every mesh.  out[g][1 + Q], +inf before the
-// launch; workgroup = (share of the stage counts, mesh, g).
+// negative where some cost is, and the smallest cost on every mesh.  out[g][1 + Q] as ordered_bits, those of
+// +inf before the launch; workgroup = (share of the stage counts, mesh, g).
 constexpr int kRateShares = 4;
 __global__ __launch_bounds__(256) void stage_rate_kernel(const MistDpShape shape, const float *__restrict__ stage_min,
-                                                         int64_t g_stride, float *__restrict__ out) {
+                                                         int64_t g_stride, int32_t *__restrict__ out) {
   __shared__ float lds[2][4];
   const int L = shape.num_layers, tri = dp_triangle(L), q = blockIdx.y;
   const float *__restrict__ in = stage_min + blockIdx.z * g_stride + (int64_t)q * tri;
@@ -1441,11 +1450,14 @@ __global__ __launch_bounds__(256) void stage_rate_kernel(const MistDpShape shape
   __syncthreads();
   if (threadIdx.x < 2) {
     float low = fminf(fminf(lds[threadIdx.x][0], lds[threadIdx.x][1]), fminf(lds[threadIdx.x][2], lds[threadIdx.x][3]));
-    if (threadIdx.x == 0) low *= (float)(shape.mesh_n[q] * shape.mesh_m[q]);
-    // (as integers: those of positive floats are in their order, and a negative one is below them all)
+    if (threadIdx.x == 0) {
+      low *= (float)(shape.mesh_n[q] * shape.mesh_m[q]);
+      // (the quotient of the smallest negative costs is a zero)
+      const float least_of_all = fminf(fminf(lds[1][0], lds[1][1]), fminf(lds[1][2], lds[1][3]));
+      if (least_of_all < 0.0f) low = fminf(low, least_of_all);
+    }
     if (low < INFINITY)
-      atomicMin(reinterpret_cast<int *>(out) + (int64_t)blockIdx.z * (1 + shape.num_mesh) + (threadIdx.x == 0 ? 0 : 1 + q),
-                __float_as_int(low));
+      atomicMin(out + (int64_t)blockIdx.z * (1 + shape.num_mesh) + (threadIdx.x == 0 ? 0 : 1 + q), ordered_bits(low));
   }
 }
 __device__ __forceinline__ int greatest_common_divisor(int a, int b) {
@@ -1501,7 +1513,7 @@ __device__ __forceinline__ void dp_write_stage(int32_t *at, int end, int n, int 
 template <bool kBottleneck, int kCols>
 __global__ __launch_bounds__(kDpHistoryThreads, 8) void dp_history_kernel(
     const MistDpShape shape, const MistDpCosts tabs, const float *__restrict__ tmax_list,
-    const int32_t *__restrict__ g_list, int n_instances, const float *__restrict__ rates,
+    const int32_t *__restrict__ g_list, int n_instances, const int32_t *__restrict__ rates,
     float *__restrict__ histories, int32_t *__restrict__ best_s_out, float *__restrict__ best_sum_out,
     float *__restrict__ stage_max_out, int32_t *__restrict__ path_out) {
   extern __shared__ float dp_lds[];
@@ -1542,13 +1554,14 @@ __global__ __launch_bounds__(kDpHistoryThreads, 8) void dp_history_kernel(
       bound[threadIdx.x] = __float_as_int(INFINITY);
       *answer = INFINITY;
     }
-    const float rate = rates != nullptr ? rates[g * (1 + Q)] : -1.0f;
+    const float rate = rates != nullptr ? from_ordered_bits(rates[g * (1 + Q)]) : -1.0f;
     const bool bounded = rate >= 0.0f && rate < INFINITY;
     const float short_by = 1.0f - 1.2e-7f * (float)(L + 8);
     // stages take whole multiples of `unit` devices: a state's column is d / unit - 1, of W
     int unit = rates != nullptr ? D : 1;
     for (int q = 0; rates != nullptr && q < Q; ++q)
-      if (rates[g * (1 + Q) + 1 + q] <= t_max) unit = greatest_common_divisor(unit, shape.mesh_n[q] * shape.mesh_m[q]);
+      if (from_ordered_bits(rates[g * (1 + Q) + 1 + q]) <= t_max)
+        unit = greatest_common_divisor(unit, shape.mesh_n[q] * shape.mesh_m[q]);
     const int W = D / unit;
     // lane = mesh: columns a stage on it takes; more than there are where none of its stages is admissible
     const int its_devices = lane < Q ? shape.mesh_n[min(lane, Q - 1)] * shape.mesh_m[min(lane, Q - 1)] : 0;
@@ -2371,7 +2384,7 @@ int mist_dp_run(const MistDpShape *shape, const MistDpCosts *costs, const float 
 
 }  // extern "C"
 
-int mist::dp_stage_rates(const MistDpShape &shape, const MistDpCosts &costs, int n_g, float *d_rates, hipStream_t stream) {
+int mist::dp_stage_rates(const MistDpShape &shape, const MistDpCosts &costs, int n_g, int32_t *d_rates, hipStream_t stream) {
   if (costs.stage_min == nullptr || n_g < 1 || n_g > 65535) return fail(MIST_E_INVALID, "no row minima or %d tables", n_g);
   hipLaunchKernelGGL(stage_rate_kernel, dim3(kRateShares, shape.num_mesh, n_g), dim3(256), 0, stream, shape,
                      costs.stage_min, costs.stage_min_g_stride, d_rates);
@@ -2420,7 +2433,7 @@ int mist::dp_run_free(const DpFreeRun *runs, int n, const float *d_tmax, const i
   return launch_dp_free(runs, n, d_tmax, d_g_index, n_tmax, mode, stream);
 }
 
-int mist::dp_run(const MistDpShape *shape, const MistDpCosts *costs, const float *d_rates, const float *d_tmax,
+int mist::dp_run(const MistDpShape *shape, const MistDpCosts *costs, const int32_t *d_rates, const float *d_tmax,
                  const int32_t *d_g_index, int n_tmax, int mode, int32_t *d_best_s, float *d_best_sum,
                  float *d_stage_max, int32_t *d_argmin, int32_t *d_path, float *d_scratch, int64_t scratch_floats,
                  void *stream) {

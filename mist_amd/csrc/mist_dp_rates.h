@@ -8,12 +8,14 @@
 #include "mist_dp.h"
 
 namespace mist {
-// d_rates[n_g][1 + num_mesh], +inf before the call: over costs.stage_min of every g the smallest stage
-// cost x devices / layers (negative where a cost is), and the smallest cost on every mesh.
-int dp_stage_rates(const MistDpShape &shape, const MistDpCosts &costs, int n_g, float *d_rates, hipStream_t stream);
+// d_rates[n_g][1 + num_mesh], kRateNone before the call: over costs.stage_min of every g the smallest stage
+// cost x devices / layers (negative where a cost is), and the smallest cost on every mesh, as the floats'
+// bits with the lower 31 of a negative one inverted: in the order of the values, for an integer minimum.
+constexpr int32_t kRateNone = 0x7f800000;  // +inf
+int dp_stage_rates(const MistDpShape &shape, const MistDpCosts &costs, int n_g, int32_t *d_rates, hipStream_t stream);
 
 // mist_dp_run_sized; `d_rates` (may be null) holds what dp_stage_rates left for every g the instances name.
-int dp_run(const MistDpShape *shape, const MistDpCosts *costs, const float *d_rates, const float *d_tmax,
+int dp_run(const MistDpShape *shape, const MistDpCosts *costs, const int32_t *d_rates, const float *d_tmax,
            const int32_t *d_g_index, int n_tmax, int mode, int32_t *d_best_s, float *d_best_sum, float *d_stage_max,
            int32_t *d_argmin, int32_t *d_path, float *d_scratch, int64_t scratch_floats, void *stream);
 

@@ -336,7 +336,7 @@ struct Search {
     if (int rc = ws->h_grad.reserve(sizeof(int32_t) * words)) return rc;
     if (int rc = ws->d_grad.reserve(sizeof(int32_t) * words)) return rc;
     std::memcpy(ws->h_grad.ptr, grad_accum, sizeof(int32_t) * n_grad_accum);
-    std::fill_n(ws->h_grad.as<float>() + n_grad_accum, words - n_grad_accum, std::numeric_limits<float>::infinity());
+    std::fill_n(ws->h_grad.as<int32_t>() + n_grad_accum, words - n_grad_accum, mist::kRateNone);
     MIST_HIP_CHECK(hipMemcpyAsync(ws->d_grad.ptr, ws->h_grad.ptr, sizeof(int32_t) * words, hipMemcpyHostToDevice, stream));
     if (n_g == 0 || n_g > 65535) return 0;
     n_rates = n_g;
@@ -345,14 +345,14 @@ struct Search {
         if (int rc = mist::dp_stage_rates(shapes[f], costs[f], n_g, rates_of(f), stream)) return rc;
     return 0;
   }
-  float *rates_of(int f) const {
+  int32_t *rates_of(int f) const {
     if (n_rates == 0 || shapes[f].free_devices != 0 || costs[f].stage_min == nullptr) return nullptr;
     const char *decided = getenv("MIST_DP_RATES");
     if (decided && *decided ? *decided == '0' : (int64_t)shapes[f].num_layers * shapes[f].num_devices <= kRatesMinStates)
       return nullptr;
     size_t at = at_rates;
     for (int before = 0; before < f; ++before) at += (size_t)n_rates * (1 + shapes[before].num_mesh);
-    return ws->d_grad.as<float>() + at;
+    return ws->d_grad.as<int32_t>() + at;
   }
 
   MistDpShape shape_of(int f) const {
