@@ -302,6 +302,12 @@ __global__ __launch_bounds__(64) void uniform_search_kernel(
 }
 
 constexpr int64_t kRatesMinStates = 1024;
+// Planes of more states get rates; for tests MIST_DP_RATES = 0 | 1 decides.
+int64_t rates_above_states() {
+  const char *decided = getenv("MIST_DP_RATES");
+  if (decided == nullptr || *decided == '\0') return kRatesMinStates;
+  return *decided == '0' ? std::numeric_limits<int64_t>::max() : 0;
+}
 
 struct Search {
   int n_families;
@@ -322,9 +328,11 @@ struct Search {
 
   // Accumulation counts of the window requests, and behind them per family the rates that end a DP
   // instance early (of the table rows below n_rates).  Not for planes of a few states, which end after
-  // a few short steps anyway (two batches and the bottleneck of 32 x 32 0.31 ms with them and 0.30
-  // without, of 24 x 2 0.04 and 0.03; of 40 x 64 0.44 and 0.58, of 80 x 256 2.7 and 7.2).  For tests
-  // MIST_DP_RATES = 0 | 1 decides.
+  // a few short steps anyway (DP launches of a search and the rates' own, us, layers x devices without ->
+  // with: 24 x 2 30 -> 45, 32 x 32 301 -> 315; 33 x 32 323 -> 251, 36 x 32 410 -> 376, 40 x 32 473 -> 405,
+  // 80 x 16 794 -> 692, 24 x 64 203 -> 186, 40 x 48 365 -> 331, 40 x 64 549 -> 450, 48 x 128 1090 -> 640,
+  // 80 x 256 6740 -> 2770).
+  const int64_t rates_above = rates_above_states();
   int n_rates = 0, at_rates = 0;
   int upload_grad_accum(const std::vector<int32_t> &rows, const int32_t *grad_accum, int n_grad_accum) {
     n_rates = 0;
@@ -347,9 +355,7 @@ struct Search {
   }
   int32_t *rates_of(int f) const {
     if (n_rates == 0 || shapes[f].free_devices != 0 || costs[f].stage_min == nullptr) return nullptr;
-    const char *decided = getenv("MIST_DP_RATES");
-    if (decided && *decided ? *decided == '0' : (int64_t)shapes[f].num_layers * shapes[f].num_devices <= kRatesMinStates)
-      return nullptr;
+    if ((int64_t)shapes[f].num_layers * shapes[f].num_devices <= rates_above) return nullptr;
     size_t at = at_rates;
     for (int before = 0; before < f; ++before) at += (size_t)n_rates * (1 + shapes[before].num_mesh);
     return ws->d_grad.as<int32_t>() + at;
