@@ -1394,8 +1394,8 @@ __global__ __launch_bounds__(kDpPlaneThreads) void dp_plane_kernel(
 // sum each, the bound is taken 1.2e-7 short for every layer.  Stage counts of all instances of a search,
 // without -> with: 40 x 64 10700 -> 3000, 48 x 128 15300 -> 6300.  And columns of F(s) are the multiples of
 // the greatest common divisor of the meshes that hold an admissible stage (80 x 256: 64 or fewer columns
-// for most instances, a quarter of the LDS reads).  Threshold batches of a search 80 x 256 5.6 -> 2.1 ms, 48 x
-// 128 0.85 -> 0.44, 40 x 64 0.42 -> 0.29; what is left are instances whose answer has many stages (16 or 32
+// for most instances, a quarter of the LDS reads).  Threshold batches of a search 80 x 256 5.6 -> 2.2 ms, 48 x
+// 128 0.85 -> 0.44, 40 x 64 0.42 -> 0.30; what is left are instances whose answer has many stages (16 or 32
 // steps in turn, of 300 VALU instructions per start layer), and their launches end with the longest.
 // ------------------------------------------------------------------------------------------
 constexpr int kDpHistoryThreads = 1024;

@@ -2099,11 +2099,6 @@ struct StageReach {
   int count_b, count_p;  // base, with_pre
   bool post, pp;
   float x, d;            // of the pseudo row
-  __device__ __forceinline__ double threshold(const double *slots, int pitch, int P, double ratio, double cutoff,
-                                              const GroupModel &m, const double *__restrict__ floor) const {
-    return Threshold(loosest_minima(true, slots, pitch, P, count_b, count_p, post, pp, cutoff), group_offsets(m, ratio))
-        .at(post_layer_offset(m, ratio, floor));
-  }
 };
 __device__ __forceinline__ StageReach stage_reach(const double *__restrict__ f, const PairConsts &k, int np,
                                                   bool do_post, bool do_pp, const GroupModel &m) {
@@ -2122,8 +2117,8 @@ __device__ __forceinline__ StageReach stage_reach(const double *__restrict__ f, 
 
 // ---- filter ----
 // Workgroup = one wavefront = (row chunk, tile, p tile as a share of the chunk's summaries), lane
-// = pair.  Summaries are wave-uniform and come through scalar loads; a visit is ~40 float64
-// instructions against the pair's loosest minima.
+// = pair.  A summary is the same for all lanes; a visit is ~40 float64 instructions against the pair's
+// loosest minima.
 // Several samples: kFilterShares wavefronts of a workgroup take as many shares of a tile and its thresholds
 // at every sample from LDS, where they get them with lane = (pair parity, sample): the minima of a slot lie
 // side by side.  A summary is tried at the sample that the last one passed first.  (A wavefront a share and
@@ -3416,7 +3411,11 @@ __global__ __launch_bounds__(256) void estimate_stage_minima_kernel(
     const MistProblem prob, const MistGroupDesc *__restrict__ groups,
     const double *__restrict__ row_terms, double ratio, double *__restrict__ partial_cost, double *gather_floor) {
   const MistGroupDesc *g = groups + blockIdx.y;
-  if (blockIdx.x >= kEstimateSplit) {  // (what the seed launch wants next needs no launch of its own)
+  // What the seed launch wants next, beside the estimate: it reads the gathered rows again and the seeds wait
+  // for it.  (us, rows estimated alone -> with it; seeds reading every row -> by these bounds: 7B on 4x8 86 -> 97,
+  // 285 -> 268; 13B on 8x8 116 -> 138, 553 -> 517; 22B on 16x8 198 -> 325, 5815 -> 4754; 70B on 32x8 239 -> 276,
+  // 1972 -> 1269.  From the gathered rows to the filter that is no gain up to 7B on 4x8, 450 -> 465.)
+  if (blockIdx.x >= kEstimateSplit) {
     gather_floors(prob, g, blockIdx.y, row_terms, ratio, gather_floor, blockIdx.x - kEstimateSplit, kGatherBlocks);
     return;
   }
@@ -4072,8 +4071,9 @@ static int launch_seeds(const MistProblem *problem, const MistGroupDesc *d_group
   int pair_split = tabs.n_samples == 1 ? 16 : 1;
   while (pair_split > 1 && pair_split * pair_bytes > kSeedLdsBytes) pair_split /= 2;
   // ... and where there would be fewer than eight workgroups per CU (16, 8 and 4 pairs: stage operator of 7B on
-  // 2x8, one group, 106, 65, 40 us; uniform-pp of 7B on 2x8 beside the summaries 123, 85, 146; the 7B plan on
-  // 4x8, 72 groups, 257, 255, 259; 70B on 32x8, 120 groups, 1250, 1490, 1930)
+  // 2x8, one group, 106, 65, 40 us; uniform-pp of 7B on 2x8, 56 groups, beside the summaries 125, 90 to 167 by run,
+  // 168, from the gathered rows to the filter 249, 251 to 277, 267; the 7B plan on 4x8, 72 groups, 257, 255, 259;
+  // 70B on 32x8, 120 groups, 1250, 1490, 1930)
   while (pair_split > 4 && (int64_t)tiles * (MIST_LC_TILE / pair_split) * n_groups < kSeedWorkgroups) pair_split /= 2;
   int sample_split = tabs.n_samples;
   while (sample_split > 1 && pair_bytes * sample_split > kSeedLdsBytes) sample_split = (sample_split + 1) / 2;
