@@ -49,6 +49,11 @@ typedef struct MistDpCosts {
    * are the same either way. */
   const float *stage_min;
   int64_t stage_min_g_stride;
+  /* Optional (NULL = all): [g][planes_g_stride] int32, per mesh how many of the first planes of the p
+   * axis hold something; the others (for 0 the mesh's rows of costs_post and costs_nopp too) count as
+   * +inf and are not read.  planes_g_stride: meshes of the tables. */
+  const int32_t *planes;
+  int64_t planes_g_stride;
 } MistDpCosts;
 
 #define MIST_DP_CKPT_TAIL 0
@@ -74,6 +79,13 @@ int mist_sizeof_dp_shape(void);
 int mist_dp_cost_tables(const MistProblem *problem, const MistOutTables *tables,
                         const int32_t *d_grad_accum, int slot, float *const d_out[4],
                         float *const d_out_pmin[4], void *stream);
+
+/* mist_dp_cost_tables of the planes that hold something, d_planes[num_grad_accum][num_mesh] as in
+ * MistDpCosts.planes; the others are not touched.  One sample, at most 255 layers.  tables->index must be
+ * there and is read in the cells that mist_finalize writes only, for which see MistProblem.sparse_tables
+ * (mist_search.h). */
+int mist_dp_cost_planes(const MistProblem *problem, const MistOutTables *tables, const int32_t *d_grad_accum,
+                        const int32_t *d_planes, float *const d_out[4], float *const d_out_pmin[4], void *stream);
 
 /* Fills MistDpCosts.stage_min for a DP family: d_out[num_grad_accum][mist_dp_stage_minima_floats()]
  * (max_stages * Q * L(L+1)/2 floats per g).  Entry (g, p, q, k, i) is the smallest cost over the

@@ -127,6 +127,9 @@ typedef struct MistProblem {
    * need: sum over groups of n_lc_tiles * MIST_LC_TILE * (2 num_p + 2); rows / 512 + 2 groups + 1;
    * sum over groups of n_lc_tiles * ceil(n_rows / mist_reduce_stage_rows()). */
   int64_t reduce_cells, reduce_supers, reduce_items;
+  /* != 0 (one sample): the tables are not pre-filled, and what reads them knows the cells that are never
+   * written (mist_dp_cost_planes); a cell without a row gets its index of -1 and no costs. */
+  int32_t sparse_tables, reserved;
 } MistProblem;
 
 /* One (gradient-accumulation steps, device mesh) group = one call of the reference's

@@ -69,6 +69,8 @@ PROBLEM_DTYPE = np.dtype(
         ("reduce_cells", "<i8"),
         ("reduce_supers", "<i8"),
         ("reduce_items", "<i8"),
+        ("sparse_tables", "<i4"),
+        ("reserved", "<i4"),
     ],
     align=True,
 )
@@ -219,6 +221,8 @@ class DpCosts(ctypes.Structure):
         ("g_stride", ctypes.c_int64 * 4),
         ("stage_min", ctypes.c_void_p),
         ("stage_min_g_stride", ctypes.c_int64),
+        ("planes", ctypes.c_void_p),
+        ("planes_g_stride", ctypes.c_int64),
     ]
 
 
@@ -228,6 +232,8 @@ _DP_SIGNATURES = {
         ctypes.c_int,
         [_VP, ctypes.POINTER(OutTables), _VP, ctypes.c_int, ctypes.c_void_p * 4, ctypes.c_void_p * 4, _VP],
     ),
+    "mist_dp_cost_planes": (
+        ctypes.c_int, [_VP, ctypes.POINTER(OutTables), _VP, _VP, ctypes.c_void_p * 4, ctypes.c_void_p * 4, _VP]),
     "mist_dp_filter_tmax": (ctypes.c_int, [_VP, ctypes.c_int, ctypes.c_double, _VP]),
     "mist_dp_windows_first_batch": (
         ctypes.c_int,

@@ -37,6 +37,7 @@ constexpr int kDpFusedMinInstances = 64;  // threshold batches of at least this 
 constexpr int kDpFusedSmallPlane = 2048;  // (L + 1)(D + 1) up to which every batch uses it
 constexpr int kDpStageBatch = 8;   // row minima a lane copies together in the one-launch kernel
 constexpr int kSelectBatch = 8;  // table values a lane of the candidate selection reads together
+constexpr int kSelectSegments = 3 * MIST_MAX_MESH;  // runs of neighbouring values it reads
 constexpr int kSelectBuffer = 4096;  // selected values a workgroup holds before it appends them
 constexpr float kDpNoThreshold = 3.402823466e+38f;  // FLT_MAX: admits every finite stage cost
 constexpr int kDpBatch = 4;  // end layers whose reads a lane of the one-lane-per-state kernel overlaps
@@ -96,6 +97,53 @@ constexpr int kCostCells = 1024;
 typedef int AnyInt4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef float AnyFloat4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef double AnyDouble2 __attribute__((ext_vector_type(2), aligned(8)));
+// A lane's four cells of a set of rows.
+struct CostLane {
+  int cell0, row[4], j[4];
+  int back;     // lanes to where the last cell's row begins
+  bool spills;  // the first cell's begins in an earlier wavefront
+  __device__ __forceinline__ explicit CostLane(int row_len) : cell0((int)threadIdx.x * 4) {
+    row[0] = cell0 / row_len;
+    j[0] = cell0 - row[0] * row_len;
+#pragma unroll
+    for (int u = 1; u < 4; ++u) {
+      const bool next = j[u - 1] + 1 == row_len;
+      row[u] = row[u - 1] + next;
+      j[u] = next ? 0 : j[u - 1] + 1;
+    }
+    back = min((int)threadIdx.x - ((cell0 + 3 - j[3]) >> 2), (int)(threadIdx.x & 63));
+    spills = cell0 - j[0] < (int)(threadIdx.x >> 6) * 256;
+  }
+};
+// Costs of a set and their running minima, by the whole workgroup; `ends`: four floats that the set before
+// does not use.
+__device__ __forceinline__ void store_costs(const CostLane &at, const float (&c)[4], int n_mine, float *__restrict__ out,
+                                            float *__restrict__ pmin, float *ends) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  float run = INFINITY;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) run = fminf(c[u], at.j[u] == 0 ? INFINITY : run);
+  run = running_minimum(run, at.back);
+  if (lane == 63) ends[wave] = run;
+  __syncthreads();
+  run = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(INFINITY), __float_as_int(run), 0x138, 0xf, 0xf,
+                                                   false));  // wave_shr:1
+  if (at.spills) run = fminf(run, ends[wave - 1]);
+  float m[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) m[u] = run = fminf(c[u], at.j[u] == 0 ? INFINITY : run);
+  if (n_mine == 4) {
+    *reinterpret_cast<AnyFloat4 *>(out) = AnyFloat4{c[0], c[1], c[2], c[3]};
+    *reinterpret_cast<AnyFloat4 *>(pmin) = AnyFloat4{m[0], m[1], m[2], m[3]};
+  } else {
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (u < n_mine) {
+        out[u] = c[u];
+        pmin[u] = m[u];
+      }
+  }
+}
 __global__ __launch_bounds__(256) void cost_rows_kernel(const CostTableJob job, const int32_t *__restrict__ grad_accum,
                                                         int row_len) {
   __shared__ float ends[2][4];
@@ -106,18 +154,9 @@ __global__ __launch_bounds__(256) void cost_rows_kernel(const CostTableJob job, 
   float *__restrict__ out = job.out[v], *__restrict__ pmin = job.pmin[v];
   const int64_t n_rows = job.n_rows[v], per_g = job.rows_per_g[v];
   const int rows_here = (kCostCells / row_len) & ~3, cells_here = rows_here * row_len;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, cell0 = (int)threadIdx.x * 4;
-  int its_row[4], j[4];
-  its_row[0] = cell0 / row_len;
-  j[0] = cell0 - its_row[0] * row_len;
-#pragma unroll
-  for (int u = 1; u < 4; ++u) {
-    const bool next = j[u - 1] + 1 == row_len;
-    its_row[u] = its_row[u - 1] + next;
-    j[u] = next ? 0 : j[u - 1] + 1;
-  }
-  const int back = min((int)threadIdx.x - ((cell0 + 3 - j[3]) >> 2), lane);  // to where the last cell's row begins
-  const bool spills = cell0 - j[0] < wave * 256;  // the first cell's begins in an earlier wavefront
+  const CostLane at_lane(row_len);
+  const int cell0 = at_lane.cell0;
+  const int(&its_row)[4] = at_lane.row;
   const int64_t row0 = (int64_t)(blockIdx.x - job.first_block[v]) * rows_here * job.runs;
   int64_t g = row0 / per_g, in_g = row0 - g * per_g;
   for (int turn = 0; turn < job.runs; ++turn) {
@@ -174,29 +213,80 @@ __global__ __launch_bounds__(256) void cost_rows_kernel(const CostTableJob job, 
       }
     }
     for (in_g += rows_here; in_g >= per_g; in_g -= per_g) ++g;
-    float run = INFINITY;
+    store_costs(at_lane, c, n_mine, out + i, pmin + i, ends[turn & 1]);
+  }
+}
+
+// Only the planes of the p axis that hold something (MistDpCosts.planes): workgroups of a (g, mesh) take its
+// sets of rows in turn, table after table.  The cells of a row that the reference never writes are known by
+// their place, so that no fill of the row indices comes before: c > l, and c == l - 1 except at p == 0 of base /
+// with_pre.  Bound: 12 bytes a cell of the planes, and latency: a set is two dependent reads and a barrier.
+// (70B on 32x8, where 21 % of the planes hold something: fill 254 us and every cell 1063 -> 243; 13B on 8x8 26 and
+// 98 -> 41; 7B on 4x8 12 and 46 -> 22.)
+constexpr int64_t kCostPlaneBlocks = 16384;
+struct CostPlanesJob {
+  const double *stable[4], *delta[4];
+  const int32_t *index[4];
+  float *out[4], *pmin[4];
+  const int32_t *planes, *grad_accum;
+  int L, P1;
+};
+__global__ __launch_bounds__(256) void cost_planes_kernel(const CostPlanesJob job) {
+  __shared__ float ends[2][4];
+  const int L = job.L, P1 = job.P1, row_len = L + 1, q = blockIdx.y, Q = gridDim.y;
+  const int64_t gq = (int64_t)blockIdx.z * Q + q;
+  const int planes = min(job.planes[gq], P1);
+  if (planes <= 0) return;
+  const float G = (float)job.grad_accum[blockIdx.z];
+  const int rows_here = (kCostCells / row_len) & ~3;
+  const CostLane at_lane(row_len);
+  const int wide_sets = (planes * L + rows_here - 1) / rows_here, post_sets = (L + rows_here - 1) / rows_here;
+  const int n_sets = 2 * wide_sets + post_sets + 1;
+  for (int set = blockIdx.x, turn = 0; set < n_sets; set += gridDim.x, ++turn) {
+    const int v = set < wide_sets ? 0 : set < 2 * wide_sets ? 1 : set < 2 * wide_sets + post_sets ? 2 : 3;
+    const int row0 = (v == 3 ? 0 : set - (v == 0 ? 0 : v * wide_sets)) * rows_here;
+    const int n_rows = v < 2 ? planes * L : v == 2 ? L : 1;
+    const int64_t first = (v < 2 ? gq * P1 * L : v == 2 ? gq * L : gq) * row_len;  // cell of the (g, mesh)'s row 0
+    const int n_cells = min(rows_here, n_rows - row0) * row_len, n_mine = min(n_cells - at_lane.cell0, 4);
+    const int64_t i = first + (int64_t)row0 * row_len + at_lane.cell0;
+    float c[4] = {INFINITY, INFINITY, INFINITY, INFINITY};
+    if (n_mine > 0) {
+      int32_t index[4] = {-1, -1, -1, -1};
+      if (n_mine == 4) {
+        const AnyInt4 four = *reinterpret_cast<const AnyInt4 *>(job.index[v] + i);
+        index[0] = four.x, index[1] = four.y, index[2] = four.z, index[3] = four.w;
+      } else {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) run = fminf(c[u], j[u] == 0 ? INFINITY : run);
-    run = running_minimum(run, back);
-    if (lane == 63) ends[turn & 1][wave] = run;
-    __syncthreads();
-    run = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(INFINITY), __float_as_int(run), 0x138, 0xf, 0xf,
-                                                     false));  // wave_shr:1
-    if (spills) run = fminf(run, ends[turn & 1][wave - 1]);
-    float m[4];
+        for (int u = 0; u < 4; ++u)
+          if (u < n_mine) index[u] = job.index[v][i + u];
+      }
+      int p = (row0 + at_lane.row[0]) / L, l = v == 3 ? L : row0 + at_lane.row[0] - p * L + 1;
+      bool holds[4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) m[u] = run = fminf(c[u], j[u] == 0 ? INFINITY : run);
-    if (n_mine == 4) {
-      *reinterpret_cast<AnyFloat4 *>(out + i) = AnyFloat4{c[0], c[1], c[2], c[3]};
-      *reinterpret_cast<AnyFloat4 *>(pmin + i) = AnyFloat4{m[0], m[1], m[2], m[3]};
-    } else {
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-        if (u < n_mine) {
-          out[i + u] = c[u];
-          pmin[i + u] = m[u];
+      for (int u = 0; u < 4; ++u) {
+        if (u > 0 && at_lane.j[u] == 0) {  // the next row
+          const bool wraps = l == L;
+          p += wraps;
+          l = wraps ? 1 : l + 1;
         }
+        const bool written = at_lane.j[u] <= l && (at_lane.j[u] != l - 1 || (v < 2 && p == 0));
+        holds[u] = u < n_mine && written && index[u] >= 0;
+      }
+      if (holds[0] || holds[1] || holds[2] || holds[3]) {
+        double its_stable[4], its_delta[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          its_stable[u] = u < n_mine ? job.stable[v][i + u] : 0.0;
+          its_delta[u] = u < n_mine ? job.delta[v][i + u] : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const float cost = (float)its_stable[u] + (float)its_delta[u] / G;
+          c[u] = holds[u] ? cost : INFINITY;
+        }
+      }
     }
+    store_costs(at_lane, c, n_mine, job.out[v] + i, job.pmin[v] + i, ends[turn & 1]);
   }
 }
 
@@ -286,8 +376,8 @@ __global__ __launch_bounds__(256) void select_candidates_kernel(
   const int r = blockIdx.y;
   const int64_t g = rows[r];
   const int64_t n0 = tabs.g_stride[0], n1 = tabs.g_stride[1], n2 = tabs.g_stride[2];
-  const int64_t n = n0 + n1 + n2;
   const float lo_r = lo[r], hi_r = hi[r];
+  if (lo_r == INFINITY && hi_r == INFINITY) return;  // (nothing is feasible there)
   const int lane = threadIdx.x & 63;
   int above = 0;
   if (threadIdx.x == 0) n_kept = 0;
@@ -308,20 +398,57 @@ __global__ __launch_bounds__(256) void select_candidates_kernel(
     if (threadIdx.x == 0) n_kept = 0;
     __syncthreads();
   };
-  // every workgroup of a request runs the same number of rounds; kSelectBatch values per lane
-  // are read together
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t base = (int64_t)blockIdx.x * blockDim.x; base < n; base += kSelectBatch * stride) {
-    float value[kSelectBatch];
+  // Batches of kSelectBatch values per lane, the next one on its way while one is tried, from segments of
+  // neighbouring values: the three tables, or per table and mesh the planes that hold something.  (Every value
+  // of the tables, the reads of a batch behind its barriers: 70B on 32x8 318 us, 7B on 4x8 21; the planes alone
+  // 200, and 80 and 16 with the next batch on its way.)
+  constexpr int kBatch = kSelectBatch * 256;
+  __shared__ const float *segment_from[kSelectSegments];
+  __shared__ int64_t segment_cells[kSelectSegments], segment_end[kSelectSegments];  // (the latter in batches)
+  const int meshes = tabs.planes == nullptr ? 1 : (int)tabs.planes_g_stride, n_segments = 3 * meshes;
+  if (threadIdx.x < 64) {  // lane = segment
+    const int v = lane / meshes, q = lane - v * meshes;
+    const int64_t of_mesh = (v == 0 ? n0 : v == 1 ? n1 : n2) / meshes;
+    int64_t cells = 0;
+    if (lane < n_segments) {
+      cells = of_mesh;
+      if (tabs.planes != nullptr) {
+        const int held = tabs.planes[g * meshes + q];
+        cells = v < 2 ? held * (n2 / meshes) : held > 0 ? of_mesh : 0;
+      }
+    }
+    int64_t end = (cells + kBatch - 1) / kBatch;
+    for (int step = 1; step < 64; step <<= 1) {
+      const int64_t before = __shfl_up((long long)end, step);
+      if (lane >= step) end += before;
+    }
+    if (lane < n_segments) {
+      segment_from[lane] = (v == 0 ? tabs.costs + g * n0 : v == 1 ? tabs.costs_pre + g * n1 : tabs.costs_post + g * n2) +
+                           q * of_mesh;
+      segment_cells[lane] = cells;
+      segment_end[lane] = end;
+    }
+  }
+  __syncthreads();
+  int segment = 0;
+  auto read = [&](int64_t batch, float (&value)[kSelectBatch]) {
+    while (segment < n_segments && segment_end[segment] <= batch) ++segment;
+    if (segment >= n_segments) return false;
+    const int64_t at = (batch - (segment > 0 ? segment_end[segment - 1] : 0)) * kBatch;
+    const float *__restrict__ from = segment_from[segment] + at;
+    const int left = (int)min(segment_cells[segment] - at, (int64_t)kBatch);
 #pragma unroll
     for (int u = 0; u < kSelectBatch; ++u) {
-      const int64_t e = base + u * stride + threadIdx.x;
-      value[u] = INFINITY;
-      if (e < n)
-        value[u] = e < n0 ? tabs.costs[g * n0 + e]
-                   : e < n0 + n1 ? tabs.costs_pre[g * n1 + (e - n0)]
-                                 : tabs.costs_post[g * n2 + (e - n0 - n1)];
+      const int in_batch = u * 256 + (int)threadIdx.x;
+      const float v = from[min(in_batch, left - 1)];
+      value[u] = in_batch < left ? v : INFINITY;
     }
+    return true;
+  };
+  float value[kSelectBatch], ahead[kSelectBatch];
+  bool more = read(blockIdx.x, value);
+  for (int64_t batch = blockIdx.x; more;) {
+    more = read(batch += gridDim.x, ahead);
 #pragma unroll
     for (int u = 0; u < kSelectBatch; ++u) {
       const float v = value[u];
@@ -345,6 +472,8 @@ __global__ __launch_bounds__(256) void select_candidates_kernel(
     const int kept_now = n_kept;
     __syncthreads();
     if (kept_now > kSelectBuffer - kSelectBatch * 256) flush();
+#pragma unroll
+    for (int u = 0; u < kSelectBatch; ++u) value[u] = ahead[u];
   }
   flush();
   // one atomic per workgroup for the "above" count
@@ -647,8 +776,9 @@ __device__ __forceinline__ int dp_j_last(const MistDpShape &shape, int k, int i)
 // The reference walks j = j_begin..j_end with "cost <= t_max and cost + prev < best".  "+ prev" is
 // monotone, so the smallest reachable sum is (smallest admissible cost) + prev, and the smallest
 // admissible cost is the row's running minimum if that is <= t_max (else nothing is admissible).
-__device__ __forceinline__ float dp_row_min(const MistDpShape &shape, const MistDpCosts &tabs,
+__device__ __forceinline__ float dp_row_min(const MistDpShape &shape, const MistDpCosts &tabs, int64_t g,
                                             const int64_t (&off)[4], int p, int k, int q, int i) {
+  if (tabs.planes != nullptr && p >= tabs.planes[g * tabs.planes_g_stride + q]) return INFINITY;
   const DpRowRef r = dp_row_ref(shape, off, p, k, q, i);
   return shape.ckpt_rule == MIST_DP_CKPT_ALL ? dp_table(tabs, r.v, false)[r.at + (i - k + 1)]
                                              : dp_table(tabs, r.v, true)[r.at + dp_j_last(shape, k, i)];
@@ -900,7 +1030,7 @@ __global__ __launch_bounds__(kDpThreads) void dp_step_kernel(
     dp_scan_state<kBottleneck, kDpTeam>(
         w, shape, t_max, k, d, member, f_prev, range_prev,
         [&](int q, int i) {
-          return relaid != nullptr ? relaid[q * tri + i] : dp_row_min(shape, tabs, off, p, k, q, i);
+          return relaid != nullptr ? relaid[q * tri + i] : dp_row_min(shape, tabs, g, off, p, k, q, i);
         });
     if constexpr (kDpTeam == 1) {
       w.resolve(L);
@@ -1847,7 +1977,7 @@ __global__ __launch_bounds__(kDpFreeThreads) void dp_free_kernel(
         const int x = x0 + u * kDpFreeThreads;
         const int i = x % L, k = i - x / L;
         const bool wanted = x < L * L && k >= 0 && i <= L - s && (s > 1 || i == L - 1);
-        value[u] = wanted ? dp_row_min(shape, tabs, off, s - 1, k, 0, i) : INFINITY;
+        value[u] = wanted ? dp_row_min(shape, tabs, g, off, s - 1, k, 0, i) : INFINITY;
       }
 #pragma unroll
       for (int u = 0; u < kDpFreeLoads; ++u) {
@@ -1890,7 +2020,7 @@ __global__ __launch_bounds__(kDpFreeThreads) void dp_free_kernel(
       const int i = i0 + lane;
       float rmin = INFINITY, target = INFINITY;
       if (i <= L - s && f_prev[i + 1] < INFINITY) {
-        rmin = dp_row_min(shape, tabs, off, s - 1, k, 0, i);
+        rmin = dp_row_min(shape, tabs, g, off, s - 1, k, 0, i);
         target = kBottleneck ? fmaxf(rmin, f_prev[i + 1]) : rmin + f_prev[i + 1];
       }
       const unsigned long long hit = __ballot(rmin <= t_max && target == best);
@@ -1953,21 +2083,76 @@ __global__ __launch_bounds__(64) void backtrack_kernel(const MistDpShape shape,
 // Row minima in the order the recurrence reads them: out[g][p][q][triangle(k, i)] =
 // dp_row_min(p, k, q, i).  A workgroup scanning stage count p + 1 of g finds all it needs in one
 // contiguous block, and the end layers i of one (q, k) lie next to each other.
+// Workgroup = (p, mesh, g).  The row minima of inner stages with l layers lie side by side for the start
+// layers, descending: read in that order (kMinimaLoads of a lane in flight), turned in LDS, written in the
+// other one.  Planes that hold nothing are written alone.  Bound: the 4 bytes an entry.  (A thread per entry,
+// each its own cache line, and as many threads for the planes that hold nothing: 70B on 32x8 409 us, 291 without
+// reading those, now 96; 7B on 4x8 18 -> 11.)
+constexpr int kMinimaLoads = 8;
+constexpr int kMinimaLayers = 180;  // the turned triangle fits 64 KB
+__device__ __forceinline__ void store_entries(float *__restrict__ to, int n, float value) {
+  for (int x = threadIdx.x * 4; x < n; x += 1024) {
+    if (x + 4 <= n) {
+      *reinterpret_cast<AnyFloat4 *>(to + x) = AnyFloat4{value, value, value, value};
+    } else {
+      for (int u = x; u < n; ++u) to[u] = value;
+    }
+  }
+}
+// (start layer, length) of an entry of the triangle
+__device__ __forceinline__ int dp_triangle_start(int L, int x) {
+  const float rows = 2.0f * (float)L + 1.0f;
+  int k = (int)((rows - __builtin_amdgcn_sqrtf(fmaxf(rows * rows - 8.0f * (float)x, 0.0f))) * 0.5f);
+  k = min(max(k, 0), L - 1);
+  while (dp_triangle_row(L, k) > x) --k;
+  while (k < L - 1 && dp_triangle_row(L, k + 1) <= x) ++k;
+  return k;
+}
 __global__ __launch_bounds__(256) void stage_minima_kernel(const MistDpShape shape,
                                                            const MistDpCosts tabs,
-                                                           float *__restrict__ out) {
+                                                           float *__restrict__ out, bool in_lds) {
+  extern __shared__ float dp_lds[];
   const int L = shape.num_layers, tri = dp_triangle(L);
-  const int x = blockIdx.x * 256 + threadIdx.x;
-  if (x >= L * L) return;
-  const int k = x / L, di = x % L;
-  if (k + di >= L) return;
-  const int p = blockIdx.y / shape.num_mesh, q = blockIdx.y % shape.num_mesh;
-  const int64_t g = blockIdx.z;
+  const int p = blockIdx.x / shape.num_mesh, q = blockIdx.x % shape.num_mesh;
+  const int64_t g = blockIdx.y;
+  float *__restrict__ mine = out + ((g * shape.max_stages + p) * shape.num_mesh + q) * tri;
+  if (tabs.planes != nullptr && p >= tabs.planes[g * tabs.planes_g_stride + q]) {
+    store_entries(mine, tri, INFINITY);
+    return;
+  }
   const int64_t off[4] = {g * tabs.g_stride[0], g * tabs.g_stride[1], g * tabs.g_stride[2],
                           g * tabs.g_stride[3]};
+  // rows of l layers, entry k: at l - 1 rows of L - l' + 1 entries each
+  if (in_lds) {
+    const DpRowRef inner = dp_row_ref(shape, off, p, 1, q, 1);  // one layer; the next rows follow it
+    const bool all = shape.ckpt_rule == MIST_DP_CKPT_ALL;
+    const float *__restrict__ table = dp_table(tabs, 0, !all) + (L > 2 ? inner.at : 0);
+    for (int x0 = threadIdx.x; x0 < tri; x0 += kMinimaLoads * 256) {
+      float value[kMinimaLoads];
+#pragma unroll
+      for (int u = 0; u < kMinimaLoads; ++u) {
+        const int x = x0 + u * 256;
+        value[u] = INFINITY;
+        if (x >= tri) continue;
+        const int l = dp_triangle_start(L, x) + 1, k = x - dp_triangle_row(L, l - 1), i = k + l - 1;
+        if (k == 0 || i == L - 1) continue;
+        value[u] = table[(int64_t)(l - 1) * (L + 1) + (all ? l : dp_j_last(shape, k, i))];
+      }
+#pragma unroll
+      for (int u = 0; u < kMinimaLoads; ++u)
+        if (x0 + u * 256 < tri) dp_lds[x0 + u * 256] = value[u];
+    }
+    __syncthreads();
+  }
   // a stage count of p + 1 leaves start layers k <= L - 1 - p
-  const float value = k <= L - 1 - p ? dp_row_min(shape, tabs, off, p, k, q, k + di) : INFINITY;
-  out[((g * shape.max_stages + p) * shape.num_mesh + q) * tri + dp_triangle_row(L, k) + di] = value;
+  for (int x = threadIdx.x; x < tri; x += 256) {
+    const int k = dp_triangle_start(L, x), di = x - dp_triangle_row(L, k);
+    float value = INFINITY;
+    if (k <= L - 1 - p)
+      value = in_lds && k > 0 && k + di < L - 1 ? dp_lds[dp_triangle_row(L, di) + k]
+                                                : dp_row_min(shape, tabs, g, off, p, k, q, k + di);
+    mine[x] = value;
+  }
 }
 
 // Dynamic LDS the one-launch kernel may use on the current device: what the device reports per
@@ -2131,6 +2316,10 @@ int check_run_arguments(const MistDpShape *shape, const MistDpCosts *costs, cons
   return 0;
 }
 
+// Workgroups of a request of the candidate selection: few, long-running ones, each of which appends to the
+// output list once per kSelectBuffer values at most.
+unsigned select_blocks(int64_t per_row) { return (unsigned)std::min<int64_t>((per_row + 16383) / 16384, 64); }
+
 // Small batches are latency-bound: spread every state over a team of lanes.
 bool dp_wide_teams(int n_tmax, int plane) { return (int64_t)n_tmax * plane <= (1 << 19); }
 
@@ -2217,6 +2406,39 @@ int mist_dp_cost_tables(const MistProblem *problem, const MistOutTables *tables,
   return 0;
 }
 
+int mist_dp_cost_planes(const MistProblem *problem, const MistOutTables *tables, const int32_t *d_grad_accum,
+                        const int32_t *d_planes, float *const d_out[4], float *const d_out_pmin[4], void *stream) {
+  if (!problem || !tables || !d_grad_accum || !d_planes || !d_out || !d_out_pmin)
+    return fail(MIST_E_INVALID, "null pointer argument");
+  const int64_t L = problem->num_layers, P1 = problem->p_dim, Gn = problem->num_grad_accum, Q = problem->num_mesh;
+  if (L <= 0 || P1 <= 0 || Gn <= 0 || Q <= 0) return fail(MIST_E_INVALID, "bad problem extents");
+  if (problem->sample_size != 1 || L + 1 > 256)
+    return fail(MIST_E_INVALID, "cost planes of one sample and rows of up to 256 cells, got %d samples, %d layers",
+                problem->sample_size, (int)L);
+  if (Gn > 65535 || Q > 65535 || P1 * L >= (int64_t)1 << 24) return fail(MIST_E_INVALID, "cost tables too large for one launch");
+  CostPlanesJob job = {};
+  for (int v = 0; v < 4; ++v) {
+    if (!tables->stable[v] || !tables->delta[v] || !tables->index[v] || !d_out[v] || !d_out_pmin[v])
+      return fail(MIST_E_INVALID, "table %d is null", v);
+    job.stable[v] = tables->stable[v];
+    job.delta[v] = tables->delta[v];
+    job.index[v] = tables->index[v];
+    job.out[v] = d_out[v];
+    job.pmin[v] = d_out_pmin[v];
+  }
+  job.planes = d_planes;
+  job.grad_accum = d_grad_accum;
+  job.L = (int)L;
+  job.P1 = (int)P1;
+  const int64_t rows_here = (kCostCells / (L + 1)) & ~3ll;
+  const int64_t sets = 2 * ((P1 * L + rows_here - 1) / rows_here) + (L + rows_here - 1) / rows_here + 1;
+  const int64_t blocks = std::max<int64_t>(1, std::min(sets, kCostPlaneBlocks / (Gn * Q)));
+  hipLaunchKernelGGL(cost_planes_kernel, dim3((unsigned)blocks, (unsigned)Q, (unsigned)Gn), dim3(256), 0,
+                     (hipStream_t)stream, job);
+  MIST_HIP_CHECK(hipGetLastError());
+  return 0;
+}
+
 int mist_dp_backtrack(const MistDpShape *shape, const int32_t *d_argmin, const int32_t *d_best_s,
                       int n_tmax, int32_t *d_path, void *stream) {
   if (int rc = check_shape(shape)) return rc;
@@ -2243,12 +2465,11 @@ int mist_dp_stage_minima(const MistDpShape *shape, const MistDpCosts *costs, int
   if (!d_out) return fail(MIST_E_INVALID, "null output pointer");
   if (num_grad_accum < 1 || num_grad_accum > 65535)
     return fail(MIST_E_INVALID, "num_grad_accum must be in [1, 65535], got %d", num_grad_accum);
-  const int L = shape->num_layers;
-  hipLaunchKernelGGL(stage_minima_kernel,
-                     dim3((unsigned)((L * L + 255) / 256),
-                          (unsigned)(shape->max_stages * shape->num_mesh),
-                          (unsigned)num_grad_accum),
-                     dim3(256), 0, (hipStream_t)stream, *shape, *costs, d_out);
+  if (shape->max_stages == 0) return 0;
+  const bool in_lds = shape->num_layers <= kMinimaLayers;
+  hipLaunchKernelGGL(stage_minima_kernel, dim3((unsigned)(shape->max_stages * shape->num_mesh), (unsigned)num_grad_accum),
+                     dim3(256), in_lds ? sizeof(float) * dp_triangle(shape->num_layers) : 0, (hipStream_t)stream, *shape,
+                     *costs, d_out, in_lds);
   MIST_HIP_CHECK(hipGetLastError());
   return 0;
 }
@@ -2302,14 +2523,14 @@ int mist_dp_select_candidates(const MistDpCosts *costs, int n_requests, const in
                               void *stream) {
   if (!costs || !costs->costs || !costs->costs_pre || !costs->costs_post)
     return fail(MIST_E_INVALID, "null cost tables");
+  if (costs->planes && (costs->planes_g_stride < 1 || costs->planes_g_stride > MIST_MAX_MESH))
+    return fail(MIST_E_INVALID, "planes of %d meshes", (int)costs->planes_g_stride);
   if (n_requests <= 0 || n_requests > 65535)
     return fail(MIST_E_INVALID, "n_requests %d outside [1, 65535]", n_requests);
   if (!d_rows || !d_lo || !d_hi || !d_out_values || !d_out_request || !d_counts || capacity <= 0)
     return fail(MIST_E_INVALID, "null pointer / empty output list");
   const int64_t per_row = costs->g_stride[0] + costs->g_stride[1] + costs->g_stride[2];
-  // few, long-running workgroups per request: each appends to the output list once per
-  // kSelectBuffer values at most
-  const unsigned blocks = (unsigned)std::min<int64_t>((per_row + 16383) / 16384, 64);
+  const unsigned blocks = select_blocks(per_row);
   hipLaunchKernelGGL(select_candidates_kernel, dim3(blocks, n_requests), dim3(256), 0,
                      (hipStream_t)stream, *costs, d_rows, d_lo, d_hi, d_out_values, d_out_request,
                      capacity, d_counts, false);
@@ -2330,6 +2551,8 @@ int mist_dp_windows_first_batch(const MistDpCosts *costs, int n_requests, const 
                                 int32_t *d_inst_row, void *stream) {
   if (!costs || !costs->costs || !costs->costs_pre || !costs->costs_post)
     return fail(MIST_E_INVALID, "null cost tables");
+  if (costs->planes && (costs->planes_g_stride < 1 || costs->planes_g_stride > MIST_MAX_MESH))
+    return fail(MIST_E_INVALID, "planes of %d meshes", (int)costs->planes_g_stride);
   if (n_requests <= 0 || n_requests > 65535)
     return fail(MIST_E_INVALID, "n_requests %d outside [1, 65535]", n_requests);
   if (!d_rows || !d_lo || !d_hi || !d_start || !d_values || !d_counts || !d_kept || !d_meta ||
@@ -2347,7 +2570,7 @@ int mist_dp_windows_first_batch(const MistDpCosts *costs, int n_requests, const 
                      d_counts, n_counts, d_inst_row, n_inst);
   MIST_HIP_CHECK(hipGetLastError());
   const int64_t per_row = costs->g_stride[0] + costs->g_stride[1] + costs->g_stride[2];
-  const unsigned blocks = (unsigned)std::min<int64_t>((per_row + 16383) / 16384, 64);
+  const unsigned blocks = select_blocks(per_row);
   hipLaunchKernelGGL(select_candidates_kernel, dim3(blocks, n_requests), dim3(256), 0, st, *costs,
                      d_rows, d_lo, d_hi, d_values, (int32_t *)nullptr, window_capacity, d_counts,
                      true);

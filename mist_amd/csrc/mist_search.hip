@@ -3576,7 +3576,12 @@ __device__ __forceinline__ FinalCell final_cell(const MistProblem &prob, const M
 }
 __device__ __forceinline__ void write_final(FinalCell &f, const MistGroupDesc *__restrict__ g, int variant, PairIndex pc,
                                             const GroupConsts &k, const double *__restrict__ row_terms, uint32_t row,
-                                            int p, const MistOutTables &tables) {
+                                            int p, const MistOutTables &tables, bool sparse) {
+  const int64_t at = f.at + p * f.plane;
+  if (sparse && row == ~0u) {  // (all that is read of such a cell)
+    tables.index[variant][at] = -1;
+    return;
+  }
   if (row == ~0u) {
     f.stable = f.delta = INFINITY;
     f.priced = row;
@@ -3589,7 +3594,6 @@ __device__ __forceinline__ void write_final(FinalCell &f, const MistGroupDesc *_
     else { f.stable = lat.spp; f.delta = lat.dpp; }
     f.priced = row;
   }
-  const int64_t at = f.at + p * f.plane;
   tables.stable[variant][at] = f.stable;
   tables.delta[variant][at] = f.delta;
   tables.index[variant][at] = (int32_t)row;
@@ -3658,7 +3662,8 @@ __global__ __launch_bounds__(256) void finalize_kernel(
     __syncthreads();
     for (int q = kFinalSlots / 4 - 1; q >= 0; --q) {
       const int slot = wave * (kFinalSlots / 4) + q;
-      if (p0 + slot < f.n_p) write_final(f, g, variant, pc, k, row_terms, winner[lane][slot], p0 + slot, tables);
+      if (p0 + slot < f.n_p) write_final(f, g, variant, pc, k, row_terms, winner[lane][slot], p0 + slot, tables,
+                                      prob.sparse_tables != 0);
     }
   }
 }
@@ -3690,7 +3695,7 @@ __global__ __launch_bounds__(256) void finalize_samples_kernel(
   uint32_t row = ~0u;
   for (int p = f.n_p - 1; p >= p_begin; --p) {
     take_lower(cost, row, tabs.best[first + (int64_t)p * n], row_number(tabs.row[first + (int64_t)p * n]));
-    if (p < p_begin + kFinalRange) write_final(f, g, variant, pc, k, row_terms, row, p, tables);
+    if (p < p_begin + kFinalRange) write_final(f, g, variant, pc, k, row_terms, row, p, tables, false);
   }
 }
 

@@ -94,10 +94,18 @@ class _DpRunner:
             out_ptrs = (ctypes.c_void_p * 4)(*[t.data_ptr() for t in self.cost])
             pmin_ptrs = (ctypes.c_void_p * 4)(*[t.data_ptr() for t in self.pmin])
             tabs = dev_tabs.as_struct()
-            rc = self.lib.mist_dp_cost_tables(
-                ctypes.c_void_p(problem.ctypes.data), ctypes.byref(tabs), d_G.data_ptr(), slot,
-                out_ptrs, pmin_ptrs, _stream(self.device),
-            )
+            # (tables of which some planes alone are filled: those, and the searches know)
+            self.planes = getattr(dev_tabs, "planes", None)
+            if self.planes is None:
+                rc = self.lib.mist_dp_cost_tables(
+                    ctypes.c_void_p(problem.ctypes.data), ctypes.byref(tabs), d_G.data_ptr(), slot,
+                    out_ptrs, pmin_ptrs, _stream(self.device),
+                )
+            else:
+                rc = self.lib.mist_dp_cost_planes(
+                    ctypes.c_void_p(problem.ctypes.data), ctypes.byref(tabs), d_G.data_ptr(), self.planes.data_ptr(),
+                    out_ptrs, pmin_ptrs, _stream(self.device),
+                )
             _lib.check(rc, "mist_dp_cost_tables")
         if uniform_device is None:
             self.families = [self._per_mesh_family(meshes)]
@@ -129,6 +137,8 @@ class _DpRunner:
         cs = _lib.DpCosts(*ptrs)
         for v in range(4):
             cs.g_stride[v] = per_q[v] * self.Q
+        if self.planes is not None:
+            cs.planes, cs.planes_g_stride = self.planes.data_ptr() + 4 * q, self.Q
         return cs
 
     def _prepare_stage_minima(self, fam: _DpFamily) -> None:

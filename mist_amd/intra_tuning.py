@@ -111,6 +111,9 @@ class DeviceTables:
     # gradient-accumulation count of every table row g (int32, on the device), uploaded with the
     # plan so that the inter-stage search need not wait for the kernels to copy it
     grad_accum: Optional[torch.Tensor] = None
+    # [row of the tables][mesh] int32 of tables without a pre-fill (``run_prepared(sparse=True)``): how many of
+    # the first planes of the p axis hold something
+    planes: Optional[torch.Tensor] = None
 
     def as_struct(self) -> _lib.OutTables:
         s = _lib.OutTables()
@@ -641,12 +644,12 @@ class IntraStageTuner:
             starts.append(starts[-1] + int(np.prod(shape)))
         return shapes, starts
 
-    def _allocate_flat(self, plan: Optional[dict] = None, fill_costs: bool = True):
+    def _allocate_flat(self, plan: Optional[dict] = None, fill_costs: bool = True, fill_index: bool = True):
         """The output tables as two flat allocations (float64 costs: stable then delta; int32
         row indices) with their pre-fill queued on the current stream, and the ``MistOutTables``
         of pointers into them.  Pre-filled with +inf / -1: everywhere, or (``plan`` of a tuner
         with ``prefill_wanted_cells_only``) in the cells ``cells_wanted`` names.  ``fill_costs``
-        False: the costs are defined where an index is not -1."""
+        False: the costs are defined where an index is not -1; ``fill_index`` False: not filled at all."""
         shapes, starts = self._table_layout()
         total, dev = starts[-1], self.device
         wanted = plan.get("wanted") if plan is not None and self.prefill_wanted_cells_only else None
@@ -655,7 +658,9 @@ class IntraStageTuner:
             costs = torch.empty((2 * total,), dtype=torch.float64, device=dev)
             if fill_costs:
                 costs.fill_(float("inf"))
-            index = torch.full((total,), -1, dtype=torch.int32, device=dev)
+            index = torch.empty((total,), dtype=torch.int32, device=dev)
+            if fill_index:
+                index.fill_(-1)
         else:
             costs = torch.empty((2 * total,), dtype=torch.float64, device=dev)
             index = torch.empty((total,), dtype=torch.int32, device=dev)
@@ -756,6 +761,13 @@ class IntraStageTuner:
                 partial_cost=torch.empty(n_cost, dtype=torch.float64, device=dev),
                 partial_index=torch.empty(n_index, dtype=torch.int32, device=dev),
             )
+        # accumulation count of every row of the tables, and the planes of the p axis that its groups fill
+        groups, n_mesh = plan["groups"], len(self.device_mesh_candidates)
+        n_rows = len(self.gradient_accumulation_steps_candidates) * len(self.tp_sizes)
+        small = np.zeros(n_rows * (1 + n_mesh), dtype=np.int32)
+        small[:n_rows] = list(self.gradient_accumulation_steps_candidates) * len(self.tp_sizes)
+        small[n_rows + groups["g_index"] * n_mesh + groups["q_index"]] = groups["num_p"]
+        small = torch.from_numpy(small).to(dev)
         # several batches alternate between two workspaces on two streams, so that the tail of
         # one batch's launches overlaps the start of the next
         workspaces = [workspace() for _ in range(2 if len(batches) > 1 else 1)]
@@ -763,9 +775,7 @@ class IntraStageTuner:
             batches=batches, workspaces=workspaces, **workspaces[0],
             n_groups=0, groups=None, terms_prefix=None, reduce_prefix=None, scout_prefix=None,
             n_terms_blocks=0, n_reduce_blocks=0, n_scout_blocks=0,
-            grad_accum=torch.tensor(
-                list(self.gradient_accumulation_steps_candidates) * len(self.tp_sizes),
-                dtype=torch.int32, device=dev),
+            grad_accum=small[:n_rows], planes=small[n_rows:].view(n_rows, n_mesh),
         )
         if batches:
             out.update({k: batches[0][k] for k in (
@@ -885,7 +895,7 @@ class IntraStageTuner:
 
     def run_prepared(self, plan, dev_plan,
                      stage_cost_cutoff: Optional[dict] = None,
-                     fill_costs: bool = True) -> List[IntraStageTunerOutput]:
+                     fill_costs: bool = True, sparse: bool = False) -> List[IntraStageTunerOutput]:
         """Device part only: fresh output tables + kernel launches for an uploaded plan; one
         output per tp size, all resident in the same tables.
 
@@ -896,8 +906,14 @@ class IntraStageTuner:
         admit.  Cells above that bound then hold some value above it, not their minimum.
 
         ``fill_costs`` False is for a caller that reads the costs of cells with a row index only:
-        the tables are not pre-filled with +inf."""
+        the tables are not pre-filled with +inf.
+
+        ``sparse`` True (one sample, every cell evaluated, at most 255 layers; ignored otherwise) is for a caller
+        that reads them through ``inter_stage_tune_batch`` only: nothing is pre-filled, and planes of the p axis
+        without a group are not touched (``DeviceTables.planes``)."""
         problem = plan["problem"]
+        sparse = sparse and self.table_samples == 1 and self.cells_wanted is None and self.num_layers <= 255
+        problem["sparse_tables"] = sparse
         problem["stage_cost_incumbent"] = 0
         if stage_cost_cutoff is not None and self.sample_size == 1 and not self.exhaustive:
             with torch.cuda.device(self.device):
@@ -908,11 +924,12 @@ class IntraStageTuner:
             problem["incumbent_num_devices"] = int(stage_cost_cutoff["num_devices"])
             problem["incumbent_ckpt_rule"] = int(stage_cost_cutoff["ckpt_rule"])
         with torch.cuda.device(self.device):
-            costs, index, struct = self._allocate_flat(plan, fill_costs)
+            costs, index, struct = self._allocate_flat(plan, fill_costs and not sparse, not sparse)
             self.launch(plan, dev_plan, struct)
             # (the tensor views of the tables are made while the kernels run)
             tables = self._table_views(costs, index)
             tables.grad_accum = dev_plan.get("grad_accum")
+            tables.planes = dev_plan["planes"] if sparse else None
         return self._outputs(plan, tables)
 
     def tune_all(self) -> List[IntraStageTunerOutput]:

@@ -224,8 +224,8 @@ class PreparedSearch:
         # (tables with a limit are searched by the library's driver only)
         cutoff = self.stage_cost_cutoff if _inter_tuning.NATIVE_SEARCH else None
         # (the cost tables of the searches take +inf where a cell has no row: mist_dp_cost_tables)
-        fill_costs = self.granularity not in ("inter-stage", "uniform-device-pp")
-        results = self.tuner.run_prepared(self.plan, self.dev_plan, cutoff, fill_costs)
+        by_search = self.granularity in ("inter-stage", "uniform-device-pp")
+        results = self.tuner.run_prepared(self.plan, self.dev_plan, cutoff, not by_search, by_search)
         if cutoff is not None:
             # the estimate the kernels ended with travels to the host behind them
             with torch.cuda.device(self.tuner.device):
