@@ -147,12 +147,13 @@ int mist_dp_select_candidates(const MistDpCosts *costs, int n_requests, const in
  * they fit, else the first `first_lead` ones and the rest of the batch spread evenly up to the
  * last one.  The instances are appended to d_inst_tmax / d_inst_row[n_requests * first_chunk]
  * (row -1 in the unused tail: mist_dp_run skips such instances and reports them infeasible).
- *   window_capacity : candidates a request may select (a power of two in [128, 8192])
+ *   window_capacity : candidates a request may select (a power of two in [128, 32768])
  *   d_values[n_requests][window_capacity], d_counts[2 + 2 n_requests] : work space
  *   d_meta[n_requests][8] : selected, candidates above d_hi[r], status, kept, offset of the
  *                   kept thresholds in d_kept, kept thresholds below d_start[r], instances,
  *                   offset of the instances
- * status 0 = done; 1 = skipped (d_start[r] = +inf); 2 = more than window_capacity candidates;
+ * status 0 = done; 1 = skipped (d_start[r] = +inf); 2 = more than window_capacity candidates, or
+ * more than 16384 different ones;
  * 3 = no certain start in the window (MIST_DP_NO_START); 4 = nothing kept at or above d_start[r];
  * 5 = d_kept too small.  A caller that meets a status above 1 decides that window on the host
  * (mist_dp_select_candidates + mist_dp_window_begin). */

@@ -18,6 +18,7 @@
 #include <map>
 #include <tuple>
 #include <mutex>
+#include <set>
 #include <type_traits>
 #include <utility>
 
@@ -528,12 +529,246 @@ __host__ __device__ __forceinline__ int dp_first_batch_index(int k, int n_avail,
 }
 
 constexpr int kWindowThreads = 1024;
+constexpr int kWindowMost = 32768;      // values of a window that is walked on the device ...
+constexpr int kWindowDistinct = 16384;  // ... and different ones among them
+constexpr int kWindowHeld = kWindowMost / kWindowThreads, kWindowOwn = kWindowDistinct / kWindowThreads;
+constexpr int kWindowProbes = 256;      // slots of the hash table (at most half full) that a value tries
+constexpr int kWindowBuckets = 4096;
+constexpr int kWindowBucketMost = 32;  // values in one bucket; where there are more the bitonic sort takes over
+// LDS: a hash table of at least twice the values (as many, of the most), then in its place the different values,
+// buckets, followers and marks
+__host__ __device__ constexpr int window_distinct(int capacity) { return capacity < kWindowDistinct ? capacity : kWindowDistinct; }
+__host__ __device__ constexpr int window_slots(int capacity) { return capacity < kWindowMost ? 2 * capacity : kWindowMost; }
+inline size_t window_lds(int capacity) {
+  const size_t walk = (size_t)window_distinct(capacity) * (sizeof(float) + sizeof(uint16_t) + sizeof(uint8_t)) +
+                      kWindowBuckets * sizeof(int32_t);
+  return std::max(walk, (size_t)window_slots(capacity) * sizeof(float));
+}
 // status of a window walked on the device (meta[r][2])
 constexpr int kWindowOk = 0, kWindowNone = 1, kWindowOverflow = 2, kWindowNoStart = 3,
               kWindowNoBound = 4, kWindowKeptOverflow = 5;
 
-// One workgroup per request of a per-request candidate selection: sorts the request's values
-// (bitonic, in LDS), walks them with the gap rule from the certain start below `start[r]` (the
+// Most values of a window come several times (a stage costs the same for every number of pre-saved
+// micro-batches that fits): the different ones of `n` through a hash table in the LDS of `v` and behind it, then in
+// any order in `v`, by the whole workgroup.  Returns how many there are, -1 if they are more than `most` or one found
+// no slot within kWindowProbes.
+__device__ __forceinline__ int window_distinct_values(const float *__restrict__ in, int n, int slots, int most, float *v) {
+  __shared__ int32_t found;
+  uint32_t *table = reinterpret_cast<uint32_t *>(v);
+  float held[kWindowHeld];
+  const int tid = threadIdx.x, lane = tid & 63;
+  constexpr uint32_t kEmpty = 0x7f800000u;  // (+inf: the values are finite)
+  int bits = 7;
+  while ((1 << bits) < slots && (1 << bits) < 2 * n) ++bits;
+  const uint32_t mask = (1u << bits) - 1u;
+  for (int i = tid; i <= (int)mask; i += kWindowThreads) table[i] = kEmpty;
+  if (tid == 0) found = 0;
+#pragma unroll
+  for (int u = 0; u < kWindowHeld; ++u) {
+    if (u * kWindowThreads >= n) break;
+    held[u] = in[min(u * kWindowThreads + tid, n - 1)];
+  }
+  __syncthreads();
+  uint32_t first = 0;  // bit u: value u is the first of its kind
+  bool lost = false;
+#pragma unroll
+  for (int u = 0; u < kWindowHeld; ++u) {
+    if (u * kWindowThreads >= n) break;
+    if (u * kWindowThreads + tid >= n) continue;
+    const uint32_t key = __float_as_uint(held[u]);
+    uint32_t at = key * 2654435761u >> (32 - bits);
+    int probes = 0;
+    for (; probes < kWindowProbes; ++probes, at = (at + 1) & mask) {
+      const uint32_t there = atomicCAS(table + at, kEmpty, key);
+      if (there == kEmpty) first |= 1u << u;
+      if (there == kEmpty || there == key) break;
+    }
+    lost = lost || probes == kWindowProbes;
+  }
+  int end = __popc(first), base = 0;
+  const int mine = end;
+  for (int step = 1; step < 64; step <<= 1) {
+    const int o = __shfl_up(end, step);
+    if (lane >= step) end += o;
+  }
+  if (lane == 63) base = atomicAdd(&found, end);
+  int at = __shfl(base, 63) + end - mine;
+  if (__syncthreads_or(lost) || found > most) return -1;
+#pragma unroll
+  for (int u = 0; u < kWindowHeld; ++u) {
+    if (u * kWindowThreads >= n) break;
+    if (first >> u & 1u) v[at++] = held[u];
+  }
+  __syncthreads();
+  return found;
+}
+
+// Sorts the `n` different values in `v` (LDS), by the whole workgroup.  They are finite and lie in a narrow range:
+// equal-width buckets, whose number does not decrease with the value, and an insertion sort of what lands in each;
+// where a bucket holds too many, or no width can be given, a bitonic sort.
+__device__ __forceinline__ void window_sort(float *v, int n, int32_t *buckets) {
+  __shared__ float low_of_wave[kWindowThreads / 64], high_of_wave[kWindowThreads / 64];
+  __shared__ int32_t wave_total[kWindowThreads / 64];
+  float held[kWindowOwn];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  float low = INFINITY, high = -INFINITY;
+#pragma unroll
+  for (int u = 0; u < kWindowOwn; ++u) {
+    if (u * kWindowThreads >= n) break;
+    held[u] = v[min(u * kWindowThreads + tid, n - 1)];
+    low = fminf(low, held[u]);
+    high = fmaxf(high, held[u]);
+  }
+  for (int step = 1; step < 64; step <<= 1) {
+    low = fminf(low, __shfl_xor(low, step));
+    high = fmaxf(high, __shfl_xor(high, step));
+  }
+  if (lane == 0) {
+    low_of_wave[wave] = low;
+    high_of_wave[wave] = high;
+  }
+  constexpr int kOwn = kWindowBuckets / kWindowThreads;  // buckets of a thread
+#pragma unroll
+  for (int u = 0; u < kOwn; ++u) buckets[u * kWindowThreads + tid] = 0;
+  __syncthreads();
+  for (int w = 0; w < kWindowThreads / 64; ++w) {
+    low = fminf(low, low_of_wave[w]);
+    high = fmaxf(high, high_of_wave[w]);
+  }
+  const float span = high - low, scale = (float)(kWindowBuckets - 1) / span;
+  const bool fits = span < INFINITY && scale < INFINITY;
+  auto bucket_of = [&](float value) { return min((int)((value - low) * scale), kWindowBuckets - 1); };
+  bool crowded = !fits;
+  int place[kWindowOwn];  // number inside the bucket
+#pragma unroll
+  for (int u = 0; u < kWindowOwn; ++u) {
+    if (!fits || u * kWindowThreads >= n) break;
+    if (u * kWindowThreads + tid >= n) continue;
+    place[u] = atomicAdd(buckets + bucket_of(held[u]), 1);
+    crowded = crowded || place[u] >= kWindowBucketMost;
+  }
+  if (__syncthreads_or(crowded)) {
+    // One compare-exchange per thread and step, thread x holds the pair (i, i + j) with i = 2 j (x / j) + x % j.
+    // For j <= 32 the 64 pairs of a wavefront lie in its own 128 consecutive values, and so do those of the
+    // following smaller j: those steps need no barrier between them (a wavefront's LDS accesses complete in order).
+    int m = 128;
+    while (m < n) m <<= 1;  // (at most the power of two that `v` holds)
+    for (int i = n + tid; i < m; i += kWindowThreads) v[i] = INFINITY;
+    __syncthreads();
+    for (int k = 2; k <= m; k <<= 1) {
+      for (int j = k >> 1; j > 0; j >>= 1) {
+        for (int x = tid; x < m / 2; x += kWindowThreads) {
+          const int i = 2 * (x & ~(j - 1)) + (x & (j - 1)), other = i + j;
+          const float a = v[i], b = v[other];
+          const bool ascending = (i & k) == 0;
+          if ((a > b) == ascending) {
+            v[i] = b;
+            v[other] = a;
+          }
+        }
+        if (j > 32) __syncthreads();
+        else __builtin_amdgcn_wave_barrier();
+      }
+      if (k >= 64) __syncthreads();  // the next k starts with j = k: other wavefronts' values
+    }
+    __syncthreads();
+    return;
+  }
+  // first value of every bucket: an exclusive scan, kOwn neighbouring buckets a thread
+  int count[kOwn], own = 0;
+#pragma unroll
+  for (int u = 0; u < kOwn; ++u) own += count[u] = buckets[tid * kOwn + u];
+  int end = own;
+  for (int step = 1; step < 64; step <<= 1) {
+    const int o = __shfl_up(end, step);
+    if (lane >= step) end += o;
+  }
+  if (lane == 63) wave_total[wave] = end;
+  __syncthreads();
+  int begin = end - own;
+  for (int w = 0; w < wave; ++w) begin += wave_total[w];
+  int next = begin;
+#pragma unroll
+  for (int u = 0; u < kOwn; ++u) {
+    buckets[tid * kOwn + u] = next;
+    next += count[u];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < kWindowOwn; ++u) {
+    if (u * kWindowThreads >= n) break;
+    if (u * kWindowThreads + tid < n) v[buckets[bucket_of(held[u])] + place[u]] = held[u];
+  }
+  __syncthreads();
+  // a thread's buckets are neighbours, and in order: values move a few places
+  for (int i = begin + 1; i < next; ++i) {
+    const float x = v[i];
+    int j = i;
+    for (; j > begin && v[j - 1] > x; --j) v[j] = v[j - 1];
+    v[j] = x;
+  }
+  __syncthreads();
+}
+
+// The walk over `n` > 0 ascending values from `first` on (mist_dp_window_begin's), by the whole workgroup.  A
+// value is followed by the first one that is not within the gap above it (float32 differences do not decrease
+// along the list), whatever was kept before it, and the walk is what the first kept value leads to: every
+// value's follower, then twice, four times .. as far, and each time what the kept ones lead to is kept too.
+__device__ __forceinline__ void window_walk(const float *v, int first, int n, double gap, uint16_t *follow, uint8_t *keep) {
+  const int tid = threadIdx.x;
+  int mine[kWindowOwn];
+#pragma unroll
+  for (int u = 0; u < kWindowOwn; ++u) {
+    const int i = u * kWindowThreads + tid;
+    if (u * kWindowThreads >= n) break;
+    if (i >= n) continue;
+    const float x = v[i];
+    int step = 1, below = i;  // (the last one known to be within the gap)
+    while (below + step < n && gap_below(v[below + step], x, gap)) {
+      below += step;
+      step *= 2;
+    }
+    for (; step > 0; step /= 2)
+      if (below + step < n && gap_below(v[below + step], x, gap)) below += step;
+    mine[u] = below + 1;
+    follow[i] = (uint16_t)mine[u];
+  }
+  // the first one starts with nothing kept (mist_dp_filter_tmax)
+  if (tid == 0) {
+    while (first < n && gap_below(v[first], 0.0f, gap)) ++first;
+    if (first < n) keep[first] = 1;
+  }
+  __syncthreads();
+  for (bool more = true; more;) {
+    more = false;
+    int further[kWindowOwn];
+#pragma unroll
+    for (int u = 0; u < kWindowOwn; ++u) {
+      if (u * kWindowThreads >= n) break;
+      further[u] = n;
+      if (u * kWindowThreads + tid >= n || mine[u] >= n) continue;
+      if (keep[u * kWindowThreads + tid] != 0) keep[mine[u]] = 1;
+      further[u] = follow[mine[u]];
+      more = true;
+    }
+    more = __syncthreads_or(more) != 0;
+#pragma unroll
+    for (int u = 0; u < kWindowOwn; ++u) {
+      if (u * kWindowThreads >= n) break;
+      if (u * kWindowThreads + tid >= n || mine[u] >= n) continue;
+      follow[u * kWindowThreads + tid] = (uint16_t)further[u];
+      mine[u] = further[u];
+    }
+    __syncthreads();
+  }
+}
+
+// (Bound: instruction issue of 16 wavefronts and the barriers between its passes; 14 us for one value, 24 for 2000
+// different ones or 8000 of 400, 50 for 8000, 90 for 16000.  All values, repeated ones too, through a bitonic sort with
+// a division per compare-exchange, and pieces between certain values walked by a thread each: GPT-7B 43 us, now 20;
+// LLaMA-70B 117, now 64; GPT-22B 105, now 52.)
+// One workgroup per request of a per-request candidate selection: sorts the request's different values
+// (in LDS), walks them with the gap rule from the certain start below `start[r]` (the
 // smallest feasible threshold; +inf = nothing feasible, the request is skipped), appends the kept
 // thresholds to one list (kept_out, cursor in counts[0]) and lays out the first scan batch: up to
 // `first_chunk` kept thresholds at or above start[r] (dp_first_batch_index) as DP instances,
@@ -542,13 +777,6 @@ constexpr int kWindowOk = 0, kWindowNone = 1, kWindowOverflow = 2, kWindowNoStar
 // its tail).
 // meta[r][8] = (selected, above hi, status, kept, offset in kept_out, kept below start, instances,
 // offset of the instances).
-//
-// The walk is the host's (mist_dp_window_begin), taken apart along its own argument: a candidate
-// whose predecessor is at least the gap below it is kept whatever came before (the last kept
-// value is at most the predecessor, and the float32 difference is monotone), so the candidates
-// from such a one up to the next are a piece that is walked on its own, by the thread that owns
-// its first element; the piece that starts at the walk's first element begins with "nothing kept
-// yet" like the host's loop.
 __global__ __launch_bounds__(kWindowThreads) void window_walk_kernel(
     const float *__restrict__ values, int capacity, int32_t *__restrict__ counts,
     const int32_t *__restrict__ rows, const float *__restrict__ lo,
@@ -556,8 +784,11 @@ __global__ __launch_bounds__(kWindowThreads) void window_walk_kernel(
     float *__restrict__ kept_out, int kept_capacity, int32_t *__restrict__ meta,
     float *__restrict__ inst_tmax, int32_t *__restrict__ inst_row) {
   extern __shared__ float win_lds[];
-  float *v = win_lds;                                               // [capacity]
-  uint8_t *keep = reinterpret_cast<uint8_t *>(win_lds + capacity);  // [capacity]
+  float *v = win_lds;  // [most]
+  const int most = window_distinct(capacity);
+  int32_t *buckets = reinterpret_cast<int32_t *>(win_lds + most);             // [kWindowBuckets]
+  uint16_t *follow = reinterpret_cast<uint16_t *>(buckets + kWindowBuckets);  // [most]
+  uint8_t *keep = reinterpret_cast<uint8_t *>(follow + most);                 // [most]
   __shared__ int32_t wave_kept[kWindowThreads / 64], wave_below[kWindowThreads / 64];
   __shared__ int32_t walk_first, kept_base, kept_overflow, inst_base;
   const int r = blockIdx.x, n_requests = gridDim.x, tid = threadIdx.x;
@@ -567,44 +798,28 @@ __global__ __launch_bounds__(kWindowThreads) void window_walk_kernel(
   int status = kWindowOk;
   if (!(start_r < INFINITY)) status = kWindowNone;
   else if (n_sel > capacity) status = kWindowOverflow;
-  const int n = status == kWindowOk ? n_sel : 0;
-  int m = 128;  // a wavefront's share of a sorting step is 128 consecutive values
-  while (m < n) m <<= 1;  // capacity is a power of two >= 128
-  for (int i = tid; i < m; i += blockDim.x) {
-    v[i] = i < n ? values[(int64_t)r * capacity + i] : INFINITY;
-    keep[i] = 0;
+  int n = 0;
+  if (status == kWindowOk && n_sel > 0) {  // (the same for the whole workgroup)
+    n = window_distinct_values(values + (int64_t)r * capacity, n_sel, window_slots(capacity), most, v);
+    if (n < 0) {
+      status = kWindowOverflow;
+      n = 0;
+    } else {
+      window_sort(v, n, buckets);
+    }
   }
+  for (int i = tid; i < n; i += blockDim.x) keep[i] = 0;
   if (tid == 0) {
     walk_first = -1;
     kept_overflow = 0;
   }
   __syncthreads();
-  // Bitonic sort, one compare-exchange per thread and step: thread x holds the pair
-  // (i, i + j) with i = 2 j (x / j) + x % j.  For j <= 32 the 64 pairs of a wavefront lie in its
-  // own 128 consecutive values, and so do those of the following smaller j: those steps need no
-  // barrier between them (a wavefront's LDS accesses complete in order).
-  for (int k = 2; k <= m; k <<= 1) {
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      for (int x = tid; x < m / 2; x += blockDim.x) {
-        const int i = 2 * j * (x / j) + x % j, other = i + j;
-        const float a = v[i], b = v[other];
-        const bool ascending = (i & k) == 0;
-        if ((a > b) == ascending) {
-          v[i] = b;
-          v[other] = a;
-        }
-      }
-      if (j > 32) __syncthreads();
-      else __builtin_amdgcn_wave_barrier();
-    }
-    if (k >= 64) __syncthreads();  // the next k starts with j = k: other wavefronts' values
-  }
-  __syncthreads();
   // start of the walk (window_walk_start with a fetch that is not open below): the last
   // candidate <= start_r whose predecessor is at least the gap below, else the first candidate
   // if it lies above start_r and is certain itself
-  const int per = (m + blockDim.x - 1) / blockDim.x;
-  const int i0 = tid * per, i1 = min(i0 + per, n);
+  // (an odd number of values a thread: neighbouring threads' lie in different LDS banks)
+  const int per = ((n + (int)blockDim.x - 1) / (int)blockDim.x) | 1;
+  const int i0 = min(tid * per, n), i1 = min(i0 + per, n);
   {
     int mine = -1;
     for (int i = i0; i < i1; ++i)
@@ -617,25 +832,8 @@ __global__ __launch_bounds__(kWindowThreads) void window_walk_kernel(
     if (v[0] > start_r && !gap_below(v[0], lo_r, gap)) first = 0;
     else status = kWindowNoStart;
   }
-  // the walk, piece by piece
-  if (status == kWindowOk && n > 0) {
-    for (int i = max(i0, first); i < i1; ++i) {
-      const bool head = i == first;
-      if (!head && gap_below(v[i], v[i - 1], gap)) continue;  // inside a piece: its owner walks it
-      float last = 0.0f;  // the walk's first piece starts with nothing kept (mist_dp_filter_tmax)
-      int j = i;
-      if (!head) {
-        keep[i] = 1;
-        last = v[i];
-        j = i + 1;
-      }
-      for (; j < n && (j == i || gap_below(v[j], v[j - 1], gap)); ++j) {
-        if (gap_below(v[j], last, gap)) continue;
-        keep[j] = 1;
-        last = v[j];
-      }
-    }
-  }
+  // the walk
+  if (status == kWindowOk && n > 0) window_walk(v, first, n, gap, follow, keep);
   __syncthreads();
   // kept values per thread (consecutive elements), those below the start among them
   int mine = 0, below = 0;
@@ -2173,6 +2371,19 @@ template <bool kBottleneck>
 size_t fused_lds_limit_of() {
   return lds_limit_of(reinterpret_cast<const void *>(&dp_fused_kernel<kBottleneck>));
 }
+// Allows the window walk the LDS of its largest windows (more than the default 64 KB), once per device.
+int allow_window_lds() {
+  static std::mutex lock;
+  static std::set<int> allowed;
+  int device = 0;
+  MIST_HIP_CHECK(hipGetDevice(&device));
+  std::lock_guard<std::mutex> guard(lock);
+  if (allowed.count(device) != 0) return 0;
+  MIST_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&window_walk_kernel),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)window_lds(kWindowMost)));
+  allowed.insert(device);
+  return 0;
+}
 size_t plane_lds_limit(int mode) {
   // per device: the attribute belongs to the device's copy of the kernel
   static std::mutex lock;
@@ -2558,8 +2769,8 @@ int mist_dp_windows_first_batch(const MistDpCosts *costs, int n_requests, const 
   if (!d_rows || !d_lo || !d_hi || !d_start || !d_values || !d_counts || !d_kept || !d_meta ||
       !d_inst_tmax || !d_inst_row)
     return fail(MIST_E_INVALID, "null pointer argument");
-  if (window_capacity < 128 || window_capacity > 8192 || (window_capacity & (window_capacity - 1)))
-    return fail(MIST_E_INVALID, "window_capacity %d is no power of two in [128, 8192]", window_capacity);
+  if (window_capacity < 128 || window_capacity > kWindowMost || (window_capacity & (window_capacity - 1)))
+    return fail(MIST_E_INVALID, "window_capacity %d is no power of two in [128, %d]", window_capacity, kWindowMost);
   if (first_chunk < 1 || kept_capacity < 1 || (int64_t)n_requests * first_chunk > 65535)
     return fail(MIST_E_INVALID, "first_chunk %d x %d requests outside [1, 65535] / empty kept list",
                 first_chunk, n_requests);
@@ -2575,7 +2786,8 @@ int mist_dp_windows_first_batch(const MistDpCosts *costs, int n_requests, const 
                      d_rows, d_lo, d_hi, d_values, (int32_t *)nullptr, window_capacity, d_counts,
                      true);
   MIST_HIP_CHECK(hipGetLastError());
-  const size_t lds = (size_t)window_capacity * (sizeof(float) + sizeof(uint8_t));
+  const size_t lds = window_lds(window_capacity);
+  if (int rc = allow_window_lds()) return rc;
   hipLaunchKernelGGL(window_walk_kernel, dim3(n_requests), dim3(kWindowThreads), lds, st, d_values,
                      window_capacity, d_counts, d_rows, d_lo, d_start, gap, first_chunk, first_lead,
                      d_kept, kept_capacity, d_meta, d_inst_tmax, d_inst_row);

@@ -48,7 +48,11 @@ constexpr double kFloorSlack = 1e-6;  // relative slack of the bound that lets t
 constexpr int kMaxChunk = 4096;   // most thresholds per G in one batch
 constexpr double kGap = 1e-6;     // inter_tuning.py:177
 constexpr int kSelectHead = 1 << 16;  // selected candidates that travel with the counts of a fetch
-constexpr int kWindowCapacity = 8192;  // candidates of a window that is walked on the device
+// Candidates of a window that is walked on the device, of at most so many bytes of lists.  (8192 left one window of
+// LLaMA-70B, 27317 candidates, and one of GPT-22B, 9332, to the host: a fetch of its own, 0.5 and 0.26 ms on the
+// host and their scans a batch late.)
+constexpr int kWindowCapacity = 32768, kWindowCapacityLeast = 8192;
+constexpr int64_t kWindowListBytes = (int64_t)64 << 20;
 constexpr int kKeptCapacity = 1 << 18;  // kept thresholds of all windows of a search, on the device
 constexpr int kKeptHead = 1 << 15;      // of which this many travel with the first round trip
 const double kInf = std::numeric_limits<double>::infinity();
@@ -910,7 +914,10 @@ static int search_families(int n_families, const MistDpShape *shapes,
 
   std::vector<int> first_batch(n_flat, 0);  // instances of a window the first batch has run
   const char *capacity_env = getenv("MIST_INTER_WINDOW_CAPACITY");  // for tests
-  const int window_capacity = capacity_env ? atoi(capacity_env) : kWindowCapacity;
+  int window_capacity = capacity_env ? atoi(capacity_env) : kWindowCapacity;
+  while (!capacity_env && window_capacity > kWindowCapacityLeast &&
+         (int64_t)sizeof(float) * window_capacity * n_flat > kWindowListBytes)
+    window_capacity /= 2;
   const bool on_device = !getenv("MIST_INTER_HOST_WINDOWS") && (int64_t)n_flat * kFirstChunk <= 65535;
   if (on_device) {
     // ---- smallest feasible threshold of every (instance, G), its window of kept thresholds
