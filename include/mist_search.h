@@ -389,6 +389,21 @@ enum MistDiagField {
 int mist_row_diagnostics(const MistProblem *problem, const MistGroupDesc *d_groups, int n_groups,
                          const int32_t *d_requests, int n_requests, double *d_out, void *stream);
 
+/* Tables to host arrays, in order of the stream; returns when they are there (not for graph capture).
+ *   rows == 0: `count` doubles from `from` (device) to `to`
+ *   rows != 0: `count` int32 row indices from `from` (device); to[count][10] doubles: the strategy row
+ *              (b, dp, tp, wre, gre, ore, wo, go, oo, ao) of the index in d_groups[group]; +inf for an
+ *              index that is not a row of the group (-1: no row), or a group of -1 (an empty space) */
+typedef struct MistFetchItem {
+  const void *from;
+  void *to;
+  int64_t count;
+  int32_t rows, group;
+} MistFetchItem;
+int mist_sizeof_fetch_item(void);
+int mist_fetch_tables(const MistFetchItem *items, int n_items, const MistGroupDesc *d_groups, int n_groups,
+                      void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -101,6 +101,11 @@ GROUP_DTYPE = np.dtype(
 )
 
 
+class FetchItem(ctypes.Structure):
+    _fields_ = [("from_", ctypes.c_void_p), ("to", ctypes.c_void_p), ("count", ctypes.c_int64),
+                ("rows", ctypes.c_int32), ("group", ctypes.c_int32)]
+
+
 class OutTables(ctypes.Structure):
     _fields_ = [
         ("stable", ctypes.c_void_p * 4),
@@ -168,6 +173,8 @@ _SIGNATURES = {
         ctypes.c_int, [_VP, _VP, ctypes.c_int, _VP, _VP, ctypes.c_int, _VP, _VP]),
     "mist_row_diagnostics": (
         ctypes.c_int, [_VP, _VP, ctypes.c_int, _VP, ctypes.c_int, _VP, _VP]),
+    "mist_sizeof_fetch_item": (ctypes.c_int, []),
+    "mist_fetch_tables": (ctypes.c_int, [ctypes.POINTER(FetchItem), ctypes.c_int, _VP, ctypes.c_int, _VP]),
     "mist_intra_stage_eval": (
         ctypes.c_int,
         [_VP, _VP, ctypes.c_int, _VP, ctypes.c_int, _VP, ctypes.c_int, _VP, ctypes.c_int,
@@ -510,6 +517,8 @@ def load():
         raise MistLibraryError(
             f"MistPlanRequest layout mismatch: C {lib.mist_sizeof_plan_request()} vs ctypes "
             f"{ctypes.sizeof(PlanRequest)}")
+    if lib.mist_sizeof_fetch_item() != ctypes.sizeof(FetchItem):
+        raise MistLibraryError("MistFetchItem layout mismatch")
     if lib.mist_sizeof_group() != GROUP_DTYPE.itemsize:
         raise MistLibraryError(
             f"MistGroupDesc layout mismatch: C {lib.mist_sizeof_group()} vs numpy {GROUP_DTYPE.itemsize}"

@@ -71,6 +71,7 @@ def batched_tune_best_latency_for_stage(
     tuner.max_possible_pre_saved_micro_batches = P
     tuner.evaluate_all_p = True
     res = tuner.tune()
+    res.fetch_with_solutions(tuner._dev_plan["groups"], tuner._dev_plan["n_groups"])
     out = []
     for v in range(4):
         out.append((res.costs_f64("stable", v)[0, 0], res.costs_f64("delta", v)[0, 0],

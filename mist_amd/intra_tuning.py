@@ -160,6 +160,24 @@ class IntraStageTunerOutput:
         """float64 ``stable`` / ``delta`` table of variant 0..3 as computed on the GPU."""
         return self._fetch(kind, variant)
 
+    def fetch_with_solutions(self, groups: torch.Tensor, n_groups: int) -> None:
+        """Every table and the decoded strategy rows of a result with one (G, mesh) to the host at once;
+        ``groups``: the call's descriptors on the device (none where its space is empty)."""
+        assert len(self.gradient_accumulation_steps_candidates) == len(self.device_mesh_candidates) == 1
+        items = (_lib.FetchItem * 12)()
+        for v in range(4):
+            for i, (kind, width) in enumerate((("stable", 1), ("delta", 1), ("index", 10))):
+                table = getattr(self.device, kind)[v]
+                host = np.empty(tuple(table.shape) + ((width,) if width > 1 else ()), dtype=np.float64)
+                self._host[f"solutions{v}" if kind == "index" else f"{kind}{v}"] = host
+                items[3 * v + i] = _lib.FetchItem(table.data_ptr(), host.ctypes.data, table.numel(), width > 1,
+                                                  0 if n_groups > 0 else -1)
+        device = self.device.index[0].device
+        with torch.cuda.device(device):
+            _lib.check(_lib.load().mist_fetch_tables(
+                items, len(items), _ptr(groups), n_groups,
+                ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)), "mist_fetch_tables")
+
     def _solutions(self, v: int) -> np.ndarray:
         key = f"solutions{v}"
         if key not in self._host:
