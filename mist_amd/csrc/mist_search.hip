@@ -945,6 +945,20 @@ __global__ __launch_bounds__(kTermsBlock) void row_terms_kernel(
   }
 }
 
+constexpr int kNumXcd = 8;
+// Workgroups are dealt round-robin to the 8 XCDs, each with its own L2.  Logical workgroups
+// that read the same rows are consecutive, so runs of kXcdRun logical workgroups are given to
+// one XCD (and the runs round-robin, which keeps the XCDs evenly loaded).  The grid is padded to
+// a multiple of kNumXcd * kXcdRun; logical indices past the end do nothing.
+constexpr int kXcdRun = 16;
+__device__ __forceinline__ int xcd_run_block(int physical) {
+  const int xcd = physical % kNumXcd, slot = physical / kNumXcd;
+  return ((slot / kXcdRun) * kNumXcd + xcd) * kXcdRun + slot % kXcdRun;
+}
+__host__ __device__ constexpr int xcd_padded_grid(int n_blocks) {
+  return (n_blocks + kNumXcd * kXcdRun - 1) / (kNumXcd * kXcdRun) * (kNumXcd * kXcdRun);
+}
+
 // Stage summaries of every row, from the key terms and without the rows themselves: the search
 // reads the rows of a few stages (22B on 16x8: 67e6 rows, 18 GB, of which 9 % is read), which
 // are computed when it is known which (stage_rows_kernel).  Wavefront = stage, lane = row.  The columns a key decides are
@@ -953,27 +967,135 @@ __global__ __launch_bounds__(kTermsBlock) void row_terms_kernel(
 // VALU: 8 evaluations of the interference model per row.
 constexpr int kFloorCols = 9;               // 6 latencies, PO, PWGO, MF
 constexpr int kFloorPitch = kStageRows + 1;
-__global__ __launch_bounds__(kTermsBlock) void stage_floor_kernel(
-    const MistProblem prob, const MistGroupDesc *__restrict__ groups, int n_groups,
-    const int32_t *__restrict__ block_prefix, double *__restrict__ stage_floor,
-    const double *__restrict__ key_terms) {
-  __shared__ __align__(16) double lds_factor[11][kFactorPitch];
-  __shared__ double lds_gpu_gpu[32];  // (of the tables, not read here)
-  __shared__ double lds_cols[kTermsBlock / kStageRows][kFloorCols * kFloorPitch];
-  __shared__ int lds_keys[kTermsBlock / kStageRows][kStageRows];
-  int local_block;
-  const MistGroupDesc *g = find_group(groups, block_prefix, n_groups, blockIdx.x, &local_block);
-  const int gi = __builtin_amdgcn_readfirstlane((int)(g - groups));
-  g = groups + gi;
-  InterferenceModel<true> I;
-  I.factors_tame = load_model_tables(prob, lds_factor, lds_gpu_gpu);
-  I.table = (LdsDouble *)&lds_factor[0][0];
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kStageRows);
-  const int64_t stage = (int64_t)local_block * (kTermsBlock / kStageRows) + wave;
-  if (stage * kStageRows >= g->n_rows) return;
+constexpr int kFloorThreads = 256, kFloorWaves = kFloorThreads / 64;
+constexpr int kFloorRun = 32;  // terms blocks (two stages each) of a workgroup of stage_floor_runs_kernel
+// Terms blocks from which on the runs are taken.  Their shared parts save a third of the float64 work (1200 vector
+// instructions a stage, 810), but a workgroup waits for more in turn and leaves less room beside the seeds.  From the
+// gathered rows to the filter, every row on its own -> runs: 22B on 16x8 (528000 blocks) 5.20 -> 4.64 ms (alone 3.0 ->
+// 2.6); 70B on 32x8 (45000) and 13B on 8x8 (30000) the same, the seeds are longer; 7B on 4x8 (25200) 447 -> 452 us,
+// uniform-pp of 7B (18900) 230 -> 271, 30 samples of 7B 443 -> 504.
+constexpr int kFloorRunBlocks = 1 << 17;
+// Parts of the lane's row, `lane` behind the first row of the wavefront: from that one's (wave-uniform), block by
+// block (four divisions of the lane's own otherwise, 90 instructions).
+__device__ __forceinline__ RowParts row_behind(const MistGroupDesc *g, const RowParts &first, int lane) {
+  const int n_tiles = (g->n_oo + kOoTile - 1) / kOoTile;
+  RowParts r = first;
+  int tile = first.oo / kOoTile, width = min(kOoTile, g->n_oo - tile * kOoTile);
+  int rest = first.pair * width + (first.oo - tile * kOoTile) + lane;
+  while (__any(rest >= width * g->n_pair)) {
+    if (rest < width * g->n_pair) continue;
+    rest -= width * g->n_pair;
+    if (++tile == n_tiles) {
+      tile = 0;
+      if (++r.ao == g->n_ao) {
+        r.ao = 0;
+        ++r.par;
+      }
+    }
+    width = min(kOoTile, g->n_oo - tile * kOoTile);
+  }
+  // (below 2^16: at most kOoTile pairs of MIST_MAX_PAIRS)
+  r.pair = width == 4 ? rest >> 2 : width == 3 ? rest * 43691 >> 17 : width == 2 ? rest >> 1 : rest;
+  r.oo = tile * kOoTile + (rest - r.pair * width);
+  return r;
+}
+
+// The forward parts that a row shares with others of its (parallelism row, activation ratio, tile of optimizer
+// ratios): of the first layer and before it per (gradient ratio, optimizer ratio), of the last layer per (weight
+// ratio, optimizer ratio), the optimizer's swaps per optimizer ratio.  One stage touches at most 64 / n_pair + 2 such
+// blocks of (n_go + n_wo + 1) kOoTile pairs, n_go + n_wo <= n_pair + 1 or 64: 1584 doubles.
+constexpr int kFloorShared = 2048;
+struct FloorBlocks {
+  int n_go, n_wo, n_tiles, per_block;
+  __device__ __forceinline__ explicit FloorBlocks(const MistGroupDesc *g) : n_tiles((g->n_oo + kOoTile - 1) / kOoTile) {
+    // (the ratios that occur in the pair list, which holds them in order)
+    n_go = n_wo = 0;
+    for (int i = threadIdx.x & 63; i < g->n_pair; i += 64) {
+      n_go = max(n_go, (int)g->pair_go[i] + 1);
+      n_wo = max(n_wo, (int)g->pair_wo[i] + 1);
+    }
+    for (int step = 1; step < 64; step <<= 1) {
+      n_go = max(n_go, __shfl_xor(n_go, step));
+      n_wo = max(n_wo, __shfl_xor(n_wo, step));
+    }
+    n_go = __builtin_amdgcn_readfirstlane(n_go);
+    n_wo = __builtin_amdgcn_readfirstlane(n_wo);
+    per_block = (n_go + n_wo + 1) * kOoTile * 2;
+  }
+  __device__ __forceinline__ int block_of(const MistGroupDesc *g, const RowParts &at) const {
+    return (at.par * g->n_ao + at.ao) * n_tiles + at.oo / kOoTile;
+  }
+  __device__ __forceinline__ int first_of_go(int go, int oo) const { return (go * kOoTile + oo % kOoTile) * 2; }
+  __device__ __forceinline__ int last_of_wo(int wo, int oo) const { return ((n_go + wo) * kOoTile + oo % kOoTile) * 2; }
+  __device__ __forceinline__ int swaps(int oo) const { return ((n_go + n_wo) * kOoTile + oo % kOoTile) * 2; }
+};
+
+// What the first forward phase reads of a row's KeyInputs, and of its key.
+__device__ __forceinline__ KeyInputs floor_inputs(const double *__restrict__ par, double2 links, double2 swapped, double gather) {
+  KeyInputs in = {};
+  in.exec_fwd = par[MIST_PAR_EXEC_FWD];
+  in.extra_fwd = par[MIST_PAR_EXTRA_FWD];
+  in.E_f = in.exec_fwd - in.extra_fwd;
+  in.ore = 1.0;
+  in.AG_w = gather;
+  in.so_W = links.x;
+  in.si_G = links.y;
+  in.so_A_ck = swapped.x;
+  in.so_A_nock = swapped.y;
+  return in;
+}
+
+// The shared parts of blocks [block0, block0 + n_blocks), by the whole workgroup.
+__device__ __forceinline__ void floor_shared_parts(const MistProblem &prob, const MistGroupDesc *__restrict__ g,
+                                                   const FloorBlocks &blocks, const InterferenceModel<true> &I,
+                                                   const double *__restrict__ key_terms, int block0, int n_blocks,
+                                                   double *shared) {
+  const bool adv = prob.adv_first_block != 0;
+  // (entry by entry of all blocks: neighbouring lanes evaluate the same)
+  const int per_entry = n_blocks * kOoTile, n_entries = (blocks.n_go + 2 * blocks.n_wo + 1) * per_entry;
+  for (int e = threadIdx.x; e < n_entries; e += kFloorThreads) {
+    const int entry = e / per_entry, what = e - entry * per_entry, slot = what / kOoTile, block = block0 + slot;
+    const int par_ao = block / blocks.n_tiles, tile = block - par_ao * blocks.n_tiles, oo_i = tile * kOoTile + what % kOoTile;
+    if (oo_i >= g->n_oo) continue;
+    const double *par = g->par[par_ao / g->n_ao];
+    const double oo = g->oo[oo_i], dp = par[MIST_PAR_DP];
+    const double O_shard = par[MIST_PAR_O] / (par[MIST_PAR_ORE] == 1.0 ? dp : 1.0);
+    const double so_O = host_link_latency(prob.gpu_cpu, O_shard * oo);
+    const double si_O = host_link_latency(prob.cpu_gpu, O_shard * oo);
+    // (the gather and the swaps of saved activations are those of any key of the block)
+    const double *__restrict__ key = key_terms + (g->key_offset + (int64_t)par_ao * g->n_pair) * MIST_KEY_TERMS;
+    const double2 swapped = make_double2(key[kKeySoA], key[kKeySoA + 1]);
+    double *out = shared + slot * blocks.per_block;
+    if (entry < blocks.n_go) {
+      const double gre_size = par[MIST_PAR_GRE] == 1.0 ? dp : 1.0;
+      const double si_G = host_link_latency(prob.cpu_gpu, par[MIST_PAR_G] / gre_size * g->go[entry]);
+      const KeyInputs in = floor_inputs(par, make_double2(0.0, si_G), swapped, key[kKeyGather]);
+      double first, extra_pre;
+      fwd_common(I, in, fwd_operands(in, true, so_O, si_O), true, adv, first, extra_pre);
+      *reinterpret_cast<double2 *>(out + blocks.first_of_go(entry, oo_i)) = make_double2(first, extra_pre);
+    } else if (entry < blocks.n_go + 2 * blocks.n_wo) {
+      const int k = (entry - blocks.n_go) & 1, wo = (entry - blocks.n_go) >> 1;  // (with ckpt in front of without)
+      const double wre_size = par[MIST_PAR_WRE] == 1.0 ? dp : 1.0;
+      const double so_W = host_link_latency(prob.gpu_cpu, par[MIST_PAR_W] / wre_size * g->wo[wo]);
+      const KeyInputs in = floor_inputs(par, make_double2(so_W, 0.0), swapped, key[kKeyGather]);
+      const FwdOperands op = fwd_operands(in, true, so_O, si_O);
+      out[blocks.last_of_wo(wo, oo_i) + k] = I.exec_g2c(in.E_f, op.g2c + (k == 0 ? in.so_A_ck : in.so_A_nock)) + in.extra_fwd;
+    } else {
+      *reinterpret_cast<double2 *>(out + blocks.swaps(oo_i)) = make_double2(so_O, si_O);
+    }
+  }
+}
+
+// (kShared false: the stage's blocks have no room, as with a pair list of a few pairs from long lists of ratios)
+template <bool kShared>
+__device__ __forceinline__ void stage_floor_of(const MistProblem &prob, const MistGroupDesc *__restrict__ g, int gi, int stage,
+                                               const FloorBlocks *blocks, int block0, const double *shared,
+                                               const InterferenceModel<true> &I, const double *__restrict__ key_terms,
+                                               double *__restrict__ stage_floor, double *mine, int *keys) {
+  const int lane = threadIdx.x & 63;
   // (lanes past the end repeat the last row: minima do not change)
-  const uint32_t row = (uint32_t)min(stage * kStageRows + lane, g->n_rows - 1);
-  const RowParts at = parts_of_position(g, row);
+  const int64_t row0 = (int64_t)stage * kStageRows;
+  const RowParts at = row_behind(g, parts_of_position(g, (uint32_t)row0), (int)min((int64_t)lane, g->n_rows - 1 - row0));
   const int key = (at.par * g->n_ao + at.ao) * g->n_pair + at.pair;
   const double2 *__restrict__ kt =
       reinterpret_cast<const double2 *>(key_terms + (g->key_offset + key) * MIST_KEY_TERMS);
@@ -989,28 +1111,30 @@ __global__ __launch_bounds__(kTermsBlock) void stage_floor_kernel(
 
   const double *par = g->par[at.par];
   const double oo = g->oo[at.oo];
+  const KeyInputs in = floor_inputs(par, links[0], links[1], gather);
   const double O_shard = par[MIST_PAR_O] / (par[MIST_PAR_ORE] == 1.0 ? par[MIST_PAR_DP] : 1.0);
-  const double so_O = host_link_latency(prob.gpu_cpu, O_shard * oo);
-  const double si_O = host_link_latency(prob.cpu_gpu, O_shard * oo);
-  KeyInputs in = {};  // what the first forward phase reads of it
-  in.exec_fwd = par[MIST_PAR_EXEC_FWD];
-  in.extra_fwd = par[MIST_PAR_EXTRA_FWD];
-  in.E_f = in.exec_fwd - in.extra_fwd;
-  in.ore = 1.0;
-  in.AG_w = gather;
-  in.so_W = links[0].x;
-  in.si_G = links[0].y;
-  in.so_A_ck = links[1].x;
-  in.so_A_nock = links[1].y;
-  const FwdOperands op = fwd_operands(in, true, so_O, si_O);
   double first, extra_pre;
-  fwd_common(I, in, op, true, prob.adv_first_block != 0, first, extra_pre);
-  double *mine = lds_cols[wave];
+  double2 of_last, swaps;
+  if constexpr (kShared) {
+    const double *its = shared + (blocks->block_of(g, at) - block0) * blocks->per_block;
+    const double2 of_first = *reinterpret_cast<const double2 *>(its + blocks->first_of_go(g->pair_go[at.pair], at.oo));
+    first = of_first.x;
+    extra_pre = of_first.y;
+    of_last = *reinterpret_cast<const double2 *>(its + blocks->last_of_wo(g->pair_wo[at.pair], at.oo));
+    swaps = *reinterpret_cast<const double2 *>(its + blocks->swaps(at.oo));
+  } else {
+    swaps = make_double2(host_link_latency(prob.gpu_cpu, O_shard * oo), host_link_latency(prob.cpu_gpu, O_shard * oo));
+    const FwdOperands op = fwd_operands(in, true, swaps.x, swaps.y);
+    fwd_common(I, in, op, true, prob.adv_first_block != 0, first, extra_pre);
+    of_last = make_double2(I.exec_g2c(in.E_f, op.g2c + in.so_A_ck) + in.extra_fwd,
+                           I.exec_g2c(in.E_f, op.g2c + in.so_A_nock) + in.extra_fwd);
+  }
+  const FwdOperands op = fwd_operands(in, true, swaps.x, swaps.y);
   const bool accumulates = g->grad_accum != 1;
 #pragma unroll
   for (int k = 0; k < 2; ++k) {
-    double layer, last, extra_post;
-    fwd_of_ckpt(I, in, op, k != 0, layer, last, extra_post);
+    const double g2c = op.g2c + (k ? in.so_A_ck : in.so_A_nock), last = k ? of_last.x : of_last.y;
+    const double layer = I(in.E_f, op.g2g, g2c, op.c2g) + in.extra_fwd, extra_post = I.g2c_only(g2c);
     // backward family of the last micro-batch: layer, first, last, extra_pre, extra_post
     const double b_layer = k ? bwd[2].y : bwd[0].x, b_first = k ? bwd[3].x : bwd[0].y;
     const double b_last = k ? bwd[3].y : bwd[1].x, b_pre = k ? bwd[4].x : bwd[1].y;
@@ -1034,7 +1158,7 @@ __global__ __launch_bounds__(kTermsBlock) void stage_floor_kernel(
   // the stage's keys, each once
   const bool new_key = lane == 0 || key != __shfl_up(key, 1);
   const uint64_t new_keys = __ballot(new_key);
-  if (new_key) lds_keys[wave][__popcll(new_keys & ((1ull << lane) - 1ull))] = key;
+  if (new_key) keys[__popcll(new_keys & ((1ull << lane) - 1ull))] = key;
   const int n_keys = __popcll(new_keys);
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -1047,7 +1171,7 @@ __global__ __launch_bounds__(kTermsBlock) void stage_floor_kernel(
         key_terms + g->key_offset * MIST_KEY_TERMS + kKeyCols + min(col, kKeyColsEnd - kKeyCols - 1);
 #pragma unroll 8
     for (int i = parity; i < n_keys; i += 2) {
-      const double v = src[(int64_t)lds_keys[wave][i] * MIST_KEY_TERMS];
+      const double v = src[(int64_t)keys[i] * MIST_KEY_TERMS];
       lo = fmin(lo, v);
       hi = fmax(hi, v);
     }
@@ -1085,6 +1209,80 @@ __global__ __launch_bounds__(kTermsBlock) void stage_floor_kernel(
   else if (lane == MIST_T_MF_BASE) v = mf + 0.025 + 0.01;
   else if (lane == kStageMaxOut) v = max_out;
   if (lane < kStageFloorPitch) out[lane] = v;
+}
+
+// Workgroup = two stages, every row on its own.
+__global__ __launch_bounds__(kTermsBlock) void stage_floor_kernel(
+    const MistProblem prob, const MistGroupDesc *__restrict__ groups, int n_groups,
+    const int32_t *__restrict__ block_prefix, double *__restrict__ stage_floor, const double *__restrict__ key_terms) {
+  constexpr int kStages = kTermsBlock / kStageRows;
+  __shared__ __align__(16) double lds_factor[11][kFactorPitch];
+  __shared__ double lds_gpu_gpu[32];  // (of the tables, not read here)
+  __shared__ double lds_cols[kStages][kFloorCols * kFloorPitch];
+  __shared__ int lds_keys[kStages][kStageRows];
+  int local_block;
+  const MistGroupDesc *g = find_group(groups, block_prefix, n_groups, blockIdx.x, &local_block);
+  const int gi = __builtin_amdgcn_readfirstlane((int)(g - groups));
+  g = groups + gi;
+  InterferenceModel<true> I;
+  I.factors_tame = load_model_tables(prob, lds_factor, lds_gpu_gpu);
+  I.table = (LdsDouble *)&lds_factor[0][0];
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kStageRows);
+  const int stage = __builtin_amdgcn_readfirstlane(local_block) * kStages + wave;
+  if ((int64_t)stage * kStageRows >= g->n_rows) return;
+  stage_floor_of<false>(prob, g, gi, stage, nullptr, 0, nullptr, I, key_terms, stage_floor, lds_cols[wave], lds_keys[wave]);
+}
+
+// Workgroup = kFloorRun terms blocks, stage by stage in its wavefronts, with what their rows share evaluated before.
+__global__ __launch_bounds__(kFloorThreads) void stage_floor_runs_kernel(
+    const MistProblem prob, const MistGroupDesc *__restrict__ groups, int n_groups,
+    const int32_t *__restrict__ block_prefix, int n_blocks, double *__restrict__ stage_floor,
+    const double *__restrict__ key_terms) {
+  __shared__ __align__(16) double lds_factor[11][kFactorPitch];
+  __shared__ double lds_gpu_gpu[32];  // (of the tables, not read here)
+  __shared__ double lds_cols[kFloorWaves][kFloorCols * kFloorPitch];
+  __shared__ int lds_keys[kFloorWaves][kStageRows];
+  __shared__ __align__(16) double shared[kFloorShared];
+  InterferenceModel<true> I;
+  I.factors_tame = load_model_tables(prob, lds_factor, lds_gpu_gpu);
+  I.table = (LdsDouble *)&lds_factor[0][0];
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  constexpr int kStages = kTermsBlock / kStageRows;
+  const int first_block = xcd_run_block(blockIdx.x) * kFloorRun;
+  const int end = min(first_block + kFloorRun, n_blocks);
+  for (int block = first_block; block < end;) {  // (a run may hold parts of several groups)
+    int local_block;
+    const MistGroupDesc *g = find_group(groups, block_prefix, n_groups, block, &local_block);
+    const int gi = __builtin_amdgcn_readfirstlane((int)(g - groups));
+    g = groups + gi;
+    const int here = min(end, block_prefix[gi + 1]) - block;
+    const int n_stages = (int)((g->n_rows + kStageRows - 1) / kStageRows);
+    const int stage1 = min((local_block + here) * kStages, n_stages);
+    const FloorBlocks blocks(g);
+    for (int stage0 = local_block * kStages; stage0 < stage1;) {
+      // as many stages as there is room for their blocks
+      const int block0 = blocks.block_of(g, parts_of_position(g, (uint32_t)stage0 * kStageRows));
+      int n = stage1 - stage0, n_touched;
+      for (;; n = (n + 1) / 2) {
+        const int64_t last = min((int64_t)(stage0 + n) * kStageRows, g->n_rows) - 1;
+        n_touched = blocks.block_of(g, parts_of_position(g, (uint32_t)last)) - block0 + 1;
+        if (n == 1 || n_touched * blocks.per_block <= kFloorShared) break;
+      }
+      if (n_touched * blocks.per_block > kFloorShared) {
+        if (wave == 0)
+          stage_floor_of<false>(prob, g, gi, stage0, &blocks, block0, shared, I, key_terms, stage_floor, lds_cols[0], lds_keys[0]);
+        ++stage0;
+        continue;
+      }
+      __syncthreads();  // the wavefronts are done with the blocks before
+      floor_shared_parts(prob, g, blocks, I, key_terms, block0, n_touched, shared);
+      __syncthreads();
+      for (int stage = stage0 + wave; stage < stage0 + n; stage += kFloorWaves)
+        stage_floor_of<true>(prob, g, gi, stage, &blocks, block0, shared, I, key_terms, stage_floor, lds_cols[wave], lds_keys[wave]);
+      stage0 += n;
+    }
+    block += here;
+  }
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1221,7 +1419,6 @@ constexpr int kSuperStages = 8;    // stages per second-level summary
 constexpr int kGatherFloor = 5;    // linear bounds of 64 gathered rows
 constexpr int kQueueShards = 64;   // counters of the item queue: one would serve an append in ~8 ns
 constexpr int kCounterPitch = 32;  // uint32 between counters: a cache line each
-constexpr int kNumXcd = 8;
 constexpr int kCounters = 3 * kQueueShards + kNumXcd;
 constexpr int kSeedThreads = 256;
 constexpr int kReduceThreads = 256;
@@ -1320,19 +1517,6 @@ struct LaneMemory {
     return scaled_pre(p, pre_saved, pre_sas) <= cap;
   }
 };
-
-// Workgroups are dealt round-robin to the 8 XCDs, each with its own L2.  Logical workgroups
-// that read the same rows are consecutive, so runs of kXcdRun logical workgroups are given to
-// one XCD (and the runs round-robin, which keeps the XCDs evenly loaded).  The grid is padded to
-// a multiple of kNumXcd * kXcdRun; logical indices past the end do nothing.
-constexpr int kXcdRun = 16;
-__device__ __forceinline__ int xcd_run_block(int physical) {
-  const int xcd = physical % kNumXcd, slot = physical / kNumXcd;
-  return ((slot / kXcdRun) * kNumXcd + xcd) * kXcdRun + slot % kXcdRun;
-}
-__host__ __device__ constexpr int xcd_padded_grid(int n_blocks) {
-  return (n_blocks + kNumXcd * kXcdRun - 1) / (kNumXcd * kXcdRun) * (kNumXcd * kXcdRun);
-}
 
 __device__ __forceinline__ LaneMemory cell_memory(const double *__restrict__ t, int l, int c);
 
@@ -3922,6 +4106,22 @@ static bool has_key_terms(const MistProblem *problem, int n_groups, const double
 }
 // key_terms_kernel over every group when the caller gave a key-term workspace and the bound the
 // grid needs; *launched tells whether the row-term kernel can read key terms.
+// (for tests MIST_STAGE_FLOOR_RUNS = 0 | 1 decides)
+static bool stage_floor_runs(int n_blocks) {
+  const char *decided = getenv("MIST_STAGE_FLOOR_RUNS");
+  return decided == nullptr || *decided == '\0' ? n_blocks >= kFloorRunBlocks : *decided != '0';
+}
+static void launch_stage_floors(const MistProblem *problem, const MistGroupDesc *d_groups, int n_groups,
+                                const int32_t *d_block_prefix, int n_blocks, double *d_stage_floor,
+                                const double *d_key_terms, hipStream_t stream) {
+  if (!stage_floor_runs(n_blocks))
+    hipLaunchKernelGGL(stage_floor_kernel, dim3(n_blocks), dim3(kTermsBlock), 0, stream, *problem, d_groups, n_groups,
+                       d_block_prefix, d_stage_floor, d_key_terms);
+  else
+    hipLaunchKernelGGL(stage_floor_runs_kernel, dim3(xcd_padded_grid((n_blocks + kFloorRun - 1) / kFloorRun)),
+                       dim3(kFloorThreads), 0, stream, *problem, d_groups, n_groups, d_block_prefix, n_blocks, d_stage_floor,
+                       d_key_terms);
+}
 static int launch_key_terms(const MistProblem *problem, const MistGroupDesc *d_groups, int n_groups,
                             double *d_key_terms, hipStream_t stream, bool *launched) {
   *launched = has_key_terms(problem, n_groups, d_key_terms);
@@ -3946,8 +4146,7 @@ int mist_row_terms(const MistProblem *problem, const MistGroupDesc *d_groups, in
   if (int rc = launch_key_terms(problem, d_groups, n_groups, d_key_terms, (hipStream_t)stream, &from_keys))
     return rc;
   if (from_keys) {
-    hipLaunchKernelGGL(stage_floor_kernel, dim3(n_blocks), dim3(kTermsBlock), 0, (hipStream_t)stream, *problem,
-                       d_groups, n_groups, d_block_prefix, d_stage_floor, d_key_terms);
+    launch_stage_floors(problem, d_groups, n_groups, d_block_prefix, n_blocks, d_stage_floor, d_key_terms, (hipStream_t)stream);
     MIST_HIP_CHECK(hipGetLastError());
     hipLaunchKernelGGL((row_terms_kernel<0, true>), dim3(n_blocks), dim3(kTermsBlock), 0,
                        (hipStream_t)stream, *problem, d_groups, n_groups, d_block_prefix, d_row_terms,
@@ -4412,8 +4611,8 @@ int mist_intra_stage_eval_samples(const MistProblem *problem, const MistGroupDes
     bool from_keys = false;
     if (int rc = launch_key_terms(problem, d_groups, n_groups, d_key_terms, main_stream, &from_keys))
       return rc;
-    hipLaunchKernelGGL(stage_floor_kernel, dim3(n_terms_blocks), dim3(kTermsBlock), 0, main_stream, *problem, d_groups,
-                       n_groups, d_terms_block_prefix, d_stage_floor, d_key_terms);
+    launch_stage_floors(problem, d_groups, n_groups, d_terms_block_prefix, n_terms_blocks, d_stage_floor, d_key_terms,
+                        main_stream);
     MIST_HIP_CHECK(hipGetLastError());
   } else {
     if (int rc = mist_row_terms(problem, d_groups, n_groups, d_terms_block_prefix, n_terms_blocks,
