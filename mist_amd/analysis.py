@@ -29,6 +29,7 @@ import torch
 from . import _lib
 from .comm_model import gpu_gpu_comm_latency
 from .config import BATCH_SIZE_CANDIDATES, MistConfig
+from .intra_tuning import to_device
 from .layer_tables import LayerTables
 from .node_database import layer_tables_for
 from .search_space import SearchSpace
@@ -219,10 +220,19 @@ def analyze_cells(config: MistConfig, tables: LayerTables, stages, device: str =
     builder = GroupInputBuilder(config, tables)
     groups = np.zeros(len(live), dtype=_lib.GROUP_DTYPE)
     requests = []
+    alike: Dict[Tuple, int] = {}  # the first record of a (mesh, G, parallelism); the others have other ratios only
     for gi, i in enumerate(live):
         n, m, G, row, cells = stages[i]
-        builder.fill(groups[gi], _single_row_space(row), 0, gi, n, m, G, 1, analysis_row=row)
-        groups[gi]["row_offset"] = gi
+        like = alike.setdefault((n, m, G, *(float(x) for x in row[:6])), gi)
+        rec = groups[gi]
+        if like == gi:
+            builder.fill(rec, _single_row_space(row), 0, gi, n, m, G, 1, analysis_row=row)
+        else:
+            groups[gi] = groups[like]
+            rec["q_index"] = gi
+            for name, ratio in zip(("wo", "go", "oo", "ao"), row[6:10]):
+                rec[name][0] = float(ratio)
+        rec["row_offset"] = gi
         for p, l, c in cells:
             if not (1 <= l <= L and 0 <= c <= l and p >= 0):
                 raise ValueError(f"cell (p={p}, l={l}, c={c}) outside 1 <= l <= {L}, 0 <= c <= l, p >= 0")
@@ -236,8 +246,7 @@ def analyze_cells(config: MistConfig, tables: LayerTables, stages, device: str =
     terms_prefix = np.arange(n_groups + 1, dtype=np.int32)  # one workgroup per single-row group
     req = np.asarray(requests, dtype=np.int32)
     with torch.cuda.device(dev):
-        to_dev = lambda a: torch.from_numpy(np.ascontiguousarray(a).view(np.uint8).reshape(-1)).to(dev)
-        d_groups, d_prefix, d_req = to_dev(groups), to_dev(terms_prefix), to_dev(req)
+        d_groups, d_prefix, d_req = to_device([groups, terms_prefix, req], dev)
         row_terms = torch.empty(n_groups * _lib.ROW_TERMS, dtype=torch.float64, device=dev)
         stage_floor = torch.empty(lib.mist_stage_floor_doubles(n_groups, n_groups), dtype=torch.float64, device=dev)
         result = torch.empty((len(requests), _lib.ANALYZE_FIELDS), dtype=torch.float64, device=dev)
@@ -250,7 +259,7 @@ def analyze_cells(config: MistConfig, tables: LayerTables, stages, device: str =
                                           d_req.data_ptr(), len(requests), result.data_ptr(), stream),
                    "mist_stage_analyze")
         if diagnostics:
-            diag_req = to_dev(np.array([(gi, 0) for gi in range(n_groups)], dtype=np.int32))
+            (diag_req,) = to_device([np.array([(gi, 0) for gi in range(n_groups)], dtype=np.int32)], dev)
             diag = torch.empty((n_groups, _lib.DIAG_FIELDS), dtype=torch.float64, device=dev)
             _lib.check(lib.mist_row_diagnostics(prob_ptr, d_groups.data_ptr(), n_groups, diag_req.data_ptr(),
                                                 n_groups, diag.data_ptr(), stream), "mist_row_diagnostics")
@@ -286,16 +295,18 @@ def _p2p_output_latency(config: MistConfig, tables: LayerTables, m: int, row) ->
         gpu_gpu_comm_params=config.hardware.gpu_gpu_comm_params)) * 2
 
 
-def _entries(values: np.ndarray, p: int, p2p: float, extra: Optional[Dict[str, float]] = None):
-    """The four per-variant dictionaries of one cell; the last two only exist for p == 0.
+def _entries(values: np.ndarray, p: int, p2p: float, extra: Optional[Dict[str, float]] = None,
+             only: Optional[int] = None):
+    """The four per-variant dictionaries of one cell (of variant ``only`` alone); the last two only exist for p == 0.
     ``extra``: the entries of ``get_extra_info``, merged into each of them as the reference
     does; without it only the stable / delta latencies of the variants are added."""
     dicts = []
-    for v, suffix in enumerate(_VARIANT_KEYS):
+    values = np.asarray(values, dtype=np.float64).tolist()
+    for v in range(len(_VARIANT_KEYS)) if only is None else (only,):
         if v >= 2 and p != 0:
             dicts.append(None)
             continue
-        stable, delta, latency, fwd, bwd = (float(x) for x in values[v])
+        _, _, latency, fwd, bwd = values[v]
         entry = {
             # the pre-and-post variant carries no p2p term (:3071)
             "latency": latency if v == 3 else latency + p2p,
@@ -308,8 +319,8 @@ def _entries(values: np.ndarray, p: int, p2p: float, extra: Optional[Dict[str, f
             for w, key in enumerate(_VARIANT_KEYS):
                 if w >= 2 and p != 0:
                     continue
-                entry["****latency_stable" + key] = float(values[w][0])
-                entry["****latency_delta" + key] = float(values[w][1])
+                entry["****latency_stable" + key] = values[w][0]
+                entry["****latency_delta" + key] = values[w][1]
         dicts.append(entry)
     return dicts
 
@@ -366,12 +377,16 @@ def analyze(mist_config: MistConfig, layer_tables: Optional[LayerTables] = None,
         keys.append((p, l, c))
     found = analyze_cells(mist_config, tables, stages, device)
     results = []
+    p2p_of: Dict[Tuple, float] = {}  # (the same layer output for most stages)
     for i, (cells, key) in enumerate(zip(found, keys)):
         variant = 3 if S == 1 else (1 if i == 0 else (2 if i == S - 1 else 0))
         entry = None
         if cells is not None:
-            p2p = _p2p_output_latency(mist_config, tables, stages[i][1], stages[i][3])
-            entry = _entries(cells[key], key[0], p2p)[variant]
+            m, row = stages[i][1], stages[i][3]
+            output = (m, row[0], row[2])
+            if output not in p2p_of:
+                p2p_of[output] = _p2p_output_latency(mist_config, tables, m, row)
+            entry = _entries(cells[key], key[0], p2p_of[output], only=variant)[0]
         if entry is None:
             raise KeyError(key)  # the reference indexes its empty result dictionary (run.py:84-93)
         results.append((entry, _VARIANT_KEYS[variant]))

@@ -24,7 +24,9 @@ from __future__ import annotations
 
 import bisect
 import ctypes
+import math
 import time
+from itertools import accumulate
 from typing import Dict, List, Optional, Tuple
 
 import numpy as np
@@ -82,9 +84,9 @@ class _DpRunner:
         with torch.cuda.device(self.device):
             # the four cost tables and their running minima: one allocation, eight views
             shapes = [tuple(t.shape[:-1]) for t in dev_tabs.stable]
-            sizes = [int(np.prod(sh)) for sh in shapes]
+            sizes = [math.prod(sh) for sh in shapes]
             flat = torch.empty(2 * sum(sizes), dtype=torch.float32, device=self.device)
-            starts = np.concatenate(([0], np.cumsum(sizes + sizes))).tolist()
+            starts = [0, *accumulate(sizes + sizes)]
             views = [flat[starts[i]:starts[i + 1]].view(shapes[i % 4]) for i in range(8)]
             self.cost, self.pmin = views[:4], views[4:]
             self._per_q = [sizes[v] // (Gn * Q) for v in range(4)]  # elements per (g, mesh)

@@ -141,7 +141,8 @@ def inter_stage_tune_batch(
         if not isinstance(res, IntraStageTunerOutput):
             raise TypeError(
                 f"intra_stage_results must be an instance of IntraStageTunerOutput, got {type(res)}")
-        _, Q, P1, L, _, P = res.device.stable[0].shape
+        # (of a result that is a part of a batch the batch is looked at, below its own rows of it)
+        _, Q, P1, L, _, P = res.batch.stable[0].shape
         if L != num_layers:
             raise ValueError(f"tables hold {L} layers, the search asks for {num_layers}")
         if tuple(res.sample_slots) != tuple(range(P)):
@@ -150,12 +151,12 @@ def inter_stage_tune_batch(
                 f"{tuple(res.sample_slots)} of {P}")
         if P > _lib.MIP_MAX_SAMPLES:
             raise ValueError(f"sample_size {P} exceeds {_lib.MIP_MAX_SAMPLES}")
-        if (res.device.stable[0].shape != first.device.stable[0].shape
+        if (res.batch.stable[0].shape[1:] != first.batch.stable[0].shape[1:]
                 or res.gradient_accumulation_steps_candidates != first.gradient_accumulation_steps_candidates
                 or res.device_mesh_candidates != first.device_mesh_candidates
-                or res.device.stable[0].device != first.device.stable[0].device):
+                or res.batch.stable[0].device != first.batch.stable[0].device):
             raise ValueError("the results of one batch must share table shape, candidates and device")
-    _, Q, P1, L, _, P = first.device.stable[0].shape
+    _, Q, P1, L, _, P = first.batch.stable[0].shape
     g_index = {g: i for i, g in enumerate(first.gradient_accumulation_steps_candidates)}
     q_index = {q: i for i, q in enumerate(first.device_mesh_candidates)}
     mode, fixed = _ckpt_mode(config)
@@ -178,12 +179,13 @@ def inter_stage_tune_batch(
     cell = np.array([r[1] for r in rows], dtype=np.int64) * Q + np.array([r[4] for r in rows], dtype=np.int64)
     for t, res in enumerate(results_list):
         part = items[t * n_items:(t + 1) * n_items]
+        its_cell = cell + res.batch_index * len(first.gradient_accumulation_steps_candidates) * Q
         for v in range(4):
-            for name, tabs in (("stable", res.device.stable), ("delta", res.device.delta)):
+            for name, tabs in (("stable", res.batch.stable), ("delta", res.batch.delta)):
                 tab = tabs[v]
                 assert tab.is_contiguous() and tab.dtype == torch.float64
-                part[name][:, v] = tab.data_ptr() + cell * (tab.stride(1) * 8)
-    dev = first.device.stable[0].device
+                part[name][:, v] = tab.data_ptr() + its_cell * (tab.stride(1) * 8)
+    dev = first.batch.stable[0].device
     with torch.cuda.device(dev):
         ratios = torch.from_numpy(alpha_ratios(P)).to(dev)
         # t_stable, t_delta (float32), index (int32), keep (uint8) of every problem in one buffer

@@ -173,7 +173,7 @@ def inter_stage_tune_batch_uniform(
             raise TypeError(
                 f"intra_stage_results must be an instance of IntraStageTunerOutput, got {type(r)}"
             )
-    if any(r.device.stable[0].device.type != "cuda" for r in results_list):
+    if any(r.batch.stable[0].device.type != "cuda" for r in results_list):
         return [_inter_stage_tune_on_host(num_layers, num_nodes, num_gpus_per_node,
                                           gradient_accumulation_steps_candidates, r, config)
                 for r in results_list]
@@ -183,7 +183,7 @@ def inter_stage_tune_batch_uniform(
         mode = 2
     first = results_list[0]
     q_index = {q: i for i, q in enumerate(first.device_mesh_candidates)}
-    P1 = first.device.stable[0].shape[2]
+    P1 = first.batch.stable[0].shape[2]
     stage_counts, q_of, meshes = [], [], []
     for num_stages in range(1, num_layers + 1):
         if num_nodes * num_gpus_per_node % num_stages != 0:
@@ -202,10 +202,11 @@ def inter_stage_tune_batch_uniform(
         g_index = {G: i for i, G in enumerate(r.gradient_accumulation_steps_candidates)}
         g_of = [g_index[G] for G in gradient_accumulation_steps_candidates]
         best = (float("inf"), None, None)
+        totals = total.tolist()
         for k in range(len(stage_counts)):  # stage counts ascending, then G in the given order; strict "<"
             for i, g in enumerate(g_of):
-                if total[g, k] < best[0]:
-                    best = (float(total[g, k]), i, k)
+                if totals[g][k] < best[0]:
+                    best = (totals[g][k], i, k)
         cost, i, k = best
         if k is None:
             out.append((float("inf"), None))

@@ -11,9 +11,11 @@ fields and layouts as the reference (:59-82); numpy copies are made lazily on fi
 from __future__ import annotations
 
 import ctypes
+import math
 import os
 from collections.abc import Mapping
 from dataclasses import dataclass, field
+from functools import lru_cache
 from typing import Dict, List, Optional, Sequence, Tuple
 
 import numpy as np
@@ -97,6 +99,21 @@ def alpha_ratios(sample_size: int) -> np.ndarray:
     return alpha / (1 - alpha)
 
 
+_cached_ratios = lru_cache(maxsize=None)(alpha_ratios)  # (read only)
+
+
+def to_device(arrays: Sequence[np.ndarray], device: torch.device) -> List[torch.Tensor]:
+    """The bytes of every array on the device, in one copy (each starts at a multiple of 256)."""
+    starts = [0]
+    for a in arrays:
+        starts.append(starts[-1] + (a.nbytes + 255) // 256 * 256)
+    packed = np.empty(max(starts[-1], 1), dtype=np.uint8)
+    for a, at in zip(arrays, starts):
+        packed[at:at + a.nbytes] = np.ascontiguousarray(a).view(np.uint8).reshape(-1)
+    there = torch.from_numpy(packed).to(device)
+    return [there[at:at + a.nbytes] for a, at in zip(arrays, starts)]
+
+
 def _ptr(t: Optional[torch.Tensor]) -> int:
     return 0 if t is None else t.data_ptr()
 
@@ -133,7 +150,7 @@ class IntraStageTunerOutput:
         self,
         gradient_accumulation_steps_candidates: List[int],
         device_mesh_candidates: List[Tuple[int, int]],
-        device: DeviceTables,
+        device: Optional[DeviceTables],
         spaces: Dict[Tuple[int, int], SearchSpace],
         sample_slots: Sequence[int],
         batch: Optional[DeviceTables] = None,
@@ -141,7 +158,7 @@ class IntraStageTunerOutput:
     ):
         self.gradient_accumulation_steps_candidates = list(gradient_accumulation_steps_candidates)
         self.device_mesh_candidates = list(device_mesh_candidates)
-        self.device = device
+        self._device = device
         self.spaces = spaces
         self.sample_slots = tuple(sample_slots)
         # Tables of every tensor-parallel candidate evaluated in the same launch (leading axis
@@ -149,6 +166,17 @@ class IntraStageTunerOutput:
         self.batch = device if batch is None else batch
         self.batch_index = batch_index
         self._host: Dict[str, np.ndarray] = {}
+
+    @property
+    def device(self) -> DeviceTables:
+        """The tables of this tensor-parallel candidate in HBM (cut out of ``batch`` when they are asked for:
+        a search over the whole batch reads none of them by candidate)."""
+        if self._device is None:
+            n = len(self.gradient_accumulation_steps_candidates)
+            rows = slice(self.batch_index * n, (self.batch_index + 1) * n)
+            cut = lambda tables: [x[rows] for x in tables]
+            self._device = DeviceTables(cut(self.batch.stable), cut(self.batch.delta), cut(self.batch.index))
+        return self._device
 
     def _fetch(self, kind: str, v: int) -> np.ndarray:
         key = f"{kind}{v}"
@@ -210,9 +238,12 @@ class IntraStageTunerOutput:
             if idx is None:
                 pending.append(i)
         if pending:
-            fetched = torch.stack(
-                [requests[i][0].device.index[requests[i][1]][requests[i][2]] for i in pending]
-            ).cpu().numpy()
+            def cell_of(res, variant, cell):  # (from the tables of the whole batch where it is a part of them)
+                if res._device is not None:
+                    return res._device.index[variant][cell]
+                n = len(res.gradient_accumulation_steps_candidates)
+                return res.batch.index[variant][(res.batch_index * n + cell[0], *cell[1:])]
+            fetched = torch.stack([cell_of(*requests[i]) for i in pending]).cpu().numpy()
             for i, row in zip(pending, fetched):
                 rows[i] = int(row)
         return [res.spaces[(cell[0], cell[1])].decode(np.array(row))
@@ -659,7 +690,7 @@ class IntraStageTuner:
         shapes = [(Gn, Qn, P1, L, L + 1, S), (Gn, Qn, P1, L, L + 1, S), (Gn, Qn, L, L + 1, S), (Gn, Qn, L + 1, S)]
         starts = [0]
         for shape in shapes:
-            starts.append(starts[-1] + int(np.prod(shape)))
+            starts.append(starts[-1] + math.prod(shape))
         return shapes, starts
 
     def _allocate_flat(self, plan: Optional[dict] = None, fill_costs: bool = True, fill_index: bool = True):
@@ -730,8 +761,6 @@ class IntraStageTuner:
         terms, stage summaries, partial minima) sized for the largest batch and shared by all.
         The top-level entries are those of the first batch (all there is for most plans)."""
         dev = self.device
-        def to_dev(a: np.ndarray) -> torch.Tensor:
-            return torch.from_numpy(np.ascontiguousarray(a).view(np.uint8).reshape(-1)).to(dev)
         lib = _lib.load()
         # sizes of the reduce workspace: the minima of every (tile, slot) of a batch's groups, the
         # second-level summaries, a queue that holds every (tile, stage)
@@ -756,12 +785,19 @@ class IntraStageTuner:
             slabs = max([int(b["reduce_prefix"][-1]) for b in plan["batches"]] + [1]) * _lib.SLOTS * _lib.LC_TILE
             n_index += slabs
             n_cost = max(n_cost, most["reduce_cells"] + slabs)
+        # accumulation count of every row of the tables, and the planes of the p axis that its groups fill
+        groups, n_mesh = plan["groups"], len(self.device_mesh_candidates)
+        n_rows = len(self.gradient_accumulation_steps_candidates) * len(self.tp_sizes)
+        small = np.zeros(n_rows * (1 + n_mesh), dtype=np.int32)
+        small[:n_rows] = list(self.gradient_accumulation_steps_candidates) * len(self.tp_sizes)
+        small[n_rows + groups["g_index"] * n_mesh + groups["q_index"]] = groups["num_p"]
+        parts = ("groups", "terms_prefix", "reduce_prefix", "scout_prefix")
+        there = to_device([b[part] for b in plan["batches"] for part in parts] + [small], dev)
+        small = there[-1].view(torch.int32)
         batches = []
-        for b in plan["batches"]:
+        for i, b in enumerate(plan["batches"]):
             batches.append(dict(
-                n_groups=len(b["groups"]), groups=to_dev(b["groups"]),
-                terms_prefix=to_dev(b["terms_prefix"]), reduce_prefix=to_dev(b["reduce_prefix"]),
-                scout_prefix=to_dev(b["scout_prefix"]),
+                zip(parts, there[len(parts) * i:]), n_groups=len(b["groups"]),
                 n_terms_blocks=int(b["terms_prefix"][-1]), n_reduce_blocks=int(b["reduce_prefix"][-1]),
                 n_scout_blocks=int(b["scout_prefix"][-1]), total_rows=b["total_rows"],
                 total_keys=b["total_keys"],
@@ -779,13 +815,6 @@ class IntraStageTuner:
                 partial_cost=torch.empty(n_cost, dtype=torch.float64, device=dev),
                 partial_index=torch.empty(n_index, dtype=torch.int32, device=dev),
             )
-        # accumulation count of every row of the tables, and the planes of the p axis that its groups fill
-        groups, n_mesh = plan["groups"], len(self.device_mesh_candidates)
-        n_rows = len(self.gradient_accumulation_steps_candidates) * len(self.tp_sizes)
-        small = np.zeros(n_rows * (1 + n_mesh), dtype=np.int32)
-        small[:n_rows] = list(self.gradient_accumulation_steps_candidates) * len(self.tp_sizes)
-        small[n_rows + groups["g_index"] * n_mesh + groups["q_index"]] = groups["num_p"]
-        small = torch.from_numpy(small).to(dev)
         # several batches alternate between two workspaces on two streams, so that the tail of
         # one batch's launches overlaps the start of the next
         workspaces = [workspace() for _ in range(2 if len(batches) > 1 else 1)]
@@ -815,7 +844,7 @@ class IntraStageTuner:
             side = _side_stream(self.device)
             streams.append(side)
             side.wait_stream(current)  # the tables are filled on the current stream
-        ratios = alpha_ratios(self.sample_size)
+        ratios = _cached_ratios(self.sample_size)
         out = tables.as_struct() if isinstance(tables, DeviceTables) else tables
         prob_ptr = ctypes.c_void_p(plan["problem"].ctypes.data)
 
@@ -895,17 +924,11 @@ class IntraStageTuner:
             current.wait_stream(streams[1])
 
     def _outputs(self, plan, tables: DeviceTables) -> List[IntraStageTunerOutput]:
-        Gn = len(self.gradient_accumulation_steps_candidates)
         outs = []
         for t in range(len(self.tp_sizes)):
-            view = DeviceTables(
-                stable=[x[t * Gn:(t + 1) * Gn] for x in tables.stable],
-                delta=[x[t * Gn:(t + 1) * Gn] for x in tables.delta],
-                index=[x[t * Gn:(t + 1) * Gn] for x in tables.index],
-            )
             spaces = _SpacesOfEntry(plan["spaces"], t)
             outs.append(IntraStageTunerOutput(
-                self.gradient_accumulation_steps_candidates, self.device_mesh_candidates, view,
+                self.gradient_accumulation_steps_candidates, self.device_mesh_candidates, None,
                 spaces, range(self.table_samples) if self.compact_samples else self.sample_slots,
                 batch=tables, batch_index=t,
             ))

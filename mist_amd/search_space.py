@@ -71,6 +71,9 @@ class SearchSpace:
         """Rows for an integer index array of any shape -> ``index.shape + (10,)`` float64;
         ``-1`` decodes to an all-``inf`` row like the reference's unfilled solutions."""
         index = np.asarray(index, dtype=np.int64)
+        if 0 < index.size <= 16:  # (the stages of a strategy)
+            rows = [self._decode_one(r) for r in index.ravel().tolist()]
+            return np.array(rows, dtype=np.float64).reshape(index.shape + (10,))
         out = np.full(index.shape + (10,), np.inf, dtype=np.float64)
         valid = index >= 0
         if self.n_rows == 0 or not valid.any():
@@ -89,6 +92,17 @@ class SearchSpace:
         rows[:, 9] = np.asarray(self.ao)[ao_i]
         out[valid] = rows
         return out
+
+    def _decode_one(self, r: int) -> List[float]:
+        if r < 0 or self.n_rows == 0:
+            return [float("inf")] * 10
+        assert r < self.n_rows, "row index outside the search space"
+        n_oo, n_ao = len(self.oo), len(self.ao)
+        par, off = divmod(r, self.n_off)
+        pair, tail = divmod(off, n_oo * n_ao)
+        oo, ao = divmod(tail, n_ao)
+        ratios = (self.wo[self.pair_wo[pair]], self.go[self.pair_go[pair]], self.oo[oo], self.ao[ao])
+        return self.par[par].tolist() + [float(x) for x in ratios]
 
     def materialize(self) -> np.ndarray:
         """The full (N, 10) matrix (tests and small cases only)."""

@@ -10,6 +10,7 @@ bit-identical to what the numpy formulation derives for the same group.
 """
 from __future__ import annotations
 
+import math
 from functools import lru_cache
 from typing import Tuple
 
@@ -46,16 +47,9 @@ def interference_factor_table(params) -> np.ndarray:
     params = [float(x) for x in params]
     if len(params) != 28:
         raise ValueError(f"Length: {len(params)}. It should be 28.")
-    table = np.ones((11, 4), dtype=np.float64)
-    table[0] = params[:4]
-    cursor = 4
-    for row, mask in enumerate(THREE_CASE_MASKS + TWO_CASE_MASKS, start=1):
-        for pos in range(4):
-            if mask[pos]:
-                table[row, pos] = params[cursor]
-                cursor += 1
-    assert cursor == 28
-    return table
+    rest = iter(params[4:])
+    return np.array([params[:4]] + [[next(rest) if used else 1.0 for used in mask]
+                                    for mask in THREE_CASE_MASKS + TWO_CASE_MASKS], dtype=np.float64)
 
 
 def latency_exec(
@@ -139,16 +133,17 @@ def make_problem(
     prob["num_grad_accum"] = num_grad_accum
     prob["num_mesh"] = num_mesh
     prob["adv_first_block"] = 1 if config.enable_advanced_opt_in_first_block else 0
-    bandwidths = np.concatenate([prob["gpu_gpu"][0][0::2], prob["cpu_gpu"][0][:1], prob["gpu_cpu"][0][:1]])
-    offsets = np.concatenate([prob["gpu_gpu"][0][1::2], prob["cpu_gpu"][0][1:], prob["gpu_cpu"][0][1:]])
-    if not (np.all(np.isfinite(bandwidths)) and np.all(bandwidths > 0)):
+    finite = lambda values: all(map(math.isfinite, values))
+    links = prob["gpu_gpu"][0].tolist() + prob["cpu_gpu"][0].tolist() + prob["gpu_cpu"][0].tolist()
+    if not (finite(links[0::2]) and min(links[0::2]) > 0):
         raise ValueError("communication bandwidths (k of every (k, b) pair) must be positive and finite")
-    if not (np.all(np.isfinite(offsets)) and np.all(offsets >= 0)):
+    if not (finite(links[1::2]) and min(links[1::2]) >= 0):
         raise ValueError("communication latencies (b of every (k, b) pair) must be non-negative and finite")
-    factors = prob["interf_factor"][0]
-    if not (np.all(np.isfinite(factors)) and np.all(factors > 0)):
+    factors = prob["interf_factor"][0].ravel().tolist()
+    if not (finite(factors) and min(factors) > 0):
         raise ValueError("interference factors must be positive and finite")
-    if not (np.isfinite(prob["mem_cap_mb"][0]) and prob["mem_cap_mb"][0] > 0):
+    capacity = float(prob["mem_cap_mb"][0])
+    if not (math.isfinite(capacity) and capacity > 0):
         raise ValueError("memory capacity must be positive and finite")
     return prob
 
@@ -169,6 +164,7 @@ class GroupInputBuilder:
         self._block = lru_cache(maxsize=None)(self._block_uncached)
         self._par_fields = lru_cache(maxsize=None)(self._par_fields_uncached)
         self._pre_post = lru_cache(maxsize=None)(self._pre_post_uncached)
+        self._analysed = {}
 
     def _exec_uncached(self, kind, b, tp, inter, intra, G):
         return latency_exec(self.tables, kind, b, tp, inter, intra, G)
@@ -253,8 +249,11 @@ class GroupInputBuilder:
         # ---- pre / post layers: the same for every tp candidate of a (mesh, G) ----
         if analysis_row is None:
             fields = self._pre_post(n, m, G)
-        else:
-            fields = self._pre_post_uncached(n, m, G, analysis_row)
+        else:  # (of the row only its pre / post strategy counts)
+            key = (n, m, G, pre_post_strategy_fields(cfg, n, m, analysis_row))
+            fields = self._analysed.get(key)
+            if fields is None:
+                fields = self._analysed[key] = self._pre_post_uncached(n, m, G, analysis_row)
         for name, value in fields.items():
             rec[name] = value
 
@@ -350,6 +349,11 @@ class GroupInputBuilder:
         pre-saved micro-batches and in every row term).  Real tables always are; a violation is
         rejected here instead of silently changing which rows get evaluated.  ``recs``: filled
         ``GROUP_DTYPE`` records (unused array slots hold zero)."""
+        first = recs.dtype.fields["pre_full_w"][1]  # (the last fields, all doubles)
+        ends = recs.view(np.uint8).reshape(len(recs), recs.dtype.itemsize)[:, first:].view(np.float64)
+        if np.all((ends >= 0) & (ends < np.inf)) and np.all((recs["par"] >= 0) & (recs["par"] < np.inf)) and all(
+                np.all((recs[name] >= 0) & (recs[name] <= 1)) for name in ("wo", "go", "oo", "ao")):
+            return
         par = recs["par"]
         if not np.all(np.isfinite(par)) or np.any(par < 0):
             raise ValueError("layer table values must be finite and non-negative")
