@@ -35,7 +35,7 @@ import torch
 
 from . import _lib
 from .inter_tuning_uniform import _uniform_device_mesh_partition
-from .intra_tuning import IntraStageTunerOutput, alpha_ratios
+from .intra_tuning import IntraStageTunerOutput, alpha_ratios, fetch_doubles, to_device
 
 MAX_VALUE = _lib.MIP_MAX_VALUE  # inter_tuning_mip.py:39
 
@@ -187,18 +187,20 @@ def inter_stage_tune_batch(
                 part[name][:, v] = tab.data_ptr() + its_cell * (tab.stride(1) * 8)
     dev = first.batch.stable[0].device
     with torch.cuda.device(dev):
-        ratios = torch.from_numpy(alpha_ratios(P)).to(dev)
+        ratios, d_items = to_device([alpha_ratios(P), items], dev)
         # t_stable, t_delta (float32), index (int32), keep (uint8) of every problem in one buffer
-        out = torch.empty(13 * total, dtype=torch.uint8, device=dev)
-        d_items = torch.from_numpy(items.view(np.uint8).reshape(-1)).to(dev)
+        words = (13 * total + 7) // 8
+        out = torch.empty(words, dtype=torch.float64, device=dev)
         rc = lib.mist_mip_stage_samples_batch(
             ctypes.c_void_p(items.ctypes.data), d_items.data_ptr(), len(items), ratios.data_ptr(),
             out.data_ptr(), out.data_ptr() + 4 * total, out.data_ptr() + 8 * total,
             out.data_ptr() + 12 * total, ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream))
         _lib.check(rc, "mist_mip_stage_samples_batch")
-        host = out.cpu().numpy()
+        host = np.empty(words, dtype=np.float64)
+        fetch_doubles(out, host)
+        host = host.view(np.uint8)
     t_stable, t_delta = host[:4 * total].view(np.float32), host[4 * total:8 * total].view(np.float32)
-    index, keep = host[8 * total:12 * total].view(np.int32), host[12 * total:]
+    index, keep = host[8 * total:12 * total].view(np.int32), host[12 * total:13 * total]
     t1 = time.perf_counter()
 
     G_of = np.array([r[0] for r in rows], dtype=np.int32)

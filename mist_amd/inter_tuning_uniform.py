@@ -19,7 +19,7 @@ import torch
 from . import _lib
 from .config import MistConfig
 from .inter_tuning import get_solution_from_intra_stage_tuner_output
-from .intra_tuning import IntraStageTunerOutput
+from .intra_tuning import IntraStageTunerOutput, to_device
 
 
 def _uniform_layer_partition(num_layers: int, num_stages: int) -> List[int]:
@@ -141,7 +141,7 @@ def _search_on_device(num_layers, stage_counts, q_of, max_stages, results_list, 
         dev = tabs.stable[0].device
         with torch.cuda.device(dev):
             Gs = np.array([G for r in results for G in r.gradient_accumulation_steps_candidates], dtype=np.int32)
-            d_in = torch.from_numpy(np.concatenate((Gs, problems.reshape(-1)))).to(dev)
+            (d_in,) = to_device([np.concatenate((Gs, problems.reshape(-1)))], dev)
             n_cells = rows * n_k * max_stages
             d_out = torch.empty(2 * rows * n_k + 2 * n_cells, dtype=torch.int32, device=dev)
             at = d_out.data_ptr()

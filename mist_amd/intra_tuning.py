@@ -99,19 +99,32 @@ def alpha_ratios(sample_size: int) -> np.ndarray:
     return alpha / (1 - alpha)
 
 
+PINNED_UPLOAD_BYTES = 256 << 10
+
 _cached_ratios = lru_cache(maxsize=None)(alpha_ratios)  # (read only)
 
 
 def to_device(arrays: Sequence[np.ndarray], device: torch.device) -> List[torch.Tensor]:
-    """The bytes of every array on the device, in one copy (each starts at a multiple of 256)."""
+    """The bytes of every array on the device, in one copy in order of the current stream (each starts at a
+    multiple of 256).  From pinned memory, since a copy of other memory returns when what was queued before it is
+    done, unless they are many: those go through another engine, which the next kernel waits for longer."""
     starts = [0]
     for a in arrays:
         starts.append(starts[-1] + (a.nbytes + 255) // 256 * 256)
-    packed = np.empty(max(starts[-1], 1), dtype=np.uint8)
+    staged = torch.empty(max(starts[-1], 1), dtype=torch.uint8,
+                         pin_memory=device.type == "cuda" and starts[-1] <= PINNED_UPLOAD_BYTES)
+    packed = staged.numpy()
     for a, at in zip(arrays, starts):
         packed[at:at + a.nbytes] = np.ascontiguousarray(a).view(np.uint8).reshape(-1)
-    there = torch.from_numpy(packed).to(device)
+    there = staged.to(device, non_blocking=True)
     return [there[at:at + a.nbytes] for a, at in zip(arrays, starts)]
+
+
+def fetch_doubles(source: torch.Tensor, out: np.ndarray) -> None:
+    """A contiguous float64 tensor on the device into a host array of as many, in order of the current stream."""
+    items = (_lib.FetchItem * 1)(_lib.FetchItem(source.data_ptr(), out.ctypes.data, source.numel(), 0, -1))
+    _lib.check(_lib.load().mist_fetch_tables(
+        items, 1, None, 0, ctypes.c_void_p(torch.cuda.current_stream(source.device).cuda_stream)), "mist_fetch_tables")
 
 
 def _ptr(t: Optional[torch.Tensor]) -> int:
