@@ -2097,17 +2097,18 @@ __global__ __launch_bounds__(kDpHistoryThreads, 8) void dp_history_kernel(
 // The recurrence of one mesh for all stages (free_devices): a state is a start layer, F(s) has
 // L + 1 values, and all of them stay in LDS.  With a launch per stage count a search of 6 stage
 // counts (1, 2, .. 32) in four batches made 250 launches of 3 to 8 us with as long a gap behind
-// each.  Here a workgroup runs an instance through all stage counts: per count it gathers the row
-// minima (consecutive end layers of a stage length are neighbours in the tables; up to
-// kDpFreeLoads reads of a lane in flight), then a wavefront takes a start layer with its lanes on
-// the end layers.  Bound: latency of that gather and two barriers, 2.5 us per stage count at 37
-// layers.  Six families of that plan: 250 launches, 3.3 ms from the first to the last -> 18, 0.75.
+// each.  Here a workgroup runs an instance through all stage counts: per count the row minima
+// (consecutive end layers of a stage length are neighbours in the tables), read while the count
+// before is worked on, go to LDS, then eight lanes take a start layer.  Bound: LDS latency and two
+// barriers, 0.8 us per stage count at 37 layers.  (Read where they are needed, each place from its
+// row and variant, and a wavefront a start layer, five in turn with six exchanges each: 2.5 us; the
+// four launches of 13B on 4x8 100, 219, 89 and 76 us, now 35, 155, 31 and 28.)  Six families of that plan: 250 launches, 3.3 ms from the first to the last -> 18, 0.75.
 // The families of a search wait for nothing of each other: up to kDpFreeFamilies go through one
 // launch, workgroup = (instance, family), the ones given last (more stage counts as a rule) first:
 // 24 launches, 0.89 ms of 13B on 4x8 -> 4, 0.50.
 // ------------------------------------------------------------------------------------------
 constexpr int kDpFreeThreads = 512;
-constexpr int kDpFreeLoads = 4;
+constexpr int kDpFreeLoads = 4, kDpFreeMostLoads = 16;  // values a thread reads ahead: up to 45 layers, up to 90
 constexpr int kDpFreeFamilies = 8;
 struct DpFreeFamily {
   MistDpCosts costs;
@@ -2122,7 +2123,17 @@ inline size_t dp_free_lds(int L, int S) {
   return ((size_t)L * L + (size_t)(S + 1) * (L + 1) + S) * sizeof(float);
 }
 
-template <bool kBottleneck>
+// Smallest value of eight neighbouring lanes, in each of them.
+__device__ __forceinline__ float eight_lane_min(float v) {
+#define MIST_MIN_DPP(CTRL) v = fminf(v, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true)))
+  MIST_MIN_DPP(0xB1);   // quad_perm [1,0,3,2]
+  MIST_MIN_DPP(0x4E);   // quad_perm [2,3,0,1]
+  MIST_MIN_DPP(0x141);  // row_half_mirror
+#undef MIST_MIN_DPP
+  return v;
+}
+
+template <bool kBottleneck, int kLoads>
 __global__ __launch_bounds__(kDpFreeThreads) void dp_free_kernel(
     const DpFreeFamilies families, int num_layers, const float *__restrict__ tmax_list,
     const int32_t *__restrict__ g_list) {
@@ -2162,38 +2173,55 @@ __global__ __launch_bounds__(kDpFreeThreads) void dp_free_kernel(
   const float t_max = kBottleneck ? kDpNoThreshold : tmax_list[t];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  constexpr int kWaves = kDpFreeThreads / 64;
   for (int k = threadIdx.x; k <= L; k += kDpFreeThreads) history[k] = k == L ? 0.0f : INFINITY;
+  // row minima of the stages (k, i) behind which s - 1 layers are left (s = 1: none); the first kLoads values of a
+  // thread are read a stage count ahead, from places that move by one plane of the tables with it
+  const bool all_ckpt = shape.ckpt_rule == MIST_DP_CKPT_ALL;
+  const float *__restrict__ inner = dp_table(tabs, 0, !all_ckpt) + off[0], *__restrict__ front = dp_table(tabs, 1, !all_ckpt) + off[1];
+  const int held = tabs.planes == nullptr ? S : tabs.planes[g * tabs.planes_g_stride];
+  int end_of[kLoads], place[kLoads];
+#pragma unroll
+  for (int u = 0; u < kLoads; ++u) {
+    const int x = threadIdx.x + u * kDpFreeThreads, i = x % L, k = i - x / L;
+    end_of[u] = x < L * L && k >= 0 ? i : L;  // (no end layer: never read)
+    place[u] = k < 0 ? 0 : (((i - k) * (L + 1) + (all_ckpt ? i - k + 1 : dp_j_last(shape, k, i))) << 1) | (k == 0 ? 1 : 0);
+  }
+  auto row_min = [&](int s, int x) {
+    const int i = x % L, k = i - x / L;
+    const bool wanted = x < L * L && k >= 0 && i <= L - s && (s > 1 || i == L - 1);
+    return wanted ? dp_row_min(shape, tabs, g, off, s - 1, k, 0, i) : INFINITY;
+  };
+  auto put = [&](int x, float value) {
+    if (x < L * L) rows[x] = value <= t_max ? value : INFINITY;
+  };
+  float value[kLoads];
+#pragma unroll
+  for (int u = 0; u < kLoads; ++u) value[u] = row_min(1, threadIdx.x + u * kDpFreeThreads);
   for (int s = 1; s <= S; ++s) {
     const float *f_prev = history + (s - 1) * (L + 1);
     float *f_cur = history + s * (L + 1);
-    // row minima of the stages (k, i) behind which s - 1 layers are left (s = 1: none)
-    for (int x0 = threadIdx.x; x0 < L * L; x0 += kDpFreeLoads * kDpFreeThreads) {
-      float value[kDpFreeLoads];
 #pragma unroll
-      for (int u = 0; u < kDpFreeLoads; ++u) {
-        const int x = x0 + u * kDpFreeThreads;
-        const int i = x % L, k = i - x / L;
-        const bool wanted = x < L * L && k >= 0 && i <= L - s && (s > 1 || i == L - 1);
-        value[u] = wanted ? dp_row_min(shape, tabs, g, off, s - 1, k, 0, i) : INFINITY;
-      }
+    for (int u = 0; u < kLoads; ++u) put(threadIdx.x + u * kDpFreeThreads, value[u]);
+    for (int x = threadIdx.x + kLoads * kDpFreeThreads; x < L * L; x += kDpFreeThreads) put(x, row_min(s, x));
+    __syncthreads();
+    if (s < S) {
+      const int64_t plane = (int64_t)s * L * (L + 1);
 #pragma unroll
-      for (int u = 0; u < kDpFreeLoads; ++u) {
-        const int x = x0 + u * kDpFreeThreads;
-        if (x < L * L) rows[x] = value[u] <= t_max ? value[u] : INFINITY;
+      for (int u = 0; u < kLoads; ++u) {
+        const float *__restrict__ from = ((place[u] & 1) != 0 ? front : inner) + plane;
+        value[u] = end_of[u] < L - s && s < held ? from[place[u] >> 1] : INFINITY;
       }
     }
-    __syncthreads();
-    for (int k = wave; k <= L; k += kWaves) {
+    // eight lanes a start layer
+    for (int k = threadIdx.x / 8; k <= L; k += kDpFreeThreads / 8) {
       float best = INFINITY;
-      for (int i = k + lane; i <= L - s; i += 64) {
+      for (int i = k + (threadIdx.x & 7); i <= L - s; i += 8) {
         const float rmin = rows[(i - k) * L + i], prev = f_prev[i + 1];
         // (an inadmissible row is +inf here, and so is its target)
         best = fminf(best, kBottleneck ? fmaxf(rmin, prev) : rmin + prev);
       }
-#pragma unroll
-      for (int step = 32; step >= 1; step >>= 1) best = fminf(best, __shfl_xor(best, step));
-      if (lane == 0) f_cur[k] = best;
+      best = eight_lane_min(best);
+      if ((threadIdx.x & 7) == 0) f_cur[k] = best;
     }
     __syncthreads();
   }
@@ -2844,12 +2872,11 @@ static int launch_dp_free(const mist::DpFreeRun *runs, int n, const float *d_tma
                             run.d_best_s, run.d_path, run.d_best_sum, run.d_stage_max};
       lds = std::max(lds, dp_free_lds(L, shape.max_stages));
     }
-    if (mode == MIST_DP_BOTTLENECK)
-      hipLaunchKernelGGL(dp_free_kernel<true>, dim3(n_tmax, here), dim3(kDpFreeThreads), lds, stream, families, L, d_tmax,
-                         d_g_index);
-    else
-      hipLaunchKernelGGL(dp_free_kernel<false>, dim3(n_tmax, here), dim3(kDpFreeThreads), lds, stream, families, L, d_tmax,
-                         d_g_index);
+    const bool few = L * L <= kDpFreeLoads * kDpFreeThreads;
+    const auto kernel = mode == MIST_DP_BOTTLENECK
+                            ? (few ? dp_free_kernel<true, kDpFreeLoads> : dp_free_kernel<true, kDpFreeMostLoads>)
+                            : (few ? dp_free_kernel<false, kDpFreeLoads> : dp_free_kernel<false, kDpFreeMostLoads>);
+    hipLaunchKernelGGL(kernel, dim3(n_tmax, here), dim3(kDpFreeThreads), lds, stream, families, L, d_tmax, d_g_index);
     MIST_HIP_CHECK(hipGetLastError());
   }
   return 0;
