@@ -153,6 +153,28 @@ class DeviceTables:
             s.index[v] = self.index[v].data_ptr()
         return s
 
+    def rows(self, rows: slice) -> "DeviceTables":
+        """Tables of some rows: views, except of tables without a pre-fill, of which complete copies are made
+        (-1 and +inf in the cells that hold nothing)."""
+        cut = lambda tables: [x[rows] for x in tables]
+        out = DeviceTables(cut(self.stable), cut(self.delta), cut(self.index),
+                           None if self.grad_accum is None else self.grad_accum[rows])
+        if self.planes is None:
+            return out
+        planes = self.planes[rows]
+        _, _, P1, L, C, _ = out.stable[0].shape
+        p, l, c = (torch.arange(first, first + n, device=planes.device) for first, n in ((0, P1), (1, L), (0, C)))
+        l, p, held = l[:, None], p[:, None, None], p < planes[:, :, None]
+        # cells that are written (batched_module_analyzer.py:3021-3023, 3103) in planes that hold something
+        inner = held[..., None, None] & (c <= l) & ((c != l - 1) | (p == 0))
+        post, single = ((c <= n) & (c != n - 1) & (planes > 0).view(*planes.shape, *[1] * n_axes)
+                        for n, n_axes in ((l, 2), (L, 1)))
+        for v, written in enumerate((inner, inner, post, single)):
+            out.index[v] = out.index[v].where(written[..., None], -1)
+            for costs in (out.stable, out.delta):
+                costs[v] = costs[v].where(out.index[v] >= 0, float("inf"))
+        return out
+
 
 class IntraStageTunerOutput:
     """Same attributes as the reference's ``IntraStageTunerOutput`` (intra_tuning.py:59-82):
@@ -186,9 +208,7 @@ class IntraStageTunerOutput:
         a search over the whole batch reads none of them by candidate)."""
         if self._device is None:
             n = len(self.gradient_accumulation_steps_candidates)
-            rows = slice(self.batch_index * n, (self.batch_index + 1) * n)
-            cut = lambda tables: [x[rows] for x in tables]
-            self._device = DeviceTables(cut(self.batch.stable), cut(self.batch.delta), cut(self.batch.index))
+            self._device = self.batch.rows(slice(self.batch_index * n, (self.batch_index + 1) * n))
         return self._device
 
     def _fetch(self, kind: str, v: int) -> np.ndarray:
@@ -252,8 +272,8 @@ class IntraStageTunerOutput:
                 pending.append(i)
         if pending:
             def cell_of(res, variant, cell):  # (from the tables of the whole batch where it is a part of them)
-                if res._device is not None:
-                    return res._device.index[variant][cell]
+                if res._device is not None or res.batch.planes is not None:
+                    return res.device.index[variant][cell]
                 n = len(res.gradient_accumulation_steps_candidates)
                 return res.batch.index[variant][(res.batch_index * n + cell[0], *cell[1:])]
             fetched = torch.stack([cell_of(*requests[i]) for i in pending]).cpu().numpy()
@@ -963,8 +983,9 @@ class IntraStageTuner:
         the tables are not pre-filled with +inf.
 
         ``sparse`` True (one sample, every cell evaluated, at most 255 layers; ignored otherwise) is for a caller
-        that reads them through ``inter_stage_tune_batch`` only: nothing is pre-filled, and planes of the p axis
-        without a group are not touched (``DeviceTables.planes``)."""
+        that reads them through ``inter_stage_tune_batch``: nothing is pre-filled, and planes of the p axis
+        without a group are not touched (``DeviceTables.planes``).  Anything else that is read of such a result
+        comes from complete copies of its tables (``DeviceTables.rows``)."""
         problem = plan["problem"]
         sparse = sparse and self.table_samples == 1 and self.cells_wanted is None and self.num_layers <= 255
         problem["sparse_tables"] = sparse

@@ -88,18 +88,81 @@ def test_planes_equal_complete_tables(L, P1, meshes):
     assert [inter_stage_tune_batch(L, D, meshes, Gs, ours, uniform_device=u) for u in searches] == want
 
 
-@pytest.mark.parametrize("granularity", ["inter-stage", "uniform-device-pp"])
-def test_tune_on_used_memory(granularity):
-    """Tables that nothing fills lie in memory that held other indices and costs."""
+def _leave_used_memory(value):
+    """Blocks of the allocator's two pools that hold ``value`` and are free again."""
     import torch
 
+    torch.cuda.empty_cache()
+    used = [torch.full((1 << bits,), value, dtype=torch.int32, device="cuda")
+            for bits in [28, 26, 24, 22, 20] + [bits for bits in range(18, 6, -1) for _ in range(48)]]
+    del used
+
+
+def _count_used_tables(monkeypatch, tuner, value):
+    """How often the tables of ``tuner`` begin as indices of ``value`` and nothing else."""
+    import torch
+
+    allocate, seen = tuner._allocate_flat, []
+
+    def allocated(*args):
+        costs, index, struct = allocate(*args)
+        seen.append(torch.equal(index, torch.full_like(index, value)))
+        return costs, index, struct
+
+    monkeypatch.setattr(tuner, "_allocate_flat", allocated)
+    return seen
+
+
+@pytest.mark.parametrize("granularity", ["inter-stage", "uniform-device-pp"])
+def test_tune_on_used_memory(monkeypatch, granularity):
+    """Tables that nothing fills lie in memory that held other indices and costs."""
     from mist_amd.tune_one_case import PreparedSearch
     from tests.util import load_plan
 
     cfg, _ = load_plan(1, tuning__tuning_granularity=granularity)
     want = PreparedSearch(cfg).run()
     for value in (0, 5, 0x3f000000):
-        torch.cuda.empty_cache()
-        used = [torch.full((n,), value, dtype=torch.int32, device="cuda") for n in (1 << 20, 1 << 24, 1 << 26)]
-        del used
-        assert PreparedSearch(cfg).run() == want
+        search = PreparedSearch(cfg)
+        seen = _count_used_tables(monkeypatch, search.tuner, value)
+        _leave_used_memory(value)
+        assert search.run() == want
+        assert seen and seen[0], value
+
+
+@pytest.mark.parametrize("native", [True, False])
+def test_parts_of_a_run_without_a_fill(monkeypatch, native):
+    """A search over some tensor-parallel candidates of such a run, and tables read from its results, know which
+    cells hold something too."""
+    import mist_amd.inter_tuning as inter_tuning
+    from mist_amd.intra_tuning import VARIANTS, IntraStageTunerOutput
+    from mist_amd.tune_one_case import PreparedSearch
+    from tests.util import load_plan
+
+    monkeypatch.setattr(inter_tuning, "NATIVE_SEARCH", native)
+    cfg, _ = load_plan(2)
+    search = PreparedSearch(cfg)
+    hw = cfg.hardware
+    find = lambda results: inter_tuning.inter_stage_tune_batch(
+        search.L, hw.num_nodes * hw.num_gpus_per_node, search.meshes, search.Gs, results)
+    complete = search.tuner.run_prepared(search.plan, search.dev_plan)
+    want = find(complete)
+    assert len(want) > 2 and sum(solution is not None for _, solution in want) > 1
+    seen = _count_used_tables(monkeypatch, search.tuner, 7)
+    run = lambda: search.tuner.run_prepared(search.plan, search.dev_plan, fill_costs=False, sparse=True)
+    _leave_used_memory(7)
+    results = run()
+    assert seen[0] and results[0].batch.planes is not None
+    assert find(results) == want
+    assert find(results[1:]) == want[1:]  # (their own tables, cut out of the batch)
+    other = run()
+    assert find([results[0], other[1]]) == want[:2]
+    for t, (a, b) in enumerate(zip(run(), complete)):
+        assert np.array_equal(a.device.grad_accum.cpu().numpy(), search.Gs)
+        for v, suffix in enumerate(VARIANTS):
+            for kind in ("indices", "costs_stable", "costs_delta"):
+                assert np.array_equal(getattr(a, kind + suffix), getattr(b, kind + suffix)), (t, v, kind)
+    some = run()[1]
+    cells = [(0, 0, 1, 3, 3, 0), (1, 1, 0, 0, 1, 0), (0, 1, 0, 4, 2, 0)]
+    for a, b in zip(IntraStageTunerOutput.solutions_at([(some, 0, cell) for cell in cells]),
+                    IntraStageTunerOutput.solutions_at([(complete[1], 0, cell) for cell in cells])):
+        assert np.array_equal(a, b)
