@@ -106,8 +106,9 @@ _cached_ratios = lru_cache(maxsize=None)(alpha_ratios)  # (read only)
 
 def to_device(arrays: Sequence[np.ndarray], device: torch.device) -> List[torch.Tensor]:
     """The bytes of every array on the device, in one copy in order of the current stream (each starts at a
-    multiple of 256).  From pinned memory, since a copy of other memory returns when what was queued before it is
-    done, unless they are many: those go through another engine, which the next kernel waits for longer."""
+    multiple of 256): on another stream they are there behind an event that is recorded after the call.  From pinned
+    memory, since a copy of other memory returns when what was queued before it is done, unless they are many: those
+    go through another engine, which the next kernel waits for longer."""
     starts = [0]
     for a in arrays:
         starts.append(starts[-1] + (a.nbytes + 255) // 256 * 256)
@@ -792,7 +793,8 @@ class IntraStageTuner:
     def upload(self, plan) -> dict:
         """Descriptors and workgroup prefixes of every batch to the device; one workspace (row
         terms, stage summaries, partial minima) sized for the largest batch and shared by all.
-        The top-level entries are those of the first batch (all there is for most plans)."""
+        The top-level entries are those of the first batch (all there is for most plans).  The copies are in order
+        of the current stream, which the result refers to: ``launch`` on another one waits for it."""
         dev = self.device
         lib = _lib.load()
         # sizes of the reduce workspace: the minima of every (tile, slot) of a batch's groups, the
@@ -856,6 +858,7 @@ class IntraStageTuner:
             n_groups=0, groups=None, terms_prefix=None, reduce_prefix=None, scout_prefix=None,
             n_terms_blocks=0, n_reduce_blocks=0, n_scout_blocks=0,
             grad_accum=small[:n_rows], planes=small[n_rows:].view(n_rows, n_mesh),
+            uploaded_on=torch.cuda.current_stream(dev),
         )
         if batches:
             out.update({k: batches[0][k] for k in (
@@ -868,10 +871,20 @@ class IntraStageTuner:
         the output tables (``DeviceTables``) or the ``MistOutTables`` of their pointers.  With
         ``events`` (a list) row terms, reduction and finalize are launched through their own entry
         points and ``(name, start_event, end_event)`` triples recorded on that stream are appended."""
+        current = torch.cuda.current_stream(self.device)
+        if current != dev_plan["uploaded_on"]:
+            # The copies, and what the upload's stream did before with the memory of the workspaces.  (An event
+            # of every upload would cost the searches on one stream 12 us, 1.2 % of 7B on 1x8.)
+            if "uploaded" not in dev_plan:
+                dev_plan["uploaded"] = dev_plan["uploaded_on"].record_event()
+            current.wait_event(dev_plan["uploaded"])
+            for tensors in (dev_plan, *dev_plan["batches"], *dev_plan["workspaces"]):
+                for tensor in tensors.values():
+                    if isinstance(tensor, torch.Tensor):
+                        tensor.record_stream(current)
         if not dev_plan["batches"]:
             return
         lib = _lib.load()
-        current = torch.cuda.current_stream(self.device)
         streams = [current]
         if len(dev_plan["workspaces"]) > 1 and events is None:
             side = _side_stream(self.device)
