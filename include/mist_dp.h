@@ -51,7 +51,8 @@ typedef struct MistDpCosts {
   int64_t stage_min_g_stride;
   /* Optional (NULL = all): [g][planes_g_stride] int32, per mesh how many of the first planes of the p
    * axis hold something; the others (for 0 the mesh's rows of costs_post and costs_nopp too) count as
-   * +inf and are not read.  planes_g_stride: meshes of the tables. */
+   * +inf and are not read.  More than p_dim counts as p_dim, less than 0 as 0.  planes_g_stride: meshes of
+   * the tables. */
   const int32_t *planes;
   int64_t planes_g_stride;
 } MistDpCosts;

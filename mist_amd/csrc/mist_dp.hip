@@ -415,7 +415,8 @@ __global__ __launch_bounds__(256) void select_candidates_kernel(
       cells = of_mesh;
       if (tabs.planes != nullptr) {
         const int held = tabs.planes[g * meshes + q];
-        cells = v < 2 ? held * (n2 / meshes) : held > 0 ? of_mesh : 0;
+        // (n2: one plane of every mesh; never more than the p axis, as in cost_planes_kernel)
+        cells = v < 2 ? min(max(held, 0) * (n2 / meshes), of_mesh) : held > 0 ? of_mesh : 0;
       }
     }
     int64_t end = (cells + kBatch - 1) / kBatch;

@@ -35,13 +35,14 @@ def test_planes_equal_complete_tables(L, P1, meshes):
     Gn, Q = entries * len(Gs), len(meshes)
     planes = rng.integers(0, P1 + 1, size=(Gn, Q)).astype(np.int32)
     planes[0, 0], planes[-1, -1] = 0, P1
+    planes[2, -1], planes[3, 0] = P1 + 3, -2  # (as P1 and 0)
     missing = []
     for v in range(4):
         gone = np.broadcast_to(_unwritten(L, P1, v), whole.index[v].shape[:-1]).copy()
         if v < 2:
             gone |= (np.arange(P1) >= planes[:, :, None])[..., None, None]
         else:
-            gone[planes == 0] = True
+            gone[planes <= 0] = True
         missing.append(torch.from_numpy(gone).cuda()[..., None])
         whole.index[v][missing[v]] = -1
         whole.stable[v][missing[v]] = float("inf")
