@@ -4,8 +4,8 @@
 #include <algorithm>
 #include <cstdint>
 #include <cstring>
-#include <map>
 #include <mutex>
+#include <utility>
 
 #include "mist_common.h"
 #include "mist_search.h"
@@ -67,29 +67,60 @@ __global__ __launch_bounds__(256) void fetch_kernel(const FetchPieces pieces, co
   }
 }
 
-// Pinned chunks and their events, per device, for the life of the process: kFetchSlots MB.
+// Pinned chunks and their events, kFetchSlots MB.  A fetch has a ring to itself, so that those of several threads
+// and devices wait for nothing of each other.  The last kFetchKept rings are kept for the next fetches, for the life
+// of the process; a fetch that finds none of its device makes one.
+constexpr int kFetchKept = 8;
 struct FetchRing {
-  char *chunk[kFetchSlots] = {};
-  hipEvent_t filled[kFetchSlots] = {};
+  int device;
+  char *chunk[kFetchSlots];
+  hipEvent_t filled[kFetchSlots];
 };
-std::mutex g_fetch_lock;  // one fetch at a time: the chunks are shared
-std::map<int, FetchRing> g_fetch_rings;
+std::mutex g_fetch_lock;  // of the kept rings, not held while anything is waited for
+FetchRing g_fetch_rings[kFetchKept];
+int g_fetch_n_kept = 0, g_fetch_oldest = 0;
 
-int fetch_ring(FetchRing **out) {
-  int device = 0;
-  MIST_HIP_CHECK(hipGetDevice(&device));
-  FetchRing &ring = g_fetch_rings[device];
+void free_ring(const FetchRing &ring) {
   for (int i = 0; i < kFetchSlots; ++i) {
-    if (ring.chunk[i] == nullptr)
-      MIST_HIP_CHECK(hipHostMalloc(reinterpret_cast<void **>(&ring.chunk[i]), kFetchChunk, hipHostMallocCoherent));
-    if (ring.filled[i] == nullptr) MIST_HIP_CHECK(hipEventCreateWithFlags(&ring.filled[i], hipEventDisableTiming));
+    if (ring.chunk[i] != nullptr) (void)hipHostFree(ring.chunk[i]);
+    if (ring.filled[i] != nullptr) (void)hipEventDestroy(ring.filled[i]);
   }
-  *out = &ring;
+}
+
+int take_ring(FetchRing *ring) {
+  MIST_HIP_CHECK(hipGetDevice(&ring->device));
+  {
+    std::lock_guard<std::mutex> guard(g_fetch_lock);
+    for (int i = 0; i < g_fetch_n_kept; ++i)
+      if (g_fetch_rings[i].device == ring->device) {
+        *ring = g_fetch_rings[i];
+        g_fetch_rings[i] = g_fetch_rings[--g_fetch_n_kept];
+        return 0;
+      }
+  }
+  for (int i = 0; i < kFetchSlots; ++i) {
+    MIST_HIP_CHECK(hipHostMalloc(reinterpret_cast<void **>(&ring->chunk[i]), kFetchChunk, hipHostMallocCoherent));
+    MIST_HIP_CHECK(hipEventCreateWithFlags(&ring->filled[i], hipEventDisableTiming));
+  }
   return 0;
 }
 
+// (of a ring that nothing writes to any more)
+void give_back_ring(FetchRing ring) {
+  {
+    std::lock_guard<std::mutex> guard(g_fetch_lock);
+    if (g_fetch_n_kept < kFetchKept) {
+      g_fetch_rings[g_fetch_n_kept++] = ring;
+      return;
+    }
+    std::swap(ring, g_fetch_rings[g_fetch_oldest]);  // (which may be one of another device)
+    g_fetch_oldest = (g_fetch_oldest + 1) % kFetchKept;
+  }
+  free_ring(ring);
+}
+
 // Chunk by chunk: the next ones are written while one is copied out to the caller's arrays.
-int fetch_items(const MistFetchItem *items, int n_items, const MistGroupDesc *d_groups, FetchRing *ring, hipStream_t stream) {
+int fetch_items(const MistFetchItem *items, int n_items, const MistGroupDesc *d_groups, const FetchRing &ring, hipStream_t stream) {
   struct Part {  // of a chunk: where a piece goes
     char *to;
     int64_t at, bytes;
@@ -121,17 +152,17 @@ int fetch_items(const MistFetchItem *items, int n_items, const MistGroupDesc *d_
     }
     n_parts[slot] = pieces.n;
     if (pieces.n == 0) return 0;
-    hipLaunchKernelGGL(fetch_kernel, dim3(kFetchBlocks), dim3(256), 0, stream, pieces, d_groups, ring->chunk[slot]);
+    hipLaunchKernelGGL(fetch_kernel, dim3(kFetchBlocks), dim3(256), 0, stream, pieces, d_groups, ring.chunk[slot]);
     MIST_HIP_CHECK(hipGetLastError());
-    MIST_HIP_CHECK(hipEventRecord(ring->filled[slot], stream));
+    MIST_HIP_CHECK(hipEventRecord(ring.filled[slot], stream));
     return 0;
   };
   for (int slot = 0; slot < kFetchSlots; ++slot)
     if (int rc = fill(slot)) return rc;
   for (int slot = 0; n_parts[slot] > 0; slot = (slot + 1) % kFetchSlots) {
-    MIST_HIP_CHECK(hipEventSynchronize(ring->filled[slot]));
+    MIST_HIP_CHECK(hipEventSynchronize(ring.filled[slot]));
     for (int k = 0; k < n_parts[slot]; ++k)
-      std::memcpy(parts[slot][k].to, ring->chunk[slot] + parts[slot][k].at, (size_t)parts[slot][k].bytes);
+      std::memcpy(parts[slot][k].to, ring.chunk[slot] + parts[slot][k].at, (size_t)parts[slot][k].bytes);
     if (int rc = fill(slot)) return rc;
   }
   return 0;
@@ -151,12 +182,16 @@ int mist_fetch_tables(const MistFetchItem *items, int n_items, const MistGroupDe
     if (items[i].rows && (items[i].group >= n_groups || (items[i].group >= 0 && !d_groups)))
       return fail(MIST_E_INVALID, "item %d: group %d of %d", i, items[i].group, n_groups);
   }
-  std::lock_guard<std::mutex> guard(g_fetch_lock);
-  FetchRing *ring = nullptr;
-  if (int rc = fetch_ring(&ring)) return rc;
-  const int rc = fetch_items(items, n_items, d_groups, ring, (hipStream_t)stream);
-  if (rc != 0) (void)hipStreamSynchronize((hipStream_t)stream);  // (the chunks may still be written)
-  return rc;
+  FetchRing ring = {};
+  int rc = take_ring(&ring);
+  if (rc == 0) rc = fetch_items(items, n_items, d_groups, ring, (hipStream_t)stream);
+  if (rc != 0) {
+    (void)hipStreamSynchronize((hipStream_t)stream);  // (the chunks may still be written)
+    free_ring(ring);
+    return rc;
+  }
+  give_back_ring(ring);
+  return 0;
 }
 
 }  // extern "C"
