@@ -533,7 +533,7 @@ constexpr int kWindowThreads = 1024;
 constexpr int kWindowMost = 32768;      // values of a window that is walked on the device ...
 constexpr int kWindowDistinct = 16384;  // ... and different ones among them
 constexpr int kWindowHeld = kWindowMost / kWindowThreads, kWindowOwn = kWindowDistinct / kWindowThreads;
-constexpr int kWindowProbes = 256;      // slots of the hash table (at most half full) that a value tries
+constexpr int kWindowProbes = 256;      // slots of the hash table (about half full at most) that a value tries
 constexpr int kWindowBuckets = 4096;
 constexpr int kWindowBucketMost = 32;  // values in one bucket; where there are more the bitonic sort takes over
 // LDS: a hash table of at least twice the values (as many, of the most), then in its place the different values,
@@ -552,9 +552,11 @@ constexpr int kWindowOk = 0, kWindowNone = 1, kWindowOverflow = 2, kWindowNoStar
 // Most values of a window come several times (a stage costs the same for every number of pre-saved
 // micro-batches that fits): the different ones of `n` through a hash table in the LDS of `v` and behind it, then in
 // any order in `v`, by the whole workgroup.  Returns how many there are, -1 if they are more than `most` or one found
-// no slot within kWindowProbes.
+// no slot within kWindowProbes.  (Launches of a window of 32768 different values, which is given up: 550 us when they
+// were counted behind the last one, now 118; 24000 119, now 95.  16384, which are walked, 156 either way; 32768 of
+// 1000, 74.5 and 75.5.)
 __device__ __forceinline__ int window_distinct_values(const float *__restrict__ in, int n, int slots, int most, float *v) {
-  __shared__ int32_t found;
+  __shared__ int32_t found, inserted;
   uint32_t *table = reinterpret_cast<uint32_t *>(v);
   float held[kWindowHeld];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -563,7 +565,7 @@ __device__ __forceinline__ int window_distinct_values(const float *__restrict__ 
   while ((1 << bits) < slots && (1 << bits) < 2 * n) ++bits;
   const uint32_t mask = (1u << bits) - 1u;
   for (int i = tid; i <= (int)mask; i += kWindowThreads) table[i] = kEmpty;
-  if (tid == 0) found = 0;
+  if (tid == 0) found = inserted = 0;
 #pragma unroll
   for (int u = 0; u < kWindowHeld; ++u) {
     if (u * kWindowThreads >= n) break;
@@ -571,10 +573,20 @@ __device__ __forceinline__ int window_distinct_values(const float *__restrict__ 
   }
   __syncthreads();
   uint32_t first = 0;  // bit u: value u is the first of its kind
+  int counted = 0;
   bool lost = false;
 #pragma unroll
   for (int u = 0; u < kWindowHeld; ++u) {
     if (u * kWindowThreads >= n) break;
+    // given up when that is certain: the fuller the table, the longer the probing
+    if (u == kWindowOwn + 1 || u == kWindowOwn + 8) {
+      int own = __popc(first) - counted;
+      counted += own;
+      for (int step = 1; step < 64; step <<= 1) own += __shfl_xor(own, step);
+      if (lane == 0) atomicAdd(&inserted, own);
+    } else if (u > kWindowOwn + 1) {
+      if (__any(lost || __hip_atomic_load(&inserted, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) > most)) break;
+    }
     if (u * kWindowThreads + tid >= n) continue;
     const uint32_t key = __float_as_uint(held[u]);
     uint32_t at = key * 2654435761u >> (32 - bits);

@@ -16,6 +16,10 @@ def _values(rng, name, n):
         v = np.linspace(1.0, 2.0, n)
     elif name == "repeated":
         v = rng.choice(1.0 + rng.random(max(1, n // 20)), n)
+    elif name == "half":  # as many different ones as are walked and one more, most of them twice
+        v = np.tile(np.linspace(1.0, 2.0, DISTINCT + 1), 2)[:n]
+    elif name == "random":
+        v = 1.0 + rng.random(n)
     elif name == "equal":
         v = np.full(n, 1.5)
     elif name == "crowded":  # all but one in one bucket of equal width: the general sort
@@ -33,7 +37,7 @@ def _values(rng, name, n):
     ("even", 1), ("even", 2), ("even", 63), ("even", 1023), ("even", 1024), ("even", 1025), ("even", 4097),
     ("even", 16383), ("even", 16384), ("even", 16385), ("equal", 1), ("equal", 5000), ("crowded", 100), ("crowded", 129),
     ("crowded", 16384), ("wide", 3000), ("narrow", 40), ("skewed", 9000), ("repeated", 5), ("repeated", 5000),
-    ("repeated", 16385), ("repeated", 32768), ("repeated", 32769),
+    ("repeated", 16385), ("repeated", 32768), ("repeated", 32769), ("random", 20000), ("random", 32768), ("half", 32768),
 ])
 def test_windows_of_any_size_and_spread_equal_the_host_walk(name, n):
     import torch
@@ -82,3 +86,30 @@ def test_windows_of_any_size_and_spread_equal_the_host_walk(name, n):
     at = [lib.mist_dp_first_batch_index(i, k - below, CHUNK, LEAD) for i in range(min(CHUNK, k - below))]
     assert n_inst == len(at) and np.array_equal(inst_t.cpu().numpy()[first:first + n_inst], want[below:][at])
     assert inst_row.tolist() == [0] * n_inst + [-1] * (CHUNK - n_inst)
+
+
+def test_a_window_of_too_many_values_is_given_up_early(monkeypatch):
+    """It costs less than the largest one that is walked."""
+    import torch
+
+    from mist_amd import _lib
+
+    lib, least = _lib.load(), []
+    call = lib.mist_dp_windows_first_batch
+
+    def timed(*args):
+        times = []
+        for _ in range(10):
+            begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            begin.record()
+            status = call(*args)
+            end.record()
+            end.synchronize()
+            times.append(begin.elapsed_time(end))
+        least.append(min(times))
+        return status
+
+    monkeypatch.setattr(lib, "mist_dp_windows_first_batch", timed)
+    for n in (DISTINCT, CAPACITY):
+        test_windows_of_any_size_and_spread_equal_the_host_walk("random", n)
+    assert least[1] < least[0], least
