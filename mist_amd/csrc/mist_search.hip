@@ -1209,6 +1209,9 @@ __device__ __forceinline__ void stage_floor_of(const MistProblem &prob, const Mi
   else if (lane == MIST_T_MF_BASE) v = mf + 0.025 + 0.01;
   else if (lane == kStageMaxOut) v = max_out;
   if (lane < kStageFloorPitch) out[lane] = v;
+  // the wavefront's next stage writes `mine` and `keys` again
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
 }
 
 // Workgroup = two stages, every row on its own.
