@@ -984,15 +984,42 @@ __device__ __forceinline__ const float *dp_table(const MistDpCosts &tabs, int v,
 __device__ __forceinline__ int dp_j_last(const MistDpShape &shape, int k, int i) {
   return shape.ckpt_rule == MIST_DP_CKPT_TAIL ? shape.num_layers - i : i - k + 1;
 }
+// What dp_row_min reads of a g.  By value: a table that is picked through a reference to the kernel's arguments
+// puts those into scratch, 176 bytes a lane of dp_free_kernel and 136 of dp_step_kernel, which then read them there for
+// every row.  (1024 instances of 32 stages: 128 layers by dp_step_kernel 2990 us, now 2645; 110 by dp_free_kernel
+// 449 -> 372, 91 250 -> 217.)
+struct DpRows {
+  const float *inner, *pre, *post, *nopp;  // costs where only the last ckpt candidate counts, else running minima
+  const int32_t *planes;                   // per mesh (MistDpCosts.planes), NULL = all
+  int L, P1, ckpt_rule;
+};
+__device__ __forceinline__ DpRows dp_rows(const MistDpShape &shape, const MistDpCosts &tabs, int64_t g) {
+  DpRows r;
+  if (shape.ckpt_rule == MIST_DP_CKPT_ALL) {
+    r.inner = tabs.costs, r.pre = tabs.costs_pre, r.post = tabs.costs_post, r.nopp = tabs.costs_nopp;
+  } else {
+    r.inner = tabs.pmin, r.pre = tabs.pmin_pre, r.post = tabs.pmin_post, r.nopp = tabs.pmin_nopp;
+  }
+  r.inner += g * tabs.g_stride[0];
+  r.pre += g * tabs.g_stride[1];
+  r.post += g * tabs.g_stride[2];
+  r.nopp += g * tabs.g_stride[3];
+  r.planes = tabs.planes == nullptr ? nullptr : tabs.planes + g * tabs.planes_g_stride;
+  r.L = shape.num_layers;
+  r.P1 = shape.p_dim;
+  r.ckpt_rule = shape.ckpt_rule;
+  return r;
+}
 // The reference walks j = j_begin..j_end with "cost <= t_max and cost + prev < best".  "+ prev" is
 // monotone, so the smallest reachable sum is (smallest admissible cost) + prev, and the smallest
 // admissible cost is the row's running minimum if that is <= t_max (else nothing is admissible).
-__device__ __forceinline__ float dp_row_min(const MistDpShape &shape, const MistDpCosts &tabs, int64_t g,
-                                            const int64_t (&off)[4], int p, int k, int q, int i) {
-  if (tabs.planes != nullptr && p >= tabs.planes[g * tabs.planes_g_stride + q]) return INFINITY;
-  const DpRowRef r = dp_row_ref(shape, off, p, k, q, i);
-  return shape.ckpt_rule == MIST_DP_CKPT_ALL ? dp_table(tabs, r.v, false)[r.at + (i - k + 1)]
-                                             : dp_table(tabs, r.v, true)[r.at + dp_j_last(shape, k, i)];
+__device__ __forceinline__ float dp_row_min(const DpRows rows, int p, int k, int q, int i) {
+  if (rows.planes != nullptr && p >= rows.planes[q]) return INFINITY;
+  const int L = rows.L, l = i - k + 1;
+  const bool first = k == 0, last = i == L - 1;
+  const float *__restrict__ table = first ? (last ? rows.nopp : rows.pre) : last ? rows.post : rows.inner;
+  const int64_t row = first && last ? q : (last ? (int64_t)q : (int64_t)q * rows.P1 + p) * L + (l - 1);
+  return table[row * (L + 1) + (rows.ckpt_rule == MIST_DP_CKPT_TAIL ? L - i : l)];
 }
 
 // Re-laid row minima (mist_dp_stage_minima): per (g, p, mesh) a triangle over (k, i >= k), row k
@@ -1218,6 +1245,7 @@ __global__ __launch_bounds__(kDpThreads) void dp_step_kernel(
   if (g < 0) return;  // an empty slot of the batch (the whole workgroup: blockIdx.y is the instance)
   const int64_t off[4] = {g * tabs.g_stride[0], g * tabs.g_stride[1], g * tabs.g_stride[2],
                           g * tabs.g_stride[3]};
+  const DpRows rows_of_g = dp_rows(shape, tabs, g);
   const int k = e / W, d = e % W;
   const int p = s - 1;
   // Most states are unreachable.  Every step records, per instance and device column, the first
@@ -1241,7 +1269,7 @@ __global__ __launch_bounds__(kDpThreads) void dp_step_kernel(
     dp_scan_state<kBottleneck, kDpTeam>(
         w, shape, t_max, k, d, member, f_prev, range_prev,
         [&](int q, int i) {
-          return relaid != nullptr ? relaid[q * tri + i] : dp_row_min(shape, tabs, g, off, p, k, q, i);
+          return relaid != nullptr ? relaid[q * tri + i] : dp_row_min(rows_of_g, p, k, q, i);
         });
     if constexpr (kDpTeam == 1) {
       w.resolve(L);
@@ -2190,8 +2218,9 @@ __global__ __launch_bounds__(kDpFreeThreads) void dp_free_kernel(
   // row minima of the stages (k, i) behind which s - 1 layers are left (s = 1: none); the first kLoads values of a
   // thread are read a stage count ahead, from places that move by one plane of the tables with it
   const bool all_ckpt = shape.ckpt_rule == MIST_DP_CKPT_ALL;
-  const float *__restrict__ inner = dp_table(tabs, 0, !all_ckpt) + off[0], *__restrict__ front = dp_table(tabs, 1, !all_ckpt) + off[1];
-  const int held = tabs.planes == nullptr ? S : tabs.planes[g * tabs.planes_g_stride];
+  const DpRows rows_of_g = dp_rows(shape, tabs, g);
+  const float *__restrict__ inner = rows_of_g.inner, *__restrict__ front = rows_of_g.pre;
+  const int held = rows_of_g.planes == nullptr ? S : rows_of_g.planes[0];
   int end_of[kLoads], place[kLoads];
 #pragma unroll
   for (int u = 0; u < kLoads; ++u) {
@@ -2202,7 +2231,7 @@ __global__ __launch_bounds__(kDpFreeThreads) void dp_free_kernel(
   auto row_min = [&](int s, int x) {
     const int i = x % L, k = i - x / L;
     const bool wanted = x < L * L && k >= 0 && i <= L - s && (s > 1 || i == L - 1);
-    return wanted ? dp_row_min(shape, tabs, g, off, s - 1, k, 0, i) : INFINITY;
+    return wanted ? dp_row_min(rows_of_g, s - 1, k, 0, i) : INFINITY;
   };
   auto put = [&](int x, float value) {
     if (x < L * L) rows[x] = value <= t_max ? value : INFINITY;
@@ -2259,7 +2288,7 @@ __global__ __launch_bounds__(kDpFreeThreads) void dp_free_kernel(
       const int i = i0 + lane;
       float rmin = INFINITY, target = INFINITY;
       if (i <= L - s && f_prev[i + 1] < INFINITY) {
-        rmin = dp_row_min(shape, tabs, g, off, s - 1, k, 0, i);
+        rmin = dp_row_min(rows_of_g, s - 1, k, 0, i);
         target = kBottleneck ? fmaxf(rmin, f_prev[i + 1]) : rmin + f_prev[i + 1];
       }
       const unsigned long long hit = __ballot(rmin <= t_max && target == best);
@@ -2355,17 +2384,15 @@ __global__ __launch_bounds__(256) void stage_minima_kernel(const MistDpShape sha
   const int p = blockIdx.x / shape.num_mesh, q = blockIdx.x % shape.num_mesh;
   const int64_t g = blockIdx.y;
   float *__restrict__ mine = out + ((g * shape.max_stages + p) * shape.num_mesh + q) * tri;
-  if (tabs.planes != nullptr && p >= tabs.planes[g * tabs.planes_g_stride + q]) {
+  const DpRows rows_of_g = dp_rows(shape, tabs, g);
+  if (rows_of_g.planes != nullptr && p >= rows_of_g.planes[q]) {
     store_entries(mine, tri, INFINITY);
     return;
   }
-  const int64_t off[4] = {g * tabs.g_stride[0], g * tabs.g_stride[1], g * tabs.g_stride[2],
-                          g * tabs.g_stride[3]};
   // rows of l layers, entry k: at l - 1 rows of L - l' + 1 entries each
   if (in_lds) {
-    const DpRowRef inner = dp_row_ref(shape, off, p, 1, q, 1);  // one layer; the next rows follow it
     const bool all = shape.ckpt_rule == MIST_DP_CKPT_ALL;
-    const float *__restrict__ table = dp_table(tabs, 0, !all) + (L > 2 ? inner.at : 0);
+    const float *__restrict__ table = rows_of_g.inner + ((int64_t)q * shape.p_dim + p) * L * (L + 1);
     for (int x0 = threadIdx.x; x0 < tri; x0 += kMinimaLoads * 256) {
       float value[kMinimaLoads];
 #pragma unroll
@@ -2389,7 +2416,7 @@ __global__ __launch_bounds__(256) void stage_minima_kernel(const MistDpShape sha
     float value = INFINITY;
     if (k <= L - 1 - p)
       value = in_lds && k > 0 && k + di < L - 1 ? dp_lds[dp_triangle_row(L, di) + k]
-                                                : dp_row_min(shape, tabs, g, off, p, k, q, k + di);
+                                                : dp_row_min(rows_of_g, p, k, q, k + di);
     mine[x] = value;
   }
 }
