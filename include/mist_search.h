@@ -179,8 +179,8 @@ typedef struct MistGroupDesc {
  *   base, with_pre : [g][q][p_dim][L][L+1][S]
  *   with_post      : [g][q][L][L+1][S]
  *   no_pp          : [g][q][L+1][S]
- * The caller pre-fills costs with +inf and indices with -1; only the cells the reference
- * writes are written. */
+ * The caller pre-fills costs with +inf and indices with -1 (but see MistProblem.sparse_tables); only the
+ * cells the reference writes are written. */
 typedef struct MistOutTables {
   double *stable[4], *delta[4];
   int32_t *index[4];

@@ -2141,9 +2141,11 @@ __global__ __launch_bounds__(kDpHistoryThreads, 8) void dp_history_kernel(
 // each.  Here a workgroup runs an instance through all stage counts: per count the row minima
 // (consecutive end layers of a stage length are neighbours in the tables), read while the count
 // before is worked on, go to LDS, then eight lanes take a start layer.  Bound: LDS latency and two
-// barriers, 0.8 us per stage count at 37 layers.  (Read where they are needed, each place from its
+// barriers, 0.7 us per stage count at 37 layers.  (Read where they are needed, each place from its
 // row and variant, and a wavefront a start layer, five in turn with six exchanges each: 2.5 us; the
-// four launches of 13B on 4x8 100, 219, 89 and 76 us, now 35, 155, 31 and 28.)  Six families of that plan: 250 launches, 3.3 ms from the first to the last -> 18, 0.75.
+// four launches of 13B on 4x8 100, 219, 89 and 76 us; then 34, 153, 30 and 27 with the tables' addresses
+// in scratch, now 25, 70, 24 and 23.)  Six families of that plan: 250 launches, 3.3 ms from the first to
+// the last -> 18, 0.75.
 // The families of a search wait for nothing of each other: up to kDpFreeFamilies go through one
 // launch, workgroup = (instance, family), the ones given last (more stage counts as a rule) first:
 // 24 launches, 0.89 ms of 13B on 4x8 -> 4, 0.50.

@@ -970,10 +970,14 @@ constexpr int kFloorPitch = kStageRows + 1;
 constexpr int kFloorThreads = 256, kFloorWaves = kFloorThreads / 64;
 constexpr int kFloorRun = 32;  // terms blocks (two stages each) of a workgroup of stage_floor_runs_kernel
 // Terms blocks from which on the runs are taken.  Their shared parts save a third of the float64 work (1200 vector
-// instructions a stage, 810), but a workgroup waits for more in turn and leaves less room beside the seeds.  From the
-// gathered rows to the filter, every row on its own -> runs: 22B on 16x8 (528000 blocks) 5.20 -> 4.64 ms (alone 3.0 ->
-// 2.6); 70B on 32x8 (45000) and 13B on 8x8 (30000) the same, the seeds are longer; 7B on 4x8 (25200) 447 -> 452 us,
-// uniform-pp of 7B (18900) 230 -> 271, 30 samples of 7B 443 -> 504.
+// instructions a stage, 810), but a workgroup waits for more in turn and, with 154 registers and three wavefronts a
+// SIMD (every row on its own: 120 and four), leaves less room beside the seeds.  Calls of 7B on 4x8, 2x8, LLaMA-13B,
+// GPT-22B and LLaMA-70B with finer and finer ratios, time of every row on its own over that of the runs:
+//   blocks      7100 - 49800  65300 - 108500  135000 - 170300  224000 - 267000  348000 - 627000
+//   inter-stage   1.00 - 1.01   1.00 - 1.02     1.01 - 1.04      1.01 - 1.01      1.01 - 1.07
+//   uniform-pp    0.96 - 0.98   0.98 - 0.98     0.99 - 1.00      1.01 - 1.01         1.02
+//   whole tables  0.99 - 1.01   1.00 - 1.01                      1.01 - 1.01
+// (GPT-22B on 16x8, 528000 blocks: the launch alone 3.0 -> 2.6 ms, from the gathered rows to the filter 5.20 -> 4.64.)
 constexpr int kFloorRunBlocks = 1 << 17;
 // Parts of the lane's row, `lane` behind the first row of the wavefront: from that one's (wave-uniform), block by
 // block (four divisions of the lane's own otherwise, 90 instructions).
@@ -4107,8 +4111,6 @@ double mist_incumbent_slack(void) { return kIncumbentSlack; }
 static bool has_key_terms(const MistProblem *problem, int n_groups, const double *d_key_terms) {
   return d_key_terms != nullptr && problem->max_group_keys > 0 && n_groups <= 65535;
 }
-// key_terms_kernel over every group when the caller gave a key-term workspace and the bound the
-// grid needs; *launched tells whether the row-term kernel can read key terms.
 // (for tests MIST_STAGE_FLOOR_RUNS = 0 | 1 decides)
 static bool stage_floor_runs(int n_blocks) {
   const char *decided = getenv("MIST_STAGE_FLOOR_RUNS");
@@ -4125,6 +4127,8 @@ static void launch_stage_floors(const MistProblem *problem, const MistGroupDesc 
                        dim3(kFloorThreads), 0, stream, *problem, d_groups, n_groups, d_block_prefix, n_blocks, d_stage_floor,
                        d_key_terms);
 }
+// key_terms_kernel over every group when the caller gave a key-term workspace and the bound the
+// grid needs; *launched tells whether the row-term kernel can read key terms.
 static int launch_key_terms(const MistProblem *problem, const MistGroupDesc *d_groups, int n_groups,
                             double *d_key_terms, hipStream_t stream, bool *launched) {
   *launched = has_key_terms(problem, n_groups, d_key_terms);
