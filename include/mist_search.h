@@ -247,7 +247,7 @@ int mist_row_terms(const MistProblem *problem, const MistGroupDesc *d_groups, in
  * rows of the group's scout pairs (MistGroupDesc.scout_stride; the search's winners sit almost
  * exclusively on rows without weight / gradient offloading; n_scout_blocks 0 = empty minima),
  * *filter* and *open* rule out 64-row stages by their summaries, *reduce* evaluates the rows of
- * what is left, *resolve* finds the rows of the minima that were lowered meanwhile.
+ * what is left and notes those that reach a minimum, *resolve* takes the rows from these notes.
  * d_block_prefix[n_groups+1]: first workgroup of each group in the filter launch; a group owns
  * n_lc_tiles*n_p_tiles*n_chunks workgroups ordered (chunk, lc_tile, p_tile), p_tile fastest.
  * n_scout_blocks > 0 asks for the seeds; d_scout_prefix[n_groups+1] (n_lc_tiles * n_p_tiles *

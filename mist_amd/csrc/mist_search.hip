@@ -1407,29 +1407,37 @@ __device__ __forceinline__ void take_min(double &best, int32_t &best_row, bool f
 //   open     runs of items per wavefront: the summary with the minima of the slots the stage can reach;
 //            which pairs stay open goes along;
 //   reduce   what is left, shared out by pairs: linear bounds of 64 rows against a pair's minima, then
-//            the reference's arithmetic for the candidates of several pairs.  A row whose cost
-//            IS the minimum at its own slot (count - 1) offers its row number there (the lowest
-//            one stays, which is the reference's first-index-wins scan, pareto.py:134-142, in any
-//            processing order); a smaller cost lowers the minimum and marks the pair, whose row
-//            numbers no longer count.  The slots below take part in finalize, which takes each
+//            the reference's arithmetic for the candidates of several pairs.  A smaller cost than the
+//            minimum at the row's own slot (count - 1) lowers it, and every row that was not above it
+//            is noted with its cost in a log.  The slots below take part in finalize, which takes each
 //            p's winner from the slots at and above it;
-//   resolve  the marked pairs of the items in which some row reached its minimum, again, with the
-//            final minima (the seeds are final for most cells: 19 changes for the 7B plan).
+//   resolve  of the rows in the log whose cost is the final minimum the lowest number stays, which is the
+//            reference's first-index-wins scan (pareto.py:134-142) in any processing order.  (A log that
+//            ran full is left alone: the opened items go through the reduce launch's code once more.)
 // What this replaces kept 34 (cost, row) minima per lane in registers (253 of them, two
 // wavefronts per SIMD), one sample and 16 p values per pass over the rows, visited every stage
 // summary with every tile and p tile, and committed rows one by one per lane: 7B on 4x8, one
 // sample: 1.35 ms (0.42 of it seeds); now seeds 0.26 beside key terms and summaries, filter 0.04, open 0.04,
-// reduce 0.19, resolve 0.03.  30 samples of the 7B plan's tables for one tensor-parallel size: 24 ms;
-// now 3.7 (reduce 2.1, resolve 0.57, open 0.42, seeds 0.33, filter 0.17).
+// reduce 0.19, resolve 0.01.  30 samples of the 7B plan's tables for one tensor-parallel size: 24 ms;
+// now 3.2 (reduce 2.1, open 0.42, seeds 0.33, filter 0.17, resolve 0.08).
 // ------------------------------------------------------------------------------------------
 constexpr int kSuperStages = 8;    // stages per second-level summary
 constexpr int kGatherFloor = 5;    // linear bounds of 64 gathered rows
 constexpr int kQueueShards = 64;   // counters of the item queue: one would serve an append in ~8 ns
 constexpr int kCounterPitch = 32;  // uint32 between counters: a cache line each
-constexpr int kCounters = 3 * kQueueShards + kNumXcd;
+// Entries of the log that a reduce wavefront takes at a time, and the most entries of a log: 16 bytes each; 7e6
+// with 30 samples of one tensor-parallel size of the 7B plan, 5e6 of 70B on 32x8, 11e6 of searches whose bound
+// prunes little, 0.1 to 2 per entry of the minima elsewhere.
+constexpr int kLogChunk = 256;
+constexpr int64_t kLogEntries = 24 << 20;
+constexpr int kLogPerCell = 4;
+constexpr int kLogTaken = 3 * kQueueShards + kNumXcd;  // counters: chunks taken, whether there were too few
+constexpr int kLogFull = kLogTaken + 1;
+constexpr int kCounters = kLogFull + 1;
 constexpr int kSeedThreads = 256;
 constexpr int kReduceThreads = 256;
 constexpr int kReduceBlocks = 2048;          // a multiple of kNumXcd
+constexpr int kAgainBlocks = 768;            // three per CU: as a rule they return at once
 constexpr int kStageRowsBlocks = 1024;       // four per CU, two stages at a time each
 constexpr int kSuperBlocks = 64;             // workgroups per group of the second-level summaries
 constexpr int kSeedLdsBytes = 40 * 1024;     // LDS aimed at per seed workgroup: four per CU
@@ -1442,7 +1450,6 @@ constexpr int kCandidateDoubles = kCandidates * 2 / 8;
 // values of p.
 constexpr int kMostBufferedSlots = kSeedLdsMost / (8 * (kReduceThreads / 64)) - kCandidateDoubles;
 static_assert(kQueueShards == 64, "a lane per shard");
-constexpr uint32_t kUnresolved = 0x80000000u;
 // Room below r x and below the terms the composite objectives add (their roundings: a few 1e-16) ...
 constexpr double kSlack = 1e-9;
 // ... and below d / G, which the base objective rounds to float32 (one part in 2^24).  Relative to
@@ -1468,25 +1475,33 @@ struct Item {
   }
 };
 
+// A row that was not above the minimum of its slot when it was looked at.
+struct Hit {
+  double cost;
+  uint32_t cell;  // of `best`
+  uint32_t row;
+};
+static_assert(sizeof(Hit) == 16, "two doubles of the workspace");
+
 // (by value in the kernel arguments)
 struct ReduceTables {
   double *best;  // [pair][slot][sample] (slots_of(num_p) slots): the smallest cost
-  // its lowest row, ~0 = none; kUnresolved + row from the reduce launch, row from the resolve launch
-  // (smaller than any of the former)
-  uint32_t *row;
-  uint32_t *changed;         // [pair's first cell / 4]: samples whose minima the reduce launch lowered
+  uint32_t *row;  // its lowest row, ~0 = none (from the resolve launch)
+  Hit *log;             // [log_chunks][kLogChunk]
+  uint32_t *log_count;  // [log_chunks]: entries of each
   double *super_floor;       // [supers][kStageFloorPitch]
   double *gather_floor;      // [stage][kGatherFloor]: what the seed launch asks of 64 gathered rows (one sample)
-  // [kQueueShards][capacity]: Item, what the filter and then what the open launch left; pairs of the
-  // latter, first the open ones, then those in which a row reached its minimum
-  unsigned long long *item, *opened, *hit;
+  // [kQueueShards][capacity]: Item, what the filter and then what the open launch left; open pairs of the
+  // latter
+  unsigned long long *item, *opened, *open_pairs;
   // [kQueueShards][capacity]: group << 32 | stage of the stages opened, each once; stage_flag (one
   // per stage summary) tells whether one is listed.  Null: the rows of all stages are there.
   unsigned long long *listed;
   uint32_t *stage_flag;
-  // at kCounterPitch: [kQueueShards] items, [kQueueShards] opened, [kQueueShards] listed, [kNumXcd] drawn
+  // at kCounterPitch: [kQueueShards] items, [kQueueShards] opened, [kQueueShards] listed, [kNumXcd] drawn,
+  // kLogTaken, kLogFull
   uint32_t *counter;
-  uint32_t capacity;
+  uint32_t capacity, log_chunks;
   int n_samples;
 };
 
@@ -2114,7 +2129,6 @@ __global__ __launch_bounds__(kSeedThreads, 3) void seed_kernel(
     tabs.best[cell0 + e] = lds_best[e];
     tabs.row[cell0 + e] = ~0u;
   }
-  if ((int)threadIdx.x < pair_split) tabs.changed[(cell0 + threadIdx.x * n_slots) / 4] = 0;
 }
 
 // No seeds (none asked for, or the minima of one pair exceed the LDS): the tables of the launch, empty.
@@ -2125,7 +2139,6 @@ __global__ __launch_bounds__(256) void empty_minima_kernel(ReduceTables tabs, in
     tabs.best[i] = INFINITY;
     tabs.row[i] = ~0u;
   }
-  for (int64_t i = first; i < cells / 4; i += step) tabs.changed[i] = 0;
 }
 
 // Several samples.  What the objectives of a row are made of, r X + Y per variant, and its counts,
@@ -2255,7 +2268,6 @@ __global__ __launch_bounds__(64 * kSeedSampleWaves) void seed_samples_kernel(
     }
     if (wave == 0) put(2 * P + v, mine[(2 * P + v) * S + sample]);
   }
-  if (threadIdx.x == 0 && first_sample == 0) tabs.changed[cell0 / 4] = 0;
 }
 
 // ---- summaries of kSuperStages stages ----
@@ -2500,32 +2512,6 @@ __device__ __forceinline__ FlatQueue flat_queue(const ReduceTables &tabs, int qu
   return q;
 }
 
-// The same in chunks of up to 64 items of one shard.
-struct ChunkQueue {
-  uint32_t end, items;  // of this lane's shard: chunks up to it, items in it
-  uint32_t chunks;
-  // first item of chunk u, number of its items
-  __device__ __forceinline__ int64_t at(uint32_t u, uint32_t capacity, int *n) const {
-    const int shard = __popcll((unsigned long long)__ballot(end <= u));
-    const uint32_t before = shard > 0 ? (uint32_t)from_lane((int)end, shard - 1) : 0u;
-    const uint32_t first = (u - before) * 64u;
-    *n = (int)min(64u, (uint32_t)from_lane((int)items, shard) - first);
-    return (int64_t)shard * capacity + first;
-  }
-};
-__device__ __forceinline__ ChunkQueue chunk_queue(const ReduceTables &tabs, int queue) {
-  const int lane = threadIdx.x & 63;
-  ChunkQueue q;
-  q.items = min(tabs.counter[(queue * kQueueShards + lane) * kCounterPitch], tabs.capacity);
-  q.end = (q.items + 63u) / 64u;
-  for (int step = 1; step < 64; step <<= 1) {
-    const uint32_t o = (uint32_t)__shfl_up((int)q.end, step);
-    if (lane >= step) q.end += o;
-  }
-  q.chunks = (uint32_t)from_lane((int)q.end, 63);
-  return q;
-}
-
 // A lane's pair of a tile.
 struct TileLane {
   PairIndex pc;
@@ -2601,7 +2587,7 @@ __global__ __launch_bounds__(kReduceThreads) void open_kernel(const MistProblem 
     base = (uint32_t)from_lane((int)base, 0);
     if (mine) {
       tabs.opened[shard0 + base + lane] = kept_word;
-      tabs.hit[shard0 + base + lane] = kept_open;
+      tabs.open_pairs[shard0 + base + lane] = kept_open;
     }
     n_kept = 0;
     if (tabs.listed == nullptr) return;
@@ -2732,8 +2718,50 @@ __global__ __launch_bounds__(kTermsBlock) void stage_rows_kernel(
 }
 
 // ---- reduce / resolve ----
-// One item with the pairs in `pairs`, one sample.  Returns the pairs in which some row reached its
-// minimum (kResolve: unused).
+// A wavefront's place in the log: it takes a chunk at a time.
+struct HitLog {
+  uint32_t chunk = ~0u, used = kLogChunk;  // (wave-uniform; ~0: none)
+  bool full = false;
+  __device__ __forceinline__ void close(const ReduceTables &tabs) const {
+    if (chunk != ~0u && (threadIdx.x & 63) == 0) tabs.log_count[chunk] = used;
+  }
+  // All lanes of the wavefront: what each notes of the four variants (`hit`: a bit per variant).
+  __device__ __forceinline__ void put(const ReduceTables &tabs, uint32_t hit, const double (&cost)[4], const uint32_t (&cell)[4],
+                                      uint32_t row) {
+    uint64_t mask[4];
+    uint32_t n = 0;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      mask[v] = __ballot((hit >> v & 1u) != 0);
+      n += __popcll(mask[v]);
+    }
+    if (n == 0 || full) return;
+    const int lane = threadIdx.x & 63;
+    static_assert(kLogChunk >= 4 * 64, "what a wavefront notes at once");
+    if (used + n > (uint32_t)kLogChunk) {
+      close(tabs);
+      uint32_t its = 0;
+      if (lane == 0) its = atomicAdd(tabs.counter + kLogTaken * kCounterPitch, 1u);
+      chunk = (uint32_t)from_lane((int)its, 0);
+      used = 0;
+      if (chunk >= tabs.log_chunks) {
+        if (lane == 0) tabs.counter[kLogFull * kCounterPitch] = 1;
+        chunk = ~0u;
+        full = true;
+        return;
+      }
+    }
+    Hit *log = tabs.log + (int64_t)chunk * kLogChunk + used;
+    used += n;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      if (hit >> v & 1u) log[__popcll(mask[v] & ((1ull << lane) - 1ull))] = Hit{cost[v], cell[v], row};
+      log += __popcll(mask[v]);
+    }
+  }
+};
+
+// One item with the pairs in `pairs`, one sample.  kResolve: after a log that ran full, with final minima.
 //   lane = pair   the slots the stage's pseudo row can reach, and with their minima a threshold;
 //   lane = row    the rows below it, by their linear bounds: two FMAs and a compare per pair;
 //   lane = row    of the pairs that have any: a bound of each row's count and the minimum there (one
@@ -2746,10 +2774,10 @@ __global__ __launch_bounds__(kTermsBlock) void stage_rows_kernel(
 // 7B on 4x8 0.28 -> 0.19.  Four wavefronts per SIMD, with 128 registers, are no faster than three.)
 // kInLds false: there are too many minima for the buffer (see kMostBufferedSlots), rows look them up in memory.
 template <bool kResolve, bool kInLds>
-__device__ __forceinline__ uint64_t reduce_item(const MistProblem &prob, const MistGroupDesc *__restrict__ g, int gi,
-                                                int tile_rel, int stage, const double *__restrict__ row_terms,
-                                                const double *__restrict__ stage_floor, double ratio,
-                                                const ReduceTables &tabs, uint64_t pairs, double *lds) {
+__device__ __forceinline__ void reduce_item(const MistProblem &prob, const MistGroupDesc *__restrict__ g, int gi,
+                                            int tile_rel, int stage, const double *__restrict__ row_terms,
+                                            const double *__restrict__ stage_floor, double ratio,
+                                            const ReduceTables &tabs, uint64_t pairs, double *lds, HitLog &log) {
   const int L = prob.num_layers, lane = threadIdx.x & 63;
   const int P = g->num_p, n_slots = slots_of(P);
   const GroupModel m = group_model(prob, g);
@@ -2780,7 +2808,7 @@ __device__ __forceinline__ uint64_t reduce_item(const MistProblem &prob, const M
     off_pre = off.pre;
     todo = pairs & __ballot(bound <= thr);
   }
-  if (todo == 0) return 0;
+  if (todo == 0) return;
 
   // ---- lane = row ----
   const int64_t row0 = (int64_t)stage * kStageRows;
@@ -2804,7 +2832,7 @@ __device__ __forceinline__ uint64_t reduce_item(const MistProblem &prob, const M
     const uint64_t pass = live & __ballot(bound.at(p.n_ck, p.n_nock, p.all_ck, p.none) <= from_lane(thr, pl));
     left |= pass != 0 ? 1ull << pl : 0ull;
   }
-  if (left == 0) return 0;
+  if (left == 0) return;
   LinearMemory mem;
   {
     RowRegs t;
@@ -2830,7 +2858,6 @@ __device__ __forceinline__ uint64_t reduce_item(const MistProblem &prob, const M
   };
 
   // ---- lane = (row, pair): the first `n` of the queue ----
-  uint64_t hits = 0;
   auto settle_candidates = [&](int n) {
     const uint32_t entry = queue[min(lane, n - 1)];
     const int pl = (int)(entry >> 6), its_row = (int)(entry & 63u);
@@ -2857,31 +2884,26 @@ __device__ __forceinline__ uint64_t reduce_item(const MistProblem &prob, const M
     const int own_b = max(cnt.b - 1, 0), own_p = P + max(cnt.p - 1, 0);
     const double *slots = tabs.best + cell;
     const double now_b = slots[own_b], now_p = slots[own_p], now_post = slots[2 * P], now_pp = slots[2 * P + 1];
-    const uint32_t number = (kResolve ? 0u : kUnresolved) + (uint32_t)row_of_position(g, row0 + its_row);
-    bool hit = false, lowered = false;
+    const uint64_t reached = __ballot(o.base <= now_b || o.pre <= now_p || o.post <= now_post || o.pp <= now_pp);
+    if (reached == 0) return;
+    const uint32_t number = (uint32_t)row_of_position(g, row0 + its_row);
     // A lowered slot may lie below the slots under it; a row above it is above the winner of its own
     // slot too, which finalize takes from the slots at and above.
-    auto offer = [&](bool ok, double cost, int own, double now) {
-      if (!(ok && cost <= now && cost <= cutoff && cost < INFINITY)) return;
-      hit = true;
-      if (cost == now) {
-        atomicMin(tabs.row + cell + own, number);
-      } else if (!kResolve) {
-        lower_minimum(tabs.best + cell + own, cost);
-        lowered = true;
-      }
+    const double cost[4] = {o.base, o.pre, o.post, o.pp};
+    const uint32_t cells[4] = {(uint32_t)cell + own_b, (uint32_t)cell + own_p, (uint32_t)cell + 2 * P, (uint32_t)cell + 2 * P + 1};
+    uint32_t hit = 0;
+    auto offer = [&](bool ok, int variant, int own, double now) {
+      const double its = cost[variant];
+      if (!(ok && its <= now && its <= cutoff && its < INFINITY)) return;
+      hit |= 1u << variant;
+      if (kResolve) atomicMin(tabs.row + cell + own, number);
+      else if (its < now) lower_minimum(tabs.best + cell + own, its);
     };
-    offer(cnt.b > 0, o.base, own_b, now_b);
-    offer(cnt.p > 0, o.pre, own_p, now_p);
-    offer(do_post && ok_post, o.post, 2 * P, now_post);
-    offer(do_pp && ok_pp, o.pp, 2 * P + 1, now_pp);
-    if (kResolve) return;
-    if (lowered) tabs.changed[cell / 4] = 1u;
-    for (uint64_t some = __ballot(hit); some != 0;) {  // a few pairs of the 64 candidates
-      const int first = from_lane(pl, __ffsll((unsigned long long)some) - 1);
-      hits |= 1ull << first;
-      some &= ~(uint64_t)__ballot(pl == first);
-    }
+    offer(cnt.b > 0, 0, own_b, now_b);
+    offer(cnt.p > 0, 1, own_p, now_p);
+    offer(do_post && ok_post, 2, 2 * P, now_post);
+    offer(do_pp && ok_pp, 3, 2 * P + 1, now_pp);
+    if (!kResolve) log.put(tabs, hit, cost, cells, number);
   };
 
   const double cap_and_room = m.cap * (1.0 + 1e-12);
@@ -2917,7 +2939,6 @@ __device__ __forceinline__ uint64_t reduce_item(const MistProblem &prob, const M
     __builtin_amdgcn_wave_barrier();
     queue[lane] = moved;
   }
-  return hits;
 }
 
 // The same for several samples.  The linear bounds of a row are those of its stable and of its delta part,
@@ -2949,7 +2970,6 @@ struct SampleQueue {
   double2 post_terms[64];
   uint32_t entry[kCandidates];         // pair | row << 6 | first sample << 12 | samples << 17
   uint32_t useful[64];                 // the same of the candidates that have a count
-  uint32_t changed[64];                // their pairs' samples
 };
 // `n` items of `width` lanes each, side by side.
 struct LaneGroups {
@@ -2966,11 +2986,12 @@ struct LaneGroups {
   }
 };
 template <bool kResolve>
-__device__ __forceinline__ uint64_t reduce_item_samples(const MistProblem &prob, const MistGroupDesc *__restrict__ g,
-                                                        int gi, int tile_rel, int stage,
-                                                        const double *__restrict__ row_terms,
-                                                        const double *__restrict__ stage_floor, const RatioList &ratios,
-                                                        const ReduceTables &tabs, uint64_t pairs, SampleQueue *queue) {
+__device__ __forceinline__ void reduce_item_samples(const MistProblem &prob, const MistGroupDesc *__restrict__ g,
+                                                    int gi, int tile_rel, int stage,
+                                                    const double *__restrict__ row_terms,
+                                                    const double *__restrict__ stage_floor, const RatioList &ratios,
+                                                    const ReduceTables &tabs, uint64_t pairs, SampleQueue *queue,
+                                                    HitLog &log) {
   SampleRows *const exact = &queue->exact;
   const int L = prob.num_layers, lane = threadIdx.x & 63, S = tabs.n_samples;
   const int my_sample = min(lane & 31, S - 1);
@@ -2994,7 +3015,7 @@ __device__ __forceinline__ uint64_t reduce_item_samples(const MistProblem &prob,
     floor_d = reach.d;
     pairs &= __ballot(tl.active && parts != 0);
   }
-  if (pairs == 0) return 0;
+  if (pairs == 0) return;
 
   // ---- lane = row ----
   const int64_t row0 = (int64_t)stage * kStageRows;
@@ -3019,7 +3040,6 @@ __device__ __forceinline__ uint64_t reduce_item_samples(const MistProblem &prob,
     queue->post_terms[lane] = post_terms;
   }
   const double cap_and_room = m.cap * (1.0 + 1e-12);
-  uint64_t hits = 0;  // of the lane's items
 
   // ---- lane = (row, pair): the first `n` of the queue; then lane = (row, sample) ----
   auto settle_candidates = [&](int n) {
@@ -3047,9 +3067,8 @@ __device__ __forceinline__ uint64_t reduce_item_samples(const MistProblem &prob,
       const int at = __popcll(some & ((1ull << lane) - 1ull));
       if (useful) {
         put_sample_row(exact, at, t, x, d, k.no_ck, m, cnt.b, cnt.p, ok_post, ok_pp, true);
-        exact->number[at] = (kResolve ? 0u : kUnresolved) + (uint32_t)row_of_position(g, row0 + its_row);
+        exact->number[at] = (uint32_t)row_of_position(g, row0 + its_row);
         queue->useful[at] = entry;
-        if (kResolve) queue->changed[at] = tabs.changed[(tile_cell + pl * n_slots) / 4];
       }
       n = __popcll(some);
     }
@@ -3075,37 +3094,31 @@ __device__ __forceinline__ uint64_t reduce_item_samples(const MistProblem &prob,
     for (int r0 = 0; r0 < n; r0 += slot.n) {
       const int r = min(r0 + slot.item, n - 1), its_pair = (int)(place & 63u), first = (int)(place >> 12 & 31u);
       const int sample = min(first + slot.offset, S - 1);
-      const bool on = slot.item < slot.n && r0 + slot.item < n && first + slot.offset < S &&
-                      (!kResolve || (queue->changed[r] >> sample & 1u) != 0);
+      const bool on = slot.item < slot.n && r0 + slot.item < n && first + slot.offset < S;
       const double its_ratio = __shfl(ratio, sample);
       const uint32_t cn = counts;
       const double nb_now = now_b, np_now = now_p, post_now = now_post, pp_now = now_pp;
       if (r0 + slot.n < n) look(min(r0 + slot.n + slot.item, n - 1));
-      bool hit = false, lowered = false;
+      const uint32_t number = exact->number[r];
+      const int nb = (int)(cn & 0x7fff), npre = (int)(cn >> 15 & 0x7fff);
+      const int64_t to = (tile_cell + its_pair * n_slots) * S + sample;
+      double cost[4];
+      uint32_t cells[4], hit = 0;
       auto offer = [&](bool ok, int variant, int own, double now) {
         const double2 xy = exact->xy[variant][r];
-        const double cost = its_ratio * xy.x + xy.y;
-        if (!(on && ok && cost <= now && cost < INFINITY)) return;
-        hit = true;
-        const int64_t to = (tile_cell + its_pair * n_slots + own) * S + sample;
-        if (cost == now) {
-          atomicMin(tabs.row + to, exact->number[r]);
-        } else if (!kResolve) {
-          lower_minimum(tabs.best + to, cost);
-          lowered = true;
-        }
+        const double its = its_ratio * xy.x + xy.y;
+        cost[variant] = its;
+        cells[variant] = (uint32_t)to + (uint32_t)(own * S);
+        if (!(on && ok && its <= now && its < INFINITY)) return;
+        hit |= 1u << variant;
+        if (kResolve) atomicMin(tabs.row + to + own * S, number);
+        else if (its < now) lower_minimum(tabs.best + to + own * S, its);
       };
-      const int nb = (int)(cn & 0x7fff), npre = (int)(cn >> 15 & 0x7fff);
       offer(nb > 0, 0, nb - 1, nb_now);
       offer(npre > 0, 1, P + npre - 1, np_now);
       offer((cn >> 30 & 1u) != 0, 2, 2 * P, post_now);
       offer((cn >> 31) != 0, 3, 2 * P + 1, pp_now);
-      if (kResolve) continue;
-      const uint64_t some = __ballot(hit), low = __ballot(lowered);
-      if (some == 0 || slot.offset != 0 || slot.item >= slot.n) continue;
-      const uint32_t samples = slot.bits(low, slot.item);
-      if (samples != 0) atomicOr(tabs.changed + (tile_cell + its_pair * n_slots) / 4, samples << first);
-      if (slot.bits(some, slot.item) != 0) hits |= 1ull << its_pair;
+      if (!kResolve) log.put(tabs, hit, cost, cells, number);
     }
   };
 
@@ -3204,9 +3217,7 @@ __device__ __forceinline__ uint64_t reduce_item_samples(const MistProblem &prob,
       thr = its.at(post_layer);
       thr_post = its.post;
       const double low = m.bound(ratio, __shfl(floor_x, pl), __shfl(floor_d, pl));
-      bool on = (lane & 31) < S;
-      if (kResolve) on = on && (tabs.changed[(tile_cell + pl * n_slots) / 4] >> (lane & 31) & 1u) != 0;
-      may = second & __ballot(on && low <= thr);
+      may = second & __ballot((lane & 31) < S && low <= thr);
     }
     if (waiting < 64 && (waiting == 0 || rest != 0 || may != 0)) continue;
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -3217,9 +3228,6 @@ __device__ __forceinline__ uint64_t reduce_item_samples(const MistProblem &prob,
     __builtin_amdgcn_wave_barrier();
     queue->entry[lane] = moved;
   }
-  if (kResolve) return 0;
-  for (int step = 1; step < 64; step *= 2) hits |= __shfl_xor((unsigned long long)hits, step);
-  return from_lane(hits, 0);
 }
 
 // Every 2^k-th pair from the first on.
@@ -3241,48 +3249,34 @@ __global__ __launch_bounds__(kReduceThreads, 3) void reduce_kernel(
   constexpr int kWaves = kReduceThreads / 64;
   const int local_wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
   const uint32_t n_waves = gridDim.x * kWaves;
-  auto work = [&](int64_t at, uint64_t word, uint64_t pairs) {
+  if (kResolve && tabs.counter[kLogFull * kCounterPitch] == 0) return;
+  HitLog log;
+  auto work = [&](uint64_t word, uint64_t pairs) {
     const Item item(word);
     const int gi = item.group, tile_rel = item.tile, stage = item.stage;
     const MistGroupDesc *g = groups + gi;
-    uint64_t hit;
     if constexpr (kSamples) {
       __shared__ SampleQueue lds_queues[kWaves];
-      hit = reduce_item_samples<kResolve>(prob, g, gi, tile_rel, stage, row_terms, stage_floor, ratios, tabs, pairs,
-                                          &lds_queues[local_wave]);
+      reduce_item_samples<kResolve>(prob, g, gi, tile_rel, stage, row_terms, stage_floor, ratios, tabs, pairs,
+                                    &lds_queues[local_wave], log);
     } else
-      hit = reduce_item<kResolve, kInLds>(prob, g, gi, tile_rel, stage, row_terms, stage_floor, ratios.r[0], tabs,
-                                          pairs, lds_rows + local_wave * wave_pitch);
-    // (the other units of the item read and write other bits)
-    if (!kResolve && hit != pairs && lane == 0) atomicAnd(tabs.hit + at, (unsigned long long)~(pairs & ~hit));
+      reduce_item<kResolve, kInLds>(prob, g, gi, tile_rel, stage, row_terms, stage_floor, ratios.r[0], tabs, pairs,
+                                    lds_rows + local_wave * wave_pitch, log);
   };
-  constexpr bool kListed = kResolve && kSamples;
-  const FlatQueue queue = flat_queue(tabs, kListed ? 0 : 1);
+  const FlatQueue queue = flat_queue(tabs, 1);
   // enough units for every wavefront several times over; a pair of several samples takes longer (30 samples
   // of one tensor-parallel size of the 7B plan: 64 pairs a unit 2.36 ms, 32 2.12, 16 2.09)
   int split = kSamples ? 2 : 0;
   while (split < 4 && ((uint64_t)queue.total << split) < (uint64_t)n_waves * 2) ++split;
   const uint64_t units = (uint64_t)queue.total << split;
-  if (kResolve) {  // few are left: handed out in turn
+  if (kResolve) {  // handed out in turn
     for (uint64_t u = (uint64_t)blockIdx.x * kWaves + local_wave; u < units; u += n_waves) {
-      int64_t at = queue.at((uint32_t)(u >> split), tabs.capacity);
-      if (kListed) at = (int64_t)from_lane((uint64_t)tabs.item[at], 0);
-      uint64_t pairs = from_lane((uint64_t)tabs.hit[at], 0) & (every_pair(split) << (u & ((1u << split) - 1u)));
-      if (pairs == 0) continue;
-      const uint64_t word = from_lane((uint64_t)tabs.opened[at], 0);
-      if (!kListed) {  // pairs whose minima changed
-        const Item item(word);
-        const MistGroupDesc *g = groups + item.group;
-        const int64_t tile_cell = g->cell_offset + (int64_t)item.tile * MIST_LC_TILE * slots_of(g->num_p);
-        pairs &= __ballot(tabs.changed[(tile_cell + lane * slots_of(g->num_p)) / 4] != 0);
-        if (pairs == 0) continue;
-      }
-      work(at, word, pairs);
+      const int64_t at = queue.at((uint32_t)(u >> split), tabs.capacity);
+      const uint64_t pairs = from_lane((uint64_t)tabs.open_pairs[at], 0) & (every_pair(split) << (u & ((1u << split) - 1u)));
+      if (pairs != 0) work(from_lane((uint64_t)tabs.opened[at], 0), pairs);
     }
     return;
   }
-  // (the resolve list goes where the filter's items were)
-  if (kSamples && blockIdx.x == 0 && threadIdx.x < kQueueShards) tabs.counter[threadIdx.x * kCounterPitch] = 0;
   for (int k = 0; k < kNumXcd; ++k) {
     const int part = ((int)blockIdx.x + k) % kNumXcd;
     const uint32_t first = (uint32_t)(units * part / kNumXcd), n = (uint32_t)(units * (part + 1) / kNumXcd) - first;
@@ -3299,49 +3293,39 @@ __global__ __launch_bounds__(kReduceThreads, 3) void reduce_kernel(
       if (u >= n) break;
       ahead = draw();
       const int64_t at = queue.at((first + u) >> split, tabs.capacity);
-      const uint64_t pairs = tabs.hit[at] & every_pair(split) << ((first + u) & ((1u << split) - 1u));
+      const uint64_t pairs = tabs.open_pairs[at] & every_pair(split) << ((first + u) & ((1u << split) - 1u));
       const uint64_t word = tabs.opened[at];
-      if (from_lane(pairs, 0) != 0) work(at, from_lane(word, 0), from_lane(pairs, 0));
+      if (from_lane(pairs, 0) != 0) work(from_lane(word, 0), from_lane(pairs, 0));
     }
   }
+  log.close(tabs);
 }
 
-// ---- resolve list (several samples) ----
-// A wavefront takes 64 neighbouring items of a shard, lane = item: of the pairs in which some row
-// reached its minimum those whose minima changed stay in `hit`, and the items that have any are
-// listed (places in `opened`).  (The resolve launch looked for them itself, a wavefront and four
-// dependent reads per item, and the few that were left sat with few wavefronts: 30 samples of one
-// tensor-parallel size of the 7B plan 2.03 ms, 1.37 with the list; the whole of 7B on 4x8 0.59 -> 0.27.)
-__global__ __launch_bounds__(kReduceThreads) void resolve_list_kernel(const MistGroupDesc *__restrict__ groups,
-                                                                      const ReduceTables tabs) {
-  constexpr int kWaves = kReduceThreads / 64;
+// ---- resolve ----
+// The lowest row of every minimum, from the log; a wavefront a chunk at a time, its four loads in flight together.
+// Bound by the scattered reads of minima and atomics on rows.  (The items in which a row had reached a minimum gone
+// through again, where the pair's minima had changed: 30 samples of one tensor-parallel size of the 7B plan 0.58 ms
+// with the list of those items, now 0.08; of 7B on 1x8 0.15 and 0.012; one sample, 70B on 32x8 0.53 and 0.05, 13B on
+// 4x8 0.12 and 0.017.  By the registers of the reduce kernel, three wavefronts a SIMD and two loads: 0.38 instead of
+// 0.08.  What the log costs the reduce launch is within its spread.)
+__global__ __launch_bounds__(kReduceThreads) void resolve_kernel(const ReduceTables tabs) {
+  constexpr int kWaves = kReduceThreads / 64, kAtOnce = kLogChunk / 64;
+  if (tabs.counter[kLogFull * kCounterPitch] != 0) return;  // reduce_kernel<true, ..> goes through everything
+  const uint32_t n_chunks = tabs.counter[kLogTaken * kCounterPitch];
   const int lane = threadIdx.x & 63;
-  const ChunkQueue queue = chunk_queue(tabs, 1);
-  for (uint32_t u = (uint32_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * kWaves + (threadIdx.x >> 6)));
-       u < queue.chunks; u += gridDim.x * kWaves) {
-    int n_here;
-    const int64_t first = queue.at(u, tabs.capacity, &n_here);
-    const int64_t at = first + min(lane, n_here - 1);
-    uint64_t left = lane < n_here ? tabs.hit[at] : 0, mine = 0;
-    if (!__any(left != 0)) continue;
-    const Item item((uint64_t)tabs.opened[at]);
-    const MistGroupDesc *g = groups + item.group;
-    const int n_slots = slots_of(g->num_p);
-    const int64_t cell0 = g->cell_offset + (int64_t)item.tile * MIST_LC_TILE * n_slots;
-    for (; left != 0; left &= left - 1) {
-      const int pair = __ffsll((unsigned long long)left) - 1;
-      if (tabs.changed[(cell0 + pair * n_slots) / 4] != 0) mine |= 1ull << pair;
-    }
-    const uint64_t found = (uint64_t)__ballot(mine != 0);
-    if (found == 0) continue;
-    const int shard = (int)(first / tabs.capacity);  // (no more than the shard's items: it cannot overflow)
-    uint32_t base = 0;
-    if (lane == 0) base = atomicAdd(tabs.counter + shard * kCounterPitch, (uint32_t)__popcll(found));
-    base = (uint32_t)from_lane((int)base, 0);
-    if (mine != 0) {
-      tabs.hit[at] = mine;
-      tabs.item[(int64_t)shard * tabs.capacity + base + __popcll(found & ((1ull << lane) - 1ull))] = (unsigned long long)at;
-    }
+  for (uint32_t chunk = (uint32_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * kWaves + (threadIdx.x >> 6)));
+       chunk < n_chunks; chunk += gridDim.x * kWaves) {
+    const int n = (int)tabs.log_count[chunk];
+    const Hit *__restrict__ log = tabs.log + (int64_t)chunk * kLogChunk;
+    Hit hit[kAtOnce];
+    double best[kAtOnce];
+#pragma unroll
+    for (int i = 0; i < kAtOnce; ++i) hit[i] = log[min(i * 64 + lane, n - 1)];
+#pragma unroll
+    for (int i = 0; i < kAtOnce; ++i) best[i] = tabs.best[hit[i].cell];
+#pragma unroll
+    for (int i = 0; i < kAtOnce; ++i)
+      if (i * 64 + lane < n && best[i] == hit[i].cost) atomicMin(tabs.row + hit[i].cell, hit[i].row);
   }
 }
 
@@ -3794,7 +3778,6 @@ __device__ __forceinline__ void take_lower(double &cost, uint32_t &row, double i
   row = its_cost < cost ? its_row : its_cost == cost ? min(row, its_row) : row;
   cost = fmin(cost, its_cost);
 }
-__device__ __forceinline__ uint32_t row_number(uint32_t held) { return held == ~0u ? held : held & ~kUnresolved; }
 
 // One sample: workgroup = (tile, variant, group).  The slots of a pair lie side by side, the tables'
 // last axis is c: kFinalSlots slots at a time are read with lane = (pair parity, slot), scanned, and
@@ -3836,7 +3819,7 @@ __global__ __launch_bounds__(256) void finalize_kernel(
       uint32_t row = ~0u;
       if (p < np) {
         cost = tabs.best[cell];
-        row = row_number(tabs.row[cell]);
+        row = tabs.row[cell];
       }
       for (int step = 1; step < kFinalSlots; step <<= 1) {
         const double its_cost = __shfl_down(cost, step, kFinalSlots);
@@ -3885,7 +3868,7 @@ __global__ __launch_bounds__(256) void finalize_samples_kernel(
   double cost = INFINITY;
   uint32_t row = ~0u;
   for (int p = f.n_p - 1; p >= p_begin; --p) {
-    take_lower(cost, row, tabs.best[first + (int64_t)p * n], row_number(tabs.row[first + (int64_t)p * n]));
+    take_lower(cost, row, tabs.best[first + (int64_t)p * n], tabs.row[first + (int64_t)p * n]);
     if (p < p_begin + kFinalRange) write_final(f, g, variant, pc, k, row_terms, row, p, tables, false);
   }
 }
@@ -4184,11 +4167,12 @@ int64_t mist_stage_floor_doubles(int64_t total_rows, int n_groups) {
 }
 
 // Sections of the reduce workspace in `d_partial_cost` (doubles): the minima of n_samples samples,
-// the second-level summaries, the four lists, their counters, a word per stage and one per pair, the
-// bounds of the gathered rows.
+// the second-level summaries, the four lists, their counters, a word per stage, the bounds of the gathered
+// rows, the log and its chunks' counts.
 struct WorkspaceLayout {
-  int64_t best, supers, items, counters, flags, changed, gathered, total;
-  int64_t capacity;  // items per shard
+  int64_t best, supers, items, counters, flags, gathered, log, log_counts, total;
+  int64_t capacity;    // items per shard
+  int64_t log_chunks;
 };
 static WorkspaceLayout workspace_layout(int64_t cells, int64_t supers, int64_t items, int n_samples) {
   WorkspaceLayout w;
@@ -4198,14 +4182,24 @@ static WorkspaceLayout workspace_layout(int64_t cells, int64_t supers, int64_t i
   w.items = w.supers + supers * kStageFloorPitch;
   w.counters = w.items + 4 * kQueueShards * w.capacity;
   w.flags = w.counters + kCounters * kCounterPitch / 2;
-  w.changed = w.flags + supers * kSuperStages / 2;
-  w.gathered = w.changed + cells / 8 + 1;
-  w.total = w.gathered + supers * kSuperStages * kGatherFloor;  // (a batch of samples may end with one alone)
+  w.gathered = w.flags + supers * kSuperStages / 2;
+  w.log = w.gathered + supers * kSuperStages * kGatherFloor;  // (a batch of samples may end with one alone)
+  w.log += w.log % 2;
+  // (a chunk of every wavefront's is as a rule not full)
+  w.log_chunks = std::min(kLogPerCell * cells * n_samples, kLogEntries) / kLogChunk + kReduceBlocks * (kReduceThreads / 64);
+  w.log_counts = w.log + w.log_chunks * kLogChunk * (int64_t)(sizeof(Hit) / 8);
+  w.total = w.log_counts + w.log_chunks / 2 + 1;
   return w;
 }
 int64_t mist_reduce_workspace_doubles(int64_t cells, int64_t supers, int64_t items, int n_samples) {
   if (cells < 0 || supers < 0 || items < 0 || n_samples < 1) return -1;
   return workspace_layout(cells, supers, items, n_samples).total;
+}
+// (cells beyond 32 bits: no log; for tests MIST_REDUCE_LOG_CHUNKS is the most)
+static uint32_t log_chunks(int64_t chunks, int64_t cells) {
+  const char *most = getenv("MIST_REDUCE_LOG_CHUNKS");
+  if (cells > (int64_t)UINT32_MAX) chunks = 0;
+  return (uint32_t)(most == nullptr || *most == '\0' ? chunks : std::min(chunks, (int64_t)atoll(most)));
 }
 // rows_present: false = only the rows the seed launch gathers are, the others follow by need
 static int reduce_tables(const MistProblem *problem, int n_samples, double *d_partial_cost, int32_t *d_partial_index,
@@ -4221,11 +4215,13 @@ static int reduce_tables(const MistProblem *problem, int n_samples, double *d_pa
   out->super_floor = d_partial_cost + w.supers;
   out->item = reinterpret_cast<unsigned long long *>(d_partial_cost + w.items);
   out->opened = out->item + kQueueShards * w.capacity;
-  out->hit = out->opened + kQueueShards * w.capacity;
-  out->listed = rows_present ? nullptr : out->hit + kQueueShards * w.capacity;
+  out->open_pairs = out->opened + kQueueShards * w.capacity;
+  out->listed = rows_present ? nullptr : out->open_pairs + kQueueShards * w.capacity;
   out->stage_flag = reinterpret_cast<uint32_t *>(d_partial_cost + w.flags);
   out->counter = reinterpret_cast<uint32_t *>(d_partial_cost + w.counters);
-  out->changed = reinterpret_cast<uint32_t *>(d_partial_cost + w.changed);
+  out->log = reinterpret_cast<Hit *>(d_partial_cost + w.log);
+  out->log_count = reinterpret_cast<uint32_t *>(d_partial_cost + w.log_counts);
+  out->log_chunks = log_chunks(w.log_chunks, problem->reduce_cells * n_samples);
   out->gather_floor = d_partial_cost + w.gathered;
   out->capacity = (uint32_t)w.capacity;
   out->n_samples = n_samples;
@@ -4362,18 +4358,15 @@ static int launch_reduce(const MistProblem *problem, const MistGroupDesc *d_grou
   if (lds > 64 * 1024)
     if (int rc = allow_large_lds()) return rc;
 #define MIST_REDUCE(RESOLVE, SAMPLES, IN_LDS)                                                               \
-  hipLaunchKernelGGL((reduce_kernel<RESOLVE, SAMPLES, IN_LDS>), dim3(kReduceBlocks), dim3(kReduceThreads), lds, \
-                     (hipStream_t)stream, *problem, d_groups, d_row_terms, d_stage_floor, ratios, tabs, wave_pitch)
+  hipLaunchKernelGGL((reduce_kernel<RESOLVE, SAMPLES, IN_LDS>), dim3(RESOLVE ? kAgainBlocks : kReduceBlocks),    \
+                     dim3(kReduceThreads), lds, (hipStream_t)stream, *problem, d_groups, d_row_terms, d_stage_floor, ratios, tabs, wave_pitch)
   if (!one) MIST_REDUCE(false, true, false);
   else if (buffered) MIST_REDUCE(false, false, true);
   else MIST_REDUCE(false, false, false);
   MIST_HIP_CHECK(hipGetLastError());
-  // (with one sample the list costs what it saves, 15 us of 1.3B on 1x2, and 70B on 32x8 gains 0.06 ms)
-  if (!one) {
-    hipLaunchKernelGGL(resolve_list_kernel, dim3(kReduceBlocks / 4), dim3(kReduceThreads), 0, (hipStream_t)stream,
-                       d_groups, tabs);
-    MIST_HIP_CHECK(hipGetLastError());
-  }
+  hipLaunchKernelGGL(resolve_kernel, dim3(kReduceBlocks), dim3(kReduceThreads), 0, (hipStream_t)stream, tabs);
+  MIST_HIP_CHECK(hipGetLastError());
+  // (returns at once unless the log ran full)
   if (!one) MIST_REDUCE(true, true, false);
   else if (buffered) MIST_REDUCE(true, false, true);
   else MIST_REDUCE(true, false, false);
