@@ -42,7 +42,13 @@ constexpr int kTermsBlock = 128;  // rows per workgroup of the row-term kernel
 constexpr int kStageRows = 64;    // rows of a stage: one summary, one item of the reduction
 constexpr int kSlots = 2 * MIST_P_TILE + 2;  // per-thread running minima: base, with_pre, post, no_pp
 constexpr int kScoutSplit = 1;    // (mist_reduce_scout_split: workgroups of a decomposition no launch has any more)
-constexpr double kIncumbentSlack = 0.25;  // relative room above MistProblem.stage_cost_incumbent / G
+// Relative room above MistProblem.stage_cost_incumbent / G.  The launches behind the seeds look for what lies
+// below it: the less room, the fewer rows.  Calls, us, at 0.25 / 0.1 / 0.02 / 0.004: 70B on 32x8 7681 / 6497 / 5775
+// / 5430, 13B on 8x8 2286 / 1976 / 1859 / 1770, 7B on 4x8 1477 / 1370 / 1200 / 1140.  A search that cannot tell from
+// tables under the limit what the complete ones give evaluates again, at any room about as often: 25 / 23 / 17 / 22
+// of 330 calls (less room, fewer (tp, G) with a partition below it; but fewer threshold candidates, too).  Results
+// above the estimate, by up to 1.7 % where the scan tries none of its thresholds, want more than the last.
+constexpr double kIncumbentSlack = 0.02;
 // Stage summaries (written with or ahead of the row terms, read by filter, open and reduce): per stage of
 // kStageRows workspace rows the term-wise minimum of the latency and memory columns and the
 // maximum of MIST_T_OUT, kStageFloorPitch doubles per stage.
