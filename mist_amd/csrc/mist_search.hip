@@ -3481,24 +3481,37 @@ __global__ __launch_bounds__(MIST_LC_TILE, MIST_EXHAUSTIVE_MIN_WAVES) void eval_
                             lds_terms, lds_row, partial_cost + block * slab, partial_index + block * slab);
 }
 
-// The equal-stage pipeline a group offers to the stage-cost estimates: S stages of L / S layers
-// on the group's mesh, or 0 when the devices or the layers do not divide, the group has too few
-// pre-saved micro-batch values, or the caller's search does not go that deep.
+// The pipeline a group offers to the stage-cost estimates: S stages of L / S layers on the group's
+// mesh (PipelineLayers where the layers do not divide), or 0 when the devices do not, the group has too few
+// pre-saved micro-batch values, or the caller's search does not go that deep.  A power of two of devices has a
+// pipeline that divides its layers, one stage on all of them, and the others seldom say more (8 of 189 such calls
+// got a lower estimate, 0.8 % of their time): those are not gone through.
 __device__ __forceinline__ int incumbent_stage_count(const MistProblem &prob,
                                                      const MistGroupDesc *__restrict__ g) {
   const int L = prob.num_layers, D = prob.incumbent_num_devices;
   const int nm = g->num_nodes * g->num_gpus_per_node;
   if (nm <= 0 || D % nm != 0) return 0;
   const int S = D / nm;
-  if (S < 1 || S > L || L % S != 0 || S - 1 >= g->num_p) return 0;
+  if (S < 1 || S > L || S - 1 >= g->num_p) return 0;
+  if (L % S != 0 && (D & (D - 1)) == 0) return 0;
   // (the per-mesh search goes up to min(devices, layers) / 2 stages, inter_tuning.py:279-281)
   if (prob.incumbent_ckpt_rule == 0 && S > (D < L ? D : L) / 2) return 0;
   return S;
 }
 
+// Its layers: the first L % S stages behind the first one, which holds the pre layer and the most micro-batches,
+// have one more.  (Of 14 nodes and 57 layers or 5 and 23, no mesh has stages that divide both; such searches
+// ran without an estimate, 39 of 232 calls: 70B, 57 layers on 14x8 10164 -> 2598 us, 13B, 23 on 5x8 1784 -> 1050.)
+struct PipelineLayers {
+  int each, extra;
+  __device__ __forceinline__ PipelineLayers(int layers, int stages) : each(layers / stages), extra(layers % stages) {}
+  __device__ __forceinline__ int of(int stage) const { return each + (stage >= 1 && stage <= extra ? 1 : 0); }
+  __device__ __forceinline__ int end(int stage) const { return (stage + 1) * each + min(stage, extra) - 1; }  // last layer
+};
+
 // Cost of the best pipeline of equal stages on equal meshes that the seeds allow
 // (sample 0 of a call with one sample, whose objective is the stage cost): group (G, mesh (n, m))
-// offers S = devices / (n m) stages of L / S layers each, the first one from the with_pre table
+// offers S = devices / (n m) stages of about L / S layers each, the first one from the with_pre table
 // at S - 1 pre-saved micro-batches, the last one from the with_post table, those between from
 // the base table, a single one from the no_pp table, each at its cheapest admissible ckpt count
 // (rule of the caller's search, MistProblem.incumbent_ckpt_rule); the cost is the sum of the
@@ -3516,9 +3529,10 @@ __global__ __launch_bounds__(64 * kIncumbentWaves) void incumbent_kernel(
   const int L = prob.num_layers;
   const int S = incumbent_stage_count(prob, g);
   if (S == 0) return;
-  const int l = L / S, P = g->num_p;
-  // seed of the stage's (l, c) cell in slot `slot` (one sample; +inf where there is none)
-  auto seed_of = [&](int slot, int c) {
+  const PipelineLayers layers(L, S);
+  const int P = g->num_p;
+  // seed of a stage's (l, c) cell in slot `slot` (one sample; +inf where there is none)
+  auto seed_of = [&](int slot, int l, int c) {
     const int pair = l * (l + 1) / 2 - 1 + c;
     const int lc_tile = pair / MIST_LC_TILE - g->lc_tile_begin;
     if (lc_tile < 0 || lc_tile >= g->n_lc_tiles) return (double)INFINITY;
@@ -3526,27 +3540,27 @@ __global__ __launch_bounds__(64 * kIncumbentWaves) void incumbent_kernel(
                      ((int64_t)lc_tile * MIST_LC_TILE + pair % MIST_LC_TILE) * slots_of(P) + slot];
   };
   // cheapest one over c = 0..c_last
-  auto cheapest = [&](int slot, int c_last) {
+  auto cheapest = [&](int slot, int l, int c_last) {
     double best = INFINITY;
-    for (int c = threadIdx.x & 63; c <= c_last; c += 64) best = fmin(best, seed_of(slot, c));
+    for (int c = threadIdx.x & 63; c <= c_last; c += 64) best = fmin(best, seed_of(slot, l, c));
     for (int step = 32; step > 0; step >>= 1) best = fmin(best, __shfl_xor(best, step));
     return best;
   };
-  auto c_last_of = [&](int end_layer) {
+  auto c_last_of = [&](int l, int end_layer) {
     return prob.incumbent_ckpt_rule == 0 ? min(l, L - end_layer) : l;
   };
   __shared__ double wave_sum[kIncumbentWaves], wave_largest[kIncumbentWaves];
   const int wave = threadIdx.x >> 6;
   double sum = 0.0, largest = 0.0;
   for (int s = wave; s < S; s += kIncumbentWaves) {
-    const int p = S - 1 - s, end_layer = (s + 1) * l - 1;
+    const int p = S - 1 - s, l = layers.of(s);
     int slot;
     if (S == 1) slot = 2 * P + 1;
     else if (s == 0) slot = P + p;
     else if (s == S - 1) slot = 2 * P;
     else slot = p;
     // (rule 2: every layer of the stage checkpointed)
-    const double cost = prob.incumbent_ckpt_rule == 2 ? seed_of(slot, l) : cheapest(slot, c_last_of(end_layer));
+    const double cost = prob.incumbent_ckpt_rule == 2 ? seed_of(slot, l, l) : cheapest(slot, l, c_last_of(l, layers.end(s)));
     sum += cost;
     largest = fmax(largest, cost);
   }
@@ -3572,7 +3586,7 @@ __global__ __launch_bounds__(64 * kIncumbentWaves) void incumbent_kernel(
 // can already leave out stage costs the caller's search cannot use.  Each group evaluates about
 // kEstimateRows of its gathered rows - every parallelism row of every scout pair without
 // activation / optimizer offloading first, then with the next ratios - for the layer count
-// l = L / S and every ckpt count, exactly as the tables would (same latency and memory code as
+// of its stages (two, where S does not divide L) and every ckpt count, exactly as the tables would (same latency and memory code as
 // the evaluate-every-cell kernel, same cells kept: c == l - 1 only at p == 0 of the base /
 // with_pre tables), and keeps per stage of the pipeline the cheapest feasible cost.  Minima over
 // fewer rows than the seeds see, so the estimate is no smaller than theirs.
@@ -3602,7 +3616,8 @@ __global__ __launch_bounds__(256) void estimate_stage_minima_kernel(
   }
   int S;
   if (!estimate_runs(prob, g, &S)) return;
-  const int L = prob.num_layers, l = L / S, rule = prob.incumbent_ckpt_rule;
+  const int L = prob.num_layers, rule = prob.incumbent_ckpt_rule;
+  const PipelineLayers layers(L, S);
   __shared__ unsigned long long stage_min[kEstimateMaxStages];
   const unsigned long long kInf = (unsigned long long)__double_as_longlong((double)INFINITY);
   for (int st = threadIdx.x; st < S; st += blockDim.x) stage_min[st] = kInf;
@@ -3611,7 +3626,8 @@ __global__ __launch_bounds__(256) void estimate_stage_minima_kernel(
   const int64_t per_pair = (int64_t)g->n_par * n_tail;
   const int64_t per_tail = (int64_t)g->n_par * max(g->scout_stride, 1);
   const int64_t n_tails = min((int64_t)n_tail, max((int64_t)1, (int64_t)kEstimateRows / per_tail));
-  const int64_t n_items = per_tail * n_tails * (l + 1);
+  const int n_cells = layers.each + 1 + (layers.extra > 0 ? layers.each + 2 : 0);  // (layers, ckpt) of a row
+  const int64_t n_items = per_tail * n_tails * n_cells;
   const GroupConsts k = group_consts(g);
   const double cap = prob.mem_cap_mb;
   const double G64 = (double)g->grad_accum;
@@ -3624,8 +3640,10 @@ __global__ __launch_bounds__(256) void estimate_stage_minima_kernel(
   };
   for (int64_t item = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; item < n_items;
        item += (int64_t)kEstimateSplit * blockDim.x) {
-    const int c = (int)(item % (l + 1));
-    const int64_t q = item / (l + 1);
+    const int cell = (int)(item % n_cells);
+    const bool longer = cell > layers.each;
+    const int l = longer ? layers.each + 1 : layers.each, c = longer ? cell - l : cell;
+    const int64_t q = item / n_cells;
     const int64_t tail = q / per_tail, rest = q - tail * per_tail;
     const int64_t pair = rest / g->n_par, par = rest - pair * g->n_par;
     if (rule == 2 && c != l) continue;  // every layer of a stage checkpointed
@@ -3635,7 +3653,7 @@ __global__ __launch_bounds__(256) void estimate_stage_minima_kernel(
     const CellLatency lat = cell_latency<true>(t, l, c, k);
     const LaneMemory mem = cell_memory(t, l, c);
     // largest ckpt count of the stage that ends with layer end_layer (rule of the caller's search)
-    auto c_last = [&](int st) { return rule == 0 ? min(l, L - ((st + 1) * l - 1)) : l; };
+    auto c_last = [&](int st) { return rule == 0 ? min(l, L - layers.end(st)) : l; };
     double peak_f, peak_b;
     mem.peaks(0, peak_f, peak_b);
     const double f_in = mem.fwd_states + g->post_states + mem.mod_saved + g->post_fwd_peak + mem.gcb;
@@ -3651,14 +3669,16 @@ __global__ __launch_bounds__(256) void estimate_stage_minima_kernel(
       continue;
     }
     // first stage: with_pre table at S - 1 pre-saved micro-batches
-    offer(0, c <= c_last(0) && mem.feasible_pre(S - 1, cap, g->pre_saved, g->pre_states_and_saved),
+    offer(0, !longer && c <= c_last(0) && mem.feasible_pre(S - 1, cap, g->pre_saved, g->pre_states_and_saved),
           ratio * lat.sp + lat.dpre / G64);
     // last stage: with_post table
-    offer(S - 1, c <= c_last(S - 1) && fmax(pf_post, pb_post) * mem.mf_pp <= cap,
+    offer(S - 1, l == layers.of(S - 1) && c <= c_last(S - 1) && fmax(pf_post, pb_post) * mem.mf_pp <= cap,
           ratio * lat.spost + lat.dpost / G64);
     // stages between: base table at S - 1 - st pre-saved micro-batches
     const double cost_base = ratio * (double)lat.x + (double)(lat.d / G32);
-    for (int st = 1; st < S - 1; ++st)
+    // (of l layers: stages 1 .. extra have the extra layer)
+    const int st_end = longer ? min(layers.extra + 1, S - 1) : S - 1;
+    for (int st = longer ? 1 : layers.extra + 1; st < st_end; ++st)
       offer(st, c <= c_last(st) && mem.feasible_base(S - 1 - st, cap), cost_base);
   }
   __syncthreads();
