@@ -99,7 +99,9 @@ int mist_inter_stage_search_families(int n_families, const MistDpShape *shapes,
  *                   reference's scan may find such a partition at a threshold above limit(G)
  *                   (its threshold candidates leave out single-stage costs and those its gap
  *                   rule drops), which these tables cannot tell: evaluate again on complete
- *                   tables. */
+ *                   tables.  Minus that number: there are such pairs, but the result (with
+ *                   only_best_path that of the best instance) is the same whether the reference
+ *                   finds those partitions or not. */
 int mist_inter_stage_search_bounded(int n_families, const MistDpShape *shapes,
                                     const MistDpCosts *costs, const MistDpCosts *select_costs,
                                     const MistStrategyIndex *strategy, int n_instances,

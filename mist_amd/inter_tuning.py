@@ -839,7 +839,8 @@ def _native_search(runner: _DpRunner, results_list, rows, Gs, n_g, g_index, q_in
                 ctypes.c_void_p(unresolved.ctypes.data))
     _lib.check(rc, "mist_inter_stage_search_families")
     if stats is not None:
-        stats["dp_unresolved"] = stats.get("dp_unresolved", 0) + int(unresolved[0])
+        stats["dp_unresolved"] = stats.get("dp_unresolved", 0) + abs(int(unresolved[0]))
+        stats["dp_undecided"] = stats.get("dp_undecided", 0) + max(int(unresolved[0]), 0)
     t_1 = time.perf_counter()
     out = []
     for t in range(n_inst):
@@ -899,7 +900,8 @@ def inter_stage_tune_batch(
     ``table_limit`` (pinned host tensor with an estimate, factor): the tables hold their values
     up to ``estimate * factor / G`` only (``IntraStageTuner.run_prepared`` with a stage-cost
     cutoff); the search then stays below that limit and ``stats['dp_unresolved']`` counts the
-    (entry, G) pairs whose result is not certain to be the reference's (library search only)."""
+    (entry, G) pairs whose result is not certain to be the reference's (library search only);
+    ``stats['dp_undecided']`` is 0 where the best entry's is the same either way."""
     if table_limit is not None and not (NATIVE_SEARCH and _same_batch(results_list)):
         raise ValueError("tables with a limit need the library's search over one batch of tables")
     for r in results_list:

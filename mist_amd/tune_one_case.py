@@ -188,8 +188,8 @@ class PreparedSearch:
         # cells (IntraStageTuner.run_prepared), given an estimate of the best cost.  ``run``
         # searches such tables below the limit up to which they are exact
         # (mist_inter_stage_search_bounded) and evaluates again without the estimate if that
-        # search reports a partition it may have missed or its result is not below the limit
-        # of the estimate that was used.  ckpt counts a stage may use, as those
+        # search reports a partition it may have missed that the result depends on, or its result
+        # is not below the limit of the estimate that was used.  ckpt counts a stage may use, as those
         # searches restrict them: inter_tuning.py:315; inter_tuning_uniform_device.py:400-404.
         self.stage_cost_cutoff = None
         self._incumbent_host = self._incumbent_read = None
@@ -241,7 +241,7 @@ class PreparedSearch:
         # that and reports where this leaves its result uncertain.
         limit_factor = (1.0 + _lib.load().mist_incumbent_slack()) * (1.0 - 1e-5)
         table_limit = None if cutoff is None else (self._incumbent_host, limit_factor)
-        unresolved_before = stats.get("dp_unresolved", 0)
+        unresolved_before, undecided_before = stats.get("dp_unresolved", 0), stats.get("dp_undecided", 0)
         if self.granularity == "inter-stage":
             outcomes = inter_stage_tune_batch(
                 self.L, hw.num_nodes * hw.num_gpus_per_node, self.meshes, self.Gs, results, slot=0, stats=stats,
@@ -270,7 +270,11 @@ class PreparedSearch:
             safe_below = estimate * limit_factor
             unresolved = stats.get("dp_unresolved", 0) - unresolved_before
             if np.isfinite(estimate) and (unresolved > 0 or not best_cost < safe_below):
+                # (counts the results in doubt, those that the search could settle by itself too)
                 stats["stage_cost_cutoff_retries"] = stats.get("stage_cost_cutoff_retries", 0) + 1
+                if stats["dp_undecided"] == undecided_before and best_cost < safe_below:
+                    return best_cost, best_solution
+                stats["stage_cost_second_evaluations"] = stats.get("stage_cost_second_evaluations", 0) + 1
                 self.stage_cost_cutoff = None
                 try:
                     return self.run(stats, split_timing)
