@@ -81,7 +81,9 @@ int mist_inter_stage_search_families(int n_families, const MistDpShape *shapes,
 /* mist_inter_stage_search_families over tables that hold their values only up to a limit per G
  * (the tables an intra-stage call with MistProblem.stage_cost_incumbent leaves: a cell whose
  * minimum is not above estimate / G * (1 + mist_incumbent_slack()) holds it, any other cell
- * holds something above).  No counterpart in the reference: it is the reference's scan
+ * holds something above; but see MistProblem.incumbent_close, whose exceptions lie below every
+ * threshold candidate read here: a window that would have to start further below counts as
+ * unresolved).  No counterpart in the reference: it is the reference's scan
  * (inter_tuning.py:163-217) made safe for such tables.
  *   host_estimate : one double in (pinned) HOST memory that holds the estimate once the work
  *                   queued on `stream` before this call has run (the search reads it after its

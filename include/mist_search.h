@@ -129,7 +129,13 @@ typedef struct MistProblem {
   int64_t reduce_cells, reduce_supers, reduce_items;
   /* != 0 (one sample): the tables are not pre-filled, and what reads them knows the cells that are never
    * written (mist_dp_cost_planes); a cell without a row gets its index of -1 and no costs. */
-  int32_t sparse_tables, reserved;
+  int32_t sparse_tables;
+  /* != 0 (with stage_cost_incumbent; the groups of the call are all groups of their table rows, those of a row
+   * side by side): for a caller whose search is all that reads the tables.  Below bound(G) a cell, too, that is
+   * in no pipeline of stages up to bound(G) may hold +inf / -1 or another row than its minimum's, as long as it
+   * then is below every threshold candidate which that search reads: those from 16 (1e-4 s + 1e-5 x) below the
+   * smallest largest stage cost x of a pipeline on. */
+  int32_t incumbent_close;
 } MistProblem;
 
 /* One (gradient-accumulation steps, device mesh) group = one call of the reference's

@@ -70,7 +70,7 @@ PROBLEM_DTYPE = np.dtype(
         ("reduce_supers", "<i8"),
         ("reduce_items", "<i8"),
         ("sparse_tables", "<i4"),
-        ("reserved", "<i4"),
+        ("incumbent_close", "<i4"),
     ],
     align=True,
 )

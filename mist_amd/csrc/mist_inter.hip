@@ -97,6 +97,8 @@ struct Workspace {
 std::mutex g_lock;  // one search at a time per process: the workspaces are shared
 std::map<int, Workspace> g_workspaces;
 
+constexpr int kExactWidenings = 2;  // (kCandidateRoom of mist_search.hip is the room they take)
+
 struct Window {
   bool exists = false;
   int row = 0, G = 1;
@@ -842,6 +844,7 @@ static int search_families(int n_families, const MistDpShape *shapes,
     }
   };
 
+  int too_wide = 0;  // windows that went further below than the tables hold their values
   // Decides windows on the host: `got[j]` = the ascending candidates of window todo[j] in
   // (lo[j], hi[j]] and how many lie above.  A window whose fetched part holds no certain start
   // of the walk is fetched again from further below; one whose first kept candidate lies higher
@@ -852,6 +855,8 @@ static int search_families(int n_families, const MistDpShape *shapes,
     std::vector<int> pending(todo.size());
     for (size_t k = 0; k < pending.size(); ++k) pending[k] = (int)k;
     for (int widen = 0; !pending.empty(); ++widen) {
+      // (tables under an estimate need not hold their values below: MistProblem.incumbent_close)
+      if (widen > kExactWidenings && host_estimate != nullptr && std::isfinite(*host_estimate)) too_wide += (int)pending.size();
       if (widen > 0) {
         std::vector<int32_t> r;
         lo.clear();
@@ -1230,7 +1235,7 @@ static int search_families(int n_families, const MistDpShape *shapes,
     for (int t = 1; t < n_instances; ++t)
       if (chains[t].best_cost < chains[winner].best_cost) winner = t;
     const double result = chains[winner].best_cost;
-    int doubtful = 0, undecided = 0;
+    int doubtful = too_wide, undecided = too_wide;
     for (int t = 0; t < n_instances; ++t) {
       std::vector<int> open;
       for (int i = 0; i < n_grad_accum; ++i) {

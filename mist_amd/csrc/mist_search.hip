@@ -1428,6 +1428,7 @@ __device__ __forceinline__ void take_min(double &best, int32_t &best_row, bool f
 // now 3.2 (reduce 2.1, open 0.42, seeds 0.33, filter 0.17, resolve 0.08).
 // ------------------------------------------------------------------------------------------
 constexpr int kSuperStages = 8;    // stages per second-level summary
+constexpr double kCandidateRoom = 16.0;  // two widenings of a window of threshold candidates (mist_inter.hip)
 constexpr int kGatherFloor = 5;    // linear bounds of 64 gathered rows
 constexpr int kQueueShards = 64;   // counters of the item queue: one would serve an append in ~8 ns
 constexpr int kCounterPitch = 32;  // uint32 between counters: a cache line each
@@ -1439,7 +1440,8 @@ constexpr int64_t kLogEntries = 24 << 20;
 constexpr int kLogPerCell = 4;
 constexpr int kLogTaken = 3 * kQueueShards + kNumXcd;  // counters: chunks taken, whether there were too few
 constexpr int kLogFull = kLogTaken + 1;
-constexpr int kCounters = kLogFull + 1;
+constexpr int kGroupsDone = kLogFull + 1;  // workgroups of the estimate that have ended
+constexpr int kCounters = kGroupsDone + 1;
 constexpr int kSeedThreads = 256;
 constexpr int kReduceThreads = 256;
 constexpr int kReduceBlocks = 2048;          // a multiple of kNumXcd
@@ -1489,6 +1491,16 @@ struct Hit {
 };
 static_assert(sizeof(Hit) == 16, "two doubles of the workspace");
 
+// What a group's stage costs can be used for (form_reach).
+struct GroupReach {
+  double per_layer, rest;  // of every row at least rest + (layers - 2) x per_layer (two layers or fewer: rest)
+  double cutoff;           // rows above it are not looked for
+  double low;              // a minimum below it, of a stage of fewer than `first` layers, is final as it is
+  int first, reserved;
+};
+static_assert(sizeof(GroupReach) == 5 * sizeof(double), "doubles of the workspace");
+constexpr int kReachGroups = 2048;  // the most groups that get one: 48 KB of LDS
+
 // (by value in the kernel arguments)
 struct ReduceTables {
   double *best;  // [pair][slot][sample] (slots_of(num_p) slots): the smallest cost
@@ -1496,6 +1508,8 @@ struct ReduceTables {
   Hit *log;             // [log_chunks][kLogChunk]
   uint32_t *log_count;  // [log_chunks]: entries of each
   double *super_floor;       // [supers][kStageFloorPitch]
+  struct GroupReach *reach;  // [group], with MistProblem.incumbent_close
+  double *reach_parts;       // [group][kSuperBlocks][2]: of each workgroup of the second-level summaries
   double *gather_floor;      // [stage][kGatherFloor]: what the seed launch asks of 64 gathered rows (one sample)
   // [kQueueShards][capacity]: Item, what the filter and then what the open launch left; open pairs of the
   // latter
@@ -1505,7 +1519,7 @@ struct ReduceTables {
   unsigned long long *listed;
   uint32_t *stage_flag;
   // at kCounterPitch: [kQueueShards] items, [kQueueShards] opened, [kQueueShards] listed, [kNumXcd] drawn,
-  // kLogTaken, kLogFull
+  // kLogTaken, kLogFull, kGroupsDone
   uint32_t *counter;
   uint32_t capacity, log_chunks;
   int n_samples;
@@ -1596,6 +1610,9 @@ __device__ __forceinline__ int cheapest_lane(bool pending, double cost) {
 // One entry of the minima in device memory / in LDS (global_atomic_min_f64, ds_min_f64).
 __device__ __forceinline__ void lower_minimum(double *entry, double cost) {
   __hip_atomic_fetch_min(entry, cost, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ double load_at_agent(const double *at) {
+  return __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ void lower_minimum_in_lds(double *entry, double cost) {
   __hip_atomic_fetch_min(entry, cost, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -1747,6 +1764,23 @@ __device__ __forceinline__ double stage_cost_cutoff(const MistProblem &prob, dou
   return prob.stage_cost_incumbent == nullptr || prob.sample_size != 1
              ? (double)INFINITY
              : *prob.stage_cost_incumbent * inv_G64 * (1.0 + kIncumbentSlack);
+}
+
+// The same with what form_reach knows of the group: rows above `cutoff` are not looked for, nor any of a
+// stage of fewer than `first` layers whose minimum is below `low`.
+struct CostLimits {
+  double cutoff, low;
+  int first;
+  __device__ __forceinline__ double closed_below(int layers) const { return layers < first ? low : -INFINITY; }
+};
+__device__ __forceinline__ CostLimits cost_limits(const MistProblem &prob, const ReduceTables &tabs, int group, double inv_G64) {
+  if (prob.incumbent_close == 0) return CostLimits{stage_cost_cutoff(prob, inv_G64), -INFINITY, 0};
+  const GroupReach &r = tabs.reach[group];
+  return CostLimits{r.cutoff, r.low, r.first};
+}
+// A minimum as a threshold.
+__device__ __forceinline__ double up_to(double minimum, double cutoff, double closed_below) {
+  return minimum < closed_below ? -INFINITY : fmin(minimum, cutoff);
 }
 
 // Group-wide terms the composite objectives add to the base latency: with x, d the
@@ -1952,15 +1986,16 @@ struct Loosest {
 };
 // (`slots`: the pair's slots of one sample, `pitch` apart; a pair that is not `wanted` reads none)
 __device__ __forceinline__ Loosest loosest_minima(bool wanted, const double *slots, int pitch, int P, int count_b,
-                                                  int count_p, bool do_post, bool do_pp, double cutoff) {
+                                                  int count_p, bool do_post, bool do_pp, double cutoff,
+                                                  double closed_below = -INFINITY) {
   Loosest t{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
   if (!wanted) return t;
   const double base = slots[max(count_b - 1, 0) * pitch], pre = slots[(P + max(count_p - 1, 0)) * pitch];
   const double post = slots[2 * P * pitch], pp = slots[(2 * P + 1) * pitch];
-  if (count_b > 0) t.base = fmin(base, cutoff);
-  if (count_p > 0) t.pre = fmin(pre, cutoff);
-  if (do_post) t.post = fmin(post, cutoff);
-  if (do_pp) t.pp = fmin(pp, cutoff);
+  if (count_b > 0) t.base = up_to(base, cutoff, closed_below);
+  if (count_p > 0) t.pre = up_to(pre, cutoff, closed_below);
+  if (do_post) t.post = up_to(post, cutoff, closed_below);
+  if (do_pp) t.pp = up_to(pp, cutoff, closed_below);
   return t;
 }
 // One threshold for GroupModel::bound that every row which could reach one of them passes: in two
@@ -2280,14 +2315,17 @@ __global__ __launch_bounds__(64 * kSeedSampleWaves) void seed_samples_kernel(
 __device__ __forceinline__ int64_t super_floor_slot(const MistGroupDesc *g, int group_index, int64_t super) {
   return stage_floor_slot(g, group_index, 0) / kSuperStages + group_index + super;
 }
+// With `close` a workgroup also leaves the smallest linear bounds of its summaries (GroupReach).
 __global__ __launch_bounds__(256) void super_floor_kernel(const MistGroupDesc *__restrict__ groups, int n_groups,
-                                                          const double *__restrict__ stage_floor,
+                                                          const double *__restrict__ stage_floor, double ratio, bool close,
                                                           const ReduceTables tabs) {
   const int gi = blockIdx.y;
   const MistGroupDesc *g = groups + gi;
   const int64_t n_stages = (g->n_rows + kStageRows - 1) / kStageRows;
   const int col = threadIdx.x % kStageFloorPitch;
   const int per_block = blockDim.x / kStageFloorPitch;
+  const double inv_G = 1.0 / (double)g->grad_accum;
+  double per_layer = INFINITY, rest = INFINITY;
   for (int64_t super = (int64_t)blockIdx.x * per_block + threadIdx.x / kStageFloorPitch;
        super * kSuperStages < n_stages; super += (int64_t)gridDim.x * per_block) {
     const double *__restrict__ src = stage_floor + (stage_floor_slot(g, gi, super * kSuperStages)) * kStageFloorPitch;
@@ -2299,7 +2337,25 @@ __global__ __launch_bounds__(256) void super_floor_kernel(const MistGroupDesc *_
     }
     tabs.super_floor[super_floor_slot(g, gi, super) * kStageFloorPitch + col] = v;
     if (tabs.listed != nullptr && col < n) tabs.stage_flag[stage_floor_slot(g, gi, super * kSuperStages) + col] = 0;
+    if (!close) continue;
+    // (the columns of a summary lie in 32 neighbouring lanes; every lane forms the same bounds)
+    const LinearBound b = linear_form([&](int stable, int delta) {
+      return less_slack(ratio * __shfl(v, stable, kStageFloorPitch)) + less_slack(__shfl(v, delta, kStageFloorPitch) * inv_G);
+    });
+    per_layer = fmin(per_layer, fmin(b.ck, b.nock));
+    rest = fmin(rest, fmin(b.all_ck, fmin(b.none, b.mid)));
   }
+  if (!close) return;
+  __shared__ double parts[256 / kStageFloorPitch][2];
+  if (col == 0) {
+    parts[threadIdx.x / kStageFloorPitch][0] = per_layer;
+    parts[threadIdx.x / kStageFloorPitch][1] = rest;
+  }
+  __syncthreads();
+  if (threadIdx.x >= 2) return;
+  double least = INFINITY;
+  for (int i = 0; i < per_block; ++i) least = fmin(least, parts[i][threadIdx.x]);
+  tabs.reach_parts[((int64_t)gi * kSuperBlocks + blockIdx.x) * 2 + threadIdx.x] = least;
 }
 
 // Lane = pair against a stage summary: the counts its pseudo row allows, hence which minima a row
@@ -2377,7 +2433,7 @@ __global__ __launch_bounds__(kSamples ? kFilterShares * 64 : 64) void filter_ker
   const int np = !active ? 0 : (pc.c == pc.l - 1 ? min(P, 1) : P);
   const bool do_post = active && pc.c != pc.l - 1, do_pp = do_post && pc.l == L;
   const GroupModel m = group_model(prob, g);
-  const double cutoff = stage_cost_cutoff(prob, m.inv_G64);
+  const CostLimits limits = cost_limits(prob, tabs, gi, m.inv_G64);
   const double *best = tabs.best + (g->cell_offset + (int64_t)tile_rel * MIST_LC_TILE * slots_of(P)) * S;
   extern __shared__ double lds_thresholds[];  // [sample][front, post][pair]
   if (kSamples) {
@@ -2391,7 +2447,7 @@ __global__ __launch_bounds__(kSamples ? kFilterShares * 64 : 64) void filter_ker
       const uint32_t its = (uint32_t)__shfl(parts, pair);
       const int n = (int)(its & 0x7fff);
       const Threshold t(loosest_minima(true, best + (int64_t)pair * slots_of(P) * S + sample, S, P, n, n,
-                                       (its >> 30 & 1u) != 0, its >> 31 != 0, cutoff), offsets);
+                                       (its >> 30 & 1u) != 0, its >> 31 != 0, limits.cutoff), offsets);
       lds_thresholds[2 * sample * kFilterPitch + pair] = t.front;
       lds_thresholds[(2 * sample + 1) * kFilterPitch + pair] = t.post;
     }
@@ -2402,8 +2458,10 @@ __global__ __launch_bounds__(kSamples ? kFilterShares * 64 : 64) void filter_ker
   const double loosest_ratio = ratios.r[kSamples ? min(lane & 31, S - 1) : 0];
   const Threshold loosest =
       kSamples ? Threshold(0.0, 0.0)
-               : Threshold(loosest_minima(true, best + (int64_t)lane * slots_of(P), 1, P, np, np, do_post, do_pp, cutoff),
+               : Threshold(loosest_minima(true, best + (int64_t)lane * slots_of(P), 1, P, np, np, do_post, do_pp, limits.cutoff,
+                                          limits.closed_below(pc.l)),
                            group_offsets(m, loosest_ratio));
+  if (!kSamples && !__any(loosest.at(0.0) > -INFINITY)) return;  // (nothing of the tile is looked for)
   int s = 0;
   auto passes = [&](const double *f) {
     float x, d;
@@ -2568,7 +2626,7 @@ __global__ __launch_bounds__(kReduceThreads) void open_kernel(const MistProblem 
   PairConsts k = {};
   GroupModel m = {};
   Offsets group = {};
-  double cutoff = INFINITY;
+  CostLimits limits = {};
   int P = 1;
   const double *best = tabs.best;
   // (the next item's summary is on its way to LDS while one is worked on, and the word of the one after it)
@@ -2637,7 +2695,7 @@ __global__ __launch_bounds__(kReduceThreads) void open_kernel(const MistProblem 
         k = pair_consts(p.pc.l, p.pc.c);
         m = group_model(prob, g);
         group = group_offsets(m, ratio);
-        cutoff = stage_cost_cutoff(prob, m.inv_G64);
+        limits = cost_limits(prob, tabs, gi, m.inv_G64);
         P = g->num_p;
         best = tabs.best + (g->cell_offset + (int64_t)item.tile * MIST_LC_TILE * slots_of(P)) * S;
       }
@@ -2647,8 +2705,8 @@ __global__ __launch_bounds__(kReduceThreads) void open_kernel(const MistProblem 
       if (!kSamples) {
         // (what lies above the cutoff needs no minima)
         const double bound = m.bound(ratio, reach.x, reach.d);
-        const Loosest low = loosest_minima(p.active && bound <= cutoff, best + lane * slots_of(P), 1, P, reach.count_b,
-                                           reach.count_p, reach.post, reach.pp, cutoff);
+        const Loosest low = loosest_minima(p.active && bound <= limits.cutoff, best + lane * slots_of(P), 1, P, reach.count_b,
+                                           reach.count_p, reach.post, reach.pp, limits.cutoff, limits.closed_below(p.pc.l));
         open = __ballot(bound <= Threshold(low, group).at(post_layer));
       } else {
         const int parts = reach.count_b | reach.count_p << 15 | (int)reach.post << 30 | (int)((unsigned)reach.pp << 31);
@@ -2787,7 +2845,8 @@ __device__ __forceinline__ void reduce_item(const MistProblem &prob, const MistG
   const int L = prob.num_layers, lane = threadIdx.x & 63;
   const int P = g->num_p, n_slots = slots_of(P);
   const GroupModel m = group_model(prob, g);
-  const double cutoff = stage_cost_cutoff(prob, m.inv_G64);
+  const CostLimits limits = cost_limits(prob, tabs, gi, m.inv_G64);
+  const double cutoff = limits.cutoff;
   const int64_t tile_cell = g->cell_offset + (int64_t)tile_rel * MIST_LC_TILE * n_slots;
   const double *best = tabs.best + tile_cell;  // [pair][slot]
 
@@ -2805,7 +2864,8 @@ __device__ __forceinline__ void reduce_item(const MistProblem &prob, const MistG
     const StageReach reach = stage_reach(f, pair_consts(tl.pc.l, tl.pc.c), tl.np, tl.do_post, tl.do_pp, m);
     const double bound = m.bound(ratio, reach.x, reach.d);
     const Loosest low = loosest_minima((pairs >> lane & 1ull) != 0 && bound <= cutoff, best + lane * n_slots, 1, P,
-                                       reach.count_b, reach.count_p, reach.post, reach.pp, cutoff);
+                                       reach.count_b, reach.count_p, reach.post, reach.pp, cutoff,
+                                       limits.closed_below(tl.pc.l));
     const Offsets off = group_offsets(m, ratio);
     const Threshold its(low, off);
     const double post_layer = post_layer_offset(m, ratio, f);
@@ -2927,8 +2987,9 @@ __device__ __forceinline__ void reduce_item(const MistProblem &prob, const MistG
       const LinearReach reach = linear_reach(mem, p, m, p.c == p.l - 1 ? min(P, 1) : P, cap_and_room);
       auto minimum = [&](int slot) { return kInLds ? lds_row[slot] : best[(int64_t)pl * n_slots + slot]; };
       const double now_b = minimum(max(reach.count_b - 1, 0)), now_p = minimum(P + max(reach.count_p - 1, 0));
-      bool may = (reach.count_b > 0 && low <= fmin(now_b, cutoff)) ||
-                 (reach.count_p > 0 && low <= fmin(now_p, cutoff) - off_pre);
+      const double closed_below = limits.closed_below(p.l);
+      bool may = (reach.count_b > 0 && low <= up_to(now_b, cutoff, closed_below)) ||
+                 (reach.count_p > 0 && low <= up_to(now_p, cutoff, closed_below) - off_pre);
       const bool may_post = low <= from_lane(thr_post, pl);
       if (__any(may_post)) may = may || (may_post && post_may_fit(reach, mem, p, L, m, cap_and_room));  // a pair in seven
       const uint64_t found = live & __ballot(may && low <= from_lane(thr, pl));
@@ -3509,6 +3570,57 @@ struct PipelineLayers {
   __device__ __forceinline__ int end(int stage) const { return (stage + 1) * each + min(stage, extra) - 1; }  // last layer
 };
 
+// What a group's stage costs can be used for, from the bounds of its rows and of the other meshes' of its table
+// row (neighbours in the list).  The search that reads the tables looks for pipelines of D devices and L layers
+// whose stages cost no more than bound(G).
+//  - A stage of l layers on d devices leaves L - l layers to D - d devices.  Some stage among those has at least
+//    its share of them, and no mesh takes more than `load` layers a device at a cost up to bound(G): what leaves
+//    more is in no such pipeline, and no stage of the table row is if all layers are more than D devices take.
+//  - The most expensive stage of every pipeline costs at least what the cheapest mesh takes for its share of all
+//    layers.  That search reads stage costs as threshold candidates from kCandidateRoom below the smallest largest
+//    cost on: of what is in no pipeline, a minimum below that is as good as any other value below it.
+// So a pair of fewer than `first` layers is left alone once its minimum is below `low`: 70 - 80 % of the pairs with
+// a minimum up to bound(G) on clusters of a power of two of nodes, 33 - 65 % on others (a mesh of all devices is
+// used with all layers only, one of half of them with close to half).  Calls, us: 7B on 4x8 1180 -> 1065, 13B on
+// 8x8 1920 -> 1615, 22B on 16x8 9000 -> 7190, 70B on 32x8 5720 -> 4290, 1.3B on 1x2 the same.  (Closed in the seeds
+// already, by about the same from the first estimate: they spend their time on the first rows of a pair; 70B 4290
+// -> 4230, 13B uniform-device-pp 1470 -> 1600.)
+// (Where a row may cost less the more layers it has - a negative share of the first micro-batch - nothing is closed.)
+// The workgroup `reach` is formed by; all its threads.
+struct ReachBounds {
+  double per_layer, rest;
+  int row, devices;
+};
+__device__ __forceinline__ void form_reach(const MistProblem &prob, const MistGroupDesc *__restrict__ groups, int n_groups,
+                                           ReachBounds *bounds, GroupReach *reach) {
+  const double L = (double)prob.num_layers, D = (double)prob.incumbent_num_devices;
+  const double incumbent = load_at_agent(prob.stage_cost_incumbent);
+  for (int i = threadIdx.x; i < n_groups; i += blockDim.x)
+    bounds[i] = ReachBounds{load_at_agent(&reach[i].per_layer), load_at_agent(&reach[i].rest), groups[i].g_index,
+                            groups[i].num_nodes * groups[i].num_gpus_per_node};
+  __syncthreads();
+  for (int gi = threadIdx.x; gi < n_groups; gi += blockDim.x) {
+    const double bound = incumbent * (1.0 / (double)groups[gi].grad_accum) * (1.0 + kIncumbentSlack);
+    double load = 0.0, cheapest = INFINITY;  // layers a device takes at most, the smallest largest stage cost
+    auto add = [&](const ReachBounds &r) {
+      const double d = (double)r.devices, share = ceil(L * d / D - 1e-9);
+      if (!(r.per_layer > 0.0)) {
+        load = L;
+        cheapest = -INFINITY;
+        return;
+      }
+      if (r.rest <= bound) load = fmax(load, fmin(L, floor((bound - r.rest) / r.per_layer * (1.0 + 1e-9)) + 2.0) / d);
+      cheapest = fmin(cheapest, r.rest + fmax(share - 2.0, 0.0) * r.per_layer);
+    };
+    const int row = bounds[gi].row;
+    for (int i = gi; i >= 0 && bounds[i].row == row; --i) add(bounds[i]);
+    for (int i = gi + 1; i < n_groups && bounds[i].row == row; ++i) add(bounds[i]);
+    reach[gi].cutoff = load * D * (1.0 + 1e-9) < L ? -INFINITY : bound;
+    reach[gi].first = (int)fmax(ceil(L - load * (D - (double)bounds[gi].devices) * (1.0 + 1e-9)), 0.0);
+    reach[gi].low = cheapest * (1.0 - 1e-6) - kCandidateRoom * (1e-4 + 1e-5 * fabs(cheapest));
+  }
+}
+
 // Cost of the best pipeline of equal stages on equal meshes that the seeds allow
 // (sample 0 of a call with one sample, whose objective is the stage cost): group (G, mesh (n, m))
 // offers S = devices / (n m) stages of about L / S layers each, the first one from the with_pre table
@@ -3520,16 +3632,30 @@ struct PipelineLayers {
 // them returns no more than this unless its scan never tries the thresholds of that pipeline
 // (a single-stage cost is no threshold candidate of the reference, and its gap rule drops
 // some), which is why the caller checks its result against the bound that was used.
-// Workgroup = group, its wavefronts take the stages in turn; lowers *incumbent.
+// Workgroup = group, its wavefronts take the stages in turn; lowers *incumbent.  With MistProblem.incumbent_close
+// the last workgroup to end forms the records of all groups.
 constexpr int kIncumbentWaves = 4;
 __global__ __launch_bounds__(64 * kIncumbentWaves) void incumbent_kernel(
     const MistProblem prob, const MistGroupDesc *__restrict__ groups, const ReduceTables tabs) {
   const MistGroupDesc *g = groups + blockIdx.x;
-  if (g->scout_stride <= 0) return;
-  const int L = prob.num_layers;
-  const int S = incumbent_stage_count(prob, g);
-  if (S == 0) return;
-  const PipelineLayers layers(L, S);
+  const int L = prob.num_layers, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const bool close = prob.incumbent_close != 0;
+  if (close && wave == 0) {
+    static_assert(kSuperBlocks == 64, "a lane per workgroup of the summaries");
+    const double *parts = tabs.reach_parts + ((int64_t)blockIdx.x * kSuperBlocks + lane) * 2;
+    double per_layer = parts[0], rest = parts[1];
+    for (int step = 32; step > 0; step >>= 1) {
+      per_layer = fmin(per_layer, __shfl_xor(per_layer, step));
+      rest = fmin(rest, __shfl_xor(rest, step));
+    }
+    if (lane == 0) {
+      __hip_atomic_store(&tabs.reach[blockIdx.x].per_layer, per_layer, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(&tabs.reach[blockIdx.x].rest, rest, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+  const int S = g->scout_stride > 0 ? incumbent_stage_count(prob, g) : 0;
+  if (S == 0 && !close) return;
+  const PipelineLayers layers(L, max(S, 1));
   const int P = g->num_p;
   // seed of a stage's (l, c) cell in slot `slot` (one sample; +inf where there is none)
   auto seed_of = [&](int slot, int l, int c) {
@@ -3550,7 +3676,6 @@ __global__ __launch_bounds__(64 * kIncumbentWaves) void incumbent_kernel(
     return prob.incumbent_ckpt_rule == 0 ? min(l, L - end_layer) : l;
   };
   __shared__ double wave_sum[kIncumbentWaves], wave_largest[kIncumbentWaves];
-  const int wave = threadIdx.x >> 6;
   double sum = 0.0, largest = 0.0;
   for (int s = wave; s < S; s += kIncumbentWaves) {
     const int p = S - 1 - s, l = layers.of(s);
@@ -3564,7 +3689,7 @@ __global__ __launch_bounds__(64 * kIncumbentWaves) void incumbent_kernel(
     sum += cost;
     largest = fmax(largest, cost);
   }
-  if ((threadIdx.x & 63) == 0) {
+  if (lane == 0) {
     wave_sum[wave] = sum;
     wave_largest[wave] = largest;
   }
@@ -3577,9 +3702,19 @@ __global__ __launch_bounds__(64 * kIncumbentWaves) void incumbent_kernel(
   }
   const double total = sum + (double)(g->grad_accum - 1) * largest;
   // (a pipeline's cost, unlike an objective of another alpha, is not negative: its bits order)
-  if (threadIdx.x == 0 && total >= 0.0 && total < INFINITY)
+  if (threadIdx.x == 0 && S > 0 && total >= 0.0 && total < INFINITY)
     atomicMin(reinterpret_cast<unsigned long long *>(prob.stage_cost_incumbent),
               (unsigned long long)__double_as_longlong(total));
+  if (!close) return;
+  __shared__ bool last;
+  __threadfence();
+  if (threadIdx.x == 0)
+    last = atomicAdd(tabs.counter + kGroupsDone * kCounterPitch, 1u) == gridDim.x - 1;
+  __syncthreads();
+  if (!last) return;
+  __threadfence();
+  extern __shared__ double lds_bounds[];
+  form_reach(prob, groups, gridDim.x, reinterpret_cast<ReachBounds *>(lds_bounds), tabs.reach);
 }
 
 // First estimate of the same pipeline cost, formed before the seeds so that the seed launch
@@ -4103,6 +4238,8 @@ int check_common(const void *d_problem, const void *d_groups, int n_groups) {
       return fail(MIST_E_INVALID, "stage-cost incumbent with %d devices, ckpt rule %d",
                   problem->incumbent_num_devices, problem->incumbent_ckpt_rule);
   }
+  if (problem->incumbent_close != 0 && problem->stage_cost_incumbent == nullptr)
+    return fail(MIST_E_INVALID, "incumbent_close without a stage-cost incumbent");
   return 0;
 }
 
@@ -4194,9 +4331,9 @@ int64_t mist_stage_floor_doubles(int64_t total_rows, int n_groups) {
 
 // Sections of the reduce workspace in `d_partial_cost` (doubles): the minima of n_samples samples,
 // the second-level summaries, the four lists, their counters, a word per stage, the bounds of the gathered
-// rows, the log and its chunks' counts.
+// rows, a record per group, the log and its chunks' counts.
 struct WorkspaceLayout {
-  int64_t best, supers, items, counters, flags, gathered, log, log_counts, total;
+  int64_t best, supers, items, counters, flags, gathered, reach, log, log_counts, total;
   int64_t capacity;    // items per shard
   int64_t log_chunks;
 };
@@ -4209,7 +4346,9 @@ static WorkspaceLayout workspace_layout(int64_t cells, int64_t supers, int64_t i
   w.counters = w.items + 4 * kQueueShards * w.capacity;
   w.flags = w.counters + kCounters * kCounterPitch / 2;
   w.gathered = w.flags + supers * kSuperStages / 2;
-  w.log = w.gathered + supers * kSuperStages * kGatherFloor;  // (a batch of samples may end with one alone)
+  w.reach = w.gathered + supers * kSuperStages * kGatherFloor;  // (a batch of samples may end with one alone)
+  // (two second-level summaries a group at least)
+  w.log = w.reach + supers / 2 * (int64_t)(sizeof(GroupReach) / 8 + 2 * kSuperBlocks);
   w.log += w.log % 2;
   // (a chunk of every wavefront's is as a rule not full)
   w.log_chunks = std::min(kLogPerCell * cells * n_samples, kLogEntries) / kLogChunk + kReduceBlocks * (kReduceThreads / 64);
@@ -4249,6 +4388,8 @@ static int reduce_tables(const MistProblem *problem, int n_samples, double *d_pa
   out->log_count = reinterpret_cast<uint32_t *>(d_partial_cost + w.log_counts);
   out->log_chunks = log_chunks(w.log_chunks, problem->reduce_cells * n_samples);
   out->gather_floor = d_partial_cost + w.gathered;
+  out->reach = reinterpret_cast<GroupReach *>(d_partial_cost + w.reach);
+  out->reach_parts = d_partial_cost + w.reach + problem->reduce_supers / 2 * (int64_t)(sizeof(GroupReach) / 8);
   out->capacity = (uint32_t)w.capacity;
   out->n_samples = n_samples;
   return 0;
@@ -4291,10 +4432,10 @@ static int allow_large_lds() {
 }
 
 // Minima tables filled with what the rows of the scout pairs give (+inf where a group has none and
-// with `scouted` false), and the estimate of the best pipeline cost they allow.
+// with `scouted` false).  *seeded: whether launch_incumbent has something to read.
 static int launch_seeds(const MistProblem *problem, const MistGroupDesc *d_groups, int n_groups,
                         const double *d_row_terms, const RatioList &ratios, bool scouted,
-                        const ReduceTables &tabs, double *d_partial_cost, void *stream) {
+                        const ReduceTables &tabs, double *d_partial_cost, bool *seeded, void *stream) {
   const int L = problem->num_layers, n_pairs = L * (L + 1) / 2 + L;
   const int tiles = (n_pairs + MIST_LC_TILE - 1) / MIST_LC_TILE;
   if (tiles > 1 << kItemTileBits)
@@ -4314,6 +4455,7 @@ static int launch_seeds(const MistProblem *problem, const MistGroupDesc *d_group
   while (sample_waves > 1 && pair_bytes + sample_waves * (int64_t)sizeof(SampleRows) > kSeedLdsMost) sample_waves /= 2;
   const int64_t bytes = pair_bytes * pair_split * sample_split + sample_waves * (int64_t)sizeof(SampleRows);
   const bool seeds = scouted && bytes <= kSeedLdsMost;  // (some 10000 values of p)
+  *seeded = seeds;
   const bool estimate = scouted && problem->stage_cost_incumbent != nullptr && problem->incumbent_first_estimate != 0 &&
                         tabs.n_samples == 1;
   // a first estimate from a few rows, so that the seed launch itself runs under a bound
@@ -4343,18 +4485,29 @@ static int launch_seeds(const MistProblem *problem, const MistGroupDesc *d_group
     hipLaunchKernelGGL(seed_samples_kernel, grid, dim3(64 * sample_waves), (size_t)bytes, (hipStream_t)stream, *problem, d_groups,
                        d_row_terms, ratios, tabs, sample_split);
   MIST_HIP_CHECK(hipGetLastError());
-  if (scouted && problem->stage_cost_incumbent != nullptr && tabs.n_samples == 1) {
-    hipLaunchKernelGGL(incumbent_kernel, dim3(n_groups), dim3(64 * kIncumbentWaves), 0, (hipStream_t)stream, *problem,
-                       d_groups, tabs);
-    MIST_HIP_CHECK(hipGetLastError());
-  }
   return 0;
 }
 
-static int launch_super_floors(const MistGroupDesc *d_groups, int n_groups, const double *d_stage_floor,
-                               const ReduceTables &tabs, void *stream) {
+// The estimate of the best pipeline cost that the seeds allow, and with MistProblem.incumbent_close what it and
+// the second-level summaries say of every group (no seeds: nothing is closed).
+static int launch_incumbent(MistProblem *problem, const MistGroupDesc *d_groups, int n_groups, bool seeded,
+                            const ReduceTables &tabs, void *stream) {
+  if (!seeded || problem->stage_cost_incumbent == nullptr || tabs.n_samples != 1) {
+    problem->incumbent_close = 0;
+    return 0;
+  }
+  if (n_groups > kReachGroups) problem->incumbent_close = 0;
+  hipLaunchKernelGGL(incumbent_kernel, dim3(n_groups), dim3(64 * kIncumbentWaves),
+                     problem->incumbent_close != 0 ? n_groups * sizeof(ReachBounds) : 0, (hipStream_t)stream, *problem, d_groups,
+                     tabs);
+  MIST_HIP_CHECK(hipGetLastError());
+  return 0;
+}
+
+static int launch_super_floors(const MistProblem *problem, const MistGroupDesc *d_groups, int n_groups,
+                               const double *d_stage_floor, double ratio, const ReduceTables &tabs, void *stream) {
   hipLaunchKernelGGL(super_floor_kernel, dim3(kSuperBlocks, n_groups), dim3(256), 0, (hipStream_t)stream, d_groups,
-                     n_groups, d_stage_floor, tabs);
+                     n_groups, d_stage_floor, ratio, problem->incumbent_close != 0, tabs);
   MIST_HIP_CHECK(hipGetLastError());
   return 0;
 }
@@ -4431,11 +4584,14 @@ int mist_eval_reduce(const MistProblem *problem, const MistGroupDesc *d_groups, 
   ratios.r[0] = ratio;
   ReduceTables tabs;
   if (int rc = reduce_tables(problem, 1, d_partial_cost, d_partial_index, &tabs)) return rc;
+  MistProblem own = *problem;
+  bool seeded = false;
   if (int rc = launch_seeds(problem, d_groups, n_groups, d_row_terms, ratios, n_scout_blocks > 0, tabs, d_partial_cost,
-                            stream))
+                            &seeded, stream))
     return rc;
-  if (int rc = launch_super_floors(d_groups, n_groups, d_stage_floor, tabs, stream)) return rc;
-  return launch_reduce(problem, d_groups, n_groups, d_block_prefix, n_blocks, d_row_terms, d_stage_floor, nullptr, ratios, tabs,
+  if (int rc = launch_super_floors(problem, d_groups, n_groups, d_stage_floor, ratio, tabs, stream)) return rc;
+  if (int rc = launch_incumbent(&own, d_groups, n_groups, seeded, tabs, stream)) return rc;
+  return launch_reduce(&own, d_groups, n_groups, d_block_prefix, n_blocks, d_row_terms, d_stage_floor, nullptr, ratios, tabs,
                        stream);
 }
 
@@ -4510,11 +4666,14 @@ int mist_eval_reduce_samples(const MistProblem *problem, const MistGroupDesc *d_
     for (int i = 0; i < count; ++i) list.r[i] = ratios[first + i];
     ReduceTables tabs;
     if (int rc = reduce_tables(problem, count, d_partial_cost, d_partial_index, &tabs)) return rc;
+    MistProblem own = *problem;
+    bool seeded = false;
     if (int rc = launch_seeds(problem, d_groups, n_groups, d_row_terms, list, n_scout_blocks > 0, tabs, d_partial_cost,
-                              stream))
+                              &seeded, stream))
       return rc;
-    if (int rc = launch_super_floors(d_groups, n_groups, d_stage_floor, tabs, stream)) return rc;
-    if (int rc = launch_reduce(problem, d_groups, n_groups, d_block_prefix, n_blocks, d_row_terms, d_stage_floor, nullptr,
+    if (int rc = launch_super_floors(problem, d_groups, n_groups, d_stage_floor, list.r[0], tabs, stream)) return rc;
+    if (int rc = launch_incumbent(&own, d_groups, n_groups, seeded, tabs, stream)) return rc;
+    if (int rc = launch_reduce(&own, d_groups, n_groups, d_block_prefix, n_blocks, d_row_terms, d_stage_floor, nullptr,
                                list, tabs, stream))
       return rc;
     if (int rc = launch_finalize(problem, d_groups, n_groups, d_row_terms, tabs, sample_index + first, tables, stream))
@@ -4653,14 +4812,17 @@ int mist_intra_stage_eval_samples(const MistProblem *problem, const MistGroupDes
     RatioList list = {};
     for (int i = 0; i < count; ++i) list.r[i] = ratios[first + i];
     const bool aside = overlap && first == 0;
+    MistProblem own = *problem;
+    bool seeded = false;
     if (int rc = launch_seeds(problem, d_groups, n_groups, d_row_terms, list, n_scout_blocks > 0, tabs, d_partial_cost,
-                              aside ? (void *)os->side : stream))
+                              &seeded, aside ? (void *)os->side : stream))
       return rc;
     if (aside) MIST_HIP_CHECK(hipEventRecord(os->seeds_done, os->side));
     // (the summaries' place depends on the number of samples)
-    if (int rc = launch_super_floors(d_groups, n_groups, d_stage_floor, tabs, stream)) return rc;
+    if (int rc = launch_super_floors(problem, d_groups, n_groups, d_stage_floor, list.r[0], tabs, stream)) return rc;
     if (aside) MIST_HIP_CHECK(hipStreamWaitEvent(main_stream, os->seeds_done, 0));
-    if (int rc = launch_reduce(problem, d_groups, n_groups, d_reduce_block_prefix, n_reduce_blocks, d_row_terms,
+    if (int rc = launch_incumbent(&own, d_groups, n_groups, seeded, tabs, stream)) return rc;
+    if (int rc = launch_reduce(&own, d_groups, n_groups, d_reduce_block_prefix, n_reduce_blocks, d_row_terms,
                                d_stage_floor, d_key_terms, list, tabs, stream))
       return rc;
     if (int rc = launch_finalize(problem, d_groups, n_groups, d_row_terms, tabs, sample_index + first, tables, stream))

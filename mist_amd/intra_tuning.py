@@ -992,7 +992,8 @@ class IntraStageTuner:
         whose inter-stage search is all that reads the tables: the scout pass turns its seeds
         into an upper bound of the best pipeline cost (``MistProblem.stage_cost_incumbent``),
         and the launches behind it do not look for stage costs that no threshold of that search can
-        admit.  Cells above that bound then hold some value above it, not their minimum.
+        admit.  Cells above that bound then hold some value above it, not their minimum.  With ``close_unused``
+        cells that are in no pipeline below it are not looked for either (``MistProblem.incumbent_close``).
 
         ``fill_costs`` False is for a caller that reads the costs of cells with a row index only:
         the tables are not pre-filled with +inf.
@@ -1004,7 +1005,7 @@ class IntraStageTuner:
         problem = plan["problem"]
         sparse = sparse and self.table_samples == 1 and self.cells_wanted is None and self.num_layers <= 255
         problem["sparse_tables"] = sparse
-        problem["stage_cost_incumbent"] = 0
+        problem["stage_cost_incumbent"] = problem["incumbent_close"] = 0
         if stage_cost_cutoff is not None and self.sample_size == 1 and not self.exhaustive:
             with torch.cuda.device(self.device):
                 if "incumbent" not in dev_plan:
@@ -1013,6 +1014,9 @@ class IntraStageTuner:
             problem["stage_cost_incumbent"] = dev_plan["incumbent"].data_ptr()
             problem["incumbent_num_devices"] = int(stage_cost_cutoff["num_devices"])
             problem["incumbent_ckpt_rule"] = int(stage_cost_cutoff["ckpt_rule"])
+            # (all meshes of a table row in one call, side by side)
+            problem["incumbent_close"] = (stage_cost_cutoff.get("close_unused", False) and len(dev_plan["batches"]) == 1
+                                          and bool(np.all(np.diff(plan["groups"]["g_index"]) >= 0)))
         with torch.cuda.device(self.device):
             costs, index, struct = self._allocate_flat(plan, fill_costs and not sparse, not sparse)
             self.launch(plan, dev_plan, struct)

@@ -196,10 +196,10 @@ class PreparedSearch:
         if sample_size == 1 and not exhaustive and os.environ.get("MIST_NO_STAGE_COST_CUTOFF") is None:
             devices = hw.num_nodes * hw.num_gpus_per_node
             if self.granularity == "inter-stage":
-                self.stage_cost_cutoff = dict(num_devices=devices, ckpt_rule=0)
+                self.stage_cost_cutoff = dict(num_devices=devices, ckpt_rule=0, close_unused=True)
             elif self.granularity == "uniform-device-pp":
                 rule = 1 if tuning.activation_checkpointing_tuning_enabled else 2
-                self.stage_cost_cutoff = dict(num_devices=devices, ckpt_rule=rule)
+                self.stage_cost_cutoff = dict(num_devices=devices, ckpt_rule=rule, close_unused=True)
 
     def counts(self) -> Dict[str, int]:
         """Search-space sizes: strategy rows, candidates = rows * (L + 1), base-variant cells

@@ -1,0 +1,80 @@
+"""Cells that are in no pipeline below the limit are not looked for: the search over such tables returns what it
+returns over complete ones."""
+import numpy as np
+import pytest
+
+from tests.test_gpu_inter import _realistic_plan
+from tests.util import load_plan
+
+pytestmark = pytest.mark.gpu
+
+
+def _compare(cfg, monkeypatch=None):
+    from mist_amd.tune_one_case import PreparedSearch
+
+    search = PreparedSearch(cfg)
+    assert search.stage_cost_cutoff["close_unused"]
+    got = search.run()
+    closed = search.tuner.run_prepared(search.plan, search.dev_plan, search.stage_cost_cutoff)[0].batch
+    without = dict(search.stage_cost_cutoff, close_unused=False)
+    open_ = search.tuner.run_prepared(search.plan, search.dev_plan, without)[0].batch
+    n_closed = n_open = 0
+    for v in range(4):
+        has, had = closed.index[v] >= 0, open_.index[v] >= 0
+        # whatever a closed table holds is the cost of a row, no smaller than the minimum
+        assert bool((closed.stable[v][has & had] + closed.delta[v][has & had] >= 0).all())
+        n_closed, n_open = n_closed + int(has.sum()), n_open + int(had.sum())
+    search.stage_cost_cutoff = None
+    assert search.run() == got
+    return n_closed, n_open
+
+
+@pytest.mark.parametrize("plan, layers, nodes, batch, device", [
+    (2, 32, 4, 512, False),   # the 7B plan
+    (3, 37, 4, 256, True),    # uniform-device-pp, odd layers
+    (3, 23, 5, 256, False),   # five nodes: no mesh of all devices
+    (4, 20, 3, 768, False),
+    (3, 9, 8, 512, False),    # fewer layers than stages of the smallest meshes
+])
+def test_search_over_tables_with_closed_cells(plan, layers, nodes, batch, device):
+    overrides = dict(tuning__tuning_granularity="uniform-device-pp") if device else {}
+    n_closed, n_open = _compare(load_plan(plan, model__num_hidden_layers=layers, hardware__num_nodes=nodes,
+                                          training__global_batch_size=batch, **overrides)[0])
+    assert n_closed < n_open
+
+
+@pytest.mark.parametrize("seed", range(300000, 300030))
+def test_random_plans_with_closed_cells(seed):
+    _compare(_realistic_plan(seed))
+
+
+@pytest.mark.parametrize("dense", [False, True])
+def test_windows_that_reach_below_what_such_tables_hold(dense):
+    """A window whose threshold candidates have no certain start within two widenings (values half a gap apart, in
+    cells of a mesh of all devices that no pipeline uses) leaves the search undecided."""
+    import torch
+
+    from mist_amd import _lib, inter_tuning
+    from tests.test_gpu_inter import _synthetic_results
+
+    L, D, Gs, meshes = 20, 16, [2], [(1, 1), (1, 2), (1, 4), (2, 4), (4, 4)]
+    (ours,), _ = _synthetic_results(np.random.default_rng(5), 1, Gs, meshes, L, 16, 1, 1 / 256, 0.1, structured=True,
+                                    structured_exponent=1.0, jitter=0.0)
+    runner = inter_tuning._DpRunner(ours, L, D, meshes, 0)
+    _, bottleneck, _ = runner.run(np.zeros(1, np.int32), np.zeros(1, np.float32), _lib.DP_BOTTLENECK)
+    tables = ours.device
+    if dense:
+        cells = [(p, l, c) for p in range(16) for l in range(2, L - 1) for c in range(l + 1) if c != l - 1 or p == 0]
+        where = torch.tensor(cells, device="cuda").T
+        values = float(bottleneck[0]) - 9e-7 * torch.arange(1, 2 * len(cells) + 1, device="cuda", dtype=torch.float64)
+        # further than sixteen times the first margin
+        assert 9e-7 * len(values) > 16 * (1e-4 + 1e-5 * float(bottleneck[0])) * 1.1
+        for v in range(2):  # base and with_pre
+            at = (0, 4, where[0], where[1] - 1, where[2], 0)
+            tables.stable[v][at], tables.delta[v][at] = values[v::2], 0.0
+            tables.index[v][at] = 0
+    limit = torch.full((1,), 1e3, dtype=torch.float64).pin_memory()
+    stats = {}
+    inter_tuning.inter_stage_tune_batch(L, D, meshes, Gs, [ours], slot=0, stats=stats, only_best_solution=True,
+                                        table_limit=(limit, 1.0))
+    assert (stats["dp_undecided"] > 0) == dense
