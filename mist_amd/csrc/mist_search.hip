@@ -3978,10 +3978,13 @@ __global__ __launch_bounds__(256) void finalize_kernel(
       const int64_t cell = first + (int64_t)pair * n_slots + p;
       double cost = INFINITY;
       uint32_t row = ~0u;
-      if (p < np) {
-        cost = tabs.best[cell];
-        row = tabs.row[cell];
+      if (p < np) row = tabs.row[cell];
+      // (no row at or above these slots: a minimum without one was not looked for)
+      if (!__any(row != ~0u || carry_row[pair] != ~0u)) {
+        winner[pair][j] = ~0u;
+        continue;
       }
+      if (p < np) cost = tabs.best[cell];
       for (int step = 1; step < kFinalSlots; step <<= 1) {
         const double its_cost = __shfl_down(cost, step, kFinalSlots);
         const uint32_t its_row = __shfl_down(row, step, kFinalSlots);
@@ -4431,11 +4434,35 @@ static int allow_large_lds() {
   return 0;
 }
 
+// The problem as the launches of one call take it: whether cells are closed is decided here.  For few (tile, stage)
+// items it does not pay: the estimate then waits for the summaries, too, 10 - 18 us of 342 to 10230 items; from 23520
+// on calls get faster, by 10 - 50 us up to 100000, then more.
+constexpr int64_t kCloseItems = 20000;
+static MistProblem closing(const MistProblem *problem, int n_groups, int n_samples) {
+  MistProblem own = *problem;
+  if (own.stage_cost_incumbent == nullptr || n_samples != 1 || n_groups > kReachGroups || own.reduce_items < kCloseItems)
+    own.incumbent_close = 0;
+  return own;
+}
+
+// The estimate of the best pipeline cost that the seeds allow, and with MistProblem.incumbent_close (behind the
+// second-level summaries) what it says of every group.
+static int launch_incumbent(const MistProblem *problem, const MistGroupDesc *d_groups, int n_groups, const ReduceTables &tabs,
+                            void *stream) {
+  if (problem->stage_cost_incumbent == nullptr || tabs.n_samples != 1) return 0;
+  hipLaunchKernelGGL(incumbent_kernel, dim3(n_groups), dim3(64 * kIncumbentWaves),
+                     problem->incumbent_close != 0 ? n_groups * sizeof(ReachBounds) : 0, (hipStream_t)stream, *problem, d_groups,
+                     tabs);
+  MIST_HIP_CHECK(hipGetLastError());
+  return 0;
+}
+
 // Minima tables filled with what the rows of the scout pairs give (+inf where a group has none and
-// with `scouted` false).  *seeded: whether launch_incumbent has something to read.
-static int launch_seeds(const MistProblem *problem, const MistGroupDesc *d_groups, int n_groups,
+// with `scouted` false), and the estimate of the best pipeline cost they allow (with MistProblem.incumbent_close that
+// is left to launch_incumbent; without seeds nothing is closed).
+static int launch_seeds(MistProblem *problem, const MistGroupDesc *d_groups, int n_groups,
                         const double *d_row_terms, const RatioList &ratios, bool scouted,
-                        const ReduceTables &tabs, double *d_partial_cost, bool *seeded, void *stream) {
+                        const ReduceTables &tabs, double *d_partial_cost, void *stream) {
   const int L = problem->num_layers, n_pairs = L * (L + 1) / 2 + L;
   const int tiles = (n_pairs + MIST_LC_TILE - 1) / MIST_LC_TILE;
   if (tiles > 1 << kItemTileBits)
@@ -4455,7 +4482,6 @@ static int launch_seeds(const MistProblem *problem, const MistGroupDesc *d_group
   while (sample_waves > 1 && pair_bytes + sample_waves * (int64_t)sizeof(SampleRows) > kSeedLdsMost) sample_waves /= 2;
   const int64_t bytes = pair_bytes * pair_split * sample_split + sample_waves * (int64_t)sizeof(SampleRows);
   const bool seeds = scouted && bytes <= kSeedLdsMost;  // (some 10000 values of p)
-  *seeded = seeds;
   const bool estimate = scouted && problem->stage_cost_incumbent != nullptr && problem->incumbent_first_estimate != 0 &&
                         tabs.n_samples == 1;
   // a first estimate from a few rows, so that the seed launch itself runs under a bound
@@ -4464,6 +4490,7 @@ static int launch_seeds(const MistProblem *problem, const MistGroupDesc *d_group
                                        seeds ? tabs.gather_floor : nullptr, stream))
       return rc;
   if (!seeds) {
+    problem->incumbent_close = 0;
     hipLaunchKernelGGL(empty_minima_kernel, dim3(kReduceBlocks), dim3(256), 0, (hipStream_t)stream, tabs,
                        problem->reduce_cells);
     MIST_HIP_CHECK(hipGetLastError());
@@ -4485,23 +4512,7 @@ static int launch_seeds(const MistProblem *problem, const MistGroupDesc *d_group
     hipLaunchKernelGGL(seed_samples_kernel, grid, dim3(64 * sample_waves), (size_t)bytes, (hipStream_t)stream, *problem, d_groups,
                        d_row_terms, ratios, tabs, sample_split);
   MIST_HIP_CHECK(hipGetLastError());
-  return 0;
-}
-
-// The estimate of the best pipeline cost that the seeds allow, and with MistProblem.incumbent_close what it and
-// the second-level summaries say of every group (no seeds: nothing is closed).
-static int launch_incumbent(MistProblem *problem, const MistGroupDesc *d_groups, int n_groups, bool seeded,
-                            const ReduceTables &tabs, void *stream) {
-  if (!seeded || problem->stage_cost_incumbent == nullptr || tabs.n_samples != 1) {
-    problem->incumbent_close = 0;
-    return 0;
-  }
-  if (n_groups > kReachGroups) problem->incumbent_close = 0;
-  hipLaunchKernelGGL(incumbent_kernel, dim3(n_groups), dim3(64 * kIncumbentWaves),
-                     problem->incumbent_close != 0 ? n_groups * sizeof(ReachBounds) : 0, (hipStream_t)stream, *problem, d_groups,
-                     tabs);
-  MIST_HIP_CHECK(hipGetLastError());
-  return 0;
+  return problem->incumbent_close != 0 ? 0 : launch_incumbent(problem, d_groups, n_groups, tabs, stream);
 }
 
 static int launch_super_floors(const MistProblem *problem, const MistGroupDesc *d_groups, int n_groups,
@@ -4584,13 +4595,13 @@ int mist_eval_reduce(const MistProblem *problem, const MistGroupDesc *d_groups, 
   ratios.r[0] = ratio;
   ReduceTables tabs;
   if (int rc = reduce_tables(problem, 1, d_partial_cost, d_partial_index, &tabs)) return rc;
-  MistProblem own = *problem;
-  bool seeded = false;
-  if (int rc = launch_seeds(problem, d_groups, n_groups, d_row_terms, ratios, n_scout_blocks > 0, tabs, d_partial_cost,
-                            &seeded, stream))
+  MistProblem own = closing(problem, n_groups, 1);
+  if (int rc = launch_seeds(&own, d_groups, n_groups, d_row_terms, ratios, n_scout_blocks > 0, tabs, d_partial_cost,
+                            stream))
     return rc;
-  if (int rc = launch_super_floors(problem, d_groups, n_groups, d_stage_floor, ratio, tabs, stream)) return rc;
-  if (int rc = launch_incumbent(&own, d_groups, n_groups, seeded, tabs, stream)) return rc;
+  if (int rc = launch_super_floors(&own, d_groups, n_groups, d_stage_floor, ratio, tabs, stream)) return rc;
+  if (own.incumbent_close != 0)
+    if (int rc = launch_incumbent(&own, d_groups, n_groups, tabs, stream)) return rc;
   return launch_reduce(&own, d_groups, n_groups, d_block_prefix, n_blocks, d_row_terms, d_stage_floor, nullptr, ratios, tabs,
                        stream);
 }
@@ -4666,13 +4677,13 @@ int mist_eval_reduce_samples(const MistProblem *problem, const MistGroupDesc *d_
     for (int i = 0; i < count; ++i) list.r[i] = ratios[first + i];
     ReduceTables tabs;
     if (int rc = reduce_tables(problem, count, d_partial_cost, d_partial_index, &tabs)) return rc;
-    MistProblem own = *problem;
-    bool seeded = false;
-    if (int rc = launch_seeds(problem, d_groups, n_groups, d_row_terms, list, n_scout_blocks > 0, tabs, d_partial_cost,
-                              &seeded, stream))
+    MistProblem own = closing(problem, n_groups, count);
+    if (int rc = launch_seeds(&own, d_groups, n_groups, d_row_terms, list, n_scout_blocks > 0, tabs, d_partial_cost,
+                              stream))
       return rc;
-    if (int rc = launch_super_floors(problem, d_groups, n_groups, d_stage_floor, list.r[0], tabs, stream)) return rc;
-    if (int rc = launch_incumbent(&own, d_groups, n_groups, seeded, tabs, stream)) return rc;
+    if (int rc = launch_super_floors(&own, d_groups, n_groups, d_stage_floor, list.r[0], tabs, stream)) return rc;
+    if (own.incumbent_close != 0)
+      if (int rc = launch_incumbent(&own, d_groups, n_groups, tabs, stream)) return rc;
     if (int rc = launch_reduce(&own, d_groups, n_groups, d_block_prefix, n_blocks, d_row_terms, d_stage_floor, nullptr,
                                list, tabs, stream))
       return rc;
@@ -4812,16 +4823,16 @@ int mist_intra_stage_eval_samples(const MistProblem *problem, const MistGroupDes
     RatioList list = {};
     for (int i = 0; i < count; ++i) list.r[i] = ratios[first + i];
     const bool aside = overlap && first == 0;
-    MistProblem own = *problem;
-    bool seeded = false;
-    if (int rc = launch_seeds(problem, d_groups, n_groups, d_row_terms, list, n_scout_blocks > 0, tabs, d_partial_cost,
-                              &seeded, aside ? (void *)os->side : stream))
+    MistProblem own = closing(problem, n_groups, count);
+    if (int rc = launch_seeds(&own, d_groups, n_groups, d_row_terms, list, n_scout_blocks > 0, tabs, d_partial_cost,
+                              aside ? (void *)os->side : stream))
       return rc;
     if (aside) MIST_HIP_CHECK(hipEventRecord(os->seeds_done, os->side));
     // (the summaries' place depends on the number of samples)
-    if (int rc = launch_super_floors(problem, d_groups, n_groups, d_stage_floor, list.r[0], tabs, stream)) return rc;
+    if (int rc = launch_super_floors(&own, d_groups, n_groups, d_stage_floor, list.r[0], tabs, stream)) return rc;
     if (aside) MIST_HIP_CHECK(hipStreamWaitEvent(main_stream, os->seeds_done, 0));
-    if (int rc = launch_incumbent(&own, d_groups, n_groups, seeded, tabs, stream)) return rc;
+    if (own.incumbent_close != 0)
+      if (int rc = launch_incumbent(&own, d_groups, n_groups, tabs, stream)) return rc;
     if (int rc = launch_reduce(&own, d_groups, n_groups, d_reduce_block_prefix, n_reduce_blocks, d_row_terms,
                                d_stage_floor, d_key_terms, list, tabs, stream))
       return rc;
