@@ -1882,7 +1882,7 @@ __device__ __forceinline__ void dp_write_stage(int32_t *at, int end, int n, int 
 template <bool kBottleneck, int kCols>
 __global__ __launch_bounds__(kDpHistoryThreads, 8) void dp_history_kernel(
     const MistDpShape shape, const MistDpCosts tabs, const float *__restrict__ tmax_list,
-    const int32_t *__restrict__ g_list, int n_instances, const int32_t *__restrict__ rates,
+    const int32_t *__restrict__ g_list, int n_instances, const int32_t *__restrict__ rates, const double *estimate,
     float *__restrict__ histories, int32_t *__restrict__ best_s_out, float *__restrict__ best_sum_out,
     float *__restrict__ stage_max_out, int32_t *__restrict__ path_out) {
   extern __shared__ float dp_lds[];
@@ -1913,10 +1913,17 @@ __global__ __launch_bounds__(kDpHistoryThreads, 8) void dp_history_kernel(
       continue;
     }
     const float *__restrict__ relaid = tabs.stage_min + g * tabs.stage_min_g_stride;
-    // the bottleneck DP has no threshold of its own: an upper bound of its answer serves as one
-    const float t_max = kBottleneck
-                            ? fminf(kDpNoThreshold, dp_uniform_mesh_bound(shape, relaid, f, n_f, reached))
-                            : tmax_list[t];
+    // the bottleneck DP has no threshold of its own: an upper bound of its answer serves as one.  (Not where the
+    // tables end a little above the answers: it then takes longer than it saves: 70B on
+    // 32x8 547 -> 412 us, 13B on 8x8 139 -> 53, 7B on 4x8 96 -> 56.)
+    float t_max = kDpNoThreshold;
+    if (!kBottleneck) {
+      t_max = tmax_list[t];
+    } else {
+      if (threadIdx.x == 0) *bound = estimate != nullptr && *estimate < (double)INFINITY;
+      __syncthreads();
+      if (*bound == 0) t_max = fminf(kDpNoThreshold, dp_uniform_mesh_bound(shape, relaid, f, n_f, reached));
+    }
     __syncthreads();  // (the bound was read by every wavefront)
     if (threadIdx.x < 3) {
       reached[threadIdx.x] = 0;
@@ -2937,7 +2944,18 @@ int mist::dp_run_free(const DpFreeRun *runs, int n, const float *d_tmax, const i
   return launch_dp_free(runs, n, d_tmax, d_g_index, n_tmax, mode, stream);
 }
 
-int mist::dp_run(const MistDpShape *shape, const MistDpCosts *costs, const int32_t *d_rates, const float *d_tmax,
+static bool history_possible(const MistDpShape &shape, const MistDpCosts &costs, int mode, int64_t scratch_floats,
+                             const HistoryPlan &plan) {
+  return plan.n_wg > 0 && costs.stage_min != nullptr && plan.floats <= scratch_floats &&
+         plan.lds <= history_lds_limit(mode, (shape.num_devices + 63) / 64);
+}
+bool mist::dp_keeps_paths(const MistDpShape &shape, const MistDpCosts &costs, int n_tmax, int mode, int64_t scratch_floats) {
+  const char *forced = getenv("MIST_DP_FORCE_SCHEDULE");
+  if (forced && *forced) return false;
+  return dp_free_runs(shape) || history_possible(shape, costs, mode, scratch_floats, history_plan(shape, n_tmax));
+}
+
+int mist::dp_run(const MistDpShape *shape, const MistDpCosts *costs, const int32_t *d_rates, const double *estimate, const float *d_tmax,
                  const int32_t *d_g_index, int n_tmax, int mode, int32_t *d_best_s, float *d_best_sum,
                  float *d_stage_max, int32_t *d_argmin, int32_t *d_path, float *d_scratch, int64_t scratch_floats,
                  void *stream) {
@@ -2945,7 +2963,8 @@ int mist::dp_run(const MistDpShape *shape, const MistDpCosts *costs, const int32
                                    d_best_sum, d_stage_max))
     return rc;
   if (!d_scratch) return fail(MIST_E_INVALID, "null scratch pointer");
-  if (d_path && !d_argmin) return fail(MIST_E_INVALID, "d_path needs d_argmin");
+  if (d_path && !d_argmin && !dp_keeps_paths(*shape, *costs, n_tmax, mode, scratch_floats))
+    return fail(MIST_E_INVALID, "d_path needs d_argmin");
   const bool whole_argmin = d_argmin != nullptr && d_path == nullptr;
   const int plane = (shape->num_layers + 1) * (shape->num_devices + 1);
   const bool wide = dp_wide_teams(n_tmax, plane);
@@ -2982,8 +3001,7 @@ int mist::dp_run(const MistDpShape *shape, const MistDpCosts *costs, const int32
     }
     const HistoryPlan plan = history_plan(*shape, n_tmax);
     const int cols = (shape->num_devices + 63) / 64;
-    const bool possible = plan.n_wg > 0 && !whole_argmin && costs->stage_min != nullptr &&
-                          plan.floats <= scratch_floats && plan.lds <= history_lds_limit(mode, cols);
+    const bool possible = !whole_argmin && history_possible(*shape, *costs, mode, scratch_floats, plan);
     if (force_history && !possible)
       return fail(MIST_E_INVALID, "forced history schedule: needs stage_min, consumed devices, D <= 256, no "
                   "back-pointers, %lld scratch floats and %zu B of LDS", (long long)plan.floats, plan.lds);
@@ -2992,7 +3010,7 @@ int mist::dp_run(const MistDpShape *shape, const MistDpCosts *costs, const int32
       const MistDpCosts costs_arg = *costs;
       int n_arg = n_tmax;
       void *args[] = {(void *)&shape_arg, (void *)&costs_arg, &d_tmax, &d_g_index, &n_arg, &d_rates,
-                      &d_scratch, &d_best_s, &d_best_sum, &d_stage_max, &d_path};
+                      &estimate, &d_scratch, &d_best_s, &d_best_sum, &d_stage_max, &d_path};
       MIST_HIP_CHECK(hipLaunchKernel(mode == MIST_DP_BOTTLENECK ? history_kernel<true>(cols)
                                                                 : history_kernel<false>(cols),
                                      dim3(plan.n_wg), dim3(kDpHistoryThreads), args, plan.lds,
@@ -3002,7 +3020,7 @@ int mist::dp_run(const MistDpShape *shape, const MistDpCosts *costs, const int32
     }
   }
   if (d_path) {
-    if (int rc = dp_run(shape, costs, d_rates, d_tmax, d_g_index, n_tmax, mode, d_best_s, d_best_sum,
+    if (int rc = dp_run(shape, costs, d_rates, estimate, d_tmax, d_g_index, n_tmax, mode, d_best_s, d_best_sum,
                         d_stage_max, d_argmin, nullptr, d_scratch, scratch_floats, stream))
       return rc;
     return mist_dp_backtrack(shape, d_argmin, d_best_s, n_tmax, d_path, stream);
@@ -3064,7 +3082,8 @@ int mist_dp_run_sized(const MistDpShape *shape, const MistDpCosts *costs, const 
                       const int32_t *d_g_index, int n_tmax, int mode, int32_t *d_best_s,
                       float *d_best_sum, float *d_stage_max, int32_t *d_argmin, int32_t *d_path,
                       float *d_scratch, int64_t scratch_floats, void *stream) {
-  return mist::dp_run(shape, costs, nullptr, d_tmax, d_g_index, n_tmax, mode, d_best_s, d_best_sum, d_stage_max,
+  if (d_path && !d_argmin) return fail(MIST_E_INVALID, "d_path needs d_argmin");
+  return mist::dp_run(shape, costs, nullptr, nullptr, d_tmax, d_g_index, n_tmax, mode, d_best_s, d_best_sum, d_stage_max,
                       d_argmin, d_path, d_scratch, scratch_floats, stream);
 }
 

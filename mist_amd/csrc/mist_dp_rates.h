@@ -15,9 +15,15 @@ constexpr int32_t kRateNone = 0x7f800000;  // +inf
 int dp_stage_rates(const MistDpShape &shape, const MistDpCosts &costs, int n_g, int32_t *d_rates, hipStream_t stream);
 
 // mist_dp_run_sized; `d_rates` (may be null) holds what dp_stage_rates left for every g the instances name.
-int dp_run(const MistDpShape *shape, const MistDpCosts *costs, const int32_t *d_rates, const float *d_tmax,
+// `estimate` (device address, may be null): where it is finite when the kernels run, the tables hold next to nothing
+// above what pipelines cost, and the bottleneck DP looks for no bound of its answer first.  d_path without d_argmin:
+// where dp_keeps_paths.
+int dp_run(const MistDpShape *shape, const MistDpCosts *costs, const int32_t *d_rates, const double *estimate, const float *d_tmax,
            const int32_t *d_g_index, int n_tmax, int mode, int32_t *d_best_s, float *d_best_sum, float *d_stage_max,
            int32_t *d_argmin, int32_t *d_path, float *d_scratch, int64_t scratch_floats, void *stream);
+
+// Whether a run without back-pointers knows the partition of every instance.
+bool dp_keeps_paths(const MistDpShape &shape, const MistDpCosts &costs, int n_tmax, int mode, int64_t scratch_floats);
 
 struct DpFreeRun {
   const MistDpShape *shape;

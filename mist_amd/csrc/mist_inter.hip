@@ -80,6 +80,7 @@ struct Buffer {
   T *as() const { return static_cast<T *>(ptr); }
 };
 
+constexpr int kPathBatches = 6;  // as many keep them: searches have two or three
 struct Workspace {
   Buffer d_in, d_out, d_scratch, d_req, d_counts, d_values, d_request, d_argmin, d_grad;
   Buffer h_in, h_out, h_req, h_counts, h_values, h_request, h_grad;
@@ -87,6 +88,7 @@ struct Workspace {
   // (requests, window descriptions, DP outputs and kept thresholds in one buffer: one copy back)
   Buffer d_win_values, d_win_counts, d_inst_t, d_inst_row, d_first;
   Buffer h_first;
+  Buffer d_paths[kPathBatches];  // partitions of the instances of a search's scan batches
   int select_capacity = 1 << 18;
   Workspace() {
     h_in.pinned = h_out.pinned = h_req.pinned = h_counts.pinned = h_values.pinned =
@@ -191,6 +193,22 @@ __global__ void window_request_kernel(const float *__restrict__ out, int n_famil
 // (end layer, n, m, ckpt), stages[k] of them) reads the row-index table of its variant
 // (inter_tuning.py:38-60: whole model / first stage / last stage / inner stage) at table row
 // g_rows[k], mesh (n, m), pre-saved micro-batches = stages after it.
+__device__ __forceinline__ int32_t strategy_row(const MistStrategyIndex &tabs, const int32_t *__restrict__ path, int n_stages,
+                                                int64_t g, int i) {
+  if (i >= n_stages) return -1;
+  const int32_t *st = path + (size_t)i * 4;
+  const int start = i == 0 ? 0 : st[-4] + 1;
+  const int end = st[0], c = st[3];
+  int q = -1;
+  for (int m = 0; m < tabs.num_mesh; ++m)
+    if (tabs.mesh_n[m] == st[1] && tabs.mesh_m[m] == st[2]) q = m;
+  const int64_t L = tabs.num_layers, C = L + 1, S = tabs.sample_size, Q = tabs.num_mesh;
+  const int64_t l = end - start + 1, p = n_stages - i - 1;
+  if (q < 0 || end < start || end >= L || c < 0 || c > L || p >= tabs.p_dim) return -1;
+  if (start == 0 && end == L - 1) return tabs.index[3][((g * Q + q) * C + c) * S + tabs.slot];
+  if (end == L - 1) return tabs.index[2][(((g * Q + q) * L + (l - 1)) * C + c) * S + tabs.slot];
+  return tabs.index[start == 0 ? 1 : 0][((((g * Q + q) * tabs.p_dim + p) * L + (l - 1)) * C + c) * S + tabs.slot];
+}
 __global__ void strategy_rows_kernel(const MistStrategyIndex tabs, const int32_t *__restrict__ path,
                                      const int32_t *__restrict__ best_s,
                                      const int32_t *__restrict__ g_rows, int n, int max_stages,
@@ -198,28 +216,14 @@ __global__ void strategy_rows_kernel(const MistStrategyIndex tabs, const int32_t
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= n * max_stages) return;
   const int k = e / max_stages, i = e % max_stages;
-  const int n_stages = best_s[k];
-  int32_t row = -1;
-  if (i < n_stages) {
-    const int32_t *st = path + (size_t)e * 4;
-    const int start = i == 0 ? 0 : path[(size_t)(e - 1) * 4] + 1;
-    const int end = st[0], c = st[3];
-    int q = -1;
-    for (int m = 0; m < tabs.num_mesh; ++m)
-      if (tabs.mesh_n[m] == st[1] && tabs.mesh_m[m] == st[2]) q = m;
-    const int64_t L = tabs.num_layers, C = L + 1, S = tabs.sample_size, Q = tabs.num_mesh;
-    const int64_t g = g_rows[k], l = end - start + 1, p = n_stages - i - 1;
-    if (q >= 0 && end >= start && end < L && c >= 0 && c <= L && p < tabs.p_dim) {
-      if (start == 0 && end == L - 1)
-        row = tabs.index[3][((g * Q + q) * C + c) * S + tabs.slot];
-      else if (end == L - 1)
-        row = tabs.index[2][(((g * Q + q) * L + (l - 1)) * C + c) * S + tabs.slot];
-      else
-        row = tabs.index[start == 0 ? 1 : 0]
-                        [((((g * Q + q) * tabs.p_dim + p) * L + (l - 1)) * C + c) * S + tabs.slot];
-    }
-  }
-  out[e] = row;
+  out[e] = strategy_row(tabs, path + (size_t)k * max_stages * 4, best_s[k], g_rows[k], i);
+}
+// The same of one partition that a scan batch left: out[0 .. 4 max_stages) its stages, then their rows.
+__global__ __launch_bounds__(64) void kept_path_kernel(const MistStrategyIndex tabs, bool with_rows, const int32_t *__restrict__ path,
+                                                       int n_stages, int64_t g, int max_stages, int32_t *__restrict__ out) {
+  for (int i = threadIdx.x; i < 4 * max_stages; i += blockDim.x) out[i] = path[i];
+  for (int i = threadIdx.x; with_rows && i < max_stages; i += blockDim.x)
+    out[4 * max_stages + i] = strategy_row(tabs, path, n_stages, g, i);
 }
 
 // Evenly split pipelines: one wavefront per (table row, stage count).  Reads a few hundred cells
@@ -372,6 +376,31 @@ struct Search {
     if (n_families == 1 && stage_limit > 0) shape.max_stages = std::min(shape.max_stages, stage_limit);
     return shape;
   }
+  const double *estimate = nullptr;  // device address of the caller's estimate, if it has one
+  // Where the scan batches leave the partitions of their instances, [batch][family][instance], so that the
+  // winner's needs no run of its own (180 us of 70B on 32x8, 23 of 7B on 4x8).  Searches over tables under an estimate; that over
+  // complete tables runs what the driver without the library runs, run for run.
+  bool keep = false;
+  int n_kept = 0;
+  int batch_instances[kPathBatches] = {};
+  bool keeps(int n) const {
+    for (int f = 0; f < n_families; ++f)
+      if (!mist::dp_keeps_paths(shapes[f], costs[f], n, MIST_DP_THRESHOLD, mist_dp_scratch_floats_sized(&shapes[f], n)))
+        return false;
+    return true;
+  }
+  // the next batch's number, -1 = without partitions
+  int keep_paths(int n) {
+    if (!keep || n_kept == kPathBatches || !keeps(n)) return -1;
+    if (ws->d_paths[n_kept].reserve(sizeof(int32_t) * path_offset(n_families, n)) != 0) return -1;
+    batch_instances[n_kept] = n;
+    return n_kept++;
+  }
+  int32_t *kept_paths(int batch, int f, int slot) const {
+    const int n = batch_instances[batch];
+    return ws->d_paths[batch].as<int32_t>() + path_offset(f, n) + (size_t)slot * path_ints(f);
+  }
+
   size_t path_ints(int f) const { return (size_t)shape_of(f).max_stages * 4; }
   // ints in front of family f's partitions in the path buffers of a batch of n instances
   size_t path_offset(int f, int n) const {
@@ -386,7 +415,7 @@ struct Search {
   // (h_rows, same order without the factor 4).  `sync` false leaves the copies of the
   // outputs queued on the stream for the caller to wait for.
   int run(const std::vector<int32_t> &g_index, const std::vector<float> &tmax, int mode,
-          bool want_path, bool sync = true) {
+          bool want_path, bool sync = true, int path_batch = -1) {
     const int n = (int)tmax.size();
     if (n == 0) return 0;
     const size_t n_out = (size_t)3 * n * n_families;
@@ -427,7 +456,7 @@ struct Search {
     for (int f = 0; f < n_families; ++f) {
       float *d_out = ws->d_out.as<float>() + (size_t)f * 3 * n;
       together.push_back({&its_shapes[f], &costs[f], reinterpret_cast<int32_t *>(d_out), d_out + n, d_out + 2 * n,
-                          want_path ? d_paths + path_offset(f, n) : nullptr});
+                          want_path ? d_paths + path_offset(f, n) : path_batch >= 0 ? kept_paths(path_batch, f, 0) : nullptr});
     }
     const int apart = mist::dp_run_free(together.data(), n_families, d_in, d_g, n, mode, stream);
     if (apart < 0) return apart;
@@ -437,9 +466,9 @@ struct Search {
       float *d_out = ws->d_out.as<float>() + (size_t)f * 3 * n;
       int32_t *d_argmin = want_path ? ws->d_argmin.as<int32_t>() : nullptr;  // no fill: the
                                                      // walk reads what the DP wrote
-      int32_t *d_path = want_path ? d_paths + path_offset(f, n) : nullptr;
+      int32_t *d_path = together[f].d_path;
       const MistDpShape &shape = its_shapes[f];
-      if (int rc = apart == 0 ? 0 : mist::dp_run(&shape, &costs[f], known ? rates_of(f) : nullptr, d_in, d_g, n, mode,
+      if (int rc = apart == 0 ? 0 : mist::dp_run(&shape, &costs[f], known ? rates_of(f) : nullptr, estimate, d_in, d_g, n, mode,
                                 reinterpret_cast<int32_t *>(d_out), d_out + n, d_out + 2 * n, d_argmin,
                                 d_path, ws->d_scratch.as<float>(), n_scratch, stream))
         return rc;
@@ -584,21 +613,22 @@ struct Search {
             reinterpret_cast<int32_t *>(d_first + at_meta), ws->d_inst_t.as<float>(),
             ws->d_inst_row.as<int32_t>(), stream))
       return rc;
+    const int path_batch = keep_paths(n_inst);
     std::vector<mist::DpFreeRun> together;
     for (int f = 0; f < n_families; ++f) {
       float *d_out = d_first + at_out + (size_t)f * 3 * n_inst;
       together.push_back({&shapes[f], &costs[f], reinterpret_cast<int32_t *>(d_out), d_out + n_inst, d_out + 2 * n_inst,
-                          nullptr});
+                          path_batch >= 0 ? kept_paths(path_batch, f, 0) : nullptr});
     }
     const int apart = mist::dp_run_free(together.data(), n_families, ws->d_inst_t.as<float>(),
                                         ws->d_inst_row.as<int32_t>(), n_inst, MIST_DP_THRESHOLD, stream);
     if (apart < 0) return apart;
     for (int f = 0; f < n_families && apart != 0; ++f) {
       float *d_out = d_first + at_out + (size_t)f * 3 * n_inst;
-      if (int rc = mist::dp_run(&shapes[f], &costs[f], rates_of(f), ws->d_inst_t.as<float>(),
+      if (int rc = mist::dp_run(&shapes[f], &costs[f], rates_of(f), estimate, ws->d_inst_t.as<float>(),
                                 ws->d_inst_row.as<int32_t>(), n_inst, MIST_DP_THRESHOLD,
                                 reinterpret_cast<int32_t *>(d_out), d_out + n_inst, d_out + 2 * n_inst,
-                                nullptr, nullptr, ws->d_scratch.as<float>(), n_scratch, stream))
+                                nullptr, together[f].d_path, ws->d_scratch.as<float>(), n_scratch, stream))
         return rc;
     }
     MIST_HIP_CHECK(hipMemcpyAsync(h_first, d_first, sizeof(float) * (at_kept + kKeptHead),
@@ -756,6 +786,7 @@ struct Outcome {
   double cost = kInf;  // total of the DP's partition, inf = infeasible
   double sum = kInf;   // smallest stage-cost sum of a feasible family
   int stages = 0;
+  int family = -1, batch = -1, slot = 0;  // where its partition is kept (batch -1: nowhere)
 };
 struct Scan {
   int G = 1;
@@ -826,6 +857,15 @@ static int search_families(int n_families, const MistDpShape *shapes,
   MIST_HIP_CHECK(hipGetDevice(&device));
   Search S{n_families, shapes, costs, select_costs, strategy, (hipStream_t)stream_,
            &g_workspaces[device]};
+  S.keep = host_estimate != nullptr;
+  // (pageable memory, which the kernels cannot read, is left to the host)
+  if (host_estimate != nullptr) {
+    void *seen = nullptr;
+    if (hipHostGetDevicePointer(&seen, const_cast<double *>(host_estimate), 0) == hipSuccess)
+      S.estimate = static_cast<const double *>(seen);
+    else
+      (void)hipGetLastError();
+  }
   const int n_flat = n_instances * n_grad_accum;
 
   std::vector<int32_t> flat_rows(rows, rows + n_flat);
@@ -1009,6 +1049,7 @@ static int search_families(int n_families, const MistDpShape *shapes,
     double best_cost = kInf;
     int best_g = -1, best_stages = 0;
     float best_t = 0.0f;
+    const Outcome *best = nullptr;  // (of a scan's `known`)
   };
   // Exact part of the caller's tables (a search over tables that hold their values up to
   // limit(G) = estimate * limit_factor / G only): the estimate has arrived with the first round
@@ -1042,7 +1083,9 @@ static int search_families(int n_families, const MistDpShape *shapes,
       const int n_avail = (int)(sc.n_kept() - sc.first);
       for (int k = 0; k < n_first; ++k) {
         Outcome o;
-        o.cost = S.total(at + k, n_flat * kFirstChunk, sc.G, nullptr, S.first_out, &o.stages, &o.sum);
+        o.cost = S.total(at + k, n_flat * kFirstChunk, sc.G, &o.family, S.first_out, &o.stages, &o.sum);
+        o.batch = S.n_kept > 0 ? 0 : -1;
+        o.slot = at + k;
         sc.known[sc.first + (size_t)mist_dp_first_batch_index(k, n_avail, kFirstChunk, kFirstLead)] = o;
       }
       if (n_first > 0) sc.limit = std::min(kMaxChunk, sc.limit * 4);
@@ -1063,7 +1106,7 @@ static int search_families(int n_families, const MistDpShape *shapes,
   };
   // advances the sequential scan as far as the computed results allow; true = this G is done
   auto replay = [&](Scan &sc, double &best_cost, bool &improved, float &best_t,
-                    int &best_stages) -> bool {
+                    const Outcome *&best) -> bool {
     for (;;) {
       if (!reach(sc, sc.pos, best_cost)) return true;
       if (sc.w->scaled[sc.pos] >= std::min(best_cost, sc.cap)) return true;  // inter_tuning.py:196-197
@@ -1077,7 +1120,7 @@ static int search_families(int n_families, const MistDpShape *shapes,
       if (o.cost < best_cost) {
         best_cost = o.cost;
         best_t = sc.w->kept[sc.pos];
-        best_stages = o.stages;
+        best = &o;
         improved = true;
       }
       ++sc.pos;
@@ -1155,13 +1198,14 @@ static int search_families(int n_families, const MistDpShape *shapes,
         Scan &sc = ch.scans[ch.current];
         bool improved = false;
         float best_t = ch.best_t;
-        int best_stages = ch.best_stages;
-        const bool finished = replay(sc, ch.best_cost, improved, best_t, best_stages);
+        const Outcome *best = ch.best;
+        const bool finished = replay(sc, ch.best_cost, improved, best_t, best);
         if (rc_inner) return rc_inner;
         if (improved) {
           ch.best_g = (int)ch.current;
           ch.best_t = best_t;
-          ch.best_stages = best_stages;
+          ch.best = best;
+          ch.best_stages = best->stages;
         }
         if (!finished) break;
         if (bounded) best_after[t * n_grad_accum + (int)ch.current] = ch.best_cost;
@@ -1201,7 +1245,8 @@ static int search_families(int n_families, const MistDpShape *shapes,
           req_t.push_back(limit_t[i % n_grad_accum]);
         }
     if (req_t.empty()) break;  // (nothing feasible anywhere)
-    if (int rc = S.run(req_g, req_t, MIST_DP_THRESHOLD, false)) return rc;
+    const int path_batch = S.keep_paths((int)req_t.size());
+    if (int rc = S.run(req_g, req_t, MIST_DP_THRESHOLD, false, true, path_batch)) return rc;
     const int n = (int)req_t.size();
     for (size_t k = 0; k < limit_of.size(); ++k)
       within_limit[limit_of[k]] = S.total(n_scan_requests + (int)k, n,
@@ -1212,7 +1257,9 @@ static int search_families(int n_families, const MistDpShape *shapes,
       Scan &sc = chains[sp.t].scans[sp.i];
       for (int k = sp.first; k < sp.first + sp.n; ++k) {
         Outcome o;
-        o.cost = S.total(k, n, req_G[k], nullptr, nullptr, &o.stages, &o.sum);
+        o.cost = S.total(k, n, req_G[k], &o.family, nullptr, &o.stages, &o.sum);
+        o.batch = path_batch;
+        o.slot = k;
         sc.known[req_at[k]] = o;
       }
     }
@@ -1254,14 +1301,15 @@ static int search_families(int n_families, const MistDpShape *shapes,
       bool same = (int)open.size() <= kMostDoubtful;
       for (uint32_t found = 1; same && found < 1u << open.size(); ++found) {
         double best_cost = kInf;
-        int best_g = -1, best_stages = 0;
+        int best_g = -1;
         float best_t = 0.0f;
+        const Outcome *best = nullptr;
         size_t next = 0;
         for (int i = 0; same && i < n_grad_accum; ++i) {
           Scan &sc = chains[t].scans[i];
           sc.pos = sc.first;
           bool improved = false;
-          same = replay(sc, best_cost, improved, best_t, best_stages);
+          same = replay(sc, best_cost, improved, best_t, best);
           if (rc_inner) return rc_inner;
           if (improved) best_g = i;
           if (next < open.size() && open[next] == i) {
@@ -1300,7 +1348,38 @@ static int search_families(int n_families, const MistDpShape *shapes,
       if (chains[t].best_cost < chains[best].best_cost) best = t;  // the first of equals stays
     winners.assign(1, best);
   }
-  if (!winners.empty()) {
+  // the partitions that the scan batches left; the others by a run of their own
+  bool kept = !winners.empty();
+  for (int t : winners) kept = kept && chains[t].best->batch >= 0;
+  if (kept) {
+    const size_t per = (size_t)5 * S_max;
+    if (int rc = S.ws->d_out.reserve(sizeof(int32_t) * per * winners.size())) return rc;
+    if (int rc = S.ws->h_out.reserve(sizeof(int32_t) * per * winners.size())) return rc;
+    int32_t *d_out = S.ws->d_out.as<int32_t>();
+    const MistStrategyIndex none = {};
+    for (size_t k = 0; k < winners.size(); ++k) {
+      const Chain &ch = chains[winners[k]];
+      const Outcome &o = *ch.best;
+      hipLaunchKernelGGL(kept_path_kernel, dim3(1), dim3(64), 0, S.stream, strategy ? *strategy : none, strategy != nullptr,
+                         S.kept_paths(o.batch, o.family, o.slot), o.stages,
+                         (int64_t)rows[winners[k] * n_grad_accum + ch.best_g], shapes[o.family].max_stages, d_out + per * k);
+      MIST_HIP_CHECK(hipGetLastError());
+    }
+    MIST_HIP_CHECK(hipMemcpyAsync(S.ws->h_out.ptr, d_out, sizeof(int32_t) * per * winners.size(), hipMemcpyDeviceToHost,
+                                  S.stream));
+    MIST_HIP_CHECK(hipStreamSynchronize(S.stream));
+    ++S.round_trips;
+    for (size_t k = 0; k < winners.size(); ++k) {
+      const int t = winners[k];
+      const Outcome &o = *chains[t].best;
+      const int32_t *back = S.ws->h_out.as<int32_t>() + per * k;
+      const int its_max = shapes[o.family].max_stages;
+      out_family[t] = o.family;
+      out_stages[t] = o.stages;
+      std::memcpy(out_path + (size_t)t * S_max * 4, back, sizeof(int32_t) * 4 * its_max);
+      if (strategy) std::memcpy(out_rows + (size_t)t * S_max, back + 4 * its_max, sizeof(int32_t) * its_max);
+    }
+  } else if (!winners.empty()) {
     std::vector<int32_t> g;
     std::vector<float> tm;
     int most_stages = 0;
