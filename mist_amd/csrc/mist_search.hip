@@ -2045,6 +2045,65 @@ __global__ __launch_bounds__(256) void gather_floor_kernel(const MistProblem pro
   gather_floors(prob, groups + blockIdx.y, blockIdx.y, row_terms, ratio, gather_floor, blockIdx.x, gridDim.x);
 }
 
+// Layers from which on a pair of the group may be in a pipeline below the limit, by about what form_reach will say,
+// from the first estimate alone (the summaries are not there yet).  The pairs below are closed mostly, once their
+// minimum is below about kLikelyLow of the cutoff: what is wrong about that only leaves them higher minima.
+constexpr double kLikelyLow = 0.88;
+__device__ __forceinline__ int likely_first(const MistProblem &prob, const MistGroupDesc *g, double cutoff) {
+  if (prob.incumbent_close == 0 || !(cutoff < INFINITY)) return 0;
+  const float L = (float)prob.num_layers, D = (float)prob.incumbent_num_devices;
+  return (int)(L - 1.05f * L * (D - (float)(g->num_nodes * g->num_gpus_per_node)) / D);
+}
+// First minima of such pairs, for which any row below what closes them does: a few rows of every kind, thread = (row,
+// pair), leave their cost at their own count, then every slot takes the ones above.  The pairs that leaves open
+// go on with all gathered rows.  (Nothing is gained where pairs are left at that: 22B on 16x8 6510 -> 6740 us, with 4
+// instead of 10 ratios 7920; nor by closing alone, the time goes into the first rows of a pair.  With both: 22B
+// 6483 -> 6158, 70B on 32x8 3890 -> 3719, 13B on 8x8 1599 -> 1541, 7B on 4x8 1051 -> 1030, drawn calls 1.1 %.)
+constexpr int kLightTails = 10;  // (activation, optimizer) offload ratios of each parallelism row and offload pair
+__device__ __forceinline__ void light_seeds(const MistProblem &prob, const MistGroupDesc *__restrict__ g,
+                                            const double *__restrict__ src, double ratio, double cutoff, int first_pair,
+                                            int n_here, int pair_split, double *lds_best) {
+  const int L = prob.num_layers, P = g->num_p, n_slots = slots_of(P);
+  const int pair = threadIdx.x % pair_split, n_tail = g->n_oo * g->n_ao;
+  const int tails = min(kLightTails, n_tail), n_rows = g->n_par * tails * g->scout_stride;
+  const GroupModel m = group_model(prob, g);
+  const PairIndex pc = decode_pair(first_pair + min(pair, n_here - 1));
+  const PairConsts k = pair_consts(pc.l, pc.c);
+  const int np = pc.c == pc.l - 1 ? min(P, 1) : P;
+  const bool do_post = pc.c != pc.l - 1, do_pp = do_post && pc.l == L;
+  double *mine = lds_best + pair * n_slots;
+  for (int r = threadIdx.x / pair_split; pair < n_here && r < n_rows; r += kSeedThreads / pair_split) {
+    const int tail = tails > 1 ? r % tails * (n_tail - 1) / (tails - 1) : 0, par = r / tails % g->n_par, which = r / tails / g->n_par;
+    const int q = (which * g->n_par + par) * n_tail + tail;
+    RowRegs t;
+    load_terms<0, MIST_ROW_TERMS>(t, src + gathered_position(g, (uint32_t)q) * MIST_ROW_TERMS);
+    float x, d;
+    pair_latency(t, k, x, d);
+    const LaneMemory mem = pair_memory(t, k);
+    const Objectives o = objectives(t, x, d, k.no_ck, ratio, m, do_post);
+    const UpperCounts upper = upper_counts(mem, m, np);
+    const RowCounts cnt = exact_counts(mem, m, upper.b, upper.p);
+    bool ok_post = false, ok_pp = false;
+    if (do_post) post_fits(t, k, mem, m, mem.out, k.no_ck ? t[MIST_T_RD] : 0.0, ok_post, ok_pp);
+    auto offer = [&](bool ok, double cost, double *slot) {
+      if (ok && cost <= cutoff) lower_minimum_in_lds(slot, cost);
+    };
+    offer(cnt.b > 0, o.base, mine + max(cnt.b - 1, 0));
+    offer(cnt.p > 0, o.pre, mine + P + max(cnt.p - 1, 0));
+    offer(ok_post, o.post, mine + 2 * P);
+    offer(do_pp && ok_pp, o.pp, mine + 2 * P + 1);
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < 2 * pair_split) {
+    double *slots = lds_best + threadIdx.x / 2 * n_slots + (threadIdx.x & 1) * P;
+    double low = INFINITY;
+    for (int p = P - 1; p >= 0; --p) {
+      low = fmin(low, slots[p]);
+      slots[p] = low;
+    }
+  }
+}
+
 // One sample.  Workgroup = (`pair_split` consecutive pairs of a tile, group) with their minima in
 // LDS.  A wavefront takes 64 gathered rows: lane = pair, the smallest of their linear bounds against the
 // pair's loosest minima and the cutoff (of 22B on 16x8's 582000 times 16 pairs 86000 have one left, 0.9e6
@@ -2073,12 +2132,18 @@ __global__ __launch_bounds__(kSeedThreads, 3) void seed_kernel(
   const int n_entries = pair_split * n_slots;  // [pair][slot]
   for (int e = threadIdx.x; e < n_entries; e += kSeedThreads) lds_best[e] = INFINITY;
   __syncthreads();
+  const double most = stage_cost_cutoff(prob, 1.0 / (double)g->grad_accum);
+  const int likely = likely_first(prob, g, most);
+  if (g->scout_stride > 0 && n_here > 0 && decode_pair(first_pair).l < likely) {
+    light_seeds(prob, g, row_terms + g->row_offset * MIST_ROW_TERMS, ratio, most, first_pair, n_here, pair_split, lds_best);
+    __syncthreads();
+  }
   if (g->scout_stride > 0 && n_here > 0) {
     constexpr int kWaves = kSeedThreads / 64;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const GroupModel m = group_model(prob, g);
     const Offsets group = group_offsets(m, ratio);
-    const double cutoff = stage_cost_cutoff(prob, m.inv_G64), cap_and_room = m.cap * (1.0 + 1e-12);
+    const double cutoff = most, cap_and_room = m.cap * (1.0 + 1e-12);
     const int n_gather = g->n_par * g->n_oo * g->n_ao * g->scout_stride;
     const int n_stages = (n_gather + 63) / 64;
     // units of work: (stage, share of the pairs), more than one share when there are few stages
@@ -2089,6 +2154,7 @@ __global__ __launch_bounds__(kSeedThreads, 3) void seed_kernel(
     const PairIndex pc = decode_pair(first_pair + my_pair);
     const int lc = pc.l | pc.c << 15, my_np = pc.c == pc.l - 1 ? min(P, 1) : P;
     const LinearPair my_lp(pc.l, pc.c);
+    const double closed_below = pc.l < likely ? kLikelyLow * cutoff : -INFINITY;
     const int64_t floor_slot = stage_floor_slot(g, blockIdx.y, 0);
     for (int unit = wave; unit < n_stages * shares; unit += kWaves) {
       const int q = unit / shares * 64 + lane;
@@ -2097,7 +2163,7 @@ __global__ __launch_bounds__(kSeedThreads, 3) void seed_kernel(
       // what a row has to reach of the lane's pair (they fall while the loop runs), against the rows' bounds
       const bool its_post = pc.c != pc.l - 1;
       const double thr = Threshold(loosest_minima(true, lds_best + my_pair * n_slots, 1, P, my_np, my_np, its_post,
-                                                  its_post && pc.l == L, cutoff), group).at(0.0);
+                                                  its_post && pc.l == L, cutoff, closed_below), group).at(0.0);
       const double *__restrict__ f = tabs.gather_floor + (floor_slot + unit / shares) * kGatherFloor;
       const LinearBound floor{f[0], f[1], f[2], f[3], f[4]};
       uint64_t open = __ballot(lane >= i0 && lane < i1 &&
