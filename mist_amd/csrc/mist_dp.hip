@@ -2837,39 +2837,9 @@ int mist_dp_windows_first_batch(const MistDpCosts *costs, int n_requests, const 
                                 float *d_values, int32_t *d_counts, float *d_kept,
                                 int kept_capacity, int32_t *d_meta, float *d_inst_tmax,
                                 int32_t *d_inst_row, void *stream) {
-  if (!costs || !costs->costs || !costs->costs_pre || !costs->costs_post)
-    return fail(MIST_E_INVALID, "null cost tables");
-  if (costs->planes && (costs->planes_g_stride < 1 || costs->planes_g_stride > MIST_MAX_MESH))
-    return fail(MIST_E_INVALID, "planes of %d meshes", (int)costs->planes_g_stride);
-  if (n_requests <= 0 || n_requests > 65535)
-    return fail(MIST_E_INVALID, "n_requests %d outside [1, 65535]", n_requests);
-  if (!d_rows || !d_lo || !d_hi || !d_start || !d_values || !d_counts || !d_kept || !d_meta ||
-      !d_inst_tmax || !d_inst_row)
-    return fail(MIST_E_INVALID, "null pointer argument");
-  if (window_capacity < 128 || window_capacity > kWindowMost || (window_capacity & (window_capacity - 1)))
-    return fail(MIST_E_INVALID, "window_capacity %d is no power of two in [128, %d]", window_capacity, kWindowMost);
-  if (first_chunk < 1 || kept_capacity < 1 || (int64_t)n_requests * first_chunk > 65535)
-    return fail(MIST_E_INVALID, "first_chunk %d x %d requests outside [1, 65535] / empty kept list",
-                first_chunk, n_requests);
-  if (first_lead < 1) return fail(MIST_E_INVALID, "first_lead %d < 1", first_lead);
-  hipStream_t st = (hipStream_t)stream;
-  const int n_counts = 2 + 2 * n_requests, n_inst = n_requests * first_chunk;
-  hipLaunchKernelGGL(window_clear_kernel, dim3((unsigned)((std::max(n_counts, n_inst) + 255) / 256)), dim3(256), 0, st,
-                     d_counts, n_counts, d_inst_row, n_inst);
-  MIST_HIP_CHECK(hipGetLastError());
-  const int64_t per_row = costs->g_stride[0] + costs->g_stride[1] + costs->g_stride[2];
-  const unsigned blocks = select_blocks(per_row);
-  hipLaunchKernelGGL(select_candidates_kernel, dim3(blocks, n_requests), dim3(256), 0, st, *costs,
-                     d_rows, d_lo, d_hi, d_values, (int32_t *)nullptr, window_capacity, d_counts,
-                     true);
-  MIST_HIP_CHECK(hipGetLastError());
-  const size_t lds = window_lds(window_capacity);
-  if (int rc = allow_window_lds()) return rc;
-  hipLaunchKernelGGL(window_walk_kernel, dim3(n_requests), dim3(kWindowThreads), lds, st, d_values,
-                     window_capacity, d_counts, d_rows, d_lo, d_start, gap, first_chunk, first_lead,
-                     d_kept, kept_capacity, d_meta, d_inst_tmax, d_inst_row);
-  MIST_HIP_CHECK(hipGetLastError());
-  return 0;
+  return mist::dp_windows_first_batch(costs, n_requests, d_rows, d_lo, d_hi, d_start, gap, window_capacity, first_chunk,
+                                      first_lead, d_values, d_counts, d_kept, kept_capacity, d_meta, d_inst_tmax,
+                                      d_inst_row, false, (hipStream_t)stream);
 }
 
 int64_t mist_dp_scratch_floats(const MistDpShape *shape, int n_tmax) {
@@ -2895,6 +2865,48 @@ int mist_dp_run(const MistDpShape *shape, const MistDpCosts *costs, const float 
 }
 
 }  // extern "C"
+
+int mist::dp_windows_first_batch(const MistDpCosts *costs, int n_requests, const int32_t *d_rows,
+                                const float *d_lo, const float *d_hi, const float *d_start,
+                                double gap, int window_capacity, int first_chunk, int first_lead,
+                                float *d_values, int32_t *d_counts, float *d_kept,
+                                int kept_capacity, int32_t *d_meta, float *d_inst_tmax,
+                                int32_t *d_inst_row, bool cleared, hipStream_t st) {
+  if (!costs || !costs->costs || !costs->costs_pre || !costs->costs_post)
+    return fail(MIST_E_INVALID, "null cost tables");
+  if (costs->planes && (costs->planes_g_stride < 1 || costs->planes_g_stride > MIST_MAX_MESH))
+    return fail(MIST_E_INVALID, "planes of %d meshes", (int)costs->planes_g_stride);
+  if (n_requests <= 0 || n_requests > 65535)
+    return fail(MIST_E_INVALID, "n_requests %d outside [1, 65535]", n_requests);
+  if (!d_rows || !d_lo || !d_hi || !d_start || !d_values || !d_counts || !d_kept || !d_meta ||
+      !d_inst_tmax || !d_inst_row)
+    return fail(MIST_E_INVALID, "null pointer argument");
+  if (window_capacity < 128 || window_capacity > kWindowMost || (window_capacity & (window_capacity - 1)))
+    return fail(MIST_E_INVALID, "window_capacity %d is no power of two in [128, %d]", window_capacity, kWindowMost);
+  if (first_chunk < 1 || kept_capacity < 1 || (int64_t)n_requests * first_chunk > 65535)
+    return fail(MIST_E_INVALID, "first_chunk %d x %d requests outside [1, 65535] / empty kept list",
+                first_chunk, n_requests);
+  if (first_lead < 1) return fail(MIST_E_INVALID, "first_lead %d < 1", first_lead);
+  const int n_counts = 2 + 2 * n_requests, n_inst = n_requests * first_chunk;
+  if (!cleared) {
+    hipLaunchKernelGGL(window_clear_kernel, dim3((unsigned)((std::max(n_counts, n_inst) + 255) / 256)), dim3(256), 0, st,
+                       d_counts, n_counts, d_inst_row, n_inst);
+    MIST_HIP_CHECK(hipGetLastError());
+  }
+  const int64_t per_row = costs->g_stride[0] + costs->g_stride[1] + costs->g_stride[2];
+  const unsigned blocks = select_blocks(per_row);
+  hipLaunchKernelGGL(select_candidates_kernel, dim3(blocks, n_requests), dim3(256), 0, st, *costs,
+                     d_rows, d_lo, d_hi, d_values, (int32_t *)nullptr, window_capacity, d_counts,
+                     true);
+  MIST_HIP_CHECK(hipGetLastError());
+  const size_t lds = window_lds(window_capacity);
+  if (int rc = allow_window_lds()) return rc;
+  hipLaunchKernelGGL(window_walk_kernel, dim3(n_requests), dim3(kWindowThreads), lds, st, d_values,
+                     window_capacity, d_counts, d_rows, d_lo, d_start, gap, first_chunk, first_lead,
+                     d_kept, kept_capacity, d_meta, d_inst_tmax, d_inst_row);
+  MIST_HIP_CHECK(hipGetLastError());
+  return 0;
+}
 
 int mist::dp_stage_rates(const MistDpShape &shape, const MistDpCosts &costs, int n_g, int32_t *d_rates, hipStream_t stream) {
   if (costs.stage_min == nullptr || n_g < 1 || n_g > 65535) return fail(MIST_E_INVALID, "no row minima or %d tables", n_g);

@@ -25,6 +25,12 @@ int dp_run(const MistDpShape *shape, const MistDpCosts *costs, const int32_t *d_
 // Whether a run without back-pointers knows the partition of every instance.
 bool dp_keeps_paths(const MistDpShape &shape, const MistDpCosts &costs, int n_tmax, int mode, int64_t scratch_floats);
 
+// mist_dp_windows_first_batch; `cleared`: d_counts (2 + 2 n_requests) hold zeros and d_inst_row -1.
+int dp_windows_first_batch(const MistDpCosts *costs, int n_requests, const int32_t *d_rows, const float *d_lo,
+                           const float *d_hi, const float *d_start, double gap, int window_capacity, int first_chunk,
+                           int first_lead, float *d_values, int32_t *d_counts, float *d_kept, int kept_capacity,
+                           int32_t *d_meta, float *d_inst_tmax, int32_t *d_inst_row, bool cleared, hipStream_t stream);
+
 struct DpFreeRun {
   const MistDpShape *shape;
   const MistDpCosts *costs;

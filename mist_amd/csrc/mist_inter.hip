@@ -155,12 +155,16 @@ struct Fetched {  // one request of a candidate fetch: ascending values and how 
 // req[0][i] = table row, req[1][i] = lo, req[2][i] = hi of the candidates to fetch, req[3][i] =
 // the smallest feasible threshold itself; an empty window (lo = hi = +inf) when no family is
 // feasible.  The bounds only size the fetch; what the scan does with the candidates follows the
-// reference's rules on the values that lie inside.
+// reference's rules on the values that lie inside.  The counters and instances of the windows
+// behind it (mist::dp_windows_first_batch) are cleared on the way.
 __global__ void window_request_kernel(const float *__restrict__ out, int n_families, int n,
                                       const int32_t *__restrict__ rows,
                                       const int32_t *__restrict__ grad_accum, int n_grad_accum,
-                                      double gap, float *__restrict__ req) {
+                                      double gap, float *__restrict__ req, int32_t *__restrict__ counts, int n_counts,
+                                      int32_t *__restrict__ inst_row, int n_inst) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n_counts) counts[i] = 0;
+  if (i < n_inst) inst_row[i] = -1;
   if (i >= n) return;
   float bott = INFINITY, sum = INFINITY;
   for (int f = 0; f < n_families; ++f) {
@@ -343,7 +347,9 @@ struct Search {
   // 80 x 16 794 -> 692, 24 x 64 203 -> 186, 40 x 48 365 -> 331, 40 x 64 549 -> 450, 48 x 128 1090 -> 640,
   // 80 x 256 6740 -> 2770).
   const int64_t rates_above = rates_above_states();
-  int n_rates = 0, at_rates = 0;
+  int n_rates = 0, at_rates = 0, at_in = 0;
+  // (and the instances of the bottleneck DP, a copy less)
+  const float *uploaded_in() const { return ws->d_grad.as<float>() + at_in; }
   int upload_grad_accum(const std::vector<int32_t> &rows, const int32_t *grad_accum, int n_grad_accum) {
     n_rates = 0;
     at_rates = n_grad_accum;
@@ -351,10 +357,14 @@ struct Search {
     for (const int32_t row : rows) n_g = std::max(n_g, row + 1);
     size_t words = n_grad_accum;
     for (int f = 0; f < n_families; ++f) words += (size_t)n_g * (1 + shapes[f].num_mesh);
+    at_in = (int)words;
+    words += 2 * rows.size();
     if (int rc = ws->h_grad.reserve(sizeof(int32_t) * words)) return rc;
     if (int rc = ws->d_grad.reserve(sizeof(int32_t) * words)) return rc;
     std::memcpy(ws->h_grad.ptr, grad_accum, sizeof(int32_t) * n_grad_accum);
-    std::fill_n(ws->h_grad.as<int32_t>() + n_grad_accum, words - n_grad_accum, mist::kRateNone);
+    std::fill_n(ws->h_grad.as<int32_t>() + n_grad_accum, at_in - n_grad_accum, mist::kRateNone);
+    std::fill_n(ws->h_grad.as<float>() + at_in, rows.size(), 0.0f);
+    std::copy(rows.begin(), rows.end(), ws->h_grad.as<int32_t>() + at_in + rows.size());
     MIST_HIP_CHECK(hipMemcpyAsync(ws->d_grad.ptr, ws->h_grad.ptr, sizeof(int32_t) * words, hipMemcpyHostToDevice, stream));
     if (n_g == 0 || n_g > 65535) return 0;
     n_rates = n_g;
@@ -413,9 +423,11 @@ struct Search {
   // bits, best_sum, stage_max); with `want_path` also the partitions (h_path, family after
   // family) and, when strategy tables were given, the strategy rows of their stages
   // (h_rows, same order without the factor 4).  `sync` false leaves the copies of the
-  // outputs queued on the stream for the caller to wait for.
+  // outputs queued on the stream for the caller to wait for.  d_uploaded: the instances ([2][n]: thresholds,
+  // table rows) are on the device; d_outputs: the outputs go there and are not copied back.
   int run(const std::vector<int32_t> &g_index, const std::vector<float> &tmax, int mode,
-          bool want_path, bool sync = true, int path_batch = -1) {
+          bool want_path, bool sync = true, int path_batch = -1, const float *d_uploaded = nullptr,
+          float *d_outputs = nullptr) {
     const int n = (int)tmax.size();
     if (n == 0) return 0;
     const size_t n_out = (size_t)3 * n * n_families;
@@ -442,19 +454,22 @@ struct Search {
     if (int rc = ws->d_scratch.reserve(sizeof(float) * (size_t)n_scratch)) return rc;
     if (want_path)
       if (int rc = ws->d_argmin.reserve(sizeof(int32_t) * slab * n)) return rc;
-    float *h_in = ws->h_in.as<float>();
-    std::memcpy(h_in, tmax.data(), sizeof(float) * n);
-    std::memcpy(h_in + n, g_index.data(), sizeof(int32_t) * n);
-    MIST_HIP_CHECK(hipMemcpyAsync(ws->d_in.ptr, h_in, sizeof(float) * 2 * n, hipMemcpyHostToDevice,
-                                  stream));
-    float *d_in = ws->d_in.as<float>();
-    const int32_t *d_g = reinterpret_cast<int32_t *>(d_in + n);
+    if (d_uploaded == nullptr) {
+      float *h_in = ws->h_in.as<float>();
+      std::memcpy(h_in, tmax.data(), sizeof(float) * n);
+      std::memcpy(h_in + n, g_index.data(), sizeof(int32_t) * n);
+      MIST_HIP_CHECK(hipMemcpyAsync(ws->d_in.ptr, h_in, sizeof(float) * 2 * n, hipMemcpyHostToDevice,
+                                    stream));
+    }
+    const float *d_in = d_uploaded != nullptr ? d_uploaded : ws->d_in.as<float>();
+    float *const d_all = d_outputs != nullptr ? d_outputs : ws->d_out.as<float>();
+    const int32_t *d_g = reinterpret_cast<const int32_t *>(d_in + n);
     const bool known = *std::max_element(g_index.begin(), g_index.end()) < n_rates;
     std::vector<mist::DpFreeRun> together;
     std::vector<MistDpShape> its_shapes;
     for (int f = 0; f < n_families; ++f) its_shapes.push_back(shape_of(f));
     for (int f = 0; f < n_families; ++f) {
-      float *d_out = ws->d_out.as<float>() + (size_t)f * 3 * n;
+      float *d_out = d_all + (size_t)f * 3 * n;
       together.push_back({&its_shapes[f], &costs[f], reinterpret_cast<int32_t *>(d_out), d_out + n, d_out + 2 * n,
                           want_path ? d_paths + path_offset(f, n) : path_batch >= 0 ? kept_paths(path_batch, f, 0) : nullptr});
     }
@@ -463,7 +478,7 @@ struct Search {
     // otherwise the families share the state planes and the back-pointer slab: they run one after
     // the other on the stream
     for (int f = 0; f < n_families; ++f) {
-      float *d_out = ws->d_out.as<float>() + (size_t)f * 3 * n;
+      float *d_out = d_all + (size_t)f * 3 * n;
       int32_t *d_argmin = want_path ? ws->d_argmin.as<int32_t>() : nullptr;  // no fill: the
                                                      // walk reads what the DP wrote
       int32_t *d_path = together[f].d_path;
@@ -482,8 +497,9 @@ struct Search {
         }
       }
     }
-    MIST_HIP_CHECK(hipMemcpyAsync(ws->h_out.ptr, ws->d_out.ptr, sizeof(float) * n_back,
-                                  hipMemcpyDeviceToHost, stream));
+    if (d_outputs == nullptr)
+      MIST_HIP_CHECK(hipMemcpyAsync(ws->h_out.ptr, ws->d_out.ptr, sizeof(float) * n_back,
+                                    hipMemcpyDeviceToHost, stream));
     launches += n_families;
     thresholds_run += (int64_t)n * n_families;
     if (sync) {
@@ -539,7 +555,7 @@ struct Search {
   }
 
   // The bottleneck DP of every (instance, G) and the first fetch of their windows in one round
-  // trip: the requests are made on the GPU from the DP's outputs.  ws->h_out holds the DP
+  // trip: the requests are made on the GPU from the DP's outputs.  `bottleneck` holds the DP
   // outputs afterwards, ws->h_req the requests as they were made ([3][n]: row, lo, hi).
   int bottleneck_and_fetch(const std::vector<int32_t> &rows, const int32_t *grad_accum,
                            int n_grad_accum, std::vector<Fetched> *out) {
@@ -548,11 +564,13 @@ struct Search {
     if (int rc = ws->d_req.reserve(sizeof(float) * 4 * n)) return rc;
     if (int rc = upload_grad_accum(rows, grad_accum, n_grad_accum)) return rc;
     const std::vector<float> zeros(n, 0.0f);
-    if (int rc = run(rows, zeros, MIST_DP_BOTTLENECK, false, /*sync=*/false)) return rc;
+    if (int rc = run(rows, zeros, MIST_DP_BOTTLENECK, false, /*sync=*/false, -1, uploaded_in())) return rc;
+    bottleneck = ws->h_out.as<float>();
     hipLaunchKernelGGL(window_request_kernel, dim3((n + 63) / 64), dim3(64), 0, stream,
                        ws->d_out.as<float>(), n_families, n,
-                       reinterpret_cast<const int32_t *>(ws->d_in.as<float>() + n),
-                       ws->d_grad.as<int32_t>(), n_grad_accum, kGap, ws->d_req.as<float>());
+                       reinterpret_cast<const int32_t *>(uploaded_in() + n),
+                       ws->d_grad.as<int32_t>(), n_grad_accum, kGap, ws->d_req.as<float>(), (int32_t *)nullptr, 0,
+                       (int32_t *)nullptr, 0);
     MIST_HIP_CHECK(hipGetLastError());
     MIST_HIP_CHECK(hipMemcpyAsync(ws->h_req.ptr, ws->d_req.ptr, sizeof(float) * 4 * n,
                                   hipMemcpyDeviceToHost, stream));
@@ -562,11 +580,12 @@ struct Search {
 
   // The same, and the windows and the first scan batch with it (mist_dp_windows_first_batch +
   // the threshold DP of its instances for every family): one round trip.  Afterwards
-  // ws->h_out holds the bottleneck DP's outputs; first_req the requests ([4][n]: row, lo, hi,
+  // `bottleneck` holds that DP's outputs; first_req the requests ([4][n]: row, lo, hi,
   // smallest feasible threshold), first_meta the windows' descriptions ([n][8]), first_kept
   // their kept thresholds and first_out the DP outputs of the batch
   // ([family][3][n * first_chunk]; the instances of window r start at first_meta[r][7]).
   const float *first_req = nullptr, *first_kept = nullptr, *first_out = nullptr;
+  const float *bottleneck = nullptr;  // outputs of the bottleneck DP, [family][3][n]
   const int32_t *first_meta = nullptr;
   // partitions and strategy rows of the last run with `want_path` (behind its outputs in ws->h_out)
   const int32_t *h_path = nullptr, *h_rows = nullptr;
@@ -578,8 +597,9 @@ struct Search {
     if (int rc = ws->d_inst_t.reserve(sizeof(float) * n_inst)) return rc;
     if (int rc = ws->d_inst_row.reserve(sizeof(int32_t) * n_inst)) return rc;
     const size_t n_out = (size_t)3 * n_inst * n_families;
-    // one buffer of 4-byte words: [requests 4 n][descriptions 8 n][outputs n_out][kept thresholds]
-    const size_t at_meta = (size_t)4 * n, at_out = at_meta + (size_t)8 * n, at_kept = at_out + n_out;
+    // one buffer of 4-byte words: [requests 4 n][descriptions 8 n][bottleneck outputs][outputs n_out][kept thresholds]
+    const size_t at_meta = (size_t)4 * n, at_bottleneck = at_meta + (size_t)8 * n;
+    const size_t at_out = at_bottleneck + (size_t)3 * n * n_families, at_kept = at_out + n_out;
     const size_t words = at_kept + kKeptCapacity;
     if (int rc = ws->d_first.reserve(sizeof(float) * words)) return rc;
     if (int rc = ws->h_first.reserve(sizeof(float) * words)) return rc;
@@ -598,20 +618,24 @@ struct Search {
     if (int rc = ws->d_scratch.reserve(sizeof(float) * (size_t)n_scratch)) return rc;
     if (int rc = upload_grad_accum(rows, grad_accum, n_grad_accum)) return rc;
     const std::vector<float> zeros(n, 0.0f);
-    if (int rc = run(rows, zeros, MIST_DP_BOTTLENECK, false, /*sync=*/false)) return rc;
+    if (int rc = run(rows, zeros, MIST_DP_BOTTLENECK, false, /*sync=*/false, -1, uploaded_in(), d_first + at_bottleneck))
+      return rc;
+    bottleneck = h_first + at_bottleneck;
     float *d_req = d_first;
-    hipLaunchKernelGGL(window_request_kernel, dim3((n + 63) / 64), dim3(64), 0, stream,
-                       ws->d_out.as<float>(), n_families, n,
-                       reinterpret_cast<const int32_t *>(ws->d_in.as<float>() + n),
-                       ws->d_grad.as<int32_t>(), n_grad_accum, kGap, d_req);
+    const int n_counts = 2 + 2 * n;
+    hipLaunchKernelGGL(window_request_kernel, dim3((std::max(n_counts, n_inst) + 255) / 256), dim3(256), 0, stream,
+                       d_first + at_bottleneck, n_families, n,
+                       reinterpret_cast<const int32_t *>(uploaded_in() + n),
+                       ws->d_grad.as<int32_t>(), n_grad_accum, kGap, d_req, ws->d_win_counts.as<int32_t>(), n_counts,
+                       ws->d_inst_row.as<int32_t>(), n_inst);
     MIST_HIP_CHECK(hipGetLastError());
-    if (int rc = mist_dp_windows_first_batch(
+    if (int rc = mist::dp_windows_first_batch(
             select_costs, n, reinterpret_cast<int32_t *>(d_req), d_req + n, d_req + 2 * n,
             d_req + 3 * n, kGap, window_capacity, first_chunk, kFirstLead,
             ws->d_win_values.as<float>(),
             ws->d_win_counts.as<int32_t>(), d_first + at_kept, kKeptCapacity,
             reinterpret_cast<int32_t *>(d_first + at_meta), ws->d_inst_t.as<float>(),
-            ws->d_inst_row.as<int32_t>(), stream))
+            ws->d_inst_row.as<int32_t>(), /*cleared=*/true, stream))
       return rc;
     const int path_batch = keep_paths(n_inst);
     std::vector<mist::DpFreeRun> together;
@@ -873,7 +897,7 @@ static int search_families(int n_families, const MistDpShape *shapes,
   // smallest feasible threshold (+inf if none) and the stage-cost sum there, from the outputs of
   // the bottleneck DP of every family (the first family with the smallest threshold)
   auto bottleneck_of = [&](int i, float *bott, float *sum) {
-    const float *h = S.ws->h_out.as<float>();
+    const float *h = S.bottleneck;
     *bott = *sum = std::numeric_limits<float>::infinity();
     for (int f = 0; f < n_families; ++f) {
       const float b = h[(size_t)f * 3 * n_flat + n_flat + i];
