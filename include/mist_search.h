@@ -130,11 +130,16 @@ typedef struct MistProblem {
   /* != 0 (one sample): the tables are not pre-filled, and what reads them knows the cells that are never
    * written (mist_dp_cost_planes); a cell without a row gets its index of -1 and no costs. */
   int32_t sparse_tables;
-  /* != 0 (with stage_cost_incumbent; the groups of the call are all groups of their table rows, those of a row
+  /* 1 (with stage_cost_incumbent; the groups of the call are all groups of their table rows, those of a row
    * side by side): for a caller whose search is all that reads the tables.  Below bound(G) a cell, too, that is
    * in no pipeline of stages up to bound(G) may hold +inf / -1 or another row than its minimum's, as long as it
    * then is below every threshold candidate which that search reads: those from 16 (1e-4 s + 1e-5 x) below the
-   * smallest largest stage cost x of a pipeline on. */
+   * smallest largest stage cost x of a pipeline on.
+   * 2 (with stage_cost_incumbent, whatever the sample_size; calls with several samples): for a caller that reads
+   * the tables for the stage assignment only (mist_mip.h; incumbent_ckpt_rule 1 or 2).  The incumbent becomes the
+   * objective of an assignment of rows that the tables may or may not hold, and a (group, layers) that is in no
+   * assignment up to incumbent * (1 + slack) may hold +inf / -1 throughout: an optimum no larger than that is the
+   * optimum of the complete tables. */
   int32_t incumbent_close;
 } MistProblem;
 

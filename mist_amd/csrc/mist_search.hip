@@ -1491,12 +1491,14 @@ struct Hit {
 };
 static_assert(sizeof(Hit) == 16, "two doubles of the workspace");
 
+// MistProblem.incumbent_close: what reads the tables.
+constexpr int kCloseSearch = 1, kCloseAssignment = 2;
 // What a group's stage costs can be used for (form_reach).
 struct GroupReach {
   double per_layer, rest;  // of every row at least rest + (layers - 2) x per_layer (two layers or fewer: rest)
   double cutoff;           // rows above it are not looked for
   double low;              // a minimum below it, of a stage of fewer than `first` layers, is final as it is
-  int first, reserved;
+  int first, last;         // for an assignment: the layers a stage may have
 };
 static_assert(sizeof(GroupReach) == 5 * sizeof(double), "doubles of the workspace");
 constexpr int kReachGroups = 2048;  // the most groups that get one: 48 KB of LDS
@@ -1761,7 +1763,7 @@ __device__ __forceinline__ RowCounts exact_counts(const LaneMemory &mem, const G
 // it are not looked for.  (The seed launch reads the first estimate, which a few rows gave
 // before it; the later launches read the one the seeds gave.)
 __device__ __forceinline__ double stage_cost_cutoff(const MistProblem &prob, double inv_G64) {
-  return prob.stage_cost_incumbent == nullptr || prob.sample_size != 1
+  return prob.stage_cost_incumbent == nullptr || prob.sample_size != 1 || prob.incumbent_close == kCloseAssignment
              ? (double)INFINITY
              : *prob.stage_cost_incumbent * inv_G64 * (1.0 + kIncumbentSlack);
 }
@@ -1774,9 +1776,13 @@ struct CostLimits {
   __device__ __forceinline__ double closed_below(int layers) const { return layers < first ? low : -INFINITY; }
 };
 __device__ __forceinline__ CostLimits cost_limits(const MistProblem &prob, const ReduceTables &tabs, int group, double inv_G64) {
-  if (prob.incumbent_close == 0) return CostLimits{stage_cost_cutoff(prob, inv_G64), -INFINITY, 0};
+  if (prob.incumbent_close != kCloseSearch) return CostLimits{stage_cost_cutoff(prob, inv_G64), -INFINITY, 0};
   const GroupReach &r = tabs.reach[group];
   return CostLimits{r.cutoff, r.low, r.first};
+}
+// Whether a pair of that many layers is in an assignment that reach_of_assignments leaves.
+__device__ __forceinline__ bool in_assignments(const MistProblem &prob, const ReduceTables &tabs, int group, int layers) {
+  return prob.incumbent_close != kCloseAssignment || (layers >= tabs.reach[group].first && layers <= tabs.reach[group].last);
 }
 // A minimum as a threshold.
 __device__ __forceinline__ double up_to(double minimum, double cutoff, double closed_below) {
@@ -2050,7 +2056,7 @@ __global__ __launch_bounds__(256) void gather_floor_kernel(const MistProblem pro
 // minimum is below about kLikelyLow of the cutoff: what is wrong about that only leaves them higher minima.
 constexpr double kLikelyLow = 0.88;
 __device__ __forceinline__ int likely_first(const MistProblem &prob, const MistGroupDesc *g, double cutoff) {
-  if (prob.incumbent_close == 0 || !(cutoff < INFINITY)) return 0;
+  if (prob.incumbent_close != kCloseSearch || !(cutoff < INFINITY)) return 0;
   const float L = (float)prob.num_layers, D = (float)prob.incumbent_num_devices;
   return (int)(L - 1.05f * L * (D - (float)(g->num_nodes * g->num_gpus_per_node)) / D);
 }
@@ -2307,7 +2313,7 @@ __global__ __launch_bounds__(64 * kSeedSampleWaves) void seed_samples_kernel(
   for (int e = threadIdx.x; e < n_slots * S; e += blockDim.x) mine[e] = INFINITY;
   __syncthreads();
   const int sample = lane & 31;
-  if (g->scout_stride > 0 && pair < n_pairs) {
+  if (g->scout_stride > 0 && pair < n_pairs && in_assignments(prob, tabs, blockIdx.y, decode_pair(pair).l)) {
     const GroupModel m = group_model(prob, g);
     const PairIndex pc = decode_pair(pair);
     const int l = __builtin_amdgcn_readfirstlane(pc.l), c = __builtin_amdgcn_readfirstlane(pc.c);
@@ -2381,16 +2387,17 @@ __global__ __launch_bounds__(64 * kSeedSampleWaves) void seed_samples_kernel(
 __device__ __forceinline__ int64_t super_floor_slot(const MistGroupDesc *g, int group_index, int64_t super) {
   return stage_floor_slot(g, group_index, 0) / kSuperStages + group_index + super;
 }
-// With `close` a workgroup also leaves the smallest linear bounds of its summaries (GroupReach).
+// With `close` a workgroup also leaves the smallest linear bounds of its summaries (GroupReach): of stage costs,
+// for an assignment of stable latencies.
 __global__ __launch_bounds__(256) void super_floor_kernel(const MistGroupDesc *__restrict__ groups, int n_groups,
-                                                          const double *__restrict__ stage_floor, double ratio, bool close,
+                                                          const double *__restrict__ stage_floor, double ratio, int close,
                                                           const ReduceTables tabs) {
   const int gi = blockIdx.y;
   const MistGroupDesc *g = groups + gi;
   const int64_t n_stages = (g->n_rows + kStageRows - 1) / kStageRows;
   const int col = threadIdx.x % kStageFloorPitch;
   const int per_block = blockDim.x / kStageFloorPitch;
-  const double inv_G = 1.0 / (double)g->grad_accum;
+  const double inv_G = close == kCloseAssignment ? 0.0 : 1.0 / (double)g->grad_accum;
   double per_layer = INFINITY, rest = INFINITY;
   for (int64_t super = (int64_t)blockIdx.x * per_block + threadIdx.x / kStageFloorPitch;
        super * kSuperStages < n_stages; super += (int64_t)gridDim.x * per_block) {
@@ -2403,7 +2410,7 @@ __global__ __launch_bounds__(256) void super_floor_kernel(const MistGroupDesc *_
     }
     tabs.super_floor[super_floor_slot(g, gi, super) * kStageFloorPitch + col] = v;
     if (tabs.listed != nullptr && col < n) tabs.stage_flag[stage_floor_slot(g, gi, super * kSuperStages) + col] = 0;
-    if (!close) continue;
+    if (close == 0) continue;
     // (the columns of a summary lie in 32 neighbouring lanes; every lane forms the same bounds)
     const LinearBound b = linear_form([&](int stable, int delta) {
       return less_slack(ratio * __shfl(v, stable, kStageFloorPitch)) + less_slack(__shfl(v, delta, kStageFloorPitch) * inv_G);
@@ -2411,7 +2418,7 @@ __global__ __launch_bounds__(256) void super_floor_kernel(const MistGroupDesc *_
     per_layer = fmin(per_layer, fmin(b.ck, b.nock));
     rest = fmin(rest, fmin(b.all_ck, fmin(b.none, b.mid)));
   }
-  if (!close) return;
+  if (close == 0) return;
   __shared__ double parts[256 / kStageFloorPitch][2];
   if (col == 0) {
     parts[threadIdx.x / kStageFloorPitch][0] = per_layer;
@@ -2492,8 +2499,10 @@ __global__ __launch_bounds__(kSamples ? kFilterShares * 64 : 64) void filter_ker
 
   const int L = prob.num_layers, n_pairs = L * (L + 1) / 2 + L, lane = threadIdx.x & 63;
   const int pair_idx = (g->lc_tile_begin + tile_rel) * MIST_LC_TILE + lane;
-  const bool active = pair_idx < n_pairs;
-  const PairIndex pc = decode_pair(active ? pair_idx : 0);
+  const bool listed = pair_idx < n_pairs;
+  const PairIndex pc = decode_pair(listed ? pair_idx : 0);
+  const bool active = listed && (!kSamples || in_assignments(prob, tabs, gi, pc.l));
+  if (kSamples && !__any(active)) return;  // (all wavefronts of the workgroup: one tile)
   const PairConsts k = pair_consts(pc.l, pc.c);
   const int P = g->num_p, S = tabs.n_samples;
   const int np = !active ? 0 : (pc.c == pc.l - 1 ? min(P, 1) : P);
@@ -2758,6 +2767,10 @@ __global__ __launch_bounds__(kReduceThreads) void open_kernel(const MistProblem 
         tile_word = its_word >> kItemStageBits;
         g = groups + gi;
         p = tile_lane(prob, g, item.tile);
+        if (kSamples && !in_assignments(prob, tabs, gi, p.pc.l)) {
+          p.active = p.do_post = p.do_pp = false;
+          p.np = 0;
+        }
         k = pair_consts(p.pc.l, p.pc.c);
         m = group_model(prob, g);
         group = group_offsets(m, ratio);
@@ -3620,7 +3633,7 @@ __device__ __forceinline__ int incumbent_stage_count(const MistProblem &prob,
   if (nm <= 0 || D % nm != 0) return 0;
   const int S = D / nm;
   if (S < 1 || S > L || S - 1 >= g->num_p) return 0;
-  if (L % S != 0 && (D & (D - 1)) == 0) return 0;
+  if (L % S != 0 && (D & (D - 1)) == 0 && prob.incumbent_close != kCloseAssignment) return 0;
   // (the per-mesh search goes up to min(devices, layers) / 2 stages, inter_tuning.py:279-281)
   if (prob.incumbent_ckpt_rule == 0 && S > (D < L ? D : L) / 2) return 0;
   return S;
@@ -3705,7 +3718,7 @@ __global__ __launch_bounds__(64 * kIncumbentWaves) void incumbent_kernel(
     const MistProblem prob, const MistGroupDesc *__restrict__ groups, const ReduceTables tabs) {
   const MistGroupDesc *g = groups + blockIdx.x;
   const int L = prob.num_layers, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const bool close = prob.incumbent_close != 0;
+  const bool close = prob.incumbent_close == kCloseSearch;
   if (close && wave == 0) {
     static_assert(kSuperBlocks == 64, "a lane per workgroup of the summaries");
     const double *parts = tabs.reach_parts + ((int64_t)blockIdx.x * kSuperBlocks + lane) * 2;
@@ -3798,11 +3811,42 @@ constexpr int kEstimateRows = 1024;
 constexpr int kEstimateMaxStages = 256;
 static_assert(kEstimateSplit <= MIST_LC_TILE, "S <= num_p: the partial minima of a group fit one tile of its minima");
 __device__ __forceinline__ bool estimate_runs(const MistProblem &prob, const MistGroupDesc *g, int *stages) {
-  if (g->scout_stride <= 0) return false;
+  if (g->scout_stride <= 0 || g->n_lc_tiles <= 0) return false;
   *stages = incumbent_stage_count(prob, g);
   return *stages > 0 && *stages <= kEstimateMaxStages;
 }
 
+// For an assignment (kAssignment) stages are chosen by stable + delta / G; the smallest float32 of that and its item
+// are kept, whose latencies the combining launch forms again.
+struct EstimateItem {
+  int l, c;
+  int64_t row;  // gathered
+};
+struct EstimateItems {
+  int n_cells, n_tail, n_par;
+  int64_t per_pair, per_tail, n_tails;
+  __device__ __forceinline__ EstimateItems(const MistGroupDesc *g, const PipelineLayers &layers) {
+    n_tail = g->n_oo * g->n_ao;
+    n_par = g->n_par;
+    per_pair = (int64_t)g->n_par * n_tail;
+    per_tail = (int64_t)g->n_par * max(g->scout_stride, 1);
+    n_tails = min((int64_t)n_tail, max((int64_t)1, (int64_t)kEstimateRows / per_tail));
+    n_cells = layers.each + 1 + (layers.extra > 0 ? layers.each + 2 : 0);  // (layers, ckpt) of a row
+  }
+  __device__ __forceinline__ int64_t count() const { return per_tail * n_tails * n_cells; }
+  __device__ __forceinline__ EstimateItem at(int64_t item, const PipelineLayers &layers) const {
+    const int cell = (int)(item % n_cells);
+    const bool longer = cell > layers.each;
+    EstimateItem i;
+    i.l = longer ? layers.each + 1 : layers.each;
+    i.c = longer ? cell - i.l : cell;
+    const int64_t q = item / n_cells, tail = q / per_tail, rest = q - tail * per_tail;
+    const int64_t pair = rest / n_par, par = rest - pair * n_par;
+    i.row = pair * per_pair + par * n_tail + tail;
+    return i;
+  }
+};
+template <bool kAssignment>
 __global__ __launch_bounds__(256) void estimate_stage_minima_kernel(
     const MistProblem prob, const MistGroupDesc *__restrict__ groups,
     const double *__restrict__ row_terms, double ratio, double *__restrict__ partial_cost, double *gather_floor) {
@@ -3823,34 +3867,28 @@ __global__ __launch_bounds__(256) void estimate_stage_minima_kernel(
   const unsigned long long kInf = (unsigned long long)__double_as_longlong((double)INFINITY);
   for (int st = threadIdx.x; st < S; st += blockDim.x) stage_min[st] = kInf;
   __syncthreads();
-  const int n_tail = g->n_oo * g->n_ao;
-  const int64_t per_pair = (int64_t)g->n_par * n_tail;
-  const int64_t per_tail = (int64_t)g->n_par * max(g->scout_stride, 1);
-  const int64_t n_tails = min((int64_t)n_tail, max((int64_t)1, (int64_t)kEstimateRows / per_tail));
-  const int n_cells = layers.each + 1 + (layers.extra > 0 ? layers.each + 2 : 0);  // (layers, ckpt) of a row
-  const int64_t n_items = per_tail * n_tails * n_cells;
+  const EstimateItems items(g, layers);
+  const int64_t n_items = items.count();
   const GroupConsts k = group_consts(g);
   const double cap = prob.mem_cap_mb;
   const double G64 = (double)g->grad_accum;
   const float G32 = (float)g->grad_accum;
   const double *__restrict__ src = row_terms + g->row_offset * MIST_ROW_TERMS;
+  int64_t item = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   auto offer = [&](int st, bool ok, double cost) {
     // (stage costs, unlike objectives of another alpha, are not negative: their bits order)
     if (ok && cost >= 0.0 && cost < INFINITY)
-      atomicMin(&stage_min[st], (unsigned long long)__double_as_longlong(cost));
+      atomicMin(&stage_min[st], kAssignment ? (unsigned long long)__float_as_uint((float)cost) << 32 | (uint32_t)item
+                                            : (unsigned long long)__double_as_longlong(cost));
   };
-  for (int64_t item = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; item < n_items;
-       item += (int64_t)kEstimateSplit * blockDim.x) {
-    const int cell = (int)(item % n_cells);
-    const bool longer = cell > layers.each;
-    const int l = longer ? layers.each + 1 : layers.each, c = longer ? cell - l : cell;
-    const int64_t q = item / n_cells;
-    const int64_t tail = q / per_tail, rest = q - tail * per_tail;
-    const int64_t pair = rest / g->n_par, par = rest - pair * g->n_par;
+  for (; item < n_items; item += (int64_t)kEstimateSplit * blockDim.x) {
+    const EstimateItem i = items.at(item, layers);
+    const int l = i.l, c = i.c;
+    const bool longer = l > layers.each;
     if (rule == 2 && c != l) continue;  // every layer of a stage checkpointed
     if (c == l - 1) continue;  // kept at p == 0 of base / with_pre only, which no stage below reads
     const double *__restrict__ t =
-        src + gathered_position(g, (uint32_t)(pair * per_pair + par * n_tail + tail)) * MIST_ROW_TERMS;
+        src + gathered_position(g, (uint32_t)i.row) * MIST_ROW_TERMS;
     const CellLatency lat = cell_latency<true>(t, l, c, k);
     const LaneMemory mem = cell_memory(t, l, c);
     // largest ckpt count of the stage that ends with layer end_layer (rule of the caller's search)
@@ -3886,6 +3924,90 @@ __global__ __launch_bounds__(256) void estimate_stage_minima_kernel(
   double *out = partial_cost + g->cell_offset + (int64_t)blockIdx.x * S;
   for (int st = threadIdx.x; st < S; st += blockDim.x)
     out[st] = __longlong_as_double((long long)stage_min[st]);
+}
+
+// Objective of the assignment that a group's chosen stages are (inter_tuning_mip.py:317-400) into *incumbent.
+__global__ __launch_bounds__(64) void estimate_assignment_kernel(const MistProblem prob, const MistGroupDesc *__restrict__ groups,
+                                                                 const double *__restrict__ row_terms,
+                                                                 const double *__restrict__ partial_cost) {
+  const MistGroupDesc *g = groups + blockIdx.x;
+  int S;
+  if (!estimate_runs(prob, g, &S)) return;
+  const PipelineLayers layers(prob.num_layers, S);
+  const EstimateItems items(g, layers);
+  const GroupConsts k = group_consts(g);
+  const unsigned long long *in = reinterpret_cast<const unsigned long long *>(partial_cost + g->cell_offset);
+  __shared__ double stable[kEstimateMaxStages], delta[kEstimateMaxStages];
+  for (int st = threadIdx.x; st < S; st += 64) {
+    unsigned long long best = ~0ull;
+    for (int part = 0; part < kEstimateSplit; ++part) best = min(best, in[(int64_t)part * S + st]);
+    double x = INFINITY, d = INFINITY;
+    if (best < (unsigned long long)__double_as_longlong((double)INFINITY)) {
+      const EstimateItem i = items.at((int64_t)(uint32_t)best, layers);
+      const double *__restrict__ t =
+          row_terms + (g->row_offset + gathered_position(g, (uint32_t)i.row)) * MIST_ROW_TERMS;
+      const CellLatency lat = cell_latency<true>(t, i.l, i.c, k);
+      x = S == 1 ? lat.spp : st == 0 ? lat.sp : st == S - 1 ? lat.spost : (double)lat.x;
+      d = S == 1 ? lat.dpp : st == 0 ? lat.dpre : st == S - 1 ? lat.dpost : (double)lat.d;
+    }
+    stable[st] = fmax(x, 0.0);
+    delta[st] = fmax(d, 0.0);
+  }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  double sum = 0.0, largest = 0.0, late = 0.0;
+  for (int st = 0; st < S; ++st) {
+    late = fmax(late, delta[st] - sum);
+    sum += stable[st];
+    largest = fmax(largest, stable[st]);
+  }
+  const double total = (double)(g->grad_accum - 1) * largest + sum + late;
+  if (total >= 0.0 && total < INFINITY)
+    atomicMin(reinterpret_cast<unsigned long long *>(prob.stage_cost_incumbent), (unsigned long long)__double_as_longlong(total));
+}
+
+// Layers a stage of a group may have in an assignment whose objective is no more than the estimate and some room
+// ((G - 1) max T + sum T and what is not negative): with l of them one of the other stages has at least its share of
+// the rest, and stable latencies are no less than the bounds of the group's rows.  Most groups keep the even number
+// of layers alone, or nothing: 30 samples of 7B on 4x8 2870 -> 2190 us, on 1x8 (small cards) 1390 -> 1265, 13B on 8x8
+// 2980 -> 1700.  (With the seeds of all pairs beside the summaries, as without an estimate: 7B on 4x8 2280, 1x8 1264.
+// Of 190 drawn calls all had an optimum between 0.93 and 1.0000 times the estimate.)
+__global__ __launch_bounds__(64) void assignment_reach_kernel(const MistProblem prob, const MistGroupDesc *__restrict__ groups,
+                                                              const ReduceTables tabs) {
+  static_assert(kSuperBlocks == 64, "a lane per workgroup of the summaries");
+  const int gi = blockIdx.x, lane = threadIdx.x, L = prob.num_layers, D = prob.incumbent_num_devices;
+  const MistGroupDesc *g = groups + gi;
+  const double *parts = tabs.reach_parts + ((int64_t)gi * kSuperBlocks + lane) * 2;
+  double per_layer = parts[0], rest = parts[1];
+  for (int step = 32; step > 0; step >>= 1) {
+    per_layer = fmin(per_layer, __shfl_xor(per_layer, step));
+    rest = fmin(rest, __shfl_xor(rest, step));
+  }
+  const double most = *prob.stage_cost_incumbent * (1.0 + kIncumbentSlack), more = (double)(g->grad_accum - 1);
+  const int nm = g->num_nodes * g->num_gpus_per_node, S = D / nm;
+  const bool bounded = D % nm == 0 && per_layer > 0.0 && most < INFINITY;
+  auto least = [&](int layers) { return rest + (double)max(layers - 2, 0) * per_layer; };
+  int first = L + 1, last = 0;
+  for (int l = 1 + lane; l <= L; l += 64) {
+    bool in = true;
+    if (bounded && S == 1) in = l == L && least(L) * (more + 1.0) * (1.0 - 1e-6) <= most;
+    else if (bounded) {
+      const int others = S - 1, left = L - l;
+      const double largest = fmax(least(l), least((left + others - 1) / others));
+      const double sum = least(l) + (double)others * rest + (double)max(left - 2 * others, 0) * per_layer;
+      in = left >= others && (more * fmax(largest, 0.0) + sum) * (1.0 - 1e-6) <= most;
+    }
+    if (!in) continue;
+    first = min(first, l);
+    last = max(last, l);
+  }
+  for (int step = 32; step > 0; step >>= 1) {
+    first = min(first, __shfl_xor(first, step));
+    last = max(last, __shfl_xor(last, step));
+  }
+  if (lane != 0) return;
+  tabs.reach[gi].first = first;
+  tabs.reach[gi].last = last;
 }
 
 // Sum of a group's stage minima + (G - 1) x the largest (inter_tuning.py:342) into *incumbent.
@@ -4299,7 +4421,7 @@ int check_common(const void *d_problem, const void *d_groups, int n_groups) {
   if (n_groups <= 0) return fail(MIST_E_INVALID, "n_groups must be positive, got %d", n_groups);
   const MistProblem *problem = static_cast<const MistProblem *>(d_problem);
   if (problem->stage_cost_incumbent != nullptr) {
-    if (problem->sample_size != 1)
+    if (problem->sample_size != 1 && problem->incumbent_close != kCloseAssignment)
       return fail(MIST_E_INVALID, "a stage-cost incumbent needs sample_size 1, got %d",
                   problem->sample_size);
     if (problem->incumbent_num_devices < 1 || problem->incumbent_ckpt_rule < 0 ||
@@ -4309,6 +4431,8 @@ int check_common(const void *d_problem, const void *d_groups, int n_groups) {
   }
   if (problem->incumbent_close != 0 && problem->stage_cost_incumbent == nullptr)
     return fail(MIST_E_INVALID, "incumbent_close without a stage-cost incumbent");
+  if (problem->incumbent_close < 0 || problem->incumbent_close > kCloseAssignment)
+    return fail(MIST_E_INVALID, "incumbent_close %d", problem->incumbent_close);
   return 0;
 }
 
@@ -4467,9 +4591,17 @@ static int reduce_tables(const MistProblem *problem, int n_samples, double *d_pa
 static int launch_first_estimate(const MistProblem *problem, const MistGroupDesc *d_groups, int n_groups,
                                  const double *d_row_terms, double ratio, double *d_partial_cost,
                                  double *gather_floor, void *stream) {
-  hipLaunchKernelGGL(estimate_stage_minima_kernel, dim3(kEstimateSplit + (gather_floor ? kGatherBlocks : 0), n_groups),
-                     dim3(256), 0, (hipStream_t)stream, *problem, d_groups, d_row_terms, ratio, d_partial_cost, gather_floor);
+  const bool assignment = problem->incumbent_close == kCloseAssignment;
+  hipLaunchKernelGGL(assignment ? estimate_stage_minima_kernel<true> : estimate_stage_minima_kernel<false>,
+                     dim3(kEstimateSplit + (gather_floor ? kGatherBlocks : 0), n_groups), dim3(256), 0, (hipStream_t)stream,
+                     *problem, d_groups, d_row_terms, assignment ? 1.0 : ratio, d_partial_cost, gather_floor);
   MIST_HIP_CHECK(hipGetLastError());
+  if (assignment) {
+    hipLaunchKernelGGL(estimate_assignment_kernel, dim3(n_groups), dim3(64), 0, (hipStream_t)stream, *problem, d_groups,
+                       d_row_terms, d_partial_cost);
+    MIST_HIP_CHECK(hipGetLastError());
+    return 0;
+  }
   hipLaunchKernelGGL(estimate_combine_kernel, dim3(n_groups), dim3(64), 0, (hipStream_t)stream,
                      *problem, d_groups, d_partial_cost);
   MIST_HIP_CHECK(hipGetLastError());
@@ -4506,7 +4638,8 @@ static int allow_large_lds() {
 constexpr int64_t kCloseItems = 20000;
 static MistProblem closing(const MistProblem *problem, int n_groups, int n_samples) {
   MistProblem own = *problem;
-  if (own.stage_cost_incumbent == nullptr || n_samples != 1 || n_groups > kReachGroups || own.reduce_items < kCloseItems)
+  if (own.incumbent_close == kCloseAssignment ? n_samples == 1
+                                              : n_samples != 1 || n_groups > kReachGroups || own.reduce_items < kCloseItems)
     own.incumbent_close = 0;
   return own;
 }
@@ -4515,9 +4648,14 @@ static MistProblem closing(const MistProblem *problem, int n_groups, int n_sampl
 // second-level summaries) what it says of every group.
 static int launch_incumbent(const MistProblem *problem, const MistGroupDesc *d_groups, int n_groups, const ReduceTables &tabs,
                             void *stream) {
+  if (problem->incumbent_close == kCloseAssignment) {
+    hipLaunchKernelGGL(assignment_reach_kernel, dim3(n_groups), dim3(64), 0, (hipStream_t)stream, *problem, d_groups, tabs);
+    MIST_HIP_CHECK(hipGetLastError());
+    return 0;
+  }
   if (problem->stage_cost_incumbent == nullptr || tabs.n_samples != 1) return 0;
   hipLaunchKernelGGL(incumbent_kernel, dim3(n_groups), dim3(64 * kIncumbentWaves),
-                     problem->incumbent_close != 0 ? n_groups * sizeof(ReachBounds) : 0, (hipStream_t)stream, *problem, d_groups,
+                     problem->incumbent_close == kCloseSearch ? n_groups * sizeof(ReachBounds) : 0, (hipStream_t)stream, *problem, d_groups,
                      tabs);
   MIST_HIP_CHECK(hipGetLastError());
   return 0;
@@ -4549,14 +4687,14 @@ static int launch_seeds(MistProblem *problem, const MistGroupDesc *d_groups, int
   const int64_t bytes = pair_bytes * pair_split * sample_split + sample_waves * (int64_t)sizeof(SampleRows);
   const bool seeds = scouted && bytes <= kSeedLdsMost;  // (some 10000 values of p)
   const bool estimate = scouted && problem->stage_cost_incumbent != nullptr && problem->incumbent_first_estimate != 0 &&
-                        tabs.n_samples == 1;
+                        tabs.n_samples == 1 && problem->sample_size == 1;
   // a first estimate from a few rows, so that the seed launch itself runs under a bound
   if (estimate)
     if (int rc = launch_first_estimate(problem, d_groups, n_groups, d_row_terms, ratios.r[0], d_partial_cost,
-                                       seeds ? tabs.gather_floor : nullptr, stream))
+                                       seeds && tabs.n_samples == 1 ? tabs.gather_floor : nullptr, stream))
       return rc;
   if (!seeds) {
-    problem->incumbent_close = 0;
+    if (problem->incumbent_close == kCloseSearch) problem->incumbent_close = 0;
     hipLaunchKernelGGL(empty_minima_kernel, dim3(kReduceBlocks), dim3(256), 0, (hipStream_t)stream, tabs,
                        problem->reduce_cells);
     MIST_HIP_CHECK(hipGetLastError());
@@ -4584,7 +4722,7 @@ static int launch_seeds(MistProblem *problem, const MistGroupDesc *d_groups, int
 static int launch_super_floors(const MistProblem *problem, const MistGroupDesc *d_groups, int n_groups,
                                const double *d_stage_floor, double ratio, const ReduceTables &tabs, void *stream) {
   hipLaunchKernelGGL(super_floor_kernel, dim3(kSuperBlocks, n_groups), dim3(256), 0, (hipStream_t)stream, d_groups,
-                     n_groups, d_stage_floor, ratio, problem->incumbent_close != 0, tabs);
+                     n_groups, d_stage_floor, problem->incumbent_close == kCloseAssignment ? 1.0 : ratio, problem->incumbent_close, tabs);
   MIST_HIP_CHECK(hipGetLastError());
   return 0;
 }
@@ -4744,6 +4882,7 @@ int mist_eval_reduce_samples(const MistProblem *problem, const MistGroupDesc *d_
     ReduceTables tabs;
     if (int rc = reduce_tables(problem, count, d_partial_cost, d_partial_index, &tabs)) return rc;
     MistProblem own = closing(problem, n_groups, count);
+    if (own.incumbent_close == kCloseAssignment) own.incumbent_close = 0;  // (mist_intra_stage_eval_samples only)
     if (int rc = launch_seeds(&own, d_groups, n_groups, d_row_terms, list, n_scout_blocks > 0, tabs, d_partial_cost,
                               stream))
       return rc;
@@ -4890,15 +5029,26 @@ int mist_intra_stage_eval_samples(const MistProblem *problem, const MistGroupDes
     for (int i = 0; i < count; ++i) list.r[i] = ratios[first + i];
     const bool aside = overlap && first == 0;
     MistProblem own = closing(problem, n_groups, count);
-    if (int rc = launch_seeds(&own, d_groups, n_groups, d_row_terms, list, n_scout_blocks > 0, tabs, d_partial_cost,
-                              aside ? (void *)os->side : stream))
+    // for an assignment only the estimate is formed beside the summaries: they leave few pairs to seed
+    const bool assignment = own.incumbent_close == kCloseAssignment;
+    void *const beside = aside ? (void *)os->side : stream;
+    if (assignment) {
+      if (first == 0 && n_scout_blocks > 0 && own.incumbent_first_estimate != 0)
+        if (int rc = launch_first_estimate(&own, d_groups, n_groups, d_row_terms, 1.0, d_partial_cost, nullptr, beside)) return rc;
+      own.incumbent_first_estimate = 0;
+    } else if (int rc = launch_seeds(&own, d_groups, n_groups, d_row_terms, list, n_scout_blocks > 0, tabs, d_partial_cost,
+                                     beside)) {
       return rc;
+    }
     if (aside) MIST_HIP_CHECK(hipEventRecord(os->seeds_done, os->side));
     // (the summaries' place depends on the number of samples)
     if (int rc = launch_super_floors(&own, d_groups, n_groups, d_stage_floor, list.r[0], tabs, stream)) return rc;
     if (aside) MIST_HIP_CHECK(hipStreamWaitEvent(main_stream, os->seeds_done, 0));
     if (own.incumbent_close != 0)
       if (int rc = launch_incumbent(&own, d_groups, n_groups, tabs, stream)) return rc;
+    if (assignment)
+      if (int rc = launch_seeds(&own, d_groups, n_groups, d_row_terms, list, n_scout_blocks > 0, tabs, d_partial_cost, stream))
+        return rc;
     if (int rc = launch_reduce(&own, d_groups, n_groups, d_reduce_block_prefix, n_reduce_blocks, d_row_terms,
                                d_stage_floor, d_key_terms, list, tabs, stream))
       return rc;

@@ -44,6 +44,10 @@ SCOUT_PAIR_SPAN = 200   # ... one more for every so many pairs of the group (GPT
 # 4.32 with further pairs for every group.  The span makes no difference on GPT-22B: 18.4 ms
 # with one pair, 18.7 - 19.4 with three.)
 SCOUT_TIGHT_FRACTION = 0.3
+# (tile, stage) items of a call from which on cells that are in no assignment near the best are left out: what tells
+# which takes 40 - 80 us (calls of 372 to 1953 items 897 - 1062 us without, 968 - 1105 with; from 2697 on they get
+# faster, 1194 -> 1107, of 40000 by a fifth).
+ASSIGNMENT_MIN_ITEMS = 2500
 SCOUT_TIGHT_PAIRS = 3
 # Upper bound of the row-term workspace (272 bytes per candidate row): the groups of a tuner call
 # go through the kernels in batches of consecutive groups whose rows fit it (a group larger than
@@ -993,7 +997,9 @@ class IntraStageTuner:
         into an upper bound of the best pipeline cost (``MistProblem.stage_cost_incumbent``),
         and the launches behind it do not look for stage costs that no threshold of that search can
         admit.  Cells above that bound then hold some value above it, not their minimum.  With ``close_unused``
-        cells that are in no pipeline below it are not looked for either (``MistProblem.incumbent_close``).
+        cells that are in no pipeline below it are not looked for either (``MistProblem.incumbent_close``).  With
+        ``assignment`` (several samples) the caller reads the tables for the stage assignment of
+        ``uniform-device-pp-mip`` alone, whose optimum it compares with ``dev_plan["incumbent"]``.
 
         ``fill_costs`` False is for a caller that reads the costs of cells with a row index only:
         the tables are not pre-filled with +inf.
@@ -1006,7 +1012,11 @@ class IntraStageTuner:
         sparse = sparse and self.table_samples == 1 and self.cells_wanted is None and self.num_layers <= 255
         problem["sparse_tables"] = sparse
         problem["stage_cost_incumbent"] = problem["incumbent_close"] = 0
-        if stage_cost_cutoff is not None and self.sample_size == 1 and not self.exhaustive:
+        assignment = stage_cost_cutoff is not None and stage_cost_cutoff.get("assignment", False)
+        if assignment and (len(self.sample_slots) == 1 or self.exhaustive
+                           or int(problem["reduce_items"][0]) < ASSIGNMENT_MIN_ITEMS):
+            stage_cost_cutoff = None
+        if stage_cost_cutoff is not None and (self.sample_size == 1 or assignment) and not self.exhaustive:
             with torch.cuda.device(self.device):
                 if "incumbent" not in dev_plan:
                     dev_plan["incumbent"] = torch.empty(1, dtype=torch.float64, device=self.device)
@@ -1017,6 +1027,8 @@ class IntraStageTuner:
             # (all meshes of a table row in one call, side by side)
             problem["incumbent_close"] = (stage_cost_cutoff.get("close_unused", False) and len(dev_plan["batches"]) == 1
                                           and bool(np.all(np.diff(plan["groups"]["g_index"]) >= 0)))
+            if assignment:
+                problem["incumbent_close"] = 2
         with torch.cuda.device(self.device):
             costs, index, struct = self._allocate_flat(plan, fill_costs and not sparse, not sparse)
             self.launch(plan, dev_plan, struct)
@@ -1026,7 +1038,7 @@ class IntraStageTuner:
             tables.planes = dev_plan["planes"] if sparse else None
         return self._outputs(plan, tables)
 
-    def tune_all(self) -> List[IntraStageTunerOutput]:
+    def tune_all(self, stage_cost_cutoff: Optional[dict] = None) -> List[IntraStageTunerOutput]:
         if self.device.type != "cuda" or not torch.cuda.is_available():
             raise _lib.MistLibraryError("IntraStageTuner needs a GPU: the search kernels have no CPU path")
         _lib.load()
@@ -1034,7 +1046,7 @@ class IntraStageTuner:
         with torch.cuda.device(self.device):
             dev_plan = self.upload(plan)
         self._plan, self._dev_plan = plan, dev_plan
-        return self.run_prepared(plan, dev_plan)
+        return self.run_prepared(plan, dev_plan, stage_cost_cutoff)
 
     def tune(self) -> IntraStageTunerOutput:
         if len(self.tp_sizes) != 1:

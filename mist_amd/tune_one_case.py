@@ -128,6 +128,14 @@ def _uniform_device_pp_mip(mist_config, device, stats):
     per_tp = len(Gs) * len(meshes) * (2 * P1 * L * (L + 1) + L * (L + 1) + (L + 1)) * tuning.sample_size * 20
     batch = max(1, min(len(tps), MIP_TABLE_BUDGET_BYTES // max(per_tp, 1)))
     best_cost, best_solution = float("inf"), None
+    # The kernels need not look for layer counts that are in no assignment below an estimate of the best one
+    # (IntraStageTuner.run_prepared): an optimum within the room above it is that of the complete tables, and
+    # otherwise they are evaluated again without it.
+    cutoff = None
+    if (not MIP_EVALUATE_ALL_CELLS and getattr(mist_config, "fixed_ckpt_value", None) is None
+            and os.environ.get("MIST_NO_STAGE_COST_CUTOFF") is None):
+        cutoff = dict(num_devices=hw.num_nodes * hw.num_gpus_per_node, assignment=True,
+                      ckpt_rule=1 if tuning.activation_checkpointing_tuning_enabled else 2)
     for first in range(0, len(tps), batch):
         t0 = time.perf_counter()
         tuner = IntraStageTuner(tables, L, meshes, Gs, tps[first:first + batch], mist_config,
@@ -136,13 +144,31 @@ def _uniform_device_pp_mip(mist_config, device, stats):
             tuner.cells_wanted = mip_cells_wanted(
                 L, hw.num_nodes, hw.num_gpus_per_node, int(getattr(tuning, "layers_offset", 2)))
             tuner.prefill_wanted_cells_only = True  # nothing else of the tables is read below
-        results = tuner.tune_all()
+        results = tuner.tune_all(cutoff)
         t1 = time.perf_counter()
         stats["intra_s"] = stats.get("intra_s", 0.0) + (t1 - t0)
-        # (the strategy rows are read back for the batch's first best candidate only)
-        for cost, solution in inter_stage_tune_batch_mip(
+        incumbent = tuner._dev_plan.get("incumbent")
+        if incumbent is not None:
+            with torch.cuda.device(tuner.device):
+                estimate = torch.empty(1, dtype=torch.float64, pin_memory=True)
+                estimate.copy_(incumbent, non_blocking=True)
+
+        def assigned():  # (the strategy rows are read back for the batch's first best candidate only)
+            return inter_stage_tune_batch_mip(
                 L, hw.num_nodes, hw.num_gpus_per_node, meshes, Gs, results, mist_config, stats=stats,
-                only_best_solution=True):
+                only_best_solution=True)
+
+        outcomes = assigned()
+        room = (1.0 + _lib.load().mist_incumbent_slack()) * (1.0 - 1e-5)
+        if incumbent is not None:
+            torch.cuda.current_stream(tuner.device).synchronize()
+        if incumbent is not None and np.isfinite(float(estimate[0])):
+            stats["mip_estimate"] = float(estimate[0])
+            if not min(cost for cost, _ in outcomes) < float(estimate[0]) * room:
+                stats["mip_second_evaluations"] = stats.get("mip_second_evaluations", 0) + 1
+                results = tuner.run_prepared(tuner._plan, tuner._dev_plan)
+                outcomes = assigned()
+        for cost, solution in outcomes:
             if cost < best_cost:
                 best_cost, best_solution = cost, solution
         stats["inter_s"] = stats.get("inter_s", 0.0) + (time.perf_counter() - t1)
