@@ -4636,11 +4636,14 @@ static int allow_large_lds() {
 // items it does not pay: the estimate then waits for the summaries, too, 10 - 18 us of 342 to 10230 items; from 23520
 // on calls get faster, by 10 - 50 us up to 100000, then more.
 constexpr int64_t kCloseItems = 20000;
-static MistProblem closing(const MistProblem *problem, int n_groups, int n_samples) {
+static MistProblem closing(const MistProblem *problem, int n_groups, int n_samples, bool assignments = true) {
   MistProblem own = *problem;
-  if (own.incumbent_close == kCloseAssignment ? n_samples == 1
-                                              : n_samples != 1 || n_groups > kReachGroups || own.reduce_items < kCloseItems)
+  if (own.incumbent_close == kCloseAssignment) {
+    // an estimate of the assignments bounds no stage cost at one of the samples
+    if (n_samples == 1 || !assignments) own.incumbent_close = 0, own.stage_cost_incumbent = nullptr;
+  } else if (n_samples != 1 || n_groups > kReachGroups || own.reduce_items < kCloseItems) {
     own.incumbent_close = 0;
+  }
   return own;
 }
 
@@ -4881,8 +4884,7 @@ int mist_eval_reduce_samples(const MistProblem *problem, const MistGroupDesc *d_
     for (int i = 0; i < count; ++i) list.r[i] = ratios[first + i];
     ReduceTables tabs;
     if (int rc = reduce_tables(problem, count, d_partial_cost, d_partial_index, &tabs)) return rc;
-    MistProblem own = closing(problem, n_groups, count);
-    if (own.incumbent_close == kCloseAssignment) own.incumbent_close = 0;  // (mist_intra_stage_eval_samples only)
+    MistProblem own = closing(problem, n_groups, count, false);
     if (int rc = launch_seeds(&own, d_groups, n_groups, d_row_terms, list, n_scout_blocks > 0, tabs, d_partial_cost,
                               stream))
       return rc;
