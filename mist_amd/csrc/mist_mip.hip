@@ -1,9 +1,10 @@
 // Stage-assignment search of the `uniform-device-pp-mip` granularity
 // (reference: mist/analyzer/inter_tuning_mip.py).
 //
-//   stage_samples_kernel  one workgroup (one wavefront) per (stage, layer count): stages the
-//                         candidate row in LDS as float32 pairs, lane a scans it for sample a,
-//                         then the lanes compare their picks to drop repeated pairs.
+//   stage_samples_kernel  one workgroup per (stage, layer count): stages the candidate row in LDS
+//                         as float32 pairs; several threads per sample scan a share of it each,
+//                         then one per sample takes the best share and the samples compare
+//                         their picks to drop repeated pairs.
 //   mist_mip_solve        host: exact optimum of the assignment the reference gives to CBC.
 //
 // Why the host solver is exact.  For fixed stage choices let Z_0 = 0, Z_{i+1} = T_i + max(Z_i,
@@ -26,7 +27,27 @@ using mist::fail;
 
 namespace {
 
-constexpr int kSampleLanes = 64;
+constexpr int kSampleLanes = 64;  // most samples
+// Threads per row.  A row is bound by its chain of LDS reads and compares, one per candidate (there are (L + 1) * P),
+// not by the 16 bytes per candidate that it reads: the candidates of a sample are shared among threads, and those
+// behind the last finite one are left out (a row of l layers has no checkpoint count above l).  With one thread per
+// sample over all of them the rows of the 7B plan with 30 samples took 177 us on 4x8 and 74 us on 1x8; shared 88 and
+// 39; without the infinite tail 45 and 21.
+constexpr int kSampleThreads = 256;
+constexpr int kMostShares = 16;  // the shares are compared one after the other
+
+// What one thread's share of the candidates gives.
+struct SharePick {
+  double cost;
+  int index;
+  float x, y;
+};
+
+// LDS of a row of n_cand candidates: the row, later the shares' picks in its place, and the picks.
+int64_t sample_lds_bytes(int64_t n_cand) {
+  const int64_t row = 2 * n_cand * (int64_t)sizeof(float), shares = kSampleThreads * (int64_t)sizeof(SharePick);
+  return std::max(row, shares) + 2 * kSampleLanes * (int64_t)sizeof(float);
+}
 
 struct StageRow {
   const double *stable, *delta;  // first candidate of the row, nullptr = every candidate +inf
@@ -66,30 +87,52 @@ __device__ __forceinline__ void stage_samples_row(
   else if (shape.ckpt_mode == MIST_MIP_CKPT_FIXED) first = shape.fixed_ckpt * P;
   else first = layers * P;
 
-  float *x = lds, *y = lds + n_cand;
-  float *pick_x = y + n_cand, *pick_y = pick_x + kSampleLanes;
+  float2 *xy = reinterpret_cast<float2 *>(lds);
+  float *pick_x = lds + max(2 * n_cand, (int)(kSampleThreads * sizeof(SharePick) / sizeof(float)));
+  float *pick_y = pick_x + kSampleLanes;
   const StageRow row = stage_row(shape, tables, stage, layers);
-  for (int n = lane; n < n_cand; n += kSampleLanes) {
-    x[n] = row.stable ? (float)row.stable[first + n] : INFINITY;
-    y[n] = row.delta ? (float)row.delta[first + n] : INFINITY;
+  int end = 0;  // behind the last candidate with a cost below +inf
+  for (int n = lane; n < n_cand; n += kSampleThreads) {
+    const float2 v = row.stable ? make_float2((float)row.stable[first + n], (float)row.delta[first + n])
+                                : make_float2(INFINITY, INFINITY);
+    xy[n] = v;
+    if (v.x < INFINITY && v.y < INFINITY) end = n + 1;
   }
+  for (int k = 32; k > 0; k >>= 1) end = max(end, __shfl_xor(end, k));
+  int *ends = reinterpret_cast<int *>(pick_x);
+  if ((lane & 63) == 0) ends[lane >> 6] = end;
+  __syncthreads();
+  end = ends[0];
+  for (int k = 1; k < kSampleThreads / 64; ++k) end = max(end, ends[k]);
+
+  const int shares = min(kSampleThreads / P, kMostShares), share = lane / P;
+  SharePick pick = {INFINITY, -1, 0.0f, 0.0f};
+  if (share < shares) {
+    const double r = ratios[lane % P];
+    for (int n = share; n < end; n += shares) {
+      const float2 v = xy[n];
+      const double cost = r * (double)v.x + (double)v.y;
+      if (cost < pick.cost) pick.cost = cost, pick.index = n;
+    }
+  }
+  // numpy reads index -1 as the last candidate (pareto.py:76-77)
+  const float2 chosen = xy[pick.index >= 0 ? pick.index : n_cand - 1];
+  pick.x = chosen.x, pick.y = chosen.y;
+  SharePick *of_share = reinterpret_cast<SharePick *>(lds);
+  __syncthreads();
+  of_share[lane] = pick;
   __syncthreads();
 
   int best = -1;
   float sx = 0.0f, sy = 0.0f;
   if (lane < P) {
-    const double r = ratios[lane];
-    double best_cost = INFINITY;
-    for (int n = 0; n < n_cand; ++n) {
-      const double cost = r * (double)x[n] + (double)y[n];
-      if (cost < best_cost) {
-        best_cost = cost;
-        best = n;
-      }
+    for (int k = 1; k < shares; ++k) {  // the first candidate of the least cost
+      const SharePick &other = of_share[k * P + lane];
+      if (other.cost < pick.cost || (other.cost == pick.cost && other.index >= 0 && other.index < pick.index)) pick = other;
     }
-    // numpy reads index -1 as the last candidate (pareto.py:76-77)
-    sx = x[best >= 0 ? best : n_cand - 1];
-    sy = y[best >= 0 ? best : n_cand - 1];
+    best = pick.index;
+    sx = pick.x;
+    sy = pick.y;
     pick_x[lane] = sx;
     pick_y[lane] = sy;
   }
@@ -109,22 +152,22 @@ __device__ __forceinline__ void stage_samples_row(
   out_keep[o] = keep ? 1 : 0;
 }
 
-__global__ __launch_bounds__(kSampleLanes) void stage_samples_kernel(
+__global__ __launch_bounds__(kSampleThreads) void stage_samples_kernel(
     MistMipShape shape, MistMipTables tables, const double *__restrict__ ratios,
     float *__restrict__ out_stable, float *__restrict__ out_delta, int32_t *__restrict__ out_index,
     uint8_t *__restrict__ out_keep) {
-  extern __shared__ float lds[];
+  extern __shared__ __align__(8) float lds[];
   stage_samples_row(shape, tables, blockIdx.x, lds, ratios, out_stable, out_delta, out_index,
                     out_keep);
 }
 
 // Every problem of a search in one launch: workgroup -> (problem, row) through the problems'
 // first workgroups (ascending); outputs of problem i start at its out_offset.
-__global__ __launch_bounds__(kSampleLanes) void stage_samples_batch_kernel(
+__global__ __launch_bounds__(kSampleThreads) void stage_samples_batch_kernel(
     const MistMipBatchItem *__restrict__ items, int n_items, const double *__restrict__ ratios,
     float *__restrict__ out_stable, float *__restrict__ out_delta, int32_t *__restrict__ out_index,
     uint8_t *__restrict__ out_keep) {
-  extern __shared__ float lds[];
+  extern __shared__ __align__(8) float lds[];
   int lo = 0, hi = n_items;  // items[lo].first_block <= blockIdx.x < items[hi].first_block
   while (hi - lo > 1) {
     const int mid = (lo + hi) >> 1;
@@ -220,7 +263,7 @@ int mist_mip_stage_samples(const MistMipShape *shape, const MistMipTables *table
                 (long long)n_cand);
   const int nl = shape->layers_max - shape->layers_min + 1;
   hipLaunchKernelGGL(stage_samples_kernel, dim3((unsigned)(shape->num_stages * nl)),
-                     dim3(kSampleLanes), (size_t)lds_bytes, (hipStream_t)stream, *shape, *tables,
+                     dim3(kSampleThreads), (size_t)sample_lds_bytes(n_cand), (hipStream_t)stream, *shape, *tables,
                      d_ratios, d_t_stable, d_t_delta, d_index, d_keep);
   MIST_HIP_CHECK(hipGetLastError());
   return 0;
@@ -236,7 +279,7 @@ int mist_mip_stage_samples_batch(const MistMipBatchItem *items, const MistMipBat
     return fail(MIST_E_INVALID, "null / empty problem list (n_items=%d)", n_items);
   if (!d_ratios || !d_t_stable || !d_t_delta || !d_index || !d_keep)
     return fail(MIST_E_INVALID, "null pointer");
-  int64_t blocks = 0, lds_bytes = 0, out = 0;
+  int64_t blocks = 0, lds_bytes = 0, lds_used = 0, out = 0;
   for (int i = 0; i < n_items; ++i) {
     const MistMipShape *s = &items[i].shape;
     if (int rc = check_mip_shape(s)) return rc;
@@ -252,12 +295,13 @@ int mist_mip_stage_samples_batch(const MistMipBatchItem *items, const MistMipBat
     const int64_t n_cand = s->ckpt_mode == MIST_MIP_CKPT_TUNED
                                ? (int64_t)(s->num_layers + 1) * s->sample_size : s->sample_size;
     lds_bytes = std::max<int64_t>(lds_bytes, (2 * n_cand + 2 * kSampleLanes) * (int64_t)sizeof(float));
+    lds_used = std::max(lds_used, sample_lds_bytes(n_cand));
   }
   if (lds_bytes > 64 * 1024)
     return fail(MIST_E_INVALID, "candidates per table row exceed the LDS staging buffer");
   if (blocks >= (int64_t)1 << 31) return fail(MIST_E_INVALID, "too many rows for one launch");
-  hipLaunchKernelGGL(stage_samples_batch_kernel, dim3((unsigned)blocks), dim3(kSampleLanes),
-                     (size_t)lds_bytes, (hipStream_t)stream, d_items, n_items, d_ratios,
+  hipLaunchKernelGGL(stage_samples_batch_kernel, dim3((unsigned)blocks), dim3(kSampleThreads),
+                     (size_t)lds_used, (hipStream_t)stream, d_items, n_items, d_ratios,
                      d_t_stable, d_t_delta, d_index, d_keep);
   MIST_HIP_CHECK(hipGetLastError());
   return 0;

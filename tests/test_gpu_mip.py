@@ -89,6 +89,26 @@ def test_sampling_kernel_matches_oracle_preprocessing(mode, L, P1, P, quantum):
             assert np.array_equal(got_i, pol[:, lo:hi + 1])
 
 
+@pytest.mark.parametrize("L,P,first_inf", [(3, 1, 4), (7, 64, 3), (9, 17, 0), (16, 16, 1), (20, 33, 21)])
+def test_sampling_kernel_shares_and_tails(L, P, first_inf):
+    """A sample's candidates shared among threads (256 / P of them, at most 16): equal costs in different shares take
+    the lowest candidate, planes from ``first_inf`` on hold nothing finite."""
+    from oracle import inter_mip
+
+    rng = np.random.default_rng(L * P)
+    stable, delta = _random_tables(rng, 3, L, P, quantum=0.5)
+    for t in stable + delta:
+        t[..., first_inf:, :] = np.inf
+    f32 = lambda a: a.astype(np.float32)
+    choices, want_s, want_d, (ck, pol) = inter_mip.preprocess_stable_and_delta_costs(
+        3, True, None, *[f32(t[v]) for v in range(4) for t in (stable, delta)])
+    got_s, got_d, got_i, got_k = _gpu_samples(stable, delta, 3, 1, L, 0, 0)
+    assert np.array_equal(got_s, want_s[:, 1:]) and np.array_equal(got_d, want_d[:, 1:])
+    assert np.array_equal(got_i // P, ck[:, 1:]) and np.array_equal(got_i % P, pol[:, 1:])
+    assert [[list(np.flatnonzero(k)) for k in row] for row in got_k] == [
+        [sorted(choices[i][j]) for j in range(1, L + 1)] for i in range(3)]
+
+
 def test_sampling_kernel_rejects_bad_arguments():
     import torch
     from mist_amd import _lib
