@@ -1442,9 +1442,11 @@ constexpr int kLogTaken = 3 * kQueueShards + kNumXcd;  // counters: chunks taken
 constexpr int kLogFull = kLogTaken + 1;
 constexpr int kGroupsDone = kLogFull + 1;  // workgroups of the estimate that have ended
 constexpr int kCounters = kGroupsDone + 1;
+constexpr int kOpenPairs = 1;  // words behind the counter of a shard's opened items: their open pairs
 constexpr int kSeedThreads = 256;
 constexpr int kReduceThreads = 256;
 constexpr int kReduceBlocks = 2048;          // a multiple of kNumXcd
+constexpr int kReduceWorkers = 768;           // three per CU, as many as are resident: 2048 end 6 us later
 constexpr int kAgainBlocks = 768;            // three per CU: as a rule they return at once
 constexpr int kStageRowsBlocks = 1024;       // four per CU, two stages at a time each
 constexpr int kSuperBlocks = 64;             // workgroups per group of the second-level summaries
@@ -1520,7 +1522,7 @@ struct ReduceTables {
   // per stage summary) tells whether one is listed.  Null: the rows of all stages are there.
   unsigned long long *listed;
   uint32_t *stage_flag;
-  // at kCounterPitch: [kQueueShards] items, [kQueueShards] opened, [kQueueShards] listed, [kNumXcd] drawn,
+  // at kCounterPitch: [kQueueShards] items, [kQueueShards] opened (with their pairs), [kQueueShards] listed, [kNumXcd] drawn,
   // kLogTaken, kLogFull, kGroupsDone
   uint32_t *counter;
   uint32_t capacity, log_chunks;
@@ -2017,7 +2019,8 @@ struct Threshold {
 // ---- seeds ----
 __device__ __forceinline__ void clear_queue(const ReduceTables &tabs) {
   if (blockIdx.x == 0 && blockIdx.y == 0)
-    for (int i = threadIdx.x; i < kCounters; i += blockDim.x) tabs.counter[i * kCounterPitch] = 0;
+    for (int i = threadIdx.x; i < kCounters; i += blockDim.x)
+      tabs.counter[i * kCounterPitch] = tabs.counter[i * kCounterPitch + kOpenPairs] = 0;
 }
 
 // Smallest linear bounds of 64 gathered rows at a time, for the seed launch: workgroup `part` of
@@ -2716,19 +2719,24 @@ __global__ __launch_bounds__(kReduceThreads) void open_kernel(const MistProblem 
   uint64_t kept_word = 0, kept_open = 0;
   uint32_t kept_shard = 0;
   int n_kept = 0;
+  uint32_t kept_pairs = 0;
   auto append = [&]() {
     if (n_kept == 0) return;
     const bool mine = lane < n_kept;
     const int64_t shard0 = (int64_t)kept_shard * tabs.capacity;
     // (no more than the shard's items are opened: it cannot overflow)
     uint32_t base = 0;
-    if (lane == 0) base = atomicAdd(tabs.counter + (kQueueShards + kept_shard) * kCounterPitch, (uint32_t)n_kept);
+    static_assert(kOpenPairs == 1, "both counters in one word");
+    if (lane == 0)
+      base = (uint32_t)atomicAdd(reinterpret_cast<unsigned long long *>(tabs.counter + (kQueueShards + kept_shard) * kCounterPitch),
+                                 (unsigned long long)kept_pairs << 32 | (uint32_t)n_kept);
     base = (uint32_t)from_lane((int)base, 0);
     if (mine) {
       tabs.opened[shard0 + base + lane] = kept_word;
       tabs.open_pairs[shard0 + base + lane] = kept_open;
     }
     n_kept = 0;
+    kept_pairs = 0;
     if (tabs.listed == nullptr) return;
     const Item item(kept_word);
     bool fresh = false;
@@ -2812,6 +2820,7 @@ __global__ __launch_bounds__(kReduceThreads) void open_kernel(const MistProblem 
         kept_open = open;
       }
       ++n_kept;
+      kept_pairs += __popcll(open);
     }
     append();
   }
@@ -3410,10 +3419,20 @@ __global__ __launch_bounds__(kReduceThreads, 3) void reduce_kernel(
                                     lds_rows + local_wave * wave_pitch, log);
   };
   const FlatQueue queue = flat_queue(tabs, 1);
-  // enough units for every wavefront several times over; a pair of several samples takes longer (30 samples
-  // of one tensor-parallel size of the 7B plan: 64 pairs a unit 2.36 ms, 32 2.12, 16 2.09)
+  // Units enough for every wavefront, and not too long ones; a pair of several samples takes longer (30 samples
+  // of one tensor-parallel size of the 7B plan: 64 pairs a unit 2.36 ms, 32 2.12, 16 2.09).  A unit costs some
+  // 8 us of loads that wait for each other before its first pair, so that splits beyond what fills the chip cost:
+  // 3700 items of 9 pairs (7B on 4x8) 1, 2, 3 and 4 halvings 68, 73, 111 and 189 us, 14800 of 10 (13B on 8x8) none to
+  // three 180, 190, 267 and 386; 6200 of 26 (uniform-pp of 7B on 2x8), where a few long units would be the launch's
+  // end, none to four 279, 207, 190, 195 and 273.  (The pairs' sum may wrap: any split is right.)
+  uint32_t n_pairs = tabs.counter[(kQueueShards + lane) * kCounterPitch + kOpenPairs];
+  for (int k = 32; k > 0; k >>= 1) n_pairs += (uint32_t)__shfl_xor((int)n_pairs, k);
+  n_pairs = (uint32_t)from_lane((int)n_pairs, 0);
   int split = kSamples ? 2 : 0;
-  while (split < 4 && ((uint64_t)queue.total << split) < (uint64_t)n_waves * 2) ++split;
+  for (uint64_t units; split < 4; ++split) {
+    units = (uint64_t)queue.total << split;
+    if (units >= n_waves * 2 && (units >= n_waves * 8 || n_pairs <= 12 * units)) break;
+  }
   const uint64_t units = (uint64_t)queue.total << split;
   if (kResolve) {  // handed out in turn
     for (uint64_t u = (uint64_t)blockIdx.x * kWaves + local_wave; u < units; u += n_waves) {
@@ -4755,7 +4774,7 @@ static int launch_reduce(const MistProblem *problem, const MistGroupDesc *d_grou
   if (lds > 64 * 1024)
     if (int rc = allow_large_lds()) return rc;
 #define MIST_REDUCE(RESOLVE, SAMPLES, IN_LDS)                                                               \
-  hipLaunchKernelGGL((reduce_kernel<RESOLVE, SAMPLES, IN_LDS>), dim3(RESOLVE ? kAgainBlocks : kReduceBlocks),    \
+  hipLaunchKernelGGL((reduce_kernel<RESOLVE, SAMPLES, IN_LDS>), dim3(RESOLVE ? kAgainBlocks : kReduceWorkers),    \
                      dim3(kReduceThreads), lds, (hipStream_t)stream, *problem, d_groups, d_row_terms, d_stage_floor, ratios, tabs, wave_pitch)
   if (!one) MIST_REDUCE(false, true, false);
   else if (buffered) MIST_REDUCE(false, false, true);
