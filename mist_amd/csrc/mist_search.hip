@@ -1432,12 +1432,14 @@ constexpr double kCandidateRoom = 16.0;  // two widenings of a window of thresho
 constexpr int kGatherFloor = 5;    // linear bounds of 64 gathered rows
 constexpr int kQueueShards = 64;   // counters of the item queue: one would serve an append in ~8 ns
 constexpr int kCounterPitch = 32;  // uint32 between counters: a cache line each
-// Entries of the log that a reduce wavefront takes at a time, and the most entries of a log: 16 bytes each; 7e6
-// with 30 samples of one tensor-parallel size of the 7B plan, 5e6 of 70B on 32x8, 11e6 of searches whose bound
-// prunes little, 0.1 to 2 per entry of the minima elsewhere.
+// Entries of the log that a reduce wavefront takes at a time, and the most entries of a log, 16 bytes each.  Used are
+// 0.1 to 2 per entry of the minima as a rule (13e6 with 30 samples of one tensor-parallel size of the 7B plan), but
+// 20e6 = 5 per entry of 70B with 48 layers on 25x8 and 39e6 = 2 of 75 layers on 8x8, both without checkpoint tuning,
+// whose bound prunes little; a log that runs full costs three times the resolve launch it replaced (the two calls
+// with room for 4 per entry and 25e6 at most: 11.1 and 30.5 ms, now 8.3 and 21.9, without a log 9.2 and 28.6).
 constexpr int kLogChunk = 256;
-constexpr int64_t kLogEntries = 24 << 20;
-constexpr int kLogPerCell = 4;
+constexpr int64_t kLogEntries = 96 << 20;
+constexpr int kLogPerCell = 8;
 constexpr int kLogTaken = 3 * kQueueShards + kNumXcd;  // counters: chunks taken, whether there were too few
 constexpr int kLogFull = kLogTaken + 1;
 constexpr int kGroupsDone = kLogFull + 1;  // workgroups of the estimate that have ended
