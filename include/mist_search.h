@@ -135,6 +135,7 @@ typedef struct MistProblem {
    * in no pipeline of stages up to bound(G) may hold +inf / -1 or another row than its minimum's, as long as it
    * then is below every threshold candidate which that search reads: those from 16 (1e-4 s + 1e-5 x) below the
    * smallest largest stage cost x of a pipeline on.
+   * (None does where the incumbent stays +inf.)
    * 2 (with stage_cost_incumbent, whatever the sample_size; calls with several samples): for a caller that reads
    * the tables for the stage assignment only (mist_mip.h; incumbent_ckpt_rule 1 or 2).  The incumbent becomes the
    * objective of an assignment of rows that the tables may or may not hold, and a (group, layers) that is in no

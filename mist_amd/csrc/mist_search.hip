@@ -3685,7 +3685,8 @@ struct PipelineLayers {
 // 8x8 1920 -> 1615, 22B on 16x8 9000 -> 7190, 70B on 32x8 5720 -> 4290, 1.3B on 1x2 the same.  (Closed in the seeds
 // already, by about the same from the first estimate: they spend their time on the first rows of a pair; 70B 4290
 // -> 4230, 13B uniform-device-pp 1470 -> 1600.)
-// (Where a row may cost less the more layers it has - a negative share of the first micro-batch - nothing is closed.)
+// (Where a row may cost less the more layers it has - a negative share of the first micro-batch - nothing is closed,
+// and neither is without an estimate: bound(G) is infinite then, but `low` would not be.)
 // The workgroup `reach` is formed by; all its threads.
 struct ReachBounds {
   double per_layer, rest;
@@ -3718,6 +3719,10 @@ __device__ __forceinline__ void form_reach(const MistProblem &prob, const MistGr
     reach[gi].cutoff = load * D * (1.0 + 1e-9) < L ? -INFINITY : bound;
     reach[gi].first = (int)fmax(ceil(L - load * (D - (double)bounds[gi].devices) * (1.0 + 1e-9)), 0.0);
     reach[gi].low = cheapest * (1.0 - 1e-6) - kCandidateRoom * (1e-4 + 1e-5 * fabs(cheapest));
+    if (!(incumbent < INFINITY)) {  // (no estimate: what reads the tables takes them for complete)
+      reach[gi].first = 0;
+      reach[gi].low = -INFINITY;
+    }
   }
 }
 

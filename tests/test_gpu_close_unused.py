@@ -48,6 +48,32 @@ def test_random_plans_with_closed_cells(seed):
     _compare(_realistic_plan(seed))
 
 
+@pytest.mark.parametrize("plan, layers, memory, device", [
+    (3, 37, 3.0, False), (3, 37, 4.0, False), (5, 79, 6.0, False), (3, 37, 3.0, True),
+])
+def test_tables_without_an_estimate_are_complete(plan, layers, memory, device):
+    """Little memory and layers that no stage count divides: the only pipeline of equal stages is one on all devices,
+    which does not fit, so there is no estimate though there are results.  What reads the tables takes them for
+    complete then: no cell is closed (one of the mesh of all devices would be, whose layers are not all there are)."""
+    from mist_amd.tune_one_case import PreparedSearch
+
+    overrides = dict(tuning__tuning_granularity="uniform-device-pp") if device else {}
+    search = PreparedSearch(load_plan(plan, model__num_hidden_layers=layers, hardware__num_nodes=4 if plan == 3 else 8,
+                                      training__global_batch_size=256, hardware__memory_capacity=memory, **overrides)[0])
+    cost, solution = search.run()
+    assert solution is not None and search.dev_plan["incumbent"].item() == float("inf")
+    closed = search.tuner.run_prepared(search.plan, search.dev_plan, search.stage_cost_cutoff)[0].batch
+    without = dict(search.stage_cost_cutoff, close_unused=False)
+    open_ = search.tuner.run_prepared(search.plan, search.dev_plan, without)[0].batch
+    for v in range(4):
+        has = open_.index[v] >= 0
+        assert bool((closed.index[v] == open_.index[v]).all())
+        for ours, theirs in ((closed.stable, open_.stable), (closed.delta, open_.delta)):
+            assert bool((ours[v][has] == theirs[v][has]).all())
+    search.stage_cost_cutoff = None
+    assert search.run() == (cost, solution)
+
+
 @pytest.mark.parametrize("dense", [False, True])
 def test_windows_that_reach_below_what_such_tables_hold(dense):
     """A window whose threshold candidates have no certain start within two widenings (values half a gap apart, in
