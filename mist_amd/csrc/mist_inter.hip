@@ -36,6 +36,7 @@
 #include "mist_dp.h"
 #include "mist_dp_rates.h"
 #include "mist_inter.h"
+#include "mist_window_margin.h"
 
 using mist::fail;
 
@@ -99,8 +100,6 @@ struct Workspace {
 std::mutex g_lock;  // one search at a time per process: the workspaces are shared
 std::map<int, Workspace> g_workspaces;
 
-constexpr int kExactWidenings = 2;  // (kCandidateRoom of mist_search.hip is the room they take)
-
 struct Window {
   bool exists = false;
   int row = 0, G = 1;
@@ -112,7 +111,7 @@ struct Window {
   bool complete = false;
 
   float lower_margin(int widen) const {
-    const double step = (1e-4 + 1e-5 * std::fabs((double)start_value)) * std::pow(4.0, widen);
+    const double step = mist::window_margin((double)start_value) * std::pow(mist::kMarginGrowth, widen);
     return start_value - (float)step;
   }
   void append(const float *values, size_t n) {
@@ -189,7 +188,7 @@ __global__ void window_request_kernel(const float *__restrict__ out, int n_famil
   const double room = (G - 1.0) * (4.0 * gap);
   float hi = nextafterf((float)((cost0 + room) * (1.0 + 1e-5) / G), INFINITY);
   hi = fmaxf(hi, (float)((double)bott * (1.0 + 2e-3) + 2e-4));
-  req[n + i] = bott - (float)(1e-4 + 1e-5 * fabs((double)bott));
+  req[n + i] = bott - (float)mist::window_margin((double)bott);
   req[2 * n + i] = hi;
 }
 
@@ -920,7 +919,7 @@ static int search_families(int n_families, const MistDpShape *shapes,
     for (size_t k = 0; k < pending.size(); ++k) pending[k] = (int)k;
     for (int widen = 0; !pending.empty(); ++widen) {
       // (tables under an estimate need not hold their values below: MistProblem.incumbent_close)
-      if (widen > kExactWidenings && host_estimate != nullptr && std::isfinite(*host_estimate)) too_wide += (int)pending.size();
+      if (widen > mist::kExactWidenings && host_estimate != nullptr && std::isfinite(*host_estimate)) too_wide += (int)pending.size();
       if (widen > 0) {
         std::vector<int32_t> r;
         lo.clear();

@@ -17,6 +17,7 @@
 
 #include "mist_common.h"
 #include "mist_search.h"
+#include "mist_window_margin.h"
 #define MIST_ARITH_FN __device__ __forceinline__
 #include "exact_arith.h"
 
@@ -1428,7 +1429,6 @@ __device__ __forceinline__ void take_min(double &best, int32_t &best_row, bool f
 // now 3.2 (reduce 2.1, open 0.42, seeds 0.33, filter 0.17, resolve 0.08).
 // ------------------------------------------------------------------------------------------
 constexpr int kSuperStages = 8;    // stages per second-level summary
-constexpr double kCandidateRoom = 16.0;  // two widenings of a window of threshold candidates (mist_inter.hip)
 constexpr int kGatherFloor = 5;    // linear bounds of 64 gathered rows
 constexpr int kQueueShards = 64;   // counters of the item queue: one would serve an append in ~8 ns
 constexpr int kCounterPitch = 32;  // uint32 between counters: a cache line each
@@ -3677,7 +3677,7 @@ struct PipelineLayers {
 //    its share of them, and no mesh takes more than `load` layers a device at a cost up to bound(G): what leaves
 //    more is in no such pipeline, and no stage of the table row is if all layers are more than D devices take.
 //  - The most expensive stage of every pipeline costs at least what the cheapest mesh takes for its share of all
-//    layers.  That search reads stage costs as threshold candidates from kCandidateRoom below the smallest largest
+//    layers.  That search reads stage costs as threshold candidates from kExactMargins below the smallest largest
 //    cost on: of what is in no pipeline, a minimum below that is as good as any other value below it.
 // So a pair of fewer than `first` layers is left alone once its minimum is below `low`: 70 - 80 % of the pairs with
 // a minimum up to bound(G) on clusters of a power of two of nodes, 33 - 65 % on others (a mesh of all devices is
@@ -3718,7 +3718,7 @@ __device__ __forceinline__ void form_reach(const MistProblem &prob, const MistGr
     for (int i = gi + 1; i < n_groups && bounds[i].row == row; ++i) add(bounds[i]);
     reach[gi].cutoff = load * D * (1.0 + 1e-9) < L ? -INFINITY : bound;
     reach[gi].first = (int)fmax(ceil(L - load * (D - (double)bounds[gi].devices) * (1.0 + 1e-9)), 0.0);
-    reach[gi].low = cheapest * (1.0 - 1e-6) - kCandidateRoom * (1e-4 + 1e-5 * fabs(cheapest));
+    reach[gi].low = cheapest * (1.0 - 1e-6) - mist::kExactMargins * mist::window_margin(cheapest);
     if (!(incumbent < INFINITY)) {  // (no estimate: what reads the tables takes them for complete)
       reach[gi].first = 0;
       reach[gi].low = -INFINITY;
