@@ -4658,16 +4658,13 @@ static int allow_large_lds() {
   return 0;
 }
 
-// The problem as the launches of one call take it: whether cells are closed is decided here.  For few (tile, stage)
-// items it does not pay: the estimate then waits for the summaries, too, 10 - 18 us of 342 to 10230 items; from 23520
-// on calls get faster, by 10 - 50 us up to 100000, then more.
-constexpr int64_t kCloseItems = 20000;
+// The problem as the launches of one call take it: cells are closed where form_reach has room for the groups.
 static MistProblem closing(const MistProblem *problem, int n_groups, int n_samples, bool assignments = true) {
   MistProblem own = *problem;
   if (own.incumbent_close == kCloseAssignment) {
     // an estimate of the assignments bounds no stage cost at one of the samples
     if (n_samples == 1 || !assignments) own.incumbent_close = 0, own.stage_cost_incumbent = nullptr;
-  } else if (n_samples != 1 || n_groups > kReachGroups || own.reduce_items < kCloseItems) {
+  } else if (n_samples != 1 || n_groups > kReachGroups) {
     own.incumbent_close = 0;
   }
   return own;

@@ -44,11 +44,15 @@ SCOUT_PAIR_SPAN = 200   # ... one more for every so many pairs of the group (GPT
 # 4.32 with further pairs for every group.  The span makes no difference on GPT-22B: 18.4 ms
 # with one pair, 18.7 - 19.4 with three.)
 SCOUT_TIGHT_FRACTION = 0.3
+SCOUT_TIGHT_PAIRS = 3
 # (tile, stage) items of a call from which on cells that are in no assignment near the best are left out: what tells
 # which takes 40 - 80 us (calls of 372 to 1953 items 897 - 1062 us without, 968 - 1105 with; from 2697 on they get
 # faster, 1194 -> 1107, of 40000 by a fifth).
 ASSIGNMENT_MIN_ITEMS = 2500
-SCOUT_TIGHT_PAIRS = 3
+# ... and those of a call whose search over tables under an estimate gets no cells that are in no pipeline below it:
+# the estimate then waits for the summaries, 10 - 18 us of calls of 342 to 10230 items; from 23520 on calls get
+# faster, by 10 - 50 us up to 100000, then more.
+CLOSE_MIN_ITEMS = 20000
 # Upper bound of the row-term workspace (272 bytes per candidate row): the groups of a tuner call
 # go through the kernels in batches of consecutive groups whose rows fit it (a group larger than
 # the bound is a batch of its own); with more than one batch two such workspaces alternate.  Only
@@ -1026,6 +1030,7 @@ class IntraStageTuner:
             problem["incumbent_ckpt_rule"] = int(stage_cost_cutoff["ckpt_rule"])
             # (all meshes of a table row in one call, side by side)
             problem["incumbent_close"] = (stage_cost_cutoff.get("close_unused", False) and len(dev_plan["batches"]) == 1
+                                          and int(problem["reduce_items"][0]) >= CLOSE_MIN_ITEMS
                                           and bool(np.all(np.diff(plan["groups"]["g_index"]) >= 0)))
             if assignment:
                 problem["incumbent_close"] = 2

@@ -13,6 +13,26 @@ def _plan(plan, layers, nodes, batch, tuned, samples=30):
                      tuning__activation_checkpointing_tuning_enabled=tuned)[0]
 
 
+def _cells_with_a_row(monkeypatch):
+    """How many cells of the tables hold a row, call by call."""
+    from mist_amd import intra_tuning
+
+    run, held = intra_tuning.IntraStageTuner.run_prepared, []
+
+    def counted(tuner, *args, **kwargs):
+        out = run(tuner, *args, **kwargs)
+        wanted = tuner._plan["wanted"]
+        n = 0
+        for g, q in zip(*(wanted[:, :, 0] >= 0).nonzero()):
+            first, last, planes = (int(x) for x in wanted[g, q, :3])
+            n += int((out[0].batch.index[2][g::wanted.shape[0], q, first - 1:last] >= 0).sum())
+        held.append(n)
+        return out
+
+    monkeypatch.setattr(intra_tuning.IntraStageTuner, "run_prepared", counted)
+    return held
+
+
 @pytest.mark.parametrize("plan, layers, nodes, batch, tuned, samples", [
     (2, 32, 4, 512, True, 30),
     (2, 17, 2, 64, True, 7),     # layers that no stage count divides
@@ -27,11 +47,13 @@ def test_assignment_over_the_cells_left(monkeypatch, plan, layers, nodes, batch,
 
     monkeypatch.setattr(intra_tuning, "ASSIGNMENT_MIN_ITEMS", 0)
     cfg = _plan(plan, layers, nodes, batch, tuned, samples)
+    held = _cells_with_a_row(monkeypatch)
     stats = {}
     got = tune(cfg, stats=stats)
     monkeypatch.setenv("MIST_NO_STAGE_COST_CUTOFF", "1")
     want = tune(cfg)
-    assert got == want
+    assert got == want and "mip_second_evaluations" not in stats
+    assert sum(held[:len(held) // 2]) < sum(held[len(held) // 2:])
     assert want[1] is None or stats["mip_estimate"] > 0
     # an optimum that is not below the estimate's room: the second evaluation
     monkeypatch.delenv("MIST_NO_STAGE_COST_CUTOFF")
