@@ -520,7 +520,8 @@ def main():
                                 if "incumbent" in search.dev_plan else None),
         "stage_cost_cutoff_retries": stats.get("stage_cost_cutoff_retries", 0),
         # (tp, G) pairs of the timed steps whose partition inside the limit of the tables under
-        # the estimate the search could not rule out (each makes a step evaluate twice)
+        # the estimate the search could not rule out (a step evaluates twice only where its result
+        # depends on them, which the retries count)
         "dp_unresolved": stats.get("dp_unresolved", 0),
         "best_cost": cost,
         "best_solution": repr(solution),

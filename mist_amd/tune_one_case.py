@@ -296,11 +296,10 @@ class PreparedSearch:
             safe_below = estimate * limit_factor
             unresolved = stats.get("dp_unresolved", 0) - unresolved_before
             if np.isfinite(estimate) and (unresolved > 0 or not best_cost < safe_below):
-                # (counts the results in doubt, those that the search could settle by itself too)
-                stats["stage_cost_cutoff_retries"] = stats.get("stage_cost_cutoff_retries", 0) + 1
-                if stats["dp_undecided"] == undecided_before and best_cost < safe_below:
+                if stats.get("dp_undecided", 0) == undecided_before and best_cost < safe_below:
+                    stats["stage_cost_doubts_settled"] = stats.get("stage_cost_doubts_settled", 0) + 1
                     return best_cost, best_solution
-                stats["stage_cost_second_evaluations"] = stats.get("stage_cost_second_evaluations", 0) + 1
+                stats["stage_cost_cutoff_retries"] = stats.get("stage_cost_cutoff_retries", 0) + 1
                 self.stage_cost_cutoff = None
                 try:
                     return self.run(stats, split_timing)

@@ -19,7 +19,7 @@ def test_partition_of_the_winner(monkeypatch, plan, device, schedule):
     monkeypatch.setenv("MIST_DP_FORCE_SCHEDULE", schedule)
     stats = {}
     got = search.run(stats)
-    assert got[1] is not None and not stats.get("stage_cost_second_evaluations")
+    assert got[1] is not None and not stats.get("stage_cost_cutoff_retries")
     monkeypatch.delenv("MIST_DP_FORCE_SCHEDULE")
     search.stage_cost_cutoff = None
     assert search.run() == got

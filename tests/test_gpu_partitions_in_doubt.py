@@ -20,6 +20,7 @@ def test_result_is_that_of_complete_tables(seed, evaluations):
     search = PreparedSearch(_sparse_candidate_plan() if seed is None else _realistic_plan(seed))
     stats = {}
     got = search.run(stats)
-    assert stats["dp_unresolved"] > 0 and stats.get("stage_cost_second_evaluations", 0) == evaluations
+    assert stats["dp_unresolved"] > 0 and stats.get("stage_cost_cutoff_retries", 0) == evaluations
+    assert stats.get("stage_cost_doubts_settled", 0) == 1 - evaluations
     search.stage_cost_cutoff = None
     assert search.run() == got
