@@ -82,6 +82,7 @@ struct Buffer {
 };
 
 constexpr int kPathBatches = 6;  // as many keep them: searches have two or three
+constexpr size_t kMostPathBytes = (size_t)64 << 20;  // of a batch: 70B on 32x8, the largest, has 3 MB in its first one
 struct Workspace {
   Buffer d_in, d_out, d_scratch, d_req, d_counts, d_values, d_request, d_argmin, d_grad;
   Buffer h_in, h_out, h_req, h_counts, h_values, h_request, h_grad;
@@ -400,8 +401,12 @@ struct Search {
   }
   // the next batch's number, -1 = without partitions
   int keep_paths(int n) {
-    if (!keep || n_kept == kPathBatches || !keeps(n)) return -1;
-    if (ws->d_paths[n_kept].reserve(sizeof(int32_t) * path_offset(n_families, n)) != 0) return -1;
+    const size_t bytes = sizeof(int32_t) * path_offset(n_families, n);
+    if (!keep || n_kept == kPathBatches || bytes > kMostPathBytes || !keeps(n)) return -1;
+    if (ws->d_paths[n_kept].reserve(bytes) != 0) {
+      (void)hipGetLastError();  // (no memory for them; the next check of a launch is not to report it)
+      return -1;
+    }
     batch_instances[n_kept] = n;
     return n_kept++;
   }
