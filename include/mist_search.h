@@ -142,6 +142,10 @@ typedef struct MistProblem {
    * assignment up to incumbent * (1 + slack) may hold +inf / -1 throughout: an optimum no larger than that is the
    * optimum of the complete tables. */
   int32_t incumbent_close;
+  /* Doubles of the reduce workspace that the caller gives, 0 = mist_reduce_workspace_doubles(..): with fewer, down to
+   * mist_reduce_workspace_least_doubles(..), the log of rows that reached a minimum is shorter, and a call whose log
+   * runs full takes longer. */
+  int64_t reduce_doubles;
 } MistProblem;
 
 /* One (gradient-accumulation steps, device mesh) group = one call of the reference's
@@ -221,6 +225,8 @@ int64_t mist_key_terms_doubles(int64_t total_keys);
  * MistProblem.reduce_cells / _supers / _items and n_samples samples per call; `d_partial_index` is
  * reduce_cells * n_samples int32 */
 int64_t mist_reduce_workspace_doubles(int64_t cells, int64_t supers, int64_t items, int n_samples);
+/* ... of which the log may be left out (MistProblem.reduce_doubles); it takes up to 1.5 GiB. */
+int64_t mist_reduce_workspace_least_doubles(int64_t cells, int64_t supers, int64_t items, int n_samples);
 
 /* Row-invariant terms of every candidate row: decodes the row index, evaluates the alpha-beta
  * communication terms, the 36 interference evaluations and the memory pieces that do not

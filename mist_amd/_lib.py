@@ -71,6 +71,7 @@ PROBLEM_DTYPE = np.dtype(
         ("reduce_items", "<i8"),
         ("sparse_tables", "<i4"),
         ("incumbent_close", "<i4"),
+        ("reduce_doubles", "<i8"),
     ],
     align=True,
 )
@@ -139,6 +140,8 @@ _SIGNATURES = {
     "mist_stage_floor_doubles": (ctypes.c_int64, [ctypes.c_int64, ctypes.c_int]),
     "mist_key_terms_doubles": (ctypes.c_int64, [ctypes.c_int64]),
     "mist_reduce_workspace_doubles": (
+        ctypes.c_int64, [ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_int]),
+    "mist_reduce_workspace_least_doubles": (
         ctypes.c_int64, [ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_int]),
     "mist_row_terms": (ctypes.c_int, [_VP, _VP, ctypes.c_int, _VP, ctypes.c_int, _VP, _VP, _VP, _VP]),
     "mist_eval_reduce": (

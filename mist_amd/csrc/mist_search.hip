@@ -4556,7 +4556,8 @@ struct WorkspaceLayout {
   int64_t capacity;    // items per shard
   int64_t log_chunks;
 };
-static WorkspaceLayout workspace_layout(int64_t cells, int64_t supers, int64_t items, int n_samples) {
+// `doubles`: what there is (0: all that is of use), at least total - log_chunks' share.
+static WorkspaceLayout workspace_layout(int64_t cells, int64_t supers, int64_t items, int n_samples, int64_t doubles) {
   WorkspaceLayout w;
   w.capacity = (items + kQueueShards - 1) / kQueueShards + 1;
   w.best = 0;
@@ -4569,21 +4570,28 @@ static WorkspaceLayout workspace_layout(int64_t cells, int64_t supers, int64_t i
   // (two second-level summaries a group at least)
   w.log = w.reach + supers / 2 * (int64_t)(sizeof(GroupReach) / 8 + 2 * kSuperBlocks);
   w.log += w.log % 2;
-  // (a chunk of every wavefront's is as a rule not full)
-  w.log_chunks = std::min(kLogPerCell * cells * n_samples, kLogEntries) / kLogChunk + kReduceBlocks * (kReduceThreads / 64);
-  w.log_counts = w.log + w.log_chunks * kLogChunk * (int64_t)(sizeof(Hit) / 8);
+  // (a chunk of every wavefront's is as a rule not full; a log's cells are 32 bits)
+  w.log_chunks = std::min(kLogPerCell * cells * n_samples, kLogEntries) / kLogChunk + kReduceWorkers * (kReduceThreads / 64);
+  if (cells * n_samples > (int64_t)UINT32_MAX) w.log_chunks = 0;
+  constexpr int64_t kChunkDoubles = kLogChunk * (int64_t)(sizeof(Hit) / 8);
+  if (doubles > 0)  // (half a double per chunk for its count, and one more)
+    w.log_chunks = std::min(w.log_chunks, std::max<int64_t>(doubles - w.log - 1, 0) * 2 / (2 * kChunkDoubles + 1));
+  w.log_counts = w.log + w.log_chunks * kChunkDoubles;
   w.total = w.log_counts + w.log_chunks / 2 + 1;
   return w;
 }
 int64_t mist_reduce_workspace_doubles(int64_t cells, int64_t supers, int64_t items, int n_samples) {
   if (cells < 0 || supers < 0 || items < 0 || n_samples < 1) return -1;
-  return workspace_layout(cells, supers, items, n_samples).total;
+  return workspace_layout(cells, supers, items, n_samples, 0).total;
 }
-// (cells beyond 32 bits: no log; for tests MIST_REDUCE_LOG_CHUNKS is the most)
-static uint32_t log_chunks(int64_t chunks, int64_t cells) {
+int64_t mist_reduce_workspace_least_doubles(int64_t cells, int64_t supers, int64_t items, int n_samples) {
+  if (cells < 0 || supers < 0 || items < 0 || n_samples < 1) return -1;
+  return workspace_layout(cells, supers, items, n_samples, 1).total;
+}
+// (for tests MIST_REDUCE_LOG_CHUNKS is the most)
+static uint32_t log_chunks(int64_t chunks) {
   const char *most = getenv("MIST_REDUCE_LOG_CHUNKS");
-  if (cells > (int64_t)UINT32_MAX) chunks = 0;
-  return (uint32_t)(most == nullptr || *most == '\0' ? chunks : std::min(chunks, (int64_t)atoll(most)));
+  return (uint32_t)(most == nullptr || *most == '\0' ? chunks : std::min(chunks, std::max<int64_t>(atoll(most), 0)));
 }
 // rows_present: false = only the rows the seed launch gathers are, the others follow by need
 static int reduce_tables(const MistProblem *problem, int n_samples, double *d_partial_cost, int32_t *d_partial_index,
@@ -4592,7 +4600,11 @@ static int reduce_tables(const MistProblem *problem, int n_samples, double *d_pa
       problem->reduce_max_p < 1)
     return fail(MIST_E_INVALID, "MistProblem.reduce_* sizes of the workspace are not set");
   const WorkspaceLayout w =
-      workspace_layout(problem->reduce_cells, problem->reduce_supers, problem->reduce_items, n_samples);
+      workspace_layout(problem->reduce_cells, problem->reduce_supers, problem->reduce_items, n_samples,
+                       std::max<int64_t>(problem->reduce_doubles, 0));
+  if (problem->reduce_doubles < 0 || (problem->reduce_doubles > 0 && problem->reduce_doubles < w.total))
+    return fail(MIST_E_INVALID, "a reduce workspace of %lld doubles needs %lld", (long long)problem->reduce_doubles,
+                (long long)w.total);
   if (w.capacity >= (int64_t)1 << 31) return fail(MIST_E_INVALID, "too many (tile, stage) items");
   out->best = d_partial_cost + w.best;
   out->row = reinterpret_cast<uint32_t *>(d_partial_index);
@@ -4605,7 +4617,7 @@ static int reduce_tables(const MistProblem *problem, int n_samples, double *d_pa
   out->counter = reinterpret_cast<uint32_t *>(d_partial_cost + w.counters);
   out->log = reinterpret_cast<Hit *>(d_partial_cost + w.log);
   out->log_count = reinterpret_cast<uint32_t *>(d_partial_cost + w.log_counts);
-  out->log_chunks = log_chunks(w.log_chunks, problem->reduce_cells * n_samples);
+  out->log_chunks = log_chunks(w.log_chunks);
   out->gather_floor = d_partial_cost + w.gathered;
   out->reach = reinterpret_cast<GroupReach *>(d_partial_cost + w.reach);
   out->reach_parts = d_partial_cost + w.reach + problem->reduce_supers / 2 * (int64_t)(sizeof(GroupReach) / 8);

@@ -63,8 +63,12 @@ ROW_TERMS_BUDGET_BYTES = 24 << 30
 ROW_TERMS_FREE_SHARE = 0.25
 ROW_TERMS_LEAST_BYTES = 2 << 30
 # Minima tables (12 bytes per (l, c) pair, variant, p and sample) the launches of a multi-sample call
-# may hold: more samples go through them in batches.
+# may hold: more samples go through them in batches.  The log behind them is not counted: it takes 1.5 GiB at most ...
 MINIMA_BYTES = 8 << 30
+# ... and this share of the memory that is free, where that is known (of plans that ask for it) and less; none where
+# an allocation with it fails.  (The workspace with the log and without it, MB: 1.3B on 1x2 16 and 0.3, 7B on 4x8 342
+# and 40, 13B on 8x8 877 and 95, 22B on 16x8 1862 and 887, 70B on 32x8 2131 and 506.)
+LOG_FREE_SHARE = 1 / 32
 
 
 def _free_device_bytes(device: torch.device) -> Optional[int]:
@@ -431,13 +435,14 @@ class IntraStageTuner:
         wanted = self._wanted_cells()
         most, least = ROW_TERMS_BUDGET_BYTES, min(ROW_TERMS_BUDGET_BYTES, ROW_TERMS_LEAST_BYTES)
         built = self._build_groups(wanted, most)
+        free = None
         if int(built[0]["n_rows"].sum()) * 8 * _lib.ROW_TERMS > least:
             free = _free_device_bytes(self.device)
             budget = most if free is None else max(min(most, int(free * ROW_TERMS_FREE_SHARE)), least)
             if budget < most:
                 built = self._build_groups(wanted, budget)
         plan = self._finish_plan(*built)
-        plan["wanted"] = wanted
+        plan["wanted"], plan["free_bytes"] = wanted, free
         return plan
 
     def _build_groups(self, wanted: Optional[np.ndarray], budget_bytes: int):
@@ -824,12 +829,14 @@ class IntraStageTuner:
         self._sample_batch = min(len(self.sample_slots), _lib.MAX_SAMPLE_BATCH,
                                  max(1, MINIMA_BYTES // (12 * most["reduce_cells"])))
         n_index = self._sample_batch * most["reduce_cells"]
-        n_cost = lib.mist_reduce_workspace_doubles(most["reduce_cells"], most["reduce_supers"],
-                                                   most["reduce_items"], self._sample_batch)
+        sizes = most["reduce_cells"], most["reduce_supers"], most["reduce_items"], self._sample_batch
+        n_cost, n_least = lib.mist_reduce_workspace_doubles(*sizes), lib.mist_reduce_workspace_least_doubles(*sizes)
+        if plan.get("free_bytes") is not None:
+            n_cost = min(n_cost, n_least + int(plan["free_bytes"] * LOG_FREE_SHARE) // 8)
         if self.exhaustive:  # its chunks' minima behind the table
             slabs = max([int(b["reduce_prefix"][-1]) for b in plan["batches"]] + [1]) * _lib.SLOTS * _lib.LC_TILE
             n_index += slabs
-            n_cost = max(n_cost, most["reduce_cells"] + slabs)
+            n_cost = n_least = max(n_least, most["reduce_cells"] + slabs)
         # accumulation count of every row of the tables, and the planes of the p axis that its groups fill
         groups, n_mesh = plan["groups"], len(self.device_mesh_candidates)
         n_rows = len(self.gradient_accumulation_steps_candidates) * len(self.tp_sizes)
@@ -850,7 +857,7 @@ class IntraStageTuner:
         max_rows = max([b["total_rows"] for b in batches], default=0)
         max_groups = max([b["n_groups"] for b in batches], default=0)
         max_keys = max([b["total_keys"] for b in batches], default=0)
-        def workspace():
+        def workspace(n_cost):
             return dict(
                 row_terms=torch.empty(max(max_rows, 1) * _lib.ROW_TERMS, dtype=torch.float64, device=dev),
                 stage_floor=torch.empty(lib.mist_stage_floor_doubles(max_rows, max_groups),
@@ -862,7 +869,17 @@ class IntraStageTuner:
             )
         # several batches alternate between two workspaces on two streams, so that the tail of
         # one batch's launches overlaps the start of the next
-        workspaces = [workspace() for _ in range(2 if len(batches) > 1 else 1)]
+        n_workspaces = 2 if len(batches) > 1 else 1
+        workspaces = None
+        try:
+            workspaces = [workspace(n_cost) for _ in range(n_workspaces)]
+        except torch.cuda.OutOfMemoryError:
+            if n_cost == n_least:
+                raise
+        if workspaces is None:  # (behind the handler, which still holds what the attempt had got)
+            n_cost = n_least
+            workspaces = [workspace(n_cost) for _ in range(n_workspaces)]
+        plan["problem"]["reduce_doubles"] = n_cost
         out = dict(
             batches=batches, workspaces=workspaces, **workspaces[0],
             n_groups=0, groups=None, terms_prefix=None, reduce_prefix=None, scout_prefix=None,

@@ -29,3 +29,80 @@ def test_rows_of_the_minima(monkeypatch, samples, seeded, chunks):
         for kind in ("index", "stable", "delta"):
             a, b = getattr(got.device, kind)[v], getattr(want.device, kind)[v]
             assert torch.equal(a, b), f"{kind} of variant {v}: {int((a != b).sum())} of {a.numel()} differ"
+
+
+def _tune(samples, exhaustive=False):
+    from mist_amd.config import tp_candidates
+    from mist_amd.intra_tuning import IntraStageTuner
+
+    cfg, tables = tiny_plan(2, layers=13, hardware__num_nodes=2, hardware__num_gpus_per_node=4,
+                            training__global_batch_size=48, hardware__memory_capacity=9.0)
+    tuner = IntraStageTuner(tables, 13, [(1, 1), (1, 4), (2, 4)], [3, 6, 24], tp_candidates(cfg)[0], cfg,
+                            sample_size=samples, exhaustive=exhaustive)
+    return tuner, tuner.tune().device
+
+
+def _same(got, want):
+    import torch
+
+    return all(torch.equal(getattr(got, kind)[v], getattr(want, kind)[v])
+               for v in range(4) for kind in ("index", "stable", "delta"))
+
+
+# (a chunk takes 512.5 doubles, and one more)
+@pytest.mark.parametrize("samples, extra", [(1, 0), (1, 512), (1, 513), (1, 4000), (1, 4104), (30, 0), (30, 100001)])
+def test_workspace_with_room_for_a_shorter_log(monkeypatch, samples, extra):
+    from mist_amd import _lib, intra_tuning
+
+    _, want = _tune(samples, exhaustive=True)
+    free = 1 << 36
+    monkeypatch.setattr(intra_tuning, "_free_device_bytes", lambda device: free)
+    monkeypatch.setattr(intra_tuning, "ROW_TERMS_LEAST_BYTES", 0)  # (every plan asks)
+    monkeypatch.setattr(intra_tuning, "LOG_FREE_SHARE", 8 * extra / free)
+    tuner, got = _tune(samples)
+    problem = tuner._plan["problem"]
+    least = _lib.load().mist_reduce_workspace_least_doubles(
+        *(int(problem[key][0]) for key in ("reduce_cells", "reduce_supers", "reduce_items")), samples)
+    assert tuner._dev_plan["partial_cost"].numel() == int(problem["reduce_doubles"][0]) == least + extra
+    assert _same(got, want)
+    # one double short of what the launches need without a log
+    problem["reduce_doubles"] = least - 1
+    with pytest.raises(_lib.MistLibraryError, match="reduce workspace"):
+        tuner.run_prepared(tuner._plan, tuner._dev_plan)
+
+
+def test_workspace_where_memory_is_short(monkeypatch):
+    """An allocation that fails with the log is tried without it; one that fails without it fails."""
+    import torch
+
+    from mist_amd import _lib
+
+    _, want = _tune(3, exhaustive=True)
+    lib, empty, asked = _lib.load(), torch.empty, []
+    whole, least = ({}, {})
+
+    def sizes_of(kind, function):
+        def sizes(*args):
+            kind["doubles"] = function(*args)
+            return kind["doubles"]
+        return sizes
+
+    monkeypatch.setattr(lib, "mist_reduce_workspace_doubles", sizes_of(whole, lib.mist_reduce_workspace_doubles))
+    monkeypatch.setattr(lib, "mist_reduce_workspace_least_doubles",
+                        sizes_of(least, lib.mist_reduce_workspace_least_doubles))
+
+    def short(refused):
+        def allocate(size, *args, **kwargs):
+            asked.append(size)
+            if size in refused():
+                raise torch.cuda.OutOfMemoryError("short of memory")
+            return empty(size, *args, **kwargs)
+        return allocate
+
+    monkeypatch.setattr(torch, "empty", short(lambda: [whole.get("doubles")]))
+    tuner, got = _tune(3)
+    assert whole["doubles"] in asked and tuner._dev_plan["partial_cost"].numel() == least["doubles"]
+    assert _same(got, want)
+    monkeypatch.setattr(torch, "empty", short(lambda: [whole.get("doubles"), least.get("doubles")]))
+    with pytest.raises(torch.cuda.OutOfMemoryError):
+        _tune(3)

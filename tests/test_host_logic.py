@@ -874,3 +874,18 @@ def test_row_term_batches_follow_the_free_memory(builder, monkeypatch):
     monkeypatch.setattr(intra_tuning, "_free_device_bytes", unexpected)
     small = load_plan(2)
     assert len(IntraStageTuner(small[1], 32, [(1, 8), (4, 8)], [8, 16], 1, small[0], sample_size=1).prepare()["batches"]) == 1
+
+
+def test_reduce_workspace_with_and_without_the_log():
+    """What may be left out of the reduce workspace is the log: 16 bytes for 8 entries per minimum, 96 Mi at most, a
+    chunk for each of 3072 wavefronts; none where its cells would not fit 32 bits."""
+    lib = _lib.load()
+    chunk = 256 * 2 + 0.5
+    for cells, samples in ((1, 1), (23040, 1), (2255616, 1), (42751488, 1), (2255616, 30), (1 << 27, 32)):
+        sizes = cells, 6441, 453600, samples
+        whole, least = lib.mist_reduce_workspace_doubles(*sizes), lib.mist_reduce_workspace_least_doubles(*sizes)
+        chunks = min(8 * cells * samples, 96 << 20) // 256 + 3072 if cells * samples < 1 << 32 else 0
+        assert whole - least == int(chunks * chunk)
+        assert least >= cells * samples
+    assert lib.mist_reduce_workspace_least_doubles(-1, 1, 1, 1) == -1
+    assert lib.mist_reduce_workspace_least_doubles(1, 1, 1, 0) == -1
