@@ -403,10 +403,7 @@ struct Search {
   int keep_paths(int n) {
     const size_t bytes = sizeof(int32_t) * path_offset(n_families, n);
     if (!keep || n_kept == kPathBatches || bytes > kMostPathBytes || !keeps(n)) return -1;
-    if (ws->d_paths[n_kept].reserve(bytes) != 0) {
-      (void)hipGetLastError();  // (no memory for them; the next check of a launch is not to report it)
-      return -1;
-    }
+    if (ws->d_paths[n_kept].reserve(bytes) != 0) return -1;
     batch_instances[n_kept] = n;
     return n_kept++;
   }

@@ -66,7 +66,7 @@ ROW_TERMS_LEAST_BYTES = 2 << 30
 # may hold: more samples go through them in batches.  The log behind them is not counted: it takes 1.5 GiB at most ...
 MINIMA_BYTES = 8 << 30
 # ... and this share of the memory that is free, where that is known (of plans that ask for it) and less; none where
-# an allocation with it fails.  (The workspace with the log and without it, MB: 1.3B on 1x2 16 and 0.3, 7B on 4x8 342
+# an allocation beside it fails: the searches then go on without.  (The workspace with the log and without it, MB: 1.3B on 1x2 16 and 0.3, 7B on 4x8 342
 # and 40, 13B on 8x8 877 and 95, 22B on 16x8 1862 and 887, 70B on 32x8 2131 and 506.)
 LOG_FREE_SHARE = 1 / 32
 
@@ -879,7 +879,7 @@ class IntraStageTuner:
         if workspaces is None:  # (behind the handler, which still holds what the attempt had got)
             n_cost = n_least
             workspaces = [workspace(n_cost) for _ in range(n_workspaces)]
-        plan["problem"]["reduce_doubles"] = n_cost
+        plan["problem"]["reduce_doubles"], plan["reduce_least"] = n_cost, n_least
         out = dict(
             batches=batches, workspaces=workspaces, **workspaces[0],
             n_groups=0, groups=None, terms_prefix=None, reduce_prefix=None, scout_prefix=None,
@@ -892,6 +892,23 @@ class IntraStageTuner:
                 "n_groups", "groups", "terms_prefix", "reduce_prefix", "scout_prefix",
                 "n_terms_blocks", "n_reduce_blocks", "n_scout_blocks")})
         return out
+
+    def give_back_log(self, plan, dev_plan) -> bool:
+        """Where memory is short: workspaces without the log of rows.  False if they had none."""
+        n_least = plan["reduce_least"]
+        if int(plan["problem"]["reduce_doubles"][0]) == n_least:
+            return False
+        with torch.cuda.device(self.device), torch.cuda.stream(dev_plan["uploaded_on"]):
+            dev_plan["partial_cost"] = None
+            for w in dev_plan["workspaces"]:
+                w["partial_cost"] = None
+            torch.cuda.empty_cache()  # (the library allocates, too)
+            for w in dev_plan["workspaces"]:
+                w["partial_cost"] = torch.empty(n_least, dtype=torch.float64, device=self.device)
+        dev_plan["partial_cost"] = dev_plan["workspaces"][0]["partial_cost"]
+        dev_plan.pop("uploaded", None)  # (a launch on another stream waits for the new memory's)
+        plan["problem"]["reduce_doubles"] = n_least
+        return True
 
     def launch(self, plan, dev_plan, tables, events: Optional[list] = None) -> None:
         """Enqueues the kernels for every requested sample on the current stream; ``tables`` are
@@ -1052,7 +1069,13 @@ class IntraStageTuner:
             if assignment:
                 problem["incumbent_close"] = 2
         with torch.cuda.device(self.device):
-            costs, index, struct = self._allocate_flat(plan, fill_costs and not sparse, not sparse)
+            while True:
+                try:
+                    costs, index, struct = self._allocate_flat(plan, fill_costs and not sparse, not sparse)
+                    break
+                except torch.cuda.OutOfMemoryError:
+                    if not self.give_back_log(plan, dev_plan):
+                        raise
             self.launch(plan, dev_plan, struct)
             # (the tensor views of the tables are made while the kernels run)
             tables = self._table_views(costs, index)

@@ -245,6 +245,14 @@ class PreparedSearch:
         of the two halves (otherwise the first is launch time only and the second includes the
         wait for the kernels)."""
         stats = {} if stats is None else stats
+        try:
+            return self._run(stats, split_timing)
+        except (torch.cuda.OutOfMemoryError, _lib.MistLibraryError) as error:
+            if "out of memory" not in str(error) or not self.tuner.give_back_log(self.plan, self.dev_plan):
+                raise
+        return self._run(stats, split_timing)
+
+    def _run(self, stats: dict, split_timing: bool):
         hw = self.config.hardware
         t0 = time.perf_counter()
         # (tables with a limit are searched by the library's driver only)

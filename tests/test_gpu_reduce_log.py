@@ -106,3 +106,56 @@ def test_workspace_where_memory_is_short(monkeypatch):
     monkeypatch.setattr(torch, "empty", short(lambda: [whole.get("doubles"), least.get("doubles")]))
     with pytest.raises(torch.cuda.OutOfMemoryError):
         _tune(3)
+
+
+@pytest.mark.parametrize("where", ["tables", "costs", "library", "elsewhere"])
+def test_search_where_memory_is_short_beside_the_log(monkeypatch, where):
+    """Tables, cost tables or the library's own buffers that find no memory beside the log: the search goes on
+    without it.  A second failure, and any other error, is the caller's."""
+    import torch
+
+    from mist_amd import _lib
+    from mist_amd.tune_one_case import PreparedSearch
+
+    cfg, _ = tiny_plan(2, layers=13, hardware__num_nodes=2, hardware__num_gpus_per_node=4, training__global_batch_size=48)
+    search = PreparedSearch(cfg)
+    want = search.run()
+    problem, empty, failures = search.plan["problem"], torch.empty, []
+    assert int(problem["reduce_doubles"][0]) > search.plan["reduce_least"]
+    total = search.tuner._table_layout()[1][-1]
+    lib = _lib.load()
+    bounded = lib.mist_inter_stage_search_bounded
+    size = {"tables": 2 * total, "costs": 2 * total // search.tuner.table_samples}.get(where)
+    dtype = torch.float64 if where == "tables" else torch.float32
+
+    def allocate(shape, *args, **kwargs):
+        n = shape[0] if isinstance(shape, tuple) else shape
+        if n == size and kwargs.get("dtype") is dtype and most > len(failures):
+            failures.append(n)
+            raise torch.cuda.OutOfMemoryError("HIP out of memory")
+        return empty(shape, *args, **kwargs)
+
+    def searched(*args):
+        if where not in ("library", "elsewhere") or len(failures) >= most:
+            return bounded(*args)
+        failures.append(where)
+        raise _lib.MistLibraryError("hipMalloc failed: out of memory" if where == "library" else "null pointer argument")
+
+    monkeypatch.setattr(torch, "empty", allocate)
+    monkeypatch.setattr(lib, "mist_inter_stage_search_bounded", searched)
+    most = 1
+    if where == "elsewhere":
+        with pytest.raises(_lib.MistLibraryError, match="null pointer"):
+            search.run()
+        assert int(problem["reduce_doubles"][0]) > search.plan["reduce_least"]
+        return
+    assert search.run() == want and len(failures) == 1
+    assert search.dev_plan["partial_cost"].numel() == int(problem["reduce_doubles"][0]) == search.plan["reduce_least"]
+    assert search.dev_plan["partial_cost"] is search.dev_plan["workspaces"][0]["partial_cost"]
+    assert search.run() == want
+    most = 2
+    with pytest.raises((torch.cuda.OutOfMemoryError, _lib.MistLibraryError), match="out of memory"):
+        search.run()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        assert search.run() == want
