@@ -55,7 +55,7 @@ def kernel_source_sha256():
     import hashlib
 
     h = hashlib.sha256()
-    for name in ("mist_search.hip", "exact_arith.h", "mist_common.h"):
+    for name in ("mist_search.hip", "exact_arith.h", "mist_common.h", "mist_window_margin.h"):
         with open(os.path.join(REPO, "mist_amd", "csrc", name), "rb") as f:
             h.update(f.read())
     with open(os.path.join(REPO, "include", "mist_search.h"), "rb") as f:
